@@ -5,9 +5,9 @@
 // What bounds the other form there: every raw score goes to memory, comes back to be normalised and mixed,
 // goes out and comes back again, eight rows share what a block loads, and the values are applied by the
 // vector unit (2,048 rows over 1,024 keys and up to 130 blocks, 32 / 8 heads of 128: 0.65 ms of
-// scores, 0.5 of mixing, 1.2 of values; the three kernels here together 0.35).  The mixing needs every head's NORMALISED weight of an entry, so a
-// single walk with a running maximum cannot do it; but scores are cheap on the matrix cores, so they are
-// formed twice instead of being kept:
+// scores, 0.5 of mixing, 1.2 of values; the three kernels here together 0.35).  The mixing needs every head's
+// NORMALISED weight of an entry, so a single walk with a running maximum cannot do it; but scores are cheap
+// on the matrix cores, so they are formed twice instead of being kept:
 //   stats:    per (16 rows of one request, four heads, share of the entries) the maximum and the sum of exponentials;
 //   weights:  per (16 rows, run of entries) the scores of ALL heads again, their normalised weights, and the
 //             mixed ones, sum_g talk[h, g] w_g, as a matrix product over the heads;
@@ -20,6 +20,7 @@
 // pages of a multiple of 16) and block means (tiles of 16, padded to chunks of 32); a chunk is
 // either all tokens or all means.  Tiles never cross a request, so blocks find theirs by counting the requests' tiles.
 #include "common.h"
+#include "request_tiles.h"
 #include "slots.h"
 
 using namespace tk;
@@ -65,42 +66,21 @@ struct Tile {
   const int* table;
 };
 
-// The tile `at` of the step, counted request by request in tiles of 16 rows; false past the last one.
-// Every wave counts for itself: 64 requests a turn, a prefix sum over the lanes.
 __device__ __forceinline__ bool find_tile(const Args& a, int at, Tile& t) {
-  const int lane = threadIdx.x & (kWave - 1);
-  int before = 0;
-  for (int base = 0; base < a.R; base += kWave) {
-    const int r = base + lane;
-    const int count = r < a.R ? (a.q_start[r + 1] - a.q_start[r] + kRows - 1) / kRows : 0;
-    int upto = count;
-#pragma unroll
-    for (int m = 1; m < kWave; m <<= 1) {
-      const int other = __shfl_up(upto, m, kWave);
-      if (lane >= m) upto += other;
-    }
-    const int total = __shfl(upto, kWave - 1, kWave);
-    if (at < before + total) {
-      const unsigned long long mine = __ballot(at >= before + upto - count && at < before + upto);
-      const int owner = __ffsll(mine) - 1;
-      const int first = __shfl(before + upto - count, owner, kWave);
-      const int req = __builtin_amdgcn_readfirstlane(base + owner);
-      t.row = __builtin_amdgcn_readfirstlane(a.q_start[req] + (at - first) * kRows);
-      t.tq = min(kRows, a.q_start[req + 1] - t.row);
-      t.i0 = __builtin_amdgcn_readfirstlane(a.positions[t.row]);
-      t.i_last = t.i0 + t.tq - 1;
-      const int behind = t.i_last - a.size - (a.pool - 1);
-      t.NB = behind >= 0 ? behind / a.pool + 1 : 0;
-      t.j0 = max(0, t.i0 - a.size + 1);
-      t.ja = t.j0 & ~15;
-      t.PC = (t.NB + kChunk - 1) / kChunk;
-      t.chunks = t.PC + (t.i_last - t.ja + kChunk) / kChunk;
-      t.table = a.tables + (size_t)req * a.table_width;
-      return true;
-    }
-    before += total;
-  }
-  return false;
+  RequestTile rt;
+  if (!find_request_tile(a.q_start, a.R, kRows, at, rt)) return false;
+  t.row = a.q_start[rt.req] + rt.index * kRows;
+  t.tq = min(kRows, a.q_start[rt.req + 1] - t.row);
+  t.i0 = __builtin_amdgcn_readfirstlane(a.positions[t.row]);
+  t.i_last = t.i0 + t.tq - 1;
+  const int behind = t.i_last - a.size - (a.pool - 1);
+  t.NB = behind >= 0 ? behind / a.pool + 1 : 0;
+  t.j0 = max(0, t.i0 - a.size + 1);
+  t.ja = t.j0 & ~15;
+  t.PC = (t.NB + kChunk - 1) / kChunk;
+  t.chunks = t.PC + (t.i_last - t.ja + kChunk) / kChunk;
+  t.table = a.tables + (size_t)rt.req * a.table_width;
+  return true;
 }
 
 // a float's leading bfloat16 pieces: two numbers at a time, each piece packed

@@ -306,6 +306,12 @@ _SIGS = {
         "tk_fixed_decay_chunks": [c_int, c_void_p, c_int, c_int, c_long, c_long, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p],
     },
+    "scan_chunks": {
+        "tk_gla_chunks": [*[c_void_p, c_int, c_int, c_long] * 5, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                          c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_void_p],
+        "tk_wkv_chunks": [*[c_void_p, c_int, c_int, c_long] * 5, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                          c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p],
+    },
     "delta": {
         "tk_sum_columns": [c_int, c_void_p, c_int, c_long, c_long, c_int, c_void_p, c_int, c_int, c_void_p],
         "tk_delta_inputs": [c_int, c_void_p, c_int, c_int, c_long, c_long, c_void_p, c_int, c_int, c_long, c_long,
@@ -1046,6 +1052,24 @@ def tanh(x: torch.Tensor, out: torch.Tensor) -> None:
 
 WKV_MAX_DIM = 256
 
+SCAN_CHUNK = 16                # tokens of a chunk (csrc/scan_chunks.hip: kTokens)
+SCAN_CHUNKS_MAX_DIM = 128
+SCAN_CHUNKS_FROM_TOKENS = 32   # a request's tokens in a step from which the scans run in chunks
+
+
+def _scan_in_chunks(dtype: torch.dtype, dim: int, vdim: int, longest: int) -> bool:
+    """Whether a scan with a decay a key channel runs in chunks of 16 tokens on the matrix cores: bfloat16 steps with a
+    portion.  float32 keeps the walk a token at a time, whose bits do not depend on how a prompt is cut."""
+    return (dtype == torch.bfloat16 and longest >= SCAN_CHUNKS_FROM_TOKENS and dim % 16 == 0 and vdim % 16 == 0
+            and max(dim, vdim) <= SCAN_CHUNKS_MAX_DIM)
+
+
+def _chunk_scratch(batch, n: int, heads: int, dim: int, vdim: int, device):
+    """(chunks of the step, their operands, the outputs before the norm) for ``csrc/scan_chunks.hip``."""
+    chunks = sum(-(-t // SCAN_CHUNK) for t in batch.q_lens)
+    return (chunks, torch.empty((chunks, heads, 33 * dim + 16 * vdim + 256), dtype=torch.float32, device=device),
+            torch.empty((n, heads * vdim), dtype=torch.float32, device=device))
+
 
 def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tensor, decay_in: torch.Tensor,
              w0: torch.Tensor, u: torch.Tensor, gain: torch.Tensor, state: torch.Tensor, out: torch.Tensor, batch,
@@ -1065,6 +1089,12 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tens
     operands = [x for t, what in ((r, "r"), (k, "k"), (v, "v"), (gate, "gate"), (decay_in, "decay_in"))
                 for x in _branch(t, n, hd, dtype, what)]
     _note(f"{n}x{heads}x{dim}", n * hd * 6 * out.element_size(), 4.0 * n * heads * dim * dim)
+    if _scan_in_chunks(dtype, dim, dim, batch.max_q_len) and gain.data_ptr() % 16 == 0 and out.data_ptr() % 16 == 0:
+        chunks, scaled, raw = _chunk_scratch(batch, n, heads, dim, dim, out.device)
+        _check(_fn("scan_chunks", "tk_wkv_chunks")(
+            *operands, _p(w0), _p(u), _p(gain), _p(state), _p(batch.q_start), _p(batch.state_slots), _p(out), _p(scaled),
+            _p(raw), n, batch.num_requests, chunks, heads, dim, float(eps), _stream()), "wkv_chunks")
+        return
     _check(_fn("recurrent", "tk_wkv_scan")(
         _code(dtype), *operands, _p(w0), _p(u), _p(gain), _p(state),
         _p(batch.q_start), _p(batch.state_slots), _p(out), batch.num_requests, heads, dim, float(eps), _stream()),
@@ -1090,6 +1120,14 @@ def gla_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tens
     operands = [x for t, what, w in ((q, "q", heads * dim), (k, "k", heads * dim), (v, "v", heads * vdim),
                                      (gate, "gate", heads * vdim), (decay_in, "decay_in", heads * dim))
                 for x in _branch(t, n, w, dtype, what)]
+    if _scan_in_chunks(dtype, dim, vdim, batch.max_q_len) and gain.data_ptr() % 16 == 0 and out.data_ptr() % 16 == 0:
+        chunks, scaled, raw = _chunk_scratch(batch, n, heads, dim, vdim, out.device)
+        _note(f"{n}x{heads}x{dim}x{vdim} chunks", n * heads * (3 * dim + 3 * vdim) * out.element_size(), 4.0 * n * heads * dim * vdim)
+        _check(_fn("scan_chunks", "tk_gla_chunks")(
+            *operands, _p(bias), _p(gain), _p(state), _p(batch.q_start), _p(batch.state_slots), _p(out), _p(scaled), _p(raw),
+            n, batch.num_requests, chunks, heads, dim, vdim, float(q_scale), 1.0 / float(tau), float(eps), _stream()),
+            "gla_chunks")
+        return
     splits = gla_column_splits(batch.num_requests, heads, vdim, batch.max_q_len)
     # (scratch of a scan with shared columns: the raw outputs, and behind them the decays)
     raw = torch.empty((n, heads * (vdim + dim)), dtype=torch.float32, device=out.device) if splits > 1 else None
