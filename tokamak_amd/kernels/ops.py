@@ -241,6 +241,9 @@ _SIGS = {
         "tk_moe_grouped": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                            c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     },
+    "moe_stream": {
+        "tk_moe_stream": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    },
     "gemm_tiled": {
         "tk_gemm_tiled": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long,
                           c_long, c_long, c_void_p],
@@ -1453,6 +1456,46 @@ def moe_down(act: torch.Tensor, down: torch.Tensor, chosen: torch.Tensor, out: t
     _note(f"{n}x{top} {w}x{f}", min(n * top, e) * w * f * act.element_size(), 2.0 * n * top * w * f)
     _check(_fn("moe", "tk_moe_down")(_code(act.dtype), _p(act), _p(down), _p(chosen), _p(out), n, w, f, top, _stream()),
            "moe_down")
+
+
+MOE_STREAM_MAX_PAIRS = 1024    # pairs a block of the streaming form can list (csrc/moe_stream.hip: kMaxPairs)
+# pairs an expert has on average up to which the streaming form is taken, and the same for small experts (width times
+# ff up to MOE_STREAM_SMALL).  Both products, streamed against grouped with its lists' kernel (16 experts, two a token):
+# 4,096 x 6,144 at 16 pairs an expert 313 + 202 against 303 + 250 us, at 32 534 + 304 against 312 + 252; 1,024 x 1,024
+# at 16 20 + 15 against 40 + 34, at 32 32 + 19 against 41 + 36; 1,024 x 1,536 at 50 58 + 39 against 55 + 52
+MOE_STREAM_PER_EXPERT = 16
+MOE_STREAM_PER_SMALL_EXPERT = 32
+MOE_STREAM_SMALL = 1 << 21
+
+
+def moe_stream_fits(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, pairs: int) -> bool:
+    """Whether a step's expert products read each expert's weights once, a block an expert and 16 channels
+    (``csrc/moe_stream.hip``): bfloat16, rows of 16-byte pieces, and so few pairs that the weights' bytes are the work.
+    Beyond 64 pairs every expert has blocks, met or not, so there must not be more experts than pairs."""
+    experts, f = gate_up.shape[0], down.shape[2]
+    most = MOE_STREAM_PER_SMALL_EXPERT if h.shape[1] * f <= MOE_STREAM_SMALL else MOE_STREAM_PER_EXPERT
+    return (h.dtype == torch.bfloat16 and h.shape[1] % 8 == 0 and f % 8 == 0 and pairs <= MOE_STREAM_MAX_PAIRS
+            and (pairs <= 64 or experts <= pairs <= most * experts)
+            and h.data_ptr() % 16 == 0 and gate_up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0)
+
+
+def moe_stream(x: torch.Tensor, weights: torch.Tensor, chosen: torch.Tensor, pair_weight: torch.Tensor | None,
+               out: torch.Tensor, *, tokens: int, top: int, gated: bool, weight_on_output: bool = False) -> None:
+    """One of the experts' two products, operands and result as ``moe_grouped``'s, straight from the lists of chosen experts."""
+    _gpu(x, weights, chosen, pair_weight, out)
+    e, rows, k = weights.shape
+    r = rows // (2 if gated else 1)
+    _need(x.dtype == weights.dtype == torch.bfloat16 and x.shape == (tokens if gated else tokens * top, k) and k % 8 == 0,
+          "streamed expert products are bfloat16 with rows of 16-byte pieces")
+    _need(chosen.dtype == torch.int32 and chosen.numel() >= tokens * top and tokens * top <= MOE_STREAM_MAX_PAIRS, "the chosen experts do not match")
+    if gated:
+        _need(out.dtype == torch.bfloat16 and out.shape == (tokens * top, r) and pair_weight is not None
+              and pair_weight.dtype == torch.float32 and pair_weight.numel() >= tokens * top, "gated output does not match")
+    else:
+        _need(out.dtype == torch.float32 and out.shape == (top, tokens, r), "the pairs' outputs are float32 [top, tokens, width]")
+    _note(f"{tokens}x{top} {rows}x{k}", min(tokens * top, e) * rows * k * 2, 2.0 * tokens * top * rows * k)
+    _check(_fn("moe_stream", "tk_moe_stream")((2 if weight_on_output else 1) if gated else 0, _p(x), _p(weights), _p(chosen),
+                                              _p(pair_weight), _p(out), tokens, top, e, r, k, _stream()), "moe_stream")
 
 
 MOE_TILE_PAIRS = 64        # pairs of one expert that a block of the grouped products takes (csrc/moe.hip: kTilePairs)

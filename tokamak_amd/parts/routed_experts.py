@@ -143,6 +143,11 @@ class RoutedExperts(FeedForward):
         on_output = self.weight_on == "output"
         act = torch.empty((n * top, self.intermediate_size), dtype=h.dtype, device=h.device)
         out = torch.empty((top, n, self.hidden_size), dtype=torch.float32, device=h.device)
+        if ops.moe_stream_fits(h, self.gate_up, self.down, n * top):
+            # few tokens: every expert the step meets reads its weights once
+            ops.moe_stream(h, self.gate_up, chosen, weight, act, tokens=n, top=top, gated=True, weight_on_output=on_output)
+            ops.moe_stream(act, self.down, chosen, None, out, tokens=n, top=top, gated=False)
+            return out
         if ops.moe_grouped_fits(h, self.gate_up, self.down, n * top):
             # many tokens: the pairs listed expert by expert, tiles of one expert on the matrix cores
             lists = ops.moe_sort(chosen, self.num_experts)
