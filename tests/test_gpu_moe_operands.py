@@ -1,0 +1,53 @@
+"""The experts' products with weights in operand order, against float64 on the same operands: an expert's weights read
+once (few tokens) and tiles of 128 pairs (many); pairs that share an expert and pairs that do not, tiles and passes that
+are nearly empty, remainders of K and of the channels."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("n,top,experts,w,f,skew", [
+    (1, 2, 16, 1024, 1024, 0), (1, 1, 1, 64, 64, 0), (8, 2, 16, 320, 192, 0), (17, 3, 5, 576, 64, 0), (32, 2, 64, 256, 1088, 0),
+    (40, 2, 16, 1088, 320, 0), (64, 1, 3, 512, 64, 0), (100, 2, 4, 128, 64, 0), (70, 2, 8, 320, 128, 1), (130, 4, 33, 64, 128, 1),
+    (257, 2, 3, 192, 576, 1)])
+@pytest.mark.parametrize("form", ["stream", "tiles"])
+@pytest.mark.parametrize("on_output", [False, True])
+def test_experts_in_operand_order(n, top, experts, w, f, skew, form, on_output):
+    from tokamak_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(n + w)
+    h = torch.randn(n, w, generator=g).bfloat16()
+    gate_up = (torch.randn(experts, 2 * f, w, generator=g) * 1.5 * w ** -0.5).bfloat16()
+    down = (torch.randn(experts, w, f, generator=g) * f ** -0.5).bfloat16()
+    score = torch.rand(n, experts, generator=g)
+    if skew:
+        score[:, 0] += 2.0      # one expert that every token takes
+    chosen = score.topk(top, dim=-1).indices.int()
+    weight = torch.rand(n, top, generator=g)
+    first, second = (ops.expert_operands(t.to(DEV)) for t in (gate_up, down))
+    hd, cd, wd = (t.to(DEV) for t in (h, chosen, weight))
+    act = torch.full((n * top, f), float("nan"), dtype=torch.bfloat16, device=DEV)
+    out = torch.full((top, n, w), float("nan"), dtype=torch.float32, device=DEV)
+    if form == "stream":
+        ops.moe_stream(hd, first, cd, wd, act, tokens=n, top=top, gated=True, weight_on_output=on_output)
+        ops.moe_stream(act, second, cd, None, out, tokens=n, top=top, gated=False)
+    else:
+        lists = ops.moe_sort(cd, experts, ops.MOE_WIDE_TILE_PAIRS)
+        ops.moe_tiles(hd, first, lists, wd, act, tokens=n, top=top, gated=True, weight_on_output=on_output)
+        ops.moe_tiles(act, second, lists, None, out, tokens=n, top=top, gated=False)
+    act, out = act.cpu(), out.cpu()
+    for e in range(experts):
+        token, place = (chosen == e).nonzero(as_tuple=True)
+        pair, x = token * top + place, weight[token, place].double()[:, None]
+        both = h[token].double() @ gate_up[e].double().T
+        gate, up = both[:, :f], both[:, f:]
+        want = torch.nn.functional.silu(gate) * up * x if on_output else torch.nn.functional.silu(x * gate) * (x * up)
+        got = act[pair].double()
+        # one rounding to bfloat16 behind float32 sums of up to 1,088 products
+        assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
+        want = got @ down[e].double().T
+        assert float((out[place, token].double() - want).abs().max().nan_to_num(0.0) if token.numel() else 0.0) <= 2e-5 * (1.0 + float(want.abs().max() if token.numel() else 0.0))
+    assert bool(torch.isfinite(out).all())

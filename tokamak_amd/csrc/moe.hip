@@ -750,12 +750,12 @@ TK_API int tk_moe_down(int dtype, const void* act, const void* down, const int* 
   return launch_status();
 }
 
-// The pairs of `chosen` [P] listed expert by expert and cut into tiles of up to tile_pairs (64):
+// The pairs of `chosen` [P] listed expert by expert and cut into tiles of up to tile_pairs (64, or 128 for moe_operands.hip):
 // order [P], tile_expert / tile_start / tile_count [P / tile_pairs + E], num_tiles [1].
 TK_API int tk_moe_sort(const int* chosen, int P, int E, int tile_pairs, int* order, int* tile_expert, int* tile_start,
                        int* tile_count, int* num_tiles, hipStream_t stream) {
   if (P <= 0) return 0;
-  if (E < 1 || (size_t)(3 * E + 1) * 4 > 60 * 1024 || tile_pairs != kTilePairs) return -1;
+  if (E < 1 || (size_t)(3 * E + 1) * 4 > 60 * 1024 || (tile_pairs != kTilePairs && tile_pairs != 2 * kTilePairs)) return -1;
   moe_sort_kernel<<<1, kSortThreads, (size_t)(3 * E + 1) * sizeof(int), stream>>>(chosen, P, E, tile_pairs, order, tile_expert,
                                                                                  tile_start, tile_count, num_tiles);
   return launch_status();

@@ -241,8 +241,10 @@ _SIGS = {
         "tk_moe_grouped": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                            c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     },
-    "moe_stream": {
+    "moe_operands": {
         "tk_moe_stream": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
+        "tk_moe_tiles": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                         c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     },
     "gemm_tiled": {
         "tk_gemm_tiled": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long,
@@ -1458,46 +1460,80 @@ def moe_down(act: torch.Tensor, down: torch.Tensor, chosen: torch.Tensor, out: t
            "moe_down")
 
 
-MOE_STREAM_MAX_PAIRS = 1024    # pairs a block of the streaming form can list (csrc/moe_stream.hip: kMaxPairs)
+MOE_STREAM_MAX_PAIRS = 1024    # pairs a block of the streaming form can list (csrc/moe_operands.hip: kMaxPairs)
 # pairs an expert has on average up to which the streaming form is taken, and the same for small experts (width times
-# ff up to MOE_STREAM_SMALL).  Both products, streamed against grouped with its lists' kernel (16 experts, two a token):
-# 4,096 x 6,144 at 16 pairs an expert 313 + 202 against 303 + 250 us, at 32 534 + 304 against 312 + 252; 1,024 x 1,024
-# at 16 20 + 15 against 40 + 34, at 32 32 + 19 against 41 + 36; 1,024 x 1,536 at 50 58 + 39 against 55 + 52
-MOE_STREAM_PER_EXPERT = 16
-MOE_STREAM_PER_SMALL_EXPERT = 32
+# ff up to MOE_STREAM_SMALL).  Both products, streamed against tiles with the kernel that lists them (some 6 us; 16
+# experts, two a token): 4,096 x 6,144 at 5 pairs an expert 277 + 147 against 274 + 146 us, at 16 333 + 198 against
+# 279 + 181; 1,024 x 1,024 at 16 20 + 14 against 26 + 19, at 32 30 + 19 against 30 + 22; 1,024 x 1,536 at 16 27 + 21
+# against 27 + 29, at 32 43 + 27 against 30 + 31
+MOE_STREAM_PER_EXPERT = 5
+MOE_STREAM_PER_SMALL_EXPERT = 24
 MOE_STREAM_SMALL = 1 << 21
 
 
-def moe_stream_fits(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, pairs: int) -> bool:
-    """Whether a step's expert products read each expert's weights once, a block an expert and 16 channels
-    (``csrc/moe_stream.hip``): bfloat16, rows of 16-byte pieces, and so few pairs that the weights' bytes are the work.
-    Beyond 64 pairs every expert has blocks, met or not, so there must not be more experts than pairs."""
-    experts, f = gate_up.shape[0], down.shape[2]
-    most = MOE_STREAM_PER_SMALL_EXPERT if h.shape[1] * f <= MOE_STREAM_SMALL else MOE_STREAM_PER_EXPERT
-    return (h.dtype == torch.bfloat16 and h.shape[1] % 8 == 0 and f % 8 == 0 and pairs <= MOE_STREAM_MAX_PAIRS
-            and (pairs <= 64 or experts <= pairs <= most * experts)
-            and h.data_ptr() % 16 == 0 and gate_up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0)
+def expert_operands(matrices: torch.Tensor) -> torch.Tensor:
+    """Matrices [E, R, K] (R a multiple of 32, K of 64) in the order of the matrix operands that ``csrc/moe_operands.hip``
+    reads, [E, R / 32, K / 32, 4, 32, 8]: blocks of 32 rows by 32 k, a block as [octet of k][row][8 k]."""
+    e, rows, k = matrices.shape
+    _need(rows % 32 == 0 and k % 64 == 0, "operand order takes rows in blocks of 32 and k in blocks of 64")
+    return matrices.view(e, rows // 32, 32, k // 32, 4, 8).permute(0, 1, 3, 4, 2, 5).contiguous()
 
 
-def moe_stream(x: torch.Tensor, weights: torch.Tensor, chosen: torch.Tensor, pair_weight: torch.Tensor | None,
-               out: torch.Tensor, *, tokens: int, top: int, gated: bool, weight_on_output: bool = False) -> None:
-    """One of the experts' two products, operands and result as ``moe_grouped``'s, straight from the lists of chosen experts."""
-    _gpu(x, weights, chosen, pair_weight, out)
-    e, rows, k = weights.shape
-    r = rows // (2 if gated else 1)
-    _need(x.dtype == weights.dtype == torch.bfloat16 and x.shape == (tokens if gated else tokens * top, k) and k % 8 == 0,
-          "streamed expert products are bfloat16 with rows of 16-byte pieces")
-    _need(chosen.dtype == torch.int32 and chosen.numel() >= tokens * top and tokens * top <= MOE_STREAM_MAX_PAIRS, "the chosen experts do not match")
+def takes_expert_operands(dtype: torch.dtype, width: int, ff: int) -> bool:
+    """Whether a mixture's experts keep their weights in operand order: bfloat16, both sizes multiples of 64."""
+    return dtype == torch.bfloat16 and width % 64 == 0 and ff % 64 == 0
+
+
+def moe_stream_fits(width: int, ff: int, experts: int, pairs: int) -> bool:
+    """Whether a step's products of experts in operand order read each expert's weights once, a block an expert and 16
+    channels (``moe_stream``), rather than once a tile of 128 pairs (``moe_tiles``): so few pairs that the
+    weights' bytes are the work.  Beyond 64 pairs every expert has blocks, met or not, so there must not be more
+    experts than pairs."""
+    most = MOE_STREAM_PER_SMALL_EXPERT if width * ff <= MOE_STREAM_SMALL else MOE_STREAM_PER_EXPERT
+    return pairs <= MOE_STREAM_MAX_PAIRS and (pairs <= 64 or experts <= pairs <= most * experts)
+
+
+def _expert_product(x, weights, pair_weight, out, tokens: int, top: int, gated: bool) -> tuple[int, int, int]:
+    """(experts, channels, k) of a product with experts in operand order, its operands checked."""
+    e, k = weights.shape[0], weights.shape[2] * 32
+    r = weights.shape[1] * 32 // (2 if gated else 1)
+    _need(x.dtype == weights.dtype == torch.bfloat16 and x.shape == (tokens if gated else tokens * top, k)
+          and tuple(weights.shape[3:]) == (4, 32, 8) and weights.is_contiguous(), "expert weights are bfloat16 in operand order")
     if gated:
         _need(out.dtype == torch.bfloat16 and out.shape == (tokens * top, r) and pair_weight is not None
               and pair_weight.dtype == torch.float32 and pair_weight.numel() >= tokens * top, "gated output does not match")
     else:
         _need(out.dtype == torch.float32 and out.shape == (top, tokens, r), "the pairs' outputs are float32 [top, tokens, width]")
+    rows = weights.shape[1] * 32
     _note(f"{tokens}x{top} {rows}x{k}", min(tokens * top, e) * rows * k * 2, 2.0 * tokens * top * rows * k)
-    _check(_fn("moe_stream", "tk_moe_stream")((2 if weight_on_output else 1) if gated else 0, _p(x), _p(weights), _p(chosen),
-                                              _p(pair_weight), _p(out), tokens, top, e, r, k, _stream()), "moe_stream")
+    return e, r, k
 
 
+def moe_stream(x: torch.Tensor, weights: torch.Tensor, chosen: torch.Tensor, pair_weight: torch.Tensor | None,
+               out: torch.Tensor, *, tokens: int, top: int, gated: bool, weight_on_output: bool = False) -> None:
+    """One of the experts' two products, operands and result as ``moe_grouped``'s but the weights in operand order
+    ([E, rows / 32, K / 32, 4, 32, 8]), straight from the lists of chosen experts."""
+    _gpu(x, weights, chosen, pair_weight, out)
+    e, r, k = _expert_product(x, weights, pair_weight, out, tokens, top, gated)
+    _need(chosen.dtype == torch.int32 and chosen.numel() >= tokens * top and tokens * top <= MOE_STREAM_MAX_PAIRS, "the chosen experts do not match")
+    _check(_fn("moe_operands", "tk_moe_stream")((2 if weight_on_output else 1) if gated else 0, _p(x), _p(weights), _p(chosen),
+                                                _p(pair_weight), _p(out), tokens, top, e, r, k, _stream()), "moe_stream")
+
+
+def moe_tiles(x: torch.Tensor, weights: torch.Tensor, lists: tuple, pair_weight: torch.Tensor | None,
+              out: torch.Tensor, *, tokens: int, top: int, gated: bool, weight_on_output: bool = False) -> None:
+    """The same product over the tiles of 128 pairs of ``lists`` (``moe_sort``)."""
+    order, tile_expert, tile_start, tile_count, num_tiles, tile_pairs = lists
+    _gpu(x, weights, pair_weight, out)
+    _, r, k = _expert_product(x, weights, pair_weight, out, tokens, top, gated)
+    _need(order.numel() == tokens * top and tile_pairs == MOE_WIDE_TILE_PAIRS, "the pairs' list does not match")
+    _check(_fn("moe_operands", "tk_moe_tiles")(
+        (2 if weight_on_output else 1) if gated else 0, _p(x), _p(weights), _p(order), _p(tile_expert), _p(tile_start),
+        _p(tile_count), _p(num_tiles), _p(pair_weight), _p(out), tokens, top, r, k, tile_expert.numel(), tile_pairs, _stream()),
+        "moe_tiles")
+
+
+MOE_WIDE_TILE_PAIRS = 128  # pairs of a tile of moe_tiles (csrc/moe_operands.hip: kTile)
 MOE_TILE_PAIRS = 64        # pairs of one expert that a block of the grouped products takes (csrc/moe.hip: kTilePairs)
 MOE_GROUPED_FROM = 65      # pairs of a step from which the experts' products run grouped on the matrix cores
 
@@ -1515,7 +1551,7 @@ def moe_sort(chosen: torch.Tensor, num_experts: int, tile_pairs: int = MOE_TILE_
     ``tile_pairs``: (order, tile_expert, tile_start, tile_count, num_tiles, tile_pairs), int32 on the device."""
     _gpu(chosen)
     pairs = chosen.numel()
-    _need(tile_pairs == MOE_TILE_PAIRS, "tiles hold 64 pairs")
+    _need(tile_pairs in (MOE_TILE_PAIRS, MOE_WIDE_TILE_PAIRS), "tiles hold 64 or 128 pairs")
     max_tiles = pairs // tile_pairs + num_experts
     lists = torch.empty(pairs + 3 * max_tiles + 1, dtype=torch.int32, device=chosen.device)
     order, rest = lists[:pairs], lists[pairs:]

@@ -74,6 +74,7 @@ class RoutedExperts(FeedForward):
         if shared_gate is not None and shared_size is None:
             raise ValueError("a gate on the shared expert goes with a shared expert")
         self.logit_bias_name, self.shared_gate_name = logit_bias, shared_gate
+        self.operand_order = ops.takes_expert_operands(dtype, self.hidden_size, self.intermediate_size)
         self.logit_bias: torch.Tensor | None = None
         self.router = self.gate_up = self.down = None
         self.correction = self.shared_gate_up = self.shared_down = None
@@ -100,8 +101,11 @@ class RoutedExperts(FeedForward):
         router, expert, gate, up, down = self.names
         self.router = fetch(prefix + router)
         bases = [prefix + expert.format(e) for e in range(self.num_experts)]
-        self.gate_up = torch.stack([torch.cat([fetch(b + gate), fetch(b + up)], dim=0) for b in bases]).contiguous()
-        self.down = torch.stack([fetch(b + down) for b in bases]).contiguous()
+        # an expert's gate rows, then its up rows; in the order of the matrix operands where the sizes allow it (see _routed)
+        first = torch.stack([fetch(b + n) for b in bases for n in (gate, up)]).view(self.num_experts, -1, self.hidden_size)
+        self.gate_up = ops.expert_operands(first) if self.operand_order else first
+        second = torch.stack([fetch(b + down) for b in bases])
+        self.down = ops.expert_operands(second) if self.operand_order else second
         if self.correction_name is not None:
             self.correction = fetch(prefix + self.correction_name)      # (None if the checkpoint has none)
         if self.shared_size is not None:
@@ -143,10 +147,15 @@ class RoutedExperts(FeedForward):
         on_output = self.weight_on == "output"
         act = torch.empty((n * top, self.intermediate_size), dtype=h.dtype, device=h.device)
         out = torch.empty((top, n, self.hidden_size), dtype=torch.float32, device=h.device)
-        if ops.moe_stream_fits(h, self.gate_up, self.down, n * top):
-            # few tokens: every expert the step meets reads its weights once
-            ops.moe_stream(h, self.gate_up, chosen, weight, act, tokens=n, top=top, gated=True, weight_on_output=on_output)
-            ops.moe_stream(act, self.down, chosen, None, out, tokens=n, top=top, gated=False)
+        if self.operand_order:
+            if ops.moe_stream_fits(self.hidden_size, self.intermediate_size, self.num_experts, n * top):
+                # few tokens: every expert the step meets reads its weights once
+                ops.moe_stream(h, self.gate_up, chosen, weight, act, tokens=n, top=top, gated=True, weight_on_output=on_output)
+                ops.moe_stream(act, self.down, chosen, None, out, tokens=n, top=top, gated=False)
+            else:
+                lists = ops.moe_sort(chosen, self.num_experts, ops.MOE_WIDE_TILE_PAIRS)
+                ops.moe_tiles(h, self.gate_up, lists, weight, act, tokens=n, top=top, gated=True, weight_on_output=on_output)
+                ops.moe_tiles(act, self.down, lists, None, out, tokens=n, top=top, gated=False)
             return out
         if ops.moe_grouped_fits(h, self.gate_up, self.down, n * top):
             # many tokens: the pairs listed expert by expert, tiles of one expert on the matrix cores
