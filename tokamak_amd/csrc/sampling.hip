@@ -37,7 +37,10 @@ __device__ __forceinline__ void argmax_take(float& bv, int& bi, float v, int i) 
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
     const float* __restrict__ logits, float* __restrict__ part_v, int* __restrict__ part_i, int V,
     long ld, const float* __restrict__ temperature, const int* __restrict__ top_k,
-    const float* __restrict__ top_p, float* __restrict__ part_mass) {
+    const float* __restrict__ top_p, float* __restrict__ part_mass, uint32_t* __restrict__ clear, size_t clear_words) {
+  // scratch that later kernels add into: `clear_words` words a row, shared out over its blocks
+  for (size_t i = (size_t)blockIdx.x * kArgmaxThreads + threadIdx.x; i < clear_words; i += (size_t)kArgmaxSegments * kArgmaxThreads)
+    clear[blockIdx.y * clear_words + i] = 0u;
   __shared__ float best_v[kArgmaxThreads / kWave];
   __shared__ int best_i[kArgmaxThreads / kWave];
   const int seg = blockIdx.x, r = blockIdx.y;
@@ -143,20 +146,7 @@ TK_API int tk_argmax(const float* logits, int* out, float* out_value, float* par
   if (M <= 0) return 0;
   if (V <= 0 || M > 65535) return -1;
   argmax_segments_kernel<<<dim3(kArgmaxSegments, M), kArgmaxThreads, 0, stream>>>(logits, part_v, part_i, V, ld,
-                                                                                   nullptr, nullptr, nullptr, nullptr);
-  argmax_pick_kernel<<<M, kWave, 0, stream>>>(part_v, part_i, out, out_value);
-  return launch_status();
-}
-
-// The same, and for the rows with temperature[m] > 0 and no threshold the mass of every segment
-// relative to its maximum at that temperature (part_mass: M * tk_argmax_segments() floats), for tk_sample.
-TK_API int tk_argmax_masses(const float* logits, int* out, float* out_value, float* part_v, int* part_i,
-                            const float* temperature, const int* top_k, const float* top_p, float* part_mass,
-                            int M, int V, long ld, hipStream_t stream) {
-  if (M <= 0) return 0;
-  if (V <= 0 || M > 65535 || !temperature || !top_k || !top_p || !part_mass) return -1;
-  argmax_segments_kernel<<<dim3(kArgmaxSegments, M), kArgmaxThreads, 0, stream>>>(
-      logits, part_v, part_i, V, ld, temperature, top_k, top_p, part_mass);
+                                                                                   nullptr, nullptr, nullptr, nullptr, nullptr, 0);
   argmax_pick_kernel<<<M, kWave, 0, stream>>>(part_v, part_i, out, out_value);
   return launch_status();
 }
@@ -200,7 +190,7 @@ TK_API int tk_argmax_no_alloc(const float* logits, int* out, float* out_value, i
   ArgmaxScratch* scratch = argmax_scratch_of_current_device();
   if (scratch == nullptr) return -4;
   argmax_segments_kernel<<<dim3(kArgmaxSegments, M), kArgmaxThreads, 0, stream>>>(
-      logits, scratch->value, scratch->index, V, ld, nullptr, nullptr, nullptr, nullptr);
+      logits, scratch->value, scratch->index, V, ld, nullptr, nullptr, nullptr, nullptr, nullptr, 0);
   argmax_pick_kernel<<<M, kWave, 0, stream>>>(scratch->value, scratch->index, out, out_value);
   return launch_status();
 }
@@ -232,25 +222,31 @@ constexpr int kSampleThreads = 1024;
 constexpr int kBins = 4096;  // histogram bins of one radix pass (12 bits)
 
 // Prefix sums of one value per thread over the block, threads in index order; `scan`
-// holds kSampleThreads entries.  Returns the sum over the threads before this one;
+// holds an entry a wave.  Returns the sum over the threads before this one;
 // `inclusive` is that plus the thread's own value as the scan computed it (so the
 // ranges [exclusive, inclusive) of the threads tile [0, total) exactly, also in
 // floating point); `total` is the sum over all threads.
 template <typename T>
 __device__ __forceinline__ T block_scan(T v, T* scan, T& inclusive, T& total) {
-  const int tid = threadIdx.x;
-  __syncthreads();
-  scan[tid] = v;
-  __syncthreads();
-  for (int step = 1; step < kSampleThreads; step <<= 1) {
-    const T add = tid >= step ? scan[tid - step] : T(0);
-    __syncthreads();
-    scan[tid] += add;
-    __syncthreads();
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave, waves = blockDim.x / kWave;
+  T upto = v;
+#pragma unroll
+  for (int step = 1; step < kWave; step <<= 1) {
+    const T other = __shfl_up(upto, step, kWave);
+    if (lane >= step) upto += other;
   }
-  total = scan[kSampleThreads - 1];
-  inclusive = scan[tid];
-  return tid > 0 ? scan[tid - 1] : T(0);
+  __syncthreads();
+  if (lane == kWave - 1) scan[wave] = upto;
+  __syncthreads();
+  T before = 0;                      // of the waves before this one
+  total = 0;
+  for (int w = 0; w < waves; ++w) {
+    if (w == wave) before = total;
+    total += scan[w];
+  }
+  inclusive = before + upto;
+  const T left = __shfl_up(inclusive, 1, kWave);     // (a wave's first thread starts where the wave before it ends)
+  return lane > 0 ? left : before;
 }
 
 // Walking the bins from the highest down: the bin in which the running sum first
@@ -259,8 +255,8 @@ __device__ __forceinline__ T block_scan(T v, T* scan, T& inclusive, T& total) {
 template <typename T>
 __device__ __forceinline__ void crossing_bin(const T* hist, int nbins, T target, T* scan, int* found_bin,
                                              T* found_above, int& bin, T& above) {
-  const int tid = threadIdx.x;
-  const int per = nbins / kSampleThreads > 0 ? nbins / kSampleThreads : 1;
+  const int tid = threadIdx.x, threads = blockDim.x;
+  const int per = nbins / threads > 0 ? nbins / threads : 1;
   // thread t owns bins [top - per*t, top - per*t - per + 1], highest first
   T mine = 0;
   const int first = nbins - 1 - tid * per;
@@ -331,6 +327,206 @@ __device__ __forceinline__ void for_row(const float* __restrict__ row, int V, F 
   if (tid < V - done) f(done + tid, row[done + tid]);
 }
 
+// Rows with a threshold, shared between blocks: a row is cut into the segments of the argmax pass, a block each.
+//   sample_hist:    the first level's histogram of the whole row (counts, and probability mass if only top-p is asked
+//                   for), added into the row's in memory; and the pick of the argmax pass for every row.
+//   sample_collect: the values in the bin that holds the threshold, with their segments, into the row's list (in any
+//                   order: sums over the list are of integers), and the mass of the bins above it in each segment; with
+//                   both thresholds the bins above it are listed too, top-p's may lie there.
+// The sampler then starts from the histogram and the list and reads the row again only where the drawn number falls.
+// (A block that reads its row alone moves some 45 GB/s: 40 rows of 152 k logits, most with thresholds, took 95 us with
+// three passes over the row in one block; shared, 12 + 13 us and 21 for the rest, of which a segment's walk, the
+// ranks and the start are each a few memory round trips.)
+constexpr int kCandidates = 16384;
+constexpr int kShareThreads = 256;
+constexpr int kFew = 256;          // values among which a threshold is found by ranks
+
+struct SharedRows {              // scratch of the rows, null: every row is sampled by one block alone
+  uint32_t* hist32;              // [M][kBins], zeroed by the argmax pass, as the others
+  unsigned long long* hist64;    // [M][kBins]
+  uint32_t* count;               // [M] entries of the list
+  uint32_t* cand;                // [M][kCandidates] ordered images
+  uint8_t* segment;              // [M][kCandidates]
+  unsigned long long* above;     // [M][segments] mass of what is kept for certain and not listed
+};
+
+// f(index, value) for every element of a segment, each by one thread of the block
+template <typename F>
+__device__ __forceinline__ void for_segment(const float* __restrict__ row, int V, int seg, F f) {
+  const int per = ((V + kArgmaxSegments - 1) / kArgmaxSegments + 3) & ~3;
+  const int begin = min(V, seg * per), end = min(V, begin + per);
+  if ((reinterpret_cast<uintptr_t>(row) & 15) == 0) {
+    const int quads = (end - begin) / 4;
+#pragma unroll 4
+    for (int q = threadIdx.x; q < quads; q += kShareThreads) {
+      const float4 v = *reinterpret_cast<const float4*>(row + begin + 4 * q);
+      f(v.x);
+      f(v.y);
+      f(v.z);
+      f(v.w);
+    }
+    const int done = begin + 4 * quads;
+    if ((int)threadIdx.x < end - done) f(row[done + threadIdx.x]);
+  } else {
+    for (int i = begin + threadIdx.x; i < end; i += kShareThreads) f(row[i]);
+  }
+}
+
+__device__ __forceinline__ bool has_threshold(const float* temperature, const int* top_k, const float* top_p, int r, int V, bool& k_on, bool& p_on) {
+  k_on = top_k[r] > 0 && top_k[r] < V;
+  p_on = top_p[r] < 1.f;
+  return temperature[r] > 0.f && (k_on || p_on);
+}
+
+struct FirstLevel {
+  int bin;                          // the first histogram's bin that holds the threshold
+  uint32_t k_remaining;             // of top-k: how many of that bin's values still count
+  unsigned long long p_remaining;   // of top-p alone: how much of that bin's mass
+  uint32_t total;                   // values in that bin and above it
+  uint32_t inside;                  // values in that bin
+};
+
+// Where the first threshold of a row lies, from its first histograms (in LDS, or in memory on a 16-byte border: a thread's bins
+// lie side by side and are asked for together).  THREADS threads call; `scan` an entry a wave, `found` one.
+template <int THREADS>
+__device__ __forceinline__ FirstLevel first_level(const uint32_t* h32, const unsigned long long* h64, bool k_on, int k, float p_keep,
+                                                  unsigned long long* scan, FirstLevel* found) {
+  constexpr int PER = kBins / THREADS;
+  const int tid = threadIdx.x, low = kBins - PER * (tid + 1);     // this thread's bins [low, low + PER), walked from the top
+  uint32_t c[PER], count = 0, upto_c, all_c;
+  unsigned long long m[PER], mass = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    c[j] = h32[low + j];
+    m[j] = 0;
+  }
+  if (!k_on) {
+#pragma unroll
+    for (int j = 0; j < PER; ++j) m[j] = h64[low + j];
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    count += c[j];
+    mass += m[j];
+  }
+  const uint32_t before_c = block_scan<uint32_t>(count, reinterpret_cast<uint32_t*>(scan), upto_c, all_c);
+  unsigned long long target = (unsigned long long)k, run = before_c, upto = upto_c, whole;
+  if (!k_on) {
+    run = block_scan<unsigned long long>(mass, scan, upto, whole);
+    // the share of the whole mass that top_p allows (at least one unit)
+    const double share = (double)p_keep * (double)whole;
+    target = share < 1.0 ? 1ull : (unsigned long long)share;
+  }
+  if (tid == THREADS - 1 && upto < target) {     // beyond everything (rounding): the lowest bin
+    const unsigned long long left = target - (upto - (k_on ? (unsigned long long)c[0] : m[0]));
+    *found = {0, (uint32_t)left, left, all_c, c[0]};
+  }
+  if (run < target && target <= upto) {
+    uint32_t seen = before_c;
+#pragma unroll
+    for (int j = PER - 1; j >= 0; --j) {
+      const unsigned long long h = k_on ? (unsigned long long)c[j] : m[j];
+      seen += c[j];
+      if (run < target && target <= run + h) *found = {low + j, (uint32_t)(target - run), target - run, seen, c[j]};
+      run += h;
+    }
+  }
+  __syncthreads();
+  return *found;
+}
+
+__global__ __launch_bounds__(kShareThreads) void sample_hist_kernel(
+    const float* __restrict__ logits, long ld, int V, const float* __restrict__ temperature, const int* __restrict__ top_k,
+    const float* __restrict__ top_p, const float* __restrict__ seg_max, const int* __restrict__ seg_index, int* __restrict__ out,
+    float* __restrict__ row_max, SharedRows sh) {
+  __shared__ uint32_t h32[kBins];
+  __shared__ unsigned long long h64[kBins];
+  const int seg = blockIdx.x, r = blockIdx.y, lane = threadIdx.x & (kWave - 1);
+  // the row's maximum (every wave for itself); the first block leaves it, and the argmax
+  float bv = lane < kArgmaxSegments ? seg_max[r * kArgmaxSegments + lane] : -INFINITY;
+  int bi = lane < kArgmaxSegments ? seg_index[r * kArgmaxSegments + lane] : 0x7fffffff;
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    const float ov = __shfl_xor(bv, m, kWave);
+    const int oi = __shfl_xor(bi, m, kWave);
+    argmax_take(bv, bi, ov, oi);
+  }
+  if (seg == 0 && threadIdx.x == 0) {
+    out[r] = (bi == 0x7fffffff) ? 0 : bi;
+    row_max[r] = bv;
+  }
+  bool k_on, p_on;
+  if (!has_threshold(temperature, top_k, top_p, r, V, k_on, p_on)) return;
+  const float inv_t = 1.f / temperature[r], mx = bv * inv_t;
+  if (!(mx > -INFINITY)) return;
+  for (int i = threadIdx.x; i < kBins; i += kShareThreads) h32[i] = 0;
+  if (!k_on)
+    for (int i = threadIdx.x; i < kBins; i += kShareThreads) h64[i] = 0;
+  __syncthreads();
+  for_segment(logits + (size_t)r * ld, V, seg, [&](float logit) {
+    const float x = scaled(logit, inv_t);
+    const uint32_t bin = ordered(x) >> 20;
+    atomicAdd(&h32[bin], 1u);
+    if (!k_on) atomicAdd(&h64[bin], fixed_mass(x, mx));
+  });
+  __syncthreads();
+  for (int i = threadIdx.x; i < kBins; i += kShareThreads) {
+    const uint32_t n = h32[i];
+    if (n == 0) continue;
+    atomicAdd(&sh.hist32[(size_t)r * kBins + i], n);
+    if (!k_on) atomicAdd(&sh.hist64[(size_t)r * kBins + i], h64[i]);
+  }
+}
+
+__global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
+    const float* __restrict__ logits, long ld, int V, const float* __restrict__ temperature, const int* __restrict__ top_k,
+    const float* __restrict__ top_p, const float* __restrict__ row_max, SharedRows sh) {
+  __shared__ uint32_t kept[kBins];
+  __shared__ unsigned long long scan[kShareThreads / kWave];
+  __shared__ FirstLevel found;
+  __shared__ uint32_t count, first;
+  const int seg = blockIdx.x, r = blockIdx.y;
+  bool k_on, p_on;
+  if (!has_threshold(temperature, top_k, top_p, r, V, k_on, p_on) || !(row_max[r] > -INFINITY)) return;
+  const float inv_t = 1.f / temperature[r];
+  if (threadIdx.x == 0) count = 0;
+  const FirstLevel level = first_level<kShareThreads>(sh.hist32 + (size_t)r * kBins, sh.hist64 + (size_t)r * kBins, k_on, top_k[r], top_p[r],
+                                                      scan, &found);
+  const int low = level.bin;
+  const bool both = k_on && p_on;
+  if ((both ? level.total : level.inside) > (uint32_t)kCandidates) return;      // (the sampler walks the row)
+  const float mx = row_max[r] * inv_t;
+  unsigned long long above = 0;
+  // this block's values, then side by side into the row's list
+  for_segment(logits + (size_t)r * ld, V, seg, [&](float logit) {
+    const float x = scaled(logit, inv_t);
+    const uint32_t o = ordered(x);
+    const int bin = (int)(o >> 20);
+    if (bin == low || (both && bin > low)) {
+      const uint32_t at = atomicAdd(&count, 1u);
+      if (at < (uint32_t)kBins) kept[at] = o;
+      else {                                      // (a segment with more: one by one)
+        const uint32_t to = atomicAdd(&sh.count[r], 1u);
+        sh.cand[(size_t)r * kCandidates + to] = o;
+        sh.segment[(size_t)r * kCandidates + to] = (uint8_t)seg;
+      }
+    } else if (bin > low) {
+      above += fixed_mass(x, mx);
+    }
+  });
+  unsigned long long upto, whole;
+  block_scan<unsigned long long>(above, scan, upto, whole);
+  if (threadIdx.x == 0) sh.above[r * kArgmaxSegments + seg] = whole;
+  __syncthreads();
+  const uint32_t n = min(count, (uint32_t)kBins);
+  if (threadIdx.x == 0) first = n ? atomicAdd(&sh.count[r], n) : 0u;
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < n; i += kShareThreads) {
+    sh.cand[(size_t)r * kCandidates + first + i] = kept[i];
+    sh.segment[(size_t)r * kCandidates + first + i] = (uint8_t)seg;
+  }
+}
+
 // One block per row.  params rows: temperature, top_k, top_p (floats);
 // seeds/counters: the request's seed and how many draws it has made.
 // probs_out (optional, [M, V]) receives the final distribution, for tests.
@@ -344,20 +540,25 @@ __device__ __forceinline__ void for_row(const float* __restrict__ row, int V, F 
 // lies; if the values of that bin and the bins above it are few (up to kCandidates; they
 // are, unless the logits are nearly all alike), a second pass copies them into LDS, and every
 // further level of both searches reads those.  The third pass is the draw's.  (Without the
-// copies: seven passes with both thresholds.)
-constexpr int kCandidates = 16384;
-
+// copies: seven passes with both thresholds.)  Up to kSharedRows rows the first pass and the copies are those of
+// sample_hist and sample_collect; with more rows a block each fills the GPU.
 __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     const float* __restrict__ logits, long ld, int V, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ top_p,
     const unsigned long long* __restrict__ seeds, const unsigned long long* __restrict__ counters,
     const float* __restrict__ row_max, const float* __restrict__ seg_max, const float* __restrict__ seg_mass,
-    int* __restrict__ out, float* __restrict__ probs_out) {
+    int* __restrict__ out, float* __restrict__ probs_out, SharedRows shared) {
   __shared__ float fs[kArgmaxSegments];  // the masses of the row's chunks (16 of the waves, or the 32 segments of the argmax pass)
   __shared__ unsigned long long hist64[kBins];
   __shared__ uint32_t hist32[kBins];
-  __shared__ unsigned long long scan64[kSampleThreads];
+  __shared__ unsigned long long scan64[kSampleThreads / kWave];
   __shared__ uint32_t cand[kCandidates];  // ordered images of the values that may hold a threshold
+  __shared__ uint8_t cand_segment[kCandidates];
+  __shared__ FirstLevel first;
+  __shared__ uint32_t few[kFew], few_count;
+  __shared__ unsigned long long few_mass[kFew];
+  __shared__ uint32_t few_cut;
+  __shared__ unsigned long long segment_mass[kArgmaxSegments];
   __shared__ uint32_t cand_count;
   __shared__ int found_bin;
   __shared__ int last_token;
@@ -383,44 +584,46 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   uint32_t k_prefix = 0, k_remaining = (uint32_t)max(k, 0);
   uint32_t p_prefix = 0;               // only top-p: its first level is found by the first pass
   unsigned long long p_remaining = 0;
+  bool listed = false;                 // cand comes with its values' segments
   int ncand = -1;                      // >= 0: cand[0 .. ncand) hold every value that can be a threshold
   if (k_on || p_on) {
-    for (int i = tid; i < kBins; i += nt) {
-      hist32[i] = 0;
-      hist64[i] = 0;
-    }
+    const bool ready = shared.hist32 != nullptr;     // (the row's first pass is done)
     if (tid == 0) cand_count = 0;
-    __syncthreads();
-    for_row(row, V, [&](int, float logit) {
-      const float x = scaled(logit, inv_t);
-      const uint32_t bin = ordered(x) >> 20;
-      atomicAdd(&hist32[bin], 1u);
-      if (!k_on) atomicAdd(&hist64[bin], fixed_mass(x, mx));
-    });
-    __syncthreads();
-    int low_bin;
-    if (k_on) {
-      uint32_t above;
-      crossing_bin<uint32_t>(hist32, kBins, k_remaining, scan32, &found_bin,
-                             reinterpret_cast<uint32_t*>(&found_above), low_bin, above);
-      k_remaining -= above;
-      k_prefix = (uint32_t)low_bin;
-    } else {
-      // the whole mass, then the share of it that top_p allows (at least one unit)
-      unsigned long long mine = 0, upto, whole, above;
-      for (int i = tid; i < kBins; i += nt) mine += hist64[i];
-      block_scan<unsigned long long>(mine, scan64, upto, whole);
-      const double share = (double)p_keep * (double)whole;
-      p_remaining = share < 1.0 ? 1ull : (unsigned long long)share;
-      crossing_bin<unsigned long long>(hist64, kBins, p_remaining, scan64, &found_bin, &found_above, low_bin, above);
-      p_remaining -= above;
-      p_prefix = (uint32_t)low_bin;
+    if (!ready) {
+      for (int i = tid; i < kBins; i += nt) {
+        hist32[i] = 0;
+        hist64[i] = 0;
+      }
+      __syncthreads();
+      for_row(row, V, [&](int, float logit) {
+        const float x = scaled(logit, inv_t);
+        const uint32_t bin = ordered(x) >> 20;
+        atomicAdd(&hist32[bin], 1u);
+        if (!k_on) atomicAdd(&hist64[bin], fixed_mass(x, mx));
+      });
+      __syncthreads();
     }
-    // the values in that bin and above it
-    uint32_t mine = 0, upto, total;
-    for (int i = tid; i < kBins; i += nt) mine += i >= low_bin ? hist32[i] : 0u;
-    block_scan<uint32_t>(mine, scan32, upto, total);
-    if (total <= (uint32_t)kCandidates) {
+    const FirstLevel level = first_level<kSampleThreads>(ready ? shared.hist32 + (size_t)r * kBins : hist32,
+                                                         ready ? shared.hist64 + (size_t)r * kBins : hist64, k_on, k, p_keep, scan64, &first);
+    const int low_bin = level.bin;
+    if (k_on) {
+      k_prefix = (uint32_t)low_bin;
+      k_remaining = level.k_remaining;
+    } else {
+      p_prefix = (uint32_t)low_bin;
+      p_remaining = level.p_remaining;
+    }
+    // the values in that bin and above it; listed: those that may be a threshold (see sample_collect)
+    const uint32_t total = level.total, entries = k_on && p_on ? level.total : level.inside;
+    if (ready && entries <= (uint32_t)kCandidates) {
+#pragma unroll 4
+      for (int i = tid; i < (int)entries; i += nt) {
+        cand[i] = shared.cand[(size_t)r * kCandidates + i];
+        cand_segment[i] = shared.segment[(size_t)r * kCandidates + i];
+      }
+      ncand = (int)entries;
+      listed = true;
+    } else if (total <= (uint32_t)kCandidates) {
       for_row(row, V, [&](int, float logit) {
         const uint32_t o = ordered(scaled(logit, inv_t));
         if ((int)(o >> 20) >= low_bin) cand[atomicAdd(&cand_count, 1u)] = o;  // (in any order: the sums below are of integers)
@@ -441,9 +644,48 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     }
   };
 
+  // Among a few values (those of the candidates that `belongs` names, at most kFew) the threshold by ranks: a value is kept
+  // iff what lies strictly above it, in numbers or in mass, is less than `target(whole)`; the least kept one.  False if
+  // they are more.  (A level of the radix search costs some 2 us whatever it looks at, and there are up to five.)
+  const auto among_few = [&](bool masses, auto belongs, auto target, uint32_t& found) {
+    if (ncand < 0) return false;
+    __syncthreads();      // (the search before this one has been read)
+    if (tid == 0) {
+      few_count = 0;
+      few_cut = 0xffffffffu;
+    }
+    __syncthreads();
+    for (int i = tid; i < ncand; i += nt) {
+      const uint32_t o = cand[i];
+      if (belongs(o)) {
+        const uint32_t at = atomicAdd(&few_count, 1u);
+        if (at < (uint32_t)kFew) {
+          few[at] = o;
+          few_mass[at] = masses ? fixed_mass(unordered(o), mx) : 1ull;
+        }
+      }
+    }
+    __syncthreads();
+    const int n = (int)few_count;
+    if (n > kFew || n == 0) return false;      // (every thread alike)
+    if (tid < n) {
+      const uint32_t mine = few[tid];
+      unsigned long long above = 0, whole = 0;
+      for (int i = 0; i < n; ++i) {
+        const unsigned long long m = few_mass[i];
+        whole += m;
+        above += few[i] > mine ? m : 0ull;
+      }
+      if (above < target(whole)) atomicMin(&few_cut, mine);
+    }
+    __syncthreads();
+    found = few_cut;
+    return true;
+  };
+
   // top-k: kth = the k-th largest scaled logit (everything >= it survives)
   uint32_t kth = 0;  // ordered(-inf) is > 0, so 0 keeps everything
-  if (k_on) {
+  if (k_on && !among_few(false, [&](uint32_t o) { return (o >> 20) == k_prefix; }, [&](unsigned long long) { return (unsigned long long)k_remaining; }, kth)) {
     uint32_t prefix = k_prefix, remaining = k_remaining;
     // (shift, bits): 20/12 (done above), 8/12, 0/8
     for (int level = 1; level < 3; ++level) {
@@ -468,7 +710,15 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   // top-p: keep x iff the mass of kept values strictly greater than x is < top_p of
   // the whole; the kept set is {x >= cut}
   uint32_t cut = kth;
-  if (p_on) {
+  const auto kept_share = [&](unsigned long long whole) {
+    const double share = (double)p_keep * (double)whole;
+    return share < 1.0 ? 1ull : (unsigned long long)share;
+  };
+  if (p_on && (k_on ? among_few(true, [&](uint32_t o) { return o >= kth; }, kept_share, cut)
+                    : among_few(true, [&](uint32_t o) { return (o >> 20) == p_prefix; }, [&](unsigned long long) { return p_remaining; }, cut))) {
+    cut = cut > kth ? cut : kth;
+  } else if (p_on) {
+    cut = kth;
     uint32_t prefix = p_prefix;
     unsigned long long remaining = p_remaining;
     for (int level = k_on ? 0 : 1; level < 3; ++level) {  // (without top-k the first pass was the first level)
@@ -486,8 +736,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
         unsigned long long mine = 0, upto, whole;
         for (int i = tid; i < kBins; i += nt) mine += hist64[i];
         block_scan<unsigned long long>(mine, scan64, upto, whole);
-        const double share = (double)p_keep * (double)whole;
-        remaining = share < 1.0 ? 1ull : (unsigned long long)share;
+        remaining = kept_share(whole);
       }
       int bin;
       unsigned long long above;
@@ -506,7 +755,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   const int lane = tid & (kWave - 1), wave = tid / kWave;
   constexpr int kWaves = kSampleThreads / kWave;
   static_assert(kWaves <= kArgmaxSegments, "fs holds either kind of chunk");
-  const bool by_segments = cut == 0 && seg_mass != nullptr;
+  // (With a list of candidates the chunks are those segments too: what is kept is in the list.)
+  const bool by_segments = listed || (cut == 0 && seg_mass != nullptr);
   const int nchunks = by_segments ? kArgmaxSegments : kWaves;
   const int chunk = by_segments ? (((V + kArgmaxSegments - 1) / kArgmaxSegments + 3) & ~3)
                                 : ((V + kWaves - 1) / kWaves + 4 * kWave - 1) / (4 * kWave) * (4 * kWave);
@@ -517,7 +767,16 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     return ordered(x) >= cut ? exp_unit(x - mx) : 0.f;
   };
   const int c_len = max(0, c_end - c_begin);
-  if (by_segments) {
+  if (listed) {
+    __syncthreads();
+    if (tid < kArgmaxSegments) segment_mass[tid] = k_on && p_on ? 0 : shared.above[r * kArgmaxSegments + tid];
+    __syncthreads();
+    for (int i = tid; i < ncand; i += nt)
+      if (cand[i] >= cut) atomicAdd(&segment_mass[cand_segment[i]], fixed_mass(unordered(cand[i]), mx));
+    __syncthreads();
+    if (tid < kArgmaxSegments) fs[tid] = (float)segment_mass[tid] * (1.f / 4294967296.f);
+    __syncthreads();
+  } else if (by_segments) {
     __syncthreads();
     if (tid < kArgmaxSegments) {
       const float m = seg_max[r * kArgmaxSegments + tid];
@@ -613,17 +872,51 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   }
 }
 
-// `out` must already hold each row's argmax and `row_max` its maximum (tk_argmax): greedy
-// rows keep the argmax, and so does a row whose search falls through (rounding at an edge).
-// seg_max, seg_mass (both or neither): what tk_argmax_masses left, [M][tk_argmax_segments()].
+constexpr int kSharedRows = 256;    // rows up to which a row with a threshold is shared between blocks (a block a CU from there on)
+constexpr size_t kSharedWords = 3 * kBins + 2;     // of a row: counts, masses, the list's length
+
+TK_API int tk_sample_scratch_bytes(int M) {
+  const long rows = M < 1 ? 0 : M;
+  const long parts = rows * kArgmaxSegments * 12 + rows * 4 + 16;
+  return (int)(parts + (rows <= kSharedRows ? rows * ((long)kSharedWords * 4 + (long)kCandidates * 5 + kArgmaxSegments * 8) : 0));
+}
+
+// Every row's next token: greedy rows (temperature 0) their argmax, the others a draw; a row whose search falls through
+// (rounding at an edge) keeps its argmax.  scratch: tk_sample_scratch_bytes(M), on a 16-byte border.
 TK_API int tk_sample(const float* logits, long ld, int M, int V, const float* temperature,
                      const int* top_k, const float* top_p, const unsigned long long* seeds,
-                     const unsigned long long* counters, const float* row_max, const float* seg_max,
-                     const float* seg_mass, int* out, float* probs_out, hipStream_t stream) {
+                     const unsigned long long* counters, int* out, float* probs_out, void* scratch, hipStream_t stream) {
   if (M <= 0) return 0;
-  if (V <= 0) return -1;
-  if (row_max == nullptr || (seg_max == nullptr) != (seg_mass == nullptr)) return -1;
+  if (V <= 0 || M > 65535 || scratch == nullptr || (uintptr_t)scratch % 16 != 0) return -1;
+  const bool share = M <= kSharedRows;
+  unsigned char* at = static_cast<unsigned char*>(scratch);
+  SharedRows sh{};
+  if (share) {      // (per row: 2 kBins words of masses, kBins of counts, two of the list's length)
+    sh.hist64 = reinterpret_cast<unsigned long long*>(at);
+    sh.hist32 = reinterpret_cast<uint32_t*>(at + (size_t)M * kBins * 8);
+    sh.count = sh.hist32 + (size_t)M * kBins;
+    sh.above = reinterpret_cast<unsigned long long*>(at + (size_t)M * kSharedWords * 4);
+    // (the words so far are cleared by the argmax pass; M times an odd number of 8 bytes: still on their border)
+    at += (size_t)M * (kSharedWords * 4 + kArgmaxSegments * 8);
+  }
+  float* seg_max = reinterpret_cast<float*>(at);
+  float* seg_mass = seg_max + (size_t)M * kArgmaxSegments;
+  int* seg_index = reinterpret_cast<int*>(seg_mass + (size_t)M * kArgmaxSegments);
+  float* row_max = reinterpret_cast<float*>(seg_index + (size_t)M * kArgmaxSegments);
+  if (share) {
+    sh.cand = reinterpret_cast<uint32_t*>(row_max + M);
+    sh.segment = reinterpret_cast<uint8_t*>(sh.cand + (size_t)M * kCandidates);
+  }
+  const dim3 shares(kArgmaxSegments, M);
+  argmax_segments_kernel<<<shares, kArgmaxThreads, 0, stream>>>(logits, seg_max, seg_index, V, ld, temperature, top_k, top_p, seg_mass,
+                                                                reinterpret_cast<uint32_t*>(sh.hist64), share ? kSharedWords : 0);
+  if (share) {
+    sample_hist_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, V, temperature, top_k, top_p, seg_max, seg_index, out, row_max, sh);
+    sample_collect_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, V, temperature, top_k, top_p, row_max, sh);
+  } else {
+    argmax_pick_kernel<<<M, kWave, 0, stream>>>(seg_max, seg_index, out, row_max);
+  }
   sample_kernel<<<M, kSampleThreads, 0, stream>>>(logits, ld, V, temperature, top_k, top_p, seeds, counters,
-                                                  row_max, seg_max, seg_mass, out, probs_out);
+                                                  row_max, seg_max, seg_mass, out, probs_out, sh);
   return launch_status();
 }
