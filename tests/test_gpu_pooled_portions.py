@@ -1,4 +1,4 @@
-"""The pooled-window attention of steps with prompt portions, on the matrix cores, against the
+"""The pooled-window attention on the matrix cores, against the
 design's equations in 64 bits on the same bfloat16 operands; and against the general form's error."""
 
 import math
@@ -35,6 +35,7 @@ CASES = {
     "window of 1": (16, 4, 64, 64, 1, 3, 16, [(2, 0), (33, 50), (1, 0)]),
     "two heads a kv head": (16, 8, 128, 64, 37, 5, 48, [(15, 201), (31, 0), (1, 90), (3, 47)]),
     "a kv head a head": (16, 16, 64, 128, 100, 7, 32, [(48, 95), (5, 700)]),
+    "single tokens": (32, 8, 128, 128, 256, 16, 16, [(1, 0), (1, 255), (1, 900), (1, 15), (1, 1200)]),
     "one kv head": (32, 1, 64, 64, 33, 1, 16, [(32, 31), (2, 255)]),
 }
 
@@ -82,7 +83,7 @@ def test_portions_on_the_matrix_cores(name, monkeypatch):
                                     dim=dim, vdim=vdim, window=window, pool=pool, page_size=page, scale=scale)
         return out.cpu().double()
 
-    assert ops.pooled_portions_pay(heads, kv, dim, vdim, page, batch.max_q_len)
+    assert ops.pooled_portions_pay(heads, kv, dim, vdim, page)
     got = run()
     # rounded once to bfloat16 (2^-9 of the result), weights kept to 2^-17: 3e-5 of the largest sum of products
     bound = 2.0 ** -8 * want.abs() + 1e-4 * float(want.abs().max())
@@ -91,3 +92,12 @@ def test_portions_on_the_matrix_cores(name, monkeypatch):
     general = run()
     # no further from the 64-bit result than the form with float32 weights (both are the final rounding away)
     assert float((got - want).norm()) <= 1.02 * float((general - want).norm())
+    # the step's own means: a mean of `pool` float32 sums in order, and nothing written beside the blocks it completes
+    fresh = [torch.full_like(t, nan) for t in arrays[2:]]
+    ops.pool_blocks(*arrays[:2], *fresh, batch.positions, batch.req_of_token, batch.block_tables[0], q.shape[0],
+                    k_width=kv * dim, v_width=kv * vdim, pool=pool, page_size=page)
+    complete = sum((n + cached) // pool - cached // pool for n, cached in spans)
+    for mean, known, width in zip(fresh, arrays[2:], (kv * dim, kv * vdim)):
+        written = ~mean.isnan()
+        assert int(written.sum()) == complete * width
+        assert bool(((mean - known)[written].abs() <= pool * 2.0 ** -23 * 8.0).all())      # (no input is beyond 8)

@@ -1,6 +1,6 @@
 // Attention over a sliding window plus pooled blocks behind it, with mixing of the heads'
 // softmax weights, on the matrix cores (gfx950; bfloat16 storage).  What is computed stands in
-// attention_pooled.hip; this is the form for steps that hold prompt portions.
+// attention_pooled.hip.
 //
 // What bounds the other form there: every raw score goes to memory, comes back to be normalised and mixed,
 // goes out and comes back again, eight rows share what a block loads, and the values are applied by the
@@ -39,6 +39,7 @@ union Frag {
 
 constexpr int kRows = 16;      // rows of a tile
 constexpr int kChunk = 32;     // entries of a chunk
+constexpr int kMaxShares = 16; // shares of a tile's entries
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLowest = -1e30f;   // a maximum of nothing (finite: differences of two stay numbers)
 
@@ -53,7 +54,7 @@ struct Args {
   const int* q_start;
   const int* tables;
   const float* talk;
-  uint32_t* weights;   // [tiles][Cmax][H][16 rows][32 entries], high half | low half of a mixed weight
+  uint32_t* weights;   // a tile's [Cmax][H][its rows][32 entries] at its first row's place: high half | low half of a mixed weight
   float* part_m;       // [tiles][H][16][S], in powers of two
   float* part_l;
   float* part_o;       // [S][N][H * vdim]
@@ -126,12 +127,12 @@ __device__ __forceinline__ void tile_scores(const Args& a, const Tile& t, int et
   for (int h = 0; h < 4; ++h) sc[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   if (et < 2 * t.PC) {
     const int b = min(et * 16 + (lane & 15), t.NB - 1);
-    const size_t per_page = (size_t)a.page_size * a.KE;
+    const unsigned per_page = (unsigned)a.page_size * a.KE;
 #pragma unroll
     for (int kv = 0; kv < KVQ; ++kv) {
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        const size_t flat = (size_t)b * KW + (kv0 + kv) * dim + 32 * s + 8 * g;     // (eight numbers lie in one page)
+        const unsigned flat = (unsigned)b * KW + (kv0 + kv) * dim + 32 * s + 8 * g;     // (eight numbers lie in one page)
         const float* p = a.k_pool + (size_t)t.table[flat / per_page] * per_page + flat % per_page;
         const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 4);
         Frag hi, mid, lo;
@@ -261,9 +262,24 @@ __global__ __launch_bounds__(16 * H) void portion_weights_kernel(Args a) {
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
     const size_t at = (((size_t)blockIdx.x * H + quad * 4 + h) * kRows + (lane & 15)) * a.S;
-    float top = kLowest, sum = 0.f;
-    for (int s = 0; s < a.S; ++s) top = fmaxf(top, a.part_m[at + s]);
-    for (int s = 0; s < a.S; ++s) sum += a.part_l[at + s] * __builtin_amdgcn_exp2f(a.part_m[at + s] - top);
+    // the four lanes of a row take a quarter of the shares each, all loads in flight (one after the other a
+    // step of single tokens, 16 shares, took 55 us; 20)
+    float pm[kMaxShares / 4], pl[kMaxShares / 4], top = kLowest, sum = 0.f;
+#pragma unroll
+    for (int x = 0; x < kMaxShares / 4; ++x) {
+      const int s = min(4 * x + (lane >> 4), a.S - 1);
+      pm[x] = a.part_m[at + s];
+      pl[x] = a.part_l[at + s];
+    }
+#pragma unroll
+    for (int x = 0; x < kMaxShares / 4; ++x) top = fmaxf(top, pm[x]);
+    top = fmaxf(top, __shfl_xor(top, 16, kWave));
+    top = fmaxf(top, __shfl_xor(top, 32, kWave));
+#pragma unroll
+    for (int x = 0; x < kMaxShares / 4; ++x)
+      if (4 * x + (lane >> 4) < a.S) sum += pl[x] * __builtin_amdgcn_exp2f(pm[x] - top);
+    sum += __shfl_xor(sum, 16, kWave);
+    sum += __shfl_xor(sum, 32, kWave);
     m[h] = top;
     il[h] = 1.f / sum;
   }
@@ -321,15 +337,15 @@ __global__ __launch_bounds__(16 * H) void portion_weights_kernel(Args a) {
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(th[s].v, bl.v, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(th[s].v, bh.v, acc, 0, 0, 0);
       }
-      uint32_t* out = a.weights + (((size_t)blockIdx.x * a.Cmax + c) * H * kRows + row) * kChunk + entry;
+      uint32_t* out = a.weights + ((size_t)t.row * a.Cmax * H + (size_t)c * H * t.tq + row) * kChunk + entry;
 #pragma unroll
       for (int x = 0; x < 16; x += 2) {
         const int h = 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3);
         if (H == 32 || x < 8) {
           uint32_t p0, p1;
           split2(acc[x], acc[x + 1], p0, p1);
-          out[(size_t)h * kRows * kChunk] = low_halves(p1, p0);
-          out[(size_t)(h + 1) * kRows * kChunk] = high_halves(p1, p0);
+          out[(size_t)h * t.tq * kChunk] = low_halves(p1, p0);
+          out[(size_t)(h + 1) * t.tq * kChunk] = high_halves(p1, p0);
         }
       }
     }
@@ -361,26 +377,29 @@ __global__ __launch_bounds__(256) void portion_values_kernel(Args a) {
     Frag wh[4], wl[4];
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
-      const uint32_t* p = a.weights + ((((size_t)blockIdx.x * a.Cmax + c) * a.H + quad * 4 + h) * kRows + min(n, t.tq - 1)) * kChunk + 8 * g;
+      const uint32_t* p = a.weights + ((size_t)t.row * a.Cmax * a.H + ((size_t)c * a.H + quad * 4 + h) * t.tq + min(n, t.tq - 1)) * kChunk + 8 * g;
       const u32x4_t x = *reinterpret_cast<const u32x4_t*>(p), y = *reinterpret_cast<const u32x4_t*>(p + 4);
       wh[h].u = u32x4_t{high_halves(x[0], x[1]), high_halves(x[2], x[3]), high_halves(y[0], y[1]), high_halves(y[2], y[3])};
       wl[h].u = u32x4_t{low_halves(x[0], x[1]), low_halves(x[2], x[3]), low_halves(y[0], y[1]), low_halves(y[2], y[3])};
     }
     if (c < t.PC) {
       const int b0 = c * kChunk + 8 * g;
-      const size_t per_page = (size_t)a.page_size * a.VE;
+      const unsigned per_page = (unsigned)a.page_size * a.VE;
 #pragma unroll
       for (int kv = 0; kv < KVQ; ++kv) {
+        const float* from[8];       // (VT numbers lie in one page)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const unsigned flat = (unsigned)max(0, min(b0 + e, t.NB - 1)) * VW + (kv0 + kv) * vdim + VT * n;
+          from[e] = a.v_pool + (size_t)t.table[flat / per_page] * per_page + flat % per_page;
+        }
 #pragma unroll
         for (int cc = 0; cc < VT; cc += 2) {
           float2 f[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            f[e] = make_float2(0.f, 0.f);
-            if (b0 + e < t.NB) {
-              const size_t flat = (size_t)(b0 + e) * VW + (kv0 + kv) * vdim + VT * n + cc;
-              f[e] = *reinterpret_cast<const float2*>(a.v_pool + (size_t)t.table[flat / per_page] * per_page + flat % per_page);
-            }
+            f[e] = *reinterpret_cast<const float2*>(from[e] + cc);
+            if (b0 + e >= t.NB) f[e] = make_float2(0.f, 0.f);
           }
 #pragma unroll
           for (int y = 0; y < 2; ++y) {
@@ -493,6 +512,7 @@ __global__ __launch_bounds__(256) void portion_merge_kernel(const float* __restr
   const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (at >= total) return;
   float4 sum = *reinterpret_cast<const float4*>(part_o + at);
+#pragma unroll 4
   for (int s = 1; s < S; ++s) {
     const float4 x = *reinterpret_cast<const float4*>(part_o + (size_t)s * total + at);
     sum.x += x.x;
@@ -523,8 +543,9 @@ TK_API int tk_pooled_window_portions(const void* q, const void* k_cache, const v
                                      int Cmax, int runs, float scale, hipStream_t stream) {
   if (N <= 0) return 0;
   if (R < 1 || (H != 16 && H != 32) || G < 1 || H % G || (dim != 64 && dim != 128) || (vdim != 64 && vdim != 128) ||
-      size < 1 || pool < 1 || page_size < 16 || page_size % 16 || tiles < 1 || S < 1 || Cmax < 1 || runs < 1 ||
-      (long)KE * pool < (long)G * dim || (long)VE * pool < (long)G * vdim)
+      size < 1 || pool < 1 || page_size < 16 || page_size % 16 || tiles < 1 || S < 1 || S > kMaxShares || Cmax < 1 || runs < 1 ||
+      (long)KE * pool < (long)G * dim || (long)VE * pool < (long)G * vdim ||
+      (long)table_width * page_size * max(KE, VE) > 0x7fffffffL)     // (places among a request's means in 32 bits)
     return -2;
   const int group = H / G, kvq = group >= 4 ? 1 : 4 / group;
   if (group > 2 && group % 4) return -2;

@@ -944,24 +944,28 @@ POOLED_CHUNK = 32
 POOLED_PORTION_BLOCKS = 512  # blocks of four waves wanted: two a CU
 
 
-def pooled_portions_pay(num_heads: int, num_kv_heads: int, dim: int, vdim: int, page_size: int, longest_span: int) -> bool:
+def pooled_portions_pay(num_heads: int, num_kv_heads: int, dim: int, vdim: int, page_size: int) -> bool:
     """Whether the pooled-window attention of a bfloat16 step runs on the matrix cores
-    (``attention_pooled_portions.hip``): a step with a portion, and sizes that its kernels are built for.
-    Single tokens fill a sixteenth of a tile and keep the form that walks a lane an entry."""
+    (``attention_pooled_portions.hip``): sizes that its kernels are built for.  Single tokens fill a sixteenth of a
+    tile and gain all the same: three of them over 3,100 positions, 32 / 8 heads of 128, a
+    layer's 82 us became 50 (scores, mixing and values on the vector unit before)."""
     group = num_heads // num_kv_heads
-    return (longest_span > 1 and num_heads in (16, 32) and (group in (1, 2) or group % 4 == 0) and dim in (64, 128)
+    return (num_heads in (16, 32) and (group in (1, 2) or group % 4 == 0) and dim in (64, 128)
             and vdim in (64, 128) and page_size % 16 == 0 and not POOLED_ONE_KERNEL_ONLY)
 
 
 def pooled_portions_plan(num_heads: int, window: int, pool: int, q_lens, longest_context: int) -> tuple[int, int, int, int]:
     """(tiles of 16 rows, shares of a tile's entries for the statistics and the values, most chunks of 32
-    entries a tile sees, runs of chunks for the weights).  A share or run holds at least four chunks."""
+    entries a tile sees, runs of chunks for the weights)."""
+    from tokamak_amd.kernels.attention import quarter_octave_at_least
+
+    # the length rounded as recorded steps round it: a step computes the same bits recorded or not
+    longest_context = quarter_octave_at_least(longest_context, 64)
     tiles = sum(-(-n // POOLED_TILE) for n in q_lens)
     means = -(-(longest_context // pool + 1) // POOLED_CHUNK)
     chunks = means + (min(longest_context - 1, window + 2 * POOLED_TILE - 3) + POOLED_CHUNK) // POOLED_CHUNK
-    most = max(1, chunks // 4)
-    shares = max(1, min(16, most, POOLED_PORTION_BLOCKS // (tiles * (num_heads // 4))))
-    runs = max(1, min(most, -(-2 * POOLED_PORTION_BLOCKS // tiles)))
+    shares = max(1, min(16, chunks // 2, POOLED_PORTION_BLOCKS // (tiles * (num_heads // 4))))
+    runs = max(1, min(chunks, -(-2 * POOLED_PORTION_BLOCKS // tiles)))
     return tiles, shares, chunks, runs
 
 
@@ -996,11 +1000,13 @@ def pooled_window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
         cached = sum(min(c + ql, window + ql - 1) * elem + (c + ql) // pool * 4 for c, ql in zip(batch.ctx_lens, batch.q_lens))
         _note(f"{n}x{num_heads}x{dim}", cached * num_kv_heads * (dim + vdim) + n * num_heads * (dim + vdim) * elem,
               2.0 * num_heads * (dim + vdim) * entries)
-    if dtype == torch.bfloat16 and pooled_portions_pay(num_heads, num_kv_heads, dim, vdim, page_size, batch.max_q_len) \
+    if dtype == torch.bfloat16 and pooled_portions_pay(num_heads, num_kv_heads, dim, vdim, page_size) \
+            and tables.shape[1] * page_size * max(ke, ve) < 2 ** 31 \
             and all(t.data_ptr() % 16 == 0 for t in (q, k_cache, v_cache, k_pool, v_pool, out)):
-        tiles, shares, chunks, runs = pooled_portions_plan(num_heads, window, pool, batch.q_lens, batch.max_seq_len)
+        tiles, shares, chunks, runs = pooled_portions_plan(num_heads, window, pool, batch.q_lens,
+                                                            batch.facts.get("context.max_len", batch.max_seq_len))
         dev = q.device
-        weights = torch.empty((tiles, chunks, num_heads, POOLED_TILE, POOLED_CHUNK), dtype=torch.int32, device=dev)
+        weights = torch.empty((n, chunks, num_heads, POOLED_CHUNK), dtype=torch.int32, device=dev)
         stats = torch.empty((2, tiles, num_heads, POOLED_TILE, shares), dtype=torch.float32, device=dev)
         part_o = torch.empty((shares, n, num_heads * vdim), dtype=torch.float32, device=dev) if shares > 1 else None
         _check(_fn("attention_pooled_portions", "tk_pooled_window_portions")(
