@@ -205,7 +205,7 @@ TK_API int tk_gemm_skinny(int out_dtype, const void* A, const void* W, void* C, 
 //   * every wave loads its 16 rows x 256 k (8 KB) with 16-byte loads in which 32
 //     consecutive lanes cover 512 contiguous bytes of one row, keeps them in
 //     registers while the previous chunk is computed, then parks them in its own
-//     LDS tile (row stride 264 elements: conflict-free 16-byte reads by row);
+//     LDS tile (pieces placed so that neither writes nor reads meet in a bank: lds_piece);
 //   * the block loads the activations' chunk [16*MT x 256] once into a shared
 //     LDS tile (they are small and sit in L2);
 //   * each wave then reads MFMA fragments back from LDS: lane (r, kb) takes
@@ -220,7 +220,13 @@ constexpr int SBK = 256;        // k per chunk
 // products (sched_group_barrier below).  With one row tile the plain loop is kept: the read-ahead
 // gains nothing there and cost the two-wave gated product of a 14B-shaped layer 8 % (63 -> 68 us).
 constexpr int READ_AHEAD_FROM = 2;
-constexpr int SLD = SBK + 8;    // LDS row stride in elements
+constexpr int SPC = SBK / 8;    // pieces of eight k of a row's chunk
+
+// Where piece c of row `row` of a tile of 16 rows lies in LDS, in pieces: [c][row ^ (c & 15)].  A loader's lanes write
+// neighbouring pieces of a row, an operand's lanes read one piece of 16 rows (and the next three pieces): either
+// way the pieces that LDS serves together lie in different banks, however it groups the lanes.  (Rows 264
+// elements apart instead: a third of the LDS cycles of the product of 64 rows were conflicts.)
+__device__ __forceinline__ int lds_piece(int c, int row) { return c * 16 + (row ^ (c & 15)); }
 
 // GATED: W is [2N, K], gate rows then up rows; the block owns 8*WAVES output columns, the
 // first half of its waves their gate rows and the second half the matching up rows, and
@@ -273,8 +279,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
   // i + 1 while others still read chunk i): 3-6 % for blocks of eight waves, which have a CU to
   // themselves anyway; nothing at up to 16 rows, and blocks of four would lose a place on the CU.
   constexpr int XBUF = (WAVES >= 6 && MT >= 2 && MT <= 4) ? 2 : 1;  // (five row tiles and more: one copy fits beside the weights)
-  __shared__ __attribute__((aligned(16))) bf16_t ws[WAVES][16][SLD];
-  __shared__ __attribute__((aligned(16))) bf16_t xs[XBUF][16 * MT][SLD];
+  __shared__ u32x4 ws[WAVES][SPC * 16];
+  __shared__ u32x4 xs[XBUF][MT][SPC * 16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, kb = lane >> 4;
   const int row_block = blockIdx.x, split = blockIdx.y;
@@ -342,12 +348,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
     const int xb_ = XBUF == 2 ? ((I_) & 1) : 0;                                                     \
     if (XBUF == 1) __syncthreads(); /* the previous chunk's fragments have been read */             \
     _Pragma("unroll") for (int i = 0; i < 8; ++i)                                                   \
-        *reinterpret_cast<u32x4*>(&ws[wave][2 * i + w_row0][w_col]) = wreg[i];                      \
+        ws[wave][lds_piece(lane & 31, 2 * i + w_row0)] = wreg[i];                                   \
     {                                                                                               \
       const bool inside_ = cur_ * SBK + x_col < K;                                                  \
       _Pragma("unroll") for (int i = 0; i < XP; ++i)                                                \
         if (XWHOLE || i * (THREADS / 32) + x_row0 < 16 * MT)                                        \
-          *reinterpret_cast<u32x4*>(&xs[xb_][i * (THREADS / 32) + x_row0][x_col]) = inside_ ? xreg[i] : zero; \
+          xs[xb_][(i * (THREADS / 32) + x_row0) / 16][lds_piece(tid & 31, (i * (THREADS / 32) + x_row0) & 15)] = inside_ ? xreg[i] : zero; \
     }                                                                                               \
     __syncthreads();                                                                                \
     if ((I_) + 1 < nchunks) {                                                                       \
@@ -358,9 +364,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
     if constexpr (MT < READ_AHEAD_FROM || MT > 4) { /* (more row tiles: no registers for two steps' fragments) */ \
       _Pragma("unroll") for (int s = 0; s < SBK / 32; ++s) {                                        \
         Frag8 wf, xf[MT];                                                                           \
-        wf.u = *reinterpret_cast<const uint4*>(&ws[wave][r][s * 32 + kb * 8]);                      \
+        wf.u = *reinterpret_cast<const uint4*>(&ws[wave][lds_piece(s * 4 + kb, r)]);                \
         _Pragma("unroll") for (int j = 0; j < MT; ++j)                                              \
-            xf[j].u = *reinterpret_cast<const uint4*>(&xs[xb_][j * 16 + r][s * 32 + kb * 8]);       \
+            xf[j].u = *reinterpret_cast<const uint4*>(&xs[xb_][j][lds_piece(s * 4 + kb, r)]);       \
         _Pragma("unroll") for (int j = 0; j < MT; ++j)                                              \
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf.v, xf[j].v, acc[j], 0, 0, 0);       \
       }                                                                                             \
@@ -369,9 +375,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
       /* wave that waits for each fragment in turn spends its time on round trips to LDS         */ \
       Frag8 wf[SBK / 32], xf[SBK / 32][MT];                                                         \
       _Pragma("unroll") for (int s = 0; s < SBK / 32; ++s) {                                        \
-        wf[s].u = *reinterpret_cast<const uint4*>(&ws[wave][r][s * 32 + kb * 8]);                   \
+        wf[s].u = *reinterpret_cast<const uint4*>(&ws[wave][lds_piece(s * 4 + kb, r)]);             \
         _Pragma("unroll") for (int j = 0; j < MT; ++j)                                              \
-            xf[s][j].u = *reinterpret_cast<const uint4*>(&xs[xb_][j * 16 + r][s * 32 + kb * 8]);    \
+            xf[s][j].u = *reinterpret_cast<const uint4*>(&xs[xb_][j][lds_piece(s * 4 + kb, r)]);    \
       }                                                                                             \
       _Pragma("unroll") for (int s = 0; s < SBK / 32; ++s)                                          \
         _Pragma("unroll") for (int j = 0; j < MT; ++j)                                              \
@@ -431,7 +437,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
   }
 
   if (GATED) {
-    float* up = reinterpret_cast<float*>(&ws[0][0][0]);  // [HALF up waves][MT][64 lanes][4]
+    float* up = reinterpret_cast<float*>(&ws[0][0]);  // [HALF up waves][MT][64 lanes][4]
     static_assert(sizeof(ws) >= sizeof(float) * HALF * MT * 64 * 4, "the exchange fits the weights' tiles");
     __syncthreads();                                      // the last chunk's fragments have been read
     if (wave >= HALF) {
