@@ -311,6 +311,10 @@ _SIGS = {
         "tk_fixed_decay_chunks": [c_int, c_void_p, c_int, c_int, c_long, c_long, c_void_p, c_void_p, c_void_p, c_void_p,
                                   c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p],
     },
+    "ssm_chunks": {
+        "tk_ssm_chunks": [c_void_p, c_void_p, c_int, c_int, c_long, c_long, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+                          c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
+    },
     "scan_chunks": {
         "tk_gla_chunks": [*[c_void_p, c_int, c_int, c_long] * 5, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                           c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_void_p],
@@ -1171,6 +1175,7 @@ SSM_SPLIT_FROM_TOKENS = 64   # a request's tokens in a step from which a head's 
 SSM_SPLIT_MIN_COLUMNS = 8
 SSM_SPLIT_BLOCKS = 1024
 SSM_CHUNK_TOKENS = 64        # tokens of a chunk of a long portion; the chunks of a portion run side by side
+SSM_MATRIX_CHUNKS_MAX_DIM = 128
 SSM_CHUNKS_FROM_TOKENS = 128  # a request's tokens in a step from which the step's portions are cut into chunks
 
 
@@ -1218,6 +1223,24 @@ def ssd_column_splits(requests: int, heads: int, vdim: int, longest: int) -> int
     return splits
 
 
+def _ssm_in_chunks(u: torch.Tensor, state_size: int, vdim: int, longest: int) -> bool:
+    """Whether the state-space scan runs in chunks of 64 tokens on the matrix cores: bfloat16 steps with a portion
+    that the general form would cut into chunks too (32 heads of 128 x 64: one portion of 128 tokens 182 us there, 35
+    here; eleven of 180, 349 and 159).  Shorter portions walk: of 64 tokens one took 90 us there and 33 here, but sixteen
+    79 and 98, since a chunk's state is written and read three times however few its tokens."""
+    return (u.dtype == torch.bfloat16 and longest >= SSM_CHUNKS_FROM_TOKENS
+            and state_size in (16, 32, 64, 128) and vdim % 16 == 0 and vdim <= SSM_MATRIX_CHUNKS_MAX_DIM and u.data_ptr() % 16 == 0)
+
+
+def ssm_chunk_heads(chunks: int, heads: int, groups: int) -> int:
+    """Heads of a group that a block takes one after the other: what B and C cost is shared by up to 4, as long as
+    two blocks a CU remain."""
+    per = 4
+    while per > 1 and (heads // groups % per or chunks * (heads // per) < 512):
+        per //= 2
+    return per
+
+
 def ssd_scan(u: torch.Tensor, proj: torch.Tensor, dt_col: int, dt_bias: torch.Tensor, a_log: torch.Tensor,
              skip: torch.Tensor, state: torch.Tensor, y: torch.Tensor, batch, *, heads: int, groups: int, state_size: int,
              vdim: int) -> None:
@@ -1237,6 +1260,17 @@ def ssd_scan(u: torch.Tensor, proj: torch.Tensor, dt_col: int, dt_bias: torch.Te
     _need(1 <= vdim <= 1024 and 1 <= state_size <= 1024 and batch.num_tokens == n, "the scan takes sizes up to 1,024")
     pointer, is_f32, parts, stride, ld = _ssm_in(proj, n, u.dtype, "projections")
     _need(0 <= dt_col and dt_col + heads <= ld, "the step sizes lie outside the projections")
+    if _ssm_in_chunks(u, state_size, vdim, batch.max_q_len):
+        chunks = sum(-(-t // SSM_CHUNK_TOKENS) for t in batch.q_lens)
+        per = ssm_chunk_heads(chunks, heads, groups)
+        chunk_state = torch.empty((chunks, heads, vdim // 4, state_size, 4), dtype=torch.float32, device=y.device)
+        chunk_decay = torch.empty((chunks, heads), dtype=torch.float32, device=y.device)
+        _note(f"{n}x{heads}x{state_size}x{vdim} chunks", n * (c * u.element_size() + heads * vdim * 4), 6.0 * n * heads * state_size * vdim)
+        _check(_fn("ssm_chunks", "tk_ssm_chunks")(
+            _p(u), pointer, is_f32, parts, stride, ld, int(dt_col), _p(dt_bias), _p(a_log), _p(skip), _p(state),
+            _p(batch.q_start), _p(batch.state_slots), _p(y), batch.num_requests, heads, groups, state_size, vdim, chunks, per,
+            _p(chunk_state), _p(chunk_decay), _stream()), "ssm_chunks")
+        return
     plan = _scan_chunks(batch, n, heads, state_size, vdim, y.device)
     _note(f"{n}x{heads}x{state_size}x{vdim}", n * (c * u.element_size() + heads * vdim * 4), 6.0 * n * heads * state_size * vdim)
     _check(_fn("ssm", "tk_ssd_scan")(_code(u.dtype), _p(u), pointer, is_f32, parts, stride, ld, int(dt_col), _p(dt_bias),
