@@ -208,60 +208,93 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
       }
 }
 
-// Few rows (M <= 16, float32): the tiles above leave most of a block idle.  Here a lane owns
-// one weight row and walks it with 16-byte loads, a cache line in eight loads one after the other; the activations are the same for every lane
-// (the compiler reads them through the scalar path).  The order of the sum is the one of the
-// tiled kernel, bit for bit: k ascending within a piece of kPiece, the pieces' sums added to the
-// total one after the other; so a row's result is still the same whatever the batch holds.
+// Few rows (M <= 16, float32): the tiles above leave most of a block idle.  Here a wave owns 64 weight rows, a lane one of
+// them, and walks them 32 k at a time; the activations are the same for every lane (the compiler reads them through
+// the scalar path).  The order of the sum is the one of the tiled kernel, bit for bit: k ascending within a piece of
+// kPiece, the pieces' sums added to the total one after the other; so a row's result is still the same whatever the batch holds.
 // With `partial` a wave sums one piece only and writes it to partial[piece][M][N]; the second
 // kernel adds the pieces in order (for matrices of too few rows to fill the GPU otherwise).
+//
+// Bound by the weights' bytes.  A tile of 64 rows by 32 k is loaded as whole cache lines (eight lanes a row's 128 bytes),
+// two tiles ahead, and changes hands through the wave's own LDS (rows 36 floats apart: sixteen lanes' pieces lie in
+// different banks).  Lanes that loaded from a row each touched 64 lines a load (4 rows:
+// weights of 4,096 x 2,048 19.8 us, now 13.1, both kernels; 12,288 x 2,048 27.2, 23.0; 151,936 x 2,048 257, 235, and 425, 248 for 8 rows).
+constexpr int kFewK = 32, kFewPitch = kFewK + 4;
 template <int MT>
 __global__ __launch_bounds__(64) void gemm_fewrows_kernel(const float* __restrict__ A,
                                                           const float* __restrict__ W,
                                                           float* __restrict__ C, float* __restrict__ partial,
                                                           int M, int N, int K, long lda, long ldw, long ldc) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  static_assert(kPiece % (2 * kFewK) == 0, "a piece is whole pairs of tiles");
+  __shared__ __attribute__((aligned(16))) float tile[64 * kFewPitch];
   const int lane = threadIdx.x;
-  const int n = blockIdx.x * 64 + lane;
-  const float* wrow = W + (size_t)min(n, N - 1) * ldw;
+  const int n0 = blockIdx.x * 64, n = n0 + lane;
   const int pieces = (K + kPiece - 1) / kPiece;
-  const int p_begin = partial ? blockIdx.y : 0;
-  const int p_end = partial ? p_begin + 1 : pieces;
-  float total[MT];
+  const int k_begin = (partial ? blockIdx.y : 0) * kPiece;
+  const int k_end = min(K, (partial ? (int)blockIdx.y + 1 : pieces) * kPiece);
+  // (rows past N are computed from a valid row and never stored; what lies past K is read at the row's end, not used)
+  const float* from[8];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) total[m] = 0.f;
-  for (int p = p_begin; p < p_end; ++p) {
-    float acc[MT];
+  for (int i = 0; i < 8; ++i) from[i] = W + (size_t)min(n0 + 8 * i + lane / 8, N - 1) * ldw;
+  const int col = lane % 8 * 4;
+  f32x4 reg[2][8];
+  const auto fetch = [&](f32x4 (&r)[8], int k0) {
+    const int k = min(k0 + col, K - 4);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = 0.f;
-    const int k_end = min(K, (p + 1) * kPiece);
-#pragma unroll 8
-    for (int k = p * kPiece; k < k_end; k += 4) {
-      const float4 w = *reinterpret_cast<const float4*>(wrow + k);
+    for (int i = 0; i < 8; ++i) r[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(from[i] + k));
+  };
+  float acc[MT], total[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) acc[m] = total[m] = 0.f;
+  const auto step = [&](int k, int at) {
+    const f32x4 w = *reinterpret_cast<const f32x4*>(tile + lane * kFewPitch + at);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const float4 a = *reinterpret_cast<const float4*>(A + (size_t)min(m, M - 1) * lda + k);
+      acc[m] = fmaf(a.x, w[0], acc[m]);
+      acc[m] = fmaf(a.y, w[1], acc[m]);
+      acc[m] = fmaf(a.z, w[2], acc[m]);
+      acc[m] = fmaf(a.w, w[3], acc[m]);
+    }
+  };
+  fetch(reg[0], k_begin);
+  if (k_begin + kFewK < k_end) fetch(reg[1], k_begin + kFewK);
+  for (int k0 = k_begin; k0 < k_end; k0 += 2 * kFewK) {
+    if (k0 > k_begin && k0 % kPiece == 0) {
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
-        const float4 a = *reinterpret_cast<const float4*>(A + (size_t)min(m, M - 1) * lda + k);
-        acc[m] = fmaf(a.x, w.x, acc[m]);
-        acc[m] = fmaf(a.y, w.y, acc[m]);
-        acc[m] = fmaf(a.z, w.z, acc[m]);
-        acc[m] = fmaf(a.w, w.w, acc[m]);
+        total[m] += acc[m];
+        acc[m] = 0.f;
       }
     }
-    if (partial) {
-      if (n < N) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-          if (m < M) partial[((size_t)p * M + m) * N + n] = acc[m];
+    for (int u = 0; u < 2; ++u) {
+      const int k = k0 + u * kFewK;
+      if (k >= k_end) break;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(tile + (8 * i + lane / 8) * kFewPitch + col) = reg[u][i];
+      if (k + 2 * kFewK < k_end) fetch(reg[u], k + 2 * kFewK);
+      wave_lds_sync();
+      if (k + kFewK <= k_end) {
+#pragma unroll
+        for (int at = 0; at < kFewK; at += 4) step(k + at, at);
+      } else {
+        for (int at = 0; k + at < k_end; at += 4) step(k + at, at);
       }
-      return;
+      wave_lds_sync();
     }
-#pragma unroll
-    for (int m = 0; m < MT; ++m) total[m] += acc[m];
   }
-  if (n < N) {
+  if (n >= N) return;
+  if (partial) {
 #pragma unroll
     for (int m = 0; m < MT; ++m)
-      if (m < M) C[(size_t)m * ldc + n] = total[m];
+      if (m < M) partial[((size_t)blockIdx.y * M + m) * N + n] = acc[m];
+    return;
   }
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+    if (m < M) C[(size_t)m * ldc + n] = total[m] + acc[m];
 }
 
 __global__ __launch_bounds__(256) void gemm_fewrows_add_kernel(const float* __restrict__ partial,
