@@ -11,7 +11,7 @@
 
 using namespace tk;
 
-constexpr int BK = 16, PAD = 4;
+constexpr int BK = 16, PAD = 4;   // of gemm_tiled_kernel
 constexpr int kPiece = 256;  // k values summed before they join the total (a multiple of BK)
 
 // A block of 256 threads owns 64H x 64H outputs (H = 1 or 2); thread (ty, tx) of 16 x 16 owns
@@ -104,8 +104,12 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const TI* __restrict__ 
 // step equal), so a walk over k in steps of two is the chain of the kernels above and below,
 // bit for bit, and the pieces of kPiece are kept as they are.  A block of four waves owns
 // 64H x 64H outputs, a wave 32H x 32H of them (H x H tiles of 32 x 32, each 16 accumulators a
-// lane and as many for the total).  The tiles of A and W lie in LDS k-major as above; a lane's
-// operand of a step is one float: A[row lane % 32][k + lane / 32].
+// lane and as many for the total).  A lane's operand of a step is one float, A[row lane % 32][k + lane / 32]: a row of
+// a stage lies in LDS as its even k, then its odd k, so that one 16-byte read is four steps' operand.
+// A wave's step is 64 cycles a pair of tiles, so a stage of 16 k of 64 x 64 outputs was over long before the next one's loads
+// had come (47 TFLOP/s): stages hold 64 k there and 32 k of 128 x 128, two of them in LDS (one barrier a stage),
+// loaded without a branch (1,000 rows: weights of 2,048 x 6,144 413 -> 267 us, 2,048 x 2,048 141 -> 92, 12,288 x 2,048 497 -> 439;
+// 130 rows: 321 -> 153, 98 -> 55, 178 -> 143).
 typedef float float16v __attribute__((ext_vector_type(16)));
 
 template <typename TO, int H>
@@ -113,17 +117,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
                                                               const float* __restrict__ W,
                                                               TO* __restrict__ C, int M, int N, int K,
                                                               long lda, long ldw, long ldc) {
-  constexpr int BM = 64 * H, BN = 64 * H;
-  __shared__ __attribute__((aligned(16))) float As[BK][BM + PAD];
-  __shared__ __attribute__((aligned(16))) float Ws[BK][BN + PAD];
+  typedef float float4v __attribute__((ext_vector_type(4)));
+  constexpr int BM = 64 * H, BN = 64 * H, SK = H == 1 ? 64 : 32, PITCH = SK + 4;
+  constexpr int LANES = SK / 4, ROWS = 256 / LANES, PASSES = BM / ROWS;   // the loader: lanes a row, rows a pass
+  static_assert(kPiece % SK == 0, "a piece is whole stages");
+  __shared__ __attribute__((aligned(16))) float As[2][BM][PITCH];
+  __shared__ __attribute__((aligned(16))) float Ws[2][BN][PITCH];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, g = lane >> 5;
   const int wm = (wave & 1) * 32 * H, wn = (wave >> 1) * 32 * H;   // this wave's corner of the block's tile
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int lrow = tid / 4, lk = (tid % 4) * 4;   // loader: rows lrow (and lrow + 64), four k from lk
-  // rows whose four k are one aligned 16-byte piece are loaded as one
-  const bool a_wide = lda % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0;
-  const bool w_wide = ldw % 4 == 0 && reinterpret_cast<uintptr_t>(W) % 16 == 0;
+  const int lrow = tid / LANES, lk = (tid % LANES) * 4;
+  // rows whose four k are one aligned 16-byte piece are loaded as one; rows past the end are read at the last row and
+  // never stored, what lies past K is read at the row's end and becomes zero
+  const bool wide = K % 4 == 0 && K >= 4 && lda % 4 == 0 && ldw % 4 == 0 &&
+                    (reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) % 16 == 0;
 
   float16v acc[H][H], total[H][H];
 #pragma unroll
@@ -133,30 +141,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = total[i][j][e] = 0.f;
 
-  float ar[H][4], wr[H][4];
+  float4v ar[PASSES], wr[PASSES];
   auto fetch = [&](int k0) {
     const int k = k0 + lk;
+    if (wide) {
 #pragma unroll
-    for (int h = 0; h < H; ++h) {
-      const int m = m0 + lrow + 64 * h, n = n0 + lrow + 64 * h;
-      if (a_wide && m < M && k + 3 < K) {
-        const float4 v = *reinterpret_cast<const float4*>(A + (size_t)m * lda + k);
-        ar[h][0] = v.x; ar[h][1] = v.y; ar[h][2] = v.z; ar[h][3] = v.w;
-      } else {
+      for (int h = 0; h < PASSES; ++h) {
+        ar[h] = *reinterpret_cast<const float4v*>(A + (size_t)min(m0 + lrow + ROWS * h, M - 1) * lda + min(k, K - 4));
+        wr[h] = *reinterpret_cast<const float4v*>(W + (size_t)min(n0 + lrow + ROWS * h, N - 1) * ldw + min(k, K - 4));
+      }
+    } else {
+#pragma unroll
+      for (int h = 0; h < PASSES; ++h) {
+        const int m = m0 + lrow + ROWS * h, n = n0 + lrow + ROWS * h;
 #pragma unroll
         for (int i = 0; i < 4; ++i) ar[h][i] = (m < M && k + i < K) ? A[(size_t)m * lda + k + i] : 0.f;
-      }
-      if (w_wide && n < N && k + 3 < K) {
-        const float4 v = *reinterpret_cast<const float4*>(W + (size_t)n * ldw + k);
-        wr[h][0] = v.x; wr[h][1] = v.y; wr[h][2] = v.z; wr[h][3] = v.w;
-      } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) wr[h][i] = (n < N && k + i < K) ? W[(size_t)n * ldw + k + i] : 0.f;
       }
     }
   };
   fetch(0);
-  for (int k0 = 0; k0 < K; k0 += BK) {
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += SK, buf ^= 1) {
     if (k0 > 0 && k0 % kPiece == 0) {
 #pragma unroll
       for (int i = 0; i < H; ++i)
@@ -167,29 +174,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
           for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
         }
     }
+    const bool inside = k0 + lk < K;       // (K a multiple of four, or `fetch` has made the zeros)
 #pragma unroll
-    for (int h = 0; h < H; ++h)
+    for (int h = 0; h < PASSES; ++h) {
+      const float4v a = inside ? ar[h] : float4v{0.f, 0.f, 0.f, 0.f}, w = inside ? wr[h] : float4v{0.f, 0.f, 0.f, 0.f};
+      float* const ap = &As[buf][lrow + ROWS * h][lk / 2];
+      float* const wp = &Ws[buf][lrow + ROWS * h][lk / 2];
+      *reinterpret_cast<float2*>(ap) = make_float2(a[0], a[2]);
+      *reinterpret_cast<float2*>(ap + SK / 2) = make_float2(a[1], a[3]);
+      *reinterpret_cast<float2*>(wp) = make_float2(w[0], w[2]);
+      *reinterpret_cast<float2*>(wp + SK / 2) = make_float2(w[1], w[3]);
+    }
+    __syncthreads();      // (one a stage: this copy is written again behind the next stage's barrier)
+    if (k0 + SK < K) fetch(k0 + SK);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        As[lk + i][lrow + 64 * h] = ar[h][i];
-        Ws[lk + i][lrow + 64 * h] = wr[h][i];
-      }
-    __syncthreads();
-    if (k0 + BK < K) fetch(k0 + BK);
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 2) {
-      float a[H], w[H];
+    for (int kk = 0; kk < SK; kk += 8) {
+      float4v a[H], w[H];
 #pragma unroll
       for (int h = 0; h < H; ++h) {
-        a[h] = As[kk + g][wm + 32 * h + r];
-        w[h] = Ws[kk + g][wn + 32 * h + r];
+        a[h] = *reinterpret_cast<const float4v*>(&As[buf][wm + 32 * h + r][g * (SK / 2) + kk / 2]);
+        w[h] = *reinterpret_cast<const float4v*>(&Ws[buf][wn + 32 * h + r][g * (SK / 2) + kk / 2]);
       }
 #pragma unroll
-      for (int i = 0; i < H; ++i)
+      for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int j = 0; j < H; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], w[j], acc[i][j], 0, 0, 0);
+        for (int i = 0; i < H; ++i)
+#pragma unroll
+          for (int j = 0; j < H; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][s], w[j][s], acc[i][j], 0, 0, 0);
     }
-    __syncthreads();
   }
   // acc[i][j][4 q + e] = C[m0 + wm + 32 i + 8 q + 4 g + e][n0 + wn + 32 j + r]
 #pragma unroll
