@@ -63,6 +63,8 @@ __device__ __forceinline__ void load_eight(const bf16_t* p, float (&v)[8]) {
 // is a chain of memory round trips; few where eight queries share the key and the
 // multiply-adds fill the time (and the registers)
 template <int QT> constexpr int key_pieces() { return QT == 1 ? 8 : QT <= 4 ? 4 : 2; }
+// pieces of four values a lane asks for together
+template <int QT> constexpr int value_pieces() { return QT == 1 ? 8 : 4; }
 
 struct GenericItems {
   const int* single;      // token rows that run alone (null: every token of the step does)
@@ -223,20 +225,21 @@ __global__ __launch_bounds__(kWaves * kWave) void paged_attention_generic_kernel
 #pragma unroll
         for (int t = 0; t < QT; ++t) a[t] = acc[i][t] * alpha[t];
         if constexpr (BATCHED) {
-          // four keys a load (16 bytes of float32) and four such loads asked for together, added
+          // four keys a load (16 bytes of float32) and four such loads, for a query alone eight, asked for together, added
           // key by key in ascending order: the same sums as one key at a time.  A key out of
           // range adds a probability times 0.
-          for (int quad0 = 0; quad0 * 4 < count; quad0 += 4) {
-            float v4[4][4];
-            bool there[4];
+          constexpr int kPieces = value_pieces<QT>();
+          for (int quad0 = 0; quad0 * 4 < count; quad0 += kPieces) {
+            float v4[kPieces][4];
+            bool there[kPieces];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < kPieces; ++u) {
               const long b = base_s[wave][quad0 + u];
               there[u] = (quad0 + u) * 4 < count && b >= 0;
               load_four(v_cache + (there[u] ? b : 0) + v_dim_off, v4[u]);   // (absent: the cache's first page, not used)
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < kPieces; ++u) {
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
                 const int key = (quad0 + u) * 4 + e;
