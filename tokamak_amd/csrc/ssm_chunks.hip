@@ -17,7 +17,8 @@
 //
 // Walked a token at a time (four state rows by four columns a thread, twice over in chunks) this was bound by
 // the LDS reads of B and C, two 16-byte reads a token for 32 multiply-adds: 2,048 tokens of 32
-// heads of 128 x 64, one group, 273 us, 84 here; of 128 heads in 8 groups 920, 255 here.  B and C belong to a group of heads: a block takes a few heads of a group and forms C B^T, and reads its operands of B and C, once for them.
+// heads of 128 x 64, one group, 273 us, 84 here; of 128 heads in 8 groups 920, 255 here.  B and C belong to a group of
+// heads: a block takes a few heads of a group and forms C B^T, and reads its operands of B and C, once for them.
 #include "common.h"
 #include "request_tiles.h"
 #include "short_conv.h"
