@@ -40,14 +40,18 @@ CASES = {
 }
 
 
-@pytest.mark.parametrize("name", list(CASES))
-def test_portions_on_the_matrix_cores(name, monkeypatch):
+def step(name, opposite=False):
+    """A case's step: what computes it, the result in 64 bits, the batch, the arrays on the GPU.  ``opposite``:
+    every second head is the one before it but for a few of its numbers' last bits, and the mixing takes their difference."""
     from tokamak_amd.kernels import ops
 
     heads, kv, dim, vdim, window, pool, page, spans = CASES[name]
     g = torch.Generator().manual_seed(len(name))
     scale, ke, ve = dim ** -0.5, -(-kv * dim // pool), -(-kv * vdim // pool)
     talk = torch.eye(heads) + 0.3 * torch.randn(heads, heads, generator=g)
+    if opposite:
+        talk = torch.eye(heads).view(heads // 2, 2, heads).clone()
+        talk = (talk - talk.flip(1)).view(heads, heads)
     total = sum(-(-(n + c) // page) for n, c in spans)
     order = torch.randperm(total + 3, generator=g).tolist()
     nan = float("nan")
@@ -61,6 +65,11 @@ def test_portions_on_the_matrix_cores(name, monkeypatch):
         k = (1.5 * torch.randn(length, kv, dim, generator=g)).bfloat16().double()
         v = torch.randn(length, kv, vdim, generator=g).bfloat16().double()
         q = torch.randn(n, heads, dim, generator=g).bfloat16()
+        if opposite:
+            q = (0.25 * q).unflatten(1, (heads // 2, 2))
+            q[:, :, 1] = q[:, :, 0]
+            q[:, :, 1, :4] *= 1.0 + 2.0 ** -7
+            q = q.flatten(1, 2)
         for p in range(length):
             at = p % page
             k_cache[table[p // page], at * kv * dim:(at + 1) * kv * dim] = k[p].flatten().float()
@@ -75,7 +84,7 @@ def test_portions_on_the_matrix_cores(name, monkeypatch):
         rows.append((n, cached, table))
     batch = make_batch(rows)
     arrays = [t.to(DEV) for t in (k_cache.bfloat16(), v_cache.bfloat16(), k_pool, v_pool)]
-    q, want = torch.cat(queries).to(DEV), torch.cat(want)
+    q = torch.cat(queries).to(DEV)
 
     def run():
         out = torch.full((q.shape[0], heads * vdim), nan, dtype=torch.bfloat16, device=DEV)
@@ -84,8 +93,28 @@ def test_portions_on_the_matrix_cores(name, monkeypatch):
         return out.cpu().double()
 
     assert ops.pooled_portions_pay(heads, kv, dim, vdim, page)
+    return run, torch.cat(want), batch, arrays
+
+
+@pytest.mark.parametrize("name", ["long", "window of 1", "two heads a kv head", "single tokens"])
+def test_heads_mixed_with_opposite_signs(name):
+    """What two nearly equal heads' weights differ by is a small part of them: it is there only if the weights, the mixing and
+    the mixed weights keep float32's bits (of 16 of them, in two bfloat16 pieces, the result would be 2^-7 off)."""
+    run, want, _, _ = step(name, opposite=True)
+    # the final rounding, at most 2^-9 of a result, and half as much for the float32 scores
+    off = float((run() - want).norm() / want.norm())
+    assert off <= 2.0 ** -9 + 2.0 ** -10, off
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_portions_on_the_matrix_cores(name, monkeypatch):
+    from tokamak_amd.kernels import ops
+
+    heads, kv, dim, vdim, window, pool, page, spans = CASES[name]
+    run, want, batch, arrays = step(name)
+    nan, tokens = float("nan"), want.shape[0]
     got = run()
-    # rounded once to bfloat16 (2^-9 of the result), weights kept to 2^-17: 3e-5 of the largest sum of products
+    # rounded once to bfloat16 (2^-9 of the result), and 1e-4 of the largest sum of products where products cancel
     bound = 2.0 ** -8 * want.abs() + 1e-4 * float(want.abs().max())
     assert bool(((got - want).abs() <= bound).all()), float(((got - want).abs() - bound).max())
     monkeypatch.setattr(ops, "pooled_portions_pay", lambda *a: False)
@@ -94,7 +123,7 @@ def test_portions_on_the_matrix_cores(name, monkeypatch):
     assert float((got - want).norm()) <= 1.02 * float((general - want).norm())
     # the step's own means: a mean of `pool` float32 sums in order, and nothing written beside the blocks it completes
     fresh = [torch.full_like(t, nan) for t in arrays[2:]]
-    ops.pool_blocks(*arrays[:2], *fresh, batch.positions, batch.req_of_token, batch.block_tables[0], q.shape[0],
+    ops.pool_blocks(*arrays[:2], *fresh, batch.positions, batch.req_of_token, batch.block_tables[0], tokens,
                     k_width=kv * dim, v_width=kv * vdim, pool=pool, page_size=page)
     complete = sum((n + cached) // pool - cached // pool for n, cached in spans)
     for mean, known, width in zip(fresh, arrays[2:], (kv * dim, kv * vdim)):

@@ -5,16 +5,17 @@
 // What bounds the other form there: every raw score goes to memory, comes back to be normalised and mixed,
 // goes out and comes back again, eight rows share what a block loads, and the values are applied by the
 // vector unit (2,048 rows over 1,024 keys and up to 130 blocks, 32 / 8 heads of 128: 0.65 ms of
-// scores, 0.5 of mixing, 1.2 of values; the three kernels here together 0.35).  The mixing needs every head's
+// scores, 0.5 of mixing, 1.2 of values; the three kernels here together 0.40).  The mixing needs every head's
 // NORMALISED weight of an entry, so a single walk with a running maximum cannot do it; but scores are cheap
 // on the matrix cores, so they are formed twice instead of being kept:
 //   stats:    per (16 rows of one request, four heads, share of the entries) the maximum and the sum of exponentials;
 //   weights:  per (16 rows, run of entries) the scores of ALL heads again, their normalised weights, and the
 //             mixed ones, sum_g talk[h, g] w_g, as a matrix product over the heads;
 //   values:   per (16 rows, four heads, share of the entries) the product of mixed weights and values.
-// Weights and the mixing matrix are float32 and stay so: each is split into a bfloat16 and a bfloat16 of what
-// is left (16 bits of mantissa; products of two splits drop only low x low), the block means, float32 as
-// well, into three (24 bits).  Sums are float32.  The mixed weights leave as such a pair in one 32-bit word.
+// Weights, the mixing matrix and the block means are float32 and stay so: as operands each is split into three
+// bfloat16, a piece of what the pieces before it leave (24 bits of mantissa; of two splits the products below 2^-24 of
+// the largest are dropped).  Sums are float32, and so are the mixed weights in memory.  (Two pieces, 16 bits, and a
+// mixed weight as such a pair hid behind the bfloat16 output, but not where heads are mixed with opposite signs.)
 //
 // Entries: a row sees tokens (tiles of 16 that begin at a multiple of 16, so that a tile lies in one page:
 // pages of a multiple of 16) and block means (tiles of 16, padded to chunks of 32); a chunk is
@@ -54,7 +55,7 @@ struct Args {
   const int* q_start;
   const int* tables;
   const float* talk;
-  uint32_t* weights;   // a tile's [Cmax][H][its rows][32 entries] at its first row's place: high half | low half of a mixed weight
+  float* weights;      // mixed: a tile's [Cmax][H][its rows][32 entries] at its first row's place
   float* part_m;       // [tiles][H][16][S], in powers of two
   float* part_l;
   float* part_o;       // [S][N][H * vdim]
@@ -85,15 +86,21 @@ __device__ __forceinline__ bool find_tile(const Args& a, int at, Tile& t) {
 }
 
 // a float's leading bfloat16 pieces: two numbers at a time, each piece packed
-__device__ __forceinline__ void split2(float x, float y, uint32_t& hi, uint32_t& lo) {
-  hi = pack_bf16x2(x, y);
-  lo = pack_bf16x2(x - __uint_as_float(hi << 16), y - __uint_as_float(hi & 0xffff0000u));
-}
 __device__ __forceinline__ void split3(float x, float y, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
   hi = pack_bf16x2(x, y);
   const float x1 = x - __uint_as_float(hi << 16), y1 = y - __uint_as_float(hi & 0xffff0000u);
   mid = pack_bf16x2(x1, y1);
   lo = pack_bf16x2(x1 - __uint_as_float(mid << 16), y1 - __uint_as_float(mid & 0xffff0000u));
+}
+__device__ __forceinline__ void split_eight(const float (&f)[8], Frag& hi, Frag& mid, Frag& lo) {
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    uint32_t h0, m0, l0;
+    split3(f[2 * x], f[2 * x + 1], h0, m0, l0);
+    hi.u[x] = h0;
+    mid.u[x] = m0;
+    lo.u[x] = l0;
+  }
 }
 // (low halves, high halves) of two words
 __device__ __forceinline__ uint32_t low_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
@@ -101,6 +108,10 @@ __device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) { return
 
 __device__ __forceinline__ f32x4_t mfma16(const Frag& a, const Frag& b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x16_t mfma32(const Frag& a, const Frag& b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, b.v, c, 0, 0, 0);
 }
 
 // The queries of four heads as the second operand: lane (row = lane & 15, k group = lane >> 4).
@@ -184,7 +195,7 @@ __device__ __forceinline__ void tile_scores(const Args& a, const Tile& t, int et
 }
 
 // Four waves take a share's tiles of 16 entries in turn.  A key tile is read once for four heads and sixteen rows.
-// Bound by the vector unit (an exponential, a mask and a maximum a score): 0.1 ms at 2,048 rows of 32 / 8 heads of 128.
+// Bound by the vector unit (an exponential, a mask and a maximum a score): 82 us at 2,048 rows of 32 / 8 heads of 128.
 template <int KS, int KVQ>
 __global__ __launch_bounds__(256) void portion_stats_kernel(Args a) {
   __shared__ float red[4][4][kRows][2];
@@ -241,16 +252,19 @@ __global__ __launch_bounds__(256) void portion_stats_kernel(Args a) {
   }
 }
 
-// H / 4 waves, a wave four heads.  A chunk: every wave's normalised weights of 16 rows by 32 entries, split in two
-// bfloat16 pieces, into LDS [row][entry][head] (two copies, one barrier a chunk), then a wave mixes whole rows: D =
-// talk (32 heads by H) times the row's weights (H by 32 entries).  114 us for 2,048 rows of 32 heads of 128 over up to
-// 1,170 entries: the vector unit again (exponential, split and packing of every weight), then 300 MB of weights written.
+// H / 4 waves, a wave four heads.  A chunk: every wave's normalised weights of 16 rows by 32 entries, float32, into LDS
+// [row][entry][head] (two copies, one barrier a chunk), then a wave mixes whole rows: D = talk (32 heads by H) times
+// the row's weights (H by 32 entries), whose pieces are split as they are read.  153 us for 2,048 rows of 32 heads of
+// 128 over 1,024 tokens and up to 130 blocks (147 with two pieces a weight): an exponential, a split and a packing of
+// every weight, then 300 MB of weights written.
 template <int KS, int KVQ, int H>
 __global__ __launch_bounds__(16 * H) void portion_weights_kernel(Args a) {
   constexpr int kWaves = H / 4, kMix = H / 16;
-  constexpr int kRowBytes = kChunk * H * 2 + 16;     // (a row's start moved by four banks: the 16 rows' writes spread)
-  constexpr int kCopy = kRows * kRowBytes;
-  __shared__ __align__(16) unsigned char lds[2][2][kCopy];   // [copy][piece]
+  constexpr int kPitch = kChunk * H + 4;     // (a row's start moved by four banks: the 16 rows' writes spread)
+  // pieces of 16 bytes (four heads) swizzled by the entry: the reads walk entries 4 H bytes apart, and sixteen of them
+  // meet all banks
+  constexpr int kPieces = H / 4, kSwizzle = H == 32 ? 1 : 2;
+  __shared__ __align__(16) float lds[2][kRows * kPitch];
   Tile t;
   if (!find_tile(a, blockIdx.x, t)) return;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, quad = wave;
@@ -284,21 +298,17 @@ __global__ __launch_bounds__(16 * H) void portion_weights_kernel(Args a) {
     il[h] = 1.f / sum;
   }
   // the mixing matrix as the first operand: lane (head = lane & 31, heads 16 s + 8 (lane >> 5) .. + 8)
-  Frag th[kMix], tl[kMix];
+  Frag th[kMix], tm[kMix], tl[kMix];
 #pragma unroll
-  for (int s = 0; s < kMix; ++s)
+  for (int s = 0; s < kMix; ++s) {
+    const int to = lane & 31, from = 16 * s + 8 * (lane >> 5);
+    float f[8];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int to = lane & 31, from = 16 * s + 8 * (lane >> 5) + 2 * x;
-      const float u = to < H ? a.talk[to * H + from] : 0.f, v = to < H ? a.talk[to * H + from + 1] : 0.f;
-      uint32_t p0, p1;
-      split2(u, v, p0, p1);
-      th[s].u[x] = p0;
-      tl[s].u[x] = p1;
-    }
+    for (int x = 0; x < 8; ++x) f[x] = to < H ? a.talk[to * H + from + x] : 0.f;
+    split_eight(f, th[s], tm[s], tl[s]);
+  }
   for (int c = lo; c < hi; ++c) {
-    unsigned char* const ph = lds[c & 1][0];
-    unsigned char* const pl = lds[c & 1][1];
+    float* const copy = lds[c & 1];
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       f32x4_t sc[4];
@@ -308,15 +318,8 @@ __global__ __launch_bounds__(16 * H) void portion_weights_kernel(Args a) {
         float w[4];
 #pragma unroll
         for (int h = 0; h < 4; ++h) w[h] = __builtin_amdgcn_exp2f(sc[h][i] - m[h]) * il[h];
-        uint32_t h0, h1, l0, l1;
-        split2(w[0], w[1], h0, l0);
-        split2(w[2], w[3], h1, l1);
-        const int entry = 16 * half + 4 * (lane >> 4) + i;
-        // pieces of 16 bytes (eight heads) swizzled by the entry: the reads below walk entries 64 bytes apart
-        const int piece = H == 32 ? ((quad >> 1) ^ ((entry >> 2) & 3)) : ((quad >> 1) ^ ((entry >> 3) & 1));
-        const int at = (lane & 15) * kRowBytes + entry * (2 * H) + piece * 16 + (quad & 1) * 8;
-        *reinterpret_cast<uint2*>(ph + at) = make_uint2(h0, h1);
-        *reinterpret_cast<uint2*>(pl + at) = make_uint2(l0, l1);
+        const int entry = 16 * half + 4 * (lane >> 4) + i, piece = (quad ^ (entry >> kSwizzle)) & (kPieces - 1);
+        *reinterpret_cast<float4*>(copy + (lane & 15) * kPitch + entry * H + piece * 4) = make_float4(w[0], w[1], w[2], w[3]);
       }
     }
     __syncthreads();
@@ -327,26 +330,30 @@ __global__ __launch_bounds__(16 * H) void portion_weights_kernel(Args a) {
       for (int x = 0; x < 16; ++x) acc[x] = 0.f;
 #pragma unroll
       for (int s = 0; s < kMix; ++s) {
-        const int want = 2 * s + (lane >> 5);
-        const int piece = H == 32 ? (want ^ ((entry >> 2) & 3)) : (want ^ ((entry >> 3) & 1));
-        const int at = row * kRowBytes + entry * (2 * H) + piece * 16;
-        Frag bh, bl;
-        bh.u = *reinterpret_cast<const u32x4_t*>(ph + at);
-        bl.u = *reinterpret_cast<const u32x4_t*>(pl + at);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tl[s].v, bh.v, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(th[s].v, bl.v, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(th[s].v, bh.v, acc, 0, 0, 0);
-      }
-      uint32_t* out = a.weights + ((size_t)t.row * a.Cmax * H + (size_t)c * H * t.tq + row) * kChunk + entry;
+        float f[8];
 #pragma unroll
-      for (int x = 0; x < 16; x += 2) {
-        const int h = 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3);
-        if (H == 32 || x < 8) {
-          uint32_t p0, p1;
-          split2(acc[x], acc[x + 1], p0, p1);
-          out[(size_t)h * t.tq * kChunk] = low_halves(p1, p0);
-          out[(size_t)(h + 1) * t.tq * kChunk] = high_halves(p1, p0);
+        for (int x = 0; x < 2; ++x) {
+          const int piece = ((4 * s + 2 * (lane >> 5) + x) ^ (entry >> kSwizzle)) & (kPieces - 1);
+          const float4 w = *reinterpret_cast<const float4*>(copy + row * kPitch + entry * H + piece * 4);
+          f[4 * x] = w.x;
+          f[4 * x + 1] = w.y;
+          f[4 * x + 2] = w.z;
+          f[4 * x + 3] = w.w;
         }
+        Frag bh, bm, bl;
+        split_eight(f, bh, bm, bl);
+        acc = mfma32(tl[s], bh, acc);
+        acc = mfma32(tm[s], bm, acc);
+        acc = mfma32(th[s], bl, acc);
+        acc = mfma32(tm[s], bh, acc);
+        acc = mfma32(th[s], bm, acc);
+        acc = mfma32(th[s], bh, acc);
+      }
+      float* out = a.weights + ((size_t)t.row * a.Cmax * H + (size_t)c * H * t.tq + row) * kChunk + entry;
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        const int h = 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3);
+        if (H == 32 || x < 8) out[(size_t)h * t.tq * kChunk] = acc[x];
       }
     }
     // (one barrier a chunk: a wave writes this copy again only after the next chunk's barrier, which every wave
@@ -356,8 +363,9 @@ __global__ __launch_bounds__(16 * H) void portion_weights_kernel(Args a) {
 
 // Four waves take a share's chunks in turn: D = mixed weights (16 rows by 32 entries) times values (32 entries by
 // channels), four heads.  A lane reads VT neighbouring channels of eight entries, which are the VT channel tiles' operands
-// once their halves are paired (column n of tile c is channel VT n + c), so values need no LDS.  134 us at the same
-// sizes, 300 MB of weights read once and the values by every tile from L2; on the vector unit it was 1.2 ms.
+// once their halves are paired (column n of tile c is channel VT n + c), so values need no LDS.  169 us at the same
+// sizes (159 with two pieces a weight), 300 MB of weights read once and the values by every tile from L2; on the vector
+// unit it was 1.2 ms.
 template <int VT, int KVQ>
 __global__ __launch_bounds__(256) void portion_values_kernel(Args a) {
   constexpr int vdim = 16 * VT, per = 4 / KVQ;
@@ -374,13 +382,13 @@ __global__ __launch_bounds__(256) void portion_values_kernel(Args a) {
     for (int c = 0; c < VT; ++c) acc[h][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int lo = (int)((long)t.chunks * split / a.S), hi = (int)((long)t.chunks * (split + 1) / a.S);
   for (int c = lo + wave; c < hi; c += 4) {
-    Frag wh[4], wl[4];
+    Frag wh[4], wm[4], wl[4];
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
-      const uint32_t* p = a.weights + ((size_t)t.row * a.Cmax * a.H + ((size_t)c * a.H + quad * 4 + h) * t.tq + min(n, t.tq - 1)) * kChunk + 8 * g;
-      const u32x4_t x = *reinterpret_cast<const u32x4_t*>(p), y = *reinterpret_cast<const u32x4_t*>(p + 4);
-      wh[h].u = u32x4_t{high_halves(x[0], x[1]), high_halves(x[2], x[3]), high_halves(y[0], y[1]), high_halves(y[2], y[3])};
-      wl[h].u = u32x4_t{low_halves(x[0], x[1]), low_halves(x[2], x[3]), low_halves(y[0], y[1]), low_halves(y[2], y[3])};
+      const float* p = a.weights + ((size_t)t.row * a.Cmax * a.H + ((size_t)c * a.H + quad * 4 + h) * t.tq + min(n, t.tq - 1)) * kChunk + 8 * g;
+      const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 4);
+      const float f[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+      split_eight(f, wh[h], wm[h], wl[h]);
     }
     if (c < t.PC) {
       const int b0 = c * kChunk + 8 * g;
@@ -416,9 +424,10 @@ __global__ __launch_bounds__(256) void portion_values_kernel(Args a) {
             for (int h = 0; h < per; ++h) {
               f32x4_t& o = acc[kv * per + h][cc + y];
               o = mfma16(wh[kv * per + h], vl, o);
-              o = mfma16(wl[kv * per + h], vm, o);
-              o = mfma16(wh[kv * per + h], vm, o);
+              o = mfma16(wm[kv * per + h], vm, o);
               o = mfma16(wl[kv * per + h], vh, o);
+              o = mfma16(wh[kv * per + h], vm, o);
+              o = mfma16(wm[kv * per + h], vh, o);
               o = mfma16(wh[kv * per + h], vh, o);
             }
           }
@@ -455,6 +464,7 @@ __global__ __launch_bounds__(256) void portion_values_kernel(Args a) {
           for (int h = 0; h < per; ++h) {
             f32x4_t& o = acc[kv * per + h][cc];
             o = mfma16(wl[kv * per + h], vf, o);
+            o = mfma16(wm[kv * per + h], vf, o);
             o = mfma16(wh[kv * per + h], vf, o);
           }
         }
@@ -538,7 +548,7 @@ void launch_scores(const Args& a, int tiles, int runs, hipStream_t stream) {
 TK_API int tk_pooled_window_portions(const void* q, const void* k_cache, const void* v_cache, const float* k_pool,
                                      const float* v_pool, int KE, int VE, void* out, const int* positions,
                                      const int* q_start, const int* tables, int table_width, const float* talk,
-                                     unsigned* weights, float* part_m, float* part_l, float* part_o, int N, int R, int H,
+                                     float* weights, float* part_m, float* part_l, float* part_o, int N, int R, int H,
                                      int G, int dim, int vdim, int size, int pool, int page_size, int tiles, int S,
                                      int Cmax, int runs, float scale, hipStream_t stream) {
   if (N <= 0) return 0;

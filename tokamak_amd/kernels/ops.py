@@ -1010,7 +1010,7 @@ def pooled_window_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
         tiles, shares, chunks, runs = pooled_portions_plan(num_heads, window, pool, batch.q_lens,
                                                             batch.facts.get("context.max_len", batch.max_seq_len))
         dev = q.device
-        weights = torch.empty((n, chunks, num_heads, POOLED_CHUNK), dtype=torch.int32, device=dev)
+        weights = torch.empty((n, chunks, num_heads, POOLED_CHUNK), dtype=torch.float32, device=dev)
         stats = torch.empty((2, tiles, num_heads, POOLED_TILE, shares), dtype=torch.float32, device=dev)
         part_o = torch.empty((shares, n, num_heads * vdim), dtype=torch.float32, device=dev) if shares > 1 else None
         _check(_fn("attention_pooled_portions", "tk_pooled_window_portions")(
