@@ -304,6 +304,16 @@ __device__ __forceinline__ unsigned long long fixed_mass(float x, float mx) {
   return (unsigned long long)(exp_unit(x - mx) * 4294967296.f);
 }
 
+// What the draw counts: the mass of what a row with thresholds keeps, a segment of the argmax pass at a time, is a sum of
+// e^(x - max) in fixed point too, so that it does not depend on which blocks form it and in what order: a row draws
+// the same token from the same number whatever else is in the step.  As many bits behind the point as V of them leave
+// (45 for 151,936): all that is cut off together is less than 2^-26 of the best token's mass up to 512 k tokens, less
+// than float32 sums lose.  (32 bits, the thresholds' own, would lose a flat tail's tokens below 2^-32.)
+__device__ __forceinline__ float draw_scale(int V) { return ldexpf(1.f, 31 + __clz(V)); }
+__device__ __forceinline__ unsigned long long draw_mass(float x, float mx, float scale) {
+  return (unsigned long long)(exp_unit(x - mx) * scale);
+}
+
 // f(index, value) for every element of a row, each by one thread of the block.  A block reads
 // its row alone, so what counts is the bytes it has in flight: 16-byte loads where the row's
 // address allows them (a pass over 152 k logits: 14 us instead of 29 and more).
@@ -495,7 +505,7 @@ __global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
   const int low = level.bin;
   const bool both = k_on && p_on;
   if ((both ? level.total : level.inside) > (uint32_t)kCandidates) return;      // (the sampler walks the row)
-  const float mx = row_max[r] * inv_t;
+  const float mx = row_max[r] * inv_t, scale = draw_scale(V);
   unsigned long long above = 0;
   // this block's values, then side by side into the row's list
   for_segment(logits + (size_t)r * ld, V, seg, [&](float logit) {
@@ -511,7 +521,7 @@ __global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
         sh.segment[(size_t)r * kCandidates + to] = (uint8_t)seg;
       }
     } else if (bin > low) {
-      above += fixed_mass(x, mx);
+      above += draw_mass(x, mx, scale);
     }
   });
   unsigned long long upto, whole;
@@ -548,7 +558,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     const unsigned long long* __restrict__ seeds, const unsigned long long* __restrict__ counters,
     const float* __restrict__ row_max, const float* __restrict__ seg_max, const float* __restrict__ seg_mass,
     int* __restrict__ out, float* __restrict__ probs_out, SharedRows shared) {
-  __shared__ float fs[kArgmaxSegments];  // the masses of the row's chunks (16 of the waves, or the 32 segments of the argmax pass)
+  __shared__ float upto[kArgmaxSegments];  // the mass of the row's segments up to and with each
   __shared__ unsigned long long hist64[kBins];
   __shared__ uint32_t hist32[kBins];
   __shared__ unsigned long long scan64[kSampleThreads / kWave];
@@ -747,62 +757,70 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     cut = prefix > kth ? prefix : kth;
   }
 
-  // final distribution over {x >= cut}.  The draw walks the tokens in index order: each
-  // wave sums a contiguous chunk of the row; the chunk that holds the target is then
-  // walked again by the whole block.
-  // Without a threshold the chunks are the segments of the argmax pass, which has left their
-  // masses (relative to each segment's own maximum): no pass over the row here.
+  // final distribution over {x >= cut}.  The draw walks the tokens in index order: the masses of the row's segments (those
+  // of the argmax pass) first, then the segment that holds the target is walked by the whole block.
+  // Without a threshold the argmax pass has left their masses (relative to each segment's own maximum); with a list of
+  // candidates what is kept is in the list; else a wave sums two segments of the row.
   const int lane = tid & (kWave - 1), wave = tid / kWave;
-  constexpr int kWaves = kSampleThreads / kWave;
-  static_assert(kWaves <= kArgmaxSegments, "fs holds either kind of chunk");
-  // (With a list of candidates the chunks are those segments too: what is kept is in the list.)
-  const bool by_segments = listed || (cut == 0 && seg_mass != nullptr);
-  const int nchunks = by_segments ? kArgmaxSegments : kWaves;
-  const int chunk = by_segments ? (((V + kArgmaxSegments - 1) / kArgmaxSegments + 3) & ~3)
-                                : ((V + kWaves - 1) / kWaves + 4 * kWave - 1) / (4 * kWave) * (4 * kWave);
-  const int c_begin = wave * chunk, c_end = min(V, c_begin + chunk);
-  float mine = 0.f;
+  const int chunk = ((V + kArgmaxSegments - 1) / kArgmaxSegments + 3) & ~3;
   const auto kept_mass = [&](float logit) {
     const float x = scaled(logit, inv_t);
     return ordered(x) >= cut ? exp_unit(x - mx) : 0.f;
   };
-  const int c_len = max(0, c_end - c_begin);
-  if (listed) {
-    __syncthreads();
-    if (tid < kArgmaxSegments) segment_mass[tid] = k_on && p_on ? 0 : shared.above[r * kArgmaxSegments + tid];
-    __syncthreads();
-    for (int i = tid; i < ncand; i += nt)
-      if (cand[i] >= cut) atomicAdd(&segment_mass[cand_segment[i]], fixed_mass(unordered(cand[i]), mx));
-    __syncthreads();
-    if (tid < kArgmaxSegments) fs[tid] = (float)segment_mass[tid] * (1.f / 4294967296.f);
-    __syncthreads();
-  } else if (by_segments) {
+  const float scale = draw_scale(V);
+  __syncthreads();
+  if (!k_on && !p_on) {
+    if (tid < kArgmaxSegments) {
+      float run = 0.f;
+      for (int w = 0; w <= tid; ++w) {
+        const float m = seg_max[r * kArgmaxSegments + w];
+        run += m > -INFINITY ? seg_mass[r * kArgmaxSegments + w] * exp_unit(m * inv_t - mx) : 0.f;
+      }
+      upto[tid] = run;
+    }
+  } else {
+    if (listed) {
+      if (tid < kArgmaxSegments) segment_mass[tid] = k_on && p_on ? 0 : shared.above[r * kArgmaxSegments + tid];
+      __syncthreads();
+      for (int i = tid; i < ncand; i += nt)
+        if (cand[i] >= cut) atomicAdd(&segment_mass[cand_segment[i]], draw_mass(unordered(cand[i]), mx, scale));
+    } else {
+      for (int seg = wave; seg < kArgmaxSegments; seg += kSampleThreads / kWave) {
+        const int begin = min(V, seg * chunk), end = min(V, begin + chunk);
+        unsigned long long mine = 0;
+        const auto add = [&](float logit) {
+          const float x = scaled(logit, inv_t);
+          if (ordered(x) >= cut) mine += draw_mass(x, mx, scale);
+        };
+        if ((reinterpret_cast<uintptr_t>(row) & 15) == 0) {  // (segments begin at multiples of four tokens)
+          const int quads = (end - begin) / 4;
+#pragma unroll 8
+          for (int q = lane; q < quads; q += kWave) {
+            const float4 v = *reinterpret_cast<const float4*>(row + begin + 4 * q);
+            add(v.x);
+            add(v.y);
+            add(v.z);
+            add(v.w);
+          }
+          if (lane < end - begin - 4 * quads) add(row[begin + 4 * quads + lane]);
+        } else {
+#pragma unroll 8
+          for (int i = begin + lane; i < end; i += kWave) add(row[i]);
+        }
+#pragma unroll
+        for (int m = kWave / 2; m >= 1; m >>= 1) mine += __shfl_xor(mine, m, kWave);
+        if (lane == 0) segment_mass[seg] = mine;
+      }
+    }
     __syncthreads();
     if (tid < kArgmaxSegments) {
-      const float m = seg_max[r * kArgmaxSegments + tid];
-      fs[tid] = m > -INFINITY ? seg_mass[r * kArgmaxSegments + tid] * exp_unit(m * inv_t - mx) : 0.f;
+      unsigned long long run = 0;      // (rounded once: as float32 numbers one after the other small segments beside a large one were lost)
+      for (int w = 0; w <= tid; ++w) run += segment_mass[w];
+      upto[tid] = (float)run / scale;
     }
-    __syncthreads();
-  } else if ((reinterpret_cast<uintptr_t>(row) & 15) == 0) {  // (chunks begin at multiples of 256 tokens)
-    const int quads = c_len / 4;
-#pragma unroll 8
-    for (int q = lane; q < quads; q += kWave) {
-      const float4 v = *reinterpret_cast<const float4*>(row + c_begin + 4 * q);
-      mine += (kept_mass(v.x) + kept_mass(v.y)) + (kept_mass(v.z) + kept_mass(v.w));
-    }
-    if (lane < c_len - 4 * quads) mine += kept_mass(row[c_begin + 4 * quads + lane]);
-  } else {
-#pragma unroll 8
-    for (int i = lane; i < c_len; i += kWave) mine += kept_mass(row[c_begin + i]);
   }
-  if (!by_segments) {
-    mine = wave_sum(mine);
-    __syncthreads();
-    if (lane == 0) fs[wave] = mine;
-    __syncthreads();
-  }
-  float total = 0.f;
-  for (int w = 0; w < nchunks; ++w) total += fs[w];
+  __syncthreads();
+  const float total = upto[kArgmaxSegments - 1];
 
   if (probs_out) {
     float* po = probs_out + (size_t)r * V;
@@ -819,16 +837,13 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   int sel = (V - 1) / chunk;
   float sel_before = 0.f;
   {
-    float run = 0.f;
     bool found = false;
-    for (int w = 0; w < nchunks; ++w) {
-      const float next = run + fs[w];
-      if (!found && (target < next || w == sel)) {
+    for (int w = 0; w < kArgmaxSegments; ++w) {
+      if (!found && (target < upto[w] || w == sel)) {
         found = true;
         sel = w;
-        sel_before = run;
+        sel_before = w > 0 ? upto[w - 1] : 0.f;
       }
-      run = next;
     }
   }
   const int s_begin = sel * chunk, s_end = min(V, s_begin + chunk);
