@@ -150,3 +150,17 @@ def test_the_streaming_product_takes_65_to_128_rows_where_it_was_measured_to_pay
         assert ops.stream_waves(m, k, False, n) == 8
         splits = stream_splits(n, k, m)
         assert splits > 1 and splits * -(-n // 128) <= 256 and -(-k // 256) // splits >= 2
+
+
+def test_scratch_of_a_scan_in_chunks_follows_from_the_steps_tokens():
+    """One portion of as many tokens stands for every step when a model's memory is measured."""
+    import random
+
+    rng = random.Random(5)
+    for size, least in ((ops.SCAN_CHUNK, ops.SCAN_CHUNKS_FROM_TOKENS), (ops.SSM_CHUNK_TOKENS, ops.SSM_MATRIX_CHUNKS_FROM_TOKENS)):
+        for _ in range(300):
+            spans = [rng.choice([1, rng.randint(1, least + size), least + 1, size + 1]) for _ in range(rng.randint(1, 70))]
+            tokens = sum(spans)
+            tiles, room = ops._tiles_of_long(spans, tokens, size, least)
+            assert tiles == sum(-(-t // size) for t in spans if t >= least)
+            assert tiles <= room == ops._tiles_of_long([tokens], tokens, size, least)[1]

@@ -167,7 +167,7 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(
     ScanIn r_in, ScanIn k_in, ScanIn v_in, ScanIn g_in, ScanIn d_in,
     const float* __restrict__ w0, const float* __restrict__ u, const float* __restrict__ gain,
     float* __restrict__ state, const int* __restrict__ q_start, const int* __restrict__ state_slots,
-    T* __restrict__ out, ScanShape sh, float eps) {
+    T* __restrict__ out, ScanShape sh, float eps, int leave) {
   constexpr int TB = kScanTokens;
   extern __shared__ float lds[];
   const int dim = sh.dim, CT = sh.columns, KS = sh.slices, slice = sh.slice;
@@ -188,6 +188,7 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(
   const int HD = sh.heads * dim;
   const int base = head * dim;
   const int first = q_start[req], end = q_start[req + 1];
+  if (end - first >= leave) return;      // (the whole block)
   float* S = state + ((size_t)state_slots[req] * sh.heads + head) * dim * dim;
   float s[SLICE];
 #pragma unroll
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(
 
 template <typename T>
 int launch_scan(ScanIn r, ScanIn k, ScanIn v, ScanIn g, ScanIn d, const float* w0, const float* u, const float* gain, float* state,
-                const int* q_start, const int* state_slots, void* out, int R, int heads, int dim, float eps,
+                const int* q_start, const int* state_slots, void* out, int R, int heads, int dim, float eps, int leave,
                 hipStream_t stream) {
   ScanShape sh;
   sh.heads = heads;
@@ -295,7 +296,7 @@ int launch_scan(ScanIn r, ScanIn k, ScanIn v, ScanIn g, ScanIn d, const float* w
       allowed = true;                                                                                         \
     }                                                                                                         \
     wkv_scan_kernel<T, SLICE, PLAIN><<<grid, threads, lds, stream>>>(r, k, v, g, d, w0, u, gain, state,       \
-                                                                     q_start, state_slots, (T*)out, sh, eps); \
+                                                                     q_start, state_slots, (T*)out, sh, eps, leave); \
   }
 #define TK_SCAN(SLICE)                 \
   {                                    \
@@ -334,7 +335,7 @@ __global__ __launch_bounds__(1024) void gla_scan_kernel(
     ScanIn q_in, ScanIn k_in, ScanIn v_in, ScanIn g_in, ScanIn z_in, const float* __restrict__ bias,
     const float* __restrict__ gain, float* __restrict__ state, const int* __restrict__ q_start,
     const int* __restrict__ state_slots, T* __restrict__ out, float* __restrict__ raw, GlaShape sh, float q_scale,
-    float inv_tau, float eps) {
+    float inv_tau, float eps, int leave) {
   constexpr int TB = kScanTokens;
   extern __shared__ float lds[];
   const int dim = sh.dim, vdim = sh.vdim, CT = sh.columns, KS = sh.slices, slice = sh.slice;
@@ -356,6 +357,7 @@ __global__ __launch_bounds__(1024) void gla_scan_kernel(
   const int KW = sh.heads * dim, VW = sh.heads * vdim;
   const int kbase = head * dim, vbase = head * vdim;
   const int first = q_start[req], end = q_start[req + 1];
+  if (end - first >= leave) return;      // (the whole block)
   float* S = state + ((size_t)state_slots[req] * sh.heads + head) * dim * vdim;
   float s[SLICE];
 #pragma unroll
@@ -476,7 +478,7 @@ __global__ __launch_bounds__(256) void gla_finish_kernel(const float* __restrict
 template <typename T>
 int launch_gla(ScanIn q, ScanIn k, ScanIn v, ScanIn g, ScanIn z, const float* bias, const float* gain, float* state,
                const int* q_start, const int* state_slots, void* out, float* raw, int N, int splits, int R, int heads,
-               int dim, int vdim, float q_scale, float inv_tau, float eps, hipStream_t stream) {
+               int dim, int vdim, float q_scale, float inv_tau, float eps, int leave, hipStream_t stream) {
   GlaShape sh;
   sh.heads = heads;
   sh.dim = dim;
@@ -513,7 +515,7 @@ int launch_gla(ScanIn q, ScanIn k, ScanIn v, ScanIn g, ScanIn z, const float* bi
     }                                                                                                         \
     gla_scan_kernel<T, SLICE, PLAIN, READY_><<<grid, threads, lds, stream>>>(q, k, v, g, z, bias, gain, state, \
                                                                              q_start, state_slots, (T*)out,   \
-                                                                             raw_out, sh, q_scale, inv_tau, eps); \
+                                                                             raw_out, sh, q_scale, inv_tau, eps, leave); \
   }
 #define TK_GLA(SLICE)                                                   \
   {                                                                     \
@@ -580,22 +582,22 @@ TK_API int tk_tanh(int dtype, const void* in, int in_f32, int parts, long part_s
 
 // r, k, v, g (gate), d (the decay's pre-activation): [N, heads * dim] in dtype, or float32, or
 // float32 partial sums [parts, N, heads * dim]; out in dtype; state [slots, heads, dim, dim]
-// float32.  dim <= 256.
+// float32.  dim <= 256.  leave: requests that bring so many tokens or more are left alone.
 TK_API int tk_wkv_scan(int dtype, const void* r, int r_f32, int r_parts, long r_stride, const void* k, int k_f32,
                        int k_parts, long k_stride, const void* v, int v_f32, int v_parts, long v_stride,
                        const void* g, int g_f32, int g_parts, long g_stride, const void* d, int d_f32, int d_parts,
                        long d_stride, const float* w0, const float* u, const float* gain, float* state,
                        const int* q_start, const int* state_slots, void* out, int R, int heads, int dim, float eps,
-                       hipStream_t stream) {
+                       int leave, hipStream_t stream) {
   if (R <= 0 || heads <= 0) return 0;
   if (dim < 1 || dim > 256) return -2;
   const ScanIn ri{r, r_f32, r_parts, r_stride}, ki{k, k_f32, k_parts, k_stride}, vi{v, v_f32, v_parts, v_stride},
       gi{g, g_f32, g_parts, g_stride}, di{d, d_f32, d_parts, d_stride};
   if (dtype == 0)
     return launch_scan<float>(ri, ki, vi, gi, di, w0, u, gain, state, q_start, state_slots, out, R, heads, dim, eps,
-                              stream);
+                              leave, stream);
   return launch_scan<bf16_t>(ri, ki, vi, gi, di, w0, u, gain, state, q_start, state_slots, out, R, heads, dim, eps,
-                             stream);
+                             leave, stream);
 }
 
 // q, k, z (the decay's pre-activation, to which `bias` is added): [N, heads * dim]; v, g (gate):
@@ -603,24 +605,24 @@ TK_API int tk_wkv_scan(int dtype, const void* r, int r_f32, int r_parts, long r_
 // [N, heads * vdim] in dtype; state [slots, heads, dim, vdim] float32.  dim, vdim <= 256.
 // splits > 1: so many blocks share a head's value columns (8 or more each) and leave the raw o in
 // raw (float32 [N, heads * vdim], and behind it room for the decays, [N, heads * dim]), which a
-// second kernel norms and gates.
+// second kernel norms and gates.  leave: requests that bring so many tokens or more are left alone (splits 1 only).
 TK_API int tk_gla_scan(int dtype, const void* q, int q_f32, int q_parts, long q_stride, const void* k, int k_f32,
                        int k_parts, long k_stride, const void* v, int v_f32, int v_parts, long v_stride,
                        const void* g, int g_f32, int g_parts, long g_stride, const void* z, int z_f32, int z_parts,
                        long z_stride, const float* bias, const float* gain, float* state, const int* q_start,
                        const int* state_slots, void* out, float* raw, int N, int splits, int R, int heads, int dim,
-                       int vdim, float q_scale, float inv_tau, float eps, hipStream_t stream) {
+                       int vdim, float q_scale, float inv_tau, float eps, int leave, hipStream_t stream) {
   if (R <= 0 || heads <= 0) return 0;
   if (dim < 1 || dim > 256 || vdim < 1 || vdim > 256) return -2;
   // shares of a head's columns: 8 columns or more each, and then the raw outputs need a place
-  if (splits < 1 || (splits > 1 && (raw == nullptr || (vdim + splits - 1) / splits < 8))) return -1;
+  if (splits < 1 || (splits > 1 && (raw == nullptr || leave != 0x7fffffff || (vdim + splits - 1) / splits < 8))) return -1;
   const ScanIn qi{q, q_f32, q_parts, q_stride}, ki{k, k_f32, k_parts, k_stride}, vi{v, v_f32, v_parts, v_stride},
       gi{g, g_f32, g_parts, g_stride}, zi{z, z_f32, z_parts, z_stride};
   if (dtype == 0)
     return launch_gla<float>(qi, ki, vi, gi, zi, bias, gain, state, q_start, state_slots, out, raw, N, splits, R, heads,
-                             dim, vdim, q_scale, inv_tau, eps, stream);
+                             dim, vdim, q_scale, inv_tau, eps, leave, stream);
   return launch_gla<bf16_t>(qi, ki, vi, gi, zi, bias, gain, state, q_start, state_slots, out, raw, N, splits, R, heads,
-                            dim, vdim, q_scale, inv_tau, eps, stream);
+                            dim, vdim, q_scale, inv_tau, eps, leave, stream);
 }
 
 TK_SLOTS(tk_token_shift)

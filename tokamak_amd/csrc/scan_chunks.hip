@@ -11,6 +11,8 @@
 // differ first and one for i = j: the product over j < l <= i is cut at the middle of the block that parts them, so both
 // factors are products of decays, at most one, and each round is a plain matrix product of scaled rows.
 //
+// Requests of `least` tokens and more; shorter ones are the walk's (recurrent.hip), whoever stands beside them.
+//
 //   chunk_operands: a block a (chunk, head), a wave 64 channels, a lane one channel of 16 tokens: decays, the scaled
 //     rows q' and k', the whole chunk's decay, M.  All chunks side by side.
 //   chunk_walk: a block a (head, 16 value columns, request), the chunks in order, the state in the waves' accumulators
@@ -70,7 +72,7 @@ __device__ __forceinline__ void load_column(const In& in, size_t first, int n, s
 }
 
 struct Shape {
-  int R, heads, dim, vdim;
+  int R, heads, dim, vdim, least;
   // per (chunk, head): q' [16][dim], k' [dim][16], the chunk's decay [dim], M (see chunk_operands), v [vdim][16]
   __host__ __device__ size_t floats() const { return (size_t)33 * dim + 256 + (size_t)16 * vdim; }
 };
@@ -84,7 +86,7 @@ __global__ __launch_bounds__(128) void chunk_operands_kernel(In q_in, In k_in, I
   __shared__ __align__(16) float rows[2][2][kTokens * kPitch];      // [wave][q', k']
   __shared__ float other[256];
   RequestTile rt;
-  if (!find_request_tile(q_start, sh.R, kTokens, blockIdx.x, rt)) return;
+  if (!find_request_tile(q_start, sh.R, kTokens, blockIdx.x, rt, sh.least)) return;
   const int head = blockIdx.y, lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int c = threadIdx.x, first = q_start[rt.req] + rt.index * kTokens, n = min(kTokens, q_start[rt.req + 1] - first);
   const bool live = c < sh.dim;
@@ -213,10 +215,9 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
   __shared__ float part[2][4][256];
   const int head = blockIdx.x, v0 = blockIdx.y * 16, req = blockIdx.z;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, x = lane & 15, g = lane >> 4;
-  const int first = q_start[req], end = q_start[req + 1], chunks = (end - first + kTokens - 1) / kTokens;
+  const int first = q_start[req], end = q_start[req + 1], chunks = request_tiles(q_start, req, kTokens, sh.least);
   if (chunks == 0) return;
-  int before = 0;
-  for (int r = 0; r < req; ++r) before += (q_start[r + 1] - q_start[r] + kTokens - 1) / kTokens;
+  const int before = tiles_before(q_start, req, kTokens, sh.least);
   const float* op = operands + ((size_t)before * sh.heads + head) * sh.floats();
   const size_t pitch = sh.heads * sh.floats();
   const int VW = sh.heads * sh.vdim;
@@ -285,21 +286,25 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(const float* __restrict
       for (int r = 0; r < 4; ++r) S[(size_t)(channel[i] + 4 * g + r) * sh.vdim] = s[i][r];
 }
 
-// out = o / rms(o) * gain * silu(gate) per (token, head): `lanes` lanes a head, four channels each (bound by its bytes)
+// out = o / rms(o) * gain * silu(gate) per (token, head) of a chunk: `lanes` lanes a head, four channels each (bound by its
+// bytes)
 __global__ __launch_bounds__(256) void chunk_finish_kernel(const float* __restrict__ raw, In g_in, const float* __restrict__ gain,
-                                                           bf16_t* __restrict__ out, int pairs, int heads, int vdim, int gain_heads,
-                                                           int lanes, float eps) {
+                                                           const int* __restrict__ q_start, bf16_t* __restrict__ out, Shape sh,
+                                                           int gain_heads, int lanes, float eps) {
+  RequestTile rt;
+  if (!find_request_tile(q_start, sh.R, kTokens, blockIdx.x, rt, sh.least)) return;
+  const int first = q_start[rt.req] + rt.index * kTokens, n = min(kTokens, q_start[rt.req + 1] - first), vdim = sh.vdim;
   const int at_lane = threadIdx.x % lanes, c = 4 * at_lane;
-  const int pair = blockIdx.x * (blockDim.x / lanes) + threadIdx.x / lanes;
-  const bool live = pair < pairs && c < vdim;
-  const size_t at = (size_t)pair * vdim + c;
+  const int pair = blockIdx.y * (blockDim.x / lanes) + threadIdx.x / lanes;      // (token of the chunk) * heads + head
+  const bool live = pair < n * sh.heads && c < vdim;
+  const size_t at = ((size_t)first * sh.heads + pair) * vdim + c;
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
   if (live) o = *reinterpret_cast<const f32x4*>(raw + at);
   float sq = o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
   for (int m = lanes / 2; m >= 1; m >>= 1) sq += __shfl_xor(sq, m, kWave);
   if (!live) return;
   const float rstd = 1.f / sqrtf(sq / (float)vdim + eps);
-  const f32x4 gn = *reinterpret_cast<const f32x4*>(gain + (pair % heads % gain_heads) * vdim + c);
+  const f32x4 gn = *reinterpret_cast<const f32x4*>(gain + (pair % sh.heads % gain_heads) * vdim + c);
   float y[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -314,7 +319,7 @@ int launch(bool wkv, In q, In k, In v, In g, In d, const float* bias, const floa
            float inv_tau, float eps, hipStream_t stream) {
   if (sh.R <= 0 || N <= 0) return 0;
   if (sh.heads < 1 || sh.heads > 65535 || sh.dim < 16 || sh.dim > kMaxDim || sh.dim % 16 || sh.vdim < 16 || sh.vdim > kMaxDim ||
-      sh.vdim % 16 || chunks < 1 || operands == nullptr || raw == nullptr)
+      sh.vdim % 16 || sh.least < 1 || chunks < 1 || operands == nullptr || raw == nullptr)
     return -2;
   const dim3 per_chunk(chunks, sh.heads);
   const int threads = (max(sh.dim, sh.vdim) + kWave - 1) / kWave * kWave;
@@ -327,35 +332,37 @@ int launch(bool wkv, In q, In k, In v, In g, In d, const float* bias, const floa
   else chunk_walk_kernel<2><<<walks, 256, 0, stream>>>(operands, state, q_start, slots, raw, sh);
   int lanes = 4;
   while (4 * lanes < sh.vdim) lanes *= 2;
-  const int pairs = N * sh.heads, per = 256 / lanes;
-  chunk_finish_kernel<<<(pairs + per - 1) / per, 256, 0, stream>>>(raw, g, gain, (bf16_t*)out, pairs, sh.heads, sh.vdim, gain_heads, lanes, eps);
+  const int per = 256 / lanes;
+  chunk_finish_kernel<<<dim3(chunks, (kTokens * sh.heads + per - 1) / per), 256, 0, stream>>>(raw, g, gain, q_start, (bf16_t*)out, sh, gain_heads,
+                                                                                            lanes, eps);
   return launch_status();
 }
 
 }  // namespace
 
 // Operands, state and output as in tk_gla_scan / tk_wkv_scan (recurrent.hip), bfloat16 storage; dim and vdim multiples of
-// 16 up to 128.  chunks: at least the chunks of 16 tokens that all requests have together; operands (float32
-// [chunks, heads, 33 dim + 16 vdim + 256]) and raw (float32 [N, heads * vdim]) are scratch on 16-byte borders.
+// 16 up to 128.  least: requests of fewer tokens are left alone; chunks: at least the chunks of 16 tokens that the others
+// have together; operands (float32 [chunks, heads, 33 dim + 16 vdim + 256]) and raw (float32 [N, heads * vdim]) are
+// scratch on 16-byte borders.
 TK_API int tk_gla_chunks(const void* q, int q_f32, int q_parts, long q_stride, const void* k, int k_f32, int k_parts,
                          long k_stride, const void* v, int v_f32, int v_parts, long v_stride, const void* g, int g_f32,
                          int g_parts, long g_stride, const void* z, int z_f32, int z_parts, long z_stride, const float* bias,
                          const float* gain, float* state, const int* q_start, const int* state_slots, void* out,
-                         float* operands, float* raw, int N, int R, int chunks, int heads, int dim, int vdim, float q_scale,
+                         float* operands, float* raw, int N, int R, int least, int chunks, int heads, int dim, int vdim, float q_scale,
                          float inv_tau, float eps, hipStream_t stream) {
   return launch(false, In{q, q_f32, q_parts, q_stride}, In{k, k_f32, k_parts, k_stride}, In{v, v_f32, v_parts, v_stride},
                 In{g, g_f32, g_parts, g_stride}, In{z, z_f32, z_parts, z_stride}, bias, nullptr, gain, 1, state, q_start, state_slots,
-                out, operands, raw, N, chunks, Shape{R, heads, dim, vdim}, q_scale, inv_tau, eps, stream);
+                out, operands, raw, N, chunks, Shape{R, heads, dim, vdim, least}, q_scale, inv_tau, eps, stream);
 }
 
 TK_API int tk_wkv_chunks(const void* r, int r_f32, int r_parts, long r_stride, const void* k, int k_f32, int k_parts,
                          long k_stride, const void* v, int v_f32, int v_parts, long v_stride, const void* g, int g_f32,
                          int g_parts, long g_stride, const void* d, int d_f32, int d_parts, long d_stride, const float* w0,
                          const float* u, const float* gain, float* state, const int* q_start, const int* state_slots, void* out,
-                         float* operands, float* raw, int N, int R, int chunks, int heads, int dim, float eps, hipStream_t stream) {
+                         float* operands, float* raw, int N, int R, int least, int chunks, int heads, int dim, float eps, hipStream_t stream) {
   return launch(true, In{r, r_f32, r_parts, r_stride}, In{k, k_f32, k_parts, k_stride}, In{v, v_f32, v_parts, v_stride},
                 In{g, g_f32, g_parts, g_stride}, In{d, d_f32, d_parts, d_stride}, w0, u, gain, heads, state, q_start, state_slots, out,
-                operands, raw, N, chunks, Shape{R, heads, dim, dim}, 1.f, 1.f, eps, stream);
+                operands, raw, N, chunks, Shape{R, heads, dim, dim, least}, 1.f, 1.f, eps, stream);
 }
 
 TK_SLOTS(tk_gla_chunks)

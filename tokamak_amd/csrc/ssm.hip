@@ -165,7 +165,7 @@ __global__ __launch_bounds__(1024) void ssd_scan_kernel(
     const T* __restrict__ u, int C, SsmIn dt_in, long ld, int dt_col, const float* __restrict__ dt_bias,
     const float* __restrict__ a_log, const float* __restrict__ skip, float* __restrict__ state,
     const int* __restrict__ q_start, const int* __restrict__ state_slots, float* __restrict__ y, ScanShape sh,
-    int chunk, int max_chunks, float* __restrict__ chunk_state, float* __restrict__ chunk_decay) {
+    int chunk, int max_chunks, float* __restrict__ chunk_state, float* __restrict__ chunk_decay, int leave) {
   constexpr int TB = kScanTokens, CS = 4;
   constexpr int nsp = KS * RS;       // rows with the padding (zeros behind ns)
   extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -176,6 +176,7 @@ __global__ __launch_bounds__(1024) void ssd_scan_kernel(
   const int req = MODE == 0 ? blockIdx.x : blockIdx.x / max_chunks, head = blockIdx.y;
   int first = q_start[req];
   int end = q_start[req + 1];
+  if (MODE == 0 && end - first >= leave) return;      // (the whole block)
   size_t place = 0;       // of this chunk in the scratch arrays
   if (MODE != 0) {
     const int ci = blockIdx.x % max_chunks;
@@ -460,7 +461,7 @@ template <typename T, bool SILU = false>
 int launch_scan(const void* u, int C, SsmIn dt, long ld, int dt_col, const float* dt_bias, const float* a_log,
                 const float* skip, float* state, const int* q_start, const int* state_slots, float* y, int R,
                 int heads, int groups, int ns, int vdim, int splits, int chunk, int max_chunks, float* chunk_state,
-                float* chunk_decay, hipStream_t stream) {
+                float* chunk_decay, int leave, hipStream_t stream) {
   ScanShape sh;
   sh.heads = heads;
   sh.groups = groups;
@@ -491,7 +492,7 @@ int launch_scan(const void* u, int C, SsmIn dt, long ld, int dt_col, const float
     ssd_scan_kernel<T, RS, KS, MODE, SILU><<<grid, threads, lds, stream>>>((const T*)u, C, dt, ld, dt_col, dt_bias, \
                                                                     a_log, skip, state, q_start, state_slots, \
                                                                     y, sh, chunk, max_chunks, chunk_state,    \
-                                                                    chunk_decay);                             \
+                                                                    chunk_decay, leave);                      \
   }
 #define TK_SSD(MODE)                               \
   {                                                \
@@ -549,12 +550,14 @@ TK_API int tk_conv_silu(int dtype, const void* proj, int in_f32, int parts, long
 // splits: blocks that share a head's value columns.  chunk > 0: portions are cut into chunks of so many tokens
 // that run side by side; max_chunks: the most chunks a request of the step has; chunk_state float32
 // [chunks of the step, heads, ceil(vdim / 4), ns, 4] and chunk_decay float32 [chunks of the step, heads] are scratch.
+// leave: requests that bring so many tokens or more are left alone (chunk 0 only).
 TK_API int tk_ssd_scan(int dtype, const void* u, const void* dt, int dt_f32, int dt_parts, long dt_stride, long ld,
                        int dt_col, const float* dt_bias, const float* a_log, const float* skip, float* state,
                        const int* q_start, const int* state_slots, float* y, int R, int heads, int groups, int ns,
-                       int vdim, int splits, int chunk, int max_chunks, float* chunk_state, float* chunk_decay,
+                       int vdim, int splits, int chunk, int max_chunks, float* chunk_state, float* chunk_decay, int leave,
                        hipStream_t stream) {
   if (R <= 0) return 0;
+  if (chunk > 0 && leave != 0x7fffffff) return -1;
   if (chunk < 0 || (chunk > 0 && (max_chunks < 1 || chunk_state == nullptr || chunk_decay == nullptr ||
                                   (long)R * max_chunks > 0x7fffffffL)))
     return -1;
@@ -565,9 +568,9 @@ TK_API int tk_ssd_scan(int dtype, const void* u, const void* dt, int dt_f32, int
   const int C = heads * vdim + 2 * groups * ns;
   if (dtype == 0)
     return launch_scan<float>(u, C, in, ld, dt_col, dt_bias, a_log, skip, state, q_start, state_slots, y, R, heads,
-                              groups, ns, vdim, splits, chunk, max_chunks, chunk_state, chunk_decay, stream);
+                              groups, ns, vdim, splits, chunk, max_chunks, chunk_state, chunk_decay, leave, stream);
   return launch_scan<bf16_t>(u, C, in, ld, dt_col, dt_bias, a_log, skip, state, q_start, state_slots, y, R, heads,
-                             groups, ns, vdim, splits, chunk, max_chunks, chunk_state, chunk_decay, stream);
+                             groups, ns, vdim, splits, chunk, max_chunks, chunk_state, chunk_decay, leave, stream);
 }
 
 // proj: [N, ld] (dtype, float32 or partial sums), its columns [v: heads * vdim | k: heads * dim | q: heads * dim | ...]
@@ -586,9 +589,9 @@ TK_API int tk_fixed_decay_scan(int dtype, const void* proj, int in_f32, int part
   const SsmIn in{proj, in_f32 || dtype == 0, parts, part_stride};
   if (dtype == 0)
     return launch_scan<float, true>(nullptr, 0, in, ld, 0, nullptr, decay, nullptr, state, q_start, state_slots, y, R, heads,
-                                    heads, dim, vdim, splits, chunk, max_chunks, chunk_state, chunk_decay, stream);
+                                    heads, dim, vdim, splits, chunk, max_chunks, chunk_state, chunk_decay, 0x7fffffff, stream);
   return launch_scan<bf16_t, true>(nullptr, 0, in, ld, 0, nullptr, decay, nullptr, state, q_start, state_slots, y, R, heads,
-                                   heads, dim, vdim, splits, chunk, max_chunks, chunk_state, chunk_decay, stream);
+                                   heads, dim, vdim, splits, chunk, max_chunks, chunk_state, chunk_decay, 0x7fffffff, stream);
 }
 
 // y float32 [N, inner]; z: column z_col .. + inner of rows ld long; weight float32 [inner], or

@@ -1,6 +1,8 @@
 // The selective state-space scan in chunks of 64 tokens on the matrix cores (gfx950): the form of portions for the scan
 // of ssm.hip.
 //
+// Requests of `least` tokens and more; shorter ones are the walk's, whoever stands beside them.
+//
 //     S <- a_t S + dt_t B_t x_t^T,  y_t = S^T C_t + D x_t,   dt_t = softplus(dt_in + bias), a_t = exp(-exp(A_log) dt_t)
 //
 // The decay is one number a head and token, so with S the state before a chunk
@@ -36,7 +38,7 @@ constexpr int kMaxDim = 128;
 constexpr int kMaxHeads = 4;      // heads a block takes, one after the other
 
 struct Shape {
-  int R, heads, groups, vdim, C, dt_col, per;      // per: heads a block takes (a divisor of a group's heads)
+  int R, heads, groups, vdim, C, dt_col, per, least;      // per: heads a block takes (a divisor of a group's heads)
   long ld;
 };
 
@@ -85,7 +87,7 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_sums_kernel(const bf16_t* 
   extern __shared__ __attribute__((aligned(16))) float xx[];
   __shared__ float dts[kMaxHeads][kTokens], as[kMaxHeads][kTokens], ws[kMaxHeads][kTokens];
   RequestTile rt;
-  if (!find_request_tile(q_start, sh.R, kTokens, blockIdx.x, rt)) return;
+  if (!find_request_tile(q_start, sh.R, kTokens, blockIdx.x, rt, sh.least)) return;
   const int first = q_start[rt.req] + rt.index * kTokens, count = min(kTokens, q_start[rt.req + 1] - first);
   const int head0 = blockIdx.y * sh.per, group = head0 / (sh.heads / sh.groups), vp = sums_pitch(sh.vdim);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, quad = lane >> 4;
@@ -145,12 +147,12 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_sums_kernel(const bf16_t* 
 // state on return; the request's state moves to the end of the step's tokens.  Eight chunks' sums in flight.
 __global__ __launch_bounds__(256) void ssm_chunk_starts_kernel(float* __restrict__ state, const int* __restrict__ q_start,
                                                                const int* __restrict__ state_slots, float* __restrict__ chunk_state,
-                                                               const float* __restrict__ chunk_decay, int heads, int elems) {
+                                                               const float* __restrict__ chunk_decay, int heads, int elems, int least) {
   const int req = blockIdx.x, head = blockIdx.y, e = blockIdx.z * blockDim.x + threadIdx.x;
-  const int count = (q_start[req + 1] - q_start[req] + kTokens - 1) / kTokens;
-  if (count == 0 || e >= elems) return;
-  int before = 0;
-  for (int r = 0; r < req; ++r) before += (q_start[r + 1] - q_start[r] + kTokens - 1) / kTokens;
+  const int count = request_tiles(q_start, req, kTokens, least);
+  if (count == 0) return;
+  const int before = tiles_before(q_start, req, kTokens, least);
+  if (e >= elems) return;
   float* S = state + ((size_t)state_slots[req] * heads + head) * elems + e;
   float* cs = chunk_state + ((size_t)before * heads + head) * elems + e;
   const float* decay = chunk_decay + (size_t)before * heads + head;
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_outputs_kernel(const bf16_
   __shared__ float dts[kMaxHeads][kTokens], as[kMaxHeads][kTokens];
   __shared__ __attribute__((aligned(16))) float whole[kTokens];
   RequestTile rt;
-  if (!find_request_tile(q_start, sh.R, kTokens, blockIdx.x, rt)) return;
+  if (!find_request_tile(q_start, sh.R, kTokens, blockIdx.x, rt, sh.least)) return;
   const int first = q_start[rt.req] + rt.index * kTokens, count = min(kTokens, q_start[rt.req + 1] - first);
   const int head0 = blockIdx.y * sh.per, group = head0 / (sh.heads / sh.groups), vp = sh.vdim + 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, quad = lane >> 4;
@@ -297,7 +299,7 @@ int launch(const bf16_t* u, RowsIn dt, const float* dt_bias, const float* a_log,
   const dim3 grid(chunks, sh.heads / sh.per);
   ssm_chunk_sums_kernel<S16><<<grid, kThreads, sums_lds, stream>>>(u, dt, dt_bias, a_log, q_start, chunk_state, chunk_decay, sh);
   ssm_chunk_starts_kernel<<<dim3(sh.R, sh.heads, (elems + 255) / 256), 256, 0, stream>>>(state, q_start, slots, chunk_state, chunk_decay,
-                                                                                       sh.heads, elems);
+                                                                                       sh.heads, elems, sh.least);
   ssm_chunk_outputs_kernel<S16><<<grid, kThreads, out_lds, stream>>>(u, dt, dt_bias, a_log, skip, q_start, chunk_state, y, sh);
   return launch_status();
 }
@@ -305,20 +307,20 @@ int launch(const bf16_t* u, RowsIn dt, const float* dt_bias, const float* a_log,
 }  // namespace
 
 // Operands, state and y as in tk_ssd_scan (ssm.hip), bfloat16 storage; ns 16, 32, 64 or 128, vdim a multiple of 16 up to 128, u on a 16-byte
-// border.  chunks: at least the chunks of 64 tokens that all requests have together; per: heads a block takes, a divisor of
+// border.  least: requests of fewer tokens are left alone; chunks: at least the chunks of 64 tokens that the others have together; per: heads a block takes, a divisor of
 // the heads of a group, up to 4; chunk_state float32 [chunks, heads, vdim / 4, ns, 4] and chunk_decay float32 [chunks,
 // heads] are scratch.
 TK_API int tk_ssm_chunks(const void* u, const void* dt, int dt_f32, int dt_parts, long dt_stride, long ld, int dt_col,
                          const float* dt_bias, const float* a_log, const float* skip, float* state, const int* q_start,
-                         const int* state_slots, float* y, int R, int heads, int groups, int ns, int vdim, int chunks, int per,
+                         const int* state_slots, float* y, int R, int heads, int groups, int ns, int vdim, int least, int chunks, int per,
                          float* chunk_state, float* chunk_decay, hipStream_t stream) {
   if (R <= 0) return 0;
   if (heads < 1 || heads > 65535 || groups < 1 || heads % groups != 0 || (ns != 16 && ns != 32 && ns != 64 && ns != 128) || vdim < 16 ||
-      vdim > kMaxDim || vdim % 16 != 0 || chunks < 1 || per < 1 || per > kMaxHeads || (heads / groups) % per != 0 || dt_parts < 1 ||
+      vdim > kMaxDim || vdim % 16 != 0 || least < 1 || chunks < 1 || per < 1 || per > kMaxHeads || (heads / groups) % per != 0 || dt_parts < 1 ||
       (dt_parts > 1 && !dt_f32) || (uintptr_t)u % 16 != 0 || chunk_state == nullptr || chunk_decay == nullptr)
     return -1;
   const RowsIn in{dt, dt_f32, dt_parts, dt_stride};
-  const Shape sh{R, heads, groups, vdim, heads * vdim + 2 * groups * ns, dt_col, per, ld};
+  const Shape sh{R, heads, groups, vdim, heads * vdim + 2 * groups * ns, dt_col, per, least, ld};
 #define TK_GO(S16_) return launch<S16_>((const bf16_t*)u, in, dt_bias, a_log, skip, state, q_start, state_slots, y, chunks, sh, chunk_state, chunk_decay, stream)
   if (ns == 16) TK_GO(1);
   if (ns == 32) TK_GO(2);

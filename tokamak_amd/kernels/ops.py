@@ -225,11 +225,11 @@ _SIGS = {
         "tk_wkv_scan": [c_int, c_void_p, c_int, c_int, c_long, c_void_p, c_int, c_int, c_long, c_void_p, c_int, c_int,
                         c_long, c_void_p, c_int, c_int, c_long, c_void_p, c_int, c_int, c_long, c_void_p,
                         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float,
-                        c_void_p],
+                        c_int, c_void_p],
         "tk_gla_scan": [c_int, c_void_p, c_int, c_int, c_long, c_void_p, c_int, c_int, c_long, c_void_p, c_int, c_int,
                         c_long, c_void_p, c_int, c_int, c_long, c_void_p, c_int, c_int, c_long, c_void_p,
                         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
-                        c_float, c_float, c_float, c_void_p],
+                        c_float, c_float, c_float, c_int, c_void_p],
     },
     "moe": {
         "tk_moe_route": [c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p,
@@ -301,7 +301,7 @@ _SIGS = {
                          c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
         "tk_ssd_scan": [c_int, c_void_p, c_void_p, c_int, c_int, c_long, c_long, c_int, c_void_p, c_void_p, c_void_p,
                         c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
-                        c_void_p, c_void_p, c_void_p],
+                        c_void_p, c_void_p, c_int, c_void_p],
         "tk_fixed_decay_scan": [c_int, c_void_p, c_int, c_int, c_long, c_long, c_void_p, c_void_p, c_void_p, c_void_p,
                                 c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
         "tk_gated_group_norm": [c_int, c_void_p, c_void_p, c_int, c_int, c_long, c_long, c_int, c_void_p, c_void_p,
@@ -313,13 +313,13 @@ _SIGS = {
     },
     "ssm_chunks": {
         "tk_ssm_chunks": [c_void_p, c_void_p, c_int, c_int, c_long, c_long, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
-                          c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
+                          c_void_p, c_void_p, c_void_p, *[c_int] * 8, c_void_p, c_void_p, c_void_p],
     },
     "scan_chunks": {
         "tk_gla_chunks": [*[c_void_p, c_int, c_int, c_long] * 5, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
-                          c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_void_p],
+                          c_void_p, c_void_p, *[c_int] * 7, c_float, c_float, c_float, c_void_p],
         "tk_wkv_chunks": [*[c_void_p, c_int, c_int, c_long] * 5, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
-                          c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_void_p],
+                          c_void_p, c_void_p, c_void_p, *[c_int] * 6, c_float, c_void_p],
     },
     "delta": {
         "tk_sum_columns": [c_int, c_void_p, c_int, c_long, c_long, c_int, c_void_p, c_int, c_int, c_void_p],
@@ -1068,20 +1068,35 @@ WKV_MAX_DIM = 256
 
 SCAN_CHUNK = 16                # tokens of a chunk (csrc/scan_chunks.hip: kTokens)
 SCAN_CHUNKS_MAX_DIM = 128
-SCAN_CHUNKS_FROM_TOKENS = 32   # a request's tokens in a step from which the scans run in chunks
+SCAN_CHUNKS_FROM_TOKENS = 32   # a request's tokens in a step from which it is scanned in chunks
+EVERY_REQUEST = 2 ** 31 - 1    # a walk that leaves no request to the chunked form
 
 
 def _scan_in_chunks(dtype: torch.dtype, dim: int, vdim: int, longest: int) -> bool:
-    """Whether a scan with a decay a key channel runs in chunks of 16 tokens on the matrix cores: bfloat16 steps with a
-    portion.  float32 keeps the walk a token at a time, whose bits do not depend on how a prompt is cut."""
+    """Whether a scan with a decay a key channel has requests that run in chunks of 16 tokens on the matrix cores:
+    bfloat16, 32 tokens and more.  The line looks at a request's own tokens alone, so that its bits do not depend on
+    its neighbours; shorter spans of the same step walk, in a launch of their own.  Walked and in chunks, us: gla, 32
+    heads of 128 x 128, one request of 24 tokens 37 and 30, of 32 46 and 30, sixteen of 24 84 and 101, of 32 107 and 102;
+    wkv, 64 heads of 64 x 64, one of 32 24 and 33, of 64 39 and 33, sixteen of 24 75 and 61, of 32 97 and 62; 60 single tokens
+    beside a portion of 1,900, gla: all in chunks 544, each in its own form 309.
+    float32 keeps the walk a token at a time, whose bits do not depend on how a prompt is cut."""
     return (dtype == torch.bfloat16 and longest >= SCAN_CHUNKS_FROM_TOKENS and dim % 16 == 0 and vdim % 16 == 0
             and max(dim, vdim) <= SCAN_CHUNKS_MAX_DIM)
 
 
+def _tiles_of_long(q_lens, tokens: int, size: int, least: int) -> tuple[int, int]:
+    """(tiles of ``size`` tokens that the requests with ``least`` or more have together; the most that any such requests
+    of ``tokens`` together could have).  Scratch is made for the second, so that a step's memory follows from its tokens
+    and the one long portion that is measured when a model is loaded stands for every step."""
+    worst = least + (1 - least) % size      # (one token in the last tile)
+    tiles = sum(-(-t // size) for t in q_lens if t >= least)
+    return tiles, max(tiles, tokens * -(-worst // size) // worst)
+
+
 def _chunk_scratch(batch, n: int, heads: int, dim: int, vdim: int, device):
     """(chunks of the step, their operands, the outputs before the norm) for ``csrc/scan_chunks.hip``."""
-    chunks = sum(-(-t // SCAN_CHUNK) for t in batch.q_lens)
-    return (chunks, torch.empty((chunks, heads, 33 * dim + 16 * vdim + 256), dtype=torch.float32, device=device),
+    chunks, room = _tiles_of_long(batch.q_lens, n, SCAN_CHUNK, SCAN_CHUNKS_FROM_TOKENS)
+    return (chunks, torch.empty((room, heads, 33 * dim + 16 * vdim + 256), dtype=torch.float32, device=device),
             torch.empty((n, heads * vdim), dtype=torch.float32, device=device))
 
 
@@ -1103,15 +1118,18 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tens
     operands = [x for t, what in ((r, "r"), (k, "k"), (v, "v"), (gate, "gate"), (decay_in, "decay_in"))
                 for x in _branch(t, n, hd, dtype, what)]
     _note(f"{n}x{heads}x{dim}", n * hd * 6 * out.element_size(), 4.0 * n * heads * dim * dim)
+    leave = EVERY_REQUEST
     if _scan_in_chunks(dtype, dim, dim, batch.max_q_len) and gain.data_ptr() % 16 == 0 and out.data_ptr() % 16 == 0:
+        leave = SCAN_CHUNKS_FROM_TOKENS
         chunks, scaled, raw = _chunk_scratch(batch, n, heads, dim, dim, out.device)
         _check(_fn("scan_chunks", "tk_wkv_chunks")(
             *operands, _p(w0), _p(u), _p(gain), _p(state), _p(batch.q_start), _p(batch.state_slots), _p(out), _p(scaled),
-            _p(raw), n, batch.num_requests, chunks, heads, dim, float(eps), _stream()), "wkv_chunks")
-        return
+            _p(raw), n, batch.num_requests, leave, chunks, heads, dim, float(eps), _stream()), "wkv_chunks")
+        if min(batch.q_lens) >= leave:
+            return
     _check(_fn("recurrent", "tk_wkv_scan")(
         _code(dtype), *operands, _p(w0), _p(u), _p(gain), _p(state),
-        _p(batch.q_start), _p(batch.state_slots), _p(out), batch.num_requests, heads, dim, float(eps), _stream()),
+        _p(batch.q_start), _p(batch.state_slots), _p(out), batch.num_requests, heads, dim, float(eps), leave, _stream()),
         "wkv_scan")
 
 
@@ -1134,21 +1152,24 @@ def gla_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tens
     operands = [x for t, what, w in ((q, "q", heads * dim), (k, "k", heads * dim), (v, "v", heads * vdim),
                                      (gate, "gate", heads * vdim), (decay_in, "decay_in", heads * dim))
                 for x in _branch(t, n, w, dtype, what)]
-    if _scan_in_chunks(dtype, dim, vdim, batch.max_q_len) and gain.data_ptr() % 16 == 0 and out.data_ptr() % 16 == 0:
+    leave, longest = EVERY_REQUEST, batch.max_q_len
+    if _scan_in_chunks(dtype, dim, vdim, longest) and gain.data_ptr() % 16 == 0 and out.data_ptr() % 16 == 0:
+        leave = SCAN_CHUNKS_FROM_TOKENS
         chunks, scaled, raw = _chunk_scratch(batch, n, heads, dim, vdim, out.device)
         _note(f"{n}x{heads}x{dim}x{vdim} chunks", n * heads * (3 * dim + 3 * vdim) * out.element_size(), 4.0 * n * heads * dim * vdim)
         _check(_fn("scan_chunks", "tk_gla_chunks")(
             *operands, _p(bias), _p(gain), _p(state), _p(batch.q_start), _p(batch.state_slots), _p(out), _p(scaled), _p(raw),
-            n, batch.num_requests, chunks, heads, dim, vdim, float(q_scale), 1.0 / float(tau), float(eps), _stream()),
+            n, batch.num_requests, leave, chunks, heads, dim, vdim, float(q_scale), 1.0 / float(tau), float(eps), _stream()),
             "gla_chunks")
-        return
-    splits = gla_column_splits(batch.num_requests, heads, vdim, batch.max_q_len)
+        if min(batch.q_lens) >= leave:
+            return
+    splits = gla_column_splits(batch.num_requests, heads, vdim, longest) if leave == EVERY_REQUEST else 1
     # (scratch of a scan with shared columns: the raw outputs, and behind them the decays)
     raw = torch.empty((n, heads * (vdim + dim)), dtype=torch.float32, device=out.device) if splits > 1 else None
     _note(f"{n}x{heads}x{dim}x{vdim}", n * heads * (3 * dim + 3 * vdim) * out.element_size(), 4.0 * n * heads * dim * vdim)
     _check(_fn("recurrent", "tk_gla_scan")(
         _code(dtype), *operands, _p(bias), _p(gain), _p(state), _p(batch.q_start), _p(batch.state_slots), _p(out),
-        _p(raw), n, splits, batch.num_requests, heads, dim, vdim, float(q_scale), 1.0 / float(tau), float(eps), _stream()),
+        _p(raw), n, splits, batch.num_requests, heads, dim, vdim, float(q_scale), 1.0 / float(tau), float(eps), leave, _stream()),
         "gla_scan")
 
 
@@ -1176,7 +1197,8 @@ SSM_SPLIT_MIN_COLUMNS = 8
 SSM_SPLIT_BLOCKS = 1024
 SSM_CHUNK_TOKENS = 64        # tokens of a chunk of a long portion; the chunks of a portion run side by side
 SSM_MATRIX_CHUNKS_MAX_DIM = 128
-SSM_CHUNKS_FROM_TOKENS = 128  # a request's tokens in a step from which the step's portions are cut into chunks
+SSM_MATRIX_CHUNKS_FROM_TOKENS = 64    # a request's tokens in a step from which it is scanned in chunks on the matrix cores
+SSM_CHUNKS_FROM_TOKENS = 128  # a request's tokens in a step from which the general form cuts the step's portions into chunks
 
 
 def _ssm_in(t: torch.Tensor, rows: int, dtype: torch.dtype, what: str):
@@ -1224,11 +1246,13 @@ def ssd_column_splits(requests: int, heads: int, vdim: int, longest: int) -> int
 
 
 def _ssm_in_chunks(u: torch.Tensor, state_size: int, vdim: int, longest: int) -> bool:
-    """Whether the state-space scan runs in chunks of 64 tokens on the matrix cores: bfloat16 steps with a portion
-    that the general form would cut into chunks too (32 heads of 128 x 64: one portion of 128 tokens 182 us there, 35
-    here; eleven of 180, 349 and 159).  Shorter portions walk: of 64 tokens one took 90 us there and 33 here, but sixteen
-    79 and 98, since a chunk's state is written and read three times however few its tokens."""
-    return (u.dtype == torch.bfloat16 and longest >= SSM_CHUNKS_FROM_TOKENS
+    """Whether the state-space scan has requests that run in chunks of 64 tokens on the matrix cores: bfloat16, 64
+    tokens and more.  The line looks at a request's own tokens alone, so that its bits do not depend on its neighbours;
+    shorter spans of the same step walk, in a launch of their own.  A chunk's state is written and read three times however
+    few its tokens.  Walked and in chunks, us: 32 heads of 128 x 64, one request of 48 tokens 38 and 30, of 64 91 and
+    33, of 128 182 and 35; sixteen of 48 52 and 72, of 64 72 and 78, of 96 113 and 104; 128 heads, sixteen of 64
+    279 and 251."""
+    return (u.dtype == torch.bfloat16 and longest >= SSM_MATRIX_CHUNKS_FROM_TOKENS
             and state_size in (16, 32, 64, 128) and vdim % 16 == 0 and vdim <= SSM_MATRIX_CHUNKS_MAX_DIM and u.data_ptr() % 16 == 0)
 
 
@@ -1261,21 +1285,25 @@ def ssd_scan(u: torch.Tensor, proj: torch.Tensor, dt_col: int, dt_bias: torch.Te
     pointer, is_f32, parts, stride, ld = _ssm_in(proj, n, u.dtype, "projections")
     _need(0 <= dt_col and dt_col + heads <= ld, "the step sizes lie outside the projections")
     if _ssm_in_chunks(u, state_size, vdim, batch.max_q_len):
-        chunks = sum(-(-t // SSM_CHUNK_TOKENS) for t in batch.q_lens)
+        leave = SSM_MATRIX_CHUNKS_FROM_TOKENS
+        chunks, room = _tiles_of_long(batch.q_lens, n, SSM_CHUNK_TOKENS, leave)
         per = ssm_chunk_heads(chunks, heads, groups)
-        chunk_state = torch.empty((chunks, heads, vdim // 4, state_size, 4), dtype=torch.float32, device=y.device)
-        chunk_decay = torch.empty((chunks, heads), dtype=torch.float32, device=y.device)
+        chunk_state = torch.empty((room, heads, vdim // 4, state_size, 4), dtype=torch.float32, device=y.device)
+        chunk_decay = torch.empty((room, heads), dtype=torch.float32, device=y.device)
         _note(f"{n}x{heads}x{state_size}x{vdim} chunks", n * (c * u.element_size() + heads * vdim * 4), 6.0 * n * heads * state_size * vdim)
         _check(_fn("ssm_chunks", "tk_ssm_chunks")(
             _p(u), pointer, is_f32, parts, stride, ld, int(dt_col), _p(dt_bias), _p(a_log), _p(skip), _p(state),
-            _p(batch.q_start), _p(batch.state_slots), _p(y), batch.num_requests, heads, groups, state_size, vdim, chunks, per,
+            _p(batch.q_start), _p(batch.state_slots), _p(y), batch.num_requests, heads, groups, state_size, vdim, leave, chunks, per,
             _p(chunk_state), _p(chunk_decay), _stream()), "ssm_chunks")
-        return
-    plan = _scan_chunks(batch, n, heads, state_size, vdim, y.device)
+        if min(batch.q_lens) >= leave:
+            return
+        plan = (ssd_column_splits(batch.num_requests, heads, vdim, leave - 1), 0, 0, None, None)
+    else:
+        leave, plan = EVERY_REQUEST, _scan_chunks(batch, n, heads, state_size, vdim, y.device)
     _note(f"{n}x{heads}x{state_size}x{vdim}", n * (c * u.element_size() + heads * vdim * 4), 6.0 * n * heads * state_size * vdim)
     _check(_fn("ssm", "tk_ssd_scan")(_code(u.dtype), _p(u), pointer, is_f32, parts, stride, ld, int(dt_col), _p(dt_bias),
                                      _p(a_log), _p(skip), _p(state), _p(batch.q_start), _p(batch.state_slots), _p(y),
-                                     batch.num_requests, heads, groups, state_size, vdim, *plan, _stream()), "ssd_scan")
+                                     batch.num_requests, heads, groups, state_size, vdim, *plan, leave, _stream()), "ssd_scan")
 
 
 FIXED_CHUNK_TOKENS = 64          # tokens of a chunk (csrc/linear_chunks.hip: kChunk)
