@@ -51,3 +51,30 @@ def test_experts_in_operand_order(n, top, experts, w, f, skew, form, on_output):
         want = got @ down[e].double().T
         assert float((out[place, token].double() - want).abs().max().nan_to_num(0.0) if token.numel() else 0.0) <= 2e-5 * (1.0 + float(want.abs().max() if token.numel() else 0.0))
     assert bool(torch.isfinite(out).all())
+
+
+@pytest.mark.parametrize("w,f,experts,top", [(4096, 320, 16, 2), (1280, 2560, 40, 3), (3072, 64, 5, 1)])
+def test_a_pair_has_the_same_bits_whoever_stands_before_it(w, f, experts, top):
+    """The form for few tokens: alone, in other orders of the step's tokens (and so of the experts it meets), among many."""
+    from tokamak_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(w)
+    n = 24
+    h = torch.randn(n, w, generator=g).bfloat16().to(DEV)
+    first, second = (ops.expert_operands((torch.randn(experts, r, k, generator=g) * k ** -0.5).bfloat16().to(DEV)) for r, k in ((2 * f, w), (w, f)))
+    chosen, weight = torch.rand(n, experts, generator=g).topk(top, dim=-1).indices.int().to(DEV), torch.rand(n, top, generator=g).to(DEV)
+
+    def run(tokens):
+        index = torch.tensor(tokens, device=DEV)
+        act = torch.empty((len(tokens) * top, f), dtype=torch.bfloat16, device=DEV)
+        out = torch.empty((top, len(tokens), w), dtype=torch.float32, device=DEV)
+        c = chosen[index].contiguous()
+        ops.moe_stream(h[index].contiguous(), first, c, weight[index].contiguous(), act, tokens=len(tokens), top=top, gated=True)
+        ops.moe_stream(act, second, c, None, out, tokens=len(tokens), top=top, gated=False)
+        return act.view(len(tokens), top, f), out
+
+    act, out = run(list(range(n)))
+    for tokens in ([3], [0, 3], [3, 0], [2, 1, 3], [7, 5, 6, 4, 3, 2, 1, 0], list(range(n))[::-1]):
+        a, o = run(tokens)
+        for place, token in enumerate(tokens):
+            assert torch.equal(a[place], act[token]) and torch.equal(o[:, place], out[:, token]), (tokens, token)

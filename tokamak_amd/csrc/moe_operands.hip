@@ -104,7 +104,9 @@ __global__ __launch_bounds__(WAVES * 64) void moe_stream_kernel(const bf16_t* __
   const int n0 = blockIdx.x * 16;
 
   const int total_chunks = (K + kChunk - 1) / kChunk, per = (total_chunks + WAVES - 1) / WAVES;
-  const int rot = (int)((blockIdx.x + blockIdx.y) % (unsigned)per);     // (blocks in step read unlike parts of their rows)
+  // (blocks in step read unlike parts of their rows; by the expert and not by the block's number, which may follow the order
+  // in which the step meets its experts: a pair's sums run in one order whoever stands before it)
+  const int rot = (int)((blockIdx.x + (unsigned)expert) % (unsigned)per);
   const auto chunk_at = [&](int i) {
     const int j = i + rot;
     return wave + (j >= per ? j - per : j) * WAVES;     // (may lie past the last chunk: skipped)
