@@ -78,3 +78,24 @@ def test_a_pair_has_the_same_bits_whoever_stands_before_it(w, f, experts, top):
         a, o = run(tokens)
         for place, token in enumerate(tokens):
             assert torch.equal(a[place], act[token]) and torch.equal(o[:, place], out[:, token]), (tokens, token)
+
+
+def test_more_experts_than_a_step_lists():
+    """5,120 experts, the router's most: their pairs cannot be listed, so their weights stay in rows and many pairs run one
+    by one."""
+    from tokamak_amd.parts.routed_experts import RoutedExperts
+
+    width, ff, experts, n = 64, 64, 5120, 100
+    g = torch.Generator().manual_seed(3)
+    part = RoutedExperts(hidden_size=width, intermediate_size=ff, num_experts=experts, top=1, dtype=torch.bfloat16, device=DEV)
+    weights = {name: (torch.randn(spec.shape, generator=g) * width ** -0.5).to(torch.float32 if spec.held == "float32" else torch.bfloat16)
+               for name, spec in part.expected_tensors("").items()}
+    part.bind("", lambda name: weights[name].to(DEV))
+    h = torch.randn(n, width, generator=g).bfloat16()
+    got = part.forward(h.to(DEV), None).sum(0).cpu().double()
+    scores = torch.sigmoid(h.double() @ weights["router"].double().T)
+    for token, (score, expert) in enumerate(zip(*(t.tolist() for t in scores.max(1)))):
+        x = score * h[token].double()
+        gate, up, down = (weights[f"e{expert}.{name}"].double() for name in ("gate", "up", "down"))
+        want = down @ (torch.nn.functional.silu(gate @ x) * (up @ x))
+        assert float((got[token] - want).abs().max()) <= 2.0 ** -7 * float(want.abs().max())      # (activations rounded to bfloat16)

@@ -1546,9 +1546,13 @@ def expert_operands(matrices: torch.Tensor) -> torch.Tensor:
     return matrices.view(e, rows // 32, 32, k // 32, 4, 8).permute(0, 1, 3, 4, 2, 5).contiguous()
 
 
-def takes_expert_operands(dtype: torch.dtype, width: int, ff: int) -> bool:
-    """Whether a mixture's experts keep their weights in operand order: bfloat16, both sizes multiples of 64."""
-    return dtype == torch.bfloat16 and width % 64 == 0 and ff % 64 == 0
+MOE_LISTED_EXPERTS = 4096      # experts that the one block listing a step's pairs takes (its counts lie in LDS)
+
+
+def takes_expert_operands(dtype: torch.dtype, width: int, ff: int, experts: int) -> bool:
+    """Whether a mixture's experts keep their weights in operand order: bfloat16, both sizes multiples of 64, and few
+    enough experts to be listed, since weights in that order have no form without lists for many pairs."""
+    return dtype == torch.bfloat16 and width % 64 == 0 and ff % 64 == 0 and experts <= MOE_LISTED_EXPERTS
 
 
 def moe_stream_fits(width: int, ff: int, experts: int, pairs: int) -> bool:
@@ -1610,7 +1614,7 @@ def moe_grouped_fits(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor,
     fill 16-byte pieces, and few enough experts for the one block that lists the pairs."""
     f = down.shape[2]
     return (h.dtype == torch.bfloat16 and pairs >= MOE_GROUPED_FROM and h.shape[1] % 8 == 0 and f % 8 == 0
-            and gate_up.shape[0] <= 4096)
+            and gate_up.shape[0] <= MOE_LISTED_EXPERTS)
 
 
 def moe_sort(chosen: torch.Tensor, num_experts: int, tile_pairs: int = MOE_TILE_PAIRS):

@@ -74,7 +74,7 @@ class RoutedExperts(FeedForward):
         if shared_gate is not None and shared_size is None:
             raise ValueError("a gate on the shared expert goes with a shared expert")
         self.logit_bias_name, self.shared_gate_name = logit_bias, shared_gate
-        self.operand_order = ops.takes_expert_operands(dtype, self.hidden_size, self.intermediate_size)
+        self.operand_order = ops.takes_expert_operands(dtype, self.hidden_size, self.intermediate_size, self.num_experts)
         self.logit_bias: torch.Tensor | None = None
         self.router = self.gate_up = self.down = None
         self.correction = self.shared_gate_up = self.shared_down = None
