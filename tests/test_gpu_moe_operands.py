@@ -99,3 +99,19 @@ def test_more_experts_than_a_step_lists():
         gate, up, down = (weights[f"e{expert}.{name}"].double() for name in ("gate", "up", "down"))
         want = down @ (torch.nn.functional.silu(gate @ x) * (up @ x))
         assert float((got[token] - want).abs().max()) <= 2.0 ** -7 * float(want.abs().max())      # (activations rounded to bfloat16)
+
+
+def test_binding_holds_one_matrix_twice_at_most():
+    from tokamak_amd.parts.routed_experts import RoutedExperts
+
+    width, ff, experts = 512, 1024, 16
+    part = RoutedExperts(hidden_size=width, intermediate_size=ff, num_experts=experts, top=2, dtype=torch.bfloat16, device=DEV)
+    expected = part.expected_tensors("")
+    make = lambda name: torch.ones(expected[name].shape, dtype=torch.float32 if expected[name].held == "float32" else torch.bfloat16, device=DEV)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    part.bind("", make)
+    peak = torch.cuda.max_memory_allocated() - before
+    # gate and up (two matrices an expert) as they are read and stacked; or they, laid out, beside down and its copy
+    assert peak <= 4 * experts * width * ff * 2 + (1 << 20), peak

@@ -104,6 +104,7 @@ class RoutedExperts(FeedForward):
         # an expert's gate rows, then its up rows; in the order of the matrix operands where the sizes allow it (see _routed)
         first = torch.stack([fetch(b + n) for b in bases for n in (gate, up)]).view(self.num_experts, -1, self.hidden_size)
         self.gate_up = ops.expert_operands(first) if self.operand_order else first
+        del first       # (the copy in rows goes before the second matrices come)
         second = torch.stack([fetch(b + down) for b in bases])
         self.down = ops.expert_operands(second) if self.operand_order else second
         if self.correction_name is not None:
