@@ -289,12 +289,14 @@ int launch(const bf16_t* u, RowsIn dt, const float* dt_bias, const float* a_log,
   const int vp = sh.vdim + 4, elems = ns * sh.vdim;
   const size_t sums_lds = (size_t)kTokens * sums_pitch(sh.vdim) * 4;
   const size_t out_lds = ((size_t)kTokens * (kTokens + 4) + (size_t)kTokens * vp + (size_t)sh.vdim * (ns + 4)) * 4;
-  static bool raised = false;
-  if (!raised) {
+  static bool raised[64] = {};      // (the attribute belongs to a function on a device)
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -1;
+  if (!raised[dev]) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_chunk_sums_kernel<S16>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) != hipSuccess ||
         hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_chunk_outputs_kernel<S16>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) != hipSuccess)
       return -1;
-    raised = true;
+    raised[dev] = true;
   }
   const dim3 grid(chunks, sh.heads / sh.per);
   ssm_chunk_sums_kernel<S16><<<grid, kThreads, sums_lds, stream>>>(u, dt, dt_bias, a_log, q_start, chunk_state, chunk_decay, sh);
