@@ -83,4 +83,6 @@ def test_chunks(form, heads, dim, vdim, spans, decays, monkeypatch):
     assert float((got - want).norm()) <= 1.02 * float((walked - want).norm())
     for slot, s in want_state.items():
         off = [float((x[slot].double() - s).norm() / s.norm()) for x in (got_state, walked_state)]
-        assert off[0] <= 1.5 * off[1] + 2e-8, off
+        # no further from the 64-bit state than the walk (a fiftieth for chance); where decays leave nothing of the token before,
+        # the walk rounds a number once and a chunk up to twice (2^-25 of it, and 2^-26 more)
+        assert off[0] <= 1.02 * off[1] + (0.0 if decays == "slow" else 2.0 ** -26), off

@@ -70,6 +70,8 @@ def test_state_space_scan_in_chunks(name, monkeypatch):
     assert float((got - want).abs().max()) <= bound
     assert float((kept - state).abs().max()) <= bound
     monkeypatch.setattr(ops, "_ssm_in_chunks", lambda *a: False)
+    monkeypatch.setattr(ops, "SSM_CHUNKS_FROM_TOKENS", 1 << 30)
     general, general_kept = run()
-    assert float((got - want).norm()) <= 1.1 * float((general - want).norm())
-    assert float((kept - state).norm()) <= 1.1 * float((general_kept - state).norm())
+    # no further from the 64-bit result than the walk (a hundredth for so few numbers' chance)
+    assert float((got - want).norm()) <= 1.01 * float((general - want).norm())
+    assert float((kept - state).norm()) <= 1.01 * float((general_kept - state).norm())

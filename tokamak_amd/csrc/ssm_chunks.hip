@@ -13,13 +13,15 @@
 // Everything is float32 behind the convolution's output, the products are the float32 matrix instruction's (16 x 16 x
 // 4).  Its k index may name any four places as long as both operands agree: index g of step r is place 4 g + r
 // of a group of 16, so that a lane's operands of four steps are one 16-byte read.  Sums run in four accumulators: one
-// chain of up to 192 products was further from the 64-bit result than the walk, whose sums run over lanes; four are
-// not (outputs 0.95, states 1.00 of the walk's distance).  float32 storage keeps the walk: with operands of 24 bits the products C B^T
+// chain of up to 192 products was further from the 64-bit result than the walk, whose sums run over lanes.  Products of
+// decays are rounded once, the newest tokens join a state's sum last, and from chunk to chunk a state is carried in float64:
+// outputs 0.91 to 0.99, states 0.93 to 1.00 of the walk's distance (products of decays rounded at each factor and states
+// carried in float32: up to 1.06 and 1.05).  float32 storage keeps the walk: with operands of 24 bits the products C B^T
 // round where the walk does not, and its outputs would be 1.2 to 1.4 times as far.
 //
 // Walked a token at a time (four state rows by four columns a thread, twice over in chunks) this was bound by
 // the LDS reads of B and C, two 16-byte reads a token for 32 multiply-adds: 2,048 tokens of 32
-// heads of 128 x 64, one group, 273 us, 84 here; of 128 heads in 8 groups 920, 255 here.  B and C belong to a group of
+// heads of 128 x 64, one group, 273 us, 82 here; of 128 heads in 8 groups 920, 233 here.  B and C belong to a group of
 // heads: a block takes a few heads of a group and forms C B^T, and reads its operands of B and C, once for them.
 #include "common.h"
 #include "request_tiles.h"
@@ -50,26 +52,29 @@ __device__ __forceinline__ f32x4 load4(const bf16_t* p) {
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // step sizes and decays of the block's heads over the chunk (behind its end: nothing enters, nothing decays)
+// `pad`: places before the first token
 __device__ __forceinline__ void step_sizes(const RowsIn& in, const Shape& sh, const float* dt_bias, const float* a_log, int head0,
-                                           int first, int count, float (*dts)[kTokens], float (*as)[kTokens]) {
-  const int h = threadIdx.x / kTokens, t = threadIdx.x % kTokens;
+                                           int first, int count, int pad, float (*dts)[kTokens], float (*as)[kTokens]) {
+  const int h = threadIdx.x / kTokens, place = threadIdx.x % kTokens, t = place - pad;
   if (h >= sh.per) return;
-  const float dt = softplus(load_in<bf16_t>(in, (size_t)(first + min(t, count - 1)) * sh.ld + sh.dt_col + head0 + h) + dt_bias[head0 + h]);
-  dts[h][t] = t < count ? dt : 0.f;
-  as[h][t] = t < count ? expf(-expf(a_log[head0 + h]) * dt) : 1.f;
+  const bool there = t >= 0 && t < count;
+  const float dt = softplus(load_in<bf16_t>(in, (size_t)(first + max(0, min(t, count - 1))) * sh.ld + sh.dt_col + head0 + h) + dt_bias[head0 + h]);
+  dts[h][place] = there ? dt : 0.f;
+  as[h][place] = there ? expf(-expf(a_log[head0 + h]) * dt) : 1.f;
 }
 
 __device__ __forceinline__ f32x4 sum4(const f32x4 (&x)[4]) { return (x[0] + x[1]) + (x[2] + x[3]); }
 
-// x of a head's chunk, times `scale` a token, into dst [64][pitch] (zeros behind the chunk's end)
+// x of a head's chunk, times `scale` a place, into dst [64][pitch] (zeros before its first and behind its last token)
 template <typename SCALE>
-__device__ __forceinline__ void stage_x(float* dst, int pitch, const bf16_t* u, const Shape& sh, int head, int first, int count, SCALE scale) {
+__device__ __forceinline__ void stage_x(float* dst, int pitch, const bf16_t* u, const Shape& sh, int head, int first, int count, int pad,
+                                        SCALE scale) {
   const int quads = sh.vdim / 4;
   for (int e = threadIdx.x; e < kTokens * quads; e += kThreads) {
-    const int t = e / quads, v = (e - t * quads) * 4;
-    f32x4 x = load4(u + (size_t)(first + min(t, count - 1)) * sh.C + head * sh.vdim + v);
-    x = t < count ? x * scale(t) : f32x4{0.f, 0.f, 0.f, 0.f};
-    *reinterpret_cast<f32x4*>(dst + t * pitch + v) = x;
+    const int place = e / quads, v = (e - place * quads) * 4, t = place - pad;
+    f32x4 x = load4(u + (size_t)(first + max(0, min(t, count - 1))) * sh.C + head * sh.vdim + v);
+    x = t >= 0 && t < count ? x * scale(place) : f32x4{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<f32x4*>(dst + place * pitch + v) = x;
   }
 }
 
@@ -78,11 +83,12 @@ __host__ __device__ inline int sums_pitch(int vdim) { return (vdim / 16 | 1) * 1
 
 // chunk_state[chunk][head] = sum_j dt_j (prod_(l > j) a_l) B_j x_j^T, chunk_decay[chunk][head] = prod a_l.  A wave takes the
 // tiles w and w + 4 of 16 state rows; its operands of B stay in registers over the heads.  Tokens enter in their order, the
-// newest, which weigh most, last: what is rounded before them is small.
+// newest, which weigh most, last: what is rounded before them is small.  So a chunk of few tokens holds them in its last
+// places here.
 template <int S16>
 __global__ __launch_bounds__(kThreads) void ssm_chunk_sums_kernel(const bf16_t* __restrict__ u, RowsIn dt_in, const float* __restrict__ dt_bias,
                                                                   const float* __restrict__ a_log, const int* __restrict__ q_start,
-                                                                  float* __restrict__ chunk_state, float* __restrict__ chunk_decay, Shape sh) {
+                                                                  float* __restrict__ chunk_state, double* __restrict__ chunk_decay, Shape sh) {
   constexpr int ns = 16 * S16, TILES = (S16 + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) float xx[];
   __shared__ float dts[kMaxHeads][kTokens], as[kMaxHeads][kTokens], ws[kMaxHeads][kTokens];
@@ -91,7 +97,8 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_sums_kernel(const bf16_t* 
   const int first = q_start[rt.req] + rt.index * kTokens, count = min(kTokens, q_start[rt.req + 1] - first);
   const int head0 = blockIdx.y * sh.per, group = head0 / (sh.heads / sh.groups), vp = sums_pitch(sh.vdim);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, quad = lane >> 4;
-  step_sizes(dt_in, sh, dt_bias, a_log, head0, first, count, dts, as);
+  const int pad = kTokens - count;
+  step_sizes(dt_in, sh, dt_bias, a_log, head0, first, count, pad, dts, as);
   float b[TILES][16];
 #pragma unroll
   for (int i = 0; i < TILES; ++i)
@@ -99,7 +106,7 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_sums_kernel(const bf16_t* 
     for (int s = 0; s < 4; ++s)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        b[i][4 * s + r] = Elem<bf16_t>::load(u + (size_t)(first + min(16 * s + 4 * r + quad, count - 1)) * sh.C + sh.heads * sh.vdim +
+        b[i][4 * s + r] = Elem<bf16_t>::load(u + (size_t)(first + max(16 * s + 4 * r + quad - pad, 0)) * sh.C + sh.heads * sh.vdim +
                                         group * ns + min(16 * (wave + 4 * i), ns - 16) + col);
   __syncthreads();
   static_assert(kTokens == kWave, "a lane a token");
@@ -111,12 +118,12 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_sums_kernel(const bf16_t* 
       if (lane + m < kTokens) p *= further;
     }
     ws[wave][lane] = (float)(dts[wave][lane] * p);
-    if (lane == 0) chunk_decay[(size_t)blockIdx.x * sh.heads + head0 + wave] = (float)(p * as[wave][0]);
+    if (lane == 0) chunk_decay[(size_t)blockIdx.x * sh.heads + head0 + wave] = p * as[wave][0];
   }
-  const int steps = (count + 15) / 16;
+  const int skipped = pad / 16;      // groups of 16 places without a token
   for (int h = 0; h < sh.per; ++h) {
     __syncthreads();
-    stage_x(xx, vp, u, sh, head0 + h, first, count, [&](int t) { return ws[h][t]; });
+    stage_x(xx, vp, u, sh, head0 + h, first, count, pad, [&](int place) { return ws[h][place]; });
     __syncthreads();
     float* out = chunk_state + ((size_t)blockIdx.x * sh.heads + head0 + h) * ns * sh.vdim;
     for (int v0 = 0; v0 < sh.vdim; v0 += 16) {
@@ -125,20 +132,24 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_sums_kernel(const bf16_t* 
       for (int i = 0; i < TILES; ++i)
 #pragma unroll
         for (int s = 0; s < 4; ++s) acc[i][s] = f32x4{0.f, 0.f, 0.f, 0.f};
+      f32x4 sum[TILES];      // the newest four tokens, which weigh most, join the others' sum
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        if (s >= steps) break;
+        if (s < skipped) continue;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float x = xx[(16 * s + 4 * r + quad) * vp + v0 + col];
 #pragma unroll
-          for (int i = 0; i < TILES; ++i) acc[i][s] = mfma4(x, b[i][4 * s + r], acc[i][s]);
+          for (int i = 0; i < TILES; ++i) {
+            if (r == 3 && s == 3) sum[i] = mfma4(x, b[i][4 * s + r], sum4(acc[i]));
+            else acc[i][s] = mfma4(x, b[i][4 * s + r], acc[i][s]);
+          }
         }
       }
 #pragma unroll
       for (int i = 0; i < TILES; ++i)
         if (16 * (wave + 4 * i) < ns)
-          *reinterpret_cast<f32x4*>(out + ((size_t)(v0 / 4 + quad) * ns + 16 * (wave + 4 * i) + col) * 4) = sum4(acc[i]);
+          *reinterpret_cast<f32x4*>(out + ((size_t)(v0 / 4 + quad) * ns + 16 * (wave + 4 * i) + col) * 4) = sum[i];
     }
   }
 }
@@ -147,7 +158,7 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_sums_kernel(const bf16_t* 
 // state on return; the request's state moves to the end of the step's tokens.  Eight chunks' sums in flight.
 __global__ __launch_bounds__(256) void ssm_chunk_starts_kernel(float* __restrict__ state, const int* __restrict__ q_start,
                                                                const int* __restrict__ state_slots, float* __restrict__ chunk_state,
-                                                               const float* __restrict__ chunk_decay, int heads, int elems, int least) {
+                                                               const double* __restrict__ chunk_decay, int heads, int elems, int least) {
   const int req = blockIdx.x, head = blockIdx.y, e = blockIdx.z * blockDim.x + threadIdx.x;
   const int count = request_tiles(q_start, req, kTokens, least);
   if (count == 0) return;
@@ -155,11 +166,12 @@ __global__ __launch_bounds__(256) void ssm_chunk_starts_kernel(float* __restrict
   if (e >= elems) return;
   float* S = state + ((size_t)state_slots[req] * heads + head) * elems + e;
   float* cs = chunk_state + ((size_t)before * heads + head) * elems + e;
-  const float* decay = chunk_decay + (size_t)before * heads + head;
+  const double* decay = chunk_decay + (size_t)before * heads + head;
   const size_t stride = (size_t)heads * elems;
-  float s = *S;
+  double s = *S;      // (rounded where a chunk reads it, not from chunk to chunk)
   for (int c0 = 0; c0 < count; c0 += 8) {
-    float own[8], d[8];
+    float own[8];
+    double d[8];
 #pragma unroll
     for (int x = 0; x < 8; ++x) {
       const int c = min(c0 + x, count - 1);
@@ -169,12 +181,12 @@ __global__ __launch_bounds__(256) void ssm_chunk_starts_kernel(float* __restrict
 #pragma unroll
     for (int x = 0; x < 8; ++x) {
       if (c0 + x < count) {
-        cs[(c0 + x) * stride] = s;
-        s = fmaf(d[x], s, own[x]);
+        cs[(c0 + x) * stride] = (float)s;
+        s = fma(d[x], s, (double)own[x]);
       }
     }
   }
-  *S = s;
+  *S = (float)s;
 }
 
 // The outputs of a chunk, wave w the tokens 16 w .. + 16: its rows of C and of C B^T stay in registers over the heads; a head's
@@ -196,7 +208,7 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_outputs_kernel(const bf16_
   float* const pd = lds;                      // [64][pp]
   float* const xx = pd + kTokens * pp;        // [64][vp]
   float* const st = xx + kTokens * vp;        // [vdim][sp]
-  step_sizes(dt_in, sh, dt_bias, a_log, head0, first, count, dts, as);
+  step_sizes(dt_in, sh, dt_bias, a_log, head0, first, count, 0, dts, as);
   const bool works = wave * 16 < count;
   const bf16_t* const bc = u + sh.heads * sh.vdim + group * ns + 4 * quad;       // a row's B from here; its C groups * ns further
   f32x4 c[S16], g[4];
@@ -221,7 +233,7 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_outputs_kernel(const bf16_
   for (int h = 0; h < sh.per; ++h) {
     const int head = head0 + h;
     __syncthreads();
-    stage_x(xx, vp, u, sh, head, first, count, [](int) { return 1.f; });
+    stage_x(xx, vp, u, sh, head, first, count, 0, [](int) { return 1.f; });
     const float* const S = chunk_state + ((size_t)blockIdx.x * sh.heads + head) * ns * sh.vdim;
     for (int e = threadIdx.x; e < sh.vdim / 4 * ns; e += kThreads) {
       const f32x4 x = *reinterpret_cast<const f32x4*>(S + 4 * e);
@@ -231,17 +243,29 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_outputs_kernel(const bf16_
     }
     __syncthreads();
     if (!works) continue;
-    // lane j: dt_j times the products of decays from behind j to each of the wave's rows; column 0 also the whole products
+    // lane j: dt_j times the products of decays from behind j to each of the wave's rows; column 0 also the whole products.
+    // Rounded once; a group of 16 places is gone past by its own product, found by a scan over the lanes.
     {
-      float p = 1.f;
       const float dt = dts[h][lane], a0 = as[h][0];
-      for (int i = 0; i < 16 * wave; ++i) p *= i > lane ? as[h][i] : 1.f;
+      double p = (lane & 15) < 15 ? as[h][lane + 1] : 1.f;      // (behind j to the end of its group)
+#pragma unroll
+      for (int m = 1; m < 16; m <<= 1) {
+        const double further = __shfl_down(p, m, kWave);
+        if ((lane & 15) + m < 16) p *= further;
+      }
+      const double group_product = p * as[h][lane];              // (of its group, in the group's first lane)
+#pragma unroll
+      for (int s = 1; s < 3; ++s) {
+        const double product = __shfl(group_product, 16 * s, kWave);
+        if (s < wave && lane < 16 * s) p *= product;
+      }
+      if (lane >= 16 * wave) p = 1.0;
 #pragma unroll
       for (int x = 0; x < 16; ++x) {
         const int i = 16 * wave + x;
         p *= i > lane ? as[h][i] : 1.f;
-        pd[i * pp + lane] = i >= lane ? p * dt : 0.f;
-        if (lane == 0) whole[i] = p * a0;
+        pd[i * pp + lane] = i >= lane ? (float)(p * dt) : 0.f;
+        if (lane == 0) whole[i] = (float)(p * a0);
       }
     }
     wave_lds_sync();
@@ -284,7 +308,7 @@ __global__ __launch_bounds__(kThreads) void ssm_chunk_outputs_kernel(const bf16_
 
 template <int S16>
 int launch(const bf16_t* u, RowsIn dt, const float* dt_bias, const float* a_log, const float* skip, float* state, const int* q_start,
-           const int* slots, float* y, int chunks, const Shape& sh, float* chunk_state, float* chunk_decay, hipStream_t stream) {
+           const int* slots, float* y, int chunks, const Shape& sh, float* chunk_state, double* chunk_decay, hipStream_t stream) {
   constexpr int ns = 16 * S16;
   const int vp = sh.vdim + 4, elems = ns * sh.vdim;
   const size_t sums_lds = (size_t)kTokens * sums_pitch(sh.vdim) * 4;
@@ -310,12 +334,12 @@ int launch(const bf16_t* u, RowsIn dt, const float* dt_bias, const float* a_log,
 
 // Operands, state and y as in tk_ssd_scan (ssm.hip), bfloat16 storage; ns 16, 32, 64 or 128, vdim a multiple of 16 up to 128, u on a 16-byte
 // border.  least: requests of fewer tokens are left alone; chunks: at least the chunks of 64 tokens that the others have together; per: heads a block takes, a divisor of
-// the heads of a group, up to 4; chunk_state float32 [chunks, heads, vdim / 4, ns, 4] and chunk_decay float32 [chunks,
+// the heads of a group, up to 4; chunk_state float32 [chunks, heads, vdim / 4, ns, 4] and chunk_decay float64 [chunks,
 // heads] are scratch.
 TK_API int tk_ssm_chunks(const void* u, const void* dt, int dt_f32, int dt_parts, long dt_stride, long ld, int dt_col,
                          const float* dt_bias, const float* a_log, const float* skip, float* state, const int* q_start,
                          const int* state_slots, float* y, int R, int heads, int groups, int ns, int vdim, int least, int chunks, int per,
-                         float* chunk_state, float* chunk_decay, hipStream_t stream) {
+                         float* chunk_state, double* chunk_decay, hipStream_t stream) {
   if (R <= 0) return 0;
   if (heads < 1 || heads > 65535 || groups < 1 || heads % groups != 0 || (ns != 16 && ns != 32 && ns != 64 && ns != 128) || vdim < 16 ||
       vdim > kMaxDim || vdim % 16 != 0 || least < 1 || chunks < 1 || per < 1 || per > kMaxHeads || (heads / groups) % per != 0 || dt_parts < 1 ||

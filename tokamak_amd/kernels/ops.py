@@ -1289,7 +1289,7 @@ def ssd_scan(u: torch.Tensor, proj: torch.Tensor, dt_col: int, dt_bias: torch.Te
         chunks, room = _tiles_of_long(batch.q_lens, n, SSM_CHUNK_TOKENS, leave)
         per = ssm_chunk_heads(chunks, heads, groups)
         chunk_state = torch.empty((room, heads, vdim // 4, state_size, 4), dtype=torch.float32, device=y.device)
-        chunk_decay = torch.empty((room, heads), dtype=torch.float32, device=y.device)
+        chunk_decay = torch.empty((room, heads), dtype=torch.float64, device=y.device)
         _note(f"{n}x{heads}x{state_size}x{vdim} chunks", n * (c * u.element_size() + heads * vdim * 4), 6.0 * n * heads * state_size * vdim)
         _check(_fn("ssm_chunks", "tk_ssm_chunks")(
             _p(u), pointer, is_f32, parts, stride, ld, int(dt_col), _p(dt_bias), _p(a_log), _p(skip), _p(state),
