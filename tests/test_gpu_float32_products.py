@@ -30,3 +30,26 @@ def test_float32_product(m, n, k, aligned):
         few.fill_(float("nan"))
         ops.gemm_tiled(x[:3], w, few, fewrows_split=split)
         assert torch.equal(few, out[:3])
+
+
+# one operand's rows on 16-byte borders, the other's not; K whole pieces, and not
+@pytest.mark.parametrize("m,n,k", [(17, 63, 4), (65, 130, 61), (129, 65, 68), (70, 200, 254), (2050, 2051, 35), (2048, 2048, 292), (66, 100, 3)])
+@pytest.mark.parametrize("off", ["x", "w", "neither"])
+def test_operands_on_and_off_their_borders(m, n, k, off):
+    from tokamak_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = (torch.randn(rows, k, generator=g).to(DEV) for rows in (m, n))
+    ld = (k + 7) // 4 * 4
+
+    def placed(t, shift):
+        there = torch.full((t.shape[0], ld), float("nan"), device=DEV)[:, shift:shift + k]
+        return there.copy_(t)
+
+    out, want = (torch.full((m, n), float("nan"), device=DEV) for _ in range(2))
+    ops.gemm_tiled(placed(x, int(off == "x")), placed(w, int(off == "w")), out)
+    ops.gemm_tiled(torch.nn.functional.pad(x, (1, 4 - (k + 1) % 4))[:, 1:1 + k], torch.nn.functional.pad(w, (1, 4 - (k + 1) % 4))[:, 1:1 + k], want)
+    assert torch.equal(out, want)
+    exact = x.cpu().double() @ w.cpu().double().T
+    bound = 2.0 ** -24 * (min(k, 256) + -(-k // 256)) * (x.cpu().double().abs() @ w.cpu().double().abs().T)
+    assert bool(((out.cpu().double() - exact).abs() <= bound).all())

@@ -128,8 +128,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   const int wm = (wave & 1) * 32 * H, wn = (wave >> 1) * 32 * H;   // this wave's corner of the block's tile
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
   const int lrow = tid / LANES, lk = (tid % LANES) * 4;
-  // rows whose four k are one aligned 16-byte piece are loaded as one; rows past the end are read at the last row and
-  // never stored, what lies past K is read at the row's end and becomes zero
+  // four k of a row are one 16-byte load; rows past the end are read at the last row and never stored, what lies past K is
+  // read at the row's end and becomes zero.  Where rows do not lie on 16-byte borders, or K ends within a piece, a whole
+  // piece is still one load of 16 bytes, on the border that its numbers have (1,000
+  // rows, weights of 6,144 x 2,048, one operand off its border 293 us, by single numbers 394; K of 2,049 300 and 407; 4 rows 54, 66).
   const bool wide = K % 4 == 0 && K >= 4 && lda % 4 == 0 && ldw % 4 == 0 &&
                     (reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) % 16 == 0;
 
@@ -142,13 +144,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
       for (int e = 0; e < 16; ++e) acc[i][j][e] = total[i][j][e] = 0.f;
 
   float4v ar[PASSES], wr[PASSES];
-  auto fetch = [&](int k0) {
+  const auto fetch = [&](int k0) {
     const int k = k0 + lk;
     if (wide) {
 #pragma unroll
       for (int h = 0; h < PASSES; ++h) {
         ar[h] = *reinterpret_cast<const float4v*>(A + (size_t)min(m0 + lrow + ROWS * h, M - 1) * lda + min(k, K - 4));
         wr[h] = *reinterpret_cast<const float4v*>(W + (size_t)min(n0 + lrow + ROWS * h, N - 1) * ldw + min(k, K - 4));
+      }
+    } else if (k + 3 < K) {
+#pragma unroll
+      for (int h = 0; h < PASSES; ++h) {
+        __builtin_memcpy(&ar[h], A + (size_t)min(m0 + lrow + ROWS * h, M - 1) * lda + k, 16);
+        __builtin_memcpy(&wr[h], W + (size_t)min(n0 + lrow + ROWS * h, N - 1) * ldw + k, 16);
       }
     } else {
 #pragma unroll
