@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("vocab,ld", [(5, 5), (33, 36), (127, 131), (4097, 4100), (20011, 20011), (151936, 151936)])
+@pytest.mark.parametrize("vocab,ld", [(5, 5), (33, 36), (127, 131), (4097, 4100), (20011, 20011), (70001, 70003), (151936, 151936)])
 @pytest.mark.parametrize("spread", ["peaked", "normal", "alike", "holes"])
 def test_shared_rows_choose_what_single_blocks_choose(vocab, ld, spread):
     from tokamak_amd.sampling.params import SamplingParams
@@ -41,7 +41,7 @@ def test_shared_rows_choose_what_single_blocks_choose(vocab, ld, spread):
     assert all(0 <= t < vocab for t in got)
 
 
-@pytest.mark.parametrize("vocab,ld", [(33, 36), (4097, 4100), (20011, 20011), (151936, 151936)])
+@pytest.mark.parametrize("vocab,ld", [(33, 36), (4097, 4100), (20011, 20011), (70001, 70003), (151936, 151936)])
 @pytest.mark.parametrize("spread", ["peaked", "normal", "alike", "flat tail"])
 def test_masses_do_not_depend_on_the_other_rows(vocab, ld, spread):
     """The distribution a row is drawn from has the same bits alone, beside others, and in a step of more rows than are
@@ -79,3 +79,18 @@ def test_masses_do_not_depend_on_the_other_rows(vocab, ld, spread):
         assert float((probs.double() - want)[:-1, 0].abs().max()) <= 2.0 ** -22
     # e^x to some 2^-20 on the exponential unit
     assert float((probs.double() - want).norm() / want.norm()) <= 2.0 ** -19
+
+
+def test_rows_without_thresholds_are_drawn_alone_as_beside_others():
+    """No row with a threshold: the launches that share such rows are left out, and nothing else changes."""
+    from tokamak_amd.sampling.params import SamplingParams
+    from tokamak_amd.sampling.sampler import sample_tokens
+
+    g = torch.Generator().manual_seed(2)
+    rows, vocab = 9, 20011
+    logits = (3.0 * torch.randn(rows + 1, vocab, generator=g)).to(DEV)
+    params = [SamplingParams(temperature=t, top_k=k) for t, k in ((0.7, 0), (1.0, vocab), (0.0, 0), (2.0, vocab + 5), (0.0, 3), (1.0, 0), (0.1, 0), (5.0, 0), (1.0, 0))]
+    seeds, draws = [13 * i + 1 for i in range(rows + 1)], list(range(rows + 1))
+    alone, probs = sample_tokens(logits[:rows], params, seeds[:rows], draws[:rows], return_probs=True)
+    beside, shared_probs = sample_tokens(logits, params + [SamplingParams(temperature=1.0, top_k=4)], seeds, draws, return_probs=True)
+    assert torch.equal(alone, beside[:rows]) and torch.equal(probs, shared_probs[:rows])

@@ -6,9 +6,9 @@
 // keeps every logit >= the k-th largest (ties at the threshold survive); top-p
 // sorts descending and drops a token iff the mass ranked before it already
 // reaches top_p (the best token always survives); softmax over what is left;
-// one draw.  No sort is done here: both thresholds are found by radix selection
-// over the ordered-integer image of the float values, three passes over the row
-// each (the row sits in L2).
+// one draw.  No sort is done here: thresholds are found over the ordered-integer image of the float values, first
+// the histogram bin that holds one (one pass over the row), then among that bin's values alone, by ranks where they
+// are few and by two more radix levels where they are many.
 #include "common.h"
 #include "no_alloc.h"
 
@@ -31,16 +31,44 @@ __device__ __forceinline__ void argmax_take(float& bv, int& bi, float v, int i) 
   }
 }
 
+constexpr int kBins = 4096;  // histogram bins of one radix pass (12 bits)
+constexpr int kCandidates = 16384;
+constexpr int kShareThreads = 256;
+constexpr int kFew = 256;          // values among which a threshold is found by ranks
+
+// Scratch of the rows with thresholds, null: every row is sampled by one block alone.  The argmax pass zeroes what the
+// kernels add into (hist32, hist64, count).
+struct SharedRows {
+  uint32_t* hist32;              // [M][kBins]
+  unsigned long long* hist64;    // [M][kBins]
+  uint32_t* count;               // [M] entries of the list
+  uint32_t* cand;                // [M][kCandidates] ordered images
+  uint8_t* segment;              // [M][kCandidates]
+  unsigned long long* above;     // [M][segments] mass of what is kept for certain and not listed
+};
+
+__device__ __forceinline__ bool has_threshold(const float* temperature, const int* top_k, const float* top_p, int r, int V, bool& k_on, bool& p_on) {
+  k_on = top_k[r] > 0 && top_k[r] < V;
+  p_on = top_p[r] < 1.f;
+  return temperature[r] > 0.f && (k_on || p_on);
+}
+
 // temperature, top_k, top_p, part_mass (all or none): for a row with temperature > 0 and no
 // threshold the block also leaves the sum of e^((x - its segment's maximum) / temperature) over its segment, from which
 // the sampler has the mass of every segment without a pass of its own over the row.
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
     const float* __restrict__ logits, float* __restrict__ part_v, int* __restrict__ part_i, int V,
     long ld, const float* __restrict__ temperature, const int* __restrict__ top_k,
-    const float* __restrict__ top_p, float* __restrict__ part_mass, uint32_t* __restrict__ clear, size_t clear_words) {
-  // scratch that later kernels add into: `clear_words` words a row, shared out over its blocks
-  for (size_t i = (size_t)blockIdx.x * kArgmaxThreads + threadIdx.x; i < clear_words; i += (size_t)kArgmaxSegments * kArgmaxThreads)
-    clear[blockIdx.y * clear_words + i] = 0u;
+    const float* __restrict__ top_p, float* __restrict__ part_mass, SharedRows clear) {
+  // scratch of a row with thresholds that later kernels add into, shared out over its blocks
+  bool k_on, p_on;
+  if (clear.hist32 != nullptr && has_threshold(temperature, top_k, top_p, blockIdx.y, V, k_on, p_on)) {
+    for (int i = blockIdx.x * kArgmaxThreads + threadIdx.x; i < kBins; i += kArgmaxSegments * kArgmaxThreads) {
+      clear.hist32[(size_t)blockIdx.y * kBins + i] = 0u;
+      clear.hist64[(size_t)blockIdx.y * kBins + i] = 0ull;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) clear.count[blockIdx.y] = 0u;
+  }
   __shared__ float best_v[kArgmaxThreads / kWave];
   __shared__ int best_i[kArgmaxThreads / kWave];
   const int seg = blockIdx.x, r = blockIdx.y;
@@ -84,7 +112,7 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
     part_i[r * kArgmaxSegments + seg] = bi;
   }
   if (part_mass == nullptr || !(temperature[r] > 0.f)) return;
-  if ((top_k[r] > 0 && top_k[r] < V) || top_p[r] < 1.f) return;  // a row with a threshold: the sampler sums what it keeps
+  if (has_threshold(temperature, top_k, top_p, r, V, k_on, p_on)) return;  // the sampler sums what it keeps
   // the segment again (it is in the cache): its mass relative to its own maximum
   const float scale = 1.4426950408889634f / temperature[r];  // e^(y / t) = 2^(y log2 e / t)
   float mass = 0.f;
@@ -146,7 +174,7 @@ TK_API int tk_argmax(const float* logits, int* out, float* out_value, float* par
   if (M <= 0) return 0;
   if (V <= 0 || M > 65535) return -1;
   argmax_segments_kernel<<<dim3(kArgmaxSegments, M), kArgmaxThreads, 0, stream>>>(logits, part_v, part_i, V, ld,
-                                                                                   nullptr, nullptr, nullptr, nullptr, nullptr, 0);
+                                                                                   nullptr, nullptr, nullptr, nullptr, SharedRows{});
   argmax_pick_kernel<<<M, kWave, 0, stream>>>(part_v, part_i, out, out_value);
   return launch_status();
 }
@@ -190,7 +218,7 @@ TK_API int tk_argmax_no_alloc(const float* logits, int* out, float* out_value, i
   ArgmaxScratch* scratch = argmax_scratch_of_current_device();
   if (scratch == nullptr) return -4;
   argmax_segments_kernel<<<dim3(kArgmaxSegments, M), kArgmaxThreads, 0, stream>>>(
-      logits, scratch->value, scratch->index, V, ld, nullptr, nullptr, nullptr, nullptr, nullptr, 0);
+      logits, scratch->value, scratch->index, V, ld, nullptr, nullptr, nullptr, nullptr, SharedRows{});
   argmax_pick_kernel<<<M, kWave, 0, stream>>>(scratch->value, scratch->index, out, out_value);
   return launch_status();
 }
@@ -219,7 +247,6 @@ __device__ __forceinline__ float uniform01(uint64_t seed, uint64_t counter) {
 }
 
 constexpr int kSampleThreads = 1024;
-constexpr int kBins = 4096;  // histogram bins of one radix pass (12 bits)
 
 // Prefix sums of one value per thread over the block, threads in index order; `scan`
 // holds an entry a wave.  Returns the sum over the threads before this one;
@@ -344,21 +371,8 @@ __device__ __forceinline__ void for_row(const float* __restrict__ row, int V, F 
 //                   order: sums over the list are of integers), and the mass of the bins above it in each segment; with
 //                   both thresholds the bins above it are listed too, top-p's may lie there.
 // The sampler then starts from the histogram and the list and reads the row again only where the drawn number falls.
-// (A block that reads its row alone moves some 45 GB/s: 40 rows of 152 k logits, most with thresholds, took 95 us with
-// three passes over the row in one block; shared, 12 + 13 us and 21 for the rest, of which a segment's walk, the
-// ranks and the start are each a few memory round trips.)
-constexpr int kCandidates = 16384;
-constexpr int kShareThreads = 256;
-constexpr int kFew = 256;          // values among which a threshold is found by ranks
-
-struct SharedRows {              // scratch of the rows, null: every row is sampled by one block alone
-  uint32_t* hist32;              // [M][kBins], zeroed by the argmax pass, as the others
-  unsigned long long* hist64;    // [M][kBins]
-  uint32_t* count;               // [M] entries of the list
-  uint32_t* cand;                // [M][kCandidates] ordered images
-  uint8_t* segment;              // [M][kCandidates]
-  unsigned long long* above;     // [M][segments] mass of what is kept for certain and not listed
-};
+// (A block that reads its row alone moves some 45 GB/s.  40 rows of 152 k logits, most with thresholds: 12 + 13 us shared and
+// 21 for the rest, of which a segment's walk, the ranks and the start are each a few memory round trips.)
 
 // f(index, value) for every element of a segment, each by one thread of the block
 template <typename F>
@@ -380,12 +394,6 @@ __device__ __forceinline__ void for_segment(const float* __restrict__ row, int V
   } else {
     for (int i = begin + threadIdx.x; i < end; i += kShareThreads) f(row[i]);
   }
-}
-
-__device__ __forceinline__ bool has_threshold(const float* temperature, const int* top_k, const float* top_p, int r, int V, bool& k_on, bool& p_on) {
-  k_on = top_k[r] > 0 && top_k[r] < V;
-  p_on = top_p[r] < 1.f;
-  return temperature[r] > 0.f && (k_on || p_on);
 }
 
 struct FirstLevel {
@@ -548,10 +556,11 @@ __global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
 // row costs 14 us (one CU reads it alone), so the row is walked as rarely as possible: the
 // first pass fills the first level's histogram and tells in which of its bins the threshold
 // lies; if the values of that bin and the bins above it are few (up to kCandidates; they
-// are, unless the logits are nearly all alike), a second pass copies them into LDS, and every
-// further level of both searches reads those.  The third pass is the draw's.  (Without the
-// copies: seven passes with both thresholds.)  Up to kSharedRows rows the first pass and the copies are those of
-// sample_hist and sample_collect; with more rows a block each fills the GPU.
+// are, unless the logits are nearly all alike), a second pass copies them into LDS with their segments, and every
+// further level of both searches and the segments' masses read those (up to kFew of a bin need no further level: their
+// ranks say).  Then the segment that holds the drawn number is walked.  (Without the copies: seven passes and the
+// draw's with both thresholds.)  Where shares_rows says so the first pass and the copies are those of sample_hist and
+// sample_collect.
 __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     const float* __restrict__ logits, long ld, int V, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ top_p,
@@ -568,7 +577,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   __shared__ uint32_t few[kFew], few_count;
   __shared__ unsigned long long few_mass[kFew];
   __shared__ uint32_t few_cut;
-  __shared__ unsigned long long segment_mass[kArgmaxSegments];
+  __shared__ unsigned long long segment_mass[kSampleThreads / kWave][kArgmaxSegments];   // (a copy a wave: its lanes' additions meet nobody else's)
   __shared__ uint32_t cand_count;
   __shared__ int found_bin;
   __shared__ int last_token;
@@ -594,7 +603,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   uint32_t k_prefix = 0, k_remaining = (uint32_t)max(k, 0);
   uint32_t p_prefix = 0;               // only top-p: its first level is found by the first pass
   unsigned long long p_remaining = 0;
-  bool listed = false;                 // cand comes with its values' segments
+  bool listed = false;                 // what is kept and not in cand has its mass, segment by segment, in shared.above
+  bool whole_list = k_on && p_on;      // (all that is kept is in cand)
+  const int chunk = ((V + kArgmaxSegments - 1) / kArgmaxSegments + 3) & ~3;      // a segment of the argmax pass
   int ncand = -1;                      // >= 0: cand[0 .. ncand) hold every value that can be a threshold
   if (k_on || p_on) {
     const bool ready = shared.hist32 != nullptr;     // (the row's first pass is done)
@@ -634,11 +645,18 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
       ncand = (int)entries;
       listed = true;
     } else if (total <= (uint32_t)kCandidates) {
-      for_row(row, V, [&](int, float logit) {
+      for_row(row, V, [&](int i, float logit) {
         const uint32_t o = ordered(scaled(logit, inv_t));
-        if ((int)(o >> 20) >= low_bin) cand[atomicAdd(&cand_count, 1u)] = o;  // (in any order: the sums below are of integers)
+        if ((int)(o >> 20) >= low_bin) {
+          const uint32_t at = atomicAdd(&cand_count, 1u);  // (in any order: the sums below are of integers)
+          int seg = (int)((float)i * (1.f / (float)chunk));      // (within one of it)
+          seg += (long)(seg + 1) * chunk <= i ? 1 : (long)seg * chunk > i ? -1 : 0;
+          cand[at] = o;
+          cand_segment[at] = (uint8_t)seg;
+        }
       });
       ncand = (int)total;
+      listed = whole_list = true;
     }
     __syncthreads();
   }
@@ -762,7 +780,6 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   // Without a threshold the argmax pass has left their masses (relative to each segment's own maximum); with a list of
   // candidates what is kept is in the list; else a wave sums two segments of the row.
   const int lane = tid & (kWave - 1), wave = tid / kWave;
-  const int chunk = ((V + kArgmaxSegments - 1) / kArgmaxSegments + 3) & ~3;
   const auto kept_mass = [&](float logit) {
     const float x = scaled(logit, inv_t);
     return ordered(x) >= cut ? exp_unit(x - mx) : 0.f;
@@ -771,19 +788,20 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   __syncthreads();
   if (!k_on && !p_on) {
     if (tid < kArgmaxSegments) {
-      float run = 0.f;
-      for (int w = 0; w <= tid; ++w) {
-        const float m = seg_max[r * kArgmaxSegments + w];
-        run += m > -INFINITY ? seg_mass[r * kArgmaxSegments + w] * exp_unit(m * inv_t - mx) : 0.f;
-      }
-      upto[tid] = run;
+      const float m = seg_max[r * kArgmaxSegments + tid];
+      upto[tid] = m > -INFINITY ? seg_mass[r * kArgmaxSegments + tid] * exp_unit(m * inv_t - mx) : 0.f;
     }
+    __syncthreads();
+    if (tid == 0)
+      for (int w = 1; w < kArgmaxSegments; ++w) upto[w] += upto[w - 1];
   } else {
+    if (tid < kSampleThreads / kWave * kArgmaxSegments)
+      segment_mass[tid / kArgmaxSegments][tid % kArgmaxSegments] =
+          listed && !whole_list && tid < kArgmaxSegments ? shared.above[r * kArgmaxSegments + tid] : 0;
+    __syncthreads();
     if (listed) {
-      if (tid < kArgmaxSegments) segment_mass[tid] = k_on && p_on ? 0 : shared.above[r * kArgmaxSegments + tid];
-      __syncthreads();
       for (int i = tid; i < ncand; i += nt)
-        if (cand[i] >= cut) atomicAdd(&segment_mass[cand_segment[i]], draw_mass(unordered(cand[i]), mx, scale));
+        if (cand[i] >= cut) atomicAdd(&segment_mass[wave][cand_segment[i]], draw_mass(unordered(cand[i]), mx, scale));
     } else {
       for (int seg = wave; seg < kArgmaxSegments; seg += kSampleThreads / kWave) {
         const int begin = min(V, seg * chunk), end = min(V, begin + chunk);
@@ -809,14 +827,19 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
         }
 #pragma unroll
         for (int m = kWave / 2; m >= 1; m >>= 1) mine += __shfl_xor(mine, m, kWave);
-        if (lane == 0) segment_mass[seg] = mine;
+        if (lane == 0) segment_mass[0][seg] = mine;
       }
     }
     __syncthreads();
     if (tid < kArgmaxSegments) {
-      unsigned long long run = 0;      // (rounded once: as float32 numbers one after the other small segments beside a large one were lost)
-      for (int w = 0; w <= tid; ++w) run += segment_mass[w];
-      upto[tid] = (float)run / scale;
+      unsigned long long run = 0;
+      for (int w = 0; w < kSampleThreads / kWave; ++w) run += segment_mass[w][tid];
+#pragma unroll
+      for (int m = 1; m < kArgmaxSegments; m <<= 1) {
+        const unsigned long long other = __shfl_up(run, m, kArgmaxSegments);
+        if (tid >= m) run += other;
+      }
+      upto[tid] = (float)run / scale;      // (rounded once: as float32 numbers one after the other small segments beside a large one were lost)
     }
   }
   __syncthreads();
@@ -887,23 +910,31 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   }
 }
 
-constexpr int kSharedRows = 256;    // rows up to which a row with a threshold is shared between blocks (a block a CU from there on)
+// Whether a step's rows with thresholds are shared between blocks: two more kernels (some 8 us, and 0.3 us a row beside its
+// bytes) against passes of one block over its row alone, which all rows make side by side.  us with top-k / with top-p
+// alone, shared against a block a row: 151,936 logits, 1 row 30 / 40 against 44 / 95, 16 rows 34 / 51 and 45 / 106, 64 rows 61 / 88
+// and 61 / 125, 100 rows 84 / 117 and 66 / 130, 200 rows 136 / 187 and 78 / 151; 65,536 logits, 1 row 26 / 36 and 28 / 42, 16
+// rows 29 / 42 and 29 / 57, 64 rows 46 / 70 and 32 / 61; 32,003 logits, 1 row 25 / 30 and 22 / 27, 64 rows 44 / 64 and 25 / 41; 4,096
+// logits, 64 rows 40 / 52 and 19 / 21.
+constexpr int kSharedVocabulary = 65536;
+inline bool shares_rows(int M, int V) { return V >= kSharedVocabulary && M <= (V - kSharedVocabulary / 2) / 1536; }
 constexpr size_t kSharedWords = 3 * kBins + 2;     // of a row: counts, masses, the list's length
 
-TK_API int tk_sample_scratch_bytes(int M) {
+TK_API int tk_sample_scratch_bytes(int M, int V) {
   const long rows = M < 1 ? 0 : M;
   const long parts = rows * kArgmaxSegments * 12 + rows * 4 + 16;
-  return (int)(parts + (rows <= kSharedRows ? rows * ((long)kSharedWords * 4 + (long)kCandidates * 5 + kArgmaxSegments * 8) : 0));
+  return (int)(parts + (shares_rows(M, V) ? rows * ((long)kSharedWords * 4 + (long)kCandidates * 5 + kArgmaxSegments * 8) : 0));
 }
 
 // Every row's next token: greedy rows (temperature 0) their argmax, the others a draw; a row whose search falls through
-// (rounding at an edge) keeps its argmax.  scratch: tk_sample_scratch_bytes(M), on a 16-byte border.
+// (rounding at an edge) keeps its argmax.  scratch: tk_sample_scratch_bytes(M, V), on a 16-byte border.  thresholds: 0 where the
+// caller knows that no row has any; the kernels that share such rows are then left out.
 TK_API int tk_sample(const float* logits, long ld, int M, int V, const float* temperature,
                      const int* top_k, const float* top_p, const unsigned long long* seeds,
-                     const unsigned long long* counters, int* out, float* probs_out, void* scratch, hipStream_t stream) {
+                     const unsigned long long* counters, int* out, float* probs_out, void* scratch, int thresholds, hipStream_t stream) {
   if (M <= 0) return 0;
   if (V <= 0 || M > 65535 || scratch == nullptr || (uintptr_t)scratch % 16 != 0) return -1;
-  const bool share = M <= kSharedRows;
+  const bool share = shares_rows(M, V) && thresholds != 0;
   unsigned char* at = static_cast<unsigned char*>(scratch);
   SharedRows sh{};
   if (share) {      // (per row: 2 kBins words of masses, kBins of counts, two of the list's length)
@@ -911,7 +942,7 @@ TK_API int tk_sample(const float* logits, long ld, int M, int V, const float* te
     sh.hist32 = reinterpret_cast<uint32_t*>(at + (size_t)M * kBins * 8);
     sh.count = sh.hist32 + (size_t)M * kBins;
     sh.above = reinterpret_cast<unsigned long long*>(at + (size_t)M * kSharedWords * 4);
-    // (the words so far are cleared by the argmax pass; M times an odd number of 8 bytes: still on their border)
+    // (the argmax pass clears a row's words so far; M times an odd number of 8 bytes: still on their border)
     at += (size_t)M * (kSharedWords * 4 + kArgmaxSegments * 8);
   }
   float* seg_max = reinterpret_cast<float*>(at);
@@ -923,8 +954,7 @@ TK_API int tk_sample(const float* logits, long ld, int M, int V, const float* te
     sh.segment = reinterpret_cast<uint8_t*>(sh.cand + (size_t)M * kCandidates);
   }
   const dim3 shares(kArgmaxSegments, M);
-  argmax_segments_kernel<<<shares, kArgmaxThreads, 0, stream>>>(logits, seg_max, seg_index, V, ld, temperature, top_k, top_p, seg_mass,
-                                                                reinterpret_cast<uint32_t*>(sh.hist64), share ? kSharedWords : 0);
+  argmax_segments_kernel<<<shares, kArgmaxThreads, 0, stream>>>(logits, seg_max, seg_index, V, ld, temperature, top_k, top_p, seg_mass, sh);
   if (share) {
     sample_hist_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, V, temperature, top_k, top_p, seg_max, seg_index, out, row_max, sh);
     sample_collect_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, V, temperature, top_k, top_p, row_max, sh);

@@ -338,8 +338,8 @@ _SIGS = {
         "tk_argmax": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_long, c_void_p],
         "tk_argmax_segments": [],
         "tk_sample": [c_void_p, c_long, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
-                      c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
-        "tk_sample_scratch_bytes": [c_int],
+                      c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
+        "tk_sample_scratch_bytes": [c_int, c_int],
     },
 }
 _LIBRARY_FILE = {"attention_fused": "attention_mfma", "attention_pooled_split": "attention_pooled"}   # signature group -> library that holds it
@@ -2331,8 +2331,9 @@ def argmax(logits: torch.Tensor, out: torch.Tensor, values: torch.Tensor | None 
 
 def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
            top_p: torch.Tensor, seeds: torch.Tensor, counters: torch.Tensor, out: torch.Tensor,
-           probs_out: torch.Tensor | None = None) -> None:
-    """Temperature / top-k / top-p sampling, one row per request."""
+           probs_out: torch.Tensor | None = None, thresholds: bool = True) -> None:
+    """Temperature / top-k / top-p sampling, one row per request.  ``thresholds``: whether any row may have a top-k or
+    top-p that leaves tokens out; without, two launches that share such rows between blocks are left out."""
     _need(logits.is_cuda and logits.dim() == 2 and logits.stride(1) == 1 and logits.dtype == torch.float32,
           "logits are float32 [M, V] on the GPU")
     _gpu(temperature, top_k, top_p, seeds, counters, out, probs_out)
@@ -2345,7 +2346,8 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
     _need(out.dtype == torch.int32, "sample output is int32")
     _need(probs_out is None or (probs_out.dtype == torch.float32 and probs_out.shape == (m, v)), "probs_out is float32 [M, V]")
     _need(m <= 65535, "at most 65535 rows")
-    scratch = torch.empty(_fn("sampling", "tk_sample_scratch_bytes")(m), dtype=torch.uint8, device=logits.device)
+    scratch = torch.empty(_fn("sampling", "tk_sample_scratch_bytes")(m, v), dtype=torch.uint8, device=logits.device)
     _check(_fn("sampling", "tk_sample")(_p(logits), logits.stride(0), m, v, _p(temperature), _p(top_k),
-                                        _p(top_p), _p(seeds), _p(counters), _p(out), _p(probs_out), _p(scratch), _stream()),
+                                        _p(top_p), _p(seeds), _p(counters), _p(out), _p(probs_out), _p(scratch),
+                                        int(bool(thresholds)), _stream()),
            "sample")

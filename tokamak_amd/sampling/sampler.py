@@ -66,5 +66,6 @@ def sample_tokens(logits: torch.Tensor, params: list[SamplingParams], seeds: lis
     top_k = packed[6 * m:]
     out = _output(out, m, dev)
     probs = torch.zeros_like(logits) if return_probs else None
-    ops.sample(logits, temperature, top_k, top_p, seed_t, draw_t, out, probs)
+    thresholds = any(p.top_p < 1.0 or 0 < p.top_k < logits.shape[1] for p in params if not p.is_greedy)
+    ops.sample(logits, temperature, top_k, top_p, seed_t, draw_t, out, probs, thresholds)
     return (out, probs) if return_probs else out
