@@ -220,13 +220,16 @@ constexpr int SBK = 256;        // k per chunk
 // products (sched_group_barrier below).  With one row tile the plain loop is kept: the read-ahead
 // gains nothing there and cost the two-wave gated product of a 14B-shaped layer 8 % (63 -> 68 us).
 constexpr int READ_AHEAD_FROM = 2;
-constexpr int SPC = SBK / 8;    // pieces of eight k of a row's chunk
 
 // Where piece c of row `row` of a tile of 16 rows lies in LDS, in pieces: [c][row ^ (c & 15)].  A loader's lanes write
 // neighbouring pieces of a row, an operand's lanes read one piece of 16 rows (and the next three pieces): either
 // way the pieces that LDS serves together lie in different banks, however it groups the lanes.  (Rows 264
-// elements apart instead: a third of the LDS cycles of the product of 64 rows were conflicts.)
-__device__ __forceinline__ int lds_piece(int c, int row) { return c * 16 + (row ^ (c & 15)); }
+// elements apart instead: 64 rows of activations take 2 to 5 % longer, 96 and 128 rows 4 to 7 %.)
+// The gated product of up to 16 rows keeps its rows 264 elements apart (not EXCHANGED): its reads are so few that conflicts do
+// not show, and one base with constant offsets leaves the compiler 40 registers and the SIMD a third wave (two-wave blocks
+// of a 14B-shaped layer, 17,408 columns of 5,120, 1 row: 63.5 us, exchanged 69).
+template <bool EXCHANGED>
+__device__ __forceinline__ int lds_piece(int row, int c) { return EXCHANGED ? (c * 16 + (row ^ (c & 15))) * 8 : row * (SBK + 8) + c * 8; }
 
 // GATED: W is [2N, K], gate rows then up rows; the block owns 8*WAVES output columns, the
 // first half of its waves their gate rows and the second half the matching up rows, and
@@ -279,8 +282,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
   // i + 1 while others still read chunk i): 3-6 % for blocks of eight waves, which have a CU to
   // themselves anyway; nothing at up to 16 rows, and blocks of four would lose a place on the CU.
   constexpr int XBUF = (WAVES >= 6 && MT >= 2 && MT <= 4) ? 2 : 1;  // (five row tiles and more: one copy fits beside the weights)
-  __shared__ u32x4 ws[WAVES][SPC * 16];
-  __shared__ u32x4 xs[XBUF][MT][SPC * 16];
+  constexpr bool EXCHANGED = !(GATED && MT == 1);
+  constexpr int TILE = 16 * (SBK + (EXCHANGED ? 0 : 8));      // elements a tile of 16 rows takes
+  __shared__ __attribute__((aligned(16))) bf16_t ws[WAVES][TILE];
+  __shared__ __attribute__((aligned(16))) bf16_t xs[XBUF][MT][TILE];
+  const auto x_piece = [&](int copy, int row) {      // where this thread's piece of a row of the activations goes
+    return MT == 1 ? &xs[copy][0][lds_piece<EXCHANGED>(row, threadIdx.x & 31)]
+                   : &xs[copy][row / 16][lds_piece<EXCHANGED>(row & 15, threadIdx.x & 31)];
+  };
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, kb = lane >> 4;
   const int row_block = blockIdx.x, split = blockIdx.y;
@@ -348,12 +357,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
     const int xb_ = XBUF == 2 ? ((I_) & 1) : 0;                                                     \
     if (XBUF == 1) __syncthreads(); /* the previous chunk's fragments have been read */             \
     _Pragma("unroll") for (int i = 0; i < 8; ++i)                                                   \
-        ws[wave][lds_piece(lane & 31, 2 * i + w_row0)] = wreg[i];                                   \
+        *reinterpret_cast<u32x4*>(&ws[wave][lds_piece<EXCHANGED>(2 * i + w_row0, lane & 31)]) = wreg[i]; \
     {                                                                                               \
       const bool inside_ = cur_ * SBK + x_col < K;                                                  \
       _Pragma("unroll") for (int i = 0; i < XP; ++i)                                                \
         if (XWHOLE || i * (THREADS / 32) + x_row0 < 16 * MT)                                        \
-          xs[xb_][(i * (THREADS / 32) + x_row0) / 16][lds_piece(tid & 31, (i * (THREADS / 32) + x_row0) & 15)] = inside_ ? xreg[i] : zero; \
+          *reinterpret_cast<u32x4*>(x_piece(xb_, i * (THREADS / 32) + x_row0)) = inside_ ? xreg[i] : zero; \
     }                                                                                               \
     __syncthreads();                                                                                \
     if ((I_) + 1 < nchunks) {                                                                       \
@@ -364,9 +373,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
     if constexpr (MT < READ_AHEAD_FROM || MT > 4) { /* (more row tiles: no registers for two steps' fragments) */ \
       _Pragma("unroll") for (int s = 0; s < SBK / 32; ++s) {                                        \
         Frag8 wf, xf[MT];                                                                           \
-        wf.u = *reinterpret_cast<const uint4*>(&ws[wave][lds_piece(s * 4 + kb, r)]);                \
+        wf.u = *reinterpret_cast<const uint4*>(&ws[wave][lds_piece<EXCHANGED>(r, s * 4 + kb)]);                \
         _Pragma("unroll") for (int j = 0; j < MT; ++j)                                              \
-            xf[j].u = *reinterpret_cast<const uint4*>(&xs[xb_][j][lds_piece(s * 4 + kb, r)]);       \
+            xf[j].u = *reinterpret_cast<const uint4*>(&xs[xb_][j][lds_piece<EXCHANGED>(r, s * 4 + kb)]);       \
         _Pragma("unroll") for (int j = 0; j < MT; ++j)                                              \
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf.v, xf[j].v, acc[j], 0, 0, 0);       \
       }                                                                                             \
@@ -375,9 +384,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
       /* wave that waits for each fragment in turn spends its time on round trips to LDS         */ \
       Frag8 wf[SBK / 32], xf[SBK / 32][MT];                                                         \
       _Pragma("unroll") for (int s = 0; s < SBK / 32; ++s) {                                        \
-        wf[s].u = *reinterpret_cast<const uint4*>(&ws[wave][lds_piece(s * 4 + kb, r)]);             \
+        wf[s].u = *reinterpret_cast<const uint4*>(&ws[wave][lds_piece<EXCHANGED>(r, s * 4 + kb)]);             \
         _Pragma("unroll") for (int j = 0; j < MT; ++j)                                              \
-            xf[s][j].u = *reinterpret_cast<const uint4*>(&xs[xb_][j][lds_piece(s * 4 + kb, r)]);    \
+            xf[s][j].u = *reinterpret_cast<const uint4*>(&xs[xb_][j][lds_piece<EXCHANGED>(r, s * 4 + kb)]);    \
       }                                                                                             \
       _Pragma("unroll") for (int s = 0; s < SBK / 32; ++s)                                          \
         _Pragma("unroll") for (int j = 0; j < MT; ++j)                                              \
