@@ -1528,14 +1528,21 @@ def moe_down(act: torch.Tensor, down: torch.Tensor, chosen: torch.Tensor, out: t
 
 
 MOE_STREAM_MAX_PAIRS = 1024    # pairs a block of the streaming form can list (csrc/moe_operands.hip: kMaxPairs)
-# pairs an expert has on average up to which the streaming form is taken, and the same for small experts (width times
-# ff up to MOE_STREAM_SMALL).  Both products, streamed against tiles with the kernel that lists them (some 6 us; 16
-# experts, two a token): 4,096 x 6,144 at 5 pairs an expert 277 + 147 against 274 + 146 us, at 16 333 + 198 against
-# 279 + 181; 1,024 x 1,024 at 16 20 + 14 against 26 + 19, at 32 30 + 19 against 30 + 22; 1,024 x 1,536 at 16 27 + 21
-# against 27 + 29, at 32 43 + 27 against 30 + 31
-MOE_STREAM_PER_EXPERT = 5
-MOE_STREAM_PER_SMALL_EXPERT = 24
-MOE_STREAM_SMALL = 1 << 21
+# pairs an expert has on average up to which the streaming form is taken, by an expert's size (width times ff), and the
+# most pairs.  Both products, streamed / in tiles with the kernel that lists them (some 6 us), us; pairs an expert:
+#   16 experts, two a token   5          8          12         16         24         32
+#   4,096 x 6,144             425 / 425  449 / 459  486 / 459  528 / 466
+#   4,096 x 4,096             300 / 321  315 / 340  340 / 341  372 / 345
+#   2,048 x 4,096             167 / 195  173 / 196  183 / 195  202 / 199  238 / 200
+#   2,048 x 2,048              95 / 103   98 / 112  103 / 112  107 / 115  132 / 119
+#   1,024 x 3,072              68 / 103   70 / 103   75 / 103   81 / 103  117 / 105
+#   1,024 x 1,024              29 / 50    31 / 51    32 / 51    34 / 51    45 / 52    50 / 56
+#   64 experts, four a token
+#   2,048 x 1,024             170 / 177  179 / 179  201 / 180  224 / 181
+#   1,024 x 512                58 / 67    60 / 65    66 / 67    76 / 67
+MOE_STREAM_PER_EXPERT = ((1 << 20, 32), (1 << 22, 16), (1 << 24, 12))
+MOE_STREAM_PER_LARGE_EXPERT = 5
+MOE_STREAM_PAYS_PAIRS = 512
 
 
 def expert_operands(matrices: torch.Tensor) -> torch.Tensor:
@@ -1560,8 +1567,8 @@ def moe_stream_fits(width: int, ff: int, experts: int, pairs: int) -> bool:
     channels (``moe_stream``), rather than once a tile of 128 pairs (``moe_tiles``): so few pairs that the
     weights' bytes are the work.  Beyond 64 pairs every expert has blocks, met or not, so there must not be more
     experts than pairs."""
-    most = MOE_STREAM_PER_SMALL_EXPERT if width * ff <= MOE_STREAM_SMALL else MOE_STREAM_PER_EXPERT
-    return pairs <= MOE_STREAM_MAX_PAIRS and (pairs <= 64 or experts <= pairs <= most * experts)
+    most = next((per for size, per in MOE_STREAM_PER_EXPERT if width * ff <= size), MOE_STREAM_PER_LARGE_EXPERT)
+    return pairs <= 64 or experts <= pairs <= min(MOE_STREAM_PAYS_PAIRS, most * experts)
 
 
 def _expert_product(x, weights, pair_weight, out, tokens: int, top: int, gated: bool) -> tuple[int, int, int]:
