@@ -258,7 +258,7 @@ def clear_of(h, w, top, n):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("width,ff,n,top", [(64, 32, 4, 2), (48, 24, 12, 1), (72, 40, 5, 5), (36, 20, 7, 3), (256, 136, 3, 2),
-                                            (128, 192, 2, 1)])
+                                            (128, 192, 2, 1), (72, 192, 2, 1), (128, 136, 2, 1)])
 def test_routed_experts_alone(dtype, width, ff, n, top):
     """Numbers of experts that are no power of two, one expert a token, every expert a token, sizes
     that do not fill 16-byte pieces; the rows whose choice of experts is no close call are compared."""
@@ -271,7 +271,9 @@ def test_routed_experts_alone(dtype, width, ff, n, top):
     assert set(part.expected_tensors("l0.mlp.")) == {k for k in w if k.startswith("l0.mlp.")}
     part.bind("l0.mlp.", fetcher(w, dtype))
     g = torch.Generator().manual_seed(3)
-    rows = 70 if n > 2 else 500         # (two experts and 500 tokens, K in chunks of 64: full tiles, their activations through LDS)
+    # two experts and 500 tokens: full tiles.  Both sizes multiples of 64: weights in operand order (bfloat16); one of them: that
+    # product has its K in chunks of 64, activations through LDS, with weights in rows
+    rows = 70 if n > 2 else 500
     h = torch.randn(rows, width, generator=g).to(dtype)
     want = plain.routed_experts(h.double(), double(w), "l0.mlp.", cfg["layers"][0]["mlp"]).float()
     got = part.forward(h.to(DEV), make_batch([(rows, 0, [0])]))

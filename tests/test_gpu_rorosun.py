@@ -46,6 +46,10 @@ SHAPES = {
     "ones": dict(cfg=model_json([layer(heads=5, kv_heads=1, dim=8, vdim=8, window=1, pool=1, r_heads=1, r_dim=64, ff=40),
                                  layer(heads=2, kv_heads=1, dim=64, vdim=32, window=5, pool=16, r_heads=2, r_dim=33, ff=None)],
                                 vocab=97, width=36, eps=1e-4), rank=6, page=16),
+    # heads and channels of the presets' attention: bfloat16 steps on the matrix cores
+    "tiles": dict(cfg=model_json([layer(heads=16, kv_heads=8, dim=64, vdim=64, window=21, pool=4),
+                                  layer(heads=32, kv_heads=8, dim=64, vdim=128, window=9, pool=5, r_heads=4, r_dim=16)]),
+                  rank=8, page=16),
 }
 
 
@@ -57,6 +61,15 @@ def models(tmp_path_factory):
         w = random_weights(spec["cfg"], seed=len(name), rank=spec["rank"])
         out[name] = (write_folder(root / name, spec["cfg"], w), spec["cfg"], w, spec["page"])
     return out
+
+
+def test_the_shape_for_the_matrix_cores_is_taken_there():
+    from tokamak_amd.kernels import ops
+
+    for name, spec in SHAPES.items():
+        left = [entry["mixer"]["left"] for entry in spec["cfg"]["layers"]]
+        taken = [ops.pooled_portions_pay(a["heads"], a["kv_heads"], a["dim"], a["vdim"], spec["page"]) for a in left]
+        assert taken == [name == "tiles"] * len(left)
 
 
 def runner_for(models, name, dtype, pool_tokens=1024, max_requests=4, **kw):
@@ -318,11 +331,12 @@ def test_window_and_pool_edges_show(tmp_path):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-def test_long_decoding_through_recorded_steps(models, dtype):
+@pytest.mark.parametrize("name", ["base", "tiles"])
+def test_long_decoding_through_recorded_steps(models, name, dtype):
     """One prompt token, then 260 tokens one by one (the recorded step of each shape replayed
     many times, two requests side by side at different lengths); and the same without recorded
     steps and without recorded layers gives the same bits."""
-    runner, cfg, w = runner_for(models, "base", dtype)
+    runner, cfg, w = runner_for(models, name, dtype)
     assert runner.use_graphs
     a, b = tokens(cfg["vocab"], 261, 11), tokens(cfg["vocab"], 200, 12)
     expected = expected_for(cfg, w, {"a": a, "b": b}, dtype)
@@ -335,7 +349,7 @@ def test_long_decoding_through_recorded_steps(models, dtype):
     got = run_steps(runner, steps)
     worst, where = worst_error(steps, got, expected)
     assert worst <= LIMIT[dtype], (dtype, worst, where)
-    plain_runner, _, _ = runner_for(models, "base", dtype, use_graphs=False)
+    plain_runner, _, _ = runner_for(models, name, dtype, use_graphs=False)
     plain_runner.model.replay_layers = False
     again = run_steps(plain_runner, steps)
     for step in got:
