@@ -195,7 +195,8 @@ __device__ __forceinline__ void tile_scores(const Args& a, const Tile& t, int et
 }
 
 // Four waves take a share's tiles of 16 entries in turn.  A key tile is read once for four heads and sixteen rows.
-// Bound by the vector unit (an exponential, a mask and a maximum a score): 82 us at 2,048 rows of 32 / 8 heads of 128.
+// The vector unit most (60 % of the time busy: an exponential, a mask and a maximum a score; the matrix units 16 %): 82 us
+// at 2,048 rows of 32 / 8 heads of 128.
 template <int KS, int KVQ>
 __global__ __launch_bounds__(256) void portion_stats_kernel(Args a) {
   __shared__ float red[4][4][kRows][2];
@@ -254,9 +255,9 @@ __global__ __launch_bounds__(256) void portion_stats_kernel(Args a) {
 
 // H / 4 waves, a wave four heads.  A chunk: every wave's normalised weights of 16 rows by 32 entries, float32, into LDS
 // [row][entry][head] (two copies, one barrier a chunk), then a wave mixes whole rows: D = talk (32 heads by H) times
-// the row's weights (H by 32 entries), whose pieces are split as they are read.  153 us for 2,048 rows of 32 heads of
-// 128 over 1,024 tokens and up to 130 blocks (147 with two pieces a weight): an exponential, a split and a packing of
-// every weight, then 300 MB of weights written.
+// the row's weights (H by 32 entries), whose pieces are split as they are read.  154 us for 2,048 rows of 32 heads of
+// 128 over 1,024 tokens and up to 130 blocks (147 with two pieces a weight): vector units 44 % busy (an exponential and a
+// split of every weight), matrix units 17 %, a quarter of the waves' time waits, 300 MB of weights written.
 template <int KS, int KVQ, int H>
 __global__ __launch_bounds__(16 * H) void portion_weights_kernel(Args a) {
   constexpr int kWaves = H / 4, kMix = H / 16;
@@ -364,8 +365,8 @@ __global__ __launch_bounds__(16 * H) void portion_weights_kernel(Args a) {
 // Four waves take a share's chunks in turn: D = mixed weights (16 rows by 32 entries) times values (32 entries by
 // channels), four heads.  A lane reads VT neighbouring channels of eight entries, which are the VT channel tiles' operands
 // once their halves are paired (column n of tile c is channel VT n + c), so values need no LDS.  169 us at the same
-// sizes (159 with two pieces a weight), 300 MB of weights read once and the values by every tile from L2; on the vector
-// unit it was 1.2 ms.
+// sizes (157 with two pieces a weight): one wave a SIMD, vector units 39 % and matrix units 18 % busy, 300 MB of weights
+// read once and the values by every tile from L2; on the vector unit it was 1.2 ms.
 template <int VT, int KVQ>
 __global__ __launch_bounds__(256) void portion_values_kernel(Args a) {
   constexpr int vdim = 16 * VT, per = 4 / KVQ;

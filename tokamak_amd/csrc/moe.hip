@@ -10,8 +10,8 @@
 //   gate(w h) = w gate(h), the weight is applied to the two products in float32 before the
 //   activation.  moe_down writes every pair's result to its own row of a float32 array
 //   [top][tokens][width]; the kernel that reads it next (the norm that adds a sub-layer's output
-//   to the stream) sums the `top` layers in order, so a token's result does not depend on what
-//   else is in the step.
+//   to the stream) sums the `top` layers in order: which of these forms and those of moe_operands.hip a step
+//   takes, and so the order of a pair's sums over k, follows how many pairs the step has, never which.
 // moe_sort / moe_grouped, the form for many tokens in bfloat16: the (token, expert) pairs are
 //   counted and listed expert by expert and cut into tiles of up to 64 pairs of one expert; a
 //   block takes a tile and 128 or 256 output channels on the matrix cores (v_mfma_f32_16x16x32_bf16;

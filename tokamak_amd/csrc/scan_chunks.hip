@@ -20,9 +20,10 @@
 //   chunk_finish: norm, gain, gate.
 //
 // Walked a token at a time a token costs a chain of some 0.5 to 0.7 us; a chunk of 16 costs a chain of two short matrix
-// products and a barrier.  2,048 tokens: gla, 32 heads of 128 x 128, 1.45 ms -> 72 + 111 + 12 us; wkv, 64 heads of 64 x
-// 64, 1.10 ms -> 63 + 61 + 12.  The operands kernel is bound by its bytes (in 50 MB, out 105), the walk by its
-// chain (0.9 us a chunk of 128 x 16 state a block: 17 matrix instructions of 32 cycles a wave, LDS, barrier).  Everything
+// products and a barrier.  2,048 tokens: gla, 32 heads of 128 x 128, 1.45 ms -> 68 + 111 + 23 us; wkv, 64 heads of 64 x
+// 64, 1.10 ms -> 61 + 70 + 23.  The operands kernel of gla is bound by the vector unit (85 % of its time busy: logarithms and
+// exponentials), of wkv by neither (45 %; in 33 MB, out 105); the walk by its chain (0.9 us a chunk of 128 x 16 state a
+// block: 17 matrix instructions of 32 cycles a wave, LDS, barrier; matrix units 29 % busy, vector 20 %).  Everything
 // is float32, the products are those of the float32 matrix instruction (16 x 16 x 4); its k index may name any four
 // channels as long as both operands agree, so index g of step r is channel 4 g + r: a lane's operands are then
 // the parts of one 16-byte load, and the state's accumulators are an operand as they are.

@@ -951,8 +951,10 @@ POOLED_PORTION_BLOCKS = 512  # blocks of four waves wanted: two a CU
 def pooled_portions_pay(num_heads: int, num_kv_heads: int, dim: int, vdim: int, page_size: int) -> bool:
     """Whether the pooled-window attention of a bfloat16 step runs on the matrix cores
     (``attention_pooled_portions.hip``): sizes that its kernels are built for.  Single tokens fill a sixteenth of a
-    tile and gain all the same: three of them over 3,100 positions, 32 / 8 heads of 128, a
-    layer's 82 us became 50 (scores, mixing and values on the vector unit before)."""
+    tile and gain all the same at every count and length (us there / in the general form; 32 / 8 heads of 128 with a
+    window of 1,024: one token over 100 positions 32 / 62, over 8,000 43 / 80, sixteen over 200 39 / 69, over 4,000 90 /
+    158, 64 over 60 35 / 71, over 1,000 144 / 404; 16 / 8 heads of 64, window 512: one over 100 31 / 38, 64 over 60 29 /
+    42, over 4,000 79 / 200).  Portions: eight of 5 tokens over 200 32 / 134, one of 2,048 over 2,000 393 / 3,249."""
     group = num_heads // num_kv_heads
     return (num_heads in (16, 32) and (group in (1, 2) or group % 4 == 0) and dim in (64, 128)
             and vdim in (64, 128) and page_size % 16 == 0 and not POOLED_ONE_KERNEL_ONLY)
