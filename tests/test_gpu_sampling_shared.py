@@ -1,5 +1,5 @@
-"""A step's rows with thresholds are shared between blocks up to 256 rows; with more a block takes a row.  Both must choose the
-same tokens: thresholds and the draws' masses are sums of integers."""
+"""A step's rows with thresholds are shared between blocks where the vocabulary is large (65,536 and more) and the rows are
+few; else a block takes a row.  Both must choose the same tokens: thresholds and the draws' masses are sums of integers."""
 
 import pytest
 import torch
