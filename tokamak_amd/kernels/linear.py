@@ -21,10 +21,12 @@ import torch
 from tokamak_amd.kernels import ops
 
 
-# A product adds into the stream itself (one block walking the whole of K for 16 columns)
+# From nine rows on a product adds into the stream itself (one block walking the whole of K for 16 columns)
 # only if K is short: up to one chunk of 256 for each of a block's sixteen waves.  With a
 # longer K the split product and the norm kernel after it are as fast (measured: the o
-# projection of an 8B-shaped layer gains 2 us, its down projection nothing).
+# projection of an 8B-shaped layer gains 2 us, its down projection nothing).  Where the direct product is
+# the faster form it adds at any K (down of an 8B-shaped layer at 8 rows: 20.3 us, split product and norm 21.3;
+# at one row 16.7 against 20.6).
 ADD_INTO_MAX_K = 16 * 256
 GATED_SPLIT_UP_TO_BLOCKS = 160      # blocks of the gated streaming product up to which K is split instead, the gate behind it
 GATED_WHOLEK_MAX_BYTES = 32 << 20   # gate and up together, up to which the whole-K form takes the gated product
@@ -103,6 +105,9 @@ def linear(x: torch.Tensor | DeferredNorm, weight: torch.Tensor, out_dtype: torc
     out_dtype = out_dtype or x.dtype
     m, n = x.shape[0], weight.shape[0]
     if isinstance(x, DeferredNorm):
+        if _few_rows_fit(m, x.scaled, weight, ops.DIRECT_MAX_ROWS) and ops.direct_pays(
+                "norm" if allow_partials else "plain", m, n, weight.shape[1]):
+            return _direct(x.scaled, weight, out_dtype, allow_partials, x.sumsq, x.eps)
         if (_few_rows_fit(m, x.scaled, weight, ops.ROW_SCALE_MAX_ROWS) and n >= gemm_bf16.STREAM_MIN_ROWS_OUT
                 and x.sumsq.shape[0] <= ops.ROW_SCALE_MAX_SLABS):
             splits = gemm_bf16.stream_splits(n, weight.shape[1], m) if allow_partials else 1
@@ -119,11 +124,24 @@ def linear(x: torch.Tensor | DeferredNorm, weight: torch.Tensor, out_dtype: torc
         out = torch.empty((m, n), dtype=out_dtype, device=x.device)
         ops.gemm_tiled(x, weight, out)
         return out
-    if (add_into is not None and weight.shape[1] <= ADD_INTO_MAX_K and _few_rows_fit(m, x, weight, ops.WHOLEK_MAX_ROWS)
-            and _sink_fits(add_into, m, n)):
-        sumsq, scaled = ops.gemm_wholek_add(x, weight, add_into.resid, add_into.gamma)
-        return Added(sumsq, scaled, add_into.gamma)
+    if add_into is not None and _few_rows_fit(m, x, weight, ops.WHOLEK_MAX_ROWS) and _sink_fits(add_into, m, n):
+        if weight.shape[1] <= ADD_INTO_MAX_K:
+            return Added(*ops.gemm_wholek_add(x, weight, add_into.resid, add_into.gamma), add_into.gamma)
+        if ops.direct_pays("add", m, n, weight.shape[1]):
+            return Added(*ops.gemm_direct_add(x, weight, add_into.resid, add_into.gamma), add_into.gamma)
+    if _few_rows_fit(m, x, weight, ops.DIRECT_MAX_ROWS) and ops.direct_pays("parts" if allow_partials else "plain", m, n, weight.shape[1]):
+        return _direct(x, weight, out_dtype, allow_partials)
     return gemm_bf16.gemm(x, weight, out_dtype, allow_partials)
+
+
+def _direct(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, allow_partials: bool,
+            sumsq: torch.Tensor | None = None, eps: float = 0.0) -> torch.Tensor:
+    """The direct product; where the reader adds partial sums, one float32 sum [1, M, N] (what the split product
+    would leave in several)."""
+    m, n = x.shape[0], weight.shape[0]
+    out = torch.empty((m, n), dtype=torch.float32 if allow_partials else out_dtype, device=x.device)
+    ops.gemm_direct(x, weight, out, sumsq=sumsq, eps=eps)
+    return out[None] if allow_partials else out
 
 
 def _sink_fits(sink: StreamSink, m: int, n: int) -> bool:
@@ -150,7 +168,9 @@ def activated_linear(x: torch.Tensor, weight: torch.Tensor, activation: str = "s
     out = torch.empty((m, n), dtype=x.dtype, device=x.device)
     if m == 0:
         return out
-    if (x.dtype == torch.bfloat16 and m <= gemm_bf16.SKINNY_MAX_ROWS and n >= gemm_bf16.STREAM_MIN_ROWS_OUT
+    if _few_rows_fit(m, x, weight, ops.DIRECT_MAX_ROWS) and ops.direct_pays("plain", m, n, k):
+        ops.gemm_direct(x, weight, out, activation=activation)
+    elif (x.dtype == torch.bfloat16 and m <= gemm_bf16.SKINNY_MAX_ROWS and n >= gemm_bf16.STREAM_MIN_ROWS_OUT
             and gemm_bf16.skinny_fits(x, weight) and gemm_bf16.stream_splits(n, k, m) < ACTIVATED_SPLIT_FROM):
         ops.gemm_stream(x, weight, out, activation=activation)
     else:
@@ -192,19 +212,19 @@ def gated_linear(x: torch.Tensor | DeferredNorm, gate_up: torch.Tensor, activati
         from tokamak_amd.kernels import gemm_bf16
 
         if x.dtype == torch.bfloat16 and m <= 64 and gemm_bf16.skinny_fits(x, gate_up):
-            if not _gated_split(x, gate_up, out, activation, limit):
+            if ops.direct_pays("gated", m, out.shape[1], x.shape[1]) or not _gated_split(x, gate_up, out, activation, limit):
                 ops.gemm_stream_swiglu(x, gate_up, out, activation=activation, limit=limit)
         else:
             ops.silu_mul(linear(x, gate_up), out, activation, limit=limit)
         return out
     inter = gate_up.shape[0] // 2
-    # A very small pair of matrices (0.6B-shaped: 13 MB) goes to the whole-K form, whose blocks of 16
-    # columns let their waves split K, which the streaming kernel cannot do under the gate: in a
-    # decode step 6.6 us against 8.6 with blocks of four waves and 7.8 with blocks of two (whose start
-    # costs more than their size saves there); from 50 MB on the streaming kernel is ahead.
+    # A small pair of matrices goes to the whole-K form, whose blocks of 16 columns let their waves split K, which
+    # the streaming kernel cannot do under the gate; from 50 MB on the streaming kernel is ahead.  (Both
+    # hand over to the direct product where it is the faster form, ops.direct_pays: up to eight rows and for the smallest pairs.)
     small = 2 * gate_up.numel() <= GATED_WHOLEK_MAX_BYTES
     if isinstance(x, DeferredNorm):
-        if _few_rows_fit(m, x.scaled, gate_up, ops.ROW_SCALE_MAX_ROWS) and x.sumsq.shape[0] <= ops.ROW_SCALE_MAX_SLABS:
+        if _few_rows_fit(m, x.scaled, gate_up, ops.ROW_SCALE_MAX_ROWS) and (
+                x.sumsq.shape[0] <= ops.ROW_SCALE_MAX_SLABS or ops.direct_pays("gated", m, inter, gate_up.shape[1])):
             out = torch.empty((m, inter), dtype=x.dtype, device=x.device)
             if small and m <= ops.WHOLEK_MAX_ROWS:
                 ops.gemm_wholek(x.scaled, gate_up, out, gated=True, sumsq=x.sumsq, eps=x.eps)
@@ -221,7 +241,7 @@ def gated_linear(x: torch.Tensor | DeferredNorm, gate_up: torch.Tensor, activati
         if gemm_bf16.skinny_fits(x, gate_up):
             if small and _few_rows_fit(m, x, gate_up, ops.WHOLEK_MAX_ROWS):
                 ops.gemm_wholek(x, gate_up, out, gated=True)
-            elif small or not _gated_split(x, gate_up, out, activation, limit):
+            elif small or ops.direct_pays("gated", m, inter, x.shape[1]) or not _gated_split(x, gate_up, out, activation, limit):
                 ops.gemm_stream_swiglu(x, gate_up, out)
             return out
     ops.silu_mul(linear(x, gate_up), out)

@@ -267,6 +267,12 @@ _SIGS = {
         "tk_gemm_wholek_add": [c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_void_p, c_long, c_void_p,
                                c_void_p, c_long, c_void_p, c_int, c_void_p],
     },
+    "gemm_direct": {
+        "tk_gemm_direct": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long,
+                           c_void_p, c_int, c_float, c_int, c_float, c_int, c_int, c_int, c_void_p],
+        "tk_gemm_direct_add": [c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_void_p, c_long, c_void_p,
+                               c_void_p, c_long, c_void_p, c_int, c_int, c_int, c_void_p],
+    },
     "blas_lt": {
         "tk_lt_gemm": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p,
                        c_size_t, c_int, c_void_p],
@@ -1853,6 +1859,10 @@ def gemm_stream_swiglu(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, w
     m, k = a.shape
     _need(w.shape[0] % 2 == 0 and w.shape[1] == k and out.shape == (m, w.shape[0] // 2), "gated product shapes disagree")
     _need(a.dtype == w.dtype == out.dtype == torch.bfloat16, "the gated product is bfloat16")
+    if (not waves and direct_pays("gated", m, w.shape[0] // 2, k) and k >= 8 and k % 8 == 0 and a.stride(0) % 8 == 0
+            and w.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and m > 0):
+        gemm_direct(a, w, out, sumsq=sumsq, eps=eps, gated=True, activation=activation, limit=limit)
+        return
     waves = waves or stream_waves(m, k, True, w.shape[0] // 2)
     _need(0 < m <= 64 and k >= 8 and k % 8 == 0 and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
           and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0, "gated product needs M <= 64 and 16-byte aligned rows")
@@ -1864,9 +1874,143 @@ def gemm_stream_swiglu(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, w
                                                      float(limit or 0.0), _stream()), "gemm_stream_swiglu")
 
 
+DIRECT_MAX_ROWS = 16    # rows of activations that the direct product takes
+
+
+def direct_plan(m: int, n: int, k: int, gated: bool = False, most_slabs: int = 0) -> tuple[int, int, int]:
+    """(rows of a group, groups of as many columns a block, waves a block) of the direct product.
+
+    Up to four rows of activations a group has four (pieces of 256 bytes a load), up to sixteen eight; five to eight rows
+    with so few columns that groups of eight leave CUs idle take groups of four and two tiles of activations (1,024 x
+    3,072: 4.8 us against 5.3).  More groups a block read the activations less often but leave fewer blocks: the
+    price of a CU's share, (rounds of 256 blocks) * groups * (1 + x / groups), with x a group's activations against its
+    weights, is within 6 % of the best of every form on the projections of 0.6B to 8B models; four groups have half as many
+    loads in flight, hence the tenth on them.  Eight waves, unless three blocks and more run on a CU.
+    ``most_slabs`` (0: any): the most blocks whose sums of squares the reader takes."""
+    rows = 4 if m <= 4 or (m <= 8 and n <= 1024) else 8
+    if rows == 4 and m > 4:
+        return 4, 1, 8
+    share = (0.25 if rows == 4 else 0.1) * m
+
+    def price(groups: int) -> float:
+        rounds = -(-(-(-n // (rows * groups))) // STREAM_CUS)
+        return rounds * (groups + share) * (1.1 if groups == 4 else 1.0)
+
+    forms = [g for g in ((1, 2, 4) if rows == 4 else (1, 2))]
+    fitting = [g for g in forms if not most_slabs or -(-n // (rows * g)) <= most_slabs] or forms[-1:]
+    groups = min(fitting, key=lambda g: (price(g), -g))
+    blocks = -(-n // (rows * groups))
+    return rows, groups, 8 if blocks <= 2 * STREAM_CUS else 4
+
+
+DIRECT_MIDDLE_BYTES = 64 << 20
+DIRECT_ANY_SIZE_ROWS = 2        # rows up to which the activations are so few that the direct product pays at every size
+
+
+def direct_pays(kind: str, m: int, n: int, k: int) -> bool:
+    """Whether the direct product is the faster form for M <= 16 rows.  ``kind``: what it competes with.
+
+    "gated" (n columns of each half), against the streaming product that cannot split K under the gate: up to four rows always
+    (12,288 x 4,096 at one row 30.9 us against 34.8, 6,144 x 2,048 10.7 against 16.3), up to eight where the other has blocks
+    of four waves or few blocks (32.4 against 33.7, 12.8 against 15.2; but 9,728 x 2,560 22.6 against 21.9), up to
+    sixteen while the matrix is small (3,072 x 1,024 6.7 against 6.9).
+    "add" (into the stream), against the whole-K product, or for a long K the split product and the norm behind it: up to
+    eight rows while the activations stay in L2's reach and the blocks fill their rounds (4,096 x 12,288 at 8 rows 20.3 us against
+    21.3, 2,048 x 6,144 8.3 against 11.5; but 5,120 x 17,408 48.8 against 33.7, 5,120 x 5,120 17.0 against 15.8); nine to
+    sixteen rows read the activations twice for every weight (1,024 x 3,072 at 16 rows 7.0 against 7.6, 4,096 x 4,096
+    10.8 against 11.5, 2,560 x 4,096 in 160 blocks 10.6 against 9.8).
+    "plain", against a product that may leave no partial sums and so has a block for every 64 columns: always (1,024 x 4,096 at
+    one row 4.2 us against 19.0), except where the columns alone are blocks enough (a logits head; up to two rows there too:
+    151,936 x 4,096 180 against 196).
+    "norm" (a row scale to apply, partial sums allowed), against the split streaming product: up to two rows (6,144 x 4,096 10.3
+    against 11.6), more while the activations are few beside L1 (4,096 x 2,048 at 8 rows 6.6 against 7.4, at 16
+    7.4 against 7.8; 6,144 x 2,560 at 8 rows 10.3 against 8.9).
+    "parts" (partial sums allowed), against the same without the scale: only the smallest (1,024 x 1,024 at up to four rows 3.0-3.2
+    against 3.2-3.4; 4,416 x 1,024 at 4 rows 4.8 against 4.5)."""
+    if not 0 < m <= DIRECT_MAX_ROWS:
+        return False
+    size = 2 * n * k
+    if kind == "gated":
+        return m <= 4 or (m <= 8 and (2 * size <= DIRECT_MIDDLE_BYTES or 2 * k % 8192 == 0)) or 2 * size <= STREAM_SMALL_MATRIX_BYTES
+    if kind == "plain":
+        return m <= DIRECT_ANY_SIZE_ROWS or n < 64 * 512
+    if kind == "norm":
+        return m <= DIRECT_ANY_SIZE_ROWS or (size <= STREAM_SMALL_MATRIX_BYTES and (m <= 8 or k <= 2048))
+    if kind == "parts":
+        return m <= 4 and n <= 2048 and k <= 1024
+    if m <= DIRECT_ANY_SIZE_ROWS:
+        return True
+    rows, groups, _ = direct_plan(m, n, k, most_slabs=ROW_SCALE_MAX_SLABS)
+    blocks = -(-n // (rows * groups))
+    even = blocks >= 0.75 * STREAM_CUS * -(-blocks // STREAM_CUS)
+    if m <= 8:
+        return k <= 12288 and (m <= 4 or even or blocks <= STREAM_CUS)
+    return size <= DIRECT_MIDDLE_BYTES and (even or n <= 1024)
+
+
+def gemm_direct(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, sumsq: torch.Tensor | None = None, eps: float = 0.0,
+                gated: bool = False, activation: str | None = None, limit: float | None = None,
+                plan: tuple[int, int, int] | None = None) -> None:
+    """out[M, N] = act((a[M, K] @ w[N, K]^T) * rstd) for M <= 16, the weights straight from memory into matrix operands
+    (csrc/gemm_direct.hip), every block holding the whole of K for its columns.  ``sumsq`` [slabs, M], ``eps``: the
+    rows' scale as in ``gemm_wholek``.  ``gated``: w = [gate; up] of 2N rows, out = act(.) * (.) bfloat16 with ``activation`` "silu"
+    (the default), "gelu_tanh" or "clamped" with its ``limit``; else ``activation`` None or "squared_relu"."""
+    m, k = _wholek_operands(a, w, "gemm_direct")
+    n = w.shape[0] // 2 if gated else w.shape[0]
+    _need(not gated or (w.shape[0] % 2 == 0 and out.dtype == torch.bfloat16), "the gated product has 2N weight rows and a bfloat16 result")
+    _need(out.is_cuda and out.dim() == 2 and out.stride(1) == 1 and out.shape == (m, n), "output must be [M, N] on the GPU")
+    if gated:
+        activation = activation or "silu"
+        _need(activation in GATE_ACTIVATIONS, f"the gate's activation is one of {sorted(GATE_ACTIVATIONS)}")
+        _need((activation == "clamped") == (limit is not None), "a limit goes with the clamped gate")
+        act = GATE_ACTIVATIONS[activation]
+    else:
+        _need(activation in (None, "squared_relu"), "the product's activation is squared_relu")
+        act = 3 if activation else 0
+    if sumsq is not None:
+        _gpu(sumsq)
+        _need(sumsq.dtype == torch.float32 and sumsq.dim() == 2 and sumsq.shape[1] == m and sumsq.shape[0] >= 1,
+              "the rows' sums of squares are float32 [slabs, M]")
+    rows, groups, waves = plan or direct_plan(m, n, k, gated)
+    _note(f"{m}x{w.shape[0]}x{k}", (w.shape[0] * k + m * k) * 2 + m * n * out.element_size(), 2.0 * m * w.shape[0] * k)
+    _check(_fn("gemm_direct", "tk_gemm_direct")(
+        _code(out.dtype), int(gated), _p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(0),
+        _p(sumsq), 0 if sumsq is None else sumsq.shape[0], float(eps), act, float(limit or 0.0), rows, groups, waves, _stream()),
+        "gemm_direct")
+
+
+def _stream_operands(resid: torch.Tensor, gamma: torch.Tensor | None, m: int, n: int) -> torch.Tensor | None:
+    """Checks the residual stream that a product adds into; the array for bf16(stream * gamma), if a weight is given."""
+    _need(resid.is_cuda and resid.dtype == torch.float32 and resid.shape == (m, n) and resid.stride(1) == 1
+          and n % 4 == 0 and resid.stride(0) % 4 == 0 and resid.data_ptr() % 16 == 0,
+          "the stream is float32 [M, N], N a multiple of 4, rows 16-byte aligned")
+    if gamma is None:
+        return None
+    _gpu(gamma)
+    _need(gamma.dtype == torch.float32 and gamma.numel() == n and gamma.data_ptr() % 16 == 0, "the norm weight is float32 [N]")
+    return torch.empty((m, n), dtype=torch.bfloat16, device=resid.device)
+
+
+def gemm_direct_add(a: torch.Tensor, w: torch.Tensor, resid: torch.Tensor, gamma: torch.Tensor | None = None,
+                    *, plan: tuple[int, int, int] | None = None) -> tuple[torch.Tensor, torch.Tensor | None]:
+    """resid[M, N] += a[M, K] @ w[N, K]^T (float32 stream, M <= 16) by the direct product.  Returns (sumsq, scaled) as
+    ``gemm_wholek_add`` does, the sums of squares over slabs of a block's columns (from three rows on, where the streaming
+    product may be the reader, at most ROW_SCALE_MAX_SLABS of them if N allows)."""
+    m, k = _wholek_operands(a, w, "gemm_direct_add")
+    n = w.shape[0]
+    scaled = _stream_operands(resid, gamma, m, n)
+    rows, groups, waves = plan or direct_plan(m, n, k, most_slabs=ROW_SCALE_MAX_SLABS if m > DIRECT_ANY_SIZE_ROWS else 0)
+    sumsq = torch.empty((-(-n // (rows * groups)), m), dtype=torch.float32, device=a.device)
+    _note(f"{m}x{n}x{k}", (n * k + m * k) * 2 + m * n * 10, 2.0 * m * n * k)
+    _check(_fn("gemm_direct", "tk_gemm_direct_add")(
+        _p(a), _p(w), m, n, k, a.stride(0), w.stride(0), _p(resid), resid.stride(0), _p(gamma), _p(scaled),
+        0 if scaled is None else scaled.stride(0), _p(sumsq), rows, groups, waves, _stream()), "gemm_direct_add")
+    return sumsq, scaled
+
+
 WHOLEK_MAX_ROWS = 16    # rows of activations that the whole-K product takes
 ROW_SCALE_MAX_ROWS = 16  # rows up to which the streaming product applies a pending row scale
-ROW_SCALE_MAX_SLABS = 512  # ... and slabs of sums of squares it takes (csrc/gemm_mfma.hip: 16 * kRowScaleLoads)
+ROW_SCALE_MAX_SLABS = 512  # ... and slabs of sums of squares it takes (csrc/gemm_mfma.hip: kRowScaleSlabs)
 
 
 def wholek_waves(n: int, k: int, gated: bool = False) -> int:
@@ -1904,6 +2048,9 @@ def gemm_wholek(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, sumsq: t
         _gpu(sumsq)
         _need(sumsq.dtype == torch.float32 and sumsq.dim() == 2 and sumsq.shape[1] == m and sumsq.shape[0] >= 1,
               "the rows' sums of squares are float32 [slabs, M]")
+    if not waves and direct_pays("gated" if gated else "plain", m, n, k):
+        gemm_direct(a, w, out, sumsq=sumsq, eps=eps, gated=gated)
+        return
     _note(f"{m}x{w.shape[0]}x{k}", (w.shape[0] * k + m * k) * 2 + m * n * out.element_size(), 2.0 * m * w.shape[0] * k)
     _check(_fn("gemm_wholek", "tk_gemm_wholek")(
         _code(out.dtype), int(gated), _p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(0),
@@ -1914,19 +2061,14 @@ def gemm_wholek(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, sumsq: t
 def gemm_wholek_add(a: torch.Tensor, w: torch.Tensor, resid: torch.Tensor, gamma: torch.Tensor | None = None,
                     *, waves: int = 0) -> tuple[torch.Tensor, torch.Tensor | None]:
     """resid[M, N] += a[M, K] @ w[N, K]^T (float32 stream, M <= 16) in the product's own kernel.
-    Returns (sumsq, scaled): sumsq float32 [N/16, M], the sums of squares of every row of the new
-    stream over slabs of 16 columns, and, given ``gamma`` [N] (the weight of the norm that reads
+    Returns (sumsq, scaled): sumsq float32 [slabs, M], the sums of squares of every row of the new
+    stream over slabs of columns (of 16 with ``waves`` given), and, given ``gamma`` [N] (the weight of the norm that reads
     the stream next), scaled = bf16(resid * gamma) [M, N]: what ``gemm_wholek`` takes."""
     m, k = _wholek_operands(a, w, "gemm_wholek_add")
     n = w.shape[0]
-    _need(resid.is_cuda and resid.dtype == torch.float32 and resid.shape == (m, n) and resid.stride(1) == 1
-          and n % 4 == 0 and resid.stride(0) % 4 == 0 and resid.data_ptr() % 16 == 0,
-          "the stream is float32 [M, N], N a multiple of 4, rows 16-byte aligned")
-    scaled = None
-    if gamma is not None:
-        _gpu(gamma)
-        _need(gamma.dtype == torch.float32 and gamma.numel() == n and gamma.data_ptr() % 16 == 0, "the norm weight is float32 [N]")
-        scaled = torch.empty((m, n), dtype=torch.bfloat16, device=a.device)
+    if not waves and direct_pays("add", m, n, k):
+        return gemm_direct_add(a, w, resid, gamma)
+    scaled = _stream_operands(resid, gamma, m, n)
     sumsq = torch.empty((-(-n // 16), m), dtype=torch.float32, device=a.device)
     _note(f"{m}x{n}x{k}", (n * k + m * k) * 2 + m * n * 10, 2.0 * m * n * k)
     _check(_fn("gemm_wholek", "tk_gemm_wholek_add")(
