@@ -1,0 +1,38 @@
+"""Recorded steps whose layers hold two branches: every replay against the same step run kernel after kernel."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("preset, layers", [("mepupel-0.6b", 6), ("supinex-0.6b", 4), ("dopirax-0.6b", 4), ("rorosun-0.6b", 4)])
+@pytest.mark.parametrize("requests", [1, 5, 18])
+def test_branches_give_the_bits_of_kernels_in_a_row(preset, layers, requests):
+    """Steps of single tokens recorded with branches, and eager (no branches): equal bits of every logit, over many
+    replays with other kernels between them, for contexts of unlike lengths."""
+    from replay_util import random_ids
+    from tokamak_amd.config import find_preset
+    from tokamak_amd.engine.runner import ModelRunner, StepEntry
+    from tokamak_amd.weights.random_init import expected_tensors_of
+    from tokamak_amd.weights.sources import RandomSource
+
+    arch, cfg = find_preset(preset)
+    plan = arch.plan(arch.shorten(cfg, layers))
+    source = RandomSource({n: s for n, s in expected_tensors_of(plan).items() if not s.ignored}, seed=3, matrix_std=0.02,
+                          vector_jitter=0.1, dtype=torch.bfloat16, device="cuda:0")
+    outs = []
+    for use_graphs in (True, False):
+        runner = ModelRunner(plan, source, dtype="bfloat16", page_size=16, kv_pool_tokens=160 * requests,
+                             max_requests=requests, use_graphs=use_graphs)
+        ids = [random_ids(plan.vocab_size, 20 + 5 * r + 12, r) for r in range(requests)]
+        runner.step([StepEntry(r, ids[r][:20 + 5 * r], []) for r in range(requests)])
+        got = []
+        for i in range(12):
+            got.append(runner.step([StepEntry(r, [ids[r][20 + 5 * r + i]], [0]) for r in range(requests)]).clone())
+            torch.randn(1 << 20, device="cuda:0").sum()       # other work of the program's between replays
+        torch.cuda.synchronize()
+        assert bool(runner._graphs) == use_graphs
+        outs.append(got)
+    for i, (a, b) in enumerate(zip(*outs)):
+        assert torch.isfinite(a).all() and torch.equal(a, b), f"step {i}"

@@ -6,7 +6,15 @@
 // patch names a slot that holds an address inside one of the layer's own tensors, the
 // tensor's place in `addresses`, and the offset inside it.  One call from the host language
 // issues the whole layer.
+//
+// tk_stream_order: what is launched on `to` from now on starts when what has been launched on `from` so far is done.  As an
+// entry point of its own it stands in recorded lists, and in a HIP graph that is being recorded it is the edge between two branches.
+#include <hip/hip_runtime.h>
+
 #include <cstdint>
+
+#include "common.h"
+#include "slots.h"
 
 typedef int (*slots_fn)(const unsigned long long*);
 
@@ -27,3 +35,16 @@ extern "C" __attribute__((visibility("default"))) int tk_replay_calls(
   }
   return -1;
 }
+
+TK_API int tk_stream_order(hipStream_t from, hipStream_t to) {
+  if (from == to) return 0;
+  hipEvent_t event;
+  hipError_t status = hipEventCreateWithFlags(&event, hipEventDisableTiming);
+  if (status != hipSuccess) return (int)status;
+  status = hipEventRecord(event, from);
+  if (status == hipSuccess) status = hipStreamWaitEvent(to, event, 0);
+  const hipError_t gone = hipEventDestroy(event);     // (its work is queued or recorded; the handle is no longer needed)
+  return (int)(status != hipSuccess ? status : gone);
+}
+
+TK_SLOTS(tk_stream_order)

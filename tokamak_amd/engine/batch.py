@@ -93,6 +93,8 @@ class StepBatch:
     max_q_len: int = 0
     max_seq_len: int = 0
     memo: dict = field(default_factory=dict)  # per-step data shared between layers
+    # while a decode step is recorded: a second stream, on which a layer may put a part beside another (parts/block.py)
+    side: torch.cuda.Stream | None = None
 
 
 NUM_FIXED = 9      # arrays in the packed buffer before the block tables

@@ -38,7 +38,7 @@ class DecodeGraph:
     whose copy has not run yet.
     """
 
-    def __init__(self, model, storage, packed: PackedBatch, device, feed=None) -> None:
+    def __init__(self, model, storage, packed: PackedBatch, device, feed=None, side=None) -> None:
         self.size = int(packed.buf.size)
         self._host = [torch.empty(self.size, dtype=torch.int32, pin_memory=True) for _ in range(2)]
         self._copied = [torch.cuda.Event(), torch.cuda.Event()]
@@ -66,8 +66,10 @@ class DecodeGraph:
         gc.disable()
         try:
             with torch.cuda.graph(self.graph):
+                self.batch.side = side
                 self.logits = model.forward(self.batch, storage)
         finally:
+            self.batch.side = None
             if collecting:
                 gc.enable()
         self.bytes = max(0, torch.cuda.max_memory_allocated(device) - before) + self.size * 4

@@ -90,6 +90,7 @@ class ModelRunner:
         self._groups = groups
         self._ctx_len: dict[object, int] = {}
         self._graphs: dict[tuple, DecodeGraph] = {}
+        self._side = torch.cuda.Stream(self.device)      # the second branch of recorded steps; nothing is ever run on it directly
         # where a sampler leaves its tokens for entries of the next step that ``feed`` on them
         self.sampled = torch.zeros(max(max_requests, 1), dtype=torch.int32, device=self.device)
         self.graph_memory_bytes = int(graph_memory_bytes)
@@ -249,7 +250,7 @@ class ModelRunner:
         graph = self._graphs.pop(key, None)
         if graph is None:
             # a new shape: this step runs eagerly, once, and is recorded for the next ones
-            graph = DecodeGraph(self.model, self.storage, packed, self.device, self._feed)
+            graph = DecodeGraph(self.model, self.storage, packed, self.device, self._feed, self._side)
             logits, graph.first_logits = graph.first_logits, None
             self._graphs[key] = graph
             self._trim_graphs()

@@ -146,6 +146,12 @@ class pinned_stream:
         return False
 
 
+def order_streams(first: torch.cuda.Stream, then: torch.cuda.Stream) -> None:
+    """What is launched on ``then`` from now on starts when what was launched on ``first`` is done; part of a list
+    that is being recorded, and of a graph."""
+    _check(_fn("replay", "tk_stream_order")(c_void_p(first.cuda_stream), c_void_p(then.cuda_stream)), "stream_order")
+
+
 def _need(cond: bool, msg: str) -> None:
     if not cond:
         raise KernelError(msg)
@@ -272,6 +278,9 @@ _SIGS = {
                            c_void_p, c_int, c_float, c_int, c_float, c_int, c_int, c_int, c_void_p],
         "tk_gemm_direct_add": [c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_void_p, c_long, c_void_p,
                                c_void_p, c_long, c_void_p, c_int, c_int, c_int, c_void_p],
+    },
+    "replay": {
+        "tk_stream_order": [c_void_p, c_void_p],
     },
     "blas_lt": {
         "tk_lt_gemm": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_void_p,

@@ -68,6 +68,11 @@ class Part:
     # Parts that do not say so never meet these types.
     fuses_residual = False
 
+    # Whether the part's ``forward`` is a chain of several kernels that touches nothing but its arguments, its own
+    # tensors and its own cache slot (in particular, leaves nothing in ``batch.memo`` by a kernel): in a recorded
+    # decode step a block may then run it as a branch beside another part (parts/block.py: ``beside``).
+    own_branch = False
+
     def __init__(self, *, dtype: torch.dtype, device: torch.device | str) -> None:
         self.dtype = dtype
         self.device = torch.device(device)

@@ -40,6 +40,7 @@ class RoutedExperts(FeedForward):
     """
 
     capturable = True
+    own_branch = True
     replayable = True
 
     def __init__(self, *, hidden_size: int, intermediate_size: int, num_experts: int, top: int,

@@ -32,6 +32,7 @@ class DecayedStateTimeMix(Mixer):
     """
 
     capturable = True
+    own_branch = True
     replayable = True
 
     def __init__(self, *, hidden_size: int, num_heads: int, head_dim: int, norm_eps: float,
