@@ -109,7 +109,7 @@ __device__ __forceinline__ void decode_head_vector(const DecodeInputs& in, size_
   }
   if (rotate) {
     // out[j] = x[j] cos_j - x[j + HD/2] sin_j ; out[j + HD/2] = x[j + HD/2] cos_j + x[j] sin_j
-    const float p0 = __shfl_xor(x0, HD / 4, kWave), p1 = __shfl_xor(x1, HD / 4, kWave);
+    const float p0 = lane_xor<HD / 4>(x0), p1 = lane_xor<HD / 4>(x1);
     const int j = d % (HD / 2);
     const float2 c = *reinterpret_cast<const float2*>(in.cos_t + (size_t)token * (HD / 2) + j);
     const float2 sn = *reinterpret_cast<const float2*>(in.sin_t + (size_t)token * (HD / 2) + j);
@@ -290,8 +290,8 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
         if (edge && c0 + kb * 4 + e > pos0) sv[e] = -INFINITY;
       }
       float tmax = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+      tmax = max16(tmax);
+      tmax = max32(tmax);
       const float m_new = fmaxf(m_run, tmax);  // finite: a tile's first key is never past the position
       const float alpha = fast_exp2(m_run - m_new);
       m_run = m_new;
@@ -334,8 +334,8 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
   float* s_m = s_dyn + (size_t)WAVES * G * HD;  // [WAVES][16]
   float* s_l = s_m + WAVES * 16;                // [WAVES][16]
   float l = l_run;
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
+  l = sum16(l);
+  l = sum32(l);
   if (c_valid) {
     float* mine = s_acc + ((size_t)wave * G + col) * HD + kb * 4;
 #pragma unroll
@@ -663,8 +663,8 @@ void attention_prefill_kernel(
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, sv[j][i]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+    tmax = max16(tmax);
+    tmax = max32(tmax);
     // the running maximum is kept in units of log2: m = max(score) * scale * log2(e)
     const float m_new = fmaxf(m_run, tmax * scale_log2);
     const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
@@ -707,8 +707,8 @@ void attention_prefill_kernel(
   }
 
   float l = l_run;
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
+  l = sum16(l);
+  l = sum32(l);
   if (c_valid && computes) {
     if (nsplit == 1) {
       if (sinks) l += fast_exp2(sinks[head] * 1.4426950408889634f - m_run);
@@ -902,7 +902,7 @@ void attention_prefill_wide_kernel(
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, sc[kb][e]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+    tmax = max32(tmax);
     // the running maximum is kept in units of log2: m = max(score) * scale * log2(e)
     const float m_new = fmaxf(m_run, tmax * scale_log2);
     const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
@@ -945,7 +945,7 @@ void attention_prefill_wide_kernel(
   }
 
   float l = l_run;
-  l += __shfl_xor(l, 32, kWave);
+  l = sum32(l);
   if (c_valid && computes) {
     if (sinks) l += fast_exp2(sinks[head] * 1.4426950408889634f - m_run);
     const float inv = 1.f / l;
@@ -1194,7 +1194,7 @@ void attention_prefill_group_kernel(
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, sc[kb][e]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+    tmax = max32(tmax);
     // the running maximum is kept in units of log2: m = max(score) * scale * log2(e)
     const float m_new = fmaxf(m_run, tmax * scale_log2);
     const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
@@ -1283,7 +1283,7 @@ void attention_prefill_group_kernel(
   }
 
   float l = l_run;
-  l += __shfl_xor(l, 32, kWave);
+  l = sum32(l);
   if (c_valid && computes) {
     if (sinks) l += fast_exp2(sinks[head] * 1.4426950408889634f - m_run);
     const float inv = 1.f / l;

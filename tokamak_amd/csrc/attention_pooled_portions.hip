@@ -288,13 +288,13 @@ __global__ __launch_bounds__(16 * H) void portion_weights_kernel(Args a) {
     }
 #pragma unroll
     for (int x = 0; x < kMaxShares / 4; ++x) top = fmaxf(top, pm[x]);
-    top = fmaxf(top, __shfl_xor(top, 16, kWave));
-    top = fmaxf(top, __shfl_xor(top, 32, kWave));
+    top = max16(top);
+    top = max32(top);
 #pragma unroll
     for (int x = 0; x < kMaxShares / 4; ++x)
       if (4 * x + (lane >> 4) < a.S) sum += pl[x] * __builtin_amdgcn_exp2f(pm[x] - top);
-    sum += __shfl_xor(sum, 16, kWave);
-    sum += __shfl_xor(sum, 32, kWave);
+    sum = sum16(sum);
+    sum = sum32(sum);
     m[h] = top;
     il[h] = 1.f / sum;
   }

@@ -114,8 +114,8 @@ __global__ __launch_bounds__(kHeadsPerBlock * 64) void attention_tiles_kernel(
       sv[e] = seen[e] ? (CAP ? cap.log2_score(sc[e]) : sc[e] * scale_log2) : -INFINITY;     // (a key that no token wrote may hold anything: chosen, not computed)
     }
     float tmax = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+    tmax = max16(tmax);
+    tmax = max32(tmax);
     const float m_new = fmaxf(m_run, tmax);
     const float m_safe = m_new == -INFINITY ? 0.f : m_new;   // a token that has seen no key yet
     const float alpha = fast_exp2(m_run - m_safe);
@@ -147,8 +147,8 @@ __global__ __launch_bounds__(kHeadsPerBlock * 64) void attention_tiles_kernel(
   }
 
   float l = l_run;
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
+  l = sum16(l);
+  l = sum32(l);
   if (sinks) l += fast_exp2(sinks[head] * 1.4426950408889634f - m_run);
   if (col >= cnt) return;
   const float inv = 1.f / l;
@@ -286,8 +286,8 @@ __global__ __launch_bounds__(HB * 64) void attention_tiles_shared_kernel(
         sv[e] = seen[e] ? (CAP ? cap.log2_score(sc[e]) : sc[e] * scale_log2) : -INFINITY;
       }
       float tmax = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+      tmax = max16(tmax);
+      tmax = max32(tmax);
       const float m_new = fmaxf(m_run, tmax);
       const float m_safe = m_new == -INFINITY ? 0.f : m_new;
       const float alpha = fast_exp2(m_run - m_safe);
@@ -327,8 +327,8 @@ __global__ __launch_bounds__(HB * 64) void attention_tiles_shared_kernel(
 
   if (!computes) return;
   float l = l_run;
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
+  l = sum16(l);
+  l = sum32(l);
   if (sinks) l += fast_exp2(sinks[head] * 1.4426950408889634f - m_run);
   if (col >= cnt) return;
   const float inv = 1.f / l;
@@ -445,8 +445,8 @@ __global__ __launch_bounds__(256) void attention_heads_kernel(
       sv[e] = seen[e] ? (CAP ? cap.log2_score(sc[e]) : sc[e] * scale_log2) : -INFINITY;
     }
     float tmax = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, kWave));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+    tmax = max16(tmax);
+    tmax = max32(tmax);
     const float m_new = fmaxf(m_run, tmax);   // finite: a step holds at least one visible key
     const float alpha = fast_exp2(m_run - m_new);
     m_run = m_new;
@@ -475,8 +475,8 @@ __global__ __launch_bounds__(256) void attention_heads_kernel(
     }
   }
   float l = l_run;
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
+  l = sum16(l);
+  l = sum32(l);
   if (!c_valid) return;
   // partial rows [item][head][part]: (maximum, sum), then the output
   const size_t prow = ((size_t)item * nh + head) * parts + part;

@@ -74,10 +74,69 @@ __device__ __forceinline__ bool rows_take_wide_stores(const T* p, long ld) {
 
 constexpr int kWave = 64;
 
+// Exchanges between lanes by the vector unit's own lane paths (__shfl_xor goes through LDS: some 100 cycles a level,
+// these 8 to 16; a reduction over the wave six levels).
+//
+// The value of the lane whose number differs in bit 0 or 1 (level 0, 1).  Levels 2 and 3 take the mirrored lane of eight
+// and of sixteen: it lies in the other four, the other eight, whose lanes all hold the same after the levels before.
+template <int LEVEL>
+__device__ __forceinline__ uint32_t lane_other(uint32_t v) {
+  static_assert(LEVEL >= 0 && LEVEL < 4, "levels 4 and 5 come as pairs");
+  constexpr int kControl = LEVEL == 0 ? 0xB1 /* quad_perm 1 0 3 2 */ : LEVEL == 1 ? 0x4E /* quad_perm 2 3 0 1 */
+                           : LEVEL == 2 ? 0x141 /* row_half_mirror */ : 0x140 /* row_mirror */;
+  return __builtin_amdgcn_update_dpp(0u, v, kControl, 0xf, 0xf, false);
+}
+template <int LEVEL>
+__device__ __forceinline__ float lane_other(float v) { return __uint_as_float(lane_other<LEVEL>(__float_as_uint(v))); }
+
+// Lanes l and l ^ 16 (l ^ 32): both get the pair (value of the lane without that bit, value of the lane with it).
+struct LanePair {
+  uint32_t first, second;
+  __device__ __forceinline__ float a() const { return __uint_as_float(first); }
+  __device__ __forceinline__ float b() const { return __uint_as_float(second); }
+};
+__device__ __forceinline__ LanePair pair16(uint32_t v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return {r[0], r[1]};
+}
+__device__ __forceinline__ LanePair pair32(uint32_t v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return {r[0], r[1]};
+}
+// v of lane l with v of lane l ^ 16, and over all four lanes l, l ^ 16, l ^ 32, l ^ 48: the same bits in each of them
+__device__ __forceinline__ float sum16(float v) { const LanePair p = pair16(__float_as_uint(v)); return p.a() + p.b(); }
+__device__ __forceinline__ float sum32(float v) { const LanePair p = pair32(__float_as_uint(v)); return p.a() + p.b(); }
+__device__ __forceinline__ float max16(float v) { const LanePair p = pair16(__float_as_uint(v)); return fmaxf(p.a(), p.b()); }
+__device__ __forceinline__ float max32(float v) { const LanePair p = pair32(__float_as_uint(v)); return fmaxf(p.a(), p.b()); }
+
+// The value of lane l ^ D.
+template <int D>
+__device__ __forceinline__ float lane_xor(float v) {
+  static_assert(D == 1 || D == 2 || D == 4 || D == 8 || D == 16 || D == 32, "a bit of the lane's number");
+  const uint32_t u = __float_as_uint(v);
+  if constexpr (D <= 2) return __uint_as_float(lane_other<D - 1>(u));
+  if constexpr (D == 4)      // the mirrored lane of eight, then the mirrored one of four
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0u, lane_other<2>(u), 0x1B /* quad_perm 3 2 1 0 */, 0xf, 0xf, false));
+  if constexpr (D == 8) return __uint_as_float(__builtin_amdgcn_update_dpp(0u, u, 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+  const LanePair p = D == 16 ? pair16(u) : pair32(u);
+  return threadIdx.x & D ? p.a() : p.b();      // (blocks are rows of threads in this library: the lane's number is threadIdx.x % 64)
+}
+// The sum over the lanes whose numbers differ in bits FROM, 2 FROM, ..., below TO.
+template <int FROM, int TO>
+__device__ __forceinline__ float sum_lanes(float v) {
+  if constexpr (FROM >= TO) return v;
+  else if constexpr (FROM == 16) return sum_lanes<32, TO>(sum16(v));
+  else if constexpr (FROM == 32) return sum32(v);
+  else return sum_lanes<FROM * 2, TO>(v + lane_xor<FROM>(v));
+}
+
+// (all lanes get the same bits: a level's two addends are the same two numbers in each of its lanes)
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, kWave);
-  return v;
+  v += lane_other<0>(v);
+  v += lane_other<1>(v);
+  v += lane_other<2>(v);
+  v += lane_other<3>(v);
+  return sum32(sum16(v));
 }
 
 // Orders one wave's LDS accesses (a wave's LDS instructions execute in order; this
@@ -89,9 +148,30 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, kWave));
-  return v;
+  v = fmaxf(v, lane_other<0>(v));
+  v = fmaxf(v, lane_other<1>(v));
+  v = fmaxf(v, lane_other<2>(v));
+  v = fmaxf(v, lane_other<3>(v));
+  return max32(max16(v));
+}
+
+// The best (value, index) of the wave in every lane; take(value, at, other value, its index) keeps the better of two, whichever
+// of them comes first.
+template <typename Take>
+__device__ __forceinline__ void wave_best(float& value, int& at, const Take& take) {
+  take(value, at, lane_other<0>(value), (int)lane_other<0>((uint32_t)at));
+  take(value, at, lane_other<1>(value), (int)lane_other<1>((uint32_t)at));
+  take(value, at, lane_other<2>(value), (int)lane_other<2>((uint32_t)at));
+  take(value, at, lane_other<3>(value), (int)lane_other<3>((uint32_t)at));
+  LanePair v = pair16(__float_as_uint(value)), i = pair16((uint32_t)at);
+  value = v.a();
+  at = (int)i.first;
+  take(value, at, v.b(), (int)i.second);
+  v = pair32(__float_as_uint(value));
+  i = pair32((uint32_t)at);
+  value = v.a();
+  at = (int)i.first;
+  take(value, at, v.b(), (int)i.second);
 }
 
 // Sum over a block of up to 1024 threads; `scratch` holds >= 16 floats of LDS.

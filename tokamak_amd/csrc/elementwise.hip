@@ -510,8 +510,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_store_vec_kernel(
       float ss = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
-#pragma unroll
-      for (int m = LPH / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, kWave);
+      ss = sum_lanes<1, LPH>(ss);
       const float rstd = rsqrtf(ss / (float)HD + eps);
       const float4 w0 = *reinterpret_cast<const float4*>(w + d0);
       const float4 w1 = *reinterpret_cast<const float4*>(w + d0 + 4);
@@ -523,7 +522,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_store_vec_kernel(
     const float sign = (d0 < HD / 2) ? -1.f : 1.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float partner = __shfl_xor(x[e], LPH / 2, kWave);
+      const float partner = lane_xor<LPH / 2>(x[e]);
       x[e] = x[e] * cs[e] + sign * partner * sn[e];
     }
   }
@@ -806,8 +805,7 @@ __global__ __launch_bounds__(256) void map_difference_kernel(const T* __restrict
       }
     }
   }
-#pragma unroll
-  for (int m = LANES / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, kWave);
+  ss = sum_lanes<1, LANES>(ss);
   const float factor = scale / sqrtf(ss / (float)vd + eps);
   T* q = out + (size_t)item * vd;
 #pragma unroll
@@ -1639,8 +1637,7 @@ __global__ __launch_bounds__(256) void rope_norm_store_vec_kernel(const TIN* __r
       float ss = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
-#pragma unroll
-      for (int m = LK / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, kWave);
+      ss = sum_lanes<1, LK>(ss);
       const float rstd = 1.f / sqrtf(ss / (float)A.hd + A.eps);
       const float* w = is_q ? A.q_weight : A.k_weight;
       if (w && mine) {

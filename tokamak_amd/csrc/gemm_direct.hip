@@ -187,8 +187,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_direct_kernel(
         for (int g = 0; g < RG; ++g) red[wave][i][t][g][(share * QUADS + kb % QUADS) * TP + own] = acc[i][t][g];
   }
   if (EPI != EPI_ADD && scale.sumsq != nullptr) {
-#pragma unroll
-    for (int d = ROWS; d < kWave; d *= 2) ss += __shfl_xor(ss, d, kWave);
+    ss = sum_lanes<ROWS, kWave>(ss);
     if (lane < ROWS) stat[wave][lane] = ss;
   }
   __syncthreads();
@@ -203,9 +202,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_direct_kernel(
       for (int w = 0; w < WAVES; ++w) total[t] += red[w][wave][t][lane / KEPT][lane % KEPT];
     }
 #pragma unroll
-    for (int d = QUADS * TP; d < KEPT; d *= 2)      // (the same sums in every lane: a + b is b + a)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) total[t][e] += __shfl_xor(total[t][e], d, kWave);
+    for (int e = 0; e < 4; ++e) total[t][e] = sum_lanes<QUADS * TP, KEPT>(total[t][e]);
   }
 
   if constexpr (EPI == EPI_ADD) {
@@ -219,10 +216,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_direct_kernel(
       sq = v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
     }
     // (lanes that finish nothing hold zeros)
-#pragma unroll
-    for (int d = TP; d < QUADS * TP; d *= 2) sq += __shfl_xor(sq, d, kWave);
-#pragma unroll
-    for (int d = KEPT; d < RG * KEPT; d *= 2) sq += __shfl_xor(sq, d, kWave);
+    sq = sum_lanes<KEPT, RG * KEPT>(sum_lanes<TP, QUADS * TP>(sq));
     if (lane < TP && m < M) sum.sumsq[(size_t)blockIdx.x * M + m] = sq;
     return;
   }

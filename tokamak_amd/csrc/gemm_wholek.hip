@@ -206,10 +206,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wholek_kernel(
       const int group = kb * WAVES + g;  // thread group*16 + r of the block holds it
       part += reinterpret_cast<const float*>(lds + (size_t)(group >> 2) * (TILES * TILE_BYTES))[TILES * 256 + (group & 3) * 16 + r];
     }
-    const float other = __shfl_xor(part, 16, kWave);
-    const float pair = kb & 1 ? other + part : part + other;    // (kb 0 + kb 1), (kb 2 + kb 3): in this order
-    const float far = __shfl_xor(pair, 32, kWave);
-    const float all = kb & 2 ? far + pair : pair + far;
+    const float all = sum32(sum16(part));     // ((kb 0 + kb 1) + (kb 2 + kb 3))
     rstd = rsqrtf(all / (float)K + scale.eps);
   }
 
@@ -223,10 +220,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_wholek_kernel(
             make_uint2(pack_bf16x2(v.x * gam.x, v.y * gam.y), pack_bf16x2(v.z * gam.z, v.w * gam.w));
       sq = v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
     }
-    const float other = __shfl_xor(sq, 16, kWave);
-    const float pair = kb & 1 ? other + sq : sq + other;
-    const float far = __shfl_xor(pair, 32, kWave);
-    const float all = kb & 2 ? far + pair : pair + far;
+    const float all = sum32(sum16(sq));
     if (kb == 0 && m < M) sum.sumsq[(size_t)blockIdx.x * M + m] = all;
     return;
   }

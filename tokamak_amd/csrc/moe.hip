@@ -53,6 +53,11 @@ template <> struct Vec<bf16_t> {
   }
 };
 
+// The larger score, the lower index among equals.
+__device__ __forceinline__ void larger(float& best, int& at, float other, int other_at) {
+  if (other > best || (other == best && other_at < at)) { best = other; at = other_at; }
+}
+
 // A block takes TOK tokens: its waves take the router's rows two at a time for all of them (lanes stride the width; the
 // rows are read once a block), then a wave a token picks the largest scores.
 //   correction (null or float32 [E]): the choice is made by score + correction, the weights are the
@@ -186,12 +191,7 @@ __global__ __launch_bounds__(kRouteWaves * kWave) void moe_route_kernel(
         const float v = group_score[g];
         if (v > best && v != INFINITY) { best = v; at = g; }
       }
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) {
-        const float ob = __shfl_xor(best, m, kWave);
-        const int oa = __shfl_xor(at, m, kWave);
-        if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
-      }
+      wave_best(best, at, larger);
       if (lane == 0 && at < groups) group_score[at] = INFINITY;
       wave_lds_sync();
     }
@@ -208,12 +208,7 @@ __global__ __launch_bounds__(kRouteWaves * kWave) void moe_route_kernel(
       const float v = choice[e];
       if (v > best) { best = v; at = e; }          // (ascending e: the lower index stays on ties)
     }
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-      const float ob = __shfl_xor(best, m, kWave);
-      const int oa = __shfl_xor(at, m, kWave);
-      if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
-    }
+    wave_best(best, at, larger);
     if (at >= E) at = 0;       // (fewer experts may be chosen than `top`: refused on the host, kept in range here)
     if (lane == 0) {
       chosen[(size_t)n * top + k] = at;

@@ -94,12 +94,7 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
   } else {
     for (int i = begin + threadIdx.x; i < end; i += kArgmaxThreads) argmax_take(bv, bi, row[i], i);
   }
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    const float ov = __shfl_xor(bv, m, kWave);
-    const int oi = __shfl_xor(bi, m, kWave);
-    argmax_take(bv, bi, ov, oi);
-  }
+  wave_best(bv, bi, argmax_take);
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   if (lane == 0) {
     best_v[wave] = bv;
@@ -153,12 +148,7 @@ __global__ __launch_bounds__(kWave) void argmax_pick_kernel(const float* __restr
   const int r = blockIdx.x, lane = threadIdx.x;
   float bv = lane < kArgmaxSegments ? part_v[r * kArgmaxSegments + lane] : -INFINITY;
   int bi = lane < kArgmaxSegments ? part_i[r * kArgmaxSegments + lane] : 0x7fffffff;
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    const float ov = __shfl_xor(bv, m, kWave);
-    const int oi = __shfl_xor(bi, m, kWave);
-    argmax_take(bv, bi, ov, oi);
-  }
+  wave_best(bv, bi, argmax_take);
   if (lane == 0) {
     out[r] = (bi == 0x7fffffff) ? 0 : bi;
     if (out_value != nullptr) out_value[r] = bv;
@@ -463,12 +453,7 @@ __global__ __launch_bounds__(kShareThreads) void sample_hist_kernel(
   // the row's maximum (every wave for itself); the first block leaves it, and the argmax
   float bv = lane < kArgmaxSegments ? seg_max[r * kArgmaxSegments + lane] : -INFINITY;
   int bi = lane < kArgmaxSegments ? seg_index[r * kArgmaxSegments + lane] : 0x7fffffff;
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    const float ov = __shfl_xor(bv, m, kWave);
-    const int oi = __shfl_xor(bi, m, kWave);
-    argmax_take(bv, bi, ov, oi);
-  }
+  wave_best(bv, bi, argmax_take);
   if (seg == 0 && threadIdx.x == 0) {
     out[r] = (bi == 0x7fffffff) ? 0 : bi;
     row_max[r] = bv;

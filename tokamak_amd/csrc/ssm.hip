@@ -97,11 +97,11 @@ __device__ __forceinline__ void sum_and_deal(float (&v)[32], int ks) {
       for (int i = 0; i < H; ++i) {
         const float send = upper ? v[i] : v[i + H];
         const float keep = upper ? v[i + H] : v[i];
-        v[i] = keep + __shfl_xor(send, M, kWave);
+        v[i] = keep + lane_xor<M>(send);
       }
       sum_and_deal<H, M / 2>(v, ks);
     } else {
-      v[0] += __shfl_xor(v[0], M, kWave);
+      v[0] += lane_xor<M>(v[0]);
       sum_and_deal<1, M / 2>(v, ks);
     }
   }
@@ -370,8 +370,7 @@ __global__ __launch_bounds__(256) void gated_group_norm_four_kernel(
   v[0] = before_norm(y4.x, z[0], after); v[1] = before_norm(y4.y, z[1], after);
   v[2] = before_norm(y4.z, z[2], after); v[3] = before_norm(y4.w, z[3], after);
   float ss = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
-#pragma unroll
-  for (int m = LANES / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, kWave);
+  ss = sum_lanes<1, LANES>(ss);
   const float rstd = 1.f / sqrtf(ss / (float)size + eps);
   store_four<T>(out + at, behind_norm(v[0] * rstd * w4.x, z[0], after), behind_norm(v[1] * rstd * w4.y, z[1], after),
                 behind_norm(v[2] * rstd * w4.z, z[2], after), behind_norm(v[3] * rstd * w4.w, z[3], after), 4, true);
