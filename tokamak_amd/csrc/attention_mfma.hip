@@ -1,12 +1,13 @@
 // Paged causal attention on the matrix cores (bf16 in, float32 softmax and
 // accumulation) for head sizes 64 and 128 and page sizes 16, 32, 64, ... (powers of two).
 //
-// Decode tokens (attention_decode_kernel): a block of sixteen waves owns one token, one kv
-// head and a range of that request's keys (a split); the waves take contiguous shares
-// of the range and merge through LDS.  A wave's 16 "columns" are the query heads of the
-// group.  Keys are taken 16 at a time (one MFMA tile, never across a page edge); a tile's
-// keys are reloaded for the wave's next tile as soon as the scores are taken, its values
-// as soon as they are multiplied:
+// Decode tokens (attention_decode_kernel): a block of eight waves owns one token, one kv
+// head and a share of that request's keys (a split).  Keys are taken 16 at a time (one MFMA
+// tile, never across a page edge); the tiles are dealt in turn to the waves of all splits, so that
+// where a wave starts follows from the block alone and its page is looked up while the
+// token's position is still on its way; the waves merge through LDS.  A wave's 16 "columns" are the
+// query heads of the group.  A tile's keys are reloaded for the wave's next tile as soon as the
+// scores are taken, its values as soon as they are multiplied:
 //   S^T[key][col] = K[key][:] . Q[col][:]      v_mfma_f32_16x16x32_bf16, K rows as A
 //   P^T = exp2(S^T * c - m[col])               float32, one column per lane
 //   O^T[d][col] += V^T[d][key] * P^T[key][col] v_mfma_f32_16x16x16_bf16, V^T rows as A
@@ -43,16 +44,13 @@ union Frag4 {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-constexpr int kDecodeWaves = 16;
+constexpr int kDecodeWaves = 8;
+constexpr int kDecodeTiles = 2;      // of 16 keys that a wave keeps in flight
 
-// The keys of one split of a decode token whose keys are cut in nsplit: the token's own keys
-// cut evenly (a whole number of 16 keys for every wave of a block), whatever the longest
-// request of the step holds, so that the blocks of a token walk equal shares; splits past the
-// token's last key hold nothing.
-__device__ __forceinline__ int decode_share(int keys, int nsplit) {
-  constexpr int unit = 16 * kDecodeWaves;
-  return ((keys + nsplit - 1) / nsplit + unit - 1) / unit * unit;
-}
+// Tiles of 16 keys that a round of one split's waves takes: split s of nsplit has the rounds s, s + nsplit, ...  Splits
+// whose first round lies past the token's last key hold nothing.
+constexpr int kRoundKeys = 16 * kDecodeWaves;
+__device__ __forceinline__ int used_splits(int position, int nsplit) { return min(nsplit, position / kRoundKeys + 1); }
 
 // What the fused form of the decode kernel takes instead of finished queries: the q/k/v
 // projection's output as it left the product (`parts` float32 partial sums of a split-K
@@ -70,24 +68,52 @@ struct DecodeInputs {
 
 // One head's vector from the projection's output: partial sums added, per-head RMSNorm,
 // half-split rotation; lane l ends up with dims 2l and 2l + 1 (HD / 2 lanes take part).
-// What the separate kernel of elementwise.hip computes, for one token and head.
+// What the separate kernel of elementwise.hip computes, for one token and head.  In two halves: what
+// is read is asked for as soon as the token is known, before its keys are, and finished while those fly.
+struct HeadInputs {
+  float2 part[4];      // (a chain of dependent loads would cost a memory round trip each)
+  float2 weight, cosine, sine;
+};
 template <int HD>
-__device__ __forceinline__ void decode_head_vector(const DecodeInputs& in, size_t row_offset, int head_col,
-                                                   const float* weight, bool rotate, int token, int lane,
-                                                   float& x0, float& x1) {
-  const bool active = lane < HD / 2;
-  const int d = 2 * (active ? lane : 0);
-  x0 = x1 = 0.f;
+__device__ __forceinline__ HeadInputs ask_head_vector(const DecodeInputs& in, size_t row_offset, int head_col,
+                                                      const float* weight, bool rotate, int token, int lane) {
+  HeadInputs h;
+  const int d = 2 * (lane < HD / 2 ? lane : 0);
+  const float2 zero = make_float2(0.f, 0.f);
   if (in.in_f32) {
     const float* src = static_cast<const float*>(in.qkv) + row_offset + (size_t)head_col * HD + d;
-    // four partial sums in flight at a time (a chain of dependent loads would cost a memory
-    // round trip each); added in split order
-    for (int p = 0; p < in.parts; p += 4) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) h.part[p] = p < in.parts ? *reinterpret_cast<const float2*>(src + (size_t)p * in.part_stride) : zero;
+  } else {
+    const uint32_t v = *reinterpret_cast<const uint32_t*>(static_cast<const bf16_t*>(in.qkv) + row_offset + (size_t)head_col * HD + d);
+    h.part[0].x = __uint_as_float(v);      // (unpacked when finished)
+    h.part[0].y = 0.f;
+    h.part[1] = h.part[2] = h.part[3] = zero;
+  }
+  h.weight = weight != nullptr ? make_float2(weight[d], weight[d + 1]) : zero;
+  const int j = d % (HD / 2);
+  h.cosine = rotate ? *reinterpret_cast<const float2*>(in.cos_t + (size_t)token * (HD / 2) + j) : zero;
+  h.sine = rotate ? *reinterpret_cast<const float2*>(in.sin_t + (size_t)token * (HD / 2) + j) : zero;
+  return h;
+}
+template <int HD>
+__device__ __forceinline__ void finish_head_vector(const HeadInputs& h, const DecodeInputs& in, size_t row_offset, int head_col,
+                                                   bool normed, bool rotate, int lane, float& x0, float& x1) {
+  const bool active = lane < HD / 2;
+  const int d = 2 * (active ? lane : 0);
+  if (in.in_f32) {
+    x0 = x1 = 0.f;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {      // in split order
+      x0 += h.part[p].x;
+      x1 += h.part[p].y;
+    }
+    const float* src = static_cast<const float*>(in.qkv) + row_offset + (size_t)head_col * HD + d;
+    for (int p = 4; p < in.parts; p += 4) {
       float2 v[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        v[u] = p + u < in.parts ? *reinterpret_cast<const float2*>(src + (size_t)(p + u) * in.part_stride)
-                                : make_float2(0.f, 0.f);
+        v[u] = p + u < in.parts ? *reinterpret_cast<const float2*>(src + (size_t)(p + u) * in.part_stride) : make_float2(0.f, 0.f);
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         x0 += v[u].x;
@@ -95,27 +121,23 @@ __device__ __forceinline__ void decode_head_vector(const DecodeInputs& in, size_
       }
     }
   } else {
-    const uint32_t v = *reinterpret_cast<const uint32_t*>(static_cast<const bf16_t*>(in.qkv) + row_offset +
-                                                          (size_t)head_col * HD + d);
+    const uint32_t v = __float_as_uint(h.part[0].x);
     x0 = __uint_as_float(v << 16);
     x1 = __uint_as_float(v & 0xffff0000u);
   }
   if (!active) x0 = x1 = 0.f;
-  if (weight != nullptr) {
+  if (normed) {
     const float ss = wave_sum(x0 * x0 + x1 * x1);
     const float rstd = rsqrtf(ss / (float)HD + in.eps);
-    x0 = x0 * rstd * weight[d];
-    x1 = x1 * rstd * weight[d + 1];
+    x0 = x0 * rstd * h.weight.x;
+    x1 = x1 * rstd * h.weight.y;
   }
   if (rotate) {
     // out[j] = x[j] cos_j - x[j + HD/2] sin_j ; out[j + HD/2] = x[j + HD/2] cos_j + x[j] sin_j
     const float p0 = lane_xor<HD / 4>(x0), p1 = lane_xor<HD / 4>(x1);
-    const int j = d % (HD / 2);
-    const float2 c = *reinterpret_cast<const float2*>(in.cos_t + (size_t)token * (HD / 2) + j);
-    const float2 sn = *reinterpret_cast<const float2*>(in.sin_t + (size_t)token * (HD / 2) + j);
     const float sign = (d < HD / 2) ? -1.f : 1.f;
-    x0 = x0 * c.x + sign * p0 * sn.x;
-    x1 = x1 * c.y + sign * p1 * sn.y;
+    x0 = x0 * h.cosine.x + sign * p0 * h.sine.x;
+    x1 = x1 * h.cosine.y + sign * p1 * h.sine.y;
   }
 }
 
@@ -125,13 +147,13 @@ __device__ __forceinline__ void decode_head_vector(const DecodeInputs& in, size_
 // the page and every wave that meets the token's position takes from LDS) from the
 // projection's output: one kernel less a layer than with the separate q/k norm kernel.
 template <int HD, int WAVES, int D, bool FUSED, bool CAP>
-__global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
+__global__ __launch_bounds__(WAVES * 64, 2) void attention_decode_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache_in,
     const bf16_t* __restrict__ v_cache_in, const int* __restrict__ block_tables, int max_pages,
     const int* __restrict__ positions, const int* __restrict__ req_of_token,
     const int* __restrict__ item_token, const int* __restrict__ item_count,
     bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml, int nsplit,
-    int split_keys, int nh, int nkv, int ps, float scale_log2, DecodeInputs in, const float* __restrict__ sinks,
+    int nh, int nkv, int ps, float scale_log2, DecodeInputs in, const float* __restrict__ sinks,
     SoftCap cap) {
   const bf16_t* __restrict__ k_cache = k_cache_in;
   const bf16_t* __restrict__ v_cache = v_cache_in;
@@ -139,90 +161,97 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
   constexpr int DBL = HD / 16;  // 16-wide blocks of the head dim (PV outputs)
   // LDS: the waves' accumulators of the group's heads [WAVES][G][HD], then their (m, l) [WAVES][16] each
   extern __shared__ __attribute__((aligned(16))) float s_dyn[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, kb = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, kb = lane >> 4;
   // splits are the slowest index of the grid: blocks start in the grid's order, so a token's
   // last split (the shortest, or one that holds no key) starts behind every first one
   const int split = blockIdx.z, item = blockIdx.y;
   const int G = nh / nkv;
   const int kvh = blockIdx.x;
+  static_assert(WAVES == kDecodeWaves, "kRoundKeys counts blocks of kDecodeWaves waves");
 
+  // the wave's tiles: t_first, t_first + t_stride, ...; their pages are looked up before the position is known
+  const int t_first = split * WAVES + wave, t_stride = nsplit * WAVES;
   const int n0 = item_token[item];
+  const int* table = block_tables + (size_t)(req_of_token ? req_of_token[n0] : n0) * max_pages;
+  const auto page_of = [&](int t) { return table[min(t * 16 / ps, max_pages - 1)]; };
+  int page[D];
+#pragma unroll
+  for (int i = 0; i < D; ++i) page[i] = page_of(t_first + i * t_stride);
   const int pos0 = positions[n0];  // the token's position: it sees keys 0 .. pos0
-  static_assert(WAVES == kDecodeWaves, "decode_share cuts for blocks of kDecodeWaves waves");
-  const int share = nsplit > 1 ? decode_share(pos0 + 1, nsplit) : split_keys;
-  const int k_begin = split * share;
-  const int k_end = min(pos0 + 1, k_begin + share);
-  if (k_begin >= k_end) return;  // the whole block: this split holds no key of the token
-  const int* table = block_tables + (size_t)req_of_token[n0] * max_pages;
+
+  // FUSED: the vectors that the block has to make (the group's queries, the new key, the new value), dealt to the waves
+  constexpr int MOST = (16 + WAVES - 1) / WAVES;      // groups of up to 14 query heads
+  HeadInputs head_in[MOST];
+  const bool stores = FUSED && in.nkv_in > 0;    // this call stores the token's key and value
+  const size_t row_offset = FUSED ? (size_t)n0 * (nh + 2 * in.nkv_in) * HD : 0;
+  const int vectors = G + (stores ? 2 : 0);
+  const auto column_of = [&](int v) { return v < G ? kvh * G + v : v == G ? nh + kvh : nh + in.nkv_in + kvh; };
+  const auto weight_of = [&](int v) { return v < G ? in.q_weight : v == G ? in.k_weight : nullptr; };
+  if constexpr (FUSED) {
+#pragma unroll
+    for (int u = 0; u < MOST; ++u) {
+      const int v = wave + u * WAVES;
+      if (v < vectors) head_in[u] = ask_head_vector<HD>(in, row_offset, column_of(v), weight_of(v), v <= G && in.rot != 0, n0, lane);
+    }
+  }
+
+  if (split * kRoundKeys > pos0) return;  // the whole block: this split holds no key of the token
+  const int last_split = used_splits(pos0, nsplit) - 1;
   const size_t page_elems = (size_t)nkv * HD * ps;
   const size_t head_off = (size_t)kvh * HD * ps;
-
-  // the split's tiles of 16 keys, in contiguous shares of the waves
-  const int tiles = (k_end - k_begin + 15) >> 4;
-  const int per = (tiles + WAVES - 1) / WAVES;
-  const int t_begin = wave * per, t_end = min(tiles, t_begin + per);
+  const int tiles = (pos0 >> 4) + 1;
+  const int own = t_first < tiles ? (tiles - t_first + t_stride - 1) / t_stride : 0;      // tiles of this wave
 
   // this lane's column is query head `col` of the group
   const int c_head = kvh * G + col;
   const bool c_valid = col < G;
 
-  // The wave's first tiles are asked for before anything else: they depend on the block
-  // table only, and the queries (which the fused form first has to make) are needed when
-  // they arrive.
   Frag8 kreg[D][KCH];
   Frag4 vreg[D][DBL];
-#define TK_TILE_ADDR(T_)                                                  \
-    const int c0_ = k_begin + (T_) * 16;                                    \
-    const int page_ = table[c0_ / ps];                                      \
-    const int off_ = c0_ % ps;
-#define TK_LOAD_K(SLOT_, T_)                                                                          \
+  // (a uniform base and one 32-bit lane offset a load: the registers of 64-bit addresses would cost a block a CU)
+  const uint32_t k_lane = (uint32_t)(kb * ps + col) * 16u, v_lane = (uint32_t)(kb * 64 + col * 4) * 2u;
+#define TK_LOAD_K(SLOT_, I_)                                                                          \
   {                                                                                                   \
-    TK_TILE_ADDR(T_)                                                                                  \
-    const bf16_t* kp_ = k_cache + (size_t)page_ * page_elems + head_off + (size_t)(off_ + col) * 8;   \
+    const int off_ = (t_first + (I_) * t_stride) * 16 % ps;                                           \
+    const char* kp_ = reinterpret_cast<const char*>(k_cache + (size_t)page[SLOT_] * page_elems + head_off + (size_t)off_ * 8); \
     _Pragma("unroll") for (int c = 0; c < KCH; ++c) kreg[SLOT_][c].w = __builtin_nontemporal_load(    \
-        reinterpret_cast<const u32x4*>(kp_ + (size_t)(c * 4 + kb) * ps * 8));                         \
+        reinterpret_cast<const u32x4*>(kp_ + (size_t)c * 64 * ps + k_lane));                          \
   }
   // V page [hd/16][ps/4][16][4]: lane (dim col, quad kb) of block d reads 8 bytes, the wave 512
   // contiguous bytes
-#define TK_LOAD_V(SLOT_, T_)                                                                          \
+#define TK_LOAD_V(SLOT_, I_)                                                                          \
   {                                                                                                   \
-    TK_TILE_ADDR(T_)                                                                                  \
-    const bf16_t* vp_ =                                                                               \
-        v_cache + (size_t)page_ * page_elems + head_off + (size_t)((off_ >> 2) + kb) * 64 + col * 4;  \
+    const int off_ = (t_first + (I_) * t_stride) * 16 % ps;                                           \
+    const char* vp_ = reinterpret_cast<const char*>(v_cache + (size_t)page[SLOT_] * page_elems + head_off + (size_t)(off_ >> 2) * 64); \
     _Pragma("unroll") for (int d = 0; d < DBL; ++d) vreg[SLOT_][d].w = __builtin_nontemporal_load(    \
-        reinterpret_cast<const u32x2*>(vp_ + (size_t)d * (ps >> 2) * 64));                            \
+        reinterpret_cast<const u32x2*>(vp_ + (size_t)d * ps * 32 + v_lane));                          \
   }
 
 #pragma unroll
   for (int i = 0; i < D; ++i)
-    if (t_begin + i < t_end) {
-      TK_LOAD_K(i, t_begin + i)
-      TK_LOAD_V(i, t_begin + i)
+    if (i < own) {
+      TK_LOAD_K(i, i)
+      TK_LOAD_V(i, i)
+      page[i] = page_of(t_first + (i + D) * t_stride);
     }
 
   // Q as B operand: lane (col, kb) holds Q[col][c*32 + kb*8 .. +8]
   bf16x8 qreg[KCH];
-  bool stores = false;    // FUSED: this call stores the token's key and value
   bf16_t* s_new = nullptr;  // FUSED: [G + 2][HD] in LDS: the group's queries, then the new key and value
   if constexpr (FUSED) {
     s_new = reinterpret_cast<bf16_t*>(s_dyn + (size_t)WAVES * G * HD + 2 * WAVES * 16);
-    stores = in.nkv_in > 0;
-    const int heads_in = nh + 2 * in.nkv_in;
-    const size_t row_offset = (size_t)n0 * heads_in * HD;
-    if (wave < G + (stores ? 2 : 0)) {
-      float x0, x1;
-      if (wave < G)
-        decode_head_vector<HD>(in, row_offset, kvh * G + wave, in.q_weight, in.rot != 0, n0, lane, x0, x1);
-      else if (wave == G)
-        decode_head_vector<HD>(in, row_offset, nh + kvh, in.k_weight, in.rot != 0, n0, lane, x0, x1);
-      else
-        decode_head_vector<HD>(in, row_offset, nh + in.nkv_in + kvh, nullptr, false, n0, lane, x0, x1);
-      if (lane < HD / 2)
-        *reinterpret_cast<uint32_t*>(s_new + (size_t)wave * HD + 2 * lane) = pack_bf16x2(x0, x1);
+#pragma unroll
+    for (int u = 0; u < MOST; ++u) {
+      const int v = wave + u * WAVES;
+      if (v < vectors) {
+        float x0, x1;
+        finish_head_vector<HD>(head_in[u], in, row_offset, column_of(v), weight_of(v) != nullptr, v <= G && in.rot != 0, lane, x0, x1);
+        if (lane < HD / 2) *reinterpret_cast<uint32_t*>(s_new + (size_t)v * HD + 2 * lane) = pack_bf16x2(x0, x1);
+      }
     }
     __syncthreads();
     // the block that holds the token's position writes its key and value to the page
-    if (stores && wave == 0 && lane < HD / 2 && k_begin <= pos0 && pos0 < k_begin + share) {
+    if (stores && wave == 0 && lane < HD / 2 && pos0 / kRoundKeys % nsplit == split) {
       const int page = table[pos0 / ps], off = pos0 % ps, d = 2 * lane;
       bf16_t* kp = const_cast<bf16_t*>(k_cache_in) + (size_t)page * page_elems + head_off;
       bf16_t* vp = const_cast<bf16_t*>(v_cache_in) + (size_t)page * page_elems + head_off;
@@ -253,12 +282,12 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
 #pragma unroll
   for (int d = 0; d < DBL; ++d) acc[d] = float4v{0.f, 0.f, 0.f, 0.f};
 
-  for (int t0 = t_begin; t0 < t_end; t0 += D) {
+  for (int t0 = 0; t0 < own; t0 += D) {
 #pragma unroll
     for (int i = 0; i < D; ++i) {
       const int t = t0 + i;
-      if (t >= t_end) break;  // the same for every lane of the wave
-      const int c0 = k_begin + t * 16;
+      if (t >= own) break;  // the same for every lane of the wave
+      const int c0 = (t_first + t * t_stride) * 16;
       const bool edge = c0 + 15 > pos0;  // some key of this tile lies past the token's position
       if constexpr (FUSED) {
         // the token's own key and value come from LDS (the page's slot is being written, or was not yet)
@@ -282,7 +311,7 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
 #pragma unroll
       for (int c = 0; c < KCH; ++c) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kreg[i][c].v, qreg[c], sc, 0, 0, 0);
       // the slot's keys have been used: its next tile's keys fly while the others are multiplied
-      if (t + D < t_end) TK_LOAD_K(i, t + D)
+      if (t + D < own) TK_LOAD_K(i, t + D)
       float sv[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -321,12 +350,14 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
         a[3] *= alpha;
         acc[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(tv, pb.v, a, 0, 0, 0);
       }
-      if (t + D < t_end) TK_LOAD_V(i, t + D)
+      if (t + D < own) {
+        TK_LOAD_V(i, t + D)
+        page[i] = page_of(t_first + (t + 2 * D) * t_stride);
+      }
     }
   }
 #undef TK_LOAD_V
 #undef TK_LOAD_K
-#undef TK_TILE_ADDR
 
   // The waves' shares meet in LDS: acc[d][e] = O^T[dim = d*16 + kb*4 + e][col], unnormalised,
   // relative to the wave's own maximum m_run (-inf and zeros for a wave without a tile).
@@ -348,37 +379,34 @@ __global__ __launch_bounds__(WAVES * 64) void attention_decode_kernel(
   }
   __syncthreads();
   // thread t sums four dims of one head over the waves
-  const int t = threadIdx.x;
-  if (t >= G * (HD / 4)) return;
-  const int head = t / (HD / 4), dim = (t % (HD / 4)) * 4;
-  float m_all = s_m[head];
+  for (int t = threadIdx.x; t < G * (HD / 4); t += WAVES * 64) {
+    const int head = t / (HD / 4), dim = (t % (HD / 4)) * 4;
+    float m_all = s_m[head];
 #pragma unroll
-  for (int w = 1; w < WAVES; ++w) m_all = fmaxf(m_all, s_m[w * 16 + head]);  // finite: wave 0 has a tile
-  float l_all = 0.f;
-  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int w = 1; w < WAVES; ++w) m_all = fmaxf(m_all, s_m[w * 16 + head]);  // finite: wave 0 has a tile
+    float l_all = 0.f;
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-  for (int w = 0; w < WAVES; ++w) {
-    const float weight = fast_exp2(s_m[w * 16 + head] - m_all);  // exp2(-inf) = 0 for a wave without a tile
-    l_all = fmaf(weight, s_l[w * 16 + head], l_all);
-    const float4 v = *reinterpret_cast<const float4*>(s_acc + ((size_t)w * G + head) * HD + dim);
-    o.x = fmaf(weight, v.x, o.x);
-    o.y = fmaf(weight, v.y, o.y);
-    o.z = fmaf(weight, v.z, o.z);
-    o.w = fmaf(weight, v.w, o.w);
-  }
-  const size_t row = (size_t)n0 * nh + kvh * G + head;
-  const size_t prow = ((size_t)item * nh + kvh * G + head) * nsplit + split;  // partials are indexed by item, not token
-  if (nsplit == 1) {
-    // a sink is one more term of the head's denominator (the maximum and the sums are in powers of two)
-    if (sinks) l_all += fast_exp2(sinks[kvh * G + head] * 1.4426950408889634f - m_all);
-    const float inv = 1.f / l_all;
-    *reinterpret_cast<uint2*>(out + row * HD + dim) =
-        make_uint2(pack_bf16x2(o.x * inv, o.y * inv), pack_bf16x2(o.z * inv, o.w * inv));
-  } else {
-    *reinterpret_cast<float4*>(part_o + prow * HD + dim) = o;
-    if (dim == 0) {
-      part_ml[prow * 2] = m_all;
-      part_ml[prow * 2 + 1] = l_all;
+    for (int w = 0; w < WAVES; ++w) {
+      const float weight = fast_exp2(s_m[w * 16 + head] - m_all);  // exp2(-inf) = 0 for a wave without a tile
+      l_all = fmaf(weight, s_l[w * 16 + head], l_all);
+      const float4 v = *reinterpret_cast<const float4*>(s_acc + ((size_t)w * G + head) * HD + dim);
+      o.x = fmaf(weight, v.x, o.x);
+      o.y = fmaf(weight, v.y, o.y);
+      o.z = fmaf(weight, v.z, o.z);
+      o.w = fmaf(weight, v.w, o.w);
+    }
+    const size_t row = (size_t)n0 * nh + kvh * G + head;
+    const size_t prow = ((size_t)item * nh + kvh * G + head) * nsplit + split;  // partials are indexed by item, not token
+    if (last_split == 0) {      // (the token's only split that holds keys)
+      // a sink is one more term of the head's denominator (the maximum and the sums are in powers of two)
+      if (sinks) l_all += fast_exp2(sinks[kvh * G + head] * 1.4426950408889634f - m_all);
+      const float inv = 1.f / l_all;
+      *reinterpret_cast<uint2*>(out + row * HD + dim) =
+          make_uint2(pack_bf16x2(o.x * inv, o.y * inv), pack_bf16x2(o.z * inv, o.w * inv));
+    } else {
+      *reinterpret_cast<float4*>(part_o + prow * HD + dim) = o;
+      if (dim == 0) *reinterpret_cast<float2*>(part_ml + prow * 2) = make_float2(m_all, l_all);
     }
   }
 }
@@ -409,7 +437,7 @@ __global__ __launch_bounds__(64) void attention_merge_kernel(
   // token's position: the first splits' partials are asked for before the position is known
   // (one memory round trip instead of three in a row; what a split that does not count left
   // there is not used).
-  constexpr int kAhead = 8;
+  constexpr int kAhead = 16;
   const float* ml = part_ml + row * nsplit * 2;
   const float* po0 = part_o + row * nsplit * HD;
   float m_first = -INFINITY, l_first = 0.f;
@@ -422,9 +450,10 @@ __global__ __launch_bounds__(64) void attention_merge_kernel(
   for (int t = 0; t < kAhead; ++t)
 #pragma unroll
     for (int i = 0; i < HD / 64; ++i) ahead[t][i] = t < nsplit ? po0[(size_t)t * HD + lane + i * 64] : 0.f;
-  // splits that hold keys: of a decode token by its own even cut, of a tile by the step's
+  // splits that hold keys: of a decode token by its own rounds, of a tile by the step's cut
   const int pos = positions[n];
-  const int used = min(nsplit, pos / (item_count == nullptr ? decode_share(pos + 1, nsplit) : split_keys) + 1);
+  const int used = item_count == nullptr ? used_splits(pos, nsplit) : min(nsplit, pos / split_keys + 1);
+  if (item_count == nullptr && used == 1) return;      // (its block has written the result)
   // lane s holds split s's (m, l): one load each, then the maximum over the wave
   float mx = lane < used ? m_first : -INFINITY;
   for (int s = lane + kWave; s < used; s += kWave) mx = fmaxf(mx, ml[s * 2]);
@@ -1405,17 +1434,21 @@ template <int HD, bool FUSED>
 static int launch(const void* q, const void* k_cache, const void* v_cache, const int* block_tables,
                   int max_pages, const int* positions, const int* req_of_token,
                   const int* item_token, const int* item_count, int num_items, void* out,
-                  float* part_o, float* part_ml, int nsplit, int split_keys, int nh, int nkv, int ps,
+                  float* part_o, float* part_ml, int nsplit, int nh, int nkv, int ps,
                   float scale, hipStream_t stream, const float* sinks, float softcap, DecodeInputs in = DecodeInputs{}) {
   if (num_items > 65535) return -1;
   // (the fused form has no capped instance: its entry point takes no cap)
   const bool capped = !FUSED && softcap > 0.f;
-  auto* const kernel = capped ? &attention_decode_kernel<HD, kDecodeWaves, 1, FUSED, !FUSED>
-                              : &attention_decode_kernel<HD, kDecodeWaves, 1, FUSED, false>;
+  auto* const kernel = capped ? &attention_decode_kernel<HD, kDecodeWaves, kDecodeTiles, FUSED, !FUSED>
+                              : &attention_decode_kernel<HD, kDecodeWaves, kDecodeTiles, FUSED, false>;
   dim3 grid(nkv, num_items, nsplit);
   const int G = nh / nkv;
-  // sixteen waves a block and one tile a wave in flight measured best at every batch size
-  // (four or eight waves with two tiles: 12 % slower at batch 64, 15 % at batch 8)
+  // Eight waves a block and two tiles a wave in flight (138 registers: a block or, where it fits, two a CU).  A CU alone pulls
+  // some 60 GB/s whatever is in flight, so few requests are split down to a round of 128 keys a block; sixteen waves of
+  // one tile, whose round is 256 keys, took 10.1 us for one request of 540 keys, these 7.8 (with the merge), 14.5 and 12.3
+  // for eight of 222 to 1,500, 19.9 and 18.0 for 64 of 25 to 700, 90 and 91 for 64 of 2,058; three or four tiles a
+  // wave are 1 to 5 % behind, four waves 5 to 20 %.  A merge by the block that finishes last instead of a kernel of
+  // its own needs a fence over the dies' caches: 2 us more at three splits, 45 us more with 8 requests.
   const size_t lds = (size_t)(kDecodeWaves * G * HD + 2 * kDecodeWaves * 16) * 4 + (FUSED ? (size_t)(G + 2) * HD * 2 : 0);
   if (lds > 160 * 1024) return -2;
   if (lds > 48 * 1024) {  // beyond the default limit of dynamic LDS (groups of 7 heads and more)
@@ -1431,20 +1464,19 @@ static int launch(const void* q, const void* k_cache, const void* v_cache, const
   }
   kernel<<<grid, kDecodeWaves * 64, lds, stream>>>(
       (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, max_pages, positions,
-      req_of_token, item_token, item_count, (bf16_t*)out, part_o, part_ml, nsplit, split_keys, nh, nkv, ps,
+      req_of_token, item_token, item_count, (bf16_t*)out, part_o, part_ml, nsplit, nh, nkv, ps,
       scale * 1.4426950408889634f, in, sinks, soft_cap(scale, softcap));
   if (nsplit > 1) {
     dim3 mgrid(num_items, nh);
     attention_merge_kernel<HD><<<mgrid, 64, 0, stream>>>(part_o, part_ml, positions, item_token, nullptr,
-                                                         (bf16_t*)out, nsplit, split_keys, nh, sinks);
+                                                         (bf16_t*)out, nsplit, kRoundKeys, nh, sinks);
   }
   return launch_status();
 }
 
-// mode 0: heads (every item is one decode token; item_count is ignored; split_keys is a multiple of
-//         16 * tk_attention_decode_waves(), a tile for every wave of a block, and nsplit of them
-//         cover the longest token; with nsplit > 1 every token's own keys are cut evenly in
-//         nsplit, see decode_share)
+// mode 0: heads (every item is one decode token; item_count is ignored; with nsplit > 1 every token's own
+//         keys are dealt to nsplit blocks in rounds of 16 * tk_attention_decode_waves(), whatever split_keys
+//         says; req_of_token may be null: token n is then request n's)
 // mode 1: tokens (item = up to 16 consecutive tokens of one request; with nsplit > 1 split_keys
 //         is a multiple of 64 and the partial buffers hold 16 rows per item)
 // mode 2: tokens, every tile over a long context (same results; the kernel built for four waves a SIMD)
@@ -1472,7 +1504,7 @@ TK_API int tk_attention_mfma(int mode, const void* q, const void* k_cache, const
   const int G = nh / nkv;
 #define TK_ARGS                                                                                   \
   q, k_cache, v_cache, block_tables, max_pages, positions, req_of_token, item_token, item_count, \
-      num_items, out, part_o, part_ml, nsplit, split_keys, nh, nkv, ps, scale, stream, sinks, softcap
+      num_items, out, part_o, part_ml, nsplit, nh, nkv, ps, scale, stream, sinks, softcap
   if (mode == 0) {
     if (G > 16) return -2;
     if (hd == 128) return launch<128, false>(TK_ARGS);
@@ -1540,21 +1572,21 @@ TK_API int tk_attention_decode_fused(const void* qkv, int in_f32, int parts, lon
                                      const float* sin_t, int rot, float eps, int nkv_in, void* k_cache,
                                      void* v_cache, const int* block_tables, int max_pages,
                                      const int* positions, const int* req_of_token, const int* item_token,
-                                     int num_items, void* out, float* part_o, float* part_ml, int nsplit,
-                                     int split_keys, int nh, int nkv, int hd, int ps, float scale,
+                                     int num_items, void* out, float* part_o, float* part_ml,
+                                     int nsplit, int split_keys, int nh, int nkv, int hd, int ps, float scale,
                                      hipStream_t stream) {
   if (num_items <= 0) return 0;
-  if (nkv <= 0 || nh % nkv != 0 || ps < 16 || (ps & (ps - 1)) != 0 || split_keys % (16 * kDecodeWaves) != 0 || nsplit < 1)
+  if (nkv <= 0 || nh % nkv != 0 || ps < 16 || (ps & (ps - 1)) != 0 || split_keys % 16 != 0 || nsplit < 1)
     return -1;
   if (num_items > 65535 || nh > 65535 || parts < 1 || (parts > 1 && !in_f32)) return -1;
   if ((nkv_in != 0 && nkv_in != nkv) || (rot != 0 && rot != hd) || (rot != 0 && (!cos_t || !sin_t))) return -1;
   if ((q_weight != nullptr) != (k_weight != nullptr) && nkv_in != 0) return -1;
   const int G = nh / nkv;
-  if (G + 2 > kDecodeWaves) return -2;
+  if (G > 14) return -2;
   DecodeInputs in{qkv, in_f32, parts, part_stride, q_weight, k_weight, cos_t, sin_t, rot, nkv_in, eps};
 #define TK_FARGS                                                                                       \
   nullptr, k_cache, v_cache, block_tables, max_pages, positions, req_of_token, item_token, nullptr,  \
-      num_items, out, part_o, part_ml, nsplit, split_keys, nh, nkv, ps, scale, stream, nullptr, 0.f, in
+      num_items, out, part_o, part_ml, nsplit, nh, nkv, ps, scale, stream, nullptr, 0.f, in
   if (hd == 128) return launch<128, true>(TK_FARGS);
   if (hd == 64) return launch<64, true>(TK_FARGS);
 #undef TK_FARGS

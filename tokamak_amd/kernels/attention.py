@@ -15,7 +15,7 @@ TILE_TOKENS = 16   # tokens per attention tile of a prompt portion (csrc/attenti
 WIDE_TOKENS = 32   # and per tile of the wide matrix-core kernel
 
 MFMA_HEAD_DIMS = (64, 128)
-DECODE_WAVES = 16           # waves of a decode block (csrc/attention_mfma.hip: kDecodeWaves)
+DECODE_WAVES = 8            # waves of a decode block (csrc/attention_mfma.hip: kDecodeWaves)
 TILE_SPLIT_UP_TO_BLOCKS = 640   # a portion with no more blocks of the narrow form than this has its keys split ...
 TILE_SPLIT_MIN_KEYS = 512       # ... into pieces no shorter than this (twice this from TILE_SPLIT_FEW_BLOCKS blocks on) ...
 TILE_SPLIT_FEW_BLOCKS = 128
@@ -168,7 +168,7 @@ def mfma_fits(dtype, head_dim, page_size, group, window) -> bool:
 # 1 to 8 requests up to 32,768 keys: the cheapest split by this price is on average 1 % and at
 # worst 18 % slower than the best measured one; the rule it replaced, "as few splits as put
 # 4,096 waves on the GPU", 5 % and 49 % on such cases).
-DECODE_CUS = 256                 # blocks that run at once: a block of sixteen waves has a CU to itself
+DECODE_CUS = 256                 # blocks that run at once at full rate
 DECODE_RATE = 5.8e12             # bytes a second of a round of DECODE_CUS blocks
 DECODE_BLOCK_RATE = 60e9         # ... and of one block with the GPU to itself
 DECODE_START = 3e-6              # a launch
@@ -283,7 +283,8 @@ def decode_attention_fused(qkv, q_weight, k_weight, cos, sin, k_cache, v_cache, 
         ops._note(f"decode {work.num_single} tokens, fused", keys * 2 * num_kv_heads * head_dim * 2,
                   keys * 4.0 * num_heads * head_dim)
     return ops.attention_decode_fused(
-        qkv, q_weight, k_weight, cos, sin, k_cache, v_cache, block_tables, batch.positions, batch.req_of_token,
+        qkv, q_weight, k_weight, cos, sin, k_cache, v_cache, block_tables, batch.positions,
+        None,       # (every request of such a step brings one token: token n is request n's)
         work.single, work.num_single, out, num_heads=num_heads, num_kv_heads=num_kv_heads,
         head_dim=head_dim, rotary_dim=rotary_dim, page_size=page_size, eps=eps, scale=scale, store=store,
         split_keys=split, num_splits=nsplit)
@@ -410,7 +411,7 @@ def _paged_attention_mfma(q, k_cache, v_cache, block_tables, batch, work, out, *
         if note is not None:
             ops._note(f"decode {work.num_single} tokens", decode_keys * kv_token_bytes, decode_keys * flops_per_pair)
         if not ops.attention_mfma("heads", q, k_cache, v_cache, block_tables, batch.positions,
-                                  batch.req_of_token, work.single, None, work.num_single, out,
+                                  batch.req_of_token if work.num_single < batch.num_tokens else None, work.single, None, work.num_single, out,
                                   split_keys=split, num_splits=nsplit, **common):
             return False
     if work.num_tiles:

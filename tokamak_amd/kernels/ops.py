@@ -2317,7 +2317,7 @@ def attention_tiles(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
 
 
 def attention_mfma(mode: str, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
-                   block_tables: torch.Tensor, positions: torch.Tensor, req_of_token: torch.Tensor,
+                   block_tables: torch.Tensor, positions: torch.Tensor, req_of_token: torch.Tensor | None,
                    item_token: torch.Tensor, item_count: torch.Tensor | None, num_items: int,
                    out: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim: int,
                    page_size: int, scale: float, split_keys: int = 256, num_splits: int = 1,
@@ -2329,8 +2329,8 @@ def attention_mfma(mode: str, q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
     "tokens_group": the same items, a block of up to eight waves holding all query heads of
     a kv head and shares of the keys, any group size).  With ``num_splits`` > 1 the keys of an item are cut into pieces of
     ``split_keys`` (a multiple of 16; of 64 in "tokens" mode), each its own block, and a
-    second kernel merges the pieces (in "heads" mode the sixteen waves of a block share a piece, so
-    ``split_keys`` is a multiple of 256).  ``chunk`` ("tokens" and "tokens_dense" without splits): a
+    second kernel merges the pieces (in "heads" mode the eight waves of a block share a piece, so
+    ``split_keys`` is a multiple of 128, and a token's keys are dealt to the pieces in rounds of 128).  ``req_of_token`` None ("heads" mode): token n is request n's.  ``chunk`` ("tokens" and "tokens_dense" without splits): a
     query sees the keys of its own chunk of that many positions only.  ``sinks``: float32
     [num_heads], one more term exp(sinks[a]) of head a's denominator.  ``softcap`` c: every score becomes
     c tanh(score / c) first.  Returns False (nothing
@@ -2345,13 +2345,15 @@ def attention_mfma(mode: str, q: torch.Tensor, k_cache: torch.Tensor, v_cache: t
           and split_keys % 16 == 0, "bad head counts, page size (a power of two >= 16) or split")
     page_elems = num_kv_heads * head_dim * page_size
     _need(k_cache.numel() % page_elems == 0 and v_cache.numel() == k_cache.numel(), "cache size is not whole pages")
-    _need(positions.dtype == torch.int32 and req_of_token.dtype == torch.int32 and block_tables.dtype == torch.int32
+    _need(req_of_token.dtype == torch.int32 if req_of_token is not None else mode == "heads" and block_tables.shape[0] >= n,
+          "the tokens' requests are int32 (or, for decode tokens that are their requests, not given)")
+    _need(positions.dtype == torch.int32 and block_tables.dtype == torch.int32
           and item_token.dtype == torch.int32 and block_tables.dim() == 2, "descriptor arrays are int32")
     _need(item_token.numel() >= num_items and 0 < num_items <= 65535, "bad item list")
     _need(mode in ("heads", "tokens", "tokens_dense", "tokens_wide", "tokens_group"),
           "mode is heads, tokens, tokens_dense, tokens_wide or tokens_group")
     _need(mode not in ("tokens_wide", "tokens_group") or num_splits == 1, "the wide and group forms do not split keys over blocks")
-    _need(mode != "heads" or num_splits == 1 or split_keys % 256 == 0, "heads mode splits keys in multiples of 256")
+    _need(mode != "heads" or num_splits == 1 or split_keys % 128 == 0, "heads mode splits keys in multiples of 128")
     _need(not chunk or (mode in ("tokens", "tokens_dense") and num_splits == 1 and chunk > 0),
           "chunked visibility: tiles of 16 tokens, keys not split")
     if mode != "heads":
@@ -2421,7 +2423,7 @@ FUSED_DECODE_MAX_GROUP = 14   # query heads per kv head the fused decode kernel 
 def attention_decode_fused(qkv: torch.Tensor, q_weight: torch.Tensor | None, k_weight: torch.Tensor | None,
                            cos: torch.Tensor | None, sin: torch.Tensor | None, k_cache: torch.Tensor,
                            v_cache: torch.Tensor, block_tables: torch.Tensor, positions: torch.Tensor,
-                           req_of_token: torch.Tensor, item_token: torch.Tensor, num_items: int,
+                           req_of_token: torch.Tensor | None, item_token: torch.Tensor, num_items: int,
                            out: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim: int,
                            rotary_dim: int, page_size: int, eps: float, scale: float, store: bool,
                            split_keys: int, num_splits: int) -> bool:
@@ -2429,7 +2431,7 @@ def attention_decode_fused(qkv: torch.Tensor, q_weight: torch.Tensor | None, k_w
     rotation of the queries (and, with ``store``, of the token's key, which is written to
     its page with the value), then attention over the pages as ``attention_mfma("heads")``.
     ``qkv``: [N, (nh + 2 nkv) hd] bfloat16, or float32 partial sums [P, N, ...] (without
-    ``store`` the rows hold queries only).  Returns False (nothing launched) if the shape is
+    ``store`` the rows hold queries only).  ``req_of_token`` None: token n is request n's.  Returns False (nothing launched) if the shape is
     not instantiated; the caller then runs the two kernels."""
     _gpu(qkv, q_weight, k_weight, cos, sin, k_cache, v_cache, block_tables, positions, req_of_token, item_token, out)
     n = positions.numel()
@@ -2451,10 +2453,12 @@ def attention_decode_fused(qkv: torch.Tensor, q_weight: torch.Tensor | None, k_w
     _need((q_weight is None) == (k_weight is None), "q and k are normed together or not at all")
     page_elems = num_kv_heads * head_dim * page_size
     _need(k_cache.numel() % page_elems == 0 and v_cache.numel() == k_cache.numel(), "cache size is not whole pages")
-    _need(positions.dtype == torch.int32 and req_of_token.dtype == torch.int32 and block_tables.dtype == torch.int32
+    _need(req_of_token.dtype == torch.int32 if req_of_token is not None else block_tables.shape[0] >= n,
+          "the tokens' requests are int32 (or, for tokens that are their requests, not given)")
+    _need(positions.dtype == torch.int32 and block_tables.dtype == torch.int32
           and item_token.dtype == torch.int32 and block_tables.dim() == 2, "descriptor arrays are int32")
     _need(item_token.numel() >= num_items and 0 < num_items <= 65535, "bad item list")
-    _need(split_keys % 256 == 0 and num_splits >= 1, "splits are multiples of 256 keys")
+    _need(split_keys % 128 == 0 and num_splits >= 1, "splits are multiples of 128 keys")
     part_o = part_ml = None
     if num_splits > 1:
         rows = num_items * num_heads * num_splits
