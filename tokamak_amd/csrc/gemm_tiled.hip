@@ -228,125 +228,147 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
       }
 }
 
-// Few rows (M <= 16, float32): the tiles above leave most of a block idle.  Here a wave owns 64 weight rows, a lane one of
-// them, and walks them 32 k at a time; the activations are the same for every lane (the compiler reads them through
-// the scalar path).  The order of the sum is the one of the tiled kernel, bit for bit: k ascending within a piece of
-// kPiece, the pieces' sums added to the total one after the other; so a row's result is still the same whatever the batch holds.
-// With `partial` a wave sums one piece only and writes it to partial[piece][M][N]; the second
-// kernel adds the pieces in order (for matrices of too few rows to fill the GPU otherwise).
+// Few rows (M <= 16, float32): the tiles above leave most of a block idle.  v_mfma_f32_16x16x4_f32 too gives the bits of
+// fmaf over its four k in ascending order, so a wave that takes a piece of kPiece k four at a time forms the piece's sum as
+// the tiled kernel does, and the pieces' sums are added to the total in their order, bit for bit; a row's result is still
+// the same whatever the batch holds.
 //
-// Bound by the weights' bytes.  A tile of 64 rows by 32 k is loaded as whole cache lines (eight lanes a row's 128 bytes),
-// two tiles ahead, and changes hands through the wave's own LDS (rows 36 floats apart: sixteen lanes' pieces lie in
-// different banks).  Lanes that loaded from a row each touched 64 lines a load (4 rows:
-// weights of 4,096 x 2,048 19.8 us, now 13.1, both kernels; 12,288 x 2,048 27.2, 23.0; 151,936 x 2,048 257, 235, and 425, 248 for 8 rows).
-constexpr int kFewK = 32, kFewPitch = kFewK + 4;
-template <int MT>
-__global__ __launch_bounds__(64) void gemm_fewrows_kernel(const float* __restrict__ A,
-                                                          const float* __restrict__ W,
-                                                          float* __restrict__ C, float* __restrict__ partial,
-                                                          int M, int N, int K, long lda, long ldw, long ldc) {
+// Bound by the weights' bytes, and for small matrices by the trips to memory.  An operand's sixteen rows are J = 16 / TP
+// pieces of K of TP weight rows, its columns the same pieces of TP rows of activations; the blocks on the
+// result's diagonal are kept.  Groups of 4 or 8 rows give small matrices four and two times the blocks.  A block's waves
+// take J pieces each a round; a round's sums meet in LDS, where one wave adds them in order.  Blocks walk over
+// groups of rows, loads running ahead over their borders.  Weights come as 256 contiguous bytes of four rows a load, two
+// or four stages of 64 k ahead, and change hands through the wave's own LDS (rows 68 floats apart: 64 banks); the activations'
+// four numbers a lane become the four k of a step by swaps between the lanes of a column.
+// (In the form before, a lane owned a weight row and multiplied in the vector unit, 64 rows and a piece a wave, the pieces' sums
+// through memory to a kernel of their own: us there and here, 4 rows, 2,048 x 2,048 17.8 and 6.7, 4,096 x 2,048 16.9 and 8.6,
+// 2,048 x 6,144 20.2 and 13.1, 12,288 x 2,048 23.8 and 19.3, 151,936 x 2,048 233 and 193.)
+template <int TP, int WAVES, int DEPTH>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2))) void gemm_fewrows_kernel(
+    const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N, int K, long lda, long ldw,
+    long ldc) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
-  static_assert(kPiece % (2 * kFewK) == 0, "a piece is whole pairs of tiles");
-  __shared__ __attribute__((aligned(16))) float tile[64 * kFewPitch];
-  const int lane = threadIdx.x;
-  const int n0 = blockIdx.x * 64, n = n0 + lane;
-  const int pieces = (K + kPiece - 1) / kPiece;
-  const int k_begin = (partial ? blockIdx.y : 0) * kPiece;
-  const int k_end = min(K, (partial ? (int)blockIdx.y + 1 : pieces) * kPiece);
-  // (rows past N are computed from a valid row and never stored; what lies past K is read at the row's end, not used)
-  const float* from[8];
+  constexpr int J = 16 / TP, STAGES = kPiece / 64, PITCH = 68, QUADS = TP / 4;
+  static_assert(kPiece == 256 && (DEPTH == 2 || DEPTH == 4), "a piece is four stages of 64 k");
+  __shared__ __attribute__((aligned(16))) float tile[WAVES][16 * PITCH];
+  __shared__ __attribute__((aligned(16))) f32x4 sums[2][WAVES * J][TP * QUADS];   // of a round: [piece][row of activations, four weight rows]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int a = lane & 15, g = lane >> 4;
+  const int pieces = (K + kPiece - 1) / kPiece, rounds = (pieces + WAVES * J - 1) / (WAVES * J);
+  const int groups = (N + TP - 1) / TP;
+  const int visits = (groups - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x * rounds;   // (group, round) pairs of this block
+
+  // this lane's place: of the loads of weights row 4 i + lane / 16 of the operand, of those of activations column a
+  const int wk = a * 4, own_m = min(a % TP, M - 1);
+  const float* const arow = A + (size_t)own_m * lda;
+  f32x4 wreg[DEPTH][4], areg[DEPTH][4];
+  // What a visit reads: the rows of its group, the first k of its pieces.  A piece past the last is never read (first k >= K);
+  // rows past N are read at the last row and never stored, what lies past K is read at the row's end and becomes zero.
+  const auto first_k = [&](int round, int share) { return ((round * WAVES + wave) * J + share) * kPiece; };
+  const auto fetch = [&](int group, int round, int stage, int buf) {
+    if (first_k(round, 0) >= K) return;      // (uniform)
 #pragma unroll
-  for (int i = 0; i < 8; ++i) from[i] = W + (size_t)min(n0 + 8 * i + lane / 8, N - 1) * ldw;
-  const int col = lane % 8 * 4;
-  f32x4 reg[2][8];
-  const auto fetch = [&](f32x4 (&r)[8], int k0) {
-    const int k = min(k0 + col, K - 4);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(from[i] + k));
-  };
-  float acc[MT], total[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) acc[m] = total[m] = 0.f;
-  const auto step = [&](int k, int at) {
-    const f32x4 w = *reinterpret_cast<const f32x4*>(tile + lane * kFewPitch + at);
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const float4 a = *reinterpret_cast<const float4*>(A + (size_t)min(m, M - 1) * lda + k);
-      acc[m] = fmaf(a.x, w[0], acc[m]);
-      acc[m] = fmaf(a.y, w[1], acc[m]);
-      acc[m] = fmaf(a.z, w[2], acc[m]);
-      acc[m] = fmaf(a.w, w[3], acc[m]);
+    for (int i = 0; i < 4; ++i) {
+      const int row = 4 * i + g;
+      const int n = min(group * TP + row % TP, N - 1), k = min(first_k(round, row / TP) + 64 * stage + wk, K - 4);
+      wreg[buf][i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(W + (size_t)n * ldw + k));
     }
-  };
-  fetch(reg[0], k_begin);
-  if (k_begin + kFewK < k_end) fetch(reg[1], k_begin + kFewK);
-  for (int k0 = k_begin; k0 < k_end; k0 += 2 * kFewK) {
-    if (k0 > k_begin && k0 % kPiece == 0) {
+    const int k0 = first_k(round, a / TP) + 64 * stage + 4 * g;
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        total[m] += acc[m];
-        acc[m] = 0.f;
+    for (int j = 0; j < 4; ++j) areg[buf][j] = *reinterpret_cast<const f32x4*>(arow + min(k0 + 16 * j, K - 4));
+  };
+
+  int group = blockIdx.x, round = 0;
+#pragma unroll
+  for (int s = 0; s < DEPTH; ++s) fetch(group, 0, s, s);
+  f32x4 total = {0.f, 0.f, 0.f, 0.f};
+  for (int v = 0; v < visits; ++v) {
+    const bool turns = round + 1 == rounds, last = v + 1 == visits;
+    const int next_round = turns ? 0 : round + 1, next_group = turns ? group + (int)gridDim.x : group;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    if (first_k(round, 0) < K) {
+      const bool whole = first_k(round, J - 1) + kPiece <= K;
+#pragma unroll
+      for (int s = 0; s < STAGES; ++s) {
+        const int buf = s % DEPTH;
+        float* const mine = tile[wave];
+        wave_lds_sync();      // (the stage before has been read)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          f32x4 w = wreg[buf][i];
+          if (!whole && first_k(round, (4 * i + g) / TP) + 64 * s + wk >= K) w = f32x4{0.f, 0.f, 0.f, 0.f};
+          *reinterpret_cast<f32x4*>(mine + (4 * i + g) * PITCH + wk) = w;
+        }
+        // areg[j][e] holds k = 16 j + 4 g + e; step[j][e] is to hold k = 16 j + 4 e + g
+        uint32_t step[4][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          f32x4 x = areg[buf][j];
+          if (!whole && first_k(round, a / TP) + 64 * s + 16 * j + 4 * g >= K) x = f32x4{0.f, 0.f, 0.f, 0.f};
+          const auto e02 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[0]), __float_as_uint(x[2]), false, false);
+          const auto e13 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[1]), __float_as_uint(x[3]), false, false);
+          const auto e01 = __builtin_amdgcn_permlane16_swap(e02[0], e13[0], false, false);
+          const auto e23 = __builtin_amdgcn_permlane16_swap(e02[1], e13[1], false, false);
+          step[j][0] = e01[0];
+          step[j][1] = e01[1];
+          step[j][2] = e23[0];
+          step[j][3] = e23[1];
+        }
+        if (s + DEPTH < STAGES) fetch(group, round, s + DEPTH, buf);
+        else if (!last) fetch(next_group, next_round, s + DEPTH - STAGES, buf);
+        wave_lds_sync();
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(mine[a * PITCH + 16 * j + 4 * e + g], __uint_as_float(step[j][e]), acc, 0, 0, 0);
+      }
+    } else if (!last) {
+#pragma unroll
+      for (int s = 0; s < DEPTH; ++s) fetch(next_group, next_round, s, s);
+    }
+    // acc[e]: weight row 4 g + e of the operand against column a of the activations
+    if (4 * g / TP == a / TP) sums[v & 1][wave * J + a / TP][a % TP * QUADS + g % QUADS] = acc;
+    __syncthreads();      // (one a round: this copy is written again behind the next round's barrier)
+    if (threadIdx.x < TP * QUADS) {
+      const int left = min(WAVES * J, pieces - round * WAVES * J);
+      for (int p = 0; p < left; ++p) total += sums[v & 1][p][threadIdx.x];
+      if (turns) {
+        const int m = threadIdx.x / QUADS, n = group * TP + threadIdx.x % QUADS * 4;
+        if (m < M && n < N) store_four<float>(C + (size_t)m * ldc + n, total[0], total[1], total[2], total[3], N - n, rows_take_wide_stores(C, ldc));
+        total = f32x4{0.f, 0.f, 0.f, 0.f};
       }
     }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int k = k0 + u * kFewK;
-      if (k >= k_end) break;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(tile + (8 * i + lane / 8) * kFewPitch + col) = reg[u][i];
-      if (k + 2 * kFewK < k_end) fetch(reg[u], k + 2 * kFewK);
-      wave_lds_sync();
-      if (k + kFewK <= k_end) {
-#pragma unroll
-        for (int at = 0; at < kFewK; at += 4) step(k + at, at);
-      } else {
-        for (int at = 0; k + at < k_end; at += 4) step(k + at, at);
-      }
-      wave_lds_sync();
-    }
+    group = next_group;
+    round = next_round;
   }
-  if (n >= N) return;
-  if (partial) {
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-      if (m < M) partial[((size_t)blockIdx.y * M + m) * N + n] = acc[m];
-    return;
-  }
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-    if (m < M) C[(size_t)m * ldc + n] = total[m] + acc[m];
 }
 
-__global__ __launch_bounds__(256) void gemm_fewrows_add_kernel(const float* __restrict__ partial,
-                                                               float* __restrict__ C, int M, int N,
-                                                               int pieces, long ldc) {
-  const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
-  if (n >= N) return;
-  float total = 0.f;
-  for (int p = 0; p < pieces; ++p) total += partial[((size_t)p * M + m) * N + n];
-  C[(size_t)m * ldc + n] = total;
-}
-
-// float32 in and out, M <= 16, K and the row strides multiples of 4, 16-byte aligned rows.
-// partial: null, or room for ceil(K / 256) * M * N floats: then every piece of K has a wave of its own.
-TK_API int tk_gemm_fewrows(const float* A, const float* W, float* C, float* partial, int M, int N, int K,
-                           long lda, long ldw, long ldc, hipStream_t stream) {
+// float32 in and out, M <= 16, K and the row strides multiples of 4, 16-byte aligned rows.  rows: of a group, 4, 8 or 16, at
+// least M; waves a block, 4, 6 or 8; depth: stages of 64 k asked for ahead, 2, or 4 for 16 rows and four waves; blocks: at most so many.
+TK_API int tk_gemm_fewrows(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc, int rows,
+                           int waves, int depth, int blocks, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 16 || K < 4 || K % 4 != 0 || lda % 4 != 0 || ldw % 4 != 0) return -1;
+  if (M > 16 || M > rows || K < 4 || K % 4 != 0 || lda % 4 != 0 || ldw % 4 != 0 || blocks < 1) return -1;
   if (reinterpret_cast<uintptr_t>(A) % 16 != 0 || reinterpret_cast<uintptr_t>(W) % 16 != 0) return -1;
-  const int pieces = (K + kPiece - 1) / kPiece;
-  if (pieces > 65535) return -1;
-  dim3 grid((N + 63) / 64, partial ? pieces : 1);
-#define TK_FEW(MT_) gemm_fewrows_kernel<MT_><<<grid, 64, 0, stream>>>(A, W, C, partial, M, N, K, lda, ldw, ldc)
-  if (M == 1) TK_FEW(1);
-  else if (M == 2) TK_FEW(2);
-  else if (M <= 4) TK_FEW(4);
-  else if (M <= 8) TK_FEW(8);
-  else TK_FEW(16);
+  const int grid = min(blocks, (N + rows - 1) / rows);
+#define TK_FEW(TP_, WAVES_, DEPTH_) \
+  if (rows == TP_ && waves == WAVES_ && depth == DEPTH_) { \
+    gemm_fewrows_kernel<TP_, WAVES_, DEPTH_><<<grid, WAVES_ * 64, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc); \
+    return launch_status(); \
+  }
+  TK_FEW(4, 4, 2)
+  TK_FEW(4, 6, 2)
+  TK_FEW(4, 8, 2)
+  TK_FEW(8, 4, 2)
+  TK_FEW(8, 6, 2)
+  TK_FEW(8, 8, 2)
+  TK_FEW(16, 4, 2)
+  TK_FEW(16, 6, 2)
+  TK_FEW(16, 8, 2)
+  TK_FEW(16, 4, 4)
 #undef TK_FEW
-  if (partial)
-    gemm_fewrows_add_kernel<<<dim3((N + 255) / 256, M), 256, 0, stream>>>(partial, C, M, N, pieces, ldc);
-  return launch_status();
+  return -1;
 }
 
 // in_dtype / out_dtype: 0 = float32, 1 = bfloat16

@@ -255,8 +255,8 @@ _SIGS = {
     "gemm_tiled": {
         "tk_gemm_tiled": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long,
                           c_long, c_long, c_void_p],
-        "tk_gemm_fewrows": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long,
-                            c_long, c_void_p],
+        "tk_gemm_fewrows": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_int, c_int,
+                            c_int, c_void_p],
     },
     "gemm_mfma": {
         "tk_gemm_stream": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long,
@@ -1683,9 +1683,8 @@ def moe_grouped(x: torch.Tensor, weights: torch.Tensor, lists: tuple, pair_weigh
         _p(pair_weight), _p(out), tokens, top, r, k, tile_expert.numel(), tokens * top, tile_pairs, _stream()), "moe_grouped")
 
 
-FEWROWS_MAX_ROWS = 64          # float32 products of up to this many rows stream the weights, a lane a weight row,
-FEWROWS_GROUP = 16             # this many rows a pass over the weights
-FEWROWS_SPLIT_BELOW = 65536    # weight rows below which every piece of 256 k gets a wave of its own
+FEWROWS_MAX_ROWS = 64          # float32 products of up to this many rows stream the weights,
+FEWROWS_GROUP = 16             # this many rows a pass over them
 
 
 def fewrows_pays(m: int, n: int) -> bool:
@@ -1702,11 +1701,37 @@ def fewrows_pays(m: int, n: int) -> bool:
     return True
 
 
+def fewrows_form(m: int, n: int, k: int, small_groups: bool | None = None) -> tuple[int, int, int, int]:
+    """(weight rows of a group, waves a block, stages of 64 k ahead, blocks) of the weight-streaming product; us at 4 rows.
+    Groups: the fewest rows for the CU that has most of them (2,048 x 2,048 in groups of 8 6.7, of 16 7.9; 5,120 x 5,120 in
+    groups of 4 24.3, of 16 29.5), the larger ones unless a smaller one is clearly better (25,600 x 5,120 of 16 92.9, of 8 95.8).
+    Blocks: as many as are on the chip at once, the groups dealt to them (25,600 x 5,120 as 768 blocks 92.9, as 534 with three
+    groups each 116).  Eight waves where no CU has a second block (2,048 x 6,144 13.1, four waves 13.4; at 16 rows 21.9 and
+    25.0), else the four or six that leave fewer idle in the last round (20,000 x 1,028 six 22.8, four 24.9); and for walks of a
+    head's length more loads ahead (151,936 x 2,048 199 -> 193, at 16 rows 268 -> 256)."""
+    least = 4 if m <= 4 else 8 if m <= 8 else 16
+    if small_groups is not None:
+        group = least if small_groups else 16
+    else:
+        group, most = 16, -(-n // (16 * 256)) * 16
+        for g in (8, 4):
+            rows = -(-n // (g * 256)) * g
+            if g >= least and rows < 0.875 * most:
+                group, most = g, rows
+    groups, shares = -(-n // group), -(-k // (256 * (16 // group)))      # shares of K: what a wave takes in a round
+    if group == 16 and groups >= 4096:
+        return group, 4, 4, 512
+    if groups <= 256:
+        return group, 8 if shares > 4 else 4, 2, groups
+    waves = min((6, 4), key=lambda w: -(-shares // w) * w)
+    return group, waves, 2, min(groups, 512 if waves == 6 else 768)
+
+
 def gemm_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, fewrows_split: bool | None = None) -> None:
     """out[M, N] = a[M, K] @ w[N, K]^T, float32 multiply-add (rows may be strided).  float32
     operands of up to 64 rows go to the weight-streaming kernel where that pays
-    (``fewrows_pays``), which gives the same bits (``fewrows_split``: that kernel with a wave
-    per piece of K or not; None chooses the kernel and the split by the shape)."""
+    (``fewrows_pays``), which gives the same bits (``fewrows_split``: that kernel with operands split between as many pieces
+    of K as the rows allow, or not split; None chooses the kernel and the split by the shape)."""
     for t in (a, w, out):
         _need(t.is_cuda and t.dim() == 2 and t.stride(1) == 1, "gemm operands are 2-D GPU tensors with unit inner stride")
     m, k = a.shape
@@ -1718,15 +1743,11 @@ def gemm_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, fewrows_spli
     if (m <= FEWROWS_MAX_ROWS and (fewrows_split is not None or fewrows_pays(m, n))
             and a.dtype == torch.float32 and out.dtype == torch.float32 and k % 4 == 0 and k >= 4
             and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
-        # the same sums in the same order, by a kernel that streams the weights; a wave for every
-        # piece of K where the matrix has too few rows to fill the GPU with a wave per 64 of them
-        pieces = -(-k // 256)
-        split = fewrows_split if fewrows_split is not None else (n < FEWROWS_SPLIT_BELOW and pieces > 1)
+        # the same sums in the same order, by a kernel that streams the weights
         for at in range(0, m, FEWROWS_GROUP):
             rows = min(FEWROWS_GROUP, m - at)
-            partial = torch.empty((pieces, rows, n), dtype=torch.float32, device=a.device) if split else None
-            _check(_fn("gemm_tiled", "tk_gemm_fewrows")(_p(a[at:]), _p(w), _p(out[at:]), _p(partial),
-                                                        rows, n, k, a.stride(0), w.stride(0), out.stride(0), _stream()),
+            _check(_fn("gemm_tiled", "tk_gemm_fewrows")(_p(a[at:]), _p(w), _p(out[at:]), rows, n, k, a.stride(0), w.stride(0),
+                                                        out.stride(0), *fewrows_form(rows, n, k, fewrows_split), _stream()),
                    "gemm_fewrows")
         return
     _check(_fn("gemm_tiled", "tk_gemm_tiled")(_code(a.dtype), _code(out.dtype), _p(a), _p(w), _p(out),
