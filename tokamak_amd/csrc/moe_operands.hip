@@ -23,6 +23,8 @@
 #include "common.h"
 #include "slots.h"
 
+#include <type_traits>
+
 using namespace tk;
 
 namespace {
@@ -213,16 +215,22 @@ constexpr int kXcds = 8;        // dies of the GPU, each with an L2 of its own; 
 constexpr int kTile = 128;      // pairs of a tile
 constexpr int kStep = 64;       // k of a step
 constexpr int kTileWaves = 4;
+__device__ __align__(16) const bf16_t kZeros[32 * kStep] = {};      // a step of 32 rows' weights
 
 // A block: a tile and the channels of its waves: with a gate a wave has 32 channels' gate and up rows, else 64 rows.  The
 // tile's activations go through LDS (two copies, 64 k each, rows' 16-byte pieces swizzled so that sixteen rows' reads of
-// one piece meet all banks), the weights come straight from memory, a step ahead.  Which tile and channels a block has
-// follows moe.hip's tile_of_block: the tiles of an expert at the same channels run side by side on one die.
-// Four waves and two blocks a CU, which wait for barriers of their own; eight waves that share a tile's activations were
-// slower (16 experts of 4,096 x 6,144, 2,000 tokens of two: 592 + 397 us against 569 + 351; rows of weights through the
-// vector memory path, moe.hip, 914 + 568).  Up to some 32 pairs an expert the weights' bytes bound it (512 tokens: 303 +
-// 209 us for 1,610 + 805 MB, 5.3 TB/s; 413 + 260 before), beyond that the walk itself: 0.71 PFLOP/s at 2,000 tokens.
-template <bool GATED>
+// one piece meet all banks), the weights come straight from memory: an operand's registers take their next step but one as
+// soon as it has been multiplied, so that twice a step's loads are under way, and a step's reads of LDS run ahead of its
+// products.  Four waves and two blocks a CU, which wait for barriers of their own; eight waves that share a tile's
+// activations were slower.  The tiles of an expert at the same channels run side by side on one die, and beside them the
+// die's other channels of the same tiles, so that a tile's activations too come from memory once a die (a channel block
+// after the other read them again for each: 2,000 tokens 561 + 316 us where this order takes 501 + 288).
+// 16 experts of 4,096 x 6,144, tokens of two, us before (loads one step ahead, a branch for every 32 pairs) and now: 300 tokens
+// 304 + 202, 292 + 153; 2,000 544 + 333, 501 + 288; 4,000 894 + 507, 817 + 446 (0.99 PFLOP/s); 16 of 1,024 x 1,024, 300 tokens 23.8 +
+// 20.6, 19.4 + 14.2.  Up to some 32 pairs an expert the weights' bytes bound it (1,610 MB in 292 us, 5.5 TB/s), beyond that bytes and
+// products in turn: half of the tiles are filled in part.
+// ODD: K is an odd number of steps, walked in pairs.
+template <bool GATED, bool ODD>
 __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_tiles_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ weights, const int* __restrict__ order,
     const int* __restrict__ tile_expert, const int* __restrict__ tile_start, const int* __restrict__ tile_count,
@@ -232,9 +240,12 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
   __shared__ __attribute__((aligned(16))) unsigned char xs[2][kTile * kStep * 2];
   const int per_die = gridDim.x / kXcds, work = (blockIdx.x % kXcds) * per_die + blockIdx.x / kXcds;
   if (work >= max_tiles * channel_blocks) return;
-  const int tile = work % max_tiles, channels = work / max_tiles;
+  // channel blocks in groups, of which a die has one where there are enough; in a group a tile's channel blocks, then the next tile's
+  const int group_blocks = max(1, channel_blocks / kXcds), group = work / (max_tiles * group_blocks), in_group = work - group * max_tiles * group_blocks;
+  const int here = min(group_blocks, channel_blocks - group * group_blocks);
+  const int tile = in_group / here, channels = group * group_blocks + in_group % here;
   if (tile >= *num_tiles) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 31, g = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31, g = lane >> 5;
   const int start = tile_start[tile], count = tile_count[tile];
   const int groups = (count + 31) / 32;                  // of 32 pairs that exist
   const int unit = channels * kTileWaves + wave;              // the wave's 32 channels (gated) or 64 rows
@@ -242,16 +253,16 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
   const bool active = GATED ? unit < row_blocks : 2 * unit < row_blocks;      // (a wave past the last still copies activations)
   const int first_block = GATED ? min(unit, row_blocks - 1) : min(2 * unit, row_blocks - 1);
   const int second_block = GATED ? first_block + row_blocks : min(first_block + 1, row_blocks - 1);
-  const bf16_t* const base = weights + (size_t)tile_expert[tile] * (GATED ? 2 : 1) * R * K + lane * 8;
+  const bf16_t* const base = weights + (size_t)tile_expert[tile] * (GATED ? 2 : 1) * R * K;      // (the same in all lanes)
   const bf16_t* const wp[2] = {base + (size_t)first_block * 32 * K, base + (size_t)second_block * 32 * K};
   const bf16_t* xp[kPieces];
-  int xat[kPieces];
+  const int part = tid & 7, swizzle = (tid >> 4) & 7;      // (row >> 1, whose low three bits are the same in all rows of a thread)
+  const int xat = (tid >> 3) * (kStep * 2) + (part ^ swizzle) * 16;
+  static_assert(kThreads / 8 % 16 == 0, "a thread's rows share their swizzle");
 #pragma unroll
   for (int i = 0; i < kPieces; ++i) {
-    const int piece = i * kThreads + tid, row = piece >> 3, part = piece & 7;
-    const int p = order[start + min(row, count - 1)];
+    const int p = order[start + min(i * (kThreads / 8) + (tid >> 3), count - 1)];
     xp[i] = x + (size_t)(GATED ? p / top : p) * K + part * 8;
-    xat[i] = row * (kStep * 2) + ((part ^ (row >> 1)) & 7) * 16;
   }
   float16v acc[2][4];
 #pragma unroll
@@ -262,48 +273,76 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
       for (int q = 0; q < 16; ++q) acc[b][j][q] = 0.f;
   Frag8 w[2][2][4];
   u32x4 xr[kPieces];
+  // Past the end nothing is used but where an odd number of steps is walked in pairs: zeros are (never a repeated step, whose
+  // infinities would meet them).
+  const auto weights_at = [&](int b, int k0) {
+    if (ODD) return k0 < K ? wp[b] + (size_t)k0 * 32 : kZeros;
+    return wp[b] + (size_t)min(k0, K - kStep) * 32;
+  };
   const auto fetch_weights = [&](int k0, Frag8 (&to)[2][4]) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < 2; ++b) {
+      const bf16_t* const from = weights_at(b, k0);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) to[b][s].u = *reinterpret_cast<const u32x4*>(wp[b] + (size_t)k0 * 32 + s * 512);
+      for (int s = 0; s < 4; ++s) to[b][s].u = *reinterpret_cast<const u32x4*>(from + s * 512 + lane * 8);
+    }
   };
   const auto fetch_rows = [&](int k0) {
 #pragma unroll
-    for (int i = 0; i < kPieces; ++i) xr[i] = *reinterpret_cast<const u32x4*>(xp[i] + k0);
+    for (int i = 0; i < kPieces; ++i) {
+      if (ODD) {
+        xr[i] = *reinterpret_cast<const u32x4*>(k0 < K ? xp[i] + k0 : kZeros);
+      } else {
+        if (k0 > 0 && k0 < K) xp[i] += kStep;
+        xr[i] = *reinterpret_cast<const u32x4*>(xp[i]);
+      }
+    }
   };
   const auto park_rows = [&](int copy) {
 #pragma unroll
-    for (int i = 0; i < kPieces; ++i) *reinterpret_cast<u32x4*>(&xs[copy][xat[i]]) = xr[i];
+    for (int i = 0; i < kPieces; ++i) *reinterpret_cast<u32x4*>(&xs[copy][xat + i * (kThreads / 8 * kStep * 2)]) = xr[i];
   };
   fetch_weights(0, w[0]);
+  fetch_weights(kStep, w[1]);
   fetch_rows(0);
   park_rows(0);
-  const auto step = [&](int k0, int copy) {
-    __syncthreads();      // this copy is written, the other one read
-    const int ahead = k0 + kStep < K ? k0 + kStep : k0;      // (past the end: the same step again, not used)
-    fetch_weights(ahead, w[copy ^ 1]);
-    fetch_rows(ahead);
-    if (active) {
+  // GROUPS: of 32 pairs that the products take, known to the compiler: a step without branches, whose reads of LDS run ahead
+  const auto walk = [&](auto groups_taken) {
+    constexpr int GROUPS = groups_taken;
+    const auto step = [&](int k0, int copy) {
+      __syncthreads();      // this copy is written, the other one read
+      fetch_rows(k0 + kStep);
+      __builtin_amdgcn_sched_barrier(0);
+      const int ahead = k0 + 2 * kStep;
+      const bf16_t* const from[2] = {weights_at(0, ahead), weights_at(1, ahead)};
+      Frag8 xf[GROUPS];
+      const auto read = [&](int s, int j) {
+        xf[j].u = *reinterpret_cast<const u32x4*>(&xs[copy][j * (32 * kStep * 2) + col * (kStep * 2) + (((2 * s + g) ^ (col >> 1)) & 7) * 16]);
+      };
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+      for (int j = 0; j < GROUPS; ++j) read(0, j);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (j < groups) {
-            Frag8 xf;
-            const int row = 32 * j + col;
-            xf.u = *reinterpret_cast<const u32x4*>(&xs[copy][row * (kStep * 2) + (((2 * s + g) ^ (row >> 1)) & 7) * 16]);
-            acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[copy][0][s].v, xf.v, acc[0][j], 0, 0, 0);
-            acc[1][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[copy][1][s].v, xf.v, acc[1][j], 0, 0, 0);
-          }
+      for (int s = 0; s < 4; ++s) {
+#pragma unroll
+        for (int j = 0; j < GROUPS; ++j) {
+          acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[copy][0][s].v, xf[j].v, acc[0][j], 0, 0, 0);
+          acc[1][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[copy][1][s].v, xf[j].v, acc[1][j], 0, 0, 0);
+          if (s < 3) read(s + 1, j);
+          __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) w[copy][b][s].u = *reinterpret_cast<const u32x4*>(from[b] + s * 512 + lane * 8);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      park_rows(copy ^ 1);
+    };
+    for (int k0 = 0; k0 < K; k0 += 2 * kStep) {
+      step(k0, 0);
+      step(k0 + kStep, 1);
     }
-    park_rows(copy ^ 1);
   };
-  for (int k0 = 0; k0 < K; k0 += 2 * kStep) {
-    step(k0, 0);
-    if (k0 + kStep < K) step(k0 + kStep, 1);
-  }
+  if (groups > 2) walk(std::integral_constant<int, 4>{});
+  else walk(std::integral_constant<int, 2>{});
   if (!active) return;
   // acc[b][j][4 i + q]: row 8 i + 4 g + q of the wave's block b, pair 32 j + col
 #pragma unroll
@@ -378,7 +417,9 @@ TK_API int tk_moe_tiles(int gated, const void* x, const void* weights, const int
   const long total = (long)max_tiles * channel_blocks;
   if (total > 0x7ffffff0L) return -1;
   const dim3 grid((unsigned)((total + kXcds - 1) / kXcds * kXcds));
-  const auto kernel = gated ? moe_tiles_kernel<true> : moe_tiles_kernel<false>;
+  const bool odd = K / kStep % 2 != 0;
+  const auto kernel = gated ? odd ? moe_tiles_kernel<true, true> : moe_tiles_kernel<true, false>
+                            : odd ? moe_tiles_kernel<false, true> : moe_tiles_kernel<false, false>;
   kernel<<<grid, kTileWaves * 64, 0, stream>>>((const bf16_t*)x, (const bf16_t*)weights, order, tile_expert, tile_start, tile_count,
                                                num_tiles, pair_weight, out, N, top, R, K, max_tiles, channel_blocks, gated == 2);
   return launch_status();
