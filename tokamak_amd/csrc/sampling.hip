@@ -45,12 +45,37 @@ struct SharedRows {
   uint32_t* cand;                // [M][kCandidates] ordered images
   uint8_t* segment;              // [M][kCandidates]
   unsigned long long* above;     // [M][segments] mass of what is kept for certain and not listed
+  struct FirstLevel* level;      // [M] where the first threshold lies
 };
 
 __device__ __forceinline__ bool has_threshold(const float* temperature, const int* top_k, const float* top_p, int r, int V, bool& k_on, bool& p_on) {
   k_on = top_k[r] > 0 && top_k[r] < V;
   p_on = top_p[r] < 1.f;
   return temperature[r] > 0.f && (k_on || p_on);
+}
+
+// Eight loads a thread of a run of quads, asked for together (a segment of 152 k logits is five: one trip to memory, not one
+// after the other), and early: what a kernel has to know before it can use them is fetched meanwhile.
+constexpr int kHeldQuads = 8;
+template <int THREADS>
+__device__ __forceinline__ void ask_quads(const float4* __restrict__ p, int quads, int base, float4 (&v)[kHeldQuads]) {
+  const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~(kWave - 1));
+#pragma unroll
+  for (int u = 0; u < kHeldQuads; ++u)
+    if (base + u * THREADS + wave0 < quads) v[u] = p[min(base + u * THREADS + (int)threadIdx.x, quads - 1)];
+}
+
+// f(4 q, p[q]) for q below `quads`, each by one of the block's THREADS threads in ascending order; v: what ask_quads has for base 0.
+template <int THREADS, typename F>
+__device__ __forceinline__ void use_quads(const float4* __restrict__ p, int quads, float4 (&v)[kHeldQuads], F f) {
+  for (int base = 0; base < quads; base += kHeldQuads * THREADS) {
+    if (base > 0) ask_quads<THREADS>(p, quads, base, v);
+#pragma unroll
+    for (int u = 0; u < kHeldQuads; ++u) {
+      const int q = base + u * THREADS + (int)threadIdx.x;
+      if (q < quads) f(4 * q, v[u]);
+    }
+  }
 }
 
 // temperature, top_k, top_p, part_mass (all or none): for a row with temperature > 0 and no
@@ -60,15 +85,6 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
     const float* __restrict__ logits, float* __restrict__ part_v, int* __restrict__ part_i, int V,
     long ld, const float* __restrict__ temperature, const int* __restrict__ top_k,
     const float* __restrict__ top_p, float* __restrict__ part_mass, SharedRows clear) {
-  // scratch of a row with thresholds that later kernels add into, shared out over its blocks
-  bool k_on, p_on;
-  if (clear.hist32 != nullptr && has_threshold(temperature, top_k, top_p, blockIdx.y, V, k_on, p_on)) {
-    for (int i = blockIdx.x * kArgmaxThreads + threadIdx.x; i < kBins; i += kArgmaxSegments * kArgmaxThreads) {
-      clear.hist32[(size_t)blockIdx.y * kBins + i] = 0u;
-      clear.hist64[(size_t)blockIdx.y * kBins + i] = 0ull;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) clear.count[blockIdx.y] = 0u;
-  }
   __shared__ float best_v[kArgmaxThreads / kWave];
   __shared__ int best_i[kArgmaxThreads / kWave];
   const int seg = blockIdx.x, r = blockIdx.y;
@@ -79,18 +95,27 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
   float bv = -INFINITY;
   int bi = 0x7fffffff;
   const bool vec = ((reinterpret_cast<uintptr_t>(row) & 15) == 0);
-  if (vec) {
-    for (int i = begin + threadIdx.x * 4; i < end; i += kArgmaxThreads * 4) {
-      if (i + 4 <= end) {
-        const float4 v = *reinterpret_cast<const float4*>(row + i);
-        argmax_take(bv, bi, v.x, i);
-        argmax_take(bv, bi, v.y, i + 1);
-        argmax_take(bv, bi, v.z, i + 2);
-        argmax_take(bv, bi, v.w, i + 3);
-      } else {
-        for (int j = i; j < end; ++j) argmax_take(bv, bi, row[j], j);
-      }
+  const int quads = max(0, end - begin) / 4, left = begin + 4 * quads;      // (what is left over: up to three)
+  const float4* const row4 = reinterpret_cast<const float4*>(row + begin);
+  float4 held[kHeldQuads];
+  if (vec) ask_quads<kArgmaxThreads>(row4, quads, 0, held);
+  // scratch of a row with thresholds that later kernels add into, shared out over its blocks
+  bool k_on, p_on;
+  if (clear.hist32 != nullptr && has_threshold(temperature, top_k, top_p, blockIdx.y, V, k_on, p_on)) {
+    for (int i = blockIdx.x * kArgmaxThreads + threadIdx.x; i < kBins; i += kArgmaxSegments * kArgmaxThreads) {
+      clear.hist32[(size_t)blockIdx.y * kBins + i] = 0u;
+      clear.hist64[(size_t)blockIdx.y * kBins + i] = 0ull;
     }
+    if (blockIdx.x == 0 && threadIdx.x == 0) clear.count[blockIdx.y] = 0u;
+  }
+  if (vec) {
+    use_quads<kArgmaxThreads>(row4, quads, held, [&](int at, const float4& v) {
+      argmax_take(bv, bi, v.x, begin + at);
+      argmax_take(bv, bi, v.y, begin + at + 1);
+      argmax_take(bv, bi, v.z, begin + at + 2);
+      argmax_take(bv, bi, v.w, begin + at + 3);
+    });
+    if (left + (int)threadIdx.x < end) argmax_take(bv, bi, row[left + threadIdx.x], left + threadIdx.x);
   } else {
     for (int i = begin + threadIdx.x; i < end; i += kArgmaxThreads) argmax_take(bv, bi, row[i], i);
   }
@@ -108,7 +133,7 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
   }
   if (part_mass == nullptr || !(temperature[r] > 0.f)) return;
   if (has_threshold(temperature, top_k, top_p, r, V, k_on, p_on)) return;  // the sampler sums what it keeps
-  // the segment again (it is in the cache): its mass relative to its own maximum
+  // the segment again: its mass relative to its own maximum
   const float scale = 1.4426950408889634f / temperature[r];  // e^(y / t) = 2^(y log2 e / t)
   float mass = 0.f;
   const auto add = [&](float x) {
@@ -116,17 +141,15 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
     if (y == y) mass += __builtin_amdgcn_exp2f(y);  // a NaN (also -inf - -inf of a segment without a number) adds nothing
   };
   if (vec) {
-    for (int i = begin + threadIdx.x * 4; i < end; i += kArgmaxThreads * 4) {
-      if (i + 4 <= end) {
-        const float4 v = *reinterpret_cast<const float4*>(row + i);
-        add(v.x);
-        add(v.y);
-        add(v.z);
-        add(v.w);
-      } else {
-        for (int j = i; j < end; ++j) add(row[j]);
-      }
-    }
+    if (quads > kHeldQuads * kArgmaxThreads) ask_quads<kArgmaxThreads>(row4, quads, 0, held);      // (else still there)
+    use_quads<kArgmaxThreads>(row4, quads, held, [&](int, const float4& v) {
+      add(v.x);
+      add(v.y);
+      add(v.z);
+      add(v.w);
+    });
+    if ((int)threadIdx.x == quads % kArgmaxThreads)      // (as if the last, partial four were one more of the walk)
+      for (int j = left; j < end; ++j) add(row[j]);
   } else {
     for (int i = begin + threadIdx.x; i < end; i += kArgmaxThreads) add(row[i]);
   }
@@ -237,6 +260,7 @@ __device__ __forceinline__ float uniform01(uint64_t seed, uint64_t counter) {
 }
 
 constexpr int kSampleThreads = 1024;
+static_assert(4 * kFew <= kSampleThreads, "four threads a value");
 
 // Prefix sums of one value per thread over the block, threads in index order; `scan`
 // holds an entry a wave.  Returns the sum over the threads before this one;
@@ -361,30 +385,44 @@ __device__ __forceinline__ void for_row(const float* __restrict__ row, int V, F 
 //                   order: sums over the list are of integers), and the mass of the bins above it in each segment; with
 //                   both thresholds the bins above it are listed too, top-p's may lie there.
 // The sampler then starts from the histogram and the list and reads the row again only where the drawn number falls.
-// (A block that reads its row alone moves some 45 GB/s.  40 rows of 152 k logits, most with thresholds: 12 + 13 us shared and
-// 21 for the rest, of which a segment's walk, the ranks and the start are each a few memory round trips.)
+// (A block that reads its row alone moves some 45 GB/s.  40 rows of 152 k logits, most with thresholds: 10.3 + 12.8 us shared and
+// 18.8 for the rest, of which a segment's walk, the ranks and the start are each a few memory round trips; 58.9 -> 53.7 us for
+// the whole since a thread asks for its piece of a segment at once, the sampler takes the first level's bin from the collecting
+// kernel and ranks are counted by four threads a value.)
 
-// f(index, value) for every element of a segment, each by one thread of the block
-template <typename F>
-__device__ __forceinline__ void for_segment(const float* __restrict__ row, int V, int seg, F f) {
-  const int per = ((V + kArgmaxSegments - 1) / kArgmaxSegments + 3) & ~3;
-  const int begin = min(V, seg * per), end = min(V, begin + per);
-  if ((reinterpret_cast<uintptr_t>(row) & 15) == 0) {
-    const int quads = (end - begin) / 4;
-#pragma unroll 4
-    for (int q = threadIdx.x; q < quads; q += kShareThreads) {
-      const float4 v = *reinterpret_cast<const float4*>(row + begin + 4 * q);
-      f(v.x);
-      f(v.y);
-      f(v.z);
-      f(v.w);
-    }
-    const int done = begin + 4 * quads;
-    if ((int)threadIdx.x < end - done) f(row[done + threadIdx.x]);
-  } else {
-    for (int i = begin + threadIdx.x; i < end; i += kShareThreads) f(row[i]);
+// A segment of a row as the threads of a block see it: asked for at once, used later (f(value) for every element, each by
+// one thread).
+struct Segment {
+  const float* row;
+  int begin, end, quads;
+  bool wide;
+  float4 held[kHeldQuads];
+
+  __device__ __forceinline__ Segment(const float* __restrict__ row_, int V, int seg) : row(row_) {
+    const int per = ((V + kArgmaxSegments - 1) / kArgmaxSegments + 3) & ~3;
+    begin = min(V, seg * per);
+    end = min(V, begin + per);
+    quads = (end - begin) / 4;
+    wide = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
+    if (wide) ask_quads<kShareThreads>(reinterpret_cast<const float4*>(row + begin), quads, 0, held);
   }
-}
+
+  template <typename F>
+  __device__ __forceinline__ void each(F f) {
+    if (wide) {
+      use_quads<kShareThreads>(reinterpret_cast<const float4*>(row + begin), quads, held, [&](int, const float4& v) {
+        f(v.x);
+        f(v.y);
+        f(v.z);
+        f(v.w);
+      });
+      const int done = begin + 4 * quads;
+      if ((int)threadIdx.x < end - done) f(row[done + threadIdx.x]);
+    } else {
+      for (int i = begin + threadIdx.x; i < end; i += kShareThreads) f(row[i]);
+    }
+  }
+};
 
 struct FirstLevel {
   int bin;                          // the first histogram's bin that holds the threshold
@@ -450,6 +488,10 @@ __global__ __launch_bounds__(kShareThreads) void sample_hist_kernel(
   __shared__ uint32_t h32[kBins];
   __shared__ unsigned long long h64[kBins];
   const int seg = blockIdx.x, r = blockIdx.y, lane = threadIdx.x & (kWave - 1);
+  bool k_on, p_on;
+  const bool thresholds = has_threshold(temperature, top_k, top_p, r, V, k_on, p_on);
+  if (!thresholds && seg > 0) return;
+  Segment segment(logits + (size_t)r * ld, thresholds ? V : 0, seg);
   // the row's maximum (every wave for itself); the first block leaves it, and the argmax
   float bv = lane < kArgmaxSegments ? seg_max[r * kArgmaxSegments + lane] : -INFINITY;
   int bi = lane < kArgmaxSegments ? seg_index[r * kArgmaxSegments + lane] : 0x7fffffff;
@@ -458,15 +500,14 @@ __global__ __launch_bounds__(kShareThreads) void sample_hist_kernel(
     out[r] = (bi == 0x7fffffff) ? 0 : bi;
     row_max[r] = bv;
   }
-  bool k_on, p_on;
-  if (!has_threshold(temperature, top_k, top_p, r, V, k_on, p_on)) return;
+  if (!thresholds) return;
   const float inv_t = 1.f / temperature[r], mx = bv * inv_t;
   if (!(mx > -INFINITY)) return;
   for (int i = threadIdx.x; i < kBins; i += kShareThreads) h32[i] = 0;
   if (!k_on)
     for (int i = threadIdx.x; i < kBins; i += kShareThreads) h64[i] = 0;
   __syncthreads();
-  for_segment(logits + (size_t)r * ld, V, seg, [&](float logit) {
+  segment.each([&](float logit) {
     const float x = scaled(logit, inv_t);
     const uint32_t bin = ordered(x) >> 20;
     atomicAdd(&h32[bin], 1u);
@@ -495,13 +536,15 @@ __global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
   if (threadIdx.x == 0) count = 0;
   const FirstLevel level = first_level<kShareThreads>(sh.hist32 + (size_t)r * kBins, sh.hist64 + (size_t)r * kBins, k_on, top_k[r], top_p[r],
                                                       scan, &found);
+  if (seg == 0 && threadIdx.x == 0) sh.level[r] = level;
   const int low = level.bin;
   const bool both = k_on && p_on;
   if ((both ? level.total : level.inside) > (uint32_t)kCandidates) return;      // (the sampler walks the row)
   const float mx = row_max[r] * inv_t, scale = draw_scale(V);
   unsigned long long above = 0;
   // this block's values, then side by side into the row's list
-  for_segment(logits + (size_t)r * ld, V, seg, [&](float logit) {
+  // (asked for here: held across the search above they cost registers, and with them blocks; 12.8 -> 15.1 us at 40 rows)
+  Segment(logits + (size_t)r * ld, V, seg).each([&](float logit) {
     const float x = scaled(logit, inv_t);
     const uint32_t o = ordered(x);
     const int bin = (int)(o >> 20);
@@ -609,8 +652,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
       });
       __syncthreads();
     }
-    const FirstLevel level = first_level<kSampleThreads>(ready ? shared.hist32 + (size_t)r * kBins : hist32,
-                                                         ready ? shared.hist64 + (size_t)r * kBins : hist64, k_on, k, p_keep, scan64, &first);
+    const FirstLevel level = ready ? shared.level[r] : first_level<kSampleThreads>(hist32, hist64, k_on, k, p_keep, scan64, &first);
     const int low_bin = level.bin;
     if (k_on) {
       k_prefix = (uint32_t)low_bin;
@@ -681,13 +723,18 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     __syncthreads();
     const int n = (int)few_count;
     if (n > kFew || n == 0) return false;      // (every thread alike)
-    if (tid < n) {
-      const uint32_t mine = few[tid];
+    if (tid < 4 * n) {      // (four neighbouring threads a value, a quarter of the others each)
+      const uint32_t mine = few[tid / 4];
       unsigned long long above = 0, whole = 0;
-      for (int i = 0; i < n; ++i) {
+      for (int i = tid & 3; i < n; i += 4) {
         const unsigned long long m = few_mass[i];
         whole += m;
         above += few[i] > mine ? m : 0ull;
+      }
+#pragma unroll
+      for (int d = 1; d < 4; d <<= 1) {
+        whole += __shfl_xor(whole, d, kWave);
+        above += __shfl_xor(above, d, kWave);
       }
       if (above < target(whole)) atomicMin(&few_cut, mine);
     }
@@ -857,14 +904,35 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   const int s_begin = sel * chunk, s_end = min(V, s_begin + chunk);
   const int run_len = ((s_end - s_begin + kSampleThreads - 1) / kSampleThreads + 3) / 4 * 4;
   const int r_begin = min(s_end, s_begin + tid * run_len), r_end = min(s_end, r_begin + run_len);
+  // eight tokens of the run at a time, asked for together; the first eight (all, up to 262 k logits) stay for the second look
+  constexpr int kHeld = 8;
+  float head[kHeld];
+  const auto hold = [&](int from, float (&v)[kHeld]) {
+    if ((reinterpret_cast<uintptr_t>(row) & 15) == 0 && from + kHeld <= r_end) {      // (runs begin at multiples of four tokens)
+      const float4 a = *reinterpret_cast<const float4*>(row + from), b = *reinterpret_cast<const float4*>(row + from + 4);
+      v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+    } else {
+#pragma unroll
+      for (int u = 0; u < kHeld; ++u) v[u] = from + u < r_end ? row[from + u] : -INFINITY;
+    }
+  };
   float mine_run = 0.f;
   int last_kept = -1;
-#pragma unroll 4
-  for (int i = r_begin; i < r_end; ++i) {
-    const float m = kept_mass(row[i]);
-    // (a kept token's mass may round to zero; it is kept all the same)
-    if (ordered(scaled(row[i], inv_t)) >= cut) last_kept = i;
-    mine_run += m;
+  const auto look = [&](int from, const float (&v)[kHeld]) {
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u)
+      if (from + u < r_end) {
+        mine_run += kept_mass(v[u]);
+        // (a kept token's mass may round to zero; it is kept all the same)
+        if (ordered(scaled(v[u], inv_t)) >= cut) last_kept = from + u;
+      }
+  };
+  hold(r_begin, head);
+  look(r_begin, head);
+  for (int i = r_begin + kHeld; i < r_end; i += kHeld) {
+    float more[kHeld];
+    hold(i, more);
+    look(i, more);
   }
   if (tid == 0) {
     found_bin = -1;   // the token that the target falls on
@@ -876,13 +944,19 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   if (sel_before + excl <= target && target < sel_before + incl) {
     float run = sel_before + excl;
     int pick = -1;
-#pragma unroll 4
-    for (int i = r_begin; i < r_end; ++i) {  // (to the run's end, so that its loads can be asked for together)
-      const float logit = row[i];
-      if (ordered(scaled(logit, inv_t)) >= cut) {
-        run += kept_mass(logit);
-        if (pick < 0 && run > target) pick = i;
-      }
+    const auto choose = [&](int from, const float (&v)[kHeld]) {
+#pragma unroll
+      for (int u = 0; u < kHeld; ++u)
+        if (from + u < r_end && ordered(scaled(v[u], inv_t)) >= cut) {
+          run += kept_mass(v[u]);
+          if (pick < 0 && run > target) pick = from + u;
+        }
+    };
+    choose(r_begin, head);
+    for (int i = r_begin + kHeld; i < r_end && pick < 0; i += kHeld) {
+      float more[kHeld];
+      hold(i, more);
+      choose(i, more);
     }
     if (pick < 0) pick = last_kept;  // rounding at the end of the run
     if (pick >= 0) atomicMax(&found_bin, pick);
@@ -908,7 +982,7 @@ constexpr size_t kSharedWords = 3 * kBins + 2;     // of a row: counts, masses, 
 TK_API int tk_sample_scratch_bytes(int M, int V) {
   const long rows = M < 1 ? 0 : M;
   const long parts = rows * kArgmaxSegments * 12 + rows * 4 + 16;
-  return (int)(parts + (shares_rows(M, V) ? rows * ((long)kSharedWords * 4 + (long)kCandidates * 5 + kArgmaxSegments * 8) : 0));
+  return (int)(parts + (shares_rows(M, V) ? rows * ((long)kSharedWords * 4 + (long)kCandidates * 5 + kArgmaxSegments * 8 + (long)sizeof(FirstLevel)) : 0));
 }
 
 // Every row's next token: greedy rows (temperature 0) their argmax, the others a draw; a row whose search falls through
@@ -928,7 +1002,9 @@ TK_API int tk_sample(const float* logits, long ld, int M, int V, const float* te
     sh.count = sh.hist32 + (size_t)M * kBins;
     sh.above = reinterpret_cast<unsigned long long*>(at + (size_t)M * kSharedWords * 4);
     // (the argmax pass clears a row's words so far; M times an odd number of 8 bytes: still on their border)
-    at += (size_t)M * (kSharedWords * 4 + kArgmaxSegments * 8);
+    sh.level = reinterpret_cast<FirstLevel*>(at + (size_t)M * (kSharedWords * 4 + kArgmaxSegments * 8));
+    at += (size_t)M * (kSharedWords * 4 + kArgmaxSegments * 8 + sizeof(FirstLevel));
+    static_assert(sizeof(FirstLevel) % 8 == 0 && kSharedWords % 2 == 0, "what lies behind stays on borders of 8 bytes");
   }
   float* seg_max = reinterpret_cast<float*>(at);
   float* seg_mass = seg_max + (size_t)M * kArgmaxSegments;
