@@ -39,3 +39,24 @@ def test_the_tiled_kernels_bits(m, n, k):
     assert torch.equal(wide[1:-1, 4:-4].view(torch.int32), whole[:m].view(torch.int32)) or torch.equal(
         wide[1:-1, 4:-4].nan_to_num(7.0), whole[:m].nan_to_num(7.0))
     assert bool(wide[0].isnan().all() and wide[-1].isnan().all() and wide[:, :4].isnan().all() and wide[:, -4:].isnan().all())
+
+
+# bundles of K dealt over the borders of groups: one piece, bundles fewer than, as many as and more than the waves, an odd last piece, blocks
+# of one group and of two, a last group of one and of three rows
+@pytest.mark.gpu
+@pytest.mark.parametrize("m, n, k", [(1, 12000, 4), (4, 12001, 256), (3, 12007, 1028), (2, 17996, 2564), (16, 18000, 260), (5, 18001, 1284),
+                                     (8, 20011, 2308), (1, 20480, 1540), (9, 18003, 772), (1, 65532, 516)])
+def test_bundles_over_the_borders_of_groups(m, n, k):
+    assert ops.fewrows_dealt(m, n)
+    test_the_tiled_kernels_bits(m, n, k)
+
+
+@pytest.mark.parametrize("m, n, k, dealt, rounds", [(1, 19456, 2560, 35.9, 39.7), (4, 19456, 2560, 37.0, 40.2), (1, 14000, 2560, 28.5, 31.5),
+                                                    (1, 18624, 2176, 33.7, 37.2), (1, 38696, 2592, 70.2, 78.6), (1, 25216, 10624, 186, 209),
+                                                    (1, 5120, 5120, 22.2, 21.6), (8, 13952, 3840, 47.0, 43.3)])
+def test_bundles_are_dealt_where_that_was_faster(m, n, k, dealt, rounds):
+    """Measured, us.  In rounds of a group 10 pieces of K keep six waves busy for ten twelfths of the time."""
+    assert ops.fewrows_dealt(m, n) == (dealt < rounds)
+    if dealt < rounds:
+        group, waves, _, blocks = ops.fewrows_form(m, n, k)
+        assert waves == 4 and group >= m and blocks <= -(-n // group)

@@ -234,16 +234,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 // the same whatever the batch holds.
 //
 // Bound by the weights' bytes, and for small matrices by the trips to memory.  An operand's sixteen rows are J = 16 / TP
-// pieces of K of TP weight rows, its columns the same pieces of TP rows of activations; the blocks on the
+// pieces of K (a bundle) of TP weight rows, its columns the same pieces of TP rows of activations; the blocks on the
 // result's diagonal are kept.  Groups of 4 or 8 rows give small matrices four and two times the blocks.  A block's waves
-// take J pieces each a round; a round's sums meet in LDS, where one wave adds them in order.  Blocks walk over
+// take a bundle each a round; a round's sums meet in LDS, where one wave adds them in order.  Blocks walk over
 // groups of rows, loads running ahead over their borders.  Weights come as 256 contiguous bytes of four rows a load, two
 // or four stages of 64 k ahead, and change hands through the wave's own LDS (rows 68 floats apart: 64 banks); the activations'
 // four numbers a lane become the four k of a step by swaps between the lanes of a column.
-// (In the form before, a lane owned a weight row and multiplied in the vector unit, 64 rows and a piece a wave, the pieces' sums
-// through memory to a kernel of their own: us there and here, 4 rows, 2,048 x 2,048 17.8 and 6.7, 4,096 x 2,048 16.9 and 8.6,
-// 2,048 x 6,144 20.2 and 13.1, 12,288 x 2,048 23.8 and 19.3, 151,936 x 2,048 233 and 193.)
-template <int TP, int WAVES, int DEPTH>
+// DEALT: the bundles of a block's groups are dealt to its waves one after the other, over the groups' borders; else a group
+// begins with a round, and where its bundles are not a multiple of the waves the last ones have none (10 pieces in rounds of
+// four leave a sixth of the waves' time).  19,456 x 2,560 at one row 39.7 us in rounds, dealt 35.9;
+// 14,000 x 2,560 31.5 and 28.5; 38,696 x 2,592 78.6 and 70.2; for smaller matrices, whose blocks have a group or two, rounds are as
+// fast or a few percent faster (2,048 x 6,144 12.3, dealt 13.2).
+// (Before, a lane owned a weight row and multiplied in the vector unit, 64 rows and a piece a wave, the pieces' sums
+// through memory to a kernel of their own: us there and here, 4 rows, 2,048 x 2,048 12.1 and 6.7, 4,096 x 2,048 13.2 and 8.7,
+// 2,048 x 6,144 19.3 and 13.1, 12,288 x 2,048 23.1 and 19.8, 151,936 x 2,048 240 and 202; at one row it was up to 8 % ahead for some
+// matrices of 18,000 rows and more, 18,624 x 2,176 31.1 and 33.7, 26,048 x 4,224 74.5 and 80.8.)
+template <int TP, int WAVES, int DEPTH, bool DEALT>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2))) void gemm_fewrows_kernel(
     const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N, int K, long lda, long ldw,
     long ldc) {
@@ -252,42 +258,60 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
   static_assert(kPiece == 256 && (DEPTH == 2 || DEPTH == 4), "a piece is four stages of 64 k");
   __shared__ __attribute__((aligned(16))) float tile[WAVES][16 * PITCH];
   __shared__ __attribute__((aligned(16))) f32x4 sums[2][WAVES * J][TP * QUADS];   // of a round: [piece][row of activations, four weight rows]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = DEALT ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
   const int a = lane & 15, g = lane >> 4;
-  const int pieces = (K + kPiece - 1) / kPiece, rounds = (pieces + WAVES * J - 1) / (WAVES * J);
-  const int groups = (N + TP - 1) / TP;
-  const int visits = (groups - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x * rounds;   // (group, round) pairs of this block
+  const int pieces = (K + kPiece - 1) / kPiece, bundles = (pieces + J - 1) / J;
+  const int rounds = (pieces + WAVES * J - 1) / (WAVES * J);      // of a group, not DEALT
+  const int own_groups = ((N + TP - 1) / TP - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int turns = own_groups * bundles;      // (group, bundle) pairs of this block
+  const int visits = DEALT ? (turns + WAVES - 1) / WAVES : own_groups * rounds;
 
   // this lane's place: of the loads of weights row 4 i + lane / 16 of the operand, of those of activations column a
   const int wk = a * 4, own_m = min(a % TP, M - 1);
   const float* const arow = A + (size_t)own_m * lda;
   f32x4 wreg[DEPTH][4], areg[DEPTH][4];
-  // What a visit reads: the rows of its group, the first k of its pieces.  A piece past the last is never read (first k >= K);
-  // rows past N are read at the last row and never stored, what lies past K is read at the row's end and becomes zero.
-  const auto first_k = [&](int round, int share) { return ((round * WAVES + wave) * J + share) * kPiece; };
-  const auto fetch = [&](int group, int round, int stage, int buf) {
-    if (first_k(round, 0) >= K) return;      // (uniform)
+  // `at`: a group's round, of which this wave has its own bundle (DEALT: the bundle).  A bundle past the last is never read (first
+  // k >= K); rows past N are read at the last row and never stored, what lies past K is read at the row's end and becomes zero.
+  const auto first_k = [&](int at, int share) { return ((DEALT ? at : at * WAVES + wave) * J + share) * kPiece; };
+  const auto fetch = [&](int group, int at, int stage, int buf) {
+    if (!DEALT && first_k(at, 0) >= K) return;      // (uniform)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = 4 * i + g;
-      const int n = min(group * TP + row % TP, N - 1), k = min(first_k(round, row / TP) + 64 * stage + wk, K - 4);
+      const int n = min(group * TP + row % TP, N - 1), k = min(first_k(at, row / TP) + 64 * stage + wk, K - 4);
       wreg[buf][i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(W + (size_t)n * ldw + k));
     }
-    const int k0 = first_k(round, a / TP) + 64 * stage + 4 * g;
+    const int k0 = first_k(at, a / TP) + 64 * stage + 4 * g;
 #pragma unroll
     for (int j = 0; j < 4; ++j) areg[buf][j] = *reinterpret_cast<const f32x4*>(arow + min(k0 + 16 * j, K - 4));
   };
 
-  int group = blockIdx.x, round = 0;
+  int group = blockIdx.x, at = 0;
+  if constexpr (DEALT) {
+    group += wave / bundles * (int)gridDim.x;
+    at = wave % bundles;
+  }
+  if (!DEALT || wave < turns) {
 #pragma unroll
-  for (int s = 0; s < DEPTH; ++s) fetch(group, 0, s, s);
+    for (int s = 0; s < DEPTH; ++s) fetch(group, at, s, s);
+  }
   f32x4 total = {0.f, 0.f, 0.f, 0.f};
   for (int v = 0; v < visits; ++v) {
-    const bool turns = round + 1 == rounds, last = v + 1 == visits;
-    const int next_round = turns ? 0 : round + 1, next_group = turns ? group + (int)gridDim.x : group;
+    bool turn, last;            // the group is done; this wave reads no more
+    int next_at, next_group;
+    if constexpr (DEALT) {
+      next_at = at + WAVES % bundles;
+      turn = next_at >= bundles;
+      last = (v + 1) * WAVES + wave >= turns;
+      next_group = group + (WAVES / bundles + (turn ? 1 : 0)) * (int)gridDim.x;
+      next_at -= turn ? bundles : 0;
+    } else {
+      turn = at + 1 == rounds, last = v + 1 == visits;
+      next_at = turn ? 0 : at + 1, next_group = turn ? group + (int)gridDim.x : group;
+    }
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    if (first_k(round, 0) < K) {
-      const bool whole = first_k(round, J - 1) + kPiece <= K;
+    if (DEALT ? v * WAVES + wave < turns : first_k(at, 0) < K) {
+      const bool whole = first_k(at, J - 1) + kPiece <= K;
 #pragma unroll
       for (int s = 0; s < STAGES; ++s) {
         const int buf = s % DEPTH;
@@ -296,7 +320,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           f32x4 w = wreg[buf][i];
-          if (!whole && first_k(round, (4 * i + g) / TP) + 64 * s + wk >= K) w = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (!whole && first_k(at, (4 * i + g) / TP) + 64 * s + wk >= K) w = f32x4{0.f, 0.f, 0.f, 0.f};
           *reinterpret_cast<f32x4*>(mine + (4 * i + g) * PITCH + wk) = w;
         }
         // areg[j][e] holds k = 16 j + 4 g + e; step[j][e] is to hold k = 16 j + 4 e + g
@@ -304,7 +328,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           f32x4 x = areg[buf][j];
-          if (!whole && first_k(round, a / TP) + 64 * s + 16 * j + 4 * g >= K) x = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (!whole && first_k(at, a / TP) + 64 * s + 16 * j + 4 * g >= K) x = f32x4{0.f, 0.f, 0.f, 0.f};
           const auto e02 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[0]), __float_as_uint(x[2]), false, false);
           const auto e13 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[1]), __float_as_uint(x[3]), false, false);
           const auto e01 = __builtin_amdgcn_permlane16_swap(e02[0], e13[0], false, false);
@@ -314,8 +338,8 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
           step[j][2] = e23[0];
           step[j][3] = e23[1];
         }
-        if (s + DEPTH < STAGES) fetch(group, round, s + DEPTH, buf);
-        else if (!last) fetch(next_group, next_round, s + DEPTH - STAGES, buf);
+        if (s + DEPTH < STAGES) fetch(group, at, s + DEPTH, buf);
+        else if (!last) fetch(next_group, next_at, s + DEPTH - STAGES, buf);
         wave_lds_sync();
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -323,50 +347,67 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
           for (int e = 0; e < 4; ++e)
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(mine[a * PITCH + 16 * j + 4 * e + g], __uint_as_float(step[j][e]), acc, 0, 0, 0);
       }
-    } else if (!last) {
+    } else if (!DEALT && !last) {
 #pragma unroll
-      for (int s = 0; s < DEPTH; ++s) fetch(next_group, next_round, s, s);
+      for (int s = 0; s < DEPTH; ++s) fetch(next_group, next_at, s, s);
     }
     // acc[e]: weight row 4 g + e of the operand against column a of the activations
     if (4 * g / TP == a / TP) sums[v & 1][wave * J + a / TP][a % TP * QUADS + g % QUADS] = acc;
     __syncthreads();      // (one a round: this copy is written again behind the next round's barrier)
-    if (threadIdx.x < TP * QUADS) {
-      const int left = min(WAVES * J, pieces - round * WAVES * J);
-      for (int p = 0; p < left; ++p) total += sums[v & 1][p][threadIdx.x];
-      if (turns) {
-        const int m = threadIdx.x / QUADS, n = group * TP + threadIdx.x % QUADS * 4;
+    if (threadIdx.x < TP * QUADS) {      // (of wave 0, whose group and bundle are the round's first)
+      const auto finish = [&](int at_group) {
+        const int m = threadIdx.x / QUADS, n = at_group * TP + threadIdx.x % QUADS * 4;
         if (m < M && n < N) store_four<float>(C + (size_t)m * ldc + n, total[0], total[1], total[2], total[3], N - n, rows_take_wide_stores(C, ldc));
         total = f32x4{0.f, 0.f, 0.f, 0.f};
+      };
+      if constexpr (DEALT) {
+        const int filled = min(WAVES, turns - v * WAVES);
+        for (int w = 0, at_group = group, at_bundle = at; w < filled;) {
+          const int run = min(filled - w, bundles - at_bundle), left = min(run * J, pieces - at_bundle * J);      // of one group
+          for (int p = 0; p < left; ++p) total += sums[v & 1][w * J + p][threadIdx.x];
+          w += run;
+          if (at_bundle + run < bundles) break;      // (goes on in the next round)
+          finish(at_group);
+          at_bundle = 0;
+          at_group += (int)gridDim.x;
+        }
+      } else {
+        const int left = min(WAVES * J, pieces - at * WAVES * J);
+        for (int p = 0; p < left; ++p) total += sums[v & 1][p][threadIdx.x];
+        if (turn) finish(group);
       }
     }
     group = next_group;
-    round = next_round;
+    at = next_at;
   }
 }
 
 // float32 in and out, M <= 16, K and the row strides multiples of 4, 16-byte aligned rows.  rows: of a group, 4, 8 or 16, at
-// least M; waves a block, 4, 6 or 8; depth: stages of 64 k asked for ahead, 2, or 4 for 16 rows and four waves; blocks: at most so many.
+// least M; waves a block, 4, 6 or 8; depth: stages of 64 k asked for ahead, 2, or 4 for 16 rows and four waves; blocks: at most so many;
+// dealt: as described above, for 8 or 16 rows and four waves.
 TK_API int tk_gemm_fewrows(const float* A, const float* W, float* C, int M, int N, int K, long lda, long ldw, long ldc, int rows,
-                           int waves, int depth, int blocks, hipStream_t stream) {
+                           int waves, int depth, int blocks, int dealt, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 16 || M > rows || K < 4 || K % 4 != 0 || lda % 4 != 0 || ldw % 4 != 0 || blocks < 1) return -1;
   if (reinterpret_cast<uintptr_t>(A) % 16 != 0 || reinterpret_cast<uintptr_t>(W) % 16 != 0) return -1;
   const int grid = min(blocks, (N + rows - 1) / rows);
-#define TK_FEW(TP_, WAVES_, DEPTH_) \
-  if (rows == TP_ && waves == WAVES_ && depth == DEPTH_) { \
-    gemm_fewrows_kernel<TP_, WAVES_, DEPTH_><<<grid, WAVES_ * 64, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc); \
+#define TK_FEW(TP_, WAVES_, DEPTH_, DEALT_) \
+  if (rows == TP_ && waves == WAVES_ && depth == DEPTH_ && (dealt != 0) == DEALT_) { \
+    gemm_fewrows_kernel<TP_, WAVES_, DEPTH_, DEALT_><<<grid, WAVES_ * 64, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc); \
     return launch_status(); \
   }
-  TK_FEW(4, 4, 2)
-  TK_FEW(4, 6, 2)
-  TK_FEW(4, 8, 2)
-  TK_FEW(8, 4, 2)
-  TK_FEW(8, 6, 2)
-  TK_FEW(8, 8, 2)
-  TK_FEW(16, 4, 2)
-  TK_FEW(16, 6, 2)
-  TK_FEW(16, 8, 2)
-  TK_FEW(16, 4, 4)
+  TK_FEW(4, 4, 2, false)
+  TK_FEW(4, 6, 2, false)
+  TK_FEW(4, 8, 2, false)
+  TK_FEW(8, 4, 2, false)
+  TK_FEW(8, 6, 2, false)
+  TK_FEW(8, 8, 2, false)
+  TK_FEW(16, 4, 2, false)
+  TK_FEW(16, 6, 2, false)
+  TK_FEW(16, 8, 2, false)
+  TK_FEW(16, 4, 4, false)
+  TK_FEW(8, 4, 2, true)
+  TK_FEW(16, 4, 2, true)
 #undef TK_FEW
   return -1;
 }

@@ -256,7 +256,7 @@ _SIGS = {
         "tk_gemm_tiled": [c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long,
                           c_long, c_long, c_void_p],
         "tk_gemm_fewrows": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_int, c_int,
-                            c_int, c_void_p],
+                            c_int, c_int, c_void_p],
     },
     "gemm_mfma": {
         "tk_gemm_stream": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long,
@@ -1701,6 +1701,14 @@ def fewrows_pays(m: int, n: int) -> bool:
     return True
 
 
+def fewrows_dealt(m: int, n: int) -> bool:
+    """Whether the weight-streaming product deals a block's bundles of K to its waves over the borders of the groups of weight
+    rows: where blocks have several groups, of which each would waste the idle waves of its last round otherwise.  Smaller
+    matrices are as fast or slower (5,120 x 5,120 21.6 us, dealt 22.2; 13,952 x 3,840 at 8 rows 43.3 and 47.0), and a head's walks
+    run with more loads ahead."""
+    return (12000 if m <= 4 else 18000) <= n < 65536
+
+
 def fewrows_form(m: int, n: int, k: int, small_groups: bool | None = None) -> tuple[int, int, int, int]:
     """(weight rows of a group, waves a block, stages of 64 k ahead, blocks) of the weight-streaming product; us at 4 rows.
     Groups: the fewest rows for the CU that has most of them (2,048 x 2,048 in groups of 8 6.7, of 16 7.9; 5,120 x 5,120 in
@@ -1708,10 +1716,17 @@ def fewrows_form(m: int, n: int, k: int, small_groups: bool | None = None) -> tu
     Blocks: as many as are on the chip at once, the groups dealt to them (25,600 x 5,120 as 768 blocks 92.9, as 534 with three
     groups each 116).  Eight waves where no CU has a second block (2,048 x 6,144 13.1, four waves 13.4; at 16 rows 21.9 and
     25.0), else the four or six that leave fewer idle in the last round (20,000 x 1,028 six 22.8, four 24.9); and for walks of a
-    head's length more loads ahead (151,936 x 2,048 199 -> 193, at 16 rows 268 -> 256)."""
+    head's length more loads ahead (151,936 x 2,048 199 -> 193, at 16 rows 268 -> 256).  Where bundles are dealt
+    (``fewrows_dealt``): groups of 16, a block each, of up to five groups a CU and more than one round of K three blocks a
+    CU (19,456 x 2,560 35.9 and 38.5, but 20,000 x 1,028 25.0 and 23.5); below 18,000 weight rows of 8 (14,000 x 2,560 28.5 and 29.7)."""
     least = 4 if m <= 4 else 8 if m <= 8 else 16
     if small_groups is not None:
         group = least if small_groups else 16
+    elif fewrows_dealt(m, n):
+        if n < 18000:
+            return 8, 4, 2, -(-n // 8)
+        groups = -(-n // 16)
+        return 16, 4, 2, 768 if groups <= 5 * 256 and k > 1536 else groups
     else:
         group, most = 16, -(-n // (16 * 256)) * 16
         for g in (8, 4):
@@ -1747,7 +1762,8 @@ def gemm_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, fewrows_spli
         for at in range(0, m, FEWROWS_GROUP):
             rows = min(FEWROWS_GROUP, m - at)
             _check(_fn("gemm_tiled", "tk_gemm_fewrows")(_p(a[at:]), _p(w), _p(out[at:]), rows, n, k, a.stride(0), w.stride(0),
-                                                        out.stride(0), *fewrows_form(rows, n, k, fewrows_split), _stream()),
+                                                        out.stride(0), *fewrows_form(rows, n, k, fewrows_split),
+                                                        int(fewrows_split is None and fewrows_dealt(rows, n)), _stream()),
                    "gemm_fewrows")
         return
     _check(_fn("gemm_tiled", "tk_gemm_tiled")(_code(a.dtype), _code(out.dtype), _p(a), _p(w), _p(out),
