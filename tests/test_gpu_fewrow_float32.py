@@ -60,3 +60,10 @@ def test_bundles_are_dealt_where_that_was_faster(m, n, k, dealt, rounds):
     if dealt < rounds:
         group, waves, _, blocks = ops.fewrows_form(m, n, k)
         assert waves == 4 and group >= m and blocks <= -(-n // group)
+
+
+@pytest.mark.parametrize("m, n, streamed, tiled", [(64, 12288, 90.0, 55.2), (48, 12288, 68.2, 55.0), (64, 6144, 84.6, 66.7), (56, 8200, 81.6, 43.6),
+                                                   (64, 4096, 0.68, 1.0), (64, 2048, 0.67, 1.0), (32, 12288, 0.84, 1.0), (17, 1024, 0.27, 1.0)])
+def test_rows_stream_the_weights_where_that_was_faster(m, n, streamed, tiled):
+    """Measured times (us, or shares of the tiled kernel's)."""
+    assert ops.fewrows_pays(m, n) == (streamed < tiled)

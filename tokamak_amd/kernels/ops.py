@@ -1689,16 +1689,15 @@ FEWROWS_GROUP = 16             # this many rows a pass over them
 
 def fewrows_pays(m: int, n: int) -> bool:
     """Whether ``m`` rows stream the weights (one pass per FEWROWS_GROUP rows) rather than take
-    the tiled kernel in tiles of 64 x 64, which reads the weights once but needs a block for
-    every CU to be worth it: measured on the shapes of an 8B-shaped layer, the tiled kernel wins
-    from 24 rows where it has a thousand tiles (the logits head at 64 rows: 4.7 -> 1.6 ms) and
-    from 48 where it has one a CU (gate/up: 546 -> 303 us); a matrix of 4,096 rows never."""
-    tiles = -(-n // 64)
-    if m >= 48 and tiles >= 256:
-        return False
-    if m >= 24 and tiles >= 1024:
-        return False
-    return True
+    the tiled kernel in tiles of 64 x 64, which reads the weights once but needs blocks for
+    the CUs to be worth it.  Measured on 48 sizes of 500 to 151,936 weight rows: from 48 rows on streaming wins up to some 4,096 weight
+    rows (4,096 x 4,096 at 64 rows 0.68 of the tiled kernel's time, 6,144 x 2,560 1.27; 12,288 x 2,048 90 us, tiled 55), with two passes
+    nearly everywhere (12,288 x 2,048 at 32 rows 0.84).  The tiled kernel keeps what has a thousand tiles from 24 rows on; there
+    two passes would be faster now (151,936 x 1,024 at 24 rows 239 us, tiled 365), as tiles would for 33 to 47 rows of 6,400
+    to 65,536 weight rows (12,288 x 2,048 at 40 rows 66 us, tiled 55)."""
+    if m >= 48:
+        return n <= 4096
+    return m < 24 or -(-n // 64) < 1024
 
 
 def fewrows_dealt(m: int, n: int) -> bool:
