@@ -120,3 +120,22 @@ def test_every_size_has_a_form_of_the_kernel():
                     blocks = -(-n // (rows * groups))
                     assert not slabs or blocks <= slabs or n > slabs * 16
     assert not ops.direct_pays("plain", 17, 64, 64) and not ops.direct_pays("add", 0, 64, 64)
+
+
+# (what it competes with, rows, columns, K, us of the direct product, us of the other form)
+MEASURED = [("activated", 16, 5120, 17408, 63.7, 33.7), ("activated", 8, 5120, 17408, 49.6, 32.9), ("activated", 3, 5120, 17408, 36.4, 32.2),
+            ("activated", 16, 5120, 5120, 21.8, 14.7), ("activated", 16, 28672, 4096, 55.3, 38.2), ("activated", 16, 4432, 7048, 34.4, 18.3),
+            ("activated", 16, 2048, 6144, 11.0, 15.5), ("activated", 16, 4096, 4096, 11.1, 12.2), ("activated", 8, 752, 9080, 9.2, 15.3),
+            ("activated", 1, 5120, 5120, 10.7, 13.6),
+            ("plain", 16, 24576, 4096, 48.1, 34.7), ("plain", 16, 28672, 4096, 55.1, 38.0), ("plain", 8, 24576, 4096, 37.2, 34.0),
+            ("plain", 16, 13544, 760, 9.9, 8.0), ("plain", 9, 18792, 11184, 107, 94), ("plain", 4, 34816, 5120, 59.7, 71.7),
+            ("plain", 16, 4096, 12288, 25.4, 64.0), ("plain", 6, 16384, 4096, 24.0, 28.6),
+            ("add", 16, 368, 11144, 18.7, 10.2), ("add", 16, 824, 14256, 22.0, 14.6), ("add", 16, 3224, 3896, 12.3, 10.4),
+            ("add", 3, 5120, 17408, 41.5, 34.5), ("add", 16, 6144, 5120, 22.0, 17.8),
+            ("add", 16, 1024, 3072, 7.1, 7.7), ("add", 8, 4096, 12288, 21.1, 21.9), ("add", 6, 4096, 14336, 22.5, 24.4), ("add", 16, 4096, 4096, 11.4, 11.6),
+            ("add", 9, 2560, 4096, 9.1, 8.3)]
+
+
+@pytest.mark.parametrize("kind, m, n, k, direct, other", MEASURED)
+def test_the_direct_product_is_taken_where_it_was_faster(kind, m, n, k, direct, other):
+    assert ops.direct_pays(kind, m, n, k) == (direct < other)

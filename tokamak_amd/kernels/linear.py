@@ -168,7 +168,7 @@ def activated_linear(x: torch.Tensor, weight: torch.Tensor, activation: str = "s
     out = torch.empty((m, n), dtype=x.dtype, device=x.device)
     if m == 0:
         return out
-    if _few_rows_fit(m, x, weight, ops.DIRECT_MAX_ROWS) and ops.direct_pays("plain", m, n, k):
+    if _few_rows_fit(m, x, weight, ops.DIRECT_MAX_ROWS) and ops.direct_pays("activated", m, n, k):
         ops.gemm_direct(x, weight, out, activation=activation)
     elif (x.dtype == torch.bfloat16 and m <= gemm_bf16.SKINNY_MAX_ROWS and n >= gemm_bf16.STREAM_MIN_ROWS_OUT
             and gemm_bf16.skinny_fits(x, weight) and gemm_bf16.stream_splits(n, k, m) < ACTIVATED_SPLIT_FROM):

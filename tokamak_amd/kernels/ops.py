@@ -1955,18 +1955,28 @@ DIRECT_ANY_SIZE_ROWS = 2        # rows up to which the activations are so few th
 def direct_pays(kind: str, m: int, n: int, k: int) -> bool:
     """Whether the direct product is the faster form for M <= 16 rows.  ``kind``: what it competes with.
 
+    Every block reads the activations for its own 4 to 16 columns, so beside the weights' bytes three things bound it from three rows
+    on: ``reads``, what all blocks read of them; ``even``, the share of the CUs' rounds that has blocks (a product whose K can be split fills
+    them); and ``own``, what one block reads, which a CU alone pulls slowly.  Measured both ways on 156 matrices of 350 to 32,000
+    by 500 to 20,000, half of them with rows of whole cache lines (other rows cost this form a few percent more), at 1 to 16 rows; us,
+    this form against the other:
+
+    "plain", against a product that may leave no partial sums and has a block for every 64 columns: while those are fewer than three
+    quarters of the CUs (1,024 x 4,096 at one row 4.2 against 19.0, 12,288 x 4,096 at 16 rows 25.3 and 25.8); beyond that up to four rows (34,816 x 5,120
+    at 4 rows 59.7 and 71.7) and to eight while the reads are few (16,384 x 4,096 at 6 rows 24.0 and 28.6; but 24,576 x 4,096 at 8
+    37.2 and 34.0, at 16 48.1 and 34.7).
+    "activated", against the split product and the activation behind it, or unsplit from where columns are enough: few reads, or more in
+    even rounds (2,048 x 6,144 at 16 rows 11.0 and 15.5, 4,096 x 4,096 11.1 and 12.2; but 5,120 x 17,408 at 8 rows 49.6 and 32.9, at 16
+    63.7 and 33.7, 5,120 x 5,120 at 16 21.8 and 14.7).
+    "add" (into the stream), against the whole-K product, or for a K beyond it the split product and the norm: up to eight rows
+    while a block's own reads are short and the rounds even, or few blocks or rows (4,096 x 14,336 at 6 rows 22.5 and 24.4,
+    4,096 x 12,288 at 8 21.1 and 21.9; but 5,120 x 17,408 at 3 rows 41.5 and 34.5); nine to sixteen rows read the activations twice for
+    every weight: the smallest matrices, and middling ones in even rounds (4,096 x 4,096 at 16 rows 11.4 and 11.6, 1,024 x 3,072 7.1 and 7.7; but
+    10,624 x 1,624 14.9 and 12.6, 6,144 x 5,120 22.0 and 17.8, 504 x 8,112 13.6 and 8.4).
     "gated" (n columns of each half), against the streaming product that cannot split K under the gate: up to four rows always
-    (12,288 x 4,096 at one row 30.9 us against 34.8, 6,144 x 2,048 10.7 against 16.3), up to eight where the other has blocks
-    of four waves or few blocks (32.4 against 33.7, 12.8 against 15.2; but 9,728 x 2,560 22.6 against 21.9), up to
-    sixteen while the matrix is small (3,072 x 1,024 6.7 against 6.9).
-    "add" (into the stream), against the whole-K product, or for a long K the split product and the norm behind it: up to
-    eight rows while the activations stay in L2's reach and the blocks fill their rounds (4,096 x 12,288 at 8 rows 20.3 us against
-    21.3, 2,048 x 6,144 8.3 against 11.5; but 5,120 x 17,408 48.8 against 33.7, 5,120 x 5,120 17.0 against 15.8); nine to
-    sixteen rows read the activations twice for every weight (1,024 x 3,072 at 16 rows 7.0 against 7.6, 4,096 x 4,096
-    10.8 against 11.5, 2,560 x 4,096 in 160 blocks 10.6 against 9.8).
-    "plain", against a product that may leave no partial sums and so has a block for every 64 columns: always (1,024 x 4,096 at
-    one row 4.2 us against 19.0), except where the columns alone are blocks enough (a logits head; up to two rows there too:
-    151,936 x 4,096 180 against 196).
+    (12,288 x 4,096 at one row 30.9 us against 34.8, 6,144 x 2,048 10.7 against 16.3; a K beyond 16,384 in uneven rounds is up to a third slower), up
+    to eight where the other has blocks of four waves or few blocks (32.4 against 33.7, 12.8 against 15.2; but 9,728 x 2,560 22.6
+    against 21.9), up to sixteen while the matrix is small (3,072 x 1,024 6.7 against 6.9).
     "norm" (a row scale to apply, partial sums allowed), against the split streaming product: up to two rows (6,144 x 4,096 10.3
     against 11.6), more while the activations are few beside L1 (4,096 x 2,048 at 8 rows 6.6 against 7.4, at 16
     7.4 against 7.8; 6,144 x 2,560 at 8 rows 10.3 against 8.9).
@@ -1977,20 +1987,29 @@ def direct_pays(kind: str, m: int, n: int, k: int) -> bool:
     size = 2 * n * k
     if kind == "gated":
         return m <= 4 or (m <= 8 and (2 * size <= DIRECT_MIDDLE_BYTES or 2 * k % 8192 == 0)) or 2 * size <= STREAM_SMALL_MATRIX_BYTES
-    if kind == "plain":
-        return m <= DIRECT_ANY_SIZE_ROWS or n < 64 * 512
     if kind == "norm":
         return m <= DIRECT_ANY_SIZE_ROWS or (size <= STREAM_SMALL_MATRIX_BYTES and (m <= 8 or k <= 2048))
     if kind == "parts":
         return m <= 4 and n <= 2048 and k <= 1024
     if m <= DIRECT_ANY_SIZE_ROWS:
         return True
-    rows, groups, _ = direct_plan(m, n, k, most_slabs=ROW_SCALE_MAX_SLABS)
+    rows, groups, _ = direct_plan(m, n, k, most_slabs=ROW_SCALE_MAX_SLABS if kind == "add" else 0)
     blocks = -(-n // (rows * groups))
-    even = blocks >= 0.75 * STREAM_CUS * -(-blocks // STREAM_CUS)
+    even = blocks / (STREAM_CUS * -(-blocks // STREAM_CUS))
+    own = 2 * m * k
+    reads = blocks * own
+    if kind == "plain":
+        return 4 * n <= 3 * 64 * STREAM_CUS or m <= 4 or (m <= 8 and reads <= 64e6)
+    if kind == "activated":
+        if m <= 8:
+            return n < 1024 or (own <= 256 << 10 and reads <= (64e6 if even >= 0.85 else 30e6))
+        if blocks <= STREAM_CUS:
+            return own <= 256 << 10 and reads <= (64e6 if even >= 0.85 else 30e6)
+        return own <= 256 << 10 and reads <= (40e6 if even >= 0.85 and 4 * n <= 3 * 64 * STREAM_CUS else 20e6)
     if m <= 8:
-        return k <= 12288 and (m <= 4 or even or blocks <= STREAM_CUS)
-    return size <= DIRECT_MIDDLE_BYTES and (even or n <= 1024)
+        return own <= 192 << 10 and (even >= 0.9 or (k <= 12288 and (m <= 4 or even >= 0.75 or blocks <= STREAM_CUS)))
+    small = size <= STREAM_SMALL_MATRIX_BYTES // 2 and reads <= 16e6 and own <= 128 << 10
+    return size <= DIRECT_MIDDLE_BYTES and own <= 192 << 10 and (small or even >= 0.9)
 
 
 def gemm_direct(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, sumsq: torch.Tensor | None = None, eps: float = 0.0,
