@@ -73,6 +73,10 @@ class Part:
     # decode step a block may then run it as a branch beside another part (parts/block.py: ``beside``).
     own_branch = False
 
+    def branch_pays(self, tokens: int) -> bool:
+        """For a part with ``own_branch``: whether a step of so many tokens is worth a fork and a join."""
+        return True
+
     def __init__(self, *, dtype: torch.dtype, device: torch.device | str) -> None:
         self.dtype = dtype
         self.device = torch.device(device)

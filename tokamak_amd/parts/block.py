@@ -18,13 +18,13 @@ def beside(batch, part, other, run):
 
     The kernels of such a step are 4 to 15 us long and leave most of the GPU idle; two chains of them side by side take little
     longer than the longer one, plus 8 to 14 us a fork and join (measured: 6 + 5 kernels of 21 us in a row 237 us, forked 137; of 1.5 us
-    18.6 and 28.4), hence only parts that say ``own_branch``: routed experts beside a mixer (0.6B-shaped, 16 requests: a pass of
+    18.6 and 28.4), hence only parts that say ``own_branch``, where ``branch_pays``: routed experts beside a mixer (0.6B-shaped, 16 requests: a pass of
     prompts and 24 tokens 34.9 -> 30.8 ms), a time mix beside pooled attention (8B-shaped, 3 requests: 37.2 -> 36.1); a mixer of
     four kernels beside another lost 1.5 %.  The part's own allocations come from its stream's memory,
     so neither branch takes up what the other is still using; its results are read behind the join by the norm
     that opens the next layer, ahead of the next fork, and its inputs are held by the caller until the join."""
     side = batch.side
-    if side is None or not part.own_branch:
+    if side is None or not part.own_branch or not part.branch_pays(batch.num_tokens):
         first = other()
         return first, run()
     main = torch.cuda.current_stream(side.device)

@@ -11,6 +11,9 @@ from tokamak_amd.parts.base import FeedForward, Fetch, RowWeighted
 from tokamak_amd.weights.spec import TensorSpec
 
 
+BRANCH_FROM_BYTES = 95e6       # of the experts that a step meets: from there on a branch of their own pays
+
+
 class RoutedExperts(FeedForward):
     """``num_experts`` feed-forwards down(silu(gate x) * up x) without biases, of which every token
     uses ``top``.
@@ -122,10 +125,25 @@ class RoutedExperts(FeedForward):
     def matrix_share(self, tokens: int) -> tuple[float, float]:
         e, top = self.num_experts, self.top
         router, expert = e * self.hidden_size, 3 * self.intermediate_size * self.hidden_size
-        met = e * (1.0 - (1.0 - top / e) ** max(tokens, 0))     # experts that a step of so many tokens meets, on average
+        met = self._experts_met(tokens)
         shared = 0 if self.shared_size is None else 3 * self.shared_size * self.hidden_size
         total = router + e * expert + shared
         return (router + top * expert + shared) / total, (router + met * expert + shared) / total
+
+    def branch_pays(self, tokens: int) -> bool:
+        """With a shared expert the part is five kernels and more, about as long as what a fork and a join cost at the smallest
+        sizes (0.6B-shaped, one request 47.6 us a layer in a row, forked 45.5; 16 requests 61.5 and 52.9).  Without one it is
+        three, which pay from some 100 MB of experts' weights on: 0.6B-shaped experts of 1,536 channels, one request 50.2 and
+        55.2 us, 4 (62 MB) 57.4 and 59.1, 8 (99 MB) 61.3 and 61.0, 40 80.0 and 72.9; of 3,072 channels, 2 (71 MB) 62.9 and
+        67.3, 4 (124 MB) 70.3 and 65.3; 4,096 wide with 1,024 channels, 2 (94 MB) 130.5 and 132.8, 4 (166 MB) 141.3 and 138.1."""
+        if self.shared_size is not None:
+            return True
+        element = torch.empty(0, dtype=self.dtype).element_size()
+        return self._experts_met(tokens) * 3 * self.intermediate_size * self.hidden_size * element >= BRANCH_FROM_BYTES
+
+    def _experts_met(self, tokens: int) -> float:
+        """Experts that a step of so many tokens meets, on average."""
+        return self.num_experts * (1.0 - (1.0 - self.top / self.num_experts) ** max(tokens, 0))
 
     def forward(self, h, batch):
         """Float32 partial sums [top, N, width]: layer k holds every token's k-th chosen expert's output;
