@@ -29,3 +29,26 @@ def test_experts_get_a_branch_where_it_was_faster(width, channels, shared, count
 
 def test_other_parts_have_none():
     assert not Part.own_branch and not GQAAttention.own_branch
+
+
+def test_a_pinned_stream_is_the_threads_own(monkeypatch):
+    """What one thread pins while it steps or records a model is not where another thread launches."""
+    import threading
+    from types import SimpleNamespace
+
+    from tokamak_amd.kernels import ops
+
+    current = threading.local()
+    current.stream = 7
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(cuda_stream=getattr(current, "stream", 9)))
+    seen = []
+    with ops.pinned_stream():
+        current.stream = 8
+        other = threading.Thread(target=lambda: seen.append(ops._stream().value))
+        other.start()
+        other.join()
+        seen.append(ops._stream().value)
+        with ops.pinned_stream():
+            seen.append(ops._stream().value)
+        seen.append(ops._stream().value)
+    assert seen == [9, 7, 8, 7] and ops._stream().value == 8

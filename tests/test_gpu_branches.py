@@ -36,3 +36,24 @@ def test_branches_give_the_bits_of_kernels_in_a_row(preset, layers, requests):
         outs.append(got)
     for i, (a, b) in enumerate(zip(*outs)):
         assert torch.isfinite(a).all() and torch.equal(a, b), f"step {i}"
+
+
+def test_a_recording_asks_for_the_stream_a_few_times_only(monkeypatch):
+    """A step of a new shape runs once and is recorded; its launches take the stream that was looked up once, not one
+    each."""
+    from tokamak_amd.config import find_preset
+    from tokamak_amd.engine.runner import ModelRunner, StepEntry
+    from tokamak_amd.weights.random_init import expected_tensors_of
+    from tokamak_amd.weights.sources import RandomSource
+
+    arch, cfg = find_preset("dopirax-0.6b")
+    plan = arch.plan(arch.shorten(cfg, 8))
+    source = RandomSource({n: s for n, s in expected_tensors_of(plan).items() if not s.ignored}, seed=3, matrix_std=0.02,
+                          dtype=torch.bfloat16, device="cuda:0")
+    runner = ModelRunner(plan, source, dtype="bfloat16", page_size=16, kv_pool_tokens=256, max_requests=4)
+    runner.step([StepEntry(r, [5, 6, 7], []) for r in range(4)])
+    asked, current = [], torch.cuda.current_stream
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: asked.append(device) or current(device))
+    runner.step([StepEntry(r, [8], [0]) for r in range(4)])
+    assert len(runner._graphs) == 1
+    assert len(asked) <= 4 * 8        # (a fork, a switch and a pin for the layers that run in Python, and what torch's own recording asks: 16)

@@ -20,6 +20,7 @@ import gc
 import torch
 
 from tokamak_amd.engine.batch import PackedBatch, batch_from_device
+from tokamak_amd.kernels import ops
 
 
 def pow2_at_least(n: int, floor: int) -> int:
@@ -48,7 +49,8 @@ class DecodeGraph:
         self._load(packed, feed)
         # this step itself, eagerly: code objects are loaded and the allocator is warm
         # before the recording starts; the recording executes nothing
-        self.first_logits = model.forward(self.batch, storage)
+        with ops.pinned_stream():
+            self.first_logits = model.forward(self.batch, storage)
         torch.cuda.synchronize(device)
         self.batch.memo.clear()
         # what the recording holds: the most that is live at once while it is recorded (its
@@ -65,7 +67,7 @@ class DecodeGraph:
         collecting = gc.isenabled()
         gc.disable()
         try:
-            with torch.cuda.graph(self.graph):
+            with torch.cuda.graph(self.graph), ops.pinned_stream():
                 self.batch.side = side
                 self.logits = model.forward(self.batch, storage)
         finally:

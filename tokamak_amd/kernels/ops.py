@@ -9,6 +9,7 @@ compiled library the call raises.
 from __future__ import annotations
 
 import ctypes
+import threading
 from ctypes import c_float, c_int, c_long, c_size_t, c_void_p
 
 import torch
@@ -122,27 +123,30 @@ def can_record() -> bool:
     return _recorder is None and _profile is None
 
 
-_pinned_stream: c_void_p | None = None
+class _ThreadStreams(threading.local):
+    pinned: c_void_p | None = None      # (a thread's own: another thread's launches go to its own current stream)
+
+
+_streams = _ThreadStreams()
 
 
 def _stream() -> c_void_p:
-    return _pinned_stream if _pinned_stream is not None else c_void_p(torch.cuda.current_stream().cuda_stream)
+    pinned = _streams.pinned
+    return pinned if pinned is not None else c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
 class pinned_stream:
     """Within the block every kernel of this module is launched on the stream that is
     current at entry, without asking torch for it launch by launch (that lookup costs
-    more than the launch).  The caller must not switch streams inside the block."""
+    more than the launch).  Whoever switches streams inside the block pins the other one there."""
 
     def __enter__(self):
-        global _pinned_stream
-        self._before = _pinned_stream
-        _pinned_stream = c_void_p(torch.cuda.current_stream().cuda_stream)
+        self._before = _streams.pinned
+        _streams.pinned = c_void_p(torch.cuda.current_stream().cuda_stream)
         return self
 
     def __exit__(self, *exc):
-        global _pinned_stream
-        _pinned_stream = self._before
+        _streams.pinned = self._before
         return False
 
 
