@@ -52,3 +52,18 @@ def test_a_pinned_stream_is_the_threads_own(monkeypatch):
             seen.append(ops._stream().value)
         seen.append(ops._stream().value)
     assert seen == [9, 7, 8, 7] and ops._stream().value == 8
+
+
+def test_a_branch_runs_no_library_product(monkeypatch):
+    """Those share one workspace a device, which the step's other branch may be using."""
+    from types import SimpleNamespace
+
+    from tokamak_amd.kernels import ops
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(cuda_stream=7))
+    a = torch.zeros(80, 64, dtype=torch.bfloat16)
+    with ops.pinned_stream(), ops.branch_stream():
+        with pytest.raises(ops.KernelError, match="share one workspace"):
+            ops.gemm_library(a, a, torch.empty(80, 80, dtype=torch.bfloat16))
+    with pytest.raises(ops.KernelError, match="GPU tensors"):        # (elsewhere as before)
+        ops.gemm_library(a, a, torch.empty(80, 80, dtype=torch.bfloat16))

@@ -8,8 +8,9 @@ layer of a kind that meets a given kind of input runs as written while its launc
 listed (``kernels.ops.recording``), and every later layer of that kind launches from the
 list, with the addresses of its own weights, cache arrays, incoming sub-layer output and
 following norm in place of the recorded layer's.  Everything else the recorded layer
-allocated is kept until the step ends and used again: layers run one after the other on
-one stream, so a buffer a layer has finished with is free for the next.
+allocated is kept until the step ends and used again: layers run one after the other, so a
+buffer a layer has finished with is free for the next.  (A layer of two branches forks behind the layer before and
+joins before it ends, and what a branch leaves is read by the norm that opens the next layer, ahead of its fork.)
 
 A block takes part only if it says ``replayable``: its parts launch all their work through
 ``kernels.ops`` and decide nothing from values that differ between layers of a kind.

@@ -125,6 +125,7 @@ def can_record() -> bool:
 
 class _ThreadStreams(threading.local):
     pinned: c_void_p | None = None      # (a thread's own: another thread's launches go to its own current stream)
+    branch = False
 
 
 _streams = _ThreadStreams()
@@ -148,6 +149,20 @@ class pinned_stream:
     def __exit__(self, *exc):
         _streams.pinned = self._before
         return False
+
+
+class branch_stream(pinned_stream):
+    """``pinned_stream`` for the stream of a branch, which runs beside the step's own: what shares memory between streams
+    refuses to run on it."""
+
+    def __enter__(self):
+        self._outer = _streams.branch
+        _streams.branch = True
+        return super().__enter__()
+
+    def __exit__(self, *exc):
+        _streams.branch = self._outer
+        return super().__exit__(*exc)
 
 
 def order_streams(first: torch.cuda.Stream, then: torch.cuda.Stream) -> None:
@@ -2171,8 +2186,10 @@ def gemm_library(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
     The plan of each shape is kept; the algorithm is the library's first choice, or with
     ``set_library_tuning(True)`` the fastest of its candidates, timed once per shape class
     (csrc/blas_lt.hip; that synchronises, so the call must not be recorded into a graph).  All calls on a
-    device share one workspace: launch them on one stream at a time (the engine has one).
+    device share one workspace: launch them on one stream at a time (the engine's steps are on one; the second one
+    of a recorded step, ``branch_stream``, is refused).
     Returns False if the library has no algorithm for the shape (nothing was computed)."""
+    _need(not _streams.branch, "library products share one workspace: a part that may run one has no branch of its own")
     for t in (a, w, out):
         _need(t.is_cuda and t.dim() == 2 and t.stride(1) == 1, "gemm operands are 2-D GPU tensors with unit inner stride")
         _need(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0, "the library product is bfloat16 with 16-byte aligned operands")

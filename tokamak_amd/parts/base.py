@@ -69,8 +69,9 @@ class Part:
     fuses_residual = False
 
     # Whether the part's ``forward`` is a chain of several kernels that touches nothing but its arguments, its own
-    # tensors and its own cache slot (in particular, leaves nothing in ``batch.memo`` by a kernel): in a recorded
-    # decode step a block may then run it as a branch beside another part (parts/block.py: ``beside``).
+    # tensors and its own cache slot (in particular, leaves nothing in ``batch.memo`` by a kernel, and runs no library
+    # product at the up to 64 tokens of a recorded step: those share a workspace): in such a
+    # step a block may then run it as a branch beside another part (parts/block.py: ``beside``).
     own_branch = False
 
     def branch_pays(self, tokens: int) -> bool:

@@ -29,7 +29,7 @@ def beside(batch, part, other, run):
         return first, run()
     main = torch.cuda.current_stream(side.device)
     ops.order_streams(main, side)
-    with torch.cuda.stream(side), ops.pinned_stream():
+    with torch.cuda.stream(side), ops.branch_stream():
         second = run()
     first = other()
     ops.order_streams(side, main)
