@@ -68,6 +68,8 @@ class DecodeGraph:
         gc.disable()
         try:
             with torch.cuda.graph(self.graph), ops.pinned_stream():
+                if side is not None and side == torch.cuda.current_stream(device):
+                    side = torch.cuda.Stream(device)      # (torch deals streams from a pool, in turn)
                 self.batch.side = side
                 self.logits = model.forward(self.batch, storage)
         finally:
