@@ -139,3 +139,19 @@ MEASURED = [("activated", 16, 5120, 17408, 63.7, 33.7), ("activated", 8, 5120, 1
 @pytest.mark.parametrize("kind, m, n, k, direct, other", MEASURED)
 def test_the_direct_product_is_taken_where_it_was_faster(kind, m, n, k, direct, other):
     assert ops.direct_pays(kind, m, n, k) == (direct < other)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m, n, k, plan", [(1, 20, 72, (4, 1, 4)), (3, 96, 200, (4, 4, 8)), (4, 1000, 1160, (4, 2, 8)), (8, 40, 72, (8, 1, 8)), (5, 36, 136, (4, 1, 8)),
+                                           (16, 100, 1096, (8, 2, 4)), (9, 20, 8, (8, 1, 8)), (2, 512, 264, None)])
+def test_an_infinite_weight_stays_what_it_is(m, n, k, plan):
+    """K is not whole steps: what the last step has no numbers for is zeros of both operands, so that a row whose last
+    weights hold an infinity is infinite, not NaN."""
+    x, w = rand(m, k, seed=1).abs().to(torch.bfloat16) + 0.125, rand(n, k, seed=2, scale=k ** -0.5).to(torch.bfloat16)
+    row = n // 2
+    w[row, k - 3] = float("inf")
+    out = torch.empty(m, n, device=DEV)
+    ops.gemm_direct(x.to(DEV), w.to(DEV), out, plan=plan)
+    want = x.double() @ w.double().T
+    assert torch.equal(out.cpu()[:, row], want[:, row].float()) and torch.isinf(want[:, row]).all()
+    assert torch.isfinite(out).sum() == m * (n - 1)

@@ -86,7 +86,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_direct_kernel(
   static_assert(RG * KEPT <= 64 && MT <= WAVES, "a wave finishes a tile of the block's result");
   __shared__ __attribute__((aligned(16))) float4v red[WAVES][MT][TILES][RG][KEPT];
   __shared__ float stat[WAVES][ROWS];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // (the wave as a scalar: its steps are then kept by branches.  The matrix units take no notice of the lanes' mask, by which
+  // a condition that could differ from lane to lane may be carried out: they would multiply what no load has filled)
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int a = lane & 15, kb = lane >> 4, own = a & (TP - 1), share = a / TP;
   const int n0 = blockIdx.x * (RG * TP);
   const int koff = (share * 4 + kb) * 8;
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_direct_kernel(
   const u32x4 zero = {0u, 0u, 0u, 0u};
 
   u32x4 wreg[U][TILES][RG], xreg[U][MT];
-  // a piece past K is the row's last piece instead and meets zeros
+  // a piece past K is the row's last piece instead and becomes zeros (of both: an infinite weight is not to meet one)
   const auto fetch = [&](int s) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -156,14 +158,25 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_direct_kernel(
   }
 
   for (int s = s_begin; s < s_end; s += U) {
+    if (K % STEP != 0 && s + U >= steps) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if ((s + u) * STEP + koff >= K) {
+#pragma unroll
+          for (int i = 0; i < MT; ++i) xreg[u][i] = zero;
+#pragma unroll
+          for (int t = 0; t < TILES; ++t)
+#pragma unroll
+            for (int g = 0; g < RG; ++g) wreg[u][t][g] = zero;
+        }
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (s + u < s_end) {
-        const bool inside = (s + u) * STEP + koff < K;
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
           Frag8 xf;
-          xf.u = inside ? xreg[u][i] : zero;
+          xf.u = xreg[u][i];
 #pragma unroll
           for (int t = 0; t < TILES; ++t)
 #pragma unroll
