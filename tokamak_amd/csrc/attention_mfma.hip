@@ -143,7 +143,7 @@ __device__ __forceinline__ void finish_head_vector(const HeadInputs& h, const De
 
 // WAVES: waves of a block (they share a split's keys and merge through LDS); D: tiles of
 // 16 keys a wave keeps in flight.  FUSED: the block first makes its queries (and, if the
-// call stores, the token's own key and value, which the block of the last split writes to
+// call stores, the token's own key and value, which the block whose round holds the position writes to
 // the page and every wave that meets the token's position takes from LDS) from the
 // projection's output: one kernel less a layer than with the separate q/k norm kernel.
 template <int HD, int WAVES, int D, bool FUSED, bool CAP>
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attention_decode_kernel(
   extern __shared__ __attribute__((aligned(16))) float s_dyn[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, kb = lane >> 4;
   // splits are the slowest index of the grid: blocks start in the grid's order, so a token's
-  // last split (the shortest, or one that holds no key) starts behind every first one
+  // last split (none has more keys, and it may hold none) starts behind every first one
   const int split = blockIdx.z, item = blockIdx.y;
   const int G = nh / nkv;
   const int kvh = blockIdx.x;
@@ -1446,12 +1446,12 @@ static int launch(const void* q, const void* k_cache, const void* v_cache, const
   // Eight waves a block and two tiles a wave in flight (138 registers: a block or, where it fits, two a CU).  A CU alone pulls
   // some 60 GB/s whatever is in flight, so few requests are split down to a round of 128 keys a block; sixteen waves of
   // one tile, whose round is 256 keys, took 10.1 us for one request of 540 keys, these 7.8 (with the merge), 14.5 and 12.3
-  // for eight of 222 to 1,500, 19.9 and 18.0 for 64 of 25 to 700, 90 and 91 for 64 of 2,058; three or four tiles a
+  // for eight of 222 to 1,500, 19.9 and 18.0 for 64 of 25 to 700, 90 and 84 for 64 of 2,058; three or four tiles a
   // wave are 1 to 5 % behind, four waves 5 to 20 %.  A merge by the block that finishes last instead of a kernel of
   // its own needs a fence over the dies' caches: 2 us more at three splits, 45 us more with 8 requests.
   const size_t lds = (size_t)(kDecodeWaves * G * HD + 2 * kDecodeWaves * 16) * 4 + (FUSED ? (size_t)(G + 2) * HD * 2 : 0);
   if (lds > 160 * 1024) return -2;
-  if (lds > 48 * 1024) {  // beyond the default limit of dynamic LDS (groups of 7 heads and more)
+  if (lds > 48 * 1024) {  // beyond the default limit of dynamic LDS (at a head size of 128, groups of 12 heads and more, FUSED 11)
     static bool raised[2] = {false, false};  // per template instance
     if (!raised[capped]) {
       if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=

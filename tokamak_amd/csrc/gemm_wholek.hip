@@ -1,6 +1,6 @@
 // bf16 products of few rows (M <= 16: decode steps of up to sixteen requests) in which one
-// block holds the whole of K for its sixteen output columns.  (Up to eight rows, and for small matrices up to sixteen,
-// gemm_direct.hip does the same work faster and is taken instead: ops.direct_pays.)
+// block holds the whole of K for its sixteen output columns.  (Where
+// gemm_direct.hip does the same work faster it is taken instead: ops.direct_pays.)
 //
 // C[M,N] = A[M,K] W[N,K]^T.  A block of WAVES waves owns 16 weight rows (with GATED also the
 // 16 matching rows of the second half of W); its waves split K between them in chunks of

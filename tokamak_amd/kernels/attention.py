@@ -164,10 +164,11 @@ def mfma_fits(dtype, head_dim, page_size, group, window) -> bool:
 
 
 # What the choice of the decode splits is priced with (seconds, bytes a second; fitted to 154
-# measured cases of 9 to 64 requests over 300 to 16,384 keys in 1 to 8 splits and checked on
-# 1 to 8 requests up to 32,768 keys: the cheapest split by this price is on average 1 % and at
-# worst 18 % slower than the best measured one; the rule it replaced, "as few splits as put
-# 4,096 waves on the GPU", 5 % and 49 % on such cases).
+# measured cases of 9 to 64 requests over 300 to 16,384 keys with blocks of sixteen waves).  With the
+# present blocks of eight, on 150 random steps (1 to 64 requests of 32 to 32,768 keys, 1 to 16 kv heads):
+# on average 2 % slower than the best of every split measured, at worst 39 % (12 requests of up to 6,711 keys, 8 kv heads of
+# 64: two splits 27.8 us, nine 20.0); pricing whole rounds of keys gains 0.4 %, constants fitted to these
+# steps 1 % on average, and up to 8 % is lost on some.
 DECODE_CUS = 256                 # blocks that run at once at full rate
 DECODE_RATE = 5.8e12             # bytes a second of a round of DECODE_CUS blocks
 DECODE_BLOCK_RATE = 60e9         # ... and of one block with the GPU to itself
@@ -181,18 +182,18 @@ DECODE_MOST_SPLITS = 64          # candidates looked at (beside the finest split
 def decode_split(num_decode: int, num_kv_heads: int, max_len: int, head_dim: int = 128) -> tuple[int, int]:
     """(keys per split, number of splits) for the decode tokens of a step.  A block of
     DECODE_WAVES waves walks one split of one request and kv head, every wave a share of
-    it (a split is a whole number of 16 keys for every wave); the splits of a token are
+    it (the price counts a split as a whole number of 16 keys for every wave); the splits of a token are
     merged by a second kernel.
 
     The blocks run in rounds of one a CU, so what a split costs follows from how its blocks
     fill the rounds: full rounds stream at the GPU's rate; the last, partial round at that
     rate or, if its blocks are few, at the rate of a block alone (17 requests of 2,048 keys in
-    two splits are 272 blocks, 256 and then 16 that take as long again: 45 us against 34 in
-    three splits; 33 requests unsplit are 264 blocks: 71 us against 60 in three splits).  The
+    two splits are 272 blocks, 256 and then 16 that take as long again: 37 us against 29 unsplit
+    or in three splits; 33 requests unsplit are 264 blocks: 64 us against 56 in three splits).  The
     cheapest of the candidates by that price is taken; equal prices go to fewer splits.  The
-    kernel cuts every token's own keys evenly in that many splits (csrc/attention_mfma.hip:
-    decode_share), so a step's shorter requests, and lengths below the step's rounded longest
-    one, still give every block of a token the same share."""
+    kernel deals every token's own keys to that many splits in rounds of 128
+    (csrc/attention_mfma.hip: kRoundKeys), so of a step's shorter requests, and below the step's rounded longest
+    length, the blocks of a token are within one round of each other; those without a round return at once."""
     pairs = max(1, num_decode * num_kv_heads)
     least = 16 * DECODE_WAVES
     most = max(1, -(-max_len // least))

@@ -21,12 +21,11 @@ import torch
 from tokamak_amd.kernels import ops
 
 
-# From nine rows on a product adds into the stream itself (one block walking the whole of K for 16 columns)
-# only if K is short: up to one chunk of 256 for each of a block's sixteen waves.  With a
-# longer K the split product and the norm kernel after it are as fast (measured: the o
-# projection of an 8B-shaped layer gains 2 us, its down projection nothing).  Where the direct product is
-# the faster form it adds at any K (down of an 8B-shaped layer at 8 rows: 20.3 us, split product and norm 21.3;
-# at one row 16.7 against 20.6).
+# Where the direct product is not the faster form (ops.direct_pays) a product adds into the stream itself (one block
+# walking the whole of K for 16 columns) only if K is short: up to one chunk of 256 for each of a block's sixteen
+# waves.  With a longer K the split product and the norm kernel after it are as fast (measured: the o projection of
+# an 8B-shaped layer gains 2 us, its down projection nothing).  The direct product adds at any K (down of an 8B-shaped
+# layer at 8 rows: 20.3 us, split product and norm 21.3; at one row 16.7 against 20.6).
 ADD_INTO_MAX_K = 16 * 256
 GATED_SPLIT_UP_TO_BLOCKS = 160      # blocks of the gated streaming product up to which K is split instead, the gate behind it
 GATED_WHOLEK_MAX_BYTES = 32 << 20   # gate and up together, up to which the whole-K form takes the gated product
@@ -220,7 +219,7 @@ def gated_linear(x: torch.Tensor | DeferredNorm, gate_up: torch.Tensor, activati
     inter = gate_up.shape[0] // 2
     # A small pair of matrices goes to the whole-K form, whose blocks of 16 columns let their waves split K, which
     # the streaming kernel cannot do under the gate; from 50 MB on the streaming kernel is ahead.  (Both
-    # hand over to the direct product where it is the faster form, ops.direct_pays: up to eight rows and for the smallest pairs.)
+    # hand over to the direct product where it is the faster form, ops.direct_pays.)
     small = 2 * gate_up.numel() <= GATED_WHOLEK_MAX_BYTES
     if isinstance(x, DeferredNorm):
         if _few_rows_fit(m, x.scaled, gate_up, ops.ROW_SCALE_MAX_ROWS) and (
