@@ -1,0 +1,90 @@
+"""Products of many rows (csrc/gemm_many.hip): every tile at its edges, in one round of blocks and in several, whole and in
+shares of K.  Operands are small whole numbers, whose sums are exact in float32 in any order, so the results are too."""
+
+import pytest
+import torch
+
+from tokamak_amd.kernels import linear, ops
+
+DEV = "cuda:0"
+TILES = [(256, 256), (256, 192), (128, 256), (256, 128), (128, 128)]
+
+
+def whole(rows, cols, most, seed):
+    return torch.randint(-most, most + 1, (rows, cols), generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16)
+
+
+def inside(t, value=float("nan")):
+    """The tensor as rows of a wider array of ``value``: what is read or written past a row's end shows."""
+    wide = torch.full((t.shape[0] + 2, t.shape[1] + 16), value, dtype=t.dtype, device=DEV)
+    wide[1:-1, 8:-8].copy_(t)
+    return wide, wide[1:-1, 8:-8]
+
+
+def outside_is_nan(wide):
+    return bool(torch.isnan(wide[0]).all() and torch.isnan(wide[-1]).all() and torch.isnan(wide[:, :8]).all() and torch.isnan(wide[:, -8:]).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("m, n, k", [(1, 8, 64), (127, 136, 128), (129, 256, 192), (257, 264, 64), (513, 520, 1088)])
+def test_tiles_and_shares_of_k(tile, m, n, k):
+    rows, columns = tile
+    x, w = whole(m, k, 3, 1), whole(n, k, 3, 2)
+    exact = x.double() @ w.double().T          # at most 9 k in size: whole numbers of float32
+    xs, ws = inside(x)[1], inside(w)[1]
+    wide, out = inside(torch.zeros(m, n, dtype=torch.bfloat16))
+    ops.gemm_many(xs, ws, out, rows=rows, columns=columns)
+    assert torch.equal(out.cpu(), exact.to(torch.bfloat16)) and outside_is_nan(wide)
+    for parts in {1, 2, 3, k // 64}:
+        if parts <= k // 64:
+            sums = torch.full((parts + 1, m, n), float("nan"), device=DEV)
+            ops.gemm_many(xs, ws, sums[:parts], rows=rows, columns=columns)
+            assert torch.equal(sums[:parts].double().sum(0).cpu(), exact) and torch.isnan(sums[parts]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile, m, n", [((256, 256), 4200, 4360), ((256, 192), 4200, 3272), ((128, 256), 2200, 4360), ((256, 128), 4200, 2312),
+                                        ((128, 128), 3000, 3080)])
+@pytest.mark.parametrize("k", [64, 192])
+def test_more_tiles_than_blocks_run_at_once(tile, m, n, k):
+    x, w = whole(m, k, 3, 3).to(DEV), whole(n, k, 3, 4).to(DEV)
+    exact = (x.float() @ w.float().T).to(torch.bfloat16)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.gemm_many(x, w, out, rows=tile[0], columns=tile[1])
+    assert torch.equal(out, exact)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [t for t in TILES if t[1] != 192])
+@pytest.mark.parametrize("m, n, k", [(1, 8, 64), (130, 72, 128), (255, 136, 192), (300, 1000, 64)])
+def test_gates(tile, m, n, k):
+    rows, columns = tile
+    x, w = whole(m, k, 3, 5), whole(2 * n, k, 1, 6)
+    sums = x.double() @ w.double().T
+    g, u = sums[:, :n], sums[:, n:]
+    xs, ws = inside(x)[1], inside(w)[1]
+    for gate, limit, want in (("silu", None, g * torch.sigmoid(g) * u),
+                              ("clamped", 2.5, g.clamp(max=2.5) * torch.sigmoid(1.702 * g.clamp(max=2.5)) * (u.clamp(-2.5, 2.5) + 1))):
+        wide, out = inside(torch.zeros(m, n, dtype=torch.bfloat16))
+        ops.gemm_many(xs, ws, out, rows=rows, columns=columns, gate=gate, limit=limit)
+        # half a unit of 2^-8 for the rounded result; the exponential's error is 2^-23 of its argument's size (up to 3 k), no more
+        assert ((out.cpu().double() - want).abs() <= (2.0 ** -8 + 3 * k * 2.0 ** -22) * want.abs() + 1e-30).all() and outside_is_nan(wide)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("activation, limit", [("silu", None), ("clamped", 7.0), ("gelu_tanh", None)])
+@pytest.mark.parametrize("m, n, k", [(128, 256, 256), (129, 256, 256), (300, 248, 320), (300, 252, 320), (300, 256, 328)])
+def test_gated_products_by_any_route(activation, limit, m, n, k):
+    """On both sides of each condition of the route, the same numbers to bfloat16's rounding."""
+    gen = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=gen).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(2 * n, k, generator=gen) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    got = linear.gated_linear(x, w, activation, limit)
+    parts = torch.empty(1, m, 2 * n, device=DEV)
+    parts[0] = (x.double() @ w.double().T).float()
+    want = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    if n % 4 == 0:
+        ops.silu_mul(parts, want, activation, limit=limit)
+        # the routes that round gate and up to bfloat16 first are off by 2^-8 of each (and of the sum of one and up)
+        assert (got.float() - want.float()).abs().max() <= 2.0 ** -6 * want.float().abs().max()

@@ -177,6 +177,21 @@ def activated_linear(x: torch.Tensor, weight: torch.Tensor, activation: str = "s
     return out
 
 
+GATED_MANY_FROM = 129       # rows from which the gated product has its own kernel with the gate behind it in registers; up to 128
+                            # the library's product and the gate's kernel are level with it (80 to 128 rows: 0.76 to 1.5 times)
+
+
+def _gated_many(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activation: str, limit: float | None) -> bool:
+    """The gated product of many rows in one kernel, whose block has a channel's gate and up sums side by side: 1.09 times as fast
+    as the library's fastest candidate and the gate's kernel at 150 to 300 rows, 1.11 to 1.25 times beyond (11 sizes of 2,048 to
+    34,816 channels, 0.82 to 2.25: rounds of blocks that end nearly empty, on either side)."""
+    if x.shape[0] < GATED_MANY_FROM or activation not in ops.MANY_MODES or not ops.gemm_many_fits(x, gate_up, out.shape[1]):
+        return False
+    rows, columns, _ = ops.many_plan(x.shape[0], out.shape[1], x.shape[1], True)
+    ops.gemm_many(x, gate_up, out, rows=rows, columns=columns, gate=activation, limit=limit)
+    return True
+
+
 def _gated_split(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activation: str, limit: float | None) -> bool:
     """The gated product of few rows as a product split over K and a gate that adds the partial sums.  The gated
     streaming kernel cannot split K under the gate: a matrix of few rows (a shared expert: 8,192 of 4,096, 128 blocks) leaves
@@ -213,7 +228,7 @@ def gated_linear(x: torch.Tensor | DeferredNorm, gate_up: torch.Tensor, activati
         if x.dtype == torch.bfloat16 and m <= 64 and gemm_bf16.skinny_fits(x, gate_up):
             if ops.direct_pays("gated", m, out.shape[1], x.shape[1]) or not _gated_split(x, gate_up, out, activation, limit):
                 ops.gemm_stream_swiglu(x, gate_up, out, activation=activation, limit=limit)
-        else:
+        elif not _gated_many(x, gate_up, out, activation, limit):
             ops.silu_mul(linear(x, gate_up), out, activation, limit=limit)
         return out
     inter = gate_up.shape[0] // 2
@@ -243,5 +258,6 @@ def gated_linear(x: torch.Tensor | DeferredNorm, gate_up: torch.Tensor, activati
             elif small or ops.direct_pays("gated", m, inter, x.shape[1]) or not _gated_split(x, gate_up, out, activation, limit):
                 ops.gemm_stream_swiglu(x, gate_up, out)
             return out
-    ops.silu_mul(linear(x, gate_up), out)
+    if not _gated_many(x, gate_up, out, activation, limit):
+        ops.silu_mul(linear(x, gate_up), out)
     return out

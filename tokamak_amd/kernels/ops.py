@@ -9,6 +9,7 @@ compiled library the call raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from ctypes import c_float, c_int, c_long, c_size_t, c_void_p
 
@@ -297,6 +298,10 @@ _SIGS = {
                            c_void_p, c_int, c_float, c_int, c_float, c_int, c_int, c_int, c_void_p],
         "tk_gemm_direct_add": [c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_void_p, c_long, c_void_p,
                                c_void_p, c_long, c_void_p, c_int, c_int, c_int, c_void_p],
+    },
+    "gemm_many": {
+        "tk_gemm_many": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_long,
+                         c_float, c_int, c_int, c_void_p],
     },
     "replay": {
         "tk_stream_order": [c_void_p, c_void_p],
@@ -2060,6 +2065,69 @@ def gemm_direct(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, sumsq: t
         _code(out.dtype), int(gated), _p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(0),
         _p(sumsq), 0 if sumsq is None else sumsq.shape[0], float(eps), act, float(limit or 0.0), rows, groups, waves, _stream()),
         "gemm_direct")
+
+
+MANY_MAX_STRIDE = 1 << 22      # (offsets within a tile's rows are 32 bits)
+
+
+def gemm_many_fits(a: torch.Tensor, w: torch.Tensor, n: int) -> bool:
+    """Whether ``gemm_many`` takes these operands for ``n`` output channels: bfloat16 rows on 16-byte borders, whole steps of 64 k."""
+    return (a.dtype == w.dtype == torch.bfloat16 and a.dim() == w.dim() == 2 and a.stride(1) == w.stride(1) == 1
+            and a.shape[1] >= 64 and a.shape[1] % 64 == 0 and n >= 8 and n % 8 == 0
+            and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and a.stride(0) <= MANY_MAX_STRIDE and w.stride(0) * (w.shape[0] + 256) < 1 << 31)
+
+
+# What a product of many rows is priced with, in microseconds: per tile (rows, columns) blocks that run at once; a step of 64 k
+# with all of them at work, and with one alone; a round's end; the start.  Fitted to 5,800 measured products (80 to 3,000 rows,
+# 1,024 to 34,816 channels of 1,024 to 17,408) within 6 to 10 % each; the tile so chosen is on average 2 % behind the best
+# one measured, at worst 30 % (128 rows).
+MANY_PRICES = {(256, 256): (256, 1.24, 0.914, 6.5, 4.3), (256, 192): (256, 0.94, 0.726, 3.7, 5.0), (128, 256): (256, 0.767, 0.533, 3.1, 4.1),
+               (256, 128): (256, 0.772, 0.556, 3.0, 3.2), (128, 128): (512, 0.913, 0.37, -0.2, 4.5)}
+
+
+@functools.lru_cache(maxsize=4096)
+def many_plan(m: int, n: int, k: int, gated: bool) -> tuple[int, int, float]:
+    """(rows of a tile, columns of a tile, microseconds expected) of the cheapest ``gemm_many`` for ``n`` output channels: the
+    tiles run in rounds of as many blocks as fit the GPU, and a round that is not full is faster a step."""
+    best = None
+    for (rows, columns), (slots, full, alone, end, start) in MANY_PRICES.items():
+        out = columns // 2 if gated else columns
+        if gated and columns % 128:
+            continue
+        rounds, rest = divmod(-(-m // rows) * -(-n // out), slots)
+        price = start + rounds * (k // 64 * full + end)
+        if rest:
+            price += k // 64 * (alone + (full - alone) * rest / slots) + end
+        if best is None or price < best[2]:
+            best = (rows, columns, price)
+    return best
+
+
+MANY_MODES = {None: 0, "silu": 2, "clamped": 3}      # of tk_gemm_many, by the gate's activation (1: partial sums)
+
+
+def gemm_many(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, rows: int, columns: int, gate: str | None = None,
+              limit: float | None = None) -> None:
+    """Products of many rows in tiles of ``rows`` by ``columns`` (256 x 256, 256 x 192 without a gate, 128 x 256, 256 x 128):
+    out[M, N] bfloat16 = a[M, K] @ w[N, K]^T; with a ``gate`` ("silu" or "clamped" with its ``limit``) w = [gate; up] and
+    out = act(a @ gate^T) * (a @ up^T), see ``silu_mul``; out [P, M, N] float32: the sums over P shares of K."""
+    for t in (a, w, out):
+        _need(t.is_cuda and t.stride(-1) == 1, "gemm operands are GPU tensors with unit inner stride")
+    split = out.dim() == 3
+    parts = out.shape[0] if split else 1
+    m, k = a.shape
+    n = out.shape[-1]
+    _need(a.dim() == w.dim() == 2 and w.shape == (n * (1 if gate is None else 2), k) and out.shape[-2] == m, "gemm shapes disagree")
+    _need(out.dtype == (torch.float32 if split else torch.bfloat16) and not (split and gate is not None),
+          "the product is bfloat16, its partial sums float32 [parts, M, N]")
+    _need(gemm_many_fits(a, w, n) and out.data_ptr() % 16 == 0 and out.stride(-2) % 8 == 0 and 1 <= parts <= k // 64,
+          "products of many rows take whole steps of 64 k and rows on 16-byte borders")
+    _need(gate in MANY_MODES and (gate == "clamped") == (limit is not None), "the gate is silu, or clamped with its limit")
+    _note(f"{m}x{w.shape[0]}x{k}", (w.shape[0] * k + m * k) * 2 + out.numel() * out.element_size(), 2.0 * m * w.shape[0] * k)
+    _check(_fn("gemm_many", "tk_gemm_many")(
+        1 if split else MANY_MODES[gate], _p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(-2), parts,
+        out.stride(0) if split else 0, float(limit or 0.0), rows, columns, _stream()), "gemm_many")
 
 
 def _stream_operands(resid: torch.Tensor, gamma: torch.Tensor | None, m: int, n: int) -> torch.Tensor | None:
