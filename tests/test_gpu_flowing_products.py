@@ -1,0 +1,87 @@
+"""Products of up to 128 rows whose weights stream through LDS (csrc/gemm_flow.hip), at the edges of its tiles and shares.
+Operands are small whole numbers, whose sums are exact in float32 in any order, so the results are too."""
+
+import pytest
+import torch
+
+from tokamak_amd.kernels import linear, ops
+
+DEV = "cuda:0"
+
+
+def whole(rows, cols, most, seed):
+    return torch.randint(-most, most + 1, (rows, cols), generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16)
+
+
+def inside(t):
+    """The tensor as rows of a wider array of NaN: what is read or written past a row's end shows."""
+    wide = torch.full((t.shape[0] + 2, t.shape[1] + 16), float("nan"), dtype=t.dtype, device=DEV)
+    wide[1:-1, 8:-8].copy_(t)
+    return wide, wide[1:-1, 8:-8]
+
+
+def outside_is_nan(wide):
+    return bool(torch.isnan(wide[0]).all() and torch.isnan(wide[-1]).all() and torch.isnan(wide[:, :8]).all() and torch.isnan(wide[:, -8:]).all())
+
+
+ROWS = [1, 15, 16, 17, 33, 64, 65, 81, 97, 127, 128]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", ROWS)
+@pytest.mark.parametrize("n, k", [(1, 128), (63, 256), (70, 384), (129, 1152), (260, 2048)])
+def test_products_and_shares_of_k(m, n, k):
+    x, w = whole(m, k, 3, 1), whole(n, k, 3, 2)
+    exact = x.double() @ w.double().T          # at most 9 k in size: whole numbers of float32
+    xs, ws = inside(x)[1], inside(w)[1]
+    for dtype in (torch.bfloat16, torch.float32):
+        wide, out = inside(torch.zeros(m, n, dtype=dtype))
+        ops.gemm_flow(xs, ws, out)
+        assert torch.equal(out.cpu(), exact.to(dtype)) and outside_is_nan(wide)
+    wide, out = inside(torch.zeros(m, n, dtype=torch.bfloat16))
+    ops.gemm_flow(xs, ws, out, activation="squared_relu")
+    assert torch.equal(out.cpu(), (exact.clamp(min=0).float() ** 2).to(torch.bfloat16)) and outside_is_nan(wide)
+    for parts in {1, 2, 3, k // 128}:
+        if parts <= k // 128:
+            sums = torch.full((parts + 1, m, n), float("nan"), device=DEV)
+            ops.gemm_flow(xs, ws, sums[:parts])
+            assert torch.equal(sums[:parts].double().sum(0).cpu(), exact) and torch.isnan(sums[parts]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", ROWS)
+@pytest.mark.parametrize("n, k", [(4, 128), (37, 256), (100, 512)])
+def test_gates(m, n, k):
+    x, w = whole(m, k, 3, 5), whole(2 * n, k, 1, 6)
+    sums = x.double() @ w.double().T
+    g, u = sums[:, :n], sums[:, n:]
+    xs, ws = inside(x)[1], inside(w)[1]
+    for gate, limit, want in (("silu", None, g * torch.sigmoid(g) * u),
+                              ("gelu_tanh", None, torch.nn.functional.gelu(g, approximate="tanh") * u),
+                              ("clamped", 2.5, g.clamp(max=2.5) * torch.sigmoid(1.702 * g.clamp(max=2.5)) * (u.clamp(-2.5, 2.5) + 1))):
+        wide, out = inside(torch.zeros(m, n, dtype=torch.bfloat16))
+        ops.gemm_flow(xs, ws, out, gate=gate, limit=limit)
+        # half a unit of 2^-8 for the rounded result; the exponential's error is 2^-23 of its argument's size (up to 3 k);
+        # 1 + tanh is off by 2^-22 of one where the tangent is near -1
+        slack = 2.0 ** -22 * (g * u).abs() if gate == "gelu_tanh" else 0.0
+        assert ((out.cpu().double() - want).abs() <= (2.0 ** -8 + 3 * k * 2.0 ** -22) * want.abs() + slack + 1e-30).all(), gate
+        assert outside_is_nan(wide)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [2, 3, 16, 17, 64, 65, 96, 97])
+@pytest.mark.parametrize("n, k", [(1040, 256), (1040, 264), (1040, 2048)])
+def test_every_route_gives_the_product(m, n, k):
+    """On both sides of each condition of the routes, exactly."""
+    x, w = whole(m, k, 2, 7).to(DEV), whole(n, k, 2, 8).to(DEV)
+    exact = x.float() @ w.float().T
+    assert torch.equal(linear.linear(x, w), exact.to(torch.bfloat16))
+    assert torch.equal(linear.linear(x, w, torch.float32), exact)
+    parts = linear.linear(x, w, allow_partials=True)
+    assert torch.equal(parts.float().sum(0) if parts.dim() == 3 else parts, exact if parts.dim() == 3 else exact.to(torch.bfloat16))
+    gate = linear.gated_linear(x, w)
+    half = n // 2
+    want = torch.nn.functional.silu(exact[:, :half].double()) * exact[:, half:].double()
+    # (some routes round gate and up to bfloat16 first: 2^-9 of each, the gate's of its argument)
+    slack = (2.0 ** -7 + 2.0 ** -9 * exact[:, :half].abs().double()) * want.abs() + 1e-30
+    assert ((gate.double() - want).abs() <= slack).all()

@@ -87,6 +87,31 @@ STREAM_PARTIALS_ROWS = 96           # rows up to which the split streaming produ
 STREAM_PARTIALS_BIG = 64 << 20      # ... and the bytes of a matrix from which it does up to 128 rows
 
 
+FLOW_SPLIT_ROWS = (3, 96)           # rows between which a product whose reader adds partial sums flows (csrc/gemm_flow.hip): beside the forms
+                                    # below, 20 sizes, weights from memory: 1.06 to 1.08 times as fast at 3 to 8 rows, 1.10 at 16,
+                                    # 1.13 to 1.15 at 17 to 64, 1.31 to 1.34 at 65 to 96; at 128 level, 0.81 at worst.  With fewer rows it is
+                                    # 1.06 times as fast alone, but beside an experts' branch its few large blocks wait for room (a
+                                    # decode step of one request 623 -> 663 us, of two 731 -> 735)
+FLOW_ROWS = (17, 64)                # ... and one into bfloat16: 1.2 to 1.6 times; with fewer rows the direct form, with more
+                                    # the library is ahead of blocks that cannot share K.  (A logits head into float32, one share
+                                    # of K: decode steps of 36 to 64 rows 7 to 53 us slower than with the streaming kernel.)
+
+
+def flows(x: torch.Tensor, weight: torch.Tensor, allow_partials: bool) -> bool:
+    """Whether a product goes to the flowing kernel: into partial sums, or into bfloat16."""
+    low, high = FLOW_SPLIT_ROWS if allow_partials else FLOW_ROWS
+    return low <= x.shape[0] <= high and ops.gemm_flow_fits(x, weight)
+
+
+def flow(x: torch.Tensor, weight: torch.Tensor, allow_partials: bool) -> torch.Tensor:
+    """Partial sums [P, M, N], or the product in bfloat16, by the flowing kernel."""
+    m, n, k = x.shape[0], *weight.shape
+    out = (torch.empty((ops.flow_parts(m, n, k), m, n), dtype=torch.float32, device=x.device) if allow_partials
+           else torch.empty((m, n), dtype=torch.bfloat16, device=x.device))
+    ops.gemm_flow(x, weight, out)
+    return out
+
+
 def stream_pays_beyond_64_rows(m: int, n: int, k: int) -> bool:
     """Whether a product of 65 to 128 rows whose reader adds partial sums goes to the streaming
     kernel (five to eight tiles of 16 rows, eight waves a block) rather than to the library.

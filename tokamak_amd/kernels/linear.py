@@ -128,6 +128,8 @@ def linear(x: torch.Tensor | DeferredNorm, weight: torch.Tensor, out_dtype: torc
             return Added(*ops.gemm_wholek_add(x, weight, add_into.resid, add_into.gamma), add_into.gamma)
         if ops.direct_pays("add", m, n, weight.shape[1]):
             return Added(*ops.gemm_direct_add(x, weight, add_into.resid, add_into.gamma), add_into.gamma)
+    if (allow_partials or out_dtype == torch.bfloat16) and gemm_bf16.flows(x, weight, allow_partials):
+        return gemm_bf16.flow(x, weight, allow_partials)
     if _few_rows_fit(m, x, weight, ops.DIRECT_MAX_ROWS) and ops.direct_pays("parts" if allow_partials else "plain", m, n, weight.shape[1]):
         return _direct(x, weight, out_dtype, allow_partials)
     return gemm_bf16.gemm(x, weight, out_dtype, allow_partials)
@@ -169,6 +171,8 @@ def activated_linear(x: torch.Tensor, weight: torch.Tensor, activation: str = "s
         return out
     if _few_rows_fit(m, x, weight, ops.DIRECT_MAX_ROWS) and ops.direct_pays("activated", m, n, k):
         ops.gemm_direct(x, weight, out, activation=activation)
+    elif gemm_bf16.flows(x, weight, False):
+        ops.gemm_flow(x, weight, out, activation=activation)
     elif (x.dtype == torch.bfloat16 and m <= gemm_bf16.SKINNY_MAX_ROWS and n >= gemm_bf16.STREAM_MIN_ROWS_OUT
             and gemm_bf16.skinny_fits(x, weight) and gemm_bf16.stream_splits(n, k, m) < ACTIVATED_SPLIT_FROM):
         ops.gemm_stream(x, weight, out, activation=activation)
@@ -179,6 +183,22 @@ def activated_linear(x: torch.Tensor, weight: torch.Tensor, activation: str = "s
 
 GATED_MANY_FROM = 129       # rows from which the gated product has its own kernel with the gate behind it in registers; up to 128
                             # the library's product and the gate's kernel are level with it (80 to 128 rows: 0.76 to 1.5 times)
+
+
+FLOW_GATED_MOST = 36 << 20      # numbers of gate and up below which their product of 17 to 96 rows flows: 2,048 x 1,024 to 12,288 x 2,048
+                                # 1.06 to 1.77 times as fast (a decode step of 24 rows of 2,048 895 -> 837 us); 19,456 x 2,560 and
+                                # more, whose blocks cannot share K, 0.8 to 1.05 (64 rows of 2,560 1,008 -> 1,044)
+
+
+def _gated_flow(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activation: str, limit: float | None) -> bool:
+    """The gated product of 17 to 96 rows of a small matrix with its weights streamed through LDS (csrc/gemm_flow.hip)."""
+    from tokamak_amd.kernels import gemm_bf16
+
+    if (not gemm_bf16.FLOW_ROWS[0] <= x.shape[0] <= gemm_bf16.FLOW_SPLIT_ROWS[1] or gate_up.numel() >= FLOW_GATED_MOST
+            or not ops.gemm_flow_fits(x, gate_up)):
+        return False
+    ops.gemm_flow(x, gate_up, out, gate=activation, limit=limit)
+    return True
 
 
 def _gated_many(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activation: str, limit: float | None) -> bool:
@@ -225,6 +245,8 @@ def gated_linear(x: torch.Tensor | DeferredNorm, gate_up: torch.Tensor, activati
             return out
         from tokamak_amd.kernels import gemm_bf16
 
+        if _gated_flow(x, gate_up, out, activation, limit):
+            return out
         if x.dtype == torch.bfloat16 and m <= 64 and gemm_bf16.skinny_fits(x, gate_up):
             if ops.direct_pays("gated", m, out.shape[1], x.shape[1]) or not _gated_split(x, gate_up, out, activation, limit):
                 ops.gemm_stream_swiglu(x, gate_up, out, activation=activation, limit=limit)
@@ -247,7 +269,7 @@ def gated_linear(x: torch.Tensor | DeferredNorm, gate_up: torch.Tensor, activati
             return out
         x = x.materialize()
     out = torch.empty((m, inter), dtype=x.dtype, device=x.device)
-    if m == 0:
+    if m == 0 or _gated_flow(x, gate_up, out, activation, limit):
         return out
     if x.dtype == torch.bfloat16 and m <= 64:
         from tokamak_amd.kernels import gemm_bf16

@@ -299,6 +299,10 @@ _SIGS = {
         "tk_gemm_direct_add": [c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_void_p, c_long, c_void_p,
                                c_void_p, c_long, c_void_p, c_int, c_int, c_int, c_void_p],
     },
+    "gemm_flow": {
+        "tk_gemm_flow": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_long, c_int,
+                         c_float, c_void_p],
+    },
     "gemm_many": {
         "tk_gemm_many": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_long,
                          c_float, c_int, c_int, c_void_p],
@@ -2065,6 +2069,77 @@ def gemm_direct(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, sumsq: t
         _code(out.dtype), int(gated), _p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(0),
         _p(sumsq), 0 if sumsq is None else sumsq.shape[0], float(eps), act, float(limit or 0.0), rows, groups, waves, _stream()),
         "gemm_direct")
+
+
+FLOW_MAX_ROWS = 128
+FLOW_GATES = {"silu": 2, "gelu_tanh": 3, "clamped": 4}      # modes of tk_gemm_flow
+
+
+def gemm_flow(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, gate: str | None = None, limit: float | None = None,
+              activation: str | None = None) -> None:
+    """Products of up to 128 rows, the weights streamed through LDS:
+    out[M, N] (bfloat16 or float32) = a[M, K] @ w[N, K]^T, with ``activation`` "squared_relu" (bfloat16) max(., 0)^2 of it; with
+    a ``gate`` w = [gate; up] and out (bfloat16) = act(a @ gate^T) * (a @ up^T), see ``silu_mul``; out [P, M, N] float32: the
+    sums over P shares of K."""
+    for t in (a, w, out):
+        _need(t.is_cuda and t.stride(-1) == 1, "gemm operands are GPU tensors with unit inner stride")
+    split = out.dim() == 3
+    parts = out.shape[0] if split else 1
+    m, k = a.shape
+    n = out.shape[-1]
+    _need(a.dim() == w.dim() == 2 and w.shape == (n * (1 if gate is None else 2), k) and out.shape[-2] == m, "gemm shapes disagree")
+    _need(gemm_flow_fits(a, w) and 1 <= parts <= k // 128, "the flowing product takes 1 to 128 rows of whole steps of 128 k on 16-byte borders")
+    _need(out.dtype == torch.float32 if split else out.dtype in _DT, "partial sums are float32")
+    plain = out.dtype == torch.bfloat16 and not split
+    _need(gate is None or (plain and gate in FLOW_GATES and activation is None), f"the gate is one of {sorted(FLOW_GATES)}, into bfloat16")
+    _need((gate == "clamped") == (limit is not None), "a limit goes with the clamped gate")
+    _need(activation is None or (plain and activation == "squared_relu"), "the product's activation is squared_relu, into bfloat16")
+    _note(f"{m}x{w.shape[0]}x{k}", (w.shape[0] * k + m * k) * 2 + out.numel() * out.element_size(), 2.0 * m * w.shape[0] * k)
+    _check(_fn("gemm_flow", "tk_gemm_flow")(
+        FLOW_GATES[gate] if gate is not None else 0 if plain else 1, _p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0),
+        out.stride(-2), parts, out.stride(0) if split else 0, int(activation is not None), float(limit or 0.0), _stream()),
+        "gemm_flow")
+
+
+# What a flowing product is priced with: its start (microseconds), the rates of a CU and of the GPU (bytes a microsecond), a float32
+# sum written and read (microseconds a byte).  Fitted to 1,650 measured products (1 to 128 rows, 384 to 12,800 channels of
+# 384 to 17,408, weights from memory) within 6 % each; the number of shares so chosen is 0.4 % behind the best one measured on
+# average, at worst 13 % (128 rows).
+FLOW_START, FLOW_CU_RATE, FLOW_RATE, FLOW_WRITE, FLOW_READ = 2.47, 44.8e3, 6.91e6, 0.536e-6, 0.222e-6
+FLOW_PARTS = (1, 2, 3, 4, 5, 6, 8, 10, 12, 16)
+FLOW_STEP, FLOW_COLUMNS = 128, 64       # k of a step, weight rows a block (csrc/gemm_flow.hip)
+
+
+@functools.lru_cache(maxsize=8192)
+def flow_parts(m: int, n: int, k: int) -> int:
+    """Shares of K of a flowing product whose reader adds partial sums.  A step of a block is its bytes at the rate of its CU,
+    whose blocks share it, and all blocks' weights at the GPU's; K is cut where more blocks carry more bytes at once,
+    which the sums' bytes then have to pay for."""
+    blocks, steps = -(-n // FLOW_COLUMNS), k // FLOW_STEP
+    weights, rows = FLOW_COLUMNS * FLOW_STEP * 2, -(-m // 16) * 16 * FLOW_STEP * 2
+    at_once = 256 * (160 * 1024 // (3 * (weights + rows)))
+
+    def step(count: int) -> float:
+        return ((-(-count // 256) * (weights + rows) / FLOW_CU_RATE) ** 3 + (count * weights / FLOW_RATE) ** 3) ** (1 / 3)
+
+    best = None
+    for parts in FLOW_PARTS:
+        if parts > max(1, steps // 2):
+            break
+        rounds, rest = divmod(blocks * parts, at_once)
+        price = FLOW_START + -(-steps // parts) * (rounds * step(at_once) + (step(rest) if rest else 0.0))
+        price += 4 * parts * m * n * ((FLOW_WRITE if parts > 1 else 0.0) + FLOW_READ)
+        if best is None or price < best[0]:
+            best = (price, parts)
+    return best[1]
+
+
+def gemm_flow_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gemm_flow`` takes these operands: bfloat16 rows on 16-byte borders, up to 128 of them, whole steps of 128 k."""
+    return (a.dtype == w.dtype == torch.bfloat16 and a.dim() == w.dim() == 2 and a.stride(1) == w.stride(1) == 1
+            and 0 < a.shape[0] <= FLOW_MAX_ROWS and a.shape[1] >= 128 and a.shape[1] % 128 == 0
+            and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and a.stride(0) <= MANY_MAX_STRIDE and w.stride(0) * (w.shape[0] + 128) < 1 << 31)
 
 
 MANY_MAX_STRIDE = 1 << 22      # (offsets within a tile's rows are 32 bits)
