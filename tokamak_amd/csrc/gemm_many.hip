@@ -1,5 +1,5 @@
-// bf16 products of many rows (prompt portions): C[M,N] = A[M,K] W[N,K]^T with float32 sums; as they are, in shares of K as
-// partial sums, or gated (W = [gate; up], C = act(A gate^T) * (A up^T)) with no array of gate and up in between.
+// bf16 products of many rows (prompt portions) with float32 sums: C[M,N] = A[M,K] W[N,K]^T in shares of K as partial sums, or
+// gated (W = [gate; up], C = act(A gate^T) * (A up^T)) with no array of gate and up in between.
 //
 // A block of four waves owns a tile, a wave a quarter of it, all of whose sums stay in accumulation registers (a 256 x 256 tile
 // takes half of a CU's registers, so a wave has its SIMD to itself).  Both operands go from memory to LDS without passing
@@ -14,7 +14,9 @@
 //
 // Beside the library's fastest candidate and the gate's kernel, gated, us: 24,576 x 4,096 at 256 / 512 / 1,024 / 2,048 rows 67 / 98 /
 // 253 / 317, here 62 / 90 / 170 / 288 (1.43 PFLOP/s); 19,456 x 2,560 at 512 / 1,024 / 2,048 rows 96 / 148 / 213, here 57 / 99 / 179;
-// 6,144 x 1,024 at 256 / 1,024 / 2,048 rows 15.1 / 33.1 / 35.5, here 11.9 / 18.5 / 28.6.
+// 6,144 x 1,024 at 256 / 1,024 / 2,048 rows 15.1 / 33.1 / 35.5, here 11.9 / 18.5 / 28.6.  In shares of K, with what the sums cost
+// their reader, beside the library's first choice: 4,096 x 12,288 at 200 / 512 / 1,024 rows 45 / 75 / 106, here 37 / 55 / 93; 2,560 x
+// 9,728 32 / 46 / 62, here 26 / 36 / 53; 5,120 x 17,408 226 / 168 / 246, here 57 / 90 / 149.
 #include "common.h"
 #include "slots.h"
 
@@ -35,7 +37,7 @@ union Frag8 {
 
 #define TK_LDS __attribute__((address_space(3)))
 
-enum { EPI_STORE, EPI_PARTS, EPI_SILU, EPI_CLAMPED };     // the last two: gated
+enum { EPI_PARTS, EPI_SILU, EPI_CLAMPED };     // the last two: gated
 
 constexpr int kCus = 256;       // blocks that run at once
 constexpr int kXcds = 8;        // dies, each with an L2 of its own; blocks go to them in turn
@@ -286,11 +288,10 @@ int launch(Job job, hipStream_t stream) {
 
 }  // namespace
 
-// mode 0: C[M, N] bfloat16 = A W^T; modes 2 and 3: W = [W_gate; W_up] of 2 N rows and C[M, N] bfloat16 =
-// act(A W_gate^T) * (A W_up^T), act silu or (3) the gate whose halves are clamped at `limit`;
-// mode 1: C float32 [parts][M, N], part_stride elements apart: the sums over `parts` shares of K.
-// rows, columns: a tile's rows of A and of W (256 x 256, 256 x 192 without a gate, 128 x 256, 256 x 128).  K a multiple of 64, N of
-// 8; rows of all operands 16-byte aligned.
+// mode 0: C float32 [parts][M, N], part_stride elements apart: the sums over `parts` shares of K; modes 1 and 2: W = [W_gate;
+// W_up] of 2 N rows and C[M, N] bfloat16 = act(A W_gate^T) * (A W_up^T), act silu or (2) the gate whose halves are clamped at
+// `limit`.  rows, columns: a tile's rows of A and of W (256 x 256, 128 x 256, 256 x 128, 128 x 128).  K a multiple of 64, N of 8;
+// rows of all operands 16-byte aligned.
 TK_API int tk_gemm_many(int mode, const void* A, const void* W, void* C, int M, int N, int K, long lda, long ldw, long ldc,
                         int parts, long part_stride, float limit, int rows, int columns, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
@@ -304,15 +305,11 @@ TK_API int tk_gemm_many(int mode, const void* A, const void* W, void* C, int M, 
   const Job job{(const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, part_stride, 0, 0, parts, limit};
 #define TK_SHAPE(MT_, NT_)                                                             \
   if (rows == 64 * MT_ && columns == 64 * NT_) {                                       \
-    if (mode == EPI_STORE) return launch<MT_, NT_, EPI_STORE>(job, stream);            \
     if (mode == EPI_PARTS) return launch<MT_, NT_, EPI_PARTS>(job, stream);            \
-    if constexpr (NT_ % 2 == 0) {                                                      \
-      if (mode == EPI_SILU) return launch<MT_, NT_, EPI_SILU>(job, stream);            \
-      return launch<MT_, NT_, EPI_CLAMPED>(job, stream);                               \
-    }                                                                                  \
+    if (mode == EPI_SILU) return launch<MT_, NT_, EPI_SILU>(job, stream);              \
+    return launch<MT_, NT_, EPI_CLAMPED>(job, stream);                                 \
   }
   TK_SHAPE(4, 4)
-  TK_SHAPE(4, 3)
   TK_SHAPE(2, 4)
   TK_SHAPE(4, 2)
   TK_SHAPE(2, 2)

@@ -112,6 +112,31 @@ def flow(x: torch.Tensor, weight: torch.Tensor, allow_partials: bool) -> torch.T
     return out
 
 
+# Rows up to which, from 129 on, a product whose reader adds partial sums is cut into shares of K (csrc/gemm_many.hip), by the K it
+# has at least: tiles of a long K that are whole leave most CUs idle.  Beside the library's first choice, reader included: 2,560 x
+# 9,728 1.07 to 1.30 times as fast, 4,096 x 12,288 1.04 to 1.98, 5,120 x 17,408 1.55 to 3.98; K of 9,728 and 12,288 at 1,300 to 2,048
+# rows 0.99 to 1.18, K of 17,408 at 2,048 1.05; K of 8,192 0.92 to 1.55, of 6,144 0.83 to 1.31, of 5,120 and less mostly below 1.  One
+# prompt of 512 / 1,000 tokens through twelve layers 4,096 wide 3.75 / 5.79 -> 3.42 / 5.44 ms, 1,000 through 2,560 wide 4.20 -> 3.91.
+MANY_SPLIT_ROWS = ((16384, 1700), (9216, 1100))
+
+
+def splits_many(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether a product of many rows is cut into shares of K for its reader to add."""
+    m, k = x.shape
+    most = next((rows for least, rows in MANY_SPLIT_ROWS if k >= least), 0)
+    return (128 < m <= most and ops.gemm_many_fits(x, weight, weight.shape[0])
+            and ops.many_split_plan(m, weight.shape[0], k)[2] > 1)
+
+
+def split_many(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """Partial sums [P, M, N] of a product of many rows."""
+    m, n, k = x.shape[0], *weight.shape
+    rows, columns, parts = ops.many_split_plan(m, n, k)
+    out = torch.empty((parts, m, n), dtype=torch.float32, device=x.device)
+    ops.gemm_many(x, weight, out, rows=rows, columns=columns)
+    return out
+
+
 def stream_pays_beyond_64_rows(m: int, n: int, k: int) -> bool:
     """Whether a product of 65 to 128 rows whose reader adds partial sums goes to the streaming
     kernel (five to eight tiles of 16 rows, eight waves a block) rather than to the library.
@@ -128,7 +153,8 @@ def stream_pays_beyond_64_rows(m: int, n: int, k: int) -> bool:
 
 def gemm(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, allow_partials: bool = False) -> torch.Tensor:
     """x[M, K] @ weight[N, K]^T -> [M, N] in ``out_dtype``; or, if the caller can
-    add them (``allow_partials``), float32 partial sums [P, M, N] of a split-K product.
+    add them (``allow_partials``), float32 partial sums [P, M, N] of a split-K product.  (What
+    ``flows`` or ``splits_many`` says is another kernel's does not come here.)
 
     Up to 64 rows (decode batches, wanted logits rows): hand-written
     weight-streaming MFMA kernels: the LDS-staged one, split over K into partial

@@ -130,6 +130,8 @@ def linear(x: torch.Tensor | DeferredNorm, weight: torch.Tensor, out_dtype: torc
             return Added(*ops.gemm_direct_add(x, weight, add_into.resid, add_into.gamma), add_into.gamma)
     if (allow_partials or out_dtype == torch.bfloat16) and gemm_bf16.flows(x, weight, allow_partials):
         return gemm_bf16.flow(x, weight, allow_partials)
+    if allow_partials and gemm_bf16.splits_many(x, weight):
+        return gemm_bf16.split_many(x, weight)
     if _few_rows_fit(m, x, weight, ops.DIRECT_MAX_ROWS) and ops.direct_pays("parts" if allow_partials else "plain", m, n, weight.shape[1]):
         return _direct(x, weight, out_dtype, allow_partials)
     return gemm_bf16.gemm(x, weight, out_dtype, allow_partials)
@@ -205,9 +207,9 @@ def _gated_many(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activ
     """The gated product of many rows in one kernel, whose block has a channel's gate and up sums side by side: 1.09 times as fast
     as the library's fastest candidate and the gate's kernel at 150 to 300 rows, 1.11 to 1.25 times beyond (11 sizes of 2,048 to
     34,816 channels, 0.82 to 2.25: rounds of blocks that end nearly empty, on either side)."""
-    if x.shape[0] < GATED_MANY_FROM or activation not in ops.MANY_MODES or not ops.gemm_many_fits(x, gate_up, out.shape[1]):
+    if x.shape[0] < GATED_MANY_FROM or activation not in ("silu", "clamped") or not ops.gemm_many_fits(x, gate_up, out.shape[1]):
         return False
-    rows, columns, _ = ops.many_plan(x.shape[0], out.shape[1], x.shape[1], True)
+    rows, columns = ops.many_plan(x.shape[0], out.shape[1], x.shape[1])
     ops.gemm_many(x, gate_up, out, rows=rows, columns=columns, gate=activation, limit=limit)
     return True
 

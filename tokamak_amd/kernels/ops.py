@@ -2157,51 +2157,59 @@ def gemm_many_fits(a: torch.Tensor, w: torch.Tensor, n: int) -> bool:
 # with all of them at work, and with one alone; a round's end; the start.  Fitted to 5,800 measured products (80 to 3,000 rows,
 # 1,024 to 34,816 channels of 1,024 to 17,408) within 6 to 10 % each; the tile so chosen is on average 2 % behind the best
 # one measured, at worst 30 % (128 rows).
-MANY_PRICES = {(256, 256): (256, 1.24, 0.914, 6.5, 4.3), (256, 192): (256, 0.94, 0.726, 3.7, 5.0), (128, 256): (256, 0.767, 0.533, 3.1, 4.1),
+MANY_PRICES = {(256, 256): (256, 1.24, 0.914, 6.5, 4.3), (128, 256): (256, 0.767, 0.533, 3.1, 4.1),
                (256, 128): (256, 0.772, 0.556, 3.0, 3.2), (128, 128): (512, 0.913, 0.37, -0.2, 4.5)}
 
 
+def _many_price(rows: int, columns: int, m: int, channels: int, k: int, parts: int) -> float:
+    slots, full, alone, end, start = MANY_PRICES[rows, columns]
+    steps = k / 64 / parts
+    rounds, rest = divmod(-(-m // rows) * -(-channels // columns) * parts, slots)
+    price = start + rounds * (steps * full + end)
+    if rest:
+        price += steps * (alone + (full - alone) * rest / slots) + end
+    return price
+
+
 @functools.lru_cache(maxsize=4096)
-def many_plan(m: int, n: int, k: int, gated: bool) -> tuple[int, int, float]:
-    """(rows of a tile, columns of a tile, microseconds expected) of the cheapest ``gemm_many`` for ``n`` output channels: the
-    tiles run in rounds of as many blocks as fit the GPU, and a round that is not full is faster a step."""
-    best = None
-    for (rows, columns), (slots, full, alone, end, start) in MANY_PRICES.items():
-        out = columns // 2 if gated else columns
-        if gated and columns % 128:
-            continue
-        rounds, rest = divmod(-(-m // rows) * -(-n // out), slots)
-        price = start + rounds * (k // 64 * full + end)
-        if rest:
-            price += k // 64 * (alone + (full - alone) * rest / slots) + end
-        if best is None or price < best[2]:
-            best = (rows, columns, price)
-    return best
+def many_plan(m: int, n: int, k: int) -> tuple[int, int]:
+    """(rows, columns) of the cheapest tile of a gated ``gemm_many`` for ``n`` output channels: the tiles run in rounds of as many
+    blocks as fit the GPU, and a round that is not full is faster a step."""
+    return min(MANY_PRICES, key=lambda tile: _many_price(*tile, m, 2 * n, k, 1))
 
 
-MANY_MODES = {None: 0, "silu": 2, "clamped": 3}      # of tk_gemm_many, by the gate's activation (1: partial sums)
+@functools.lru_cache(maxsize=4096)
+def many_split_plan(m: int, n: int, k: int) -> tuple[int, int, int]:
+    """(rows, columns of a tile, shares of K) of the cheapest ``gemm_many`` into partial sums, which cost their reader four bytes a
+    number each where the product itself costs two (at 4.5 TB/s)."""
+    plans = [(_many_price(*tile, m, n, k, parts) + (4 * parts - 2) * m * n / 4.5e6, *tile, parts)
+             for tile in MANY_PRICES for parts in (1, 2, 3, 4, 6, 8, 12) if parts == 1 or k // 64 // parts >= 4]
+    return min(plans)[1:]
+
+
+MANY_MODES = {None: 0, "silu": 1, "clamped": 2}      # of tk_gemm_many, by the gate's activation
 
 
 def gemm_many(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, rows: int, columns: int, gate: str | None = None,
               limit: float | None = None) -> None:
-    """Products of many rows in tiles of ``rows`` by ``columns`` (256 x 256, 256 x 192 without a gate, 128 x 256, 256 x 128):
-    out[M, N] bfloat16 = a[M, K] @ w[N, K]^T; with a ``gate`` ("silu" or "clamped" with its ``limit``) w = [gate; up] and
-    out = act(a @ gate^T) * (a @ up^T), see ``silu_mul``; out [P, M, N] float32: the sums over P shares of K."""
+    """Products of many rows in tiles of ``rows`` by ``columns`` (256 x 256, 128 x 256, 256 x 128, 128 x 128): out [P, M, N] float32,
+    the sums of a[M, K] @ w[N, K]^T over P shares of K; or with a ``gate`` ("silu", or "clamped" with its ``limit``) w = [gate; up]
+    and out[M, N] bfloat16 = act(a @ gate^T) * (a @ up^T), see ``silu_mul``."""
     for t in (a, w, out):
         _need(t.is_cuda and t.stride(-1) == 1, "gemm operands are GPU tensors with unit inner stride")
-    split = out.dim() == 3
+    split = gate is None
+    _need(out.dim() == (3 if split else 2) and out.dtype == (torch.float32 if split else torch.bfloat16),
+          "partial sums are float32 [parts, M, N], a gated product bfloat16")
     parts = out.shape[0] if split else 1
     m, k = a.shape
     n = out.shape[-1]
-    _need(a.dim() == w.dim() == 2 and w.shape == (n * (1 if gate is None else 2), k) and out.shape[-2] == m, "gemm shapes disagree")
-    _need(out.dtype == (torch.float32 if split else torch.bfloat16) and not (split and gate is not None),
-          "the product is bfloat16, its partial sums float32 [parts, M, N]")
+    _need(a.dim() == w.dim() == 2 and w.shape == (n * (1 if split else 2), k) and out.shape[-2] == m, "gemm shapes disagree")
     _need(gemm_many_fits(a, w, n) and out.data_ptr() % 16 == 0 and out.stride(-2) % 8 == 0 and 1 <= parts <= k // 64,
           "products of many rows take whole steps of 64 k and rows on 16-byte borders")
     _need(gate in MANY_MODES and (gate == "clamped") == (limit is not None), "the gate is silu, or clamped with its limit")
     _note(f"{m}x{w.shape[0]}x{k}", (w.shape[0] * k + m * k) * 2 + out.numel() * out.element_size(), 2.0 * m * w.shape[0] * k)
     _check(_fn("gemm_many", "tk_gemm_many")(
-        1 if split else MANY_MODES[gate], _p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(-2), parts,
+        MANY_MODES[gate], _p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(-2), parts,
         out.stride(0) if split else 0, float(limit or 0.0), rows, columns, _stream()), "gemm_many")
 
 
