@@ -18,7 +18,6 @@ A block takes part only if it says ``replayable``: its parts launch all their wo
 
 from __future__ import annotations
 
-import bisect
 import dataclasses
 from ctypes import c_void_p
 from dataclasses import dataclass, field
@@ -91,6 +90,24 @@ def call_tensors(own: dict, pending, then) -> dict[tuple, torch.Tensor]:
     return out
 
 
+def patched_calls(calls: list[tuple], tensors: dict[tuple, torch.Tensor]) -> list[tuple]:
+    """Recorded calls (function, arguments, status) with the arguments that are addresses inside one of ``tensors``: (function,
+    arguments, ((argument index, tensor key, byte offset), ...), status)."""
+    spans = sorted((t.data_ptr(), t.data_ptr() + _span_bytes(t), key) for key, t in tensors.items() if t.numel())
+    places = [(c, index, arg.value) for c, (_, args, _) in enumerate(calls) for index, arg in enumerate(args)
+              if arg.__class__ is c_void_p and arg.value]
+    patches: list[list[tuple]] = [[] for _ in calls]
+    if spans and places:
+        values = np.array([value for _, _, value in places], dtype=np.int64)
+        starts, ends = (np.array([s[i] for s in spans], dtype=np.int64) for i in (0, 1))
+        at = np.searchsorted(starts, values, side="right") - 1      # (the spans of different tensors do not overlap)
+        for i in np.flatnonzero((at >= 0) & (values < ends[at])).tolist():
+            c, index, value = places[i]
+            start, _, key = spans[at[i]]
+            patches[c].append((index, key, value - start))
+    return [(fn, args, tuple(own), status) for (fn, args, status), own in zip(calls, patches)]
+
+
 class PackedCalls:
     """A recording's calls laid out for ``ops.replay_calls``: the slot forms' addresses, every
     call's arguments as 64-bit slots in one array, and the patches (slot, index of the tensor
@@ -132,9 +149,7 @@ class PackedCalls:
                                                             self.addresses, self.expected, self.got))
 
     def launch(self, tensors: dict[tuple, torch.Tensor]) -> None:
-        addresses = self.addresses
-        for i, key in enumerate(self.keys):
-            addresses[i] = tensors[key].data_ptr()
+        self.addresses[:len(self.keys)] = [tensors[key].data_ptr() for key in self.keys]
         bad = ops.replay_calls(len(self.expected), *self.pointers, len(self.patch_slot), *self.patch_pointers)
         if bad >= 0:
             raise ops.KernelError(f"replayed launch {bad} returned {int(self.got[0])}, the recorded one "
@@ -143,27 +158,42 @@ class PackedCalls:
 
 @dataclass
 class LayerRecording:
-    """The list is packed for the one-call form after its first replay, not when it is made:
-    the first layers of a step are launched while the GPU has nothing else to do, and the
-    packing (some 0.1 ms) would hold up the second layer's kernels; after it, the GPU has that
-    layer's work and the host's time is hidden (a step of 2,048 tokens at 0.6B width, timed
-    from an idle GPU: 5.46 ms packed at once, 5.36 never packed or packed after the first replay)."""
+    """A recorded layer's launches.  What a replay needs beyond them, which arguments are the layer's own tensors and the packed
+    list, is worked out at the first replay: a kind that no other layer of the step has costs nothing, and a step of small layers
+    (whose host time is what it takes) has no layer launched call by call (a portion of 1,024 tokens through twelve mixed layers
+    1,024 wide 3.30 -> 3.08 ms)."""
 
-    calls: list[tuple]          # (function, arguments, ((argument index, tensor key, byte offset), ...), status)
+    calls: list[tuple]          # (function, arguments, status)
     keep: list[torch.Tensor]
     result: object
+    tensors: dict[tuple, torch.Tensor] = field(repr=False)      # the recorded layer's own
+    patched: list[tuple] | None = field(default=None, repr=False)
     packed: PackedCalls | None = field(default=None, repr=False)
     pack_tried: bool = field(default=False, repr=False)
     # fields of the result that are tensors of the layer itself (a bias that its last product leaves to
     # the residual add): (field, tensor key); a replayed layer hands on its own
     result_own: tuple = ()
 
+    def _prepare(self) -> None:
+        self.patched = patched_calls(self.calls, self.tensors)
+        if not self.pack_tried:
+            self.pack_tried = True
+            packed = PackedCalls(self.patched)
+            self.packed = packed if packed.ok else None
+        result = self.result
+        if dataclasses.is_dataclass(result):
+            by_address = {(t.data_ptr(), tuple(t.shape)): key for key, t in self.tensors.items() if key[0] == "part" and t.numel()}
+            self.result_own = tuple((name, by_address[(t.data_ptr(), tuple(t.shape))]) for name, t in _fields(result)
+                                    if (t.data_ptr(), tuple(t.shape)) in by_address)
+
     def launch(self, tensors: dict[tuple, torch.Tensor], then):
+        if self.patched is None:
+            self._prepare()
         if self.packed is not None:
             self.packed.launch(tensors)         # the whole layer in one foreign call
         else:
             address = {key: t.data_ptr() for key, t in tensors.items()}     # once a layer, not once a patch
-            for fn, args, patches, status in self.calls:
+            for fn, args, patches, status in self.patched:
                 if patches:
                     args = list(args)
                     for index, key, offset in patches:
@@ -171,10 +201,6 @@ class LayerRecording:
                 got = fn(*args)
                 if got != status:
                     raise ops.KernelError(f"a replayed launch returned {got}, the recorded one {status}")
-            if not self.pack_tried:
-                self.pack_tried = True
-                packed = PackedCalls(self.calls)
-                self.packed = packed if packed.ok else None
         result = self.result
         if self.result_own:
             result = dataclasses.replace(result, **{name: tensors[key] for name, key in self.result_own})
@@ -189,23 +215,4 @@ def record(run, tensors: dict[tuple, torch.Tensor]):
     None if what ran cannot be replayed)."""
     with ops.recording() as recorder:
         result = run()
-    if not recorder.valid:
-        return result, None
-    spans = sorted((t.data_ptr(), t.data_ptr() + _span_bytes(t), key) for key, t in tensors.items() if t.numel())
-    starts = [s[0] for s in spans]
-    calls = []
-    for fn, args, status in recorder.calls:
-        patches = []
-        for index, arg in enumerate(args):
-            if not isinstance(arg, c_void_p) or not arg.value:
-                continue
-            at = bisect.bisect_right(starts, arg.value) - 1     # (the spans of different tensors do not overlap)
-            if at >= 0 and spans[at][0] <= arg.value < spans[at][1]:
-                patches.append((index, spans[at][2], arg.value - spans[at][0]))
-        calls.append((fn, args, tuple(patches), status))
-    result_own = ()
-    if dataclasses.is_dataclass(result):
-        by_address = {(t.data_ptr(), tuple(t.shape)): key for key, t in tensors.items() if key[0] == "part" and t.numel()}
-        result_own = tuple((name, by_address[(t.data_ptr(), tuple(t.shape))]) for name, t in _fields(result)
-                           if (t.data_ptr(), tuple(t.shape)) in by_address)
-    return result, LayerRecording(calls, recorder.keep, result, result_own=result_own)
+    return result, LayerRecording(recorder.calls, recorder.keep, result, tensors) if recorder.valid else None

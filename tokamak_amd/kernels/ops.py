@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import struct
 import threading
 from ctypes import c_float, c_int, c_long, c_size_t, c_void_p
 
@@ -80,20 +81,13 @@ def slots_of(fn, args: tuple) -> list[int] | None:
     """The arguments of a recorded call as 64-bit slots (csrc/slots.h): integers and
     addresses as they are (negative ones in two's complement), a float by its bits.  None if
     the entry point has no slot form."""
-    import struct
-
     if getattr(fn, "slots_address", None) is None or len(args) != len(fn.argtypes):
         return None
-    out = []
-    for kind, arg in zip(fn.argtypes, args):
-        value = getattr(arg, "value", arg)
+    values = [arg if arg.__class__ is int else getattr(arg, "value", arg) or 0 for arg in args]
+    for at, kind in enumerate(fn.argtypes):
         if kind is c_float:
-            out.append(struct.unpack("<I", struct.pack("<f", float(value)))[0])
-        elif kind is c_void_p:
-            out.append(int(value or 0))
-        else:
-            out.append(int(value) & 0xFFFFFFFFFFFFFFFF)
-    return out
+            values[at] = struct.unpack("<I", struct.pack("<f", values[at]))[0]
+    return [int(value) & 0xFFFFFFFFFFFFFFFF for value in values]
 
 
 _replay_fn = None
