@@ -1,8 +1,9 @@
 """y = x @ W^T for the projections of a step.
 
 float32: hand-written kernels with true 32-bit multiply-add and one summation order
-(tiled, or weight-streaming for up to 64 rows; row-wise deterministic, equal bits).  bfloat16: hand-written MFMA kernels for up to 64 rows, else
-the library product that torch binds (as the reference's nn.Linear does).
+(tiled, or weight-streaming for up to 64 rows; row-wise deterministic, equal bits).  bfloat16: hand-written MFMA kernels for up to 64 rows, up
+to 128 whose reader adds partial sums, for gated products of any number and long ones of up to 1,100 or 1,700; else the library
+product (as the reference's nn.Linear does).
 
 Decode steps of few rows (bfloat16, up to 16) can do without the kernels between the
 products: a part's last product adds its result into the float32 residual stream itself
