@@ -60,6 +60,7 @@ def test_gates(tile, m, n, k):
     g, u = sums[:, :n], sums[:, n:]
     xs, ws = inside(x)[1], inside(w)[1]
     for gate, limit, want in (("silu", None, g * torch.sigmoid(g) * u),
+                              ("gelu_tanh", None, g * torch.sigmoid(2 * (2 / torch.pi) ** 0.5 * (g + 0.044715 * g ** 3)) * u),
                               ("clamped", 2.5, g.clamp(max=2.5) * torch.sigmoid(1.702 * g.clamp(max=2.5)) * (u.clamp(-2.5, 2.5) + 1))):
         wide, out = inside(torch.zeros(m, n, dtype=torch.bfloat16))
         ops.gemm_many(xs, ws, out, rows=rows, columns=columns, gate=gate, limit=limit)

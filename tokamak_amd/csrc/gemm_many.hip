@@ -37,7 +37,7 @@ union Frag8 {
 
 #define TK_LDS __attribute__((address_space(3)))
 
-enum { EPI_PARTS, EPI_SILU, EPI_CLAMPED };     // the last two: gated
+enum { EPI_PARTS, EPI_SILU, EPI_CLAMPED, EPI_GELU };     // the last three: gated
 
 constexpr int kCus = 256;       // blocks that run at once
 constexpr int kXcds = 8;        // dies, each with an L2 of its own; blocks go to them in turn
@@ -55,6 +55,8 @@ struct Job {
 template <int EPI>
 __device__ __forceinline__ float gated(float z, float u, float limit) {
   if (EPI == EPI_SILU) return z / (1.f + __expf(-z)) * u;
+  // (half of z (1 + tanh y) is z / (1 + exp(-2 y)))
+  if (EPI == EPI_GELU) return z / (1.f + __expf(-1.5957691216057308f * (z + 0.044715f * z * z * z))) * u;
   const float g = fminf(z, limit);
   return g / (1.f + __expf(-1.702f * g)) * (fminf(fmaxf(u, -limit), limit) + 1.f);
 }
@@ -288,15 +290,15 @@ int launch(Job job, hipStream_t stream) {
 
 }  // namespace
 
-// mode 0: C float32 [parts][M, N], part_stride elements apart: the sums over `parts` shares of K; modes 1 and 2: W = [W_gate;
-// W_up] of 2 N rows and C[M, N] bfloat16 = act(A W_gate^T) * (A W_up^T), act silu or (2) the gate whose halves are clamped at
-// `limit`.  rows, columns: a tile's rows of A and of W (256 x 256, 128 x 256, 256 x 128, 128 x 128).  K a multiple of 64, N of 8;
+// mode 0: C float32 [parts][M, N], part_stride elements apart: the sums over `parts` shares of K; modes 1 to 3: W = [W_gate;
+// W_up] of 2 N rows and C[M, N] bfloat16 = act(A W_gate^T) * (A W_up^T), act silu, (2) the gate whose halves are clamped at
+// `limit` or (3) the tanh form of gelu.  rows, columns: a tile's rows of A and of W (256 x 256, 128 x 256, 256 x 128, 128 x 128).  K a multiple of 64, N of 8;
 // rows of all operands 16-byte aligned.
 TK_API int tk_gemm_many(int mode, const void* A, const void* W, void* C, int M, int N, int K, long lda, long ldw, long ldc,
                         int parts, long part_stride, float limit, int rows, int columns, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   const bool gate = mode >= EPI_SILU;
-  if (mode < 0 || mode > EPI_CLAMPED) return -1;
+  if (mode < 0 || mode > EPI_GELU) return -1;
   if (K < kStep || K % kStep != 0 || N % 8 != 0 || lda % 8 != 0 || ldw % 8 != 0 || ldc % 8 != 0 || part_stride % 4 != 0) return -1;
   if (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15) return -1;
   if (parts < 1 || parts > K / kStep || (mode != EPI_PARTS && parts != 1)) return -1;
@@ -307,6 +309,7 @@ TK_API int tk_gemm_many(int mode, const void* A, const void* W, void* C, int M, 
   if (rows == 64 * MT_ && columns == 64 * NT_) {                                       \
     if (mode == EPI_PARTS) return launch<MT_, NT_, EPI_PARTS>(job, stream);            \
     if (mode == EPI_SILU) return launch<MT_, NT_, EPI_SILU>(job, stream);              \
+    if (mode == EPI_GELU) return launch<MT_, NT_, EPI_GELU>(job, stream);              \
     return launch<MT_, NT_, EPI_CLAMPED>(job, stream);                                 \
   }
   TK_SHAPE(4, 4)

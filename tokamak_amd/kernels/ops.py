@@ -2181,13 +2181,13 @@ def many_split_plan(m: int, n: int, k: int) -> tuple[int, int, int]:
     return min(plans)[1:]
 
 
-MANY_MODES = {None: 0, "silu": 1, "clamped": 2}      # of tk_gemm_many, by the gate's activation
+MANY_MODES = {None: 0, "silu": 1, "clamped": 2, "gelu_tanh": 3}      # of tk_gemm_many, by the gate's activation
 
 
 def gemm_many(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, rows: int, columns: int, gate: str | None = None,
               limit: float | None = None) -> None:
     """Products of many rows in tiles of ``rows`` by ``columns`` (256 x 256, 128 x 256, 256 x 128, 128 x 128): out [P, M, N] float32,
-    the sums of a[M, K] @ w[N, K]^T over P shares of K; or with a ``gate`` ("silu", or "clamped" with its ``limit``) w = [gate; up]
+    the sums of a[M, K] @ w[N, K]^T over P shares of K; or with a ``gate`` ("silu", "gelu_tanh", or "clamped" with its ``limit``) w = [gate; up]
     and out[M, N] bfloat16 = act(a @ gate^T) * (a @ up^T), see ``silu_mul``."""
     for t in (a, w, out):
         _need(t.is_cuda and t.stride(-1) == 1, "gemm operands are GPU tensors with unit inner stride")
@@ -2200,7 +2200,7 @@ def gemm_many(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, rows: int,
     _need(a.dim() == w.dim() == 2 and w.shape == (n * (1 if split else 2), k) and out.shape[-2] == m, "gemm shapes disagree")
     _need(gemm_many_fits(a, w, n) and out.data_ptr() % 16 == 0 and out.stride(-2) % 8 == 0 and 1 <= parts <= k // 64,
           "products of many rows take whole steps of 64 k and rows on 16-byte borders")
-    _need(gate in MANY_MODES and (gate == "clamped") == (limit is not None), "the gate is silu, or clamped with its limit")
+    _need(gate in MANY_MODES and (gate == "clamped") == (limit is not None), "the gate is silu, gelu_tanh, or clamped with its limit")
     _note(f"{m}x{w.shape[0]}x{k}", (w.shape[0] * k + m * k) * 2 + out.numel() * out.element_size(), 2.0 * m * w.shape[0] * k)
     _check(_fn("gemm_many", "tk_gemm_many")(
         MANY_MODES[gate], _p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(-2), parts,
