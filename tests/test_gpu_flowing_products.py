@@ -85,3 +85,21 @@ def test_every_route_gives_the_product(m, n, k):
     # (some routes round gate and up to bfloat16 first: 2^-9 of each, the gate's of its argument)
     slack = (2.0 ** -7 + 2.0 ** -9 * exact[:, :half].abs().double()) * want.abs() + 1e-30
     assert ((gate.double() - want).abs() <= slack).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [3, 16, 17, 64])
+def test_rows_that_overlap_have_their_product(m):
+    """One row of activations for all, and windows of one: rows closer together than they are long."""
+    k, n = 256, 1040
+    line, w = whole(1, k + 8 * m, 2, 9).to(DEV), whole(n, k, 2, 10).to(DEV)
+    for x in (line[:, :k].expand(m, k), line.as_strided((m, k), (8, 1))):
+        exact = x.float() @ w.float().T
+        assert torch.equal(linear.linear(x, w), exact.to(torch.bfloat16))
+        parts = linear.linear(x, w, allow_partials=True)
+        assert torch.equal(parts.float().sum(0) if parts.dim() == 3 else parts, exact if parts.dim() == 3 else exact.to(torch.bfloat16))
+        assert torch.equal(linear.activated_linear(x, w), (exact.clamp(min=0) ** 2).to(torch.bfloat16))
+        g, u = exact[:, :n // 2].double(), exact[:, n // 2:].double()
+        want = torch.nn.functional.silu(g) * u
+        # (some routes round gate and up to bfloat16 first: 2^-9 of each, the gate's of its argument)
+        assert ((linear.gated_linear(x, w).double() - want).abs() <= (2.0 ** -7 + 2.0 ** -9 * g.abs()) * want.abs() + 1e-30).all()

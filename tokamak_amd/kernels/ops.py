@@ -2129,9 +2129,11 @@ def flow_parts(m: int, n: int, k: int) -> int:
 
 
 def gemm_flow_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ``gemm_flow`` takes these operands: bfloat16 rows on 16-byte borders, up to 128 of them, whole steps of 128 k."""
+    """Whether ``gemm_flow`` takes these operands: bfloat16 rows on 16-byte borders that do not overlap, up to 128 of them, whole
+    steps of 128 k."""
     return (a.dtype == w.dtype == torch.bfloat16 and a.dim() == w.dim() == 2 and a.stride(1) == w.stride(1) == 1
             and 0 < a.shape[0] <= FLOW_MAX_ROWS and a.shape[1] >= 128 and a.shape[1] % 128 == 0
+            and a.stride(0) >= a.shape[1] and w.stride(0) >= w.shape[1]
             and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and a.stride(0) <= MANY_MAX_STRIDE and w.stride(0) * (w.shape[0] + 128) < 1 << 31)
 
@@ -2140,9 +2142,11 @@ MANY_MAX_STRIDE = 1 << 22      # (offsets within a tile's rows are 32 bits)
 
 
 def gemm_many_fits(a: torch.Tensor, w: torch.Tensor, n: int) -> bool:
-    """Whether ``gemm_many`` takes these operands for ``n`` output channels: bfloat16 rows on 16-byte borders, whole steps of 64 k."""
+    """Whether ``gemm_many`` takes these operands for ``n`` output channels: bfloat16 rows on 16-byte borders that do not overlap,
+    whole steps of 64 k."""
     return (a.dtype == w.dtype == torch.bfloat16 and a.dim() == w.dim() == 2 and a.stride(1) == w.stride(1) == 1
             and a.shape[1] >= 64 and a.shape[1] % 64 == 0 and n >= 8 and n % 8 == 0
+            and a.stride(0) >= a.shape[1] and w.stride(0) >= w.shape[1]
             and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and a.stride(0) <= MANY_MAX_STRIDE and w.stride(0) * (w.shape[0] + 256) < 1 << 31)
 
