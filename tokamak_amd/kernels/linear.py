@@ -273,7 +273,7 @@ def gated_linear(x: torch.Tensor | DeferredNorm, gate_up: torch.Tensor, activati
             return out
         x = x.materialize()
     out = torch.empty((m, inter), dtype=x.dtype, device=x.device)
-    if m == 0 or _gated_flow(x, gate_up, out, activation, limit):
+    if m == 0 or _gated_flow(x, gate_up, out, activation, None):      # (silu has no limit, one that is given is not looked at)
         return out
     if x.dtype == torch.bfloat16 and m <= 64:
         from tokamak_amd.kernels import gemm_bf16
@@ -284,6 +284,6 @@ def gated_linear(x: torch.Tensor | DeferredNorm, gate_up: torch.Tensor, activati
             elif small or ops.direct_pays("gated", m, inter, x.shape[1]) or not _gated_split(x, gate_up, out, activation, limit):
                 ops.gemm_stream_swiglu(x, gate_up, out)
             return out
-    if not _gated_many(x, gate_up, out, activation, limit):
+    if not _gated_many(x, gate_up, out, activation, None):
         ops.silu_mul(linear(x, gate_up), out)
     return out
