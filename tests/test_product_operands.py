@@ -3,7 +3,7 @@
 import pytest
 import torch
 
-from tokamak_amd.kernels import linear, ops
+from tokamak_amd.kernels import gemm_bf16, linear, ops
 
 
 def rows(n, k, stride):
@@ -29,3 +29,22 @@ def test_a_limit_beside_the_silu_gate_is_not_looked_at(monkeypatch, m):
     x, w = (torch.zeros(r, 256, dtype=torch.bfloat16) for r in (m, 2048))
     assert linear.gated_linear(x, w, "silu", 7.0).shape == (m, 1024)
     assert given == [("silu", None)]
+
+
+# (rows, weight rows, k, us by the forms for few rows, us by the flowing one), plain products into bfloat16
+WHOLE = [(17, 64, 4096, 11.1, 14.9), (32, 64, 4096, 14.1, 16.0), (33, 64, 4096, 21.8, 16.7), (64, 64, 4096, 27.7, 19.5),
+         (17, 768, 2048, 7.2, 8.5), (33, 768, 2048, 13.9, 9.5), (17, 1024, 2048, 13.1, 8.5), (17, 12800, 4096, 30.9, 27.5),
+         (64, 12800, 4096, 48.3, 31.4), (17, 16384, 5120, 39.5, 30.7), (32, 16384, 4096, 30.4, 34.7), (33, 16384, 4096, 40.3, 35.0),
+         (64, 16384, 1024, 13.1, 9.7), (33, 16448, 2560, 26.1, 29.5), (64, 20480, 4096, 41.0, 55.0), (17, 20480, 5120, 48.9, 45.3),
+         (32, 32768, 4096, 45.8, 62.3)]
+
+
+@pytest.mark.parametrize("m, n, k, few, flow", WHOLE)
+def test_a_product_in_one_share_flows_where_it_was_faster(m, n, k, few, flow):
+    assert gemm_bf16.flows_whole(m, n, k) == (flow < few)
+
+
+@pytest.mark.parametrize("m, n, taken", [(16, 1024, False), (17, 1016, False), (17, 1024, True), (32, 8, False), (33, 8, True), (64, 8, True), (65, 1024, False)])
+def test_narrow_products_flow_from_33_rows(m, n, taken):
+    x, w = (torch.zeros(r, 128, dtype=torch.bfloat16) for r in (m, n))
+    assert gemm_bf16.flows(x, w, False) is taken and gemm_bf16.flows(x, w, True) is (m <= 96)

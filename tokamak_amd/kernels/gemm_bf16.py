@@ -92,15 +92,31 @@ FLOW_SPLIT_ROWS = (3, 96)           # rows between which a product whose reader 
                                     # 1.13 to 1.15 at 17 to 64, 1.31 to 1.34 at 65 to 96; at 128 level, 0.81 at worst.  With fewer rows it is
                                     # 1.06 times as fast alone, but beside an experts' branch its few large blocks wait for room (a
                                     # decode step of one request 623 -> 663 us, of two 731 -> 735)
-FLOW_ROWS = (17, 64)                # ... and one into bfloat16: 1.2 to 1.6 times; with fewer rows the direct form, with more
-                                    # the library is ahead of blocks that cannot share K.  (A logits head into float32, one share
+FLOW_ROWS = (17, 64)                # ... and one into bfloat16, which nobody can add, in one share of K, where ``flows_whole`` says; with fewer rows
+                                    # the direct form, with more the library is ahead of it.  (A logits head into float32, one share
                                     # of K: decode steps of 36 to 64 rows 7 to 53 us slower than with the streaming kernel.)
+FLOW_WHOLE_MOST = 16384             # weight rows of a product in one share from 33 rows on: 256 blocks, of which a CU holds one
+
+
+def flows_whole(m: int, n: int, stride: int) -> bool:
+    """Whether a product of 17 to 64 rows in one share of K flows, by its weight rows and the numbers between them.  A block owns 64
+    of them and walks all of K.  Beside the forms below (110 sizes of 64 to 65,536 rows of 1,024 to 17,408, weights from memory):
+
+    - 33 to 64 rows: 1.15 to 2.07 times as fast up to 16,384 weight rows (64 x 4,096 at 64 rows 28 -> 20 us); beyond, where a second
+      round of blocks begins, 0.71 to 1.05 (at 28,672, whose rounds are even, 1.13 to 1.52).
+    - 17 to 32 rows: below 1,024 weight rows 0.67 to 1.00 but for one size (64 x 4,096 at 17 rows 11 -> 15 us): a few blocks, where
+      gemm_skinny shares K among sixteen waves of four times as many.  From there on 1.00 to 1.63, beyond 16,384 0.94 to 1.15;
+      but 0.73 to 0.93 from 16,384 weight rows on if they lie a multiple of 8 KB apart (16,384 x 4,096 reaches 3.8 TB/s, x 5,120 5.5)."""
+    if m > 32:
+        return n <= FLOW_WHOLE_MOST
+    return n >= STREAM_MIN_ROWS_OUT and (n <= 14336 or stride % 4096 != 0)
 
 
 def flows(x: torch.Tensor, weight: torch.Tensor, allow_partials: bool) -> bool:
     """Whether a product goes to the flowing kernel: into partial sums, or into bfloat16."""
     low, high = FLOW_SPLIT_ROWS if allow_partials else FLOW_ROWS
-    return low <= x.shape[0] <= high and ops.gemm_flow_fits(x, weight)
+    return (low <= x.shape[0] <= high and (allow_partials or flows_whole(x.shape[0], weight.shape[0], weight.stride(0)))
+            and ops.gemm_flow_fits(x, weight))
 
 
 def flow(x: torch.Tensor, weight: torch.Tensor, allow_partials: bool) -> torch.Tensor:
