@@ -103,3 +103,13 @@ def test_rows_that_overlap_have_their_product(m):
         want = torch.nn.functional.silu(g) * u
         # (some routes round gate and up to bfloat16 first: 2^-9 of each, the gate's of its argument)
         assert ((linear.gated_linear(x, w).double() - want).abs() <= (2.0 ** -7 + 2.0 ** -9 * g.abs()) * want.abs() + 1e-30).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [16, 17, 32, 33, 64, 65])
+@pytest.mark.parametrize("n, k", [(40, 256), (1040, 256), (520, 4096), (16392, 128)])
+def test_squared_relu_by_every_route(m, n, k):
+    """In the epilogue of each product and behind shares of K.  Sums and their squares are exact in float32."""
+    x, w = whole(m, k, 1, 11).to(DEV), whole(n, k, 1, 12).to(DEV)
+    exact = (x.double() @ w.double().T).clamp(min=0) ** 2
+    assert torch.equal(linear.activated_linear(x, w), exact.to(torch.bfloat16))

@@ -48,3 +48,26 @@ def test_a_product_in_one_share_flows_where_it_was_faster(m, n, k, few, flow):
 def test_narrow_products_flow_from_33_rows(m, n, taken):
     x, w = (torch.zeros(r, 128, dtype=torch.bfloat16) for r in (m, n))
     assert gemm_bf16.flows(x, w, False) is taken and gemm_bf16.flows(x, w, True) is (m <= 96)
+
+
+# (rows, weight rows, k, us of the flowing product with the activation in its epilogue, us in shares of K with the activation's kernel)
+SHARES = [(17, 256, 1024, 5.6, 5.5), (17, 8192, 1024, 6.4, 7.5), (64, 8192, 1024, 8.1, 11.0), (17, 4096, 2048, 9.0, 7.9),
+          (64, 12800, 2048, 15.3, 19.3), (32, 4096, 4096, 17.7, 11.1), (33, 8192, 4096, 22.5, 17.9), (64, 12800, 4096, 31.5, 35.3),
+          (17, 64, 8192, 29.4, 8.9), (48, 4096, 17408, 75.7, 30.6)]
+
+
+@pytest.mark.parametrize("m, n, k, whole, shares", SHARES)
+def test_k_is_shared_ahead_of_an_activation_where_that_was_faster(m, n, k, whole, shares):
+    assert ops.flow_shares_pay(m, n, k) == (shares < whole)
+
+
+@pytest.mark.parametrize("m, n, k, forms", [(17, 1024, 256, ["flow"]), (32, 8, 256, ["flow"]), (64, 8, 256, ["flow"]), (17, 512, 4096, ["shares", "relu"]),
+                                            (33, 16384, 256, ["flow"]), (33, 16392, 256, ["stream"]), (65, 512, 4096, ["shares", "relu"])])
+def test_squared_relus_form(monkeypatch, m, n, k, forms):
+    """In the flowing product's epilogue, behind shares of K, or in the streaming product's, on both sides of each line."""
+    seen = []
+    monkeypatch.setattr(ops, "gemm_flow", lambda x, w, out, **kwargs: seen.append("shares" if out.dim() == 3 else "flow"))
+    monkeypatch.setattr(ops, "gemm_stream", lambda *args, **kwargs: seen.append("stream"))
+    monkeypatch.setattr(ops, "squared_relu", lambda *args: seen.append("relu"))
+    linear.activated_linear(torch.zeros(m, k, dtype=torch.bfloat16), torch.zeros(n, k, dtype=torch.bfloat16))
+    assert seen == forms

@@ -161,9 +161,9 @@ ACTIVATED_SPLIT_FROM = 3    # shares of K that the product would be cut in from 
 def activated_linear(x: torch.Tensor, weight: torch.Tensor, activation: str = "squared_relu") -> torch.Tensor:
     """act(x @ weight^T) -> [M, N]; ``activation`` "squared_relu": max(z, 0)^2.
 
-    bfloat16 with up to 64 rows and enough weight rows to fill the GPU unsplit: in the streaming product's
-    epilogue.  Otherwise the product (in partial sums where that pays), then the activation's kernel, which adds
-    partial sums before it."""
+    bfloat16: in the epilogue of the direct product (up to 16 rows), of the flowing one (17 to 64 rows, K a multiple of
+    128) or of the streaming one (up to 64 rows), where K need not be shared to fill the GPU.  Otherwise the product (in
+    partial sums where that pays), then the activation's kernel, which adds partial sums before it."""
     from tokamak_amd.kernels import gemm_bf16
 
     if activation != "squared_relu":
@@ -172,11 +172,15 @@ def activated_linear(x: torch.Tensor, weight: torch.Tensor, activation: str = "s
     out = torch.empty((m, n), dtype=x.dtype, device=x.device)
     if m == 0:
         return out
+    # Beside the streaming forms, 284 sizes: 1.01 to 1.70 times as fast (4,096 x 4,096 at 32 rows 13.9 -> 11.1 us, 512 x 17,408 19.7 ->
+    # 14.2; always in one share of K 0.21 to 1.70, those two 17.7 and 73).  Narrow ones too: here their other form is two kernels as well.
+    flowing = (gemm_bf16.FLOW_ROWS[0] <= m <= gemm_bf16.FLOW_ROWS[1] and ops.gemm_flow_fits(x, weight)
+               and gemm_bf16.flows_whole(m, max(n, gemm_bf16.STREAM_MIN_ROWS_OUT), weight.stride(0)))
     if _few_rows_fit(m, x, weight, ops.DIRECT_MAX_ROWS) and ops.direct_pays("activated", m, n, k):
         ops.gemm_direct(x, weight, out, activation=activation)
-    elif gemm_bf16.flows(x, weight, False):
+    elif flowing and not ops.flow_shares_pay(m, n, k):
         ops.gemm_flow(x, weight, out, activation=activation)
-    elif (x.dtype == torch.bfloat16 and m <= gemm_bf16.SKINNY_MAX_ROWS and n >= gemm_bf16.STREAM_MIN_ROWS_OUT
+    elif (not flowing and x.dtype == torch.bfloat16 and m <= gemm_bf16.SKINNY_MAX_ROWS and n >= gemm_bf16.STREAM_MIN_ROWS_OUT
             and gemm_bf16.skinny_fits(x, weight) and gemm_bf16.stream_splits(n, k, m) < ACTIVATED_SPLIT_FROM):
         ops.gemm_stream(x, weight, out, activation=activation)
     else:

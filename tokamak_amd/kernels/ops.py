@@ -2104,11 +2104,10 @@ FLOW_PARTS = (1, 2, 3, 4, 5, 6, 8, 10, 12, 16)
 FLOW_STEP, FLOW_COLUMNS = 128, 64       # k of a step, weight rows a block (csrc/gemm_flow.hip)
 
 
-@functools.lru_cache(maxsize=8192)
-def flow_parts(m: int, n: int, k: int) -> int:
-    """Shares of K of a flowing product whose reader adds partial sums.  A step of a block is its bytes at the rate of its CU,
-    whose blocks share it, and all blocks' weights at the GPU's; K is cut where more blocks carry more bytes at once,
-    which the sums' bytes then have to pay for."""
+def _flow_price(m: int, n: int, k: int, parts: int) -> float:
+    """What a flowing product into sums costs with their reader: a step of a block is its bytes at the rate of its CU, whose
+    blocks share it, and all blocks' weights at the GPU's; K is cut where more blocks carry more bytes at once, which
+    the sums' bytes then have to pay for."""
     blocks, steps = -(-n // FLOW_COLUMNS), k // FLOW_STEP
     weights, rows = FLOW_COLUMNS * FLOW_STEP * 2, -(-m // 16) * 16 * FLOW_STEP * 2
     at_once = 256 * (160 * 1024 // (3 * (weights + rows)))
@@ -2116,16 +2115,31 @@ def flow_parts(m: int, n: int, k: int) -> int:
     def step(count: int) -> float:
         return ((-(-count // 256) * (weights + rows) / FLOW_CU_RATE) ** 3 + (count * weights / FLOW_RATE) ** 3) ** (1 / 3)
 
-    best = None
-    for parts in FLOW_PARTS:
-        if parts > max(1, steps // 2):
-            break
-        rounds, rest = divmod(blocks * parts, at_once)
-        price = FLOW_START + -(-steps // parts) * (rounds * step(at_once) + (step(rest) if rest else 0.0))
-        price += 4 * parts * m * n * ((FLOW_WRITE if parts > 1 else 0.0) + FLOW_READ)
-        if best is None or price < best[0]:
-            best = (price, parts)
-    return best[1]
+    rounds, rest = divmod(blocks * parts, at_once)
+    price = FLOW_START + -(-steps // parts) * (rounds * step(at_once) + (step(rest) if rest else 0.0))
+    return price + 4 * parts * m * n * ((FLOW_WRITE if parts > 1 else 0.0) + FLOW_READ)
+
+
+@functools.lru_cache(maxsize=8192)
+def flow_parts(m: int, n: int, k: int) -> int:
+    """Shares of K of a flowing product whose reader adds partial sums."""
+    return min((parts for parts in FLOW_PARTS if parts == 1 or parts <= k // FLOW_STEP // 2),
+               key=lambda parts: _flow_price(m, n, k, parts))
+
+
+# Microseconds of a kernel behind a flowing product that adds its shares and applies an activation or a gate to ``n`` sums a row: with it,
+# the cheaper of that and the same in the epilogue of one share is picked within 1 % on average and 9 % at worst (630 products
+# of 17 to 96 rows, 64 to 17,408 weight rows of 1,024 to 17,408, squared relu and silu gates; 0 us: 24 to 31 % at worst, 4 us: 12 to 14).
+FLOW_BEHIND = 2.5
+
+
+@functools.lru_cache(maxsize=8192)
+def flow_shares_pay(m: int, n: int, k: int) -> bool:
+    """Whether a flowing product with an activation or a gate behind it is cheaper in shares of K, which a kernel adds before
+    it, than in one, whose epilogue has it: one share of 4,096 x 4,096 at 32 rows, squared relu, takes 17.8 us, four and the kernel 11.2."""
+    whole = _flow_price(m, n, k, 1) - 4 * m * n * FLOW_READ
+    parts = flow_parts(m, n, k)
+    return parts > 1 and _flow_price(m, n, k, parts) + FLOW_BEHIND < whole
 
 
 def gemm_flow_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
