@@ -71,3 +71,20 @@ def test_squared_relus_form(monkeypatch, m, n, k, forms):
     monkeypatch.setattr(ops, "squared_relu", lambda *args: seen.append("relu"))
     linear.activated_linear(torch.zeros(m, k, dtype=torch.bfloat16), torch.zeros(n, k, dtype=torch.bfloat16))
     assert seen == forms
+
+
+# rows, channels, k of a product whose reader adds shares of K, and the microseconds of both by the number of shares
+PARTS = [(3, 5120, 8192, {1: 32.7, 2: 22.6, 3: 20.3, 4: 24.3, 5: 21.6, 6: 22.0, 8: 25.1, 10: 24.7, 12: 23.8, 16: 26.3}),
+         (4, 3072, 4096, {1: 19.6, 2: 13.4, 3: 11.6, 4: 10.3, 5: 10.4, 6: 12.1, 8: 11.3, 10: 11.9, 12: 12.1, 16: 12.6}),
+         (3, 6144, 2048, {1: 13.3, 2: 10.8, 3: 12.8, 4: 11.7, 5: 11.8, 6: 12.8, 8: 12.9}),
+         (3, 12288, 1024, {1: 11.7, 2: 12.6, 3: 13.8, 4: 13.4}),
+         (8, 4096, 4096, {1: 18.8, 2: 13.2, 3: 11.7, 4: 11.3, 5: 12.7, 6: 12.4, 8: 12.2, 10: 13.9, 12: 14.1, 16: 14.8}),
+         (16, 1024, 3072, {1: 16.4, 2: 11.2, 3: 9.6, 4: 8.3, 5: 8.1, 6: 8.0, 8: 7.2, 10: 7.8, 12: 7.2}),
+         (24, 2560, 9728, {1: 44.6, 2: 27.0, 3: 21.6, 4: 18.1, 5: 17.0, 6: 16.3, 8: 20.1, 10: 19.1, 12: 18.4, 16: 20.3}),
+         (64, 4096, 12288, {1: 68.2, 2: 40.8, 3: 32.5, 4: 28.9, 5: 39.2, 6: 36.3, 8: 34.0, 10: 38.9, 12: 37.9, 16: 41.0}),
+         (96, 5120, 17408, {1: 119.7, 2: 69.1, 3: 54.1, 4: 72.1, 5: 63.7, 6: 59.6, 8: 65.2, 10: 73.0, 12: 67.8, 16: 70.0})]
+
+
+@pytest.mark.parametrize("m, n, k, took", PARTS)
+def test_shares_of_k_are_near_the_best_measured(m, n, k, took):
+    assert took[ops.flow_parts(m, n, k)] <= 1.09 * min(took.values())

@@ -2096,10 +2096,11 @@ def gemm_flow(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, gate: str 
 
 
 # What a flowing product is priced with: its start (microseconds), the rates of a CU and of the GPU (bytes a microsecond), a float32
-# sum written and read (microseconds a byte).  Fitted to 1,650 measured products (1 to 128 rows, 384 to 12,800 channels of
-# 384 to 17,408, weights from memory) within 6 % each; the number of shares so chosen is 0.4 % behind the best one measured on
-# average, at worst 13 % (128 rows).
-FLOW_START, FLOW_CU_RATE, FLOW_RATE, FLOW_WRITE, FLOW_READ = 2.47, 44.8e3, 6.91e6, 0.536e-6, 0.222e-6
+# sum written and read (microseconds a byte), what each further round of blocks costs to begin.  Fitted to 1,650 measured products (1 to
+# 128 rows, 384 to 12,800 channels of 384 to 17,408, weights from memory) within 6 % each; over 984 (3 to 96 rows, 1,024 to 12,288
+# channels of 512 to 17,408) the number of shares so chosen is 0.5 % behind the best one measured on average, at worst 8 %
+# (30 % if further rounds cost nothing: 5,120 x 8,192 at 3 rows, 24 us in 16 shares).
+FLOW_START, FLOW_CU_RATE, FLOW_RATE, FLOW_WRITE, FLOW_READ, FLOW_ROUND = 2.47, 44.8e3, 6.91e6, 0.536e-6, 0.222e-6, 1.0
 FLOW_PARTS = (1, 2, 3, 4, 5, 6, 8, 10, 12, 16)
 FLOW_STEP, FLOW_COLUMNS = 128, 64       # k of a step, weight rows a block (csrc/gemm_flow.hip)
 
@@ -2116,7 +2117,7 @@ def _flow_price(m: int, n: int, k: int, parts: int) -> float:
         return ((-(-count // 256) * (weights + rows) / FLOW_CU_RATE) ** 3 + (count * weights / FLOW_RATE) ** 3) ** (1 / 3)
 
     rounds, rest = divmod(blocks * parts, at_once)
-    price = FLOW_START + -(-steps // parts) * (rounds * step(at_once) + (step(rest) if rest else 0.0))
+    price = FLOW_START + (rounds - (not rest)) * FLOW_ROUND + -(-steps // parts) * (rounds * step(at_once) + (step(rest) if rest else 0.0))
     return price + 4 * parts * m * n * ((FLOW_WRITE if parts > 1 else 0.0) + FLOW_READ)
 
 
