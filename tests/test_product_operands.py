@@ -88,3 +88,9 @@ PARTS = [(3, 5120, 8192, {1: 32.7, 2: 22.6, 3: 20.3, 4: 24.3, 5: 21.6, 6: 22.0, 
 @pytest.mark.parametrize("m, n, k, took", PARTS)
 def test_shares_of_k_are_near_the_best_measured(m, n, k, took):
     assert took[ops.flow_parts(m, n, k)] <= 1.09 * min(took.values())
+
+
+@pytest.mark.parametrize("m, n, k, taken", [(3, 1024, 512, False), (4, 1024, 512, False), (5, 1024, 512, True), (2, 4096, 4096, False), (3, 4096, 4096, True)])
+def test_small_matrices_of_three_and_four_rows_stay_with_the_direct_product(m, n, k, taken):
+    x, w = (torch.zeros(r, k, dtype=torch.bfloat16) for r in (m, n))
+    assert gemm_bf16.flows(x, w, True) is taken

@@ -88,10 +88,12 @@ STREAM_PARTIALS_BIG = 64 << 20      # ... and the bytes of a matrix from which i
 
 
 FLOW_SPLIT_ROWS = (3, 96)           # rows between which a product whose reader adds partial sums flows (csrc/gemm_flow.hip): beside the forms
-                                    # below, 20 sizes, weights from memory: 1.06 to 1.08 times as fast at 3 to 8 rows, 1.10 at 16,
-                                    # 1.13 to 1.15 at 17 to 64, 1.31 to 1.34 at 65 to 96; at 128 level, 0.81 at worst.  With fewer rows it is
+                                    # below, 123 sizes of 1,024 to 12,288 channels, weights from memory, reader included: 1.09 times as fast at 3 to
+                                    # 8 rows, 1.11 at 16, 1.15 at 24 to 64, 1.24 at 96, at worst 0.94 (12,288 x 4,096 at 48); 128 rows: level, 0.81 at worst.  With fewer rows it is
                                     # 1.06 times as fast alone, but beside an experts' branch its few large blocks wait for room (a
                                     # decode step of one request 623 -> 663 us, of two 731 -> 735)
+FLOW_BEHIND_DIRECT_ROWS = 4         # rows up to which the direct product, where it pays (ops.direct_pays: K of up to 1,024), is ahead of it in
+                                    # turn: 60 products 0.84 to 1.02 (1,024 x 512 at 4 rows, reader included, 5.2 us against 5.9); with 5 rows 1.01 to 1.09
 FLOW_ROWS = (17, 64)                # ... and one into bfloat16, which nobody can add, in one share of K, where ``flows_whole`` says; with fewer rows
                                     # the direct form, with more the library is ahead of it.  (A logits head into float32, one share
                                     # of K: decode steps of 36 to 64 rows 7 to 53 us slower than with the streaming kernel.)
@@ -114,9 +116,14 @@ def flows_whole(m: int, n: int, stride: int) -> bool:
 
 def flows(x: torch.Tensor, weight: torch.Tensor, allow_partials: bool) -> bool:
     """Whether a product goes to the flowing kernel: into partial sums, or into bfloat16."""
-    low, high = FLOW_SPLIT_ROWS if allow_partials else FLOW_ROWS
-    return (low <= x.shape[0] <= high and (allow_partials or flows_whole(x.shape[0], weight.shape[0], weight.stride(0)))
-            and ops.gemm_flow_fits(x, weight))
+    m, n = x.shape[0], weight.shape[0]
+    if allow_partials:
+        low, high = FLOW_SPLIT_ROWS
+        taken = low <= m <= high and not (m <= FLOW_BEHIND_DIRECT_ROWS and ops.direct_pays("parts", m, n, weight.shape[1]))
+    else:
+        low, high = FLOW_ROWS
+        taken = low <= m <= high and flows_whole(m, n, weight.stride(0))
+    return taken and ops.gemm_flow_fits(x, weight)
 
 
 def flow(x: torch.Tensor, weight: torch.Tensor, allow_partials: bool) -> torch.Tensor:
