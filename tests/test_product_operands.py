@@ -94,3 +94,17 @@ def test_shares_of_k_are_near_the_best_measured(m, n, k, took):
 def test_small_matrices_of_three_and_four_rows_stay_with_the_direct_product(m, n, k, taken):
     x, w = (torch.zeros(r, k, dtype=torch.bfloat16) for r in (m, n))
     assert gemm_bf16.flows(x, w, True) is taken
+
+
+@pytest.mark.parametrize("m, n, k, forms", [
+    (16, 1024, 4096, []), (17, 1024, 4096, ["shares", "gate"]), (17, 1024, 128, ["flow"]), (64, 6144, 1024, ["flow"]), (17, 1028, 4096, ["flow"]),
+    (65, 1028, 4096, []), (65, 1032, 4096, ["shares", "gate"]), (96, 1024, 4096, ["shares", "gate"]), (97, 1024, 4096, []),
+    (32, 16400, 128, ["flow"]), (33, 16384, 128, ["flow"]), (33, 16400, 128, []), (64, 16400, 128, []), (65, 16400, 128, ["flow"])])
+def test_gated_products_of_few_rows(monkeypatch, m, n, k, forms):
+    """One share of K, several with the gate's kernel, or other forms, on both sides of each line."""
+    seen = []
+    monkeypatch.setattr(ops, "gemm_flow", lambda x, w, out, **kwargs: seen.append("shares" if out.dim() == 3 else "flow"))
+    monkeypatch.setattr(ops, "silu_mul", lambda *args, **kwargs: seen.append("gate"))
+    x, w = torch.zeros(m, k, dtype=torch.bfloat16), torch.zeros(n, k, dtype=torch.bfloat16)
+    taken = linear._gated_flow(x, w, torch.empty(m, n // 2, dtype=torch.bfloat16), "clamped", 7.0)
+    assert taken == bool(forms) and seen == forms

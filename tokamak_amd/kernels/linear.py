@@ -192,17 +192,29 @@ GATED_MANY_FROM = 129       # rows from which the gated product has its own kern
                             # the library's product and the gate's kernel are level with it (80 to 128 rows: 0.76 to 1.5 times)
 
 
-FLOW_GATED_MOST = 36 << 20      # numbers of gate and up below which their product of 17 to 96 rows flows: 2,048 x 1,024 to 12,288 x 2,048
-                                # 1.06 to 1.77 times as fast (a decode step of 24 rows of 2,048 895 -> 837 us); 19,456 x 2,560 and
-                                # more, whose blocks cannot share K, 0.8 to 1.05 (64 rows of 2,560 1,008 -> 1,044)
+FLOW_GATED_MOST = 36 << 20      # numbers of gate and up below which their product of 17 to 96 rows flows (a decode step of 24 rows of 2,048
+                                # 895 -> 837 us); one of more is long enough for the forms below: in one share 0.71 to 1.6 times as fast
+                                # (9,728 to 34,816 weight rows of 2,048 to 8,192; a decode step of 64 rows of 2,560 1,008 -> 1,044)
 
 
 def _gated_flow(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activation: str, limit: float | None) -> bool:
-    """The gated product of 17 to 96 rows of a small matrix with its weights streamed through LDS (csrc/gemm_flow.hip)."""
+    """The gated product of 17 to 96 rows of a small matrix with its weights streamed through LDS (csrc/gemm_flow.hip): the gate
+    behind one share of K, or, where the blocks of one leave CUs idle, in a kernel that adds the shares of several.  Beside the
+    streaming form (up to 64 rows) and the library's product with the gate's kernel, 51 sizes of 128 to 34,816 weight rows of
+    1,024 to 8,192: 0.96 to 5.3 times as fast, in one share alone 0.28 to 1.75 (1,024 x 4,096 at 96 rows 14.8 -> 11.5 us, in one share
+    26.7; 4,096 x 5,120 at 17 15.0 -> 12.2, 21.4).  From 33 to 64 rows more than 256 blocks stay with the streaming form: a CU
+    holds one, and a second round that is not full was 0.87 to 1.12 times as fast (18,432 x 1,024 at 64 rows 14.5 us against 16.8)."""
     from tokamak_amd.kernels import gemm_bf16
 
-    if (not gemm_bf16.FLOW_ROWS[0] <= x.shape[0] <= gemm_bf16.FLOW_SPLIT_ROWS[1] or gate_up.numel() >= FLOW_GATED_MOST
-            or not ops.gemm_flow_fits(x, gate_up)):
+    m, (n, k) = x.shape[0], gate_up.shape
+    if (not gemm_bf16.FLOW_ROWS[0] <= m <= gemm_bf16.FLOW_SPLIT_ROWS[1] or gate_up.numel() >= FLOW_GATED_MOST
+            or (32 < m <= gemm_bf16.SKINNY_MAX_ROWS and n > gemm_bf16.FLOW_WHOLE_MOST) or not ops.gemm_flow_fits(x, gate_up)):
+        return False
+    shares = ops.flow_shares_pay(m, n, k)
+    if shares and n % 8 == 0:
+        ops.silu_mul(gemm_bf16.flow(x, gate_up, True), out, activation, limit=limit)
+        return True
+    if shares and m > gemm_bf16.SKINNY_MAX_ROWS:      # (the gate's kernel takes whole groups of four channels; the library is ahead of one share)
         return False
     ops.gemm_flow(x, gate_up, out, gate=activation, limit=limit)
     return True
