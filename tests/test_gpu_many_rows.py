@@ -70,7 +70,8 @@ def test_gates(tile, m, n, k):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("activation, limit", [("silu", None), ("clamped", 7.0), ("gelu_tanh", None)])
-@pytest.mark.parametrize("m, n, k", [(128, 256, 256), (129, 256, 256), (300, 248, 320), (300, 252, 320), (300, 256, 328)])
+@pytest.mark.parametrize("m, n, k", [(128, 256, 256), (129, 256, 256), (300, 248, 320), (300, 252, 320), (300, 256, 328), (300, 504, 1024), (300, 512, 1024),
+                                     (129, 128, 2048), (700, 2048, 2048)])
 def test_gated_products_by_any_route(activation, limit, m, n, k):
     """On both sides of each condition of the route, the same numbers to bfloat16's rounding."""
     gen = torch.Generator().manual_seed(m + n + k)

@@ -108,3 +108,15 @@ def test_gated_products_of_few_rows(monkeypatch, m, n, k, forms):
     x, w = torch.zeros(m, k, dtype=torch.bfloat16), torch.zeros(n, k, dtype=torch.bfloat16)
     taken = linear._gated_flow(x, w, torch.empty(m, n // 2, dtype=torch.bfloat16), "clamped", 7.0)
     assert taken == bool(forms) and seen == forms
+
+
+# rows, weight rows, k of a gated product, us by the library and the gate's kernel, us by the many-rows kernel
+GATED = [(256, 256, 512, 19.4, 8.0), (129, 1024, 1024, 13.8, 12.6), (256, 512, 1024, 13.2, 14.8), (512, 4096, 2048, 21.3, 22.1),
+         (700, 4096, 2048, 26.6, 22.0), (200, 16384, 2048, 32.4, 25.8), (256, 1024, 4096, 15.6, 38.3), (700, 4096, 4096, 36.5, 39.2),
+         (1024, 4096, 4096, 46.4, 42.0), (200, 28672, 4096, 94.7, 71.9), (384, 8192, 5120, 53.1, 62.4), (2048, 28672, 5120, 514.8, 464.4),
+         (512, 512, 8192, 22.6, 67.7), (512, 8192, 8192, 82.5, 80.2)]
+
+
+@pytest.mark.parametrize("m, n, k, library, many", GATED)
+def test_gated_products_of_many_rows_go_where_they_were_faster(m, n, k, library, many):
+    assert ops.many_gate_pays(m, n // 2, k) == (many < library)

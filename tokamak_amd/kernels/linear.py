@@ -221,11 +221,12 @@ def _gated_flow(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activ
 
 
 def _gated_many(x: torch.Tensor, gate_up: torch.Tensor, out: torch.Tensor, activation: str, limit: float | None) -> bool:
-    """The gated product of many rows in one kernel, whose block has a channel's gate and up sums side by side: 1.09 times as fast
-    as the library's fastest candidate and the gate's kernel at 150 to 300 rows, 1.11 to 1.25 times beyond (11 sizes of 2,048 to
-    34,816 channels, 0.82 to 2.25: rounds of blocks that end nearly empty, on either side).  With the tanh form of gelu 1.00 to 1.23
+    """The gated product of many rows in one kernel, whose block has a channel's gate and up sums side by side, where its tiles fill
+    enough of the GPU (``ops.many_gate_pays``): 1.25 times as fast on average as the library's first choice and the gate's kernel
+    (24,576 x 4,096 at 2,048 rows 317 -> 288 us).  With the tanh form of gelu 1.00 to 1.23
     times at 24,576 x 4,096 and 19,456 x 2,560 (2,048 rows 329 -> 307 and 230 -> 187 us), 1.16 to 1.59 at 6,144 x 1,024."""
-    if x.shape[0] < GATED_MANY_FROM or activation not in ops.MANY_MODES or not ops.gemm_many_fits(x, gate_up, out.shape[1]):
+    if (x.shape[0] < GATED_MANY_FROM or activation not in ops.MANY_MODES or not ops.gemm_many_fits(x, gate_up, out.shape[1])
+            or not ops.many_gate_pays(x.shape[0], out.shape[1], x.shape[1])):
         return False
     rows, columns = ops.many_plan(x.shape[0], out.shape[1], x.shape[1])
     ops.gemm_many(x, gate_up, out, rows=rows, columns=columns, gate=activation, limit=limit)

@@ -2192,6 +2192,23 @@ def many_plan(m: int, n: int, k: int) -> tuple[int, int]:
 
 
 @functools.lru_cache(maxsize=4096)
+def many_gate_pays(m: int, n: int, k: int) -> bool:
+    """Whether the gated product of more than 128 rows for ``n`` output channels goes to ``gemm_many`` rather than to the library,
+    which shares K where there are few tiles, and the gate's kernel: by the share of the blocks that run at once which its tiles
+    fill, the more of it the longer K is.  54 sizes of 128 to 28,672 weight rows, 129 to 2,048 rows of activations, weights from memory:
+
+    - K of 512: 1.15 to 2.5 times as fast; of 1,024 from 1,024 weight rows on 1.02 to 1.55, below 0.89 to 1.06;
+    - K of 2,048: 0.53 to 0.96 with up to a quarter filled (one product 1.25), from three eighths on 0.96 to 1.29 (4,096 weight rows
+      at 700 rows 26.6 -> 22.0 us);
+    - K of 4,096 to 8,192: 0.19 to 0.94 up to three eighths (two products 1.06 and 1.10; 1,024 x 4,096 at 256 rows 15.6 us against
+      38.3), beyond 0.83 to 1.32: 11 of 80 products more than 5 % behind, most of them of few rows and 16,384 and more weight rows."""
+    if k <= 512 or (k <= 1024 and 2 * n >= 1024):
+        return True
+    rows, columns = many_plan(m, n, k)
+    return -(-m // rows) * -(-2 * n // columns) >= (0.3 if k <= 2048 else 0.4) * MANY_PRICES[rows, columns][0]
+
+
+@functools.lru_cache(maxsize=4096)
 def many_split_plan(m: int, n: int, k: int) -> tuple[int, int, int]:
     """(rows, columns of a tile, shares of K) of the cheapest ``gemm_many`` into partial sums, which cost their reader four bytes a
     number each where the product itself costs two (at 4.5 TB/s)."""
