@@ -193,6 +193,25 @@ def test_all_36_layers_of_8b_width_in_float32():
     assert e1 < 2e-4 and e2 < 2e-4      # 36 layers deep: four times the two-layer bound
 
 
+def test_step_memory_covers_steps_of_fewer_rows_whose_products_are_shared():
+    """A long product of some hundred rows leaves several float32 shares where one of more rows leaves its result once: every
+    such step, too, finds the memory that was kept aside."""
+    from tokamak_amd.engine.runner import ModelRunner, StepEntry
+
+    _, _, plan, source, _ = shaped("qwen3-0.6b", on_gpu=True, num_layers=4, vocab_size=2048, intermediate_size=12288, max_position_embeddings=2048)
+    runner = ModelRunner(plan, source, dtype="bfloat16", page_size=16, kv_pool_tokens=None, max_requests=4, tokens_per_request=2048, max_step_tokens=1200)
+    for rows in (200, 600, 900, 1024, 1100, 1101, 1200):
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        runner.step([StepEntry("a", [0] * rows, [rows - 1])])
+        runner.end("a")
+        torch.cuda.synchronize()
+        took = torch.cuda.max_memory_allocated() - before
+        print(f"{rows} rows: {took / 2**20:.1f} MiB of {runner.step_memory_bytes / 2**20:.1f}")
+        assert took <= runner.step_memory_bytes, rows
+
+
 def test_32b_width_default_pool_leaves_room_for_steps_and_graphs():
     """Construction as generation does it (pool sized from free memory, 64 requests)
     with memory_fraction 0.97 and no other cap: after the pool is taken, a 2,048-token

@@ -102,6 +102,11 @@ class LayeredModel:
         if self.plan.tie_word_embeddings:
             self.head.tie(self.embedding)
 
+    def matrix_shapes(self, dtype: torch.dtype) -> set[tuple[int, int]]:
+        """The (rows, columns) of the parts' matrices of a type."""
+        return {tuple(t.shape) for part in self._all_parts() for t in vars(part).values()
+                if isinstance(t, torch.Tensor) and t.dim() == 2 and t.dtype == dtype}
+
     # -- what the parts ask of a step ------------------------------------------
     def step_planners(self) -> list:
         """The parts' planners of work lists, one per name, in the order first met."""

@@ -22,6 +22,7 @@ from tokamak_amd.engine.decode_graph import DecodeGraph, pow2_at_least
 from tokamak_amd.engine.model import LayeredModel
 from tokamak_amd.engine.storage import CacheStorage
 from tokamak_amd.kernels import ops
+from tokamak_amd.kernels.gemm_bf16 import rows_of_most_shares
 from tokamak_amd.weights.loader import load_weights
 from tokamak_amd.weights.sources import SafetensorsSource
 
@@ -114,18 +115,19 @@ class ModelRunner:
                                     dtype=self.dtype, device=self.device)
 
     def _measure_step_memory(self, max_step_tokens: int, max_requests: int) -> int:
-        """Peak device memory, beyond weights and cache, of the two largest kinds of
-        step: one request bringing ``max_step_tokens`` tokens, and ``max_requests``
-        requests bringing one token each.  Run for real against a throw-away cache
-        just large enough, so whatever the parts allocate is counted, workspaces of
-        library products included."""
+        """Peak device memory, beyond weights and cache, of the largest kinds of
+        step: one request bringing ``max_step_tokens`` tokens, or fewer where a long product of
+        theirs holds more (its shares of K), and ``max_requests`` requests bringing one
+        token each.  Run for real against a throw-away cache just large enough, so whatever
+        the parts allocate is counted, workspaces of library products included."""
         tokens = max(1, min(max_step_tokens, self.plan.max_position_embeddings))
         self._make_cache(-(-tokens // self.page_size) + max_requests, max_requests)
         torch.cuda.synchronize(self.device)
         before = torch.cuda.memory_allocated(self.device)
         torch.cuda.reset_peak_memory_stats(self.device)
-        self.step([StepEntry("measure", [0] * tokens, [tokens - 1])])
-        self.end("measure")
+        for rows in sorted({tokens} | {rows_of_most_shares(n, k, tokens) for n, k in self.model.matrix_shapes(torch.bfloat16)}):
+            self.step([StepEntry("measure", [0] * rows, [rows - 1])])
+            self.end("measure")
         self.step([StepEntry(("measure", i), [0], [0]) for i in range(max_requests)])
         self.end_all()
         torch.cuda.synchronize(self.device)

@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from tokamak_amd.kernels import ops
@@ -158,6 +160,20 @@ def split_many(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     out = torch.empty((parts, m, n), dtype=torch.float32, device=x.device)
     ops.gemm_many(x, weight, out, rows=rows, columns=columns)
     return out
+
+
+@functools.lru_cache(maxsize=256)
+def rows_of_most_shares(n: int, k: int, most: int) -> int:
+    """The number of rows, up to ``most``, at which the product of a matrix [N, K] whose reader adds shares of K holds most memory,
+    operand and result: ``most``, unless fewer rows are cut into so many shares that their sums are more (1,024 rows of 12,288 and
+    four shares of 4,096 sums are 92 MB, 2,048 rows and their product 67 MB)."""
+    limit = min(most, next((rows for least, rows in MANY_SPLIT_ROWS if k >= least), 0)) if k % 64 == 0 and n % 8 == 0 else 0
+
+    def held(m: int) -> int:
+        parts = ops.many_split_plan.__wrapped__(m, n, k)[2] if 128 < m <= limit else 1
+        return 2 * m * k + (4 * parts if parts > 1 else 2) * m * n
+
+    return max((most, *range(129, limit + 1)), key=held)
 
 
 def stream_pays_beyond_64_rows(m: int, n: int, k: int) -> bool:
