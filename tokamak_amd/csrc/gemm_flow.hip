@@ -69,9 +69,9 @@ __device__ __forceinline__ void each(const F& f) {
 template <bool ONCE>
 __device__ __forceinline__ void copy_to_lds(uint32_t to, uint32_t from, const char* base) {
   if constexpr (ONCE)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(to), "v"(from), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(to), "v"(from), "s"(base) : "memory", "m0");
   else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(from), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(from), "s"(base) : "memory", "m0");
 }
 
 constexpr int D = 3;                  // steps of the ring

@@ -74,7 +74,7 @@ __device__ __forceinline__ void each(const F& f) {
 // it: the wave's count of vector memory operations says when it has come.
 template <int AT>
 __device__ __forceinline__ void copy_to_lds(uint32_t to, uint32_t from, const char* base) {
-  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(from), "s"(base), "n"(AT) : "memory", "scc");
+  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(from), "s"(base), "n"(AT) : "memory", "scc", "m0");
 }
 
 // The same number, which the compiler cannot follow: what is computed from it is computed where it stands and not kept in
