@@ -32,6 +32,7 @@
 // So a decode layer of few rows runs q/k/v product, attention, o product, gate/up product and down product
 // with no kernel in between.
 #include "common.h"
+#include "gate.h"
 #include "slots.h"
 
 using namespace tk;
@@ -65,14 +66,6 @@ struct StreamSum {       // ADD
 };
 
 enum { EPI_STORE = 0, EPI_GATED = 1, EPI_ADD = 2 };
-
-// act(z) * u; 2: with g = min(z, limit), g sigmoid(1.702 g) (clamp(u, -limit, limit) + 1)
-__device__ __forceinline__ float gated_value(float z, float u, const RowScale& s) {
-  if (s.act == 0) return z / (1.f + __expf(-z)) * u;
-  if (s.act == 1) return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))) * u;
-  const float g = fminf(z, s.limit);
-  return g / (1.f + __expf(-1.702f * g)) * (fminf(fmaxf(u, -s.limit), s.limit) + 1.f);
-}
 
 template <int TP, int MT, int RG, int EPI, typename TO, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void gemm_direct_kernel(
@@ -246,7 +239,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_direct_kernel(
   for (int e = 0; e < 4; ++e) {
     res[e] = total[0][e] * rstd;
     if constexpr (EPI == EPI_GATED) {
-      res[e] = gated_value(res[e], total[TILES - 1][e] * rstd, scale);
+      res[e] = gated_value(res[e], total[TILES - 1][e] * rstd, scale.act, scale.limit);
     } else if (scale.act == 3) {
       const float v = fmaxf(res[e], 0.f);
       res[e] = v * v;

@@ -13,24 +13,13 @@
 // 14.1 / 10.3 / 8.7 -> 11.1 / 8.7 / 7.9, 2,560 x 9,728 19.2 / 15.1 / 12.5 -> 15.6 / 12.4 / 11.3, 1,024 x 3,072 6.4 / 5.0 / 4.3 -> 6.4 / 4.7 /
 // 4.0; 6,144 x 1,024 gated 9.9 / 7.7 / - -> 8.2 / 6.5 / -; 12,800 x 4,096 into bfloat16 46 / 30 / - -> 27 / 22 / -.
 #include "common.h"
+#include "gate.h"
+#include "lds_copy.h"
 #include "slots.h"
-
-#include <type_traits>
 
 using namespace tk;
 
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-union Frag8 {
-  u32x4 u;
-  bf16x8 v;
-};
-
-#define TK_LDS __attribute__((address_space(3)))
 
 enum { EPI_BF16, EPI_FLOAT, EPI_SILU, EPI_GELU, EPI_CLAMPED };      // the last three: gated
 
@@ -46,33 +35,6 @@ struct Job {
   int squared;          // C = max(., 0)^2
   float limit;          // of the clamped gate
 };
-
-template <int EPI>
-__device__ __forceinline__ float gated(float z, float u, float limit) {
-  if (EPI == EPI_SILU) return z / (1.f + __expf(-z)) * u;
-  if (EPI == EPI_GELU) return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))) * u;
-  const float g = fminf(z, limit);
-  return g / (1.f + __expf(-1.702f * g)) * (fminf(fmaxf(u, -limit), limit) + 1.f);
-}
-
-// f(0), ..., f(N - 1) with the number known to the compiler
-template <int I, int N, typename F>
-__device__ __forceinline__ void each(const F& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    each<I + 1, N>(f);
-  }
-}
-
-// 64 lanes' 16 bytes from base + from (a lane's own) to LDS address to, lane after lane.  No register waits for it: the wave's
-// count of vector memory operations says when it has come.  ONCE: what nobody else will read (a streaming load).
-template <bool ONCE>
-__device__ __forceinline__ void copy_to_lds(uint32_t to, uint32_t from, const char* base) {
-  if constexpr (ONCE)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(to), "v"(from), "s"(base) : "memory", "m0");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(from), "s"(base) : "memory", "m0");
-}
 
 constexpr int D = 3;                  // steps of the ring
 constexpr int kWeightRows = 64;       // of a block
@@ -174,7 +136,7 @@ __global__ __launch_bounds__(256) void gemm_flow_kernel(Job job) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       v[q] = acc[t][q];
-      if (GATED) v[q] = gated<EPI>(v[q], pair32(__float_as_uint(v[q])).b(), job.limit);      // lanes 0 .. 31 hold the gate's sums, 32 .. 63 up's
+      if (GATED) v[q] = gated_value(v[q], pair32(__float_as_uint(v[q])).b(), EPI - EPI_SILU, job.limit);      // lanes 0 .. 31 hold the gate's sums, 32 .. 63 up's
       if (EPI == EPI_BF16 && job.squared) v[q] = fmaxf(v[q], 0.f) * fmaxf(v[q], 0.f);
     }
     if (m >= job.M || n >= job.N || (GATED && g > 1)) continue;

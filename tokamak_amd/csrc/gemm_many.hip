@@ -18,24 +18,13 @@
 // their reader, beside the library's first choice: 4,096 x 12,288 at 200 / 512 / 1,024 rows 45 / 75 / 106, here 37 / 55 / 93; 2,560 x
 // 9,728 32 / 46 / 62, here 26 / 36 / 53; 5,120 x 17,408 226 / 168 / 246, here 57 / 90 / 149.
 #include "common.h"
+#include "gate.h"
+#include "lds_copy.h"
 #include "slots.h"
-
-#include <type_traits>
 
 using namespace tk;
 
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-union Frag8 {
-  u32x4 u;
-  bf16x8 v;
-};
-
-#define TK_LDS __attribute__((address_space(3)))
 
 enum { EPI_PARTS, EPI_SILU, EPI_CLAMPED, EPI_GELU };     // the last three: gated
 
@@ -54,27 +43,8 @@ struct Job {
 
 template <int EPI>
 __device__ __forceinline__ float gated(float z, float u, float limit) {
-  if (EPI == EPI_SILU) return z / (1.f + __expf(-z)) * u;
-  // (half of z (1 + tanh y) is z / (1 + exp(-2 y)))
-  if (EPI == EPI_GELU) return z / (1.f + __expf(-1.5957691216057308f * (z + 0.044715f * z * z * z))) * u;
-  const float g = fminf(z, limit);
-  return g / (1.f + __expf(-1.702f * g)) * (fminf(fmaxf(u, -limit), limit) + 1.f);
-}
-
-// f(0), ..., f(N - 1) with the number known to the compiler
-template <int I, int N, typename F>
-__device__ __forceinline__ void each(const F& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    each<I + 1, N>(f);
-  }
-}
-
-// 64 lanes' 16 bytes from base + from (a lane's own) to LDS address to + AT, lane after lane.  No register waits for
-// it: the wave's count of vector memory operations says when it has come.
-template <int AT>
-__device__ __forceinline__ void copy_to_lds(uint32_t to, uint32_t from, const char* base) {
-  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(from), "s"(base), "n"(AT) : "memory", "scc", "m0");
+  if (EPI == EPI_GELU) return gelu_by_exp(z, u);
+  return gated_value(z, u, EPI == EPI_SILU ? 0 : 2, limit);
 }
 
 // The same number, which the compiler cannot follow: what is computed from it is computed where it stands and not kept in
@@ -159,8 +129,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(blocks_a_cu
   Cursor cx{(int)blockIdx.x, 0, 0, WRING, nullptr}, cw{(int)blockIdx.x, 0, 0, 0, nullptr};
   aim_x(cx);
   aim_w(cw);
-  const auto load_x = [&](auto j) { copy_to_lds<decltype(j)::value * 4096>(lds_wave + cx.slot, xo[decltype(j)::value], cx.base); };
-  const auto load_w = [&](auto j) { copy_to_lds<decltype(j)::value * 4096>(lds_wave + cw.slot, wo[decltype(j)::value], cw.base); };
+  const auto load_x = [&](auto j) { copy_to_lds_at<decltype(j)::value * 4096>(lds_wave + cx.slot, xo[decltype(j)::value], cx.base); };
+  const auto load_w = [&](auto j) { copy_to_lds_at<decltype(j)::value * 4096>(lds_wave + cw.slot, wo[decltype(j)::value], cw.base); };
   constexpr int READS = 2 * (MT + NT), PRODS = 4 * MT * NT;      // of half a step
 #pragma unroll
   for (int t = 0; t < 2; ++t) {

@@ -14,6 +14,7 @@
 // waves' partial sums are added in wave order through LDS (a fixed order, so
 // the result is deterministic) and written as bf16 or float32.
 #include "common.h"
+#include "gate.h"
 #include "slots.h"
 
 using namespace tk;
@@ -260,14 +261,6 @@ struct RowScale {
   float limit;         // of the clamped gate
 };
 
-// act(z) * u; 2: with g = min(z, limit), g sigmoid(1.702 g) (clamp(u, -limit, limit) + 1)
-__device__ __forceinline__ float gated_value(float z, float u, const RowScale& s) {
-  if (s.act == 0) return z / (1.f + __expf(-z)) * u;
-  if (s.act == 1) return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))) * u;
-  const float g = fminf(z, s.limit);
-  return g / (1.f + __expf(-1.702f * g)) * (fminf(fmaxf(u, -s.limit), s.limit) + 1.f);
-}
-
 template <int MT, typename TO, bool GATED, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, TO* __restrict__ C, int M, int N,
@@ -460,10 +453,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
       const float4 u = *reinterpret_cast<const float4*>(up + ((size_t)(wave * MT + j) * 64 + lane) * 4);
-      acc[j][0] = gated_value(acc[j][0], u.x, scale);
-      acc[j][1] = gated_value(acc[j][1], u.y, scale);
-      acc[j][2] = gated_value(acc[j][2], u.z, scale);
-      acc[j][3] = gated_value(acc[j][3], u.w, scale);
+      acc[j][0] = gated_value(acc[j][0], u.x, scale.act, scale.limit);
+      acc[j][1] = gated_value(acc[j][1], u.y, scale.act, scale.limit);
+      acc[j][2] = gated_value(acc[j][2], u.z, scale.act, scale.limit);
+      acc[j][3] = gated_value(acc[j][3], u.w, scale.act, scale.limit);
     }
   }
 
