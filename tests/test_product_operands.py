@@ -132,3 +132,18 @@ def test_no_number_of_rows_holds_more_than_the_one_that_is_measured(n, k, most):
 
     found = gemm_bf16.rows_of_most_shares(n, k, most)
     assert 1 <= found <= most and held(found) >= max(held(m) for m in range(max(1, most - 2000), most + 1))
+
+
+# rows, weight rows, k of a long product whose reader adds partial sums, us by the library, us in shares of K on the many-rows kernel
+LONG = [(129, 64, 9216, 12.4, 11.6), (1024, 6144, 9216, 127.1, 125.8), (1700, 6144, 17408, 535.7, 326.6), (1024, 8192, 9216, 149.8, 145.1),
+        (1100, 8192, 12288, 216.6, 230.2), (1100, 8192, 16384, 482.9, 290.1), (1536, 8192, 17408, 346.2, 386.6), (512, 12288, 12288, 168.9, 162.3),
+        (768, 12288, 9216, 175.1, 186.3), (1024, 12288, 17408, 358.5, 386.4), (1700, 12288, 17408, 987.3, 656.9), (256, 16384, 9216, 122.8, 112.1),
+        (300, 16384, 9216, 124.1, 137.3), (640, 16384, 10240, 197.0, 269.4), (1100, 16384, 12288, 625.8, 468.5), (160, 24576, 25600, 385.9, 610.8),
+        (384, 24576, 9216, 264.2, 367.5)]
+
+
+@pytest.mark.parametrize("m, n, k, library, shares", LONG)
+def test_long_products_are_shared_where_that_was_faster(m, n, k, library, shares):
+    assert gemm_bf16.many_shares_pay(m, n, k) == (shares < library)
+    x, w = (torch.empty(rows, k, dtype=torch.bfloat16, device="meta") for rows in (m, n))
+    assert gemm_bf16.splits_many(x, w) == (shares < library)

@@ -145,12 +145,28 @@ def flow(x: torch.Tensor, weight: torch.Tensor, allow_partials: bool) -> torch.T
 MANY_SPLIT_ROWS = ((16384, 1700), (9216, 1100))
 
 
+def many_shares_pay(m: int, n: int, k: int) -> bool:
+    """Whether a product of more than 128 rows whose reader adds partial sums may be cut into shares of K.  A wide one's whole tiles of
+    256 x 256 fill most of the GPU by themselves, and the shares' sums are more to write and read; what the last round of such tiles
+    leaves idle decides.  Beside the library's first choice, reader included, weights from memory, 1,442 products of 64 to 24,576
+    weight rows of 9,216 to 28,672:
+
+    - up to 6,144 weight rows: 1.72 times as fast on average, 0.94 to 4.6;
+    - up to 16,384 with few of a round's 256 blocks left over (8,192 weight rows: 128, or 160 with K of 16,384 and more; beyond: 112):
+      1.29, 0.89 to 2.7, three of 200 more than 5 % behind; with more left 1.04, 0.73 to 1.66, 33 of 75 (16,384 x 10,240 at 640 rows
+      197 us, here 269 in three shares);
+    - beyond: 0.96, 0.63 to 1.28, 44 of 87 (24,576 x 25,600 at 160 rows 386 us, here 611)."""
+    most = next((rows for least, rows in MANY_SPLIT_ROWS if k >= least), 0)
+    left = -(-m // 256) * -(-n // 256) % 256
+    wide = n <= 16384 and left <= (112 if n > 8192 else 160 if k >= 16384 else 128)
+    return 128 < m <= most and (n <= 6144 or wide)
+
+
 def splits_many(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether a product of many rows is cut into shares of K for its reader to add."""
-    m, k = x.shape
-    most = next((rows for least, rows in MANY_SPLIT_ROWS if k >= least), 0)
-    return (128 < m <= most and ops.gemm_many_fits(x, weight, weight.shape[0])
-            and ops.many_split_plan(m, weight.shape[0], k)[2] > 1)
+    m, n, k = x.shape[0], *weight.shape
+    return (many_shares_pay(m, n, k) and ops.gemm_many_fits(x, weight, n)
+            and ops.many_split_plan(m, n, k)[2] > 1)
 
 
 def split_many(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -167,10 +183,10 @@ def rows_of_most_shares(n: int, k: int, most: int) -> int:
     """The number of rows, up to ``most``, at which the product of a matrix [N, K] whose reader adds shares of K holds most memory,
     operand and result: ``most``, unless fewer rows are cut into so many shares that their sums are more (1,024 rows of 12,288 and
     four shares of 4,096 sums are 92 MB, 2,048 rows and their product 67 MB)."""
-    limit = min(most, next((rows for least, rows in MANY_SPLIT_ROWS if k >= least), 0)) if k % 64 == 0 and n % 8 == 0 else 0
+    limit = min(most, MANY_SPLIT_ROWS[0][1]) if k % 64 == 0 and n % 8 == 0 else 0
 
     def held(m: int) -> int:
-        parts = ops.many_split_plan.__wrapped__(m, n, k)[2] if 128 < m <= limit else 1
+        parts = ops.many_split_plan.__wrapped__(m, n, k)[2] if m <= limit and many_shares_pay(m, n, k) else 1
         return 2 * m * k + (4 * parts if parts > 1 else 2) * m * n
 
     return max((most, *range(129, limit + 1)), key=held)
