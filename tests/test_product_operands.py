@@ -122,16 +122,20 @@ def test_gated_products_of_many_rows_go_where_they_were_faster(m, n, k, library,
     assert ops.many_gate_pays(m, n // 2, k) == (many < library)
 
 
-@pytest.mark.parametrize("n, k", [(4096, 12288), (5120, 17408), (1024, 9216), (1024, 8192), (1020, 9216)])
+@pytest.mark.parametrize("n, k", [(4096, 12288), (5120, 17408), (1024, 9216), (1024, 8192), (1020, 9216), (8192, 28672)])
 @pytest.mark.parametrize("most", [1, 128, 129, 1000, 1100, 1200, 2048, 8192])
-def test_no_number_of_rows_holds_more_than_the_one_that_is_measured(n, k, most):
+def test_no_number_of_rows_holds_more_than_those_that_are_measured(n, k, most):
+    """Whatever a row takes beside the product's operand and result."""
     def held(m):
         x, w = (torch.empty(rows, k, dtype=torch.bfloat16, device="meta") for rows in (m, n))
         parts = ops.many_split_plan(m, n, k)[2] if gemm_bf16.splits_many(x, w) else 1
         return 2 * m * k + (4 * parts if parts > 1 else 2) * m * n
 
     found = gemm_bf16.rows_of_most_shares(n, k, most)
-    assert 1 <= found <= most and held(found) >= max(held(m) for m in range(max(1, most - 2000), most + 1))
+    assert most in found and all(1 <= m <= most for m in found) and len(found) <= 8
+    product = {m: held(m) for m in range(max(1, most - 2000), most + 1)}
+    for row in (0, 20e3, 50e3, 100e3, 150e3, 200e3, 1e6):
+        assert max(held(m) + row * m for m in found) >= max(took + row * m for m, took in product.items())
 
 
 # rows, weight rows, k of a long product whose reader adds partial sums, us by the library, us in shares of K on the many-rows kernel

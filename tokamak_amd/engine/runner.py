@@ -125,7 +125,7 @@ class ModelRunner:
         torch.cuda.synchronize(self.device)
         before = torch.cuda.memory_allocated(self.device)
         torch.cuda.reset_peak_memory_stats(self.device)
-        for rows in sorted({tokens} | {rows_of_most_shares(n, k, tokens) for n, k in self.model.matrix_shapes(torch.bfloat16)}):
+        for rows in sorted({tokens}.union(*(rows_of_most_shares(n, k, tokens) for n, k in self.model.matrix_shapes(torch.bfloat16)))):
             self.step([StepEntry("measure", [0] * rows, [rows - 1])])
             self.end("measure")
         self.step([StepEntry(("measure", i), [0], [0]) for i in range(max_requests)])

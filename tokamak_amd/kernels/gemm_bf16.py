@@ -179,17 +179,19 @@ def split_many(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 
 @functools.lru_cache(maxsize=256)
-def rows_of_most_shares(n: int, k: int, most: int) -> int:
-    """The number of rows, up to ``most``, at which the product of a matrix [N, K] whose reader adds shares of K holds most memory,
-    operand and result: ``most``, unless fewer rows are cut into so many shares that their sums are more (1,024 rows of 12,288 and
-    four shares of 4,096 sums are 92 MB, 2,048 rows and their product 67 MB)."""
+def rows_of_most_shares(n: int, k: int, most: int) -> tuple[int, ...]:
+    """The numbers of rows, up to ``most``, among which is the one at which a step holds most memory that a matrix [N, K] takes part in
+    whose reader adds shares of K: those whose operand and result take more than those of any larger number (1,024 rows of 12,288 and
+    four shares of 4,096 sums 92 MB, 1,100 and three 81, 2,048 and their product 67).  What else a step holds grows with its rows."""
     limit = min(most, MANY_SPLIT_ROWS[0][1]) if k % 64 == 0 and n % 8 == 0 else 0
-
-    def held(m: int) -> int:
+    found, held_most = [], 0
+    for m in (most, *range(min(limit, most - 1), 128, -1)):
         parts = ops.many_split_plan.__wrapped__(m, n, k)[2] if m <= limit and many_shares_pay(m, n, k) else 1
-        return 2 * m * k + (4 * parts if parts > 1 else 2) * m * n
-
-    return max((most, *range(129, limit + 1)), key=held)
+        held = 2 * m * k + (4 * parts if parts > 1 else 2) * m * n
+        if held > held_most:
+            found.append(m)
+            held_most = held
+    return tuple(found)
 
 
 def stream_pays_beyond_64_rows(m: int, n: int, k: int) -> bool:
