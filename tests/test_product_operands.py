@@ -151,3 +151,27 @@ def test_long_products_are_shared_where_that_was_faster(m, n, k, library, shares
     assert gemm_bf16.many_shares_pay(m, n, k) == (shares < library)
     x, w = (torch.empty(rows, k, dtype=torch.bfloat16, device="meta") for rows in (m, n))
     assert gemm_bf16.splits_many(x, w) == (shares < library)
+
+
+# rows, weight rows, k of a product whose reader adds partial sums, us by the forms before, us by the flowing one
+PARTIAL = [(3, 8, 4096, 6.2, 5.8), (80, 8, 4096, 15.9, 7.1), (17, 1016, 16384, 13.5, 11.5), (32, 12800, 4096, 34.0, 31.5), (16, 14336, 8192, 53.2, 42.7),
+           (8, 16384, 4096, 31.7, 40.0), (64, 13824, 4096, 35.0, 37.2), (65, 13824, 4096, 39.2, 38.0), (24, 20480, 2048, 121.1, 62.1),
+           (16, 24576, 3072, 100.1, 78.0), (32, 17408, 8192, 142.6, 157.5), (33, 17408, 2048, 56.3, 75.1), (48, 20480, 8192, 109.5, 188.4),
+           (64, 24576, 4096, 91.3, 129.7), (80, 20480, 2048, 83.6, 72.1), (80, 24576, 4096, 113.1, 134.8), (65, 28672, 8192, 209.1, 161.5)]
+
+
+@pytest.mark.parametrize("m, n, k, before, flow", PARTIAL)
+def test_products_into_partial_sums_flow_where_that_was_faster(m, n, k, before, flow):
+    x, w = (torch.empty(rows, k, dtype=torch.bfloat16, device="meta") for rows in (m, n))
+    assert gemm_bf16.flows(x, w, True) == (flow < before)
+
+
+@pytest.mark.parametrize("m, n, k, forms", [(17, 20480, 2048, ["shares", "relu"]), (17, 20480, 8192, ["flow"])])
+def test_squared_relu_of_wide_matrices_is_shared_only_where_shares_flow(monkeypatch, m, n, k, forms):
+    seen = []
+    monkeypatch.setattr(ops, "flow_shares_pay", lambda *shape: True)
+    monkeypatch.setattr(ops, "gemm_flow", lambda x, w, out, **kwargs: seen.append("shares" if out.dim() == 3 else "flow"))
+    monkeypatch.setattr(ops, "squared_relu", lambda *args: seen.append("relu"))
+    monkeypatch.setattr(gemm_bf16, "flows_whole", lambda *shape: True)
+    linear.activated_linear(*(torch.empty(rows, k, dtype=torch.bfloat16, device="meta") for rows in (m, n)))
+    assert seen == forms

@@ -89,8 +89,8 @@ STREAM_PARTIALS_ROWS = 96           # rows up to which the split streaming produ
 STREAM_PARTIALS_BIG = 64 << 20      # ... and the bytes of a matrix from which it does up to 128 rows
 
 
-FLOW_SPLIT_ROWS = (3, 96)           # rows between which a product whose reader adds partial sums flows (csrc/gemm_flow.hip): beside the forms
-                                    # below, 123 sizes of 1,024 to 12,288 channels, weights from memory, reader included: 1.09 times as fast at 3 to
+FLOW_SPLIT_ROWS = (3, 96)           # rows between which a product whose reader adds partial sums flows (csrc/gemm_flow.hip), if it is not very
+                                    # wide (``flows_shared``): beside the forms below, 123 sizes of 1,024 to 12,288 channels, weights from memory, reader included: 1.09 times as fast at 3 to
                                     # 8 rows, 1.11 at 16, 1.15 at 24 to 64, 1.24 at 96, at worst 0.94 (12,288 x 4,096 at 48); 128 rows: level, 0.81 at worst.  With fewer rows it is
                                     # 1.06 times as fast alone, but beside an experts' branch its few large blocks wait for room (a
                                     # decode step of one request 623 -> 663 us, of two 731 -> 735)
@@ -116,12 +116,31 @@ def flows_whole(m: int, n: int, stride: int) -> bool:
     return n >= STREAM_MIN_ROWS_OUT and (n <= 14336 or stride % 4096 != 0)
 
 
+def flows_shared(m: int, n: int, k: int, stride: int) -> bool:
+    """Whether a product of 3 to 96 rows whose reader adds partial sums flows, by its weight rows and the numbers between them.
+    Beside the forms below (2,900 products of 8 to 65,536 weight rows of 512 to 17,408, weights from memory, reader included):
+
+    - up to 16,384 weight rows, a round of 256 blocks: 1.15 times as fast on average, 28 of 1,744 more than 5 % behind (8 x 4,096 at 80
+      rows 15.9 -> 7.1 us); but 0.87, 0.79 to 1.07, beyond 12,800 if they lie 8 KB apart and up to 64 rows read them (16,384 x 4,096 at
+      8 rows 31.7 us, here 40.0).
+    - More, up to 32 rows: up to 80 M numbers 1.18, 0.87 to 2.1 (20,480 x 2,048 at 24 rows 121 -> 62); beyond, where shares fill several
+      rounds badly, 0.98, 0.66 to 1.37, 86 of 324 (17,408 x 8,192 at 32 rows 143, here 158).
+    - More, 33 to 64 rows: 0.86, 0.58 to 1.09 (20,480 x 8,192 at 48 rows 110, here 188), only 28,672, whose rounds are even, 0.99 to 1.38.
+    - More, 65 to 96 rows: 1.08 at K of up to 2,048, 1.12 from 28,672 weight rows on, 3 of 147; else 0.91, 0.66 to 1.30, 78 of 126."""
+    if n <= 16384:
+        return m > SKINNY_MAX_ROWS or n <= 12800 or stride != 4096
+    if m <= 32:
+        return n * k <= 80 << 20
+    return m > SKINNY_MAX_ROWS and (k <= 2048 or n >= 28672)
+
+
 def flows(x: torch.Tensor, weight: torch.Tensor, allow_partials: bool) -> bool:
     """Whether a product goes to the flowing kernel: into partial sums, or into bfloat16."""
     m, n = x.shape[0], weight.shape[0]
     if allow_partials:
         low, high = FLOW_SPLIT_ROWS
-        taken = low <= m <= high and not (m <= FLOW_BEHIND_DIRECT_ROWS and ops.direct_pays("parts", m, n, weight.shape[1]))
+        taken = (low <= m <= high and flows_shared(m, n, weight.shape[1], weight.stride(0))
+                 and not (m <= FLOW_BEHIND_DIRECT_ROWS and ops.direct_pays("parts", m, n, weight.shape[1])))
     else:
         low, high = FLOW_ROWS
         taken = low <= m <= high and flows_whole(m, n, weight.stride(0))

@@ -178,7 +178,7 @@ def activated_linear(x: torch.Tensor, weight: torch.Tensor, activation: str = "s
                and gemm_bf16.flows_whole(m, max(n, gemm_bf16.STREAM_MIN_ROWS_OUT), weight.stride(0)))
     if _few_rows_fit(m, x, weight, ops.DIRECT_MAX_ROWS) and ops.direct_pays("activated", m, n, k):
         ops.gemm_direct(x, weight, out, activation=activation)
-    elif flowing and not ops.flow_shares_pay(m, n, k):
+    elif flowing and not (ops.flow_shares_pay(m, n, k) and gemm_bf16.flows(x, weight, True)):
         ops.gemm_flow(x, weight, out, activation=activation)
     elif (not flowing and x.dtype == torch.bfloat16 and m <= gemm_bf16.SKINNY_MAX_ROWS and n >= gemm_bf16.STREAM_MIN_ROWS_OUT
             and gemm_bf16.skinny_fits(x, weight) and gemm_bf16.stream_splits(n, k, m) < ACTIVATED_SPLIT_FROM):
