@@ -114,7 +114,8 @@ def test_gated_products_of_few_rows(monkeypatch, m, n, k, forms):
 GATED = [(256, 256, 512, 19.4, 8.0), (129, 1024, 1024, 13.8, 12.6), (256, 512, 1024, 13.2, 14.8), (512, 4096, 2048, 21.3, 22.1),
          (700, 4096, 2048, 26.6, 22.0), (200, 16384, 2048, 32.4, 25.8), (256, 1024, 4096, 15.6, 38.3), (700, 4096, 4096, 36.5, 39.2),
          (1024, 4096, 4096, 46.4, 42.0), (200, 28672, 4096, 94.7, 71.9), (384, 8192, 5120, 53.1, 62.4), (2048, 28672, 5120, 514.8, 464.4),
-         (512, 512, 8192, 22.6, 67.7), (512, 8192, 8192, 82.5, 80.2)]
+         (512, 512, 8192, 22.6, 67.7), (512, 8192, 8192, 82.5, 80.2), (6000, 24576, 4096, 926.9, 912.1), (8192, 24576, 4096, 1219.3, 1259.9),
+         (16384, 2048, 4096, 196.1, 210.4), (8192, 28672, 8192, 2593.1, 3565.3), (8192, 19456, 2560, 779.3, 695.2)]
 
 
 @pytest.mark.parametrize("m, n, k, library, many", GATED)

@@ -2201,7 +2201,11 @@ def many_gate_pays(m: int, n: int, k: int) -> bool:
     - K of 2,048: 0.53 to 0.96 with up to a quarter filled (one product 1.25), from three eighths on 0.96 to 1.29 (4,096 weight rows
       at 700 rows 26.6 -> 22.0 us);
     - K of 4,096 to 8,192: 0.19 to 0.94 up to three eighths (two products 1.06 and 1.10; 1,024 x 4,096 at 256 rows 15.6 us against
-      38.3), beyond 0.83 to 1.32: 11 of 80 products more than 5 % behind, most of them of few rows and 16,384 and more weight rows."""
+      38.3), beyond 0.83 to 1.32: 11 of 80 products more than 5 % behind, most of them of few rows and 16,384 and more weight rows;
+    - 3,000 to 16,384 rows, 10 sizes: K of up to 2,560 0.97 to 1.8; more 0.95 to 1.28 up to 6,000 rows (24,576 x 4,096 at 4,096 rows 604 us,
+      the library and the gate 620), from 8,192 rows on 0.73 to 1.04, 0.94 on average (2,521 us against 2,373 at 16,384)."""
+    if m >= 8192 and k > 2560:
+        return False
     if k <= 512 or (k <= 1024 and 2 * n >= 1024):
         return True
     rows, columns = many_plan(m, n, k)
