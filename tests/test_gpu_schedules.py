@@ -299,6 +299,7 @@ def test_layers_launched_from_a_recorded_layer_give_the_same_bits(dtype):
     step of 70 tokens), and the same cache afterwards; and the list was in fact used."""
     from tokamak_amd.engine import layer_replay
     from tokamak_amd.engine.runner import ModelRunner, StepEntry
+    from tokamak_amd.kernels import ops
 
     cfg, cfg_json, plan, source, w = shaped("qwen3-0.6b", on_gpu=True, num_layers=5, vocab_size=2048,
                                             max_position_embeddings=1024)
@@ -320,17 +321,26 @@ def test_layers_launched_from_a_recorded_layer_give_the_same_bits(dtype):
         cache = [a.clone() for slot in sorted(runner.storage._slots) for a in runner.storage.slot(slot).arrays.values()]
         return [o.cpu() for o in out], cache
 
-    packed = []
+    packed, issued = [], []
+    replay_calls = ops.replay_calls
 
     def counted(self, tensors, then):
         launched.append(len(self.calls))
-        packed.append(self.packed is not None and len(self.packed.expected) == len(self.calls))
-        return launch(self, tensors, then)
+        before = len(issued)
+        result = launch(self, tensors, then)
+        packed.append(issued[before:] == [len(self.calls)])
+        return result
+
+    def issue(count, *lists):
+        issued.append(count)
+        return replay_calls(count, *lists)
 
     plainly, cache_plain = run(False)
     try:
+        ops.replay_calls = issue
         layer_replay.LayerRecording.launch = counted
         replayed, cache_replayed = run(True)
+        whole_lists = len(issued)
         # ... and once more with the lists issued call by call from Python (what a recording falls
         # back to when an entry point has no slot form)
         layer_replay.LayerRecording.launch = lambda self, tensors, then: (
@@ -338,11 +348,11 @@ def test_layers_launched_from_a_recorded_layer_give_the_same_bits(dtype):
         by_call, cache_by_call = run(True)
     finally:
         layer_replay.LayerRecording.launch = launch
+        ops.replay_calls = replay_calls
     assert len(launched) == 5 * (cfg.num_layers - 2), "three of five layers of every step are launched from the list"
     assert min(launched) >= 5
-    # a list is issued call by call at its first replay and packed behind it: of the three replayed
-    # layers of a step the second and third go out in one foreign call each (csrc/replay.hip)
-    assert packed == [False, True, True] * 5, packed
+    # a list is packed at its first replay: each of the three replayed layers of a step goes out in one foreign call (csrc/replay.hip)
+    assert packed == [True, True, True] * 5 and len(issued) == whole_lists == 15, (packed, issued)
     for a, b in zip(replayed, by_call):
         assert torch.equal(a, b)
     for a, b in zip(cache_replayed, cache_by_call):
