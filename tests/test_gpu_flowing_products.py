@@ -4,6 +4,7 @@ Operands are small whole numbers, whose sums are exact in float32 in any order, 
 import pytest
 import torch
 
+from gated_reference import gated, rounded
 from tokamak_amd.kernels import linear, ops
 
 DEV = "cuda:0"
@@ -49,6 +50,39 @@ def test_products_and_shares_of_k(m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [3, 17, 40, 96])
+@pytest.mark.parametrize("parts", [2, 3, 4])
+def test_shares_of_fewer_steps_than_there_are_tiles(m, parts):
+    """Blocks of a share begin at each of its steps, and go round from its last to its first."""
+    n, k = 700, 1408          # 11 tiles; 11 steps in shares of 2 to 6
+    x, w = whole(m, k, 3, 15).to(DEV), whole(n, k, 3, 16).to(DEV)
+    sums = torch.full((parts + 1, m, n), float("nan"), device=DEV)
+    ops.gemm_flow(x, w, sums[:parts])
+    for p in range(parts):
+        cut = slice(p * 11 // parts * 128, (p + 1) * 11 // parts * 128)
+        assert torch.equal(sums[p], x[:, cut].float() @ w[:, cut].float().T), p
+    assert torch.isnan(sums[parts]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [3, 17, 40, 65, 96])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_what_is_not_finite_stays_in_its_row_and_channel(m, bad):
+    n, k = 136, 384
+    x, w = whole(m, k, 3, 17).to(DEV), whole(n, k, 3, 18).to(DEV)
+    exact = x.float() @ w.float().T
+    x[m - 1, k - 1] = w[n - 1, 0] = bad
+    out = torch.empty(2, m, n, device=DEV)
+    ops.gemm_flow(x, w, out)
+    assert torch.equal(out.sum(0)[:-1, :-1], exact[:-1, :-1])
+    sums = x.float() @ w.float().T
+    assert torch.equal(out.sum(0)[-1].nan_to_num(7.0), sums[-1].nan_to_num(7.0)) and torch.equal(out.sum(0)[:, -1].nan_to_num(7.0), sums[:, -1].nan_to_num(7.0))
+    products = torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+    ops.gemm_flow(x, w, products, gate="silu")
+    assert torch.isfinite(products[:-1, :-1]).all() and not torch.isfinite(products[:-1, -1]).any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m", ROWS)
 @pytest.mark.parametrize("n, k", [(4, 128), (37, 256), (100, 512)])
 def test_gates(m, n, k):
@@ -79,12 +113,9 @@ def test_every_route_gives_the_product(m, n, k):
     assert torch.equal(linear.linear(x, w, torch.float32), exact)
     parts = linear.linear(x, w, allow_partials=True)
     assert torch.equal(parts.float().sum(0) if parts.dim() == 3 else parts, exact if parts.dim() == 3 else exact.to(torch.bfloat16))
-    gate = linear.gated_linear(x, w)
-    half = n // 2
-    want = torch.nn.functional.silu(exact[:, :half].double()) * exact[:, half:].double()
-    # (some routes round gate and up to bfloat16 first: 2^-9 of each, the gate's of its argument)
-    slack = (2.0 ** -7 + 2.0 ** -9 * exact[:, :half].abs().double()) * want.abs() + 1e-30
-    assert ((gate.double() - want).abs() <= slack).all()
+    # (some routes round gate and up to bfloat16 first)
+    want, slack = gated(exact.double(), rounded(exact.double()))
+    assert ((linear.gated_linear(x, w).double() - want).abs() <= slack).all()
 
 
 @pytest.mark.gpu
@@ -99,10 +130,8 @@ def test_rows_that_overlap_have_their_product(m):
         parts = linear.linear(x, w, allow_partials=True)
         assert torch.equal(parts.float().sum(0) if parts.dim() == 3 else parts, exact if parts.dim() == 3 else exact.to(torch.bfloat16))
         assert torch.equal(linear.activated_linear(x, w), (exact.clamp(min=0) ** 2).to(torch.bfloat16))
-        g, u = exact[:, :n // 2].double(), exact[:, n // 2:].double()
-        want = torch.nn.functional.silu(g) * u
-        # (some routes round gate and up to bfloat16 first: 2^-9 of each, the gate's of its argument)
-        assert ((linear.gated_linear(x, w).double() - want).abs() <= (2.0 ** -7 + 2.0 ** -9 * g.abs()) * want.abs() + 1e-30).all()
+        want, slack = gated(exact.double(), rounded(exact.double()))
+        assert ((linear.gated_linear(x, w).double() - want).abs() <= slack).all()
 
 
 @pytest.mark.gpu
@@ -120,16 +149,9 @@ def test_squared_relu_by_every_route(m, n, k):
 @pytest.mark.parametrize("m", [17, 32, 33, 64, 65, 96])
 @pytest.mark.parametrize("n, k", [(64, 4096), (1028, 2048), (1032, 2048), (16400, 128)])
 def test_gates_behind_one_share_and_several(activation, limit, m, n, k):
-    """Sums are exact, below 256 also in bfloat16, in which the library's route leaves them.  The result is off by half a unit of
-    2^-8, the exponential by 2^-23 of its argument's size (at most 88), one and the tangent by 2^-22 where it is near -1."""
+    """Sums are exact, below 256 also in bfloat16, in which the library's route leaves them."""
     x, w = whole(m, k, 1, 13).to(DEV), whole(n, k, 1, 14).to(DEV)
     sums = x.double() @ w.double().T
-    g, u = sums[:, :n // 2], sums[:, n // 2:]
-    got = linear.gated_linear(x, w, activation, limit).double()
-    if activation == "clamped":
-        g, u = g.clamp(max=limit), u.clamp(-limit, limit) + 1
-        want = g * torch.sigmoid(1.702 * g) * u
-    else:
-        want = u * (torch.nn.functional.silu(g) if activation == "silu" else torch.nn.functional.gelu(g, approximate="tanh"))
+    want, slack = gated(sums, torch.zeros_like(sums), activation, limit)
     assert sums.abs().max() <= 256
-    assert ((got - want).abs() <= (2.0 ** -8 + 88 * 2.0 ** -22) * want.abs() + 2.0 ** -22 * (g * u).abs() + 1e-30).all()
+    assert ((linear.gated_linear(x, w, activation, limit).double() - want).abs() <= slack).all()

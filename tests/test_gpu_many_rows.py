@@ -4,6 +4,7 @@ gated.  Operands are small whole numbers, whose sums are exact in float32 in any
 import pytest
 import torch
 
+from gated_reference import gated
 from tokamak_amd.kernels import linear, ops
 
 DEV = "cuda:0"
@@ -68,6 +69,55 @@ def test_gates(tile, m, n, k):
         assert ((out.cpu().double() - want).abs() <= (2.0 ** -8 + 3 * k * 2.0 ** -22) * want.abs() + 1e-30).all() and outside_is_nan(wide)
 
 
+SEVERAL = [((256, 256), 2100, 2568), ((128, 256), 1100, 2568), ((256, 128), 2100, 1288), ((128, 128), 2100, 1288)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile, m, n", SEVERAL)
+@pytest.mark.parametrize("parts, k", [(3, 320), (6, 704)])
+def test_several_rounds_of_shares_of_unlike_length(tile, m, n, parts, k):
+    """A block goes on to a unit of another share, longer or shorter than its own, while the loads of both are under way."""
+    x, w = whole(m, k, 3, 9).to(DEV), whole(n, k, 3, 10).to(DEV)
+    out = torch.full((parts + 1, m, n), float("nan"), device=DEV)
+    ops.gemm_many(x, w, out[:parts], rows=tile[0], columns=tile[1])
+    steps = k // 64
+    for p in range(parts):
+        cut = slice(p * steps // parts * 64, (p + 1) * steps // parts * 64)
+        assert torch.equal(out[p], x[:, cut].float() @ w[:, cut].float().T), p
+    assert torch.isnan(out[parts]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile, m, n", [((256, 256), 2100, 3720), ((128, 256), 2100, 2056), ((256, 128), 4200, 1032), ((128, 128), 3000, 1480)])
+@pytest.mark.parametrize("k", [64, 192])
+def test_gates_in_several_rounds(tile, m, n, k):
+    """Sums are exact, so the result is off by half a unit of 2^-8 and the exponential's error, 2^-23 of its argument's size."""
+    x, w = whole(m, k, 1, 11).to(DEV), whole(2 * n, k, 1, 12).to(DEV)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.gemm_many(x, w, out, rows=tile[0], columns=tile[1], gate="silu")
+    sums = (x.float() @ w.float().T).double()
+    want = torch.nn.functional.silu(sums[:, :n]) * sums[:, n:]
+    assert ((out.double() - want).abs() <= (2.0 ** -8 + k * 2.0 ** -22) * want.abs() + 1e-30).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_what_is_not_finite_stays_in_its_row_and_channel(tile, bad):
+    m, n, k = 300, 272, 192
+    x, w = whole(m, k, 3, 13).to(DEV), whole(n, k, 3, 14).to(DEV)
+    exact = x.float() @ w.float().T
+    x[m - 1, k - 1] = w[n - 1, 0] = bad
+    out = torch.empty(3, m, n, device=DEV)
+    ops.gemm_many(x, w, out, rows=tile[0], columns=tile[1])
+    assert torch.equal(out.sum(0)[:-1, :-1], exact[:-1, :-1])
+    sums = x.float() @ w.float().T
+    assert torch.equal(out.sum(0)[-1].nan_to_num(7.0), sums[-1].nan_to_num(7.0)) and torch.equal(out.sum(0)[:, -1].nan_to_num(7.0), sums[:, -1].nan_to_num(7.0))
+    products = torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+    ops.gemm_many(x, w, products, rows=tile[0], columns=tile[1], gate="silu")
+    assert torch.isfinite(products[:-1, :-1]).all() and not torch.isfinite(products[:-1, -1]).any()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("activation, limit", [("silu", None), ("clamped", 7.0), ("gelu_tanh", None)])
 @pytest.mark.parametrize("m, n, k", [(128, 256, 256), (129, 256, 256), (300, 248, 320), (300, 252, 320), (300, 256, 328), (300, 504, 1024), (300, 512, 1024),
@@ -77,14 +127,12 @@ def test_gated_products_by_any_route(activation, limit, m, n, k):
     gen = torch.Generator().manual_seed(m + n + k)
     x = torch.randn(m, k, generator=gen).to(torch.bfloat16).to(DEV)
     w = (torch.randn(2 * n, k, generator=gen) * k ** -0.5).to(torch.bfloat16).to(DEV)
-    got = linear.gated_linear(x, w, activation, limit)
-    parts = torch.empty(1, m, 2 * n, device=DEV)
-    parts[0] = (x.double() @ w.double().T).float()
-    want = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
-    if n % 4 == 0:
-        ops.silu_mul(parts, want, activation, limit=limit)
-        # the routes that round gate and up to bfloat16 first are off by 2^-8 of each (and of the sum of one and up)
-        assert (got.float() - want.float()).abs().max() <= 2.0 ** -6 * want.float().abs().max()
+    got = linear.gated_linear(x, w, activation, limit).double()
+    sums = x.double() @ w.double().T
+    # a float32 sum of k products, then (some routes) rounded to bfloat16, whose eight bits are off by up to 2^-8
+    off = 2.0 ** -8 * sums.abs() + k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    want, slack = gated(sums, off, activation, limit)
+    assert ((got - want).abs() <= slack).all()
 
 
 @pytest.mark.gpu
