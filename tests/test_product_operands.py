@@ -51,7 +51,7 @@ def test_narrow_products_flow_from_33_rows(m, n, taken):
 
 
 # (rows, weight rows, k, us of the flowing product with the activation in its epilogue, us in shares of K with the activation's kernel)
-SHARES = [(17, 256, 1024, 5.6, 5.5), (17, 8192, 1024, 6.4, 7.5), (64, 8192, 1024, 8.1, 11.0), (17, 4096, 2048, 9.0, 7.9),
+SHARES = [(24, 2048, 1024, 5.8, 6.4), (17, 1024, 1024, 5.6, 5.9), (64, 1024, 2048, 11.3, 8.8), (17, 8192, 1024, 6.4, 7.5), (64, 8192, 1024, 8.1, 11.0), (17, 4096, 2048, 9.0, 7.9),
           (64, 12800, 2048, 15.3, 19.3), (32, 4096, 4096, 17.7, 11.1), (33, 8192, 4096, 22.5, 17.9), (64, 12800, 4096, 31.5, 35.3),
           (17, 64, 8192, 29.4, 8.9), (48, 4096, 17408, 75.7, 30.6)]
 

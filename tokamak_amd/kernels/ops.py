@@ -2129,9 +2129,9 @@ def flow_parts(m: int, n: int, k: int) -> int:
 
 
 # Microseconds of a kernel behind a flowing product that adds its shares and applies an activation or a gate to ``n`` sums a row: with it,
-# the cheaper of that and the same in the epilogue of one share is picked within 1 % on average and 9 % at worst (630 products
-# of 17 to 96 rows, 64 to 17,408 weight rows of 1,024 to 17,408, squared relu and silu gates; 0 us: 24 to 31 % at worst, 4 us: 12 to 14).
-FLOW_BEHIND = 2.5
+# the cheaper of that and the same in the epilogue of one share is picked within 0.1 % on average and 6 % at worst (1,116 products
+# of 17 to 96 rows, 128 to 12,288 weight rows of 512 to 8,192, squared relu and silu gates; 2.5 us: 12 to 17 % at worst, 4.5 us: 13 to 14).
+FLOW_BEHIND = 3.5
 
 
 @functools.lru_cache(maxsize=8192)
