@@ -136,14 +136,15 @@ def flows_shared(m: int, n: int, k: int, stride: int) -> bool:
 
 def flows(x: torch.Tensor, weight: torch.Tensor, allow_partials: bool) -> bool:
     """Whether a product goes to the flowing kernel: into partial sums, or into bfloat16."""
-    m, n = x.shape[0], weight.shape[0]
+    m = x.shape[0]
+    low, high = FLOW_SPLIT_ROWS if allow_partials else FLOW_ROWS
+    if not low <= m <= high:
+        return False
+    (n, k), stride = weight.shape, weight.stride(0)
     if allow_partials:
-        low, high = FLOW_SPLIT_ROWS
-        taken = (low <= m <= high and flows_shared(m, n, weight.shape[1], weight.stride(0))
-                 and not (m <= FLOW_BEHIND_DIRECT_ROWS and ops.direct_pays("parts", m, n, weight.shape[1])))
+        taken = flows_shared(m, n, k, stride) and not (m <= FLOW_BEHIND_DIRECT_ROWS and ops.direct_pays("parts", m, n, k))
     else:
-        low, high = FLOW_ROWS
-        taken = low <= m <= high and flows_whole(m, n, weight.stride(0))
+        taken = flows_whole(m, n, stride)
     return taken and ops.gemm_flow_fits(x, weight)
 
 
@@ -175,17 +176,16 @@ def many_shares_pay(m: int, n: int, k: int) -> bool:
       1.29, 0.89 to 2.7, three of 200 more than 5 % behind; with more left 1.04, 0.73 to 1.66, 33 of 75 (16,384 x 10,240 at 640 rows
       197 us, here 269 in three shares);
     - beyond: 0.96, 0.63 to 1.28, 44 of 87 (24,576 x 25,600 at 160 rows 386 us, here 611)."""
-    most = next((rows for least, rows in MANY_SPLIT_ROWS if k >= least), 0)
+    if m <= 128 or k < MANY_SPLIT_ROWS[-1][0] or m > next(rows for least, rows in MANY_SPLIT_ROWS if k >= least):
+        return False
     left = -(-m // 256) * -(-n // 256) % 256
-    wide = n <= 16384 and left <= (112 if n > 8192 else 160 if k >= 16384 else 128)
-    return 128 < m <= most and (n <= 6144 or wide)
+    return n <= 6144 or (n <= 16384 and left <= (112 if n > 8192 else 160 if k >= 16384 else 128))
 
 
 def splits_many(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether a product of many rows is cut into shares of K for its reader to add."""
-    m, n, k = x.shape[0], *weight.shape
-    return (many_shares_pay(m, n, k) and ops.gemm_many_fits(x, weight, n)
-            and ops.many_split_plan(m, n, k)[2] > 1)
+    m, (n, k) = x.shape[0], weight.shape
+    return many_shares_pay(m, n, k) and ops.gemm_many_fits(x, weight, n) and ops.many_split_plan(m, n, k)[2] > 1
 
 
 def split_many(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:

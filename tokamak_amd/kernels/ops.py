@@ -2143,14 +2143,20 @@ def flow_shares_pay(m: int, n: int, k: int) -> bool:
     return parts > 1 and _flow_price(m, n, k, parts) + FLOW_BEHIND < whole
 
 
+def _apart(a: torch.Tensor, w: torch.Tensor, step: int, beyond: int) -> bool:
+    """Whether both are bfloat16 matrices with rows on 16-byte borders that do not overlap, K whole steps, offsets within ``beyond``
+    rows more than the weights have in 32 bits."""
+    if not a.dtype == w.dtype == torch.bfloat16 or not a.dim() == w.dim() == 2:
+        return False
+    k, (n, wk), (lda, a_inner), (ldw, w_inner) = a.shape[1], w.shape, a.stride(), w.stride()
+    return (a_inner == w_inner == 1 and k >= step and k % step == 0 and k <= lda <= MANY_MAX_STRIDE and wk <= ldw
+            and (lda | ldw) % 8 == 0 and (a.data_ptr() | w.data_ptr()) % 16 == 0 and ldw * (n + beyond) < 1 << 31)
+
+
 def gemm_flow_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gemm_flow`` takes these operands: bfloat16 rows on 16-byte borders that do not overlap, up to 128 of them, whole
     steps of 128 k."""
-    return (a.dtype == w.dtype == torch.bfloat16 and a.dim() == w.dim() == 2 and a.stride(1) == w.stride(1) == 1
-            and 0 < a.shape[0] <= FLOW_MAX_ROWS and a.shape[1] >= 128 and a.shape[1] % 128 == 0
-            and a.stride(0) >= a.shape[1] and w.stride(0) >= w.shape[1]
-            and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and a.stride(0) <= MANY_MAX_STRIDE and w.stride(0) * (w.shape[0] + 128) < 1 << 31)
+    return _apart(a, w, 128, 128) and 0 < a.shape[0] <= FLOW_MAX_ROWS
 
 
 MANY_MAX_STRIDE = 1 << 22      # (offsets within a tile's rows are 32 bits)
@@ -2159,11 +2165,7 @@ MANY_MAX_STRIDE = 1 << 22      # (offsets within a tile's rows are 32 bits)
 def gemm_many_fits(a: torch.Tensor, w: torch.Tensor, n: int) -> bool:
     """Whether ``gemm_many`` takes these operands for ``n`` output channels: bfloat16 rows on 16-byte borders that do not overlap,
     whole steps of 64 k."""
-    return (a.dtype == w.dtype == torch.bfloat16 and a.dim() == w.dim() == 2 and a.stride(1) == w.stride(1) == 1
-            and a.shape[1] >= 64 and a.shape[1] % 64 == 0 and n >= 8 and n % 8 == 0
-            and a.stride(0) >= a.shape[1] and w.stride(0) >= w.shape[1]
-            and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and a.stride(0) <= MANY_MAX_STRIDE and w.stride(0) * (w.shape[0] + 256) < 1 << 31)
+    return n >= 8 and n % 8 == 0 and _apart(a, w, 64, 256)
 
 
 # What a product of many rows is priced with, in microseconds: per tile (rows, columns) blocks that run at once; a step of 64 k
