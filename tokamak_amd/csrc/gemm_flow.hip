@@ -1,4 +1,5 @@
-// bf16 products of 3 to 128 rows (decode steps of many requests): C[M,N] = A[M,K] W[N,K]^T, the weights streamed through LDS.
+// bf16 products of up to 128 rows (decode steps of many requests; the routes take 3 to 96): C[M,N] = A[M,K] W[N,K]^T, the weights
+// streamed through LDS.
 //
 // What bounds it is the weights' bytes.  Weights and activations go from memory to LDS without passing through registers
 // (global_load_lds): a ring of three steps of 128 k, two of which are asked for ahead, 256 contiguous bytes of a row (with 128 the memory

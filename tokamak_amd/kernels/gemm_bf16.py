@@ -237,7 +237,8 @@ def gemm(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, allow_pa
     sums when the matrix has few rows and the caller adds them; the
     direct-operand one for very small matrices.  65 to 128 rows, if the caller adds partial
     sums: the same kernel with five to eight tiles of 16 rows where it was measured to pay
-    (``stream_pays_beyond_64_rows``).  Else more than 64 rows
+    (``stream_pays_beyond_64_rows``; up to 96 these are the products that do not flow: K not a
+    multiple of 128, or a very wide matrix).  Else more than 64 rows
     with bfloat16 output: the library product (hipBLASLt, as the reference's
     nn.Linear ends in a library; csrc/blas_lt.hip); with float32 output: 128 rows at a time.
     """

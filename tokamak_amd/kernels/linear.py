@@ -1,9 +1,10 @@
 """y = x @ W^T for the projections of a step.
 
 float32: hand-written kernels with true 32-bit multiply-add and one summation order
-(tiled, or weight-streaming for up to 64 rows; row-wise deterministic, equal bits).  bfloat16: hand-written MFMA kernels for up to 64 rows, up
-to 128 whose reader adds partial sums, for gated products of any number and long ones of up to 1,100 or 1,700; else the library
-product (as the reference's nn.Linear does).
+(tiled, or weight-streaming for up to 64 rows; row-wise deterministic, equal bits).  bfloat16: hand-written MFMA kernels for up to 64 rows; up
+to 96 (large matrices 128) whose reader adds partial sums; gated products of 65 to 96 rows of small matrices, and of more than 128
+that fill the GPU; long products of up to 1,100 or 1,700 rows whose reader adds partial sums.  Else the library product (as the
+reference's nn.Linear does).
 
 Decode steps of few rows (bfloat16, up to 16) can do without the kernels between the
 products: a part's last product adds its result into the float32 residual stream itself
@@ -253,9 +254,12 @@ def gated_linear(x: torch.Tensor | DeferredNorm, gate_up: torch.Tensor, activati
                  limit: float | None = None) -> torch.Tensor:
     """act(x @ gate^T) * (x @ up^T) for ``gate_up`` = [gate; up] ([2I, K]) -> [M, I].
 
-    bfloat16 with up to 64 rows: one fused weight-streaming kernel (the whole-K form for very small
-    matrices has the SiLU gate only).  Otherwise the product, then the gate kernel (``activation``:
-    "silu", "gelu_tanh", or "clamped" with its ``limit``: both halves clamped, see ``ops.silu_mul``).
+    ``activation``: "silu", "gelu_tanh", or "clamped" with its ``limit``: both halves clamped, see ``ops.silu_mul``.
+
+    bfloat16 by rows: up to 16 the whole-K form (very small matrices, silu alone), the direct or the streaming one; 17 to 96, K
+    a multiple of 128 and below ``FLOW_GATED_MOST`` numbers, the flowing one (``_gated_flow``); else up to 64 the streaming one,
+    or it split over K and the gate's kernel; from 129, K a multiple of 64, I of 8 and enough tiles (``ops.many_gate_pays``), the
+    many-rows one.  Otherwise, and in float32, the product, then the gate's kernel.
     """
     m = x.shape[0]
     if activation != "silu":

@@ -2071,7 +2071,7 @@ FLOW_GATES = {"silu": 2, "gelu_tanh": 3, "clamped": 4}      # modes of tk_gemm_f
 
 def gemm_flow(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, gate: str | None = None, limit: float | None = None,
               activation: str | None = None) -> None:
-    """Products of up to 128 rows, the weights streamed through LDS:
+    """Products of up to 128 rows (``gemm_bf16.flows`` and the gated routes take 3 to 96), the weights streamed through LDS:
     out[M, N] (bfloat16 or float32) = a[M, K] @ w[N, K]^T, with ``activation`` "squared_relu" (bfloat16) max(., 0)^2 of it; with
     a ``gate`` w = [gate; up] and out (bfloat16) = act(a @ gate^T) * (a @ up^T), see ``silu_mul``; out [P, M, N] float32: the
     sums over P shares of K."""
