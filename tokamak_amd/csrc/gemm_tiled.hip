@@ -98,7 +98,8 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const TI* __restrict__ 
   }
 }
 
-// The same product on the matrix cores: v_mfma_f32_32x32x2_f32 multiplies and adds in full
+// The same product on the matrix cores, for operands that gemm_float32.hip does not take (rows off 16-byte borders, K not a
+// multiple of four): v_mfma_f32_32x32x2_f32 multiplies and adds in full
 // float32 and, for every output element, gives exactly the bits of fmaf over its two k in
 // ascending order (measured against the chain on random operands: every output of every
 // step equal), so a walk over k in steps of two is the chain of the kernels above and below,
@@ -128,13 +129,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   const int wm = (wave & 1) * 32 * H, wn = (wave >> 1) * 32 * H;   // this wave's corner of the block's tile
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
   const int lrow = tid / LANES, lk = (tid % LANES) * 4;
-  // four k of a row are one 16-byte load; rows past the end are read at the last row and never stored, what lies past K is
-  // read at the row's end and becomes zero.  Where rows do not lie on 16-byte borders, or K ends within a piece, a whole
-  // piece is still one load of 16 bytes, on the border that its numbers have (1,000
-  // rows, weights of 6,144 x 2,048, one operand off its border 293 us, by single numbers 394; K of 2,049 300 and 407; 4 rows 54, 66).
-  const bool wide = K % 4 == 0 && K >= 4 && lda % 4 == 0 && ldw % 4 == 0 &&
-                    (reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) % 16 == 0;
-
+  // Four k of a row are one load of 16 bytes, on the border that its numbers have (1,000 rows, weights of 6,144 x 2,048, one operand off
+  // its border 293 us, by single numbers 394; K of 2,049 300 and 407; 4 rows 54, 66); rows past the end are read at the last row
+  // and never stored, what lies past K becomes zero.
   float16v acc[H][H], total[H][H];
 #pragma unroll
   for (int i = 0; i < H; ++i)
@@ -146,13 +143,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   float4v ar[PASSES], wr[PASSES];
   const auto fetch = [&](int k0) {
     const int k = k0 + lk;
-    if (wide) {
-#pragma unroll
-      for (int h = 0; h < PASSES; ++h) {
-        ar[h] = *reinterpret_cast<const float4v*>(A + (size_t)min(m0 + lrow + ROWS * h, M - 1) * lda + min(k, K - 4));
-        wr[h] = *reinterpret_cast<const float4v*>(W + (size_t)min(n0 + lrow + ROWS * h, N - 1) * ldw + min(k, K - 4));
-      }
-    } else if (k + 3 < K) {
+    if (k + 3 < K) {
 #pragma unroll
       for (int h = 0; h < PASSES; ++h) {
         __builtin_memcpy(&ar[h], A + (size_t)min(m0 + lrow + ROWS * h, M - 1) * lda + k, 16);
@@ -182,10 +173,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
           for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
         }
     }
-    const bool inside = k0 + lk < K;       // (K a multiple of four, or `fetch` has made the zeros)
 #pragma unroll
     for (int h = 0; h < PASSES; ++h) {
-      const float4v a = inside ? ar[h] : float4v{0.f, 0.f, 0.f, 0.f}, w = inside ? wr[h] : float4v{0.f, 0.f, 0.f, 0.f};
+      const float4v a = ar[h], w = wr[h];
       float* const ap = &As[buf][lrow + ROWS * h][lk / 2];
       float* const wp = &Ws[buf][lrow + ROWS * h][lk / 2];
       *reinterpret_cast<float2*>(ap) = make_float2(a[0], a[2]);

@@ -272,6 +272,9 @@ _SIGS = {
         "tk_gemm_fewrows": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_int, c_int,
                             c_int, c_int, c_void_p],
     },
+    "gemm_float32": {
+        "tk_gemm_float32": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_int, c_void_p],
+    },
     "gemm_mfma": {
         "tk_gemm_stream": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long,
                            c_long, c_int, c_long, c_int, c_void_p, c_int, c_float, c_int, c_void_p],
@@ -1707,6 +1710,7 @@ def moe_grouped(x: torch.Tensor, weights: torch.Tensor, lists: tuple, pair_weigh
 
 FEWROWS_MAX_ROWS = 64          # float32 products of up to this many rows stream the weights,
 FEWROWS_GROUP = 16             # this many rows a pass over them
+FLOAT32_MAX_STRIDE = 1 << 22   # (offsets within a tile's rows are 32 bits)
 
 
 def fewrows_pays(m: int, n: int) -> bool:
@@ -1720,6 +1724,36 @@ def fewrows_pays(m: int, n: int) -> bool:
     if m >= 48:
         return n <= 4096
     return m < 24 or -(-n // 64) < 1024
+
+
+# What a float32 product is priced with, in microseconds: per tile (rows, columns) a stage of 32 k of a CU's only tile, of each
+# of several, and the start.  Fitted to 480 products (8 to 2,048 rows, 16 to 151,936 columns of 64 to 6,144, weights from memory)
+# within 1 to 2 % each, tiles of 32 x 32 13 %; the tile so chosen is the fastest of the five or at worst 5 % behind it.
+FLOAT32_PRICES = {(32, 32): (0.461, 0.183, 2.0), (64, 96): (0.918, 0.801, 3.0), (64, 128): (1.17, 1.033, 4.0),
+                  (96, 96): (1.272, 1.122, 4.0), (160, 64): (1.113, 1.425, 3.0)}
+
+
+def _float32_price(rows: int, columns: int, m: int, n: int, k: int) -> float:
+    only, each, start = FLOAT32_PRICES[rows, columns]
+    on_a_cu = -(-(-(-m // rows) * -(-n // columns)) // 256)
+    return start + -(-k // 32) * max(only, on_a_cu * each)
+
+
+@functools.lru_cache(maxsize=4096)
+def float32_tile(m: int, n: int, k: int) -> tuple[int, int]:
+    """(rows, columns) of the cheapest tile of ``gemm_float32``: by the tiles of the CU that has most of them."""
+    return min(FLOAT32_PRICES, key=lambda tile: _float32_price(*tile, m, n, k))
+
+
+@functools.lru_cache(maxsize=4096)
+def float32_tiles_pay(m: int, n: int, k: int) -> bool:
+    """Whether a float32 product of up to ``FEWROWS_MAX_ROWS`` rows takes tiles where ``fewrows_pays`` would stream the weights, once
+    for every 16 rows: where the passes (each the trips of K, or the weights at 5 TB/s) are priced well above the tiles, whose
+    price knows nothing of rows that meet in the same memory channels.  In recorded chains, weights from memory, us: 24 rows, 151,936 x
+    1,024 360 -> 157; 40, 1,024 x 6,144 27.6 -> 18.2 (12,288 x 2,048 66 -> 50; 4,096 x 2,048 stays, 28.2 against 44); 64, 1,024 x
+    1,024 23.2 -> 16.5, 512 x 1,024 22.3 -> 12.2 (2,048 x 6,144 stays, 87 against 126)."""
+    passes = -(-m // FEWROWS_GROUP) * max(4.0 + k / 350, 2.0 + n * k / 1.25e6)
+    return passes > 1.4 * _float32_price(*float32_tile(m, n, k), m, n, k)
 
 
 def fewrows_dealt(m: int, n: int) -> bool:
@@ -1766,7 +1800,8 @@ def fewrows_form(m: int, n: int, k: int, small_groups: bool | None = None) -> tu
 def gemm_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, fewrows_split: bool | None = None) -> None:
     """out[M, N] = a[M, K] @ w[N, K]^T, float32 multiply-add (rows may be strided).  float32
     operands of up to 64 rows go to the weight-streaming kernel where that pays
-    (``fewrows_pays``), which gives the same bits (``fewrows_split``: that kernel with operands split between as many pieces
+    (``fewrows_pays``, ``float32_tiles_pay``), others whose rows lie on 16-byte borders to tiles of a size that the product asks
+    for (csrc/gemm_float32.hip); all give the same bits (``fewrows_split``: that kernel with operands split between as many pieces
     of K as the rows allow, or not split; None chooses the kernel and the split by the shape)."""
     for t in (a, w, out):
         _need(t.is_cuda and t.dim() == 2 and t.stride(1) == 1, "gemm operands are 2-D GPU tensors with unit inner stride")
@@ -1776,9 +1811,10 @@ def gemm_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, fewrows_spli
     _need(a.dtype == w.dtype, "gemm inputs must share a dtype")
     _need(m <= 64 * 65535, "too many rows for one launch")
     _note(f"{m}x{n}x{k}", (n * k + m * k) * a.element_size() + m * n * out.element_size(), 2.0 * m * n * k)
-    if (m <= FEWROWS_MAX_ROWS and (fewrows_split is not None or fewrows_pays(m, n))
-            and a.dtype == torch.float32 and out.dtype == torch.float32 and k % 4 == 0 and k >= 4
-            and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+    on_borders = (a.dtype == torch.float32 and out.dtype == torch.float32 and k % 4 == 0 and k >= 4
+                  and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+    if on_borders and m <= FEWROWS_MAX_ROWS and (
+            fewrows_split is not None or (fewrows_pays(m, n) and (m <= FEWROWS_GROUP or not float32_tiles_pay(m, n, k)))):
         # the same sums in the same order, by a kernel that streams the weights
         for at in range(0, m, FEWROWS_GROUP):
             rows = min(FEWROWS_GROUP, m - at)
@@ -1786,6 +1822,10 @@ def gemm_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, fewrows_spli
                                                         out.stride(0), *fewrows_form(rows, n, k, fewrows_split),
                                                         int(fewrows_split is None and fewrows_dealt(rows, n)), _stream()),
                    "gemm_fewrows")
+        return
+    if on_borders and m > 0 and n > 0 and max(a.stride(0), w.stride(0)) <= FLOAT32_MAX_STRIDE:
+        _check(_fn("gemm_float32", "tk_gemm_float32")(_p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(0),
+                                                      *float32_tile(m, n, k), _stream()), "gemm_float32")
         return
     _check(_fn("gemm_tiled", "tk_gemm_tiled")(_code(a.dtype), _code(out.dtype), _p(a), _p(w), _p(out),
                                               m, n, k, a.stride(0), w.stride(0), out.stride(0),
