@@ -23,6 +23,7 @@
 //
 // Cache pages: K [nkv][hd/8][ps][8], V [nkv][vd/16][ps/4][16][4] (see elementwise.hip).
 #include "common.h"
+#include "lds_copy.h"
 #include "slots.h"
 
 using namespace tk;
@@ -59,12 +60,35 @@ __device__ __forceinline__ void load_eight(const bf16_t* p, float (&v)[8]) {
   }
 }
 
-// pieces of a key (8 dimensions each) asked for together: many for a query alone, whose walk
-// is a chain of memory round trips; few where eight queries share the key and the
+// The same as they lie in memory, for a query alone: a round's loads are held until they are used.
+typedef float f32x4 __attribute__((ext_vector_type(4)));     // (arrays of HIP's own vectors end up in scratch)
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+template <typename T> struct Held;
+template <> struct Held<float> {
+  struct Eight { f32x4 a, b; };
+  typedef f32x4 Four;
+  static __device__ __forceinline__ Eight eight(const float* p) { return {*reinterpret_cast<const f32x4*>(p), *reinterpret_cast<const f32x4*>(p + 4)}; }
+  static __device__ __forceinline__ Four four(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+  static __device__ __forceinline__ float at(const Eight& x, int e) { return e < 4 ? x.a[e] : x.b[e - 4]; }
+  static __device__ __forceinline__ float at(const Four& x, int e) { return x[e]; }
+};
+template <> struct Held<bf16_t> {
+  typedef u32x4 Eight;
+  typedef u32x2 Four;
+  static __device__ __forceinline__ Eight eight(const bf16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
+  static __device__ __forceinline__ Four four(const bf16_t* p) { return *reinterpret_cast<const u32x2*>(p); }
+  static __device__ __forceinline__ float half(uint32_t w, int e) { return __uint_as_float(e & 1 ? w & 0xffff0000u : w << 16); }
+  static __device__ __forceinline__ float at(const Eight& x, int e) { return half(x[e / 2], e); }
+  static __device__ __forceinline__ float at(const Four& x, int e) { return half(x[e / 2], e); }
+};
+
+// pieces of a key (8 dimensions each) asked for together where heads share it: few where eight queries do and the
 // multiply-adds fill the time (and the registers)
-template <int QT> constexpr int key_pieces() { return QT == 1 ? 8 : QT <= 4 ? 4 : 2; }
-// pieces of four values a lane asks for together
-template <int QT> constexpr int value_pieces() { return QT == 1 ? 8 : 4; }
+template <int QT> constexpr int key_pieces() { return QT <= 4 ? 4 : 2; }
+constexpr int kValuePieces = 4;      // of four values, that a lane asks for together there
+
+// What all lanes hold alike, as a scalar (conditions on it are then scalar work, not the vector unit's masks).
+__device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 struct GenericItems {
   const int* single;      // token rows that run alone (null: every token of the step does)
@@ -75,8 +99,9 @@ struct GenericItems {
 // QT: queries of a block; HEADS: they are heads of one group at one token (blockIdx.y is the kv
 // head, blockIdx.z the piece of the group), else tokens of one tile at one head (blockIdx.y).
 // SLOTS: value dimensions a lane owns (vd <= 64 * SLOTS).
-template <typename T, int QT, bool HEADS, int SLOTS>
-__global__ __launch_bounds__(kWaves * kWave) void paged_attention_generic_kernel(
+// MANY, of queries alone: more blocks than CUs, of which one then holds two (half of the registers a wave).
+template <typename T, int QT, bool HEADS, int SLOTS, bool MANY = false>
+__global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(MANY ? 4 : 2))) void paged_attention_generic_kernel(
     const T* __restrict__ q, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
     const int* __restrict__ block_tables, const int* __restrict__ positions,
     const int* __restrict__ req_of_token, GenericItems items, T* __restrict__ out, int nh, int nkv,
@@ -88,22 +113,22 @@ __global__ __launch_bounds__(kWaves * kWave) void paged_attention_generic_kernel
   __shared__ float acc_s[kWaves][kMaxHd];
 
   const int tid = threadIdx.x;
-  const int lane = tid & (kWave - 1), wave = tid / kWave;
+  const int lane = tid & (kWave - 1), wave = scalar(tid / kWave);
   const int group = nh / nkv;
   int n0, cnt, head0, kvh;
   if (HEADS) {
-    n0 = items.single ? items.single[blockIdx.x] : (int)blockIdx.x;
+    n0 = items.single ? scalar(items.single[blockIdx.x]) : (int)blockIdx.x;
     kvh = blockIdx.y;
     head0 = kvh * group + blockIdx.z * QT;
     cnt = min(QT, group - (int)blockIdx.z * QT);
   } else {
-    n0 = items.tile_first[blockIdx.x] + blockIdx.z * QT;
-    cnt = min(QT, items.tile_count[blockIdx.x] - (int)blockIdx.z * QT);
+    n0 = scalar(items.tile_first[blockIdx.x]) + blockIdx.z * QT;
+    cnt = min(QT, scalar(items.tile_count[blockIdx.x]) - (int)blockIdx.z * QT);
     head0 = blockIdx.y;
     kvh = head0 / group;
   }
   if (cnt <= 0) return;
-  const int* table = block_tables + (size_t)req_of_token[n0] * max_pages;
+  const int* table = block_tables + (size_t)scalar(req_of_token[n0]) * max_pages;
   // query t: its row of q and out, its position and the first key it sees
   size_t row[QT];
   int pos[QT], first[QT];
@@ -111,7 +136,7 @@ __global__ __launch_bounds__(kWaves * kWave) void paged_attention_generic_kernel
   for (int t = 0; t < QT; ++t) {
     const int u = min(t, cnt - 1);
     row[t] = HEADS ? (size_t)n0 * nh + head0 + u : (size_t)(n0 + u) * nh + head0;
-    pos[t] = positions[HEADS ? n0 : n0 + u];
+    pos[t] = scalar(positions[HEADS ? n0 : n0 + u]);
     first[t] = span > 0 ? (pos[t] - span + 1 > 0 ? pos[t] - span + 1 : 0) : span < 0 ? pos[t] - pos[t] % (-span) : 0;
   }
   const int lo = first[0], hi = pos[QT - 1];  // positions ascend within a tile
@@ -144,18 +169,58 @@ __global__ __launch_bounds__(kWaves * kWave) void paged_attention_generic_kernel
     float dot[QT];
 #pragma unroll
     for (int t = 0; t < QT; ++t) dot[t] = 0.f;
+    // A query alone is a chain of trips to memory: a round's keys (of float32 half of them) and the values of its first dimensions are asked
+    // for together, the values of the next ones behind the keys' products, and only then comes the softmax (four requests of up to 600 keys, heads of 128, float32
+    // 20.9 -> 14.1 us, bfloat16 20.2 -> 13.4; of 2,048 keys 51 -> 34, 48 -> 31).
+    constexpr bool ALONE = HEADS && QT == 1;
+    constexpr int BUFFERS = MANY ? 1 : 2;
+    typename Held<T>::Four held_v[ALONE ? BUFFERS : 1][kWave / 4];
+    unsigned long quad = 0, seen = 0;      // where the values of this lane's key and its three neighbours lie; the round's keys that are seen
+    const auto ask_values = [&](int slot, int buffer) {
+      const int d = min(lane + slot * kWave, vd - 1);      // (a dimension past the head's is another one's, and not used)
+      const uint32_t v_dim_off = (uint32_t)(d >> 4) * (ps >> 2) * 64 + (d & 15) * 4;
+#pragma unroll
+      for (int u = 0; u < kWave / 4; ++u) {      // (the same for all lanes: scalars)
+        const uint32_t low = __builtin_amdgcn_readlane((uint32_t)quad, 4 * u), high = __builtin_amdgcn_readlane((uint32_t)(quad >> 32), 4 * u);
+        held_v[buffer][u] = Held<T>::four(v_cache + (((unsigned long)high << 32) | low) + v_dim_off);
+      }
+    };
+    if constexpr (ALONE) {
+      constexpr int kHeldPieces = 32 / sizeof(T) / (MANY ? 2 : 1);      // of a key, eight dimensions each: 64 registers (MANY 32)
+      // (a lane whose key and its three neighbours nobody sees, whose page may be another's, takes the last key and does not use it)
+      const int there = c <= hi && ((c | 3) >= lo || c < keep) ? c : hi, page = table[there / ps];
+      const T* const kp = k_cache + (size_t)page * page_elems + head_off + (size_t)(there % ps) * 8;
+      seen = __ballot(loaded);
+      quad = (size_t)page * v_page_elems + v_head_off + (size_t)((there % ps) >> 2) * 64;
+      const int pieces = hd / 8;
+      for (int j0 = 0; j0 < pieces; j0 += kHeldPieces) {
+        typename Held<T>::Eight held_k[kHeldPieces];
+#pragma unroll
+        for (int u = 0; u < kHeldPieces; ++u) held_k[u] = Held<T>::eight(kp + (size_t)min(j0 + u, pieces - 1) * ps * 8);
+        if (!MANY && j0 == 0) ask_values(0, 0);
+#pragma unroll
+        for (int u = 0; u < kHeldPieces; ++u)
+          if (j0 + u < pieces) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dot[0] = fmaf(q_s[0][(j0 + u) * 8 + e], Held<T>::at(held_k[u], e), dot[0]);
+          }
+      }
+      __builtin_amdgcn_sched_barrier(0);      // (the registers of the keys)
+      if (MANY) ask_values(0, 0);
+      else if (SLOTS > 1 && kWave < vd) ask_values(1, 1);
+    }
     // Tokens that run alone (decode) are bound by round trips to memory, not by arithmetic: they
     // ask for eight pieces of a key at once and for the values of four keys in one piece (four
     // such pieces at once).  Tiles of a prompt portion, eight queries to a key, are bound by
     // their multiply-adds and keep the plain loops.  The order of every sum is the same.
     constexpr bool BATCHED = HEADS;
     long vbase = -1;
-    if (BATCHED && (lane & 3) == 0 && c <= hi && (c + 3 >= lo || c < keep)) {
+    if (BATCHED && !ALONE && (lane & 3) == 0 && c <= hi && (c + 3 >= lo || c < keep)) {
       // the values of four consecutive keys of a dimension are one piece of a page
       const int page = table[c / ps];
       vbase = (long)((size_t)page * v_page_elems + v_head_off + (size_t)((c % ps) >> 2) * 64);
     }
-    if (loaded) {
+    if (!ALONE && loaded) {
       const int page = table[c / ps];
       const int off = c % ps;
       const T* kp = k_cache + (size_t)page * page_elems + head_off;
@@ -213,7 +278,7 @@ __global__ __launch_bounds__(kWaves * kWave) void paged_attention_generic_kernel
 #pragma unroll
     for (int t = 0; t < QT; ++t) p_s[wave][lane][t] = p[t];
     if (!BATCHED) base_s[wave][lane] = vbase;
-    else if ((lane & 3) == 0) base_s[wave][lane >> 2] = vbase;
+    else if (!ALONE && (lane & 3) == 0) base_s[wave][lane >> 2] = vbase;
     wave_lds_sync();
     const int count = (hi - c0 + 1 < kWave) ? hi - c0 + 1 : kWave;
 #pragma unroll
@@ -224,11 +289,26 @@ __global__ __launch_bounds__(kWaves * kWave) void paged_attention_generic_kernel
         float a[QT];
 #pragma unroll
         for (int t = 0; t < QT; ++t) a[t] = acc[i][t] * alpha[t];
-        if constexpr (BATCHED) {
-          // four keys a load (16 bytes of float32) and four such loads, for a query alone eight, asked for together, added
+        if constexpr (ALONE) {
+          // (bit k of `seen`: key k of the round is one that somebody sees; it is asked for in scalars)
+          const auto add = [&](auto ALL) {
+#pragma unroll
+            for (int u = 0; u < kWave / 4; ++u) {
+              const f32x4 p4 = *reinterpret_cast<const f32x4*>(&p_s[wave][4 * u][0]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float v = Held<T>::at(held_v[i % BUFFERS][u], e);
+                a[0] = fmaf(p4[e], decltype(ALL)::value || (seen >> (4 * u + e) & 1) ? v : 0.f, a[0]);
+              }
+            }
+          };
+          if (seen == ~0ul) add(std::true_type{});
+          else add(std::false_type{});
+        } else if constexpr (BATCHED) {
+          // four keys a load (16 bytes of float32) and four such loads asked for together, added
           // key by key in ascending order: the same sums as one key at a time.  A key out of
           // range adds a probability times 0.
-          constexpr int kPieces = value_pieces<QT>();
+          constexpr int kPieces = kValuePieces;
           for (int quad0 = 0; quad0 * 4 < count; quad0 += kPieces) {
             float v4[kPieces][4];
             bool there[kPieces];
@@ -263,6 +343,7 @@ __global__ __launch_bounds__(kWaves * kWave) void paged_attention_generic_kernel
 #pragma unroll
         for (int t = 0; t < QT; ++t) acc[i][t] = a[t];
       }
+      if (ALONE && i + BUFFERS < SLOTS && (i + BUFFERS) * kWave < vd) ask_values(i + BUFFERS, i % BUFFERS);
     }
   }
   // merge, one query after the other: a wave that had no round of the query's brings
@@ -301,6 +382,253 @@ __global__ __launch_bounds__(kWaves * kWave) void paged_attention_generic_kernel
   }
 }
 
+// Tiles of a float32 prompt portion on the matrix cores (heads of 64 or 128, pages of whole 16s of keys): the sums of the kernel above in the
+// same order, bit for bit, by
+// v_mfma_f32_16x16x4_f32, which gives the bits of fmaf over its four k in ascending order.  A wave multiplies its round's 64 keys by
+// the tile's 16 tokens at H heads of a group (scores: rows keys, columns tokens; output: rows dimensions), so a number loaded from a
+// page meets H times 16 queries, where the kernel above has eight multiply-adds for it.  The matrix unit waits for every vector
+// instruction of the wave, so operands come as they are multiplied, at scalar addresses and a lane's fixed place.  16 query heads over 8 kv
+// heads of 128, us: 1,053 tokens of four requests 236 -> 88, one prompt of 1,024 316 -> 108, of 2,048 865 -> 296, 1,024 behind 1,024
+// 652 -> 198 (with keys as 4-byte loads of operands 236 -> 126, 874 -> 548).  What is left: the waves of a block have unlike numbers
+// of rounds, and a block has its CU to itself.
+template <int HD, int H>
+__global__ __launch_bounds__(kWaves * kWave) void attention_float32_tiles_kernel(
+    const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache, const int* __restrict__ block_tables,
+    const int* __restrict__ positions, const int* __restrict__ req_of_token, GenericItems items, float* __restrict__ out, int nh, int nkv,
+    int ps, int max_pages, float scale, int span, int keep, const float* __restrict__ sinks, float cap) {
+  constexpr int STEPS = HD / 4, DIMS = HD / 16, KEYS = kWave / 16;      // products of a score, 16s of dimensions and of a round's keys
+  constexpr int OWN = kWave * 32, SUMS = kWaves * kTileTokens * (HD + 4);
+  static_assert(H * kTileTokens <= 32, "the probabilities take no more room than the keys");
+  __shared__ __attribute__((aligned(16))) float shared_s[kWaves * OWN > SUMS ? kWaves * OWN : SUMS];
+  __shared__ float q_s[H * STEPS * kWave], m_s[kWaves][kTileTokens], l_s[kWaves][kTileTokens];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave), a = lane & 15, g = lane >> 4;
+  const int tile = (int)gridDim.x - 1 - (int)blockIdx.x;      // (the list is shortest walk first)
+  const int n0 = scalar(items.tile_first[tile]), cnt = min(kTileTokens, scalar(items.tile_count[tile]));
+  if (cnt <= 0) return;
+  const int head0 = blockIdx.y * H, kvh = head0 / (nh / nkv);
+  const int* const table = block_tables + (size_t)scalar(req_of_token[n0]) * max_pages;
+  // this lane's token: its position and the first key it sees (tokens of a tile are consecutive)
+  const int pos0 = scalar(positions[n0]), pos = pos0 + min(a, cnt - 1), hi = pos0 + cnt - 1;
+  const auto first_of = [&](int at) { return span > 0 ? (at - span + 1 > 0 ? at - span + 1 : 0) : span < 0 ? at - at % (-span) : 0; };
+  const int first = first_of(pos), lo = first_of(pos0);
+  const size_t page_elems = (size_t)nkv * HD * ps;
+  const float* const k_head = k_cache + (size_t)kvh * HD * ps;
+  const float* const v_head = v_cache + (size_t)kvh * HD * ps;
+
+  // the queries as an operand, [head][step of four dimensions s][lane]: column a, dimension 4 s + g
+  for (int at = tid; at < H * STEPS * kWave; at += kWaves * kWave) {
+    const int column = at & 15, d = at / kWave % STEPS * 4 + (at >> 4 & 3), h = at / (kWave * STEPS);
+    q_s[at] = q[((size_t)(n0 + min(column, cnt - 1)) * nh + head0 + h) * HD + d] * scale;
+  }
+  __syncthreads();
+  float m[H], l[H];
+  float4v acc[H][DIMS];      // [.][i][e]: dimension 16 i + 4 g + e of column a
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    m[h] = -INFINITY;
+    l[h] = 0.f;
+#pragma unroll
+    for (int i = 0; i < DIMS; ++i) acc[h][i] = float4v{0.f, 0.f, 0.f, 0.f};
+  }
+  // a wave's own: 32 dimensions of a round's keys, then the round's probabilities
+  float* const mine = shared_s + wave * OWN;
+  const uint32_t key_place = (uint32_t)(lane >> 5) * ps * 8 + (lane & 31) * 4;
+
+  const int round0 = keep > 0 ? 0 : lo / kWave;
+  for (int rd = round0 + (wave - round0 % kWaves + kWaves) % kWaves; rd * kWave <= hi; rd += kWaves) {
+    const int c0 = rd * kWave;
+    if (c0 >= keep && c0 + kWave - 1 < lo) continue;
+    int page[KEYS], off[KEYS];      // of each 16 keys (of 16 that nobody sees, whose page may be another's: the last key's)
+#pragma unroll
+    for (int t = 0; t < KEYS; ++t) {
+      const int at = c0 + 16 * t, c = at <= hi && (at + 15 >= lo || at < keep) ? at : hi & ~15;
+      page[t] = scalar(table[c / ps]);
+      off[t] = c % ps;
+    }
+    // Operands, asked for while the ones before are multiplied: 32 dimensions of the round's keys, 16 bytes a lane (what an
+    // operand takes, 16 of 32 bytes of every key, the vector memory path serves at a quarter of its rate) and through the wave's own LDS, then
+    // 16 keys of all dimensions of the values, 256 bytes a load.
+    constexpr int GROUPS = HD / 32;
+    static_assert(GROUPS % 2 == 0 && DIMS <= 8, "values take the first of two sets of registers; 16 keys of a head are a set");
+    float4v held[2][8];
+    const auto ask_keys = [&](int group) {
+#pragma unroll
+      for (int t = 0; t < KEYS; ++t) {
+        const float* const base = k_head + (size_t)page[t] * page_elems + (size_t)off[t] * 8;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) held[group & 1][2 * t + j] = *reinterpret_cast<const float4v*>(base + (size_t)(4 * group + 2 * j) * ps * 8 + key_place);
+      }
+    };
+    const auto ask_values = [&](int t) {
+      const float* const base = v_head + (size_t)page[t] * page_elems + (size_t)(off[t] >> 2) * 64;
+#pragma unroll
+      for (int i = 0; i < DIMS; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) held[t & 1][i][s] = base[(size_t)i * (ps >> 2) * 64 + s * 64 + (uint32_t)(a * 4 + g)];
+    };
+    float4v sc[H][KEYS];      // [.][t][e]: key 16 t + 4 g + e
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int t = 0; t < KEYS; ++t) sc[h][t] = float4v{0.f, 0.f, 0.f, 0.f};
+    ask_keys(0);
+#pragma unroll
+    for (int group = 0; group < GROUPS; ++group) {
+      wave_lds_sync();      // (the group before has been read, and the round before's probabilities)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) *reinterpret_cast<float4v*>(mine + i * 256 + lane * 4) = held[group & 1][i];
+      if (group + 1 < GROUPS) ask_keys(group + 1);
+      else ask_values(0);
+      wave_lds_sync();
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        float kr[KEYS];      // key 16 t + a, dimension 32 group + 4 s + g
+#pragma unroll
+        for (int t = 0; t < KEYS; ++t) kr[t] = mine[t * 512 + (s / 2) * 128 + a * 8 + 4 * (s & 1) + g];
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+          const float qr = q_s[(h * STEPS + 8 * group + s) * kWave + lane];
+#pragma unroll
+          for (int t = 0; t < KEYS; ++t) sc[h][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[t], qr, sc[h][t], 0, 0, 0);
+        }
+      }
+    }
+    // a round that holds none of the token's keys leaves its sums as they are
+    const bool takes = c0 <= pos && (c0 + kWave - 1 >= first || c0 < keep);
+    const auto sees = [&](int c) { return takes && (c >= first || c < keep) && c <= pos; };
+    float alpha[H];
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      float top = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < KEYS; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = c0 + 16 * t + 4 * g + e;
+          if (cap > 0.f) sc[h][t][e] = cap * tanhf(sc[h][t][e] / cap);
+          top = fmaxf(top, sees(c) ? sc[h][t][e] : -INFINITY);
+        }
+      const float m_new = fmaxf(m[h], max32(max16(top)));
+      float part[KEYS];      // the sum over the wave's keys, pairs of neighbours first, as lanes of a wave are added
+#pragma unroll
+      for (int t = 0; t < KEYS; ++t) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float weight = expf(sc[h][t][e] - m_new);
+          sc[h][t][e] = sees(c0 + 16 * t + 4 * g + e) ? weight : 0.f;
+        }
+        part[t] = sum32(sum16((sc[h][t][0] + sc[h][t][1]) + (sc[h][t][2] + sc[h][t][3])));
+      }
+      static_assert(KEYS == 4, "four 16s of keys a round");
+      alpha[h] = 1.f;
+      if (takes) {
+        alpha[h] = expf(m[h] - m_new);
+        l[h] = l[h] * alpha[h] + ((part[0] + part[1]) + (part[2] + part[3]));
+        m[h] = m_new;
+      }
+    }
+    wave_lds_sync();      // the keys have been read
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int t = 0; t < KEYS; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mine[(h * kWave + 16 * t + 4 * g + e) * kTileTokens + a] = sc[h][t][e];
+    wave_lds_sync();
+    const bool whole = (c0 >= lo || c0 + kWave <= keep) && c0 + kWave - 1 <= hi;      // no key of the round is another's or none
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int i = 0; i < DIMS; ++i) acc[h][i] *= alpha[h];
+#pragma unroll
+    for (int t = 0; t < KEYS; ++t) {
+      float pr[H][4];      // column a, key 16 t + 4 s + g
+#pragma unroll
+      for (int h = 0; h < H; ++h)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) pr[h][s] = mine[(h * kWave + 16 * t + 4 * s) * kTileTokens + lane];
+      if (t + 1 < KEYS) ask_values(t + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (!whole) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int c = c0 + 16 * t + 4 * s + g;
+          const bool in = (c >= lo || c < keep) && c <= hi;
+#pragma unroll
+          for (int i = 0; i < DIMS; ++i) held[t & 1][i][s] = in ? held[t & 1][i][s] : 0.f;
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < DIMS; ++i)
+#pragma unroll
+          for (int h = 0; h < H; ++h) acc[h][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(held[t & 1][i][s], pr[h][s], acc[h][i], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // merge in wave order, a head after the other
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    __syncthreads();
+    if (g == 0) {
+      m_s[wave][a] = m[h];
+      l_s[wave][a] = l[h];
+    }
+#pragma unroll
+    for (int i = 0; i < DIMS; ++i)
+      *reinterpret_cast<float4v*>(&shared_s[(wave * kTileTokens + a) * (HD + 4) + 16 * i + 4 * g]) = acc[h][i];
+    __syncthreads();
+    // every wave's weight and the whole sum once a token, then the dimensions
+    if (tid < kTileTokens) {
+      const float sink = sinks ? sinks[head0 + h] : -INFINITY;
+      float top = m_s[0][tid];
+#pragma unroll
+      for (int w = 1; w < kWaves; ++w) top = fmaxf(top, m_s[w][tid]);
+      top = fmaxf(top, sink);
+      float sum = 0.f;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        const float e = expf(m_s[w][tid] - top);
+        sum = fmaf(l_s[w][tid], e, sum);
+        m_s[w][tid] = e;
+      }
+      l_s[0][tid] = sinks ? sum + expf(sink - top) : sum;
+    }
+    __syncthreads();
+    for (int at = tid; at < cnt * HD; at += kWaves * kWave) {
+      const int t = at / HD, d = at % HD;
+      float o = 0.f;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) o = fmaf(shared_s[(w * kTileTokens + t) * (HD + 4) + d], m_s[w][t], o);
+      out[((size_t)(n0 + t) * nh + head0 + h) * HD + d] = o / l_s[0][t];
+    }
+  }
+}
+
+// Whether a portion's tiles took that kernel.
+template <typename T>
+static bool launch_float32_tiles(const T*, const T*, const T*, const int*, const int*, const int*, GenericItems, int, T*, int, int, int, int, int,
+                                 int, float, int, int, const float*, float, hipStream_t) {
+  return false;
+}
+template <>
+bool launch_float32_tiles<float>(const float* q, const float* k_cache, const float* v_cache, const int* block_tables, const int* positions,
+                                 const int* req_of_token, GenericItems items, int num_tiles, float* out, int nh, int nkv, int hd, int vd,
+                                 int ps, int max_pages, float scale, int span, int keep, const float* sinks, float cap, hipStream_t stream) {
+  if (hd != vd || (hd != 64 && hd != 128) || ps % 16 != 0) return false;
+  const bool pairs = nh / nkv % 2 == 0;
+#define TK_TILES(HD_, H_)                                                                                                   \
+  attention_float32_tiles_kernel<HD_, H_><<<dim3(num_tiles, nh / H_), kWaves * kWave, 0, stream>>>(                          \
+      q, k_cache, v_cache, block_tables, positions, req_of_token, items, out, nh, nkv, ps, max_pages, scale, span, keep, sinks, cap)
+  if (hd == 64 && pairs) TK_TILES(64, 2);
+  else if (hd == 64) TK_TILES(64, 1);
+  else if (pairs) TK_TILES(128, 2);
+  else TK_TILES(128, 1);
+#undef TK_TILES
+  return true;
+}
+
 template <typename T, int SLOTS>
 static void launch_generic(const T* q, const T* k_cache, const T* v_cache, const int* block_tables,
                            const int* positions, const int* req_of_token, GenericItems items,
@@ -308,23 +636,26 @@ static void launch_generic(const T* q, const T* k_cache, const T* v_cache, const
                            int max_pages, float scale, int span, int keep, int share_heads, const float* sinks,
                            float cap, hipStream_t stream) {
   const int group = nh / nkv;
-#define TK_ALONE(QT_)                                                                               \
-  paged_attention_generic_kernel<T, QT_, true, SLOTS>                                               \
+#define TK_ALONE(QT_, MANY_)                                                                        \
+  paged_attention_generic_kernel<T, QT_, true, SLOTS, MANY_>                                        \
       <<<dim3(num_single, nkv, (group + QT_ - 1) / QT_), kWaves * kWave, 0, stream>>>(              \
           q, k_cache, v_cache, block_tables, positions, req_of_token, items, out, nh, nkv, hd, vd,  \
           ps, max_pages, scale, span, keep, sinks, cap)
   if (num_single > 0) {
-    // the heads of a group share a block if that still gives every CU one (the result is the
-    // same either way): at batch 64 of an 8B-shaped layer a third faster, at batch 8 slower
+    // The heads of a group share a block (the result is the same either way) where each in a block of its own would be more blocks
+    // than two a CU and some, us alone and shared: bfloat16, 300 and 1,100 keys, 32 requests of 16 heads over 8 kv heads 15.5 | 20.4 and
+    // 40.9 | 52.3, 40 requests 23.4 | 24.2 and 61.2 | 60.6, 48 28.1 | 24.6 and 69 | 62, 64 of 16 over 4 27.7 | 21.8 and 83 | 54;
+    // float32, whose keys are twice the bytes, 24 15.4 | 21.3 and 54 | 55, 32 18.4 | 22.6 and 80 | 67, 48 36 | 28 and 133 | 97.
     const int qt = group <= 4 ? 4 : kQueries;
-    const bool shared = group > 1 && (share_heads < 0 ? (long)num_single * nkv * ((group + qt - 1) / qt) >= 256
-                                                      : share_heads > 0);
-    if (!shared) TK_ALONE(1);
-    else if (qt == 4) TK_ALONE(4);
-    else TK_ALONE(kQueries);
+    const bool shared = group > 1 && (share_heads < 0 ? (long)num_single * nh > (sizeof(T) == 4 ? 511 : 640) : share_heads > 0);
+    if (!shared && (long)num_single * nh > 256) TK_ALONE(1, true);
+    else if (!shared) TK_ALONE(1, false);
+    else if (qt == 4) TK_ALONE(4, false);
+    else TK_ALONE(kQueries, false);
   }
 #undef TK_ALONE
-  if (num_tiles > 0)
+  if (num_tiles > 0 && !launch_float32_tiles<T>(q, k_cache, v_cache, block_tables, positions, req_of_token, items, num_tiles, out, nh, nkv,
+                                                hd, vd, ps, max_pages, scale, span, keep, sinks, cap, stream))
     paged_attention_generic_kernel<T, kQueries, false, SLOTS>
         <<<dim3(num_tiles, nh, kTileTokens / kQueries), kWaves * kWave, 0, stream>>>(
             q, k_cache, v_cache, block_tables, positions, req_of_token, items, out, nh, nkv, hd, vd, ps,
