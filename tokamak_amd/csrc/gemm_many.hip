@@ -17,6 +17,10 @@
 // 6,144 x 1,024 at 256 / 1,024 / 2,048 rows 15.1 / 33.1 / 35.5, here 11.9 / 18.5 / 28.6.  In shares of K, with what the sums cost
 // their reader, beside the library's first choice: 4,096 x 12,288 at 200 / 512 / 1,024 rows 45 / 75 / 106, here 37 / 55 / 93; 2,560 x
 // 9,728 32 / 46 / 62, here 26 / 36 / 53; 5,120 x 17,408 226 / 168 / 246, here 57 / 90 / 149.
+//
+// Several products of one shape (a time mix's four projections) are one list of tiles: one alone is 64 to 256 tiles, a part of a round
+// or one that ends unevenly.  Four of 4,096 x 4,096 at 129 / 512 / 1,000 / 2,048 rows, us: the library's launches 91 / 123 / 164 / 241, here 44
+// / 59 / 96 / 184 (1.50 PFLOP/s).
 #include "common.h"
 #include "gate.h"
 #include "lds_copy.h"
@@ -26,7 +30,7 @@ using namespace tk;
 
 namespace {
 
-enum { EPI_PARTS, EPI_SILU, EPI_CLAMPED, EPI_GELU };     // the last three: gated
+enum { EPI_PARTS, EPI_SILU, EPI_CLAMPED, EPI_GELU, EPI_SEVERAL };     // the three in the middle: gated; SEVERAL: independent products, bfloat16
 
 constexpr int kCus = 256;       // blocks that run at once
 constexpr int kXcds = 8;        // dies, each with an L2 of its own; blocks go to them in turn
@@ -37,8 +41,9 @@ struct Job {
   void* c;
   int M, N, K;
   long lda, ldw, ldc, part_stride;
-  int tiles_m, tiles_n, parts;
-  float limit;      // of the clamped gate
+  int tiles_m, tiles_n, parts;      // parts: shares of K, or products (EPI_SEVERAL)
+  float limit;                      // of the clamped gate
+  long a_next, w_next;              // EPI_SEVERAL: from a product's operands to the next one's (part_stride: of the results)
 };
 
 template <int EPI>
@@ -67,7 +72,7 @@ constexpr int blocks_a_cu(int mt, int nt) { return mt * nt <= 4 ? 2 : 1; }
 template <int MT, int NT, int EPI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(blocks_a_cu(MT, NT), blocks_a_cu(MT, NT)))) void gemm_many_kernel(Job job) {
   constexpr int kSlots = kCus * blocks_a_cu(MT, NT);      // blocks that run at once
-  constexpr bool GATED = EPI >= EPI_SILU;
+  constexpr bool GATED = EPI == EPI_SILU || EPI == EPI_CLAMPED || EPI == EPI_GELU, SEVERAL = EPI == EPI_SEVERAL;
   constexpr int BM = 64 * MT, BN = 64 * NT, OUT = GATED ? BN / 2 : BN;   // OUT: output channels of a tile
   constexpr uint32_t WB = BN * 128, XB = BM * 128, WRING = 3 * WB, XRING = 2 * XB;
   extern __shared__ __attribute__((aligned(1024))) unsigned char many_lds[];
@@ -87,11 +92,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(blocks_a_cu
     tm = tile - tn * job.tiles_m;
   };
   uint32_t xo[2 * MT], wo[2 * NT];
-  const auto begin = [&](Cursor& c, int part, const bf16_t* rows) {
-    const int first = (int)((unsigned)(part * all_steps) / (unsigned)job.parts);
-    c.steps = (int)((unsigned)((part + 1) * all_steps) / (unsigned)job.parts) - first;
+  const auto begin = [&](Cursor& c, int part, const bf16_t* rows, long next) {
+    const int first = SEVERAL ? 0 : (int)((unsigned)(part * all_steps) / (unsigned)job.parts);
+    c.steps = SEVERAL ? all_steps : (int)((unsigned)((part + 1) * all_steps) / (unsigned)job.parts) - first;
     c.step = 0;
-    c.base = reinterpret_cast<const char*>(rows + first * kStep);
+    c.base = reinterpret_cast<const char*>(rows + (SEVERAL ? part * next : (long)first * kStep));
   };
   const auto aim_x = [&](Cursor& c) {
     int tm, tn, part;
@@ -100,7 +105,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(blocks_a_cu
 #pragma unroll
     for (int j = 0; j < 2 * MT; ++j)
       xo[j] = (uint32_t)min(8 * (4 * j + wave) + (at >> 3), job.M - 1 - m0) * (uint32_t)(job.lda * 2) + piece * 16;
-    begin(c, part, job.a + (size_t)m0 * job.lda);
+    begin(c, part, job.a + (size_t)m0 * job.lda, job.a_next);
   };
   const auto aim_w = [&](Cursor& c) {
     int tm, tn, part;
@@ -116,7 +121,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(blocks_a_cu
       }
       wo[j] = (uint32_t)from * (uint32_t)(job.ldw * 2) + piece * 16;
     }
-    begin(c, part, job.w + (size_t)n0 * job.ldw);
+    begin(c, part, job.w + (size_t)n0 * job.ldw, job.w_next);
   };
   const auto next_w = [](uint32_t s) { return s == WRING - WB ? 0u : s + WB; };
   const auto next_x = [](uint32_t s) { return s == WRING ? WRING + XB : WRING; };
@@ -166,7 +171,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(blocks_a_cu
   for (int unit = blockIdx.x; unit < total; unit += gridDim.x) {
     int tm, tn, part;
     place(unit, tm, tn, part);
-    const int steps = (int)((unsigned)((part + 1) * all_steps) / (unsigned)job.parts) - (int)((unsigned)(part * all_steps) / (unsigned)job.parts);
+    const int steps = SEVERAL ? all_steps
+                              : (int)((unsigned)((part + 1) * all_steps) / (unsigned)job.parts) - (int)((unsigned)(part * all_steps) / (unsigned)job.parts);
     float4v acc[2 * NT][2 * MT];
 #pragma unroll
     for (int i = 0; i < 2 * NT; ++i)
@@ -228,7 +234,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(blocks_a_cu
           *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
           *reinterpret_cast<float4*>(dst + 4) = make_float4(v[4], v[5], v[6], v[7]);
         } else {
-          *reinterpret_cast<uint4*>(static_cast<bf16_t*>(job.c) + (size_t)m * job.ldc + n) =
+          *reinterpret_cast<uint4*>(static_cast<bf16_t*>(job.c) + (SEVERAL ? part * job.part_stride : 0) + (size_t)m * job.ldc + n) =
               make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
         }
       }
@@ -239,7 +245,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(blocks_a_cu
 
 template <int MT, int NT, int EPI>
 int launch(Job job, hipStream_t stream) {
-  constexpr int BM = 64 * MT, OUT = EPI >= EPI_SILU ? 32 * NT : 64 * NT, bytes = (3 * NT + 2 * MT) * 64 * 128;
+  constexpr int BM = 64 * MT, OUT = EPI == EPI_PARTS || EPI == EPI_SEVERAL ? 64 * NT : 32 * NT, bytes = (3 * NT + 2 * MT) * 64 * 128;
   static bool raised[64] = {};      // (the attribute belongs to a function on a device)
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -1;
@@ -274,7 +280,7 @@ TK_API int tk_gemm_many(int mode, const void* A, const void* W, void* C, int M, 
   if (parts < 1 || parts > K / kStep || (mode != EPI_PARTS && parts != 1)) return -1;
   // offsets within a tile are 32 bits
   if (lda < K || ldw < K || lda * 2 * 256 > 0xffffffffL || ldw * 2 * ((gate ? (long)N : 0) + 256) > 0xffffffffL) return -1;
-  const Job job{(const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, part_stride, 0, 0, parts, limit};
+  const Job job{(const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, part_stride, 0, 0, parts, limit, 0, 0};
 #define TK_SHAPE(MT_, NT_)                                                             \
   if (rows == 64 * MT_ && columns == 64 * NT_) {                                       \
     if (mode == EPI_PARTS) return launch<MT_, NT_, EPI_PARTS>(job, stream);            \
@@ -290,4 +296,24 @@ TK_API int tk_gemm_many(int mode, const void* A, const void* W, void* C, int M, 
   return -1;
 }
 
+// `count` products of one shape: C_i[M, N] bfloat16 = A_i W_i^T, the operands and results a_next, w_next and c_next numbers apart.
+TK_API int tk_gemm_several(const void* A, const void* W, void* C, int M, int N, int K, long lda, long ldw, long ldc, int count, long a_next,
+                           long w_next, long c_next, int rows, int columns, hipStream_t stream) {
+  if (M <= 0 || N <= 0 || count <= 0) return 0;
+  if (K < kStep || K % kStep != 0 || N % 8 != 0 || lda % 8 != 0 || ldw % 8 != 0 || ldc % 8 != 0) return -1;
+  if ((((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15) || a_next % 8 != 0 || w_next % 8 != 0 || c_next % 8 != 0 || count > 64) return -1;
+  // offsets within a tile are 32 bits
+  if (lda < K || ldw < K || lda * 2 * 256 > 0xffffffffL || ldw * 2 * 256 > 0xffffffffL) return -1;
+  const Job job{(const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldw, ldc, c_next, 0, 0, count, 0.f, a_next, w_next};
+#define TK_SHAPE(MT_, NT_) \
+  if (rows == 64 * MT_ && columns == 64 * NT_) return launch<MT_, NT_, EPI_SEVERAL>(job, stream);
+  TK_SHAPE(4, 4)
+  TK_SHAPE(2, 4)
+  TK_SHAPE(4, 2)
+  TK_SHAPE(2, 2)
+#undef TK_SHAPE
+  return -1;
+}
+
 TK_SLOTS(tk_gemm_many)
+TK_SLOTS(tk_gemm_several)

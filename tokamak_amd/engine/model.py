@@ -12,7 +12,7 @@ from tokamak_amd.config.registry import get_part
 from tokamak_amd.engine import layer_replay
 from tokamak_amd.kernels import ops
 from tokamak_amd.kernels.linear import Added
-from tokamak_amd.parts.base import Block, CacheRequest, Part, StateArray
+from tokamak_amd.parts.base import Block, CacheRequest, Mixer, Part, StateArray
 from tokamak_amd.weights.spec import TensorSpec
 
 
@@ -103,9 +103,9 @@ class LayeredModel:
             self.head.tie(self.embedding)
 
     def matrix_shapes(self, dtype: torch.dtype) -> set[tuple[int, int]]:
-        """The (rows, columns) of the parts' matrices of a type."""
-        return {tuple(t.shape) for part in self._all_parts() for t in vars(part).values()
-                if isinstance(t, torch.Tensor) and t.dim() == 2 and t.dtype == dtype}
+        """The (rows, columns) of the parts' matrices of a type, of those that lie together (a mixer's) of each."""
+        return {tuple(t.shape[-2:]) for part in self._all_parts() for t in vars(part).values()
+                if isinstance(t, torch.Tensor) and t.dim() in ((2, 3) if isinstance(part, Mixer) else (2,)) and t.dtype == dtype}
 
     # -- what the parts ask of a step ------------------------------------------
     def step_planners(self) -> list:

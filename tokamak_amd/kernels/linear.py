@@ -139,6 +139,19 @@ def linear(x: torch.Tensor | DeferredNorm, weight: torch.Tensor, out_dtype: torc
     return gemm_bf16.gemm(x, weight, out_dtype, allow_partials)
 
 
+def several_linears(x: torch.Tensor, weights: torch.Tensor) -> list[torch.Tensor]:
+    """``linear(x_i, weights[i], allow_partials=True)`` for every i: ``weights`` [C, N, K], ``x`` [C, M, K], or [M, K] for all of them.  More than
+    128 rows: one launch where that pays (``ops.several_pay``)."""
+    count, n, k = weights.shape
+    m = x.shape[-2]
+    if (m > ops.STREAM_MAX_ROWS and x.dtype == torch.bfloat16 and ops.gemm_many_fits(x if x.dim() == 2 else x[0], weights[0], n)
+            and ops.several_pay(count, m, n, k)):
+        out = torch.empty((count, m, n), dtype=x.dtype, device=x.device)
+        ops.gemm_several(x, weights, out)
+        return list(out)
+    return [linear(x if x.dim() == 2 else x[i], weights[i], allow_partials=True) for i in range(count)]
+
+
 def _direct(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, allow_partials: bool,
             sumsq: torch.Tensor | None = None, eps: float = 0.0) -> torch.Tensor:
     """The direct product; where the reader adds partial sums, one float32 sum [1, M, N] (what the split product

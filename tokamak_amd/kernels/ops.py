@@ -303,6 +303,8 @@ _SIGS = {
     "gemm_many": {
         "tk_gemm_many": [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_long,
                          c_float, c_int, c_int, c_void_p],
+        "tk_gemm_several": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long, c_long, c_int, c_long, c_long, c_long,
+                            c_int, c_int, c_void_p],
     },
     "replay": {
         "tk_stream_order": [c_void_p, c_void_p],
@@ -2216,10 +2218,10 @@ MANY_PRICES = {(256, 256): (256, 1.24, 0.914, 6.5, 4.3), (128, 256): (256, 0.767
                (256, 128): (256, 0.772, 0.556, 3.0, 3.2), (128, 128): (512, 0.913, 0.37, -0.2, 4.5)}
 
 
-def _many_price(rows: int, columns: int, m: int, channels: int, k: int, parts: int) -> float:
+def _many_price(rows: int, columns: int, m: int, channels: int, k: int, parts: int, count: int = 1) -> float:
     slots, full, alone, end, start = MANY_PRICES[rows, columns]
     steps = k / 64 / parts
-    rounds, rest = divmod(-(-m // rows) * -(-channels // columns) * parts, slots)
+    rounds, rest = divmod(-(-m // rows) * -(-channels // columns) * parts * count, slots)
     price = start + rounds * (steps * full + end)
     if rest:
         price += steps * (alone + (full - alone) * rest / slots) + end
@@ -2287,6 +2289,37 @@ def gemm_many(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, rows: int,
     _check(_fn("gemm_many", "tk_gemm_many")(
         MANY_MODES[gate], _p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(-2), parts,
         out.stride(0) if split else 0, float(limit or 0.0), rows, columns, _stream()), "gemm_many")
+
+
+@functools.lru_cache(maxsize=4096)
+def several_plan(count: int, m: int, n: int, k: int) -> tuple[int, int]:
+    """(rows, columns) of the cheapest tile of ``count`` products with ``n`` output channels each."""
+    return min(MANY_PRICES, key=lambda tile: _many_price(*tile, m, n, k, 1, count))
+
+
+def several_pay(count: int, m: int, n: int, k: int) -> bool:
+    """Whether ``count`` products of more than 128 rows go out as one launch of ``gemm_several`` rather than each to the library: by the
+    share of the blocks that run at once which their tiles fill, or K short enough.  Beside as many launches of the library, weights from memory:
+    four of 4,096 x 4,096 at 129 / 512 / 1,000 / 2,048 rows 91 / 123 / 164 / 241 us, here 44 / 59 / 96 / 184; three of 2,048 x 2,048 at 2,048
+    rows 69 and 49; one alone 0.6 to 1.06 times as fast.  (A product's 64 to 256 tiles are a fraction of a round; several fill whole ones.)"""
+    rows, columns = several_plan(count, m, n, k)
+    return count > 1 and (k <= 2048 or -(-m // rows) * -(-n // columns) * count >= 0.4 * MANY_PRICES[rows, columns][0])
+
+
+def gemm_several(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
+    """out[i] = a[i] @ w[i]^T in bfloat16, i below the number of matrices: w [C, N, K], out [C, M, N], a [C, M, K], or [M, K] for all."""
+    for t in (a, w, out):
+        _need(t.is_cuda and t.stride(-1) == 1 and t.dtype == torch.bfloat16, "gemm operands are bfloat16 GPU tensors with unit inner stride")
+    count, n, k = w.shape
+    m = a.shape[-2]
+    _need(a.shape[-1] == k and out.shape == (count, m, n) and (a.dim() == 2 or a.shape[0] == count), "gemm shapes disagree")
+    first = a if a.dim() == 2 else a[0]
+    _need(gemm_many_fits(first, w[0], n) and out.data_ptr() % 16 == 0 and out.stride(1) % 8 == 0 and count <= 64
+          and all(t.dim() == 2 or t.stride(0) % 8 == 0 for t in (a, w, out)), "products of many rows take whole steps of 64 k and rows on 16-byte borders")
+    _note(f"{count}x{m}x{n}x{k}", count * (n * k + m * k + m * n) * 2, 2.0 * count * m * n * k)
+    _check(_fn("gemm_many", "tk_gemm_several")(
+        _p(a), _p(w), _p(out), m, n, k, first.stride(0), w.stride(1), out.stride(1), count, 0 if a.dim() == 2 else a.stride(0), w.stride(0),
+        out.stride(0), *several_plan(count, m, n, k), _stream()), "gemm_several")
 
 
 def _stream_operands(resid: torch.Tensor, gamma: torch.Tensor | None, m: int, n: int) -> torch.Tensor | None:

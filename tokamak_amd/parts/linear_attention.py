@@ -6,7 +6,7 @@ import torch
 
 from tokamak_amd.config.registry import register_part
 from tokamak_amd.kernels import ops
-from tokamak_amd.kernels.linear import linear
+from tokamak_amd.kernels.linear import linear, several_linears
 from tokamak_amd.parts.base import Fetch, Mixer, PositionData, StateArray
 from tokamak_amd.weights.spec import TensorSpec
 
@@ -44,7 +44,8 @@ class GatedLinearAttention(Mixer):
             raise ValueError(f"tau must be positive, got {tau}")
         self.tau, self.norm_eps = float(tau), float(norm_eps)
         self.decay_rank = None if decay_rank is None else int(decay_rank)
-        self.q = self.k = self.v = self.g = self.o = self.a1 = self.a2 = None
+        # matrices of one shape lie together: q, k and v, g, or all four
+        self.qk = self.vg = self.qkvg = self.o = self.a1 = self.a2 = None
         self.bias = self.gain = None
 
     def expected_tensors(self, prefix: str) -> dict[str, TensorSpec]:
@@ -59,7 +60,10 @@ class GatedLinearAttention(Mixer):
         }
 
     def bind(self, prefix: str, fetch: Fetch) -> None:
-        for n in ("q", "k", "v", "g", "o", "a1", "a2"):
+        groups = ("qkvg",) if self.head_dim == self.value_dim else ("qk", "vg")
+        for names in groups:
+            setattr(self, names, torch.stack([fetch(prefix + n) for n in names]))
+        for n in ("o", "a1", "a2"):
             setattr(self, n, fetch(prefix + n))
         if self.a2.shape[1] != self.a1.shape[0]:
             raise ValueError(f"the two matrices of the decay disagree on its rank: {tuple(self.a1.shape)} and {tuple(self.a2.shape)}")
@@ -72,7 +76,10 @@ class GatedLinearAttention(Mixer):
     def forward(self, h, batch, store, writes_cache: bool = True, position: PositionData | None = None):
         n = h.shape[0]
         # (split products leave float32 partial sums, which the scan adds as it loads)
-        q, k, v, gate = (linear(h, w, allow_partials=True) for w in (self.q, self.k, self.v, self.g))
+        if self.qkvg is not None:
+            q, k, v, gate = several_linears(h, self.qkvg)
+        else:
+            q, k, v, gate = *several_linears(h, self.qk), *several_linears(h, self.vg)
         low = linear(h, self.a1)
         # (few rows: float32 or split partial sums from the streaming product; a long portion: the
         # library's product in the compute dtype, as for the other projections)

@@ -6,7 +6,7 @@ import torch
 
 from tokamak_amd.config.registry import register_part
 from tokamak_amd.kernels import ops
-from tokamak_amd.kernels.linear import linear
+from tokamak_amd.kernels.linear import linear, several_linears
 from tokamak_amd.parts.base import Fetch, Mixer, PositionData, StateArray
 from tokamak_amd.weights.spec import TensorSpec
 
@@ -45,7 +45,7 @@ class DecayedStateTimeMix(Mixer):
         self.decay_rank = None if decay_rank is None else int(decay_rank)
         self.width = self.num_heads * self.head_dim
         self.mu: torch.Tensor | None = None
-        self.r = self.k = self.v = self.g = self.w1 = self.w2 = self.o = None
+        self.rkvg = self.w1 = self.w2 = self.o = None
         self.w0 = self.u = self.gain = None
 
     def expected_tensors(self, prefix: str) -> dict[str, TensorSpec]:
@@ -63,7 +63,8 @@ class DecayedStateTimeMix(Mixer):
 
     def bind(self, prefix: str, fetch: Fetch) -> None:
         self.mu = torch.stack([fetch(prefix + "mu." + s) for s in MIXES]).contiguous()
-        for n in ("r", "k", "v", "g", "w1", "w2", "o", "w0"):
+        self.rkvg = torch.stack([fetch(prefix + n) for n in MIXES[:4]])
+        for n in ("w1", "w2", "o", "w0"):
             setattr(self, n, fetch(prefix + n))
         if self.w2.shape[1] != self.w1.shape[0]:
             raise ValueError(f"the two matrices of the decay disagree on its rank: {tuple(self.w1.shape)} and {tuple(self.w2.shape)}")
@@ -79,7 +80,7 @@ class DecayedStateTimeMix(Mixer):
         mixes = torch.empty((len(MIXES), n, self.hidden_size), dtype=self.dtype, device=h.device)
         ops.token_shift(h, self.mu, store.state["last"], mixes, batch)
         # (split products leave float32 partial sums, which the scan adds as it loads)
-        r, k, v, gate = (linear(mixes[i], getattr(self, s), allow_partials=True) for i, s in enumerate(MIXES[:4]))
+        r, k, v, gate = several_linears(mixes[:4], self.rkvg)
         low = torch.empty((n, self.w1.shape[0]), dtype=self.dtype, device=h.device)
         ops.tanh(linear(mixes[4], self.w1, allow_partials=True), low)
         decay_in = linear(low, self.w2, out_dtype=torch.float32, allow_partials=True)
