@@ -240,7 +240,8 @@ def gemm(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, allow_pa
     (``stream_pays_beyond_64_rows``; up to 96 these are the products that do not flow: K not a
     multiple of 128, or a very wide matrix).  Else more than 64 rows
     with bfloat16 output: the library product (hipBLASLt, as the reference's
-    nn.Linear ends in a library; csrc/blas_lt.hip); with float32 output: 128 rows at a time.
+    nn.Linear ends in a library; csrc/blas_lt.hip); with float32 output: up to 128 rows the streaming kernel, more the many-rows one (where
+    K is no multiple of 64 or N none of 8, the streaming one 128 rows at a time).
     """
     m = x.shape[0]
     n, k = weight.shape
@@ -252,6 +253,13 @@ def gemm(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, allow_pa
             out = torch.empty((splits, m, n), dtype=torch.float32, device=dev)
             used = ops.gemm_stream(x, weight, out, splits=splits)
             return out[:used]
+    if m > ops.STREAM_MAX_ROWS and out_dtype == torch.float32 and ops.gemm_many_fits(x, weight, n):
+        # The many-rows kernel in one share of K.  Beside the streaming one 128 rows at a time: 2,048 rows, 4,096 x 64 (a decay's low rank, whose
+        # sums stay in float32) 194 -> 14 us, 4,096 x 4,096 1,000 -> 61; 129 rows 28 -> 12 and 84 -> 33, 151,936 x 1,024 164 -> 102
+        out = torch.empty((m, n), dtype=torch.float32, device=dev)
+        rows, columns = ops.several_plan(1, m, n, k)
+        ops.gemm_many(x, weight, out[None], rows=rows, columns=columns)
+        return out
     if fits and (m <= SKINNY_MAX_ROWS or out_dtype == torch.float32):
         out = torch.empty((m, n), dtype=out_dtype, device=dev)
         # (a logits head over 65 to 128 rows at once: 320-365 us at 8B width, 490-530 in two passes)
