@@ -12,7 +12,9 @@
 #include "common.h"
 #include "no_alloc.h"
 
+#include <cstring>
 #include <mutex>
+#include <type_traits>
 
 using namespace tk;
 
@@ -32,15 +34,18 @@ __device__ __forceinline__ void argmax_take(float& bv, int& bi, float v, int i) 
 }
 
 constexpr int kBins = 4096;  // histogram bins of one radix pass (12 bits)
+constexpr int kCoarse = kBins / kWave;
+constexpr int kHistWords = kBins + kCoarse;     // of a row in memory
 constexpr int kCandidates = 16384;
 constexpr int kShareThreads = 256;
 constexpr int kFew = 256;          // values among which a threshold is found by ranks
+constexpr int kLevelBins = 1024;   // of the second and the third level (ten bits each)
 
 // Scratch of the rows with thresholds, null: every row is sampled by one block alone.  The argmax pass zeroes what the
 // kernels add into (hist32, hist64, count).
 struct SharedRows {
-  uint32_t* hist32;              // [M][kBins]
-  unsigned long long* hist64;    // [M][kBins]
+  uint32_t* hist32;              // [M][kBins + kCoarse]: the bins, then the sums of every 64 of them
+  unsigned long long* hist64;    // [M][kBins + kCoarse]
   uint32_t* count;               // [M] entries of the list
   uint32_t* cand;                // [M][kCandidates] ordered images
   uint8_t* segment;              // [M][kCandidates]
@@ -48,10 +53,30 @@ struct SharedRows {
   struct FirstLevel* level;      // [M] where the first threshold lies
 };
 
-__device__ __forceinline__ bool has_threshold(const float* temperature, const int* top_k, const float* top_p, int r, int V, bool& k_on, bool& p_on) {
-  k_on = top_k[r] > 0 && top_k[r] < V;
-  p_on = top_p[r] < 1.f;
-  return temperature[r] > 0.f && (k_on || p_on);
+// A step's sampling parameters in device memory.
+struct RowParams {
+  const unsigned long long *seeds, *draws;     // [M] the request's seed and how many draws it has made
+  const float *temperature, *top_p;            // [M]
+  const int* top_k;                            // [M]
+  const int* rows;                             // [shared] the rows that have a threshold
+};
+
+// The same of up to kInlineRows rows as an argument of the first launch, which leaves them in device memory for the others: a copy
+// through pinned memory costs the GPU 3.5 us and the host 9.
+constexpr int kInlineRows = 64;
+struct InlineParams {
+  unsigned long long seeds[kInlineRows], draws[kInlineRows];
+  float temperature[kInlineRows], top_p[kInlineRows];
+  int top_k[kInlineRows], rows[kInlineRows];
+  RowParams to;
+  int shared;
+};
+struct NoParams {};      // an argmax alone
+
+__device__ __forceinline__ bool has_threshold(float temperature, int top_k, float top_p, int V, bool& k_on, bool& p_on) {
+  k_on = top_k > 0 && top_k < V;
+  p_on = top_p < 1.f;
+  return temperature > 0.f && (k_on || p_on);
 }
 
 // Eight loads a thread of a run of quads, asked for together (a segment of 152 k logits is five: one trip to memory, not one
@@ -78,13 +103,12 @@ __device__ __forceinline__ void use_quads(const float4* __restrict__ p, int quad
   }
 }
 
-// temperature, top_k, top_p, part_mass (all or none): for a row with temperature > 0 and no
-// threshold the block also leaves the sum of e^((x - its segment's maximum) / temperature) over its segment, from which
-// the sampler has the mass of every segment without a pass of its own over the row.
+// With parameters: for a row with temperature > 0 and no threshold the block also leaves the sum of e^((x - its segment's maximum) /
+// temperature) over its segment, from which the sampler has the mass of every segment without a pass of its own over the row.
+template <typename P>
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
-    const float* __restrict__ logits, float* __restrict__ part_v, int* __restrict__ part_i, int V,
-    long ld, const float* __restrict__ temperature, const int* __restrict__ top_k,
-    const float* __restrict__ top_p, float* __restrict__ part_mass, SharedRows clear) {
+    const float* __restrict__ logits, float* __restrict__ part_v, int* __restrict__ part_i, int V, long ld, P params, float* __restrict__ part_mass,
+    SharedRows clear) {
   __shared__ float best_v[kArgmaxThreads / kWave];
   __shared__ int best_i[kArgmaxThreads / kWave];
   const int seg = blockIdx.x, r = blockIdx.y;
@@ -99,12 +123,28 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
   const float4* const row4 = reinterpret_cast<const float4*>(row + begin);
   float4 held[kHeldQuads];
   if (vec) ask_quads<kArgmaxThreads>(row4, quads, 0, held);
+  float temperature = 0.f;
+  bool thresholds = false;
+  if constexpr (!std::is_same_v<P, NoParams>) {
+    bool k_on, p_on;
+    temperature = params.temperature[r];
+    thresholds = has_threshold(temperature, params.top_k[r], params.top_p[r], V, k_on, p_on);
+  }
+  if constexpr (std::is_same_v<P, InlineParams>) {
+    if (seg == 0 && threadIdx.x == 0) {
+      const_cast<unsigned long long*>(params.to.seeds)[r] = params.seeds[r];
+      const_cast<unsigned long long*>(params.to.draws)[r] = params.draws[r];
+      const_cast<float*>(params.to.temperature)[r] = temperature;
+      const_cast<float*>(params.to.top_p)[r] = params.top_p[r];
+      const_cast<int*>(params.to.top_k)[r] = params.top_k[r];
+      if (r < params.shared) const_cast<int*>(params.to.rows)[r] = params.rows[r];
+    }
+  }
   // scratch of a row with thresholds that later kernels add into, shared out over its blocks
-  bool k_on, p_on;
-  if (clear.hist32 != nullptr && has_threshold(temperature, top_k, top_p, blockIdx.y, V, k_on, p_on)) {
-    for (int i = blockIdx.x * kArgmaxThreads + threadIdx.x; i < kBins; i += kArgmaxSegments * kArgmaxThreads) {
-      clear.hist32[(size_t)blockIdx.y * kBins + i] = 0u;
-      clear.hist64[(size_t)blockIdx.y * kBins + i] = 0ull;
+  if (clear.hist32 != nullptr && thresholds) {
+    for (int i = blockIdx.x * kArgmaxThreads + threadIdx.x; i < kHistWords; i += kArgmaxSegments * kArgmaxThreads) {
+      clear.hist32[(size_t)blockIdx.y * kHistWords + i] = 0u;
+      clear.hist64[(size_t)blockIdx.y * kHistWords + i] = 0ull;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) clear.count[blockIdx.y] = 0u;
   }
@@ -131,10 +171,9 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
     part_v[r * kArgmaxSegments + seg] = bv;
     part_i[r * kArgmaxSegments + seg] = bi;
   }
-  if (part_mass == nullptr || !(temperature[r] > 0.f)) return;
-  if (has_threshold(temperature, top_k, top_p, r, V, k_on, p_on)) return;  // the sampler sums what it keeps
+  if (part_mass == nullptr || !(temperature > 0.f) || thresholds) return;      // (with thresholds the sampler sums what it keeps)
   // the segment again: its mass relative to its own maximum
-  const float scale = 1.4426950408889634f / temperature[r];  // e^(y / t) = 2^(y log2 e / t)
+  const float scale = 1.4426950408889634f / temperature;  // e^(y / t) = 2^(y log2 e / t)
   float mass = 0.f;
   const auto add = [&](float x) {
     const float y = (x - bv) * scale;
@@ -186,8 +225,7 @@ TK_API int tk_argmax(const float* logits, int* out, float* out_value, float* par
                      int V, long ld, hipStream_t stream) {
   if (M <= 0) return 0;
   if (V <= 0 || M > 65535) return -1;
-  argmax_segments_kernel<<<dim3(kArgmaxSegments, M), kArgmaxThreads, 0, stream>>>(logits, part_v, part_i, V, ld,
-                                                                                   nullptr, nullptr, nullptr, nullptr, SharedRows{});
+  argmax_segments_kernel<<<dim3(kArgmaxSegments, M), kArgmaxThreads, 0, stream>>>(logits, part_v, part_i, V, ld, NoParams{}, nullptr, SharedRows{});
   argmax_pick_kernel<<<M, kWave, 0, stream>>>(part_v, part_i, out, out_value);
   return launch_status();
 }
@@ -231,7 +269,7 @@ TK_API int tk_argmax_no_alloc(const float* logits, int* out, float* out_value, i
   ArgmaxScratch* scratch = argmax_scratch_of_current_device();
   if (scratch == nullptr) return -4;
   argmax_segments_kernel<<<dim3(kArgmaxSegments, M), kArgmaxThreads, 0, stream>>>(
-      logits, scratch->value, scratch->index, V, ld, nullptr, nullptr, nullptr, nullptr, SharedRows{});
+      logits, scratch->value, scratch->index, V, ld, NoParams{}, nullptr, SharedRows{});
   argmax_pick_kernel<<<M, kWave, 0, stream>>>(scratch->value, scratch->index, out, out_value);
   return launch_status();
 }
@@ -244,6 +282,8 @@ __device__ __forceinline__ uint32_t ordered(float f) {
   const uint32_t u = __float_as_uint(f);
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
+
+constexpr uint32_t kOrderedMinusInf = 0x007fffffu;      // ordered(-infinity)
 
 __device__ __forceinline__ float unordered(uint32_t o) {
   const uint32_t u = (o & 0x80000000u) ? (o & 0x7fffffffu) : ~o;
@@ -260,7 +300,6 @@ __device__ __forceinline__ float uniform01(uint64_t seed, uint64_t counter) {
 }
 
 constexpr int kSampleThreads = 1024;
-static_assert(4 * kFew <= kSampleThreads, "four threads a value");
 
 // Prefix sums of one value per thread over the block, threads in index order; `scan`
 // holds an entry a wave.  Returns the sum over the threads before this one;
@@ -292,7 +331,7 @@ __device__ __forceinline__ T block_scan(T v, T* scan, T& inclusive, T& total) {
 
 // Walking the bins from the highest down: the bin in which the running sum first
 // reaches `target` (sum of higher bins < target <= that sum + the bin), and the sum
-// of the higher bins.  Every thread gets the result.  `nbins` is 4096 or 256.
+// of the higher bins.  Every thread gets the result.  `nbins` is 4096 or 1024.
 template <typename T>
 __device__ __forceinline__ void crossing_bin(const T* hist, int nbins, T target, T* scan, int* found_bin,
                                              T* found_above, int& bin, T& above) {
@@ -385,10 +424,11 @@ __device__ __forceinline__ void for_row(const float* __restrict__ row, int V, F 
 //                   order: sums over the list are of integers), and the mass of the bins above it in each segment; with
 //                   both thresholds the bins above it are listed too, top-p's may lie there.
 // The sampler then starts from the histogram and the list and reads the row again only where the drawn number falls.
-// (A block that reads its row alone moves some 45 GB/s.  40 rows of 152 k logits, most with thresholds: 10.3 + 12.8 us shared and
-// 18.8 for the rest, of which a segment's walk, the ranks and the start are each a few memory round trips; 58.9 -> 53.7 us for
-// the whole since a thread asks for its piece of a segment at once, the sampler takes the first level's bin from the collecting
-// kernel and ranks are counted by four threads a value.)
+// (A block that reads its row alone moves some 45 GB/s.  40 rows of 151,936 logits, 24 of them with thresholds: argmax 6.9, histograms 8.6, lists
+// 10.5 and the rest 14.5 us, 54.6 -> 40.6 for the whole with its parameters, which came by a copy of their own: only rows that have a threshold
+// get blocks (10.0 us, in two rounds, for the histograms of all), a wave finds the first level's bin from sums of 64 bins (the
+// block's search 3.8 us, this 2.2), what cannot be listed is passed over by one comparison, and the rest asks for its
+// list and its numbers at once and stops at the level that leaves a few values.)
 
 // A segment of a row as the threads of a block see it: asked for at once, used later (f(value) for every element, each by
 // one thread).
@@ -481,27 +521,73 @@ __device__ __forceinline__ FirstLevel first_level(const uint32_t* h32, const uns
   return *found;
 }
 
+// The sum over the wave of whole numbers, in every lane.
+__device__ __forceinline__ uint32_t wave_sum_of(uint32_t v) {
+  v += lane_other<0>(v);
+  v += lane_other<1>(v);
+  v += lane_other<2>(v);
+  v += lane_other<3>(v);
+  LanePair p = pair16(v);
+  p = pair32(p.first + p.second);
+  return p.first + p.second;
+}
+
+// Walking 64 numbers from the highest place down, a lane each (lane l has place 63 - l): the place at which the running sum first
+// reaches `target`, or the lowest one, and the sum above it.
+__device__ __forceinline__ int crossing_place(unsigned long long mine, unsigned long long target, unsigned long long& above) {
+  const int lane = threadIdx.x & (kWave - 1);
+  unsigned long long upto = mine;
+#pragma unroll
+  for (int step = 1; step < kWave; step <<= 1) {
+    const unsigned long long other = __shfl_up(upto, step, kWave);
+    if (lane >= step) upto += other;
+  }
+  const unsigned long long reached = __ballot(target <= upto);
+  const int at = reached ? __ffsll(reached) - 1 : kWave - 1;
+  above = __shfl(upto - mine, at, kWave);
+  return kWave - 1 - at;
+}
+
+// The same from a row's histograms in memory, by a wave alone: among the sums of every 64 bins, then among those 64 (two trips to
+// memory and no barrier; all bins by the block took 3.8 us).
+__device__ __forceinline__ FirstLevel first_level_by_wave(const uint32_t* __restrict__ h32, const unsigned long long* __restrict__ h64, bool k_on,
+                                                          int k, float p_keep) {
+  const int place = kWave - 1 - (threadIdx.x & (kWave - 1));
+  const uint32_t coarse = h32[kBins + place];
+  unsigned long long target = (unsigned long long)k, sums = coarse, before;
+  if (!k_on) {
+    sums = h64[kBins + place];
+    unsigned long long whole = sums;
+#pragma unroll
+    for (int m = 1; m < kWave; m <<= 1) whole += __shfl_xor(whole, m, kWave);
+    // the share of the whole mass that top_p allows (at least one unit)
+    const double share = (double)p_keep * (double)whole;
+    target = share < 1.0 ? 1ull : (unsigned long long)share;
+  }
+  const int group = crossing_place(sums, target, before);
+  const uint32_t c = h32[group * kWave + place];
+  unsigned long long inside;
+  const int bin = crossing_place(k_on ? (unsigned long long)c : h64[group * kWave + place], target - before, inside);
+  // (values at and above the bin: of the groups above it, and of its group)
+  const uint32_t seen = wave_sum_of((place > group ? coarse : 0u) + (place >= bin ? c : 0u));
+  const unsigned long long left = target - before - inside;
+  return {group * kWave + bin, (uint32_t)left, left, seen, __shfl(c, kWave - 1 - bin, kWave)};
+}
+
 __global__ __launch_bounds__(kShareThreads) void sample_hist_kernel(
-    const float* __restrict__ logits, long ld, int V, const float* __restrict__ temperature, const int* __restrict__ top_k,
-    const float* __restrict__ top_p, const float* __restrict__ seg_max, const int* __restrict__ seg_index, int* __restrict__ out,
-    float* __restrict__ row_max, SharedRows sh) {
+    const float* __restrict__ logits, long ld, int V, RowParams params, const float* __restrict__ seg_max, float* __restrict__ row_max,
+    SharedRows sh) {
   __shared__ uint32_t h32[kBins];
   __shared__ unsigned long long h64[kBins];
-  const int seg = blockIdx.x, r = blockIdx.y, lane = threadIdx.x & (kWave - 1);
+  const int seg = blockIdx.x, r = params.rows[blockIdx.y], lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   bool k_on, p_on;
-  const bool thresholds = has_threshold(temperature, top_k, top_p, r, V, k_on, p_on);
-  if (!thresholds && seg > 0) return;
-  Segment segment(logits + (size_t)r * ld, thresholds ? V : 0, seg);
-  // the row's maximum (every wave for itself); the first block leaves it, and the argmax
-  float bv = lane < kArgmaxSegments ? seg_max[r * kArgmaxSegments + lane] : -INFINITY;
-  int bi = lane < kArgmaxSegments ? seg_index[r * kArgmaxSegments + lane] : 0x7fffffff;
-  wave_best(bv, bi, argmax_take);
-  if (seg == 0 && threadIdx.x == 0) {
-    out[r] = (bi == 0x7fffffff) ? 0 : bi;
-    row_max[r] = bv;
-  }
-  if (!thresholds) return;
-  const float inv_t = 1.f / temperature[r], mx = bv * inv_t;
+  const float temperature = params.temperature[r];
+  if (!has_threshold(temperature, params.top_k[r], params.top_p[r], V, k_on, p_on)) return;
+  Segment segment(logits + (size_t)r * ld, V, seg);
+  // the row's maximum (every wave for itself)
+  const float bv = wave_max(lane < kArgmaxSegments ? seg_max[r * kArgmaxSegments + lane] : -INFINITY);
+  if (seg == 0 && threadIdx.x == 0) row_max[r] = bv;
+  const float inv_t = 1.f / temperature, mx = bv * inv_t;
   if (!(mx > -INFINITY)) return;
   for (int i = threadIdx.x; i < kBins; i += kShareThreads) h32[i] = 0;
   if (!k_on)
@@ -514,37 +600,52 @@ __global__ __launch_bounds__(kShareThreads) void sample_hist_kernel(
     if (!k_on) atomicAdd(&h64[bin], fixed_mass(x, mx));
   });
   __syncthreads();
-  for (int i = threadIdx.x; i < kBins; i += kShareThreads) {
+  // a wave 64 neighbouring bins at a time, and their sum (most are empty)
+  for (int group = wave; group < kCoarse; group += kShareThreads / kWave) {
+    const int i = group * kWave + lane;
     const uint32_t n = h32[i];
-    if (n == 0) continue;
-    atomicAdd(&sh.hist32[(size_t)r * kBins + i], n);
-    if (!k_on) atomicAdd(&sh.hist64[(size_t)r * kBins + i], h64[i]);
+    if (__ballot(n != 0) == 0) continue;
+    const size_t at = (size_t)r * kHistWords;
+    const uint32_t all = wave_sum_of(n);
+    if (n != 0) atomicAdd(&sh.hist32[at + i], n);
+    if (lane == 0) atomicAdd(&sh.hist32[at + kBins + group], all);
+    if (k_on) continue;
+    const unsigned long long mass = h64[i];
+    unsigned long long sum = mass;
+#pragma unroll
+    for (int m = 1; m < kWave; m <<= 1) sum += __shfl_xor(sum, m, kWave);
+    if (n != 0) atomicAdd(&sh.hist64[at + i], mass);
+    if (lane == 0) atomicAdd(&sh.hist64[at + kBins + group], sum);
   }
 }
 
 __global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
-    const float* __restrict__ logits, long ld, int V, const float* __restrict__ temperature, const int* __restrict__ top_k,
-    const float* __restrict__ top_p, const float* __restrict__ row_max, SharedRows sh) {
+    const float* __restrict__ logits, long ld, int V, RowParams params, const float* __restrict__ row_max, SharedRows sh) {
   __shared__ uint32_t kept[kBins];
   __shared__ unsigned long long scan[kShareThreads / kWave];
-  __shared__ FirstLevel found;
   __shared__ uint32_t count, first;
-  const int seg = blockIdx.x, r = blockIdx.y;
+  const int seg = blockIdx.x, r = params.rows[blockIdx.y];
   bool k_on, p_on;
-  if (!has_threshold(temperature, top_k, top_p, r, V, k_on, p_on) || !(row_max[r] > -INFINITY)) return;
-  const float inv_t = 1.f / temperature[r];
+  const float temperature = params.temperature[r], p_keep = params.top_p[r];
+  const int k = params.top_k[r];
+  if (!has_threshold(temperature, k, p_keep, V, k_on, p_on) || !(row_max[r] > -INFINITY)) return;
+  const float inv_t = 1.f / temperature;
   if (threadIdx.x == 0) count = 0;
-  const FirstLevel level = first_level<kShareThreads>(sh.hist32 + (size_t)r * kBins, sh.hist64 + (size_t)r * kBins, k_on, top_k[r], top_p[r],
-                                                      scan, &found);
+  Segment segment(logits + (size_t)r * ld, V, seg);
+  const FirstLevel level = first_level_by_wave(sh.hist32 + (size_t)r * kHistWords, sh.hist64 + (size_t)r * kHistWords, k_on, k, p_keep);
   if (seg == 0 && threadIdx.x == 0) sh.level[r] = level;
   const int low = level.bin;
   const bool both = k_on && p_on;
   if ((both ? level.total : level.inside) > (uint32_t)kCandidates) return;      // (the sampler walks the row)
   const float mx = row_max[r] * inv_t, scale = draw_scale(V);
   unsigned long long above = 0;
+  __syncthreads();
   // this block's values, then side by side into the row's list
-  // (asked for here: held across the search above they cost registers, and with them blocks; 12.8 -> 15.1 us at 40 rows)
-  Segment(logits + (size_t)r * ld, V, seg).each([&](float logit) {
+  // (what lies below the bin, nearly all, is passed over by one comparison; the lowest bins, where a NaN counts, have none)
+  const float least = low > (int)(kOrderedMinusInf >> 20) ? unordered((uint32_t)low << 20) : -INFINITY;
+  const bool every = !(least > -INFINITY);
+  segment.each([&](float logit) {
+    if (!(every || logit * inv_t >= least)) return;
     const float x = scaled(logit, inv_t);
     const uint32_t o = ordered(x);
     const int bin = (int)(o >> 20);
@@ -573,12 +674,11 @@ __global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
   }
 }
 
-// One block per row.  params rows: temperature, top_k, top_p (floats);
-// seeds/counters: the request's seed and how many draws it has made.
+// One block per row.
 // probs_out (optional, [M, V]) receives the final distribution, for tests.
 //
 // Both thresholds are found by radix selection over the ordered-integer image of the
-// scaled logits: three levels (12, 12 and 8 bits), each filling a histogram in LDS (counts
+// scaled logits: three levels (12, 10 and 10 bits), each filling a histogram in LDS (counts
 // for top-k, fixed-point probability mass for top-p) in which the bin that holds the
 // threshold is found; the next level looks only at the values of that bin.  A pass over the
 // row costs 14 us (one CU reads it alone), so the row is walked as rarely as possible: the
@@ -590,10 +690,7 @@ __global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
 // draw's with both thresholds.)  Where shares_rows says so the first pass and the copies are those of sample_hist and
 // sample_collect.
 __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
-    const float* __restrict__ logits, long ld, int V, const float* __restrict__ temperature,
-    const int* __restrict__ top_k, const float* __restrict__ top_p,
-    const unsigned long long* __restrict__ seeds, const unsigned long long* __restrict__ counters,
-    const float* __restrict__ row_max, const float* __restrict__ seg_max, const float* __restrict__ seg_mass,
+    const float* __restrict__ logits, long ld, int V, RowParams params, const float* __restrict__ seg_max, const int* __restrict__ seg_index, const float* __restrict__ seg_mass,
     int* __restrict__ out, float* __restrict__ probs_out, SharedRows shared) {
   __shared__ float upto[kArgmaxSegments];  // the mass of the row's segments up to and with each
   __shared__ unsigned long long hist64[kBins];
@@ -614,16 +711,26 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   float* scanf_ = reinterpret_cast<float*>(scan64);
 
   const int r = blockIdx.x, tid = threadIdx.x, nt = kSampleThreads;
-  if (!(temperature[r] > 0.f)) return;  // greedy row: the argmax pre-pass has written it
+  // the row's maximum and its place from those of its segments, every wave for itself: the token of a greedy row, and of one whose
+  // search falls through
+  float best = (tid & (kWave - 1)) < kArgmaxSegments ? seg_max[r * kArgmaxSegments + (tid & (kWave - 1))] : -INFINITY;
+  int best_at = (tid & (kWave - 1)) < kArgmaxSegments ? seg_index[r * kArgmaxSegments + (tid & (kWave - 1))] : 0x7fffffff;
+  wave_best(best, best_at, argmax_take);
+  if (tid == 0) out[r] = best_at == 0x7fffffff ? 0 : best_at;
+  const float temperature = params.temperature[r];
+  if (!(temperature > 0.f)) return;
+  // (asked for ahead of their use)
+  const float drawn = uniform01(params.seeds[r], params.draws[r]);
+  const uint32_t first_cand = shared.hist32 != nullptr ? shared.cand[(size_t)r * kCandidates + tid] : 0u;
+  const uint8_t first_segment = shared.hist32 != nullptr ? shared.segment[(size_t)r * kCandidates + tid] : (uint8_t)0;
   const float* row = logits + (size_t)r * ld;
-  const float inv_t = 1.f / temperature[r];
-  const int k = top_k[r];
-  const float p_keep = top_p[r];
+  const float inv_t = 1.f / temperature;
+  const int k = params.top_k[r];
+  const float p_keep = params.top_p[r];
   const bool k_on = k > 0 && k < V, p_on = p_keep < 1.f;
 
-  // the row's maximum comes from the argmax pass that ran before (temperature > 0
-  // keeps the order); a row without any number has nothing to draw from
-  const float mx = row_max[r] * inv_t;
+  // (temperature > 0 keeps the order; a row without any number has nothing to draw from)
+  const float mx = best * inv_t;
   if (!(mx > -INFINITY)) return;
 
   // First pass: the first level's histogram (counts; probability mass too if only top-p is
@@ -664,8 +771,12 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     // the values in that bin and above it; listed: those that may be a threshold (see sample_collect)
     const uint32_t total = level.total, entries = k_on && p_on ? level.total : level.inside;
     if (ready && entries <= (uint32_t)kCandidates) {
+      if (tid < (int)entries) {
+        cand[tid] = first_cand;
+        cand_segment[tid] = first_segment;
+      }
 #pragma unroll 4
-      for (int i = tid; i < (int)entries; i += nt) {
+      for (int i = tid + nt; i < (int)entries; i += nt) {
         cand[i] = shared.cand[(size_t)r * kCandidates + i];
         cand_segment[i] = shared.segment[(size_t)r * kCandidates + i];
       }
@@ -723,10 +834,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     __syncthreads();
     const int n = (int)few_count;
     if (n > kFew || n == 0) return false;      // (every thread alike)
-    if (tid < 4 * n) {      // (four neighbouring threads a value, a quarter of the others each)
-      const uint32_t mine = few[tid / 4];
+    for (int v = tid; v < 4 * n; v += kSampleThreads) {      // (four neighbouring threads a value, a quarter of the others each)
+      const uint32_t mine = few[v / 4];
       unsigned long long above = 0, whole = 0;
-      for (int i = tid & 3; i < n; i += 4) {
+      for (int i = v & 3; i < n; i += 4) {
         const unsigned long long m = few_mass[i];
         whole += m;
         above += few[i] > mine ? m : 0ull;
@@ -747,22 +858,22 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   uint32_t kth = 0;  // ordered(-inf) is > 0, so 0 keeps everything
   if (k_on && !among_few(false, [&](uint32_t o) { return (o >> 20) == k_prefix; }, [&](unsigned long long) { return (unsigned long long)k_remaining; }, kth)) {
     uint32_t prefix = k_prefix, remaining = k_remaining;
-    // (shift, bits): 20/12 (done above), 8/12, 0/8
-    for (int level = 1; level < 3; ++level) {
-      const int shift = level == 1 ? 8 : 0;
-      const int nbins = level == 2 ? 256 : kBins;
-      for (int i = tid; i < kBins; i += nt) hist32[i] = 0;
+    for (int level = 1; level < 3; ++level) {      // (12 bits are known, ten more each)
+      const int shift = level == 1 ? 10 : 0;
+      for (int i = tid; i < kLevelBins; i += nt) hist32[i] = 0;
       __syncthreads();
       each([&](uint32_t o, float) {
-        if ((o >> (shift + (level == 1 ? 12 : 8))) == prefix) atomicAdd(&hist32[(o >> shift) & (uint32_t)(nbins - 1)], 1u);
+        if ((o >> (shift + 10)) == prefix) atomicAdd(&hist32[(o >> shift) & (uint32_t)(kLevelBins - 1)], 1u);
       });
       __syncthreads();
       int bin;
       uint32_t above;
-      crossing_bin<uint32_t>(hist32, nbins, remaining, scan32, &found_bin,
+      crossing_bin<uint32_t>(hist32, kLevelBins, remaining, scan32, &found_bin,
                              reinterpret_cast<uint32_t*>(&found_above), bin, above);
       remaining -= above;
-      prefix = (prefix << (level == 2 ? 8 : 12)) | (uint32_t)bin;
+      prefix = (prefix << 10) | (uint32_t)bin;
+      const auto in_bin = [&](uint32_t o) { return (o >> 10) == prefix; };
+      if (level == 1 && among_few(false, in_bin, [&](unsigned long long) { return (unsigned long long)remaining; }, prefix)) break;
     }
     kth = prefix;
   }
@@ -778,16 +889,14 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
                     : among_few(true, [&](uint32_t o) { return (o >> 20) == p_prefix; }, [&](unsigned long long) { return p_remaining; }, cut))) {
     cut = cut > kth ? cut : kth;
   } else if (p_on) {
-    cut = kth;
     uint32_t prefix = p_prefix;
     unsigned long long remaining = p_remaining;
     for (int level = k_on ? 0 : 1; level < 3; ++level) {  // (without top-k the first pass was the first level)
-      const int shift = level == 0 ? 20 : level == 1 ? 8 : 0;
-      const int nbins = level == 2 ? 256 : kBins;
-      for (int i = tid; i < kBins; i += nt) hist64[i] = 0;
+      const int shift = level == 0 ? 20 : level == 1 ? 10 : 0, nbins = level == 0 ? kBins : kLevelBins;
+      for (int i = tid; i < nbins; i += nt) hist64[i] = 0;
       __syncthreads();
       each([&](uint32_t o, float x) {
-        const bool in_bin = level == 0 || (o >> (shift + (level == 1 ? 12 : 8))) == prefix;
+        const bool in_bin = level == 0 || (o >> (shift + 10)) == prefix;
         if (in_bin && o >= kth) atomicAdd(&hist64[(o >> shift) & (uint32_t)(nbins - 1)], fixed_mass(x, mx));
       });
       __syncthreads();
@@ -802,7 +911,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
       unsigned long long above;
       crossing_bin<unsigned long long>(hist64, nbins, remaining, scan64, &found_bin, &found_above, bin, above);
       remaining -= above;
-      prefix = (prefix << (level == 2 ? 8 : 12)) | (uint32_t)bin;
+      prefix = (prefix << (level == 0 ? 12 : 10)) | (uint32_t)bin;
+      const auto in_bin = [&](uint32_t o) { return (o >> 10) == prefix && o >= kth; };
+      if (level == 1 && among_few(true, in_bin, [&](unsigned long long) { return remaining; }, prefix)) break;
     }
     cut = prefix > kth ? prefix : kth;
   }
@@ -827,9 +938,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     if (tid == 0)
       for (int w = 1; w < kArgmaxSegments; ++w) upto[w] += upto[w - 1];
   } else {
-    if (tid < kSampleThreads / kWave * kArgmaxSegments)
-      segment_mass[tid / kArgmaxSegments][tid % kArgmaxSegments] =
-          listed && !whole_list && tid < kArgmaxSegments ? shared.above[r * kArgmaxSegments + tid] : 0;
+    for (int i = tid; i < kSampleThreads / kWave * kArgmaxSegments; i += kSampleThreads)
+      segment_mass[i / kArgmaxSegments][i % kArgmaxSegments] =
+          listed && !whole_list && i < kArgmaxSegments ? shared.above[r * kArgmaxSegments + i] : 0;
     __syncthreads();
     if (listed) {
       for (int i = tid; i < ncand; i += nt)
@@ -885,22 +996,13 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
     });
   }
 
-  const float target = uniform01(seeds[r], counters[r]) * total;
+  const float target = drawn * total;
   // The chunk that holds the target (every thread finds the same one; the last chunk of
   // the row catches rounding), then all threads walk that chunk: each sums a contiguous
   // run of it, a prefix sum over the block finds the run, and its thread walks it.
-  int sel = (V - 1) / chunk;
-  float sel_before = 0.f;
-  {
-    bool found = false;
-    for (int w = 0; w < kArgmaxSegments; ++w) {
-      if (!found && (target < upto[w] || w == sel)) {
-        found = true;
-        sel = w;
-        sel_before = w > 0 ? upto[w - 1] : 0.f;
-      }
-    }
-  }
+  const int last_segment = (V - 1) / chunk;
+  const int sel = __ffsll(__ballot(lane >= last_segment || target < upto[min(lane, kArgmaxSegments - 1)])) - 1;
+  const float sel_before = sel > 0 ? upto[sel - 1] : 0.f;
   const int s_begin = sel * chunk, s_end = min(V, s_begin + chunk);
   const int run_len = ((s_end - s_begin + kSampleThreads - 1) / kSampleThreads + 3) / 4 * 4;
   const int r_begin = min(s_end, s_begin + tid * run_len), r_end = min(s_end, r_begin + run_len);
@@ -909,8 +1011,11 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   float head[kHeld];
   const auto hold = [&](int from, float (&v)[kHeld]) {
     if ((reinterpret_cast<uintptr_t>(row) & 15) == 0 && from + kHeld <= r_end) {      // (runs begin at multiples of four tokens)
-      const float4 a = *reinterpret_cast<const float4*>(row + from), b = *reinterpret_cast<const float4*>(row + from + 4);
-      v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+#pragma unroll
+      for (int u = 0; u < kHeld; u += 4) {
+        const float4 a = *reinterpret_cast<const float4*>(row + from + u);
+        v[u] = a.x, v[u + 1] = a.y, v[u + 2] = a.z, v[u + 3] = a.w;
+      }
     } else {
 #pragma unroll
       for (int u = 0; u < kHeld; ++u) v[u] = from + u < r_end ? row[from + u] : -INFINITY;
@@ -940,7 +1045,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   }
   float incl, chunk_total;
   const float excl = block_scan<float>(mine_run, scanf_, incl, chunk_total);  // (its barriers order the two writes above)
-  if (last_kept >= 0) atomicMax(&last_token, last_kept);
+  // (a wave's runs lie in the order of its lanes: the last that keeps a token speaks for it)
+  const unsigned long long keeping = __ballot(last_kept >= 0);
+  if (keeping != 0 && lane == kWave - 1 - __clzll(keeping)) atomicMax(&last_token, last_kept);
   if (sel_before + excl <= target && target < sel_before + incl) {
     float run = sel_before + excl;
     int pick = -1;
@@ -971,35 +1078,39 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
 
 // Whether a step's rows with thresholds are shared between blocks: two more kernels (some 8 us, and 0.3 us a row beside its
 // bytes) against passes of one block over its row alone, which all rows make side by side.  us with top-k / with top-p
-// alone, shared against a block a row: 151,936 logits, 1 row 30 / 40 against 44 / 95, 16 rows 34 / 51 and 45 / 106, 64 rows 61 / 88
-// and 61 / 125, 100 rows 84 / 117 and 66 / 130, 200 rows 136 / 187 and 78 / 151; 65,536 logits, 1 row 26 / 36 and 28 / 42, 16
-// rows 29 / 42 and 29 / 57, 64 rows 46 / 70 and 32 / 61; 32,003 logits, 1 row 25 / 30 and 22 / 27, 64 rows 44 / 64 and 25 / 41; 4,096
-// logits, 64 rows 40 / 52 and 19 / 21.
+// alone, shared against a block a row: 151,936 logits, 1 row 25 / 37 against 42 / 91, 16 rows 33 / 43 and 44 / 99, 64 rows 59 / 77
+// and 60 / 128, 77 rows 66 / 90 and 62 / 131, 140 rows 91 / 123 and 68 / 136; 65,536 logits, 1 row 23 / 28 and 27 / 43, 16
+// rows 29 / 37 and 28 / 50, 64 rows 47 / 62 and 31 / 54; 32,003 logits, 1 row 23 / 28 and 21 / 31, 64 rows 47 / 53 and 24 / 36.
 constexpr int kSharedVocabulary = 65536;
 inline bool shares_rows(int M, int V) { return V >= kSharedVocabulary && M <= (V - kSharedVocabulary / 2) / 1536; }
-constexpr size_t kSharedWords = 3 * kBins + 2;     // of a row: counts, masses, the list's length
+constexpr size_t kSharedWords = 3 * kHistWords + 2;     // of a row: counts, masses, the list's length
 
 TK_API int tk_sample_scratch_bytes(int M, int V) {
   const long rows = M < 1 ? 0 : M;
-  const long parts = rows * kArgmaxSegments * 12 + rows * 4 + 16;
+  const long parts = rows * kArgmaxSegments * 12 + rows * 4 + 16 + rows * 32;
   return (int)(parts + (shares_rows(M, V) ? rows * ((long)kSharedWords * 4 + (long)kCandidates * 5 + kArgmaxSegments * 8 + (long)sizeof(FirstLevel)) : 0));
 }
 
 // Every row's next token: greedy rows (temperature 0) their argmax, the others a draw; a row whose search falls through
-// (rounding at an edge) keeps its argmax.  scratch: tk_sample_scratch_bytes(M, V), on a 16-byte border.  thresholds: 0 where the
-// caller knows that no row has any; the kernels that share such rows are then left out.
-TK_API int tk_sample(const float* logits, long ld, int M, int V, const float* temperature,
-                     const int* top_k, const float* top_p, const unsigned long long* seeds,
-                     const unsigned long long* counters, int* out, float* probs_out, void* scratch, int thresholds, hipStream_t stream) {
+// (rounding at an edge) keeps its argmax.  scratch: tk_sample_scratch_bytes(M, V), on a 16-byte border.  params: seeds and draw counts
+// (M 64-bit numbers each), temperatures and top-p (M floats each), top-k (M integers) and the numbers of the `shared` rows that
+// have a threshold (integers; those kernels are left out where there are none), one behind the other, on an 8-byte border; in device memory, or (on_host,
+// up to tk_sample_inline_rows() rows) in host memory that is free again when the call returns.
+TK_API int tk_sample_inline_rows() { return kInlineRows; }
+
+TK_API int tk_sample(const float* logits, long ld, int M, int V, const void* params, int on_host, int shared, int* out, float* probs_out,
+                     void* scratch, hipStream_t stream) {
   if (M <= 0) return 0;
-  if (V <= 0 || M > 65535 || scratch == nullptr || (uintptr_t)scratch % 16 != 0) return -1;
-  const bool share = shares_rows(M, V) && thresholds != 0;
+  if (V <= 0 || M > 65535 || scratch == nullptr || (uintptr_t)scratch % 16 != 0 || params == nullptr || (uintptr_t)params % 8 != 0 ||
+      shared < 0 || shared > M || (on_host != 0 && M > kInlineRows))
+    return -1;
+  const bool share = shares_rows(M, V) && shared != 0;
   unsigned char* at = static_cast<unsigned char*>(scratch);
   SharedRows sh{};
-  if (share) {      // (per row: 2 kBins words of masses, kBins of counts, two of the list's length)
+  if (share) {      // (per row: 2 kHistWords words of masses, kHistWords of counts, two of the list's length)
     sh.hist64 = reinterpret_cast<unsigned long long*>(at);
-    sh.hist32 = reinterpret_cast<uint32_t*>(at + (size_t)M * kBins * 8);
-    sh.count = sh.hist32 + (size_t)M * kBins;
+    sh.hist32 = reinterpret_cast<uint32_t*>(at + (size_t)M * kHistWords * 8);
+    sh.count = sh.hist32 + (size_t)M * kHistWords;
     sh.above = reinterpret_cast<unsigned long long*>(at + (size_t)M * kSharedWords * 4);
     // (the argmax pass clears a row's words so far; M times an odd number of 8 bytes: still on their border)
     sh.level = reinterpret_cast<FirstLevel*>(at + (size_t)M * (kSharedWords * 4 + kArgmaxSegments * 8));
@@ -1014,15 +1125,40 @@ TK_API int tk_sample(const float* logits, long ld, int M, int V, const float* te
     sh.cand = reinterpret_cast<uint32_t*>(row_max + M);
     sh.segment = reinterpret_cast<uint8_t*>(sh.cand + (size_t)M * kCandidates);
   }
-  const dim3 shares(kArgmaxSegments, M);
-  argmax_segments_kernel<<<shares, kArgmaxThreads, 0, stream>>>(logits, seg_max, seg_index, V, ld, temperature, top_k, top_p, seg_mass, sh);
-  if (share) {
-    sample_hist_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, V, temperature, top_k, top_p, seg_max, seg_index, out, row_max, sh);
-    sample_collect_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, V, temperature, top_k, top_p, row_max, sh);
+  const auto laid_out = [M](const void* at) {
+    const unsigned long long* seeds = static_cast<const unsigned long long*>(at);
+    const float* temperature = reinterpret_cast<const float*>(seeds + 2 * M);
+    const int* top_k = reinterpret_cast<const int*>(temperature + 2 * M);
+    return RowParams{seeds, seeds + M, temperature, temperature + M, top_k, top_k + M};
+  };
+  const dim3 all(kArgmaxSegments, M);
+  RowParams rows;
+  if (on_host) {
+    // (behind the scratch of the rest, on its border of 8 bytes)
+    unsigned char* const end = static_cast<unsigned char*>(scratch) + tk_sample_scratch_bytes(M, V) - (size_t)M * 32;
+    rows = laid_out(reinterpret_cast<void*>((uintptr_t)end & ~(uintptr_t)7));
+    InlineParams in;
+    const RowParams from = laid_out(params);
+    std::memcpy(in.seeds, from.seeds, sizeof(*from.seeds) * M);
+    std::memcpy(in.draws, from.draws, sizeof(*from.draws) * M);
+    std::memcpy(in.temperature, from.temperature, sizeof(float) * M);
+    std::memcpy(in.top_p, from.top_p, sizeof(float) * M);
+    std::memcpy(in.top_k, from.top_k, sizeof(int) * M);
+    std::memcpy(in.rows, from.rows, sizeof(int) * shared);
+    for (int i = 0; i < shared; ++i)
+      if (in.rows[i] < 0 || in.rows[i] >= M) return -1;
+    in.to = rows;
+    in.shared = shared;
+    argmax_segments_kernel<<<all, kArgmaxThreads, 0, stream>>>(logits, seg_max, seg_index, V, ld, in, seg_mass, sh);
   } else {
-    argmax_pick_kernel<<<M, kWave, 0, stream>>>(seg_max, seg_index, out, row_max);
+    rows = laid_out(params);
+    argmax_segments_kernel<<<all, kArgmaxThreads, 0, stream>>>(logits, seg_max, seg_index, V, ld, rows, seg_mass, sh);
   }
-  sample_kernel<<<M, kSampleThreads, 0, stream>>>(logits, ld, V, temperature, top_k, top_p, seeds, counters,
-                                                  row_max, seg_max, seg_mass, out, probs_out, sh);
+  if (share) {
+    const dim3 shares(kArgmaxSegments, shared);
+    sample_hist_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, V, rows, seg_max, row_max, sh);
+    sample_collect_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, V, rows, row_max, sh);
+  }
+  sample_kernel<<<M, kSampleThreads, 0, stream>>>(logits, ld, V, rows, seg_max, seg_index, seg_mass, out, probs_out, sh);
   return launch_status();
 }

@@ -14,6 +14,7 @@ import struct
 import threading
 from ctypes import c_float, c_int, c_long, c_size_t, c_void_p
 
+import numpy as np
 import torch
 
 from tokamak_amd.kernels.build import load_library
@@ -379,8 +380,7 @@ _SIGS = {
     "sampling": {
         "tk_argmax": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_long, c_void_p],
         "tk_argmax_segments": [],
-        "tk_sample": [c_void_p, c_long, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
-                      c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
+        "tk_sample": [c_void_p, c_long, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
         "tk_sample_scratch_bytes": [c_int, c_int],
     },
 }
@@ -2829,25 +2829,30 @@ def argmax(logits: torch.Tensor, out: torch.Tensor, values: torch.Tensor | None 
                                         logits.stride(0), _stream()), "argmax")
 
 
-def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
-           top_p: torch.Tensor, seeds: torch.Tensor, counters: torch.Tensor, out: torch.Tensor,
-           probs_out: torch.Tensor | None = None, thresholds: bool = True) -> None:
-    """Temperature / top-k / top-p sampling, one row per request.  ``thresholds``: whether any row may have a top-k or
-    top-p that leaves tokens out; without, two launches that share such rows between blocks are left out."""
+SAMPLE_INLINE_ROWS = 64     # rows up to which the parameters travel as an argument of the launch (csrc/sampling.hip: kInlineRows)
+
+
+def sample(logits: torch.Tensor, params: torch.Tensor | np.ndarray, out: torch.Tensor, probs_out: torch.Tensor | None = None,
+           shared: int = 0) -> None:
+    """Temperature / top-k / top-p sampling, one row per request.  ``params`` int32: the rows' seeds and draw counts (64 bits each), temperatures
+    and top-p (float32), top-k, and the numbers of the ``shared`` rows that have a threshold, one behind the other; on the GPU, or,
+    of up to ``SAMPLE_INLINE_ROWS`` rows, a numpy array, which the launch takes along.  Two launches share the rows with a threshold between
+    blocks; without such rows they are left out."""
     _need(logits.is_cuda and logits.dim() == 2 and logits.stride(1) == 1 and logits.dtype == torch.float32,
           "logits are float32 [M, V] on the GPU")
-    _gpu(temperature, top_k, top_p, seeds, counters, out, probs_out)
+    _gpu(out, probs_out)
     m, v = logits.shape
-    _need(temperature.dtype == torch.float32 and top_p.dtype == torch.float32 and top_k.dtype == torch.int32,
-          "temperature/top_p float32, top_k int32")
-    _need(seeds.dtype == torch.int64 and counters.dtype == torch.int64, "seeds and counters are int64")
-    for t in (temperature, top_k, top_p, seeds, counters, out):
-        _need(t.numel() >= m, "one sampling parameter per row is required")
-    _need(out.dtype == torch.int32, "sample output is int32")
+    on_host = isinstance(params, np.ndarray)
+    if on_host:
+        _need(m <= SAMPLE_INLINE_ROWS and params.dtype == np.int32 and params.flags.c_contiguous and params.ctypes.data % 8 == 0
+              and params.size >= 7 * m + shared, "parameters on the host: int32, of up to 64 rows")
+    else:
+        _gpu(params)
+        _need(params.dtype == torch.int32 and params.numel() >= 7 * m + shared and params.data_ptr() % 8 == 0, "parameters are seven int32 a row and the rows with thresholds")
+    _need(0 <= shared <= m, "as many rows with thresholds as there are rows")
+    _need(out.dtype == torch.int32 and out.numel() >= m, "sample output is int32 [M]")
     _need(probs_out is None or (probs_out.dtype == torch.float32 and probs_out.shape == (m, v)), "probs_out is float32 [M, V]")
     _need(m <= 65535, "at most 65535 rows")
     scratch = torch.empty(_fn("sampling", "tk_sample_scratch_bytes")(m, v), dtype=torch.uint8, device=logits.device)
-    _check(_fn("sampling", "tk_sample")(_p(logits), logits.stride(0), m, v, _p(temperature), _p(top_k),
-                                        _p(top_p), _p(seeds), _p(counters), _p(out), _p(probs_out), _p(scratch),
-                                        int(bool(thresholds)), _stream()),
-           "sample")
+    _check(_fn("sampling", "tk_sample")(_p(logits), logits.stride(0), m, v, c_void_p(params.ctypes.data) if on_host else _p(params),
+                                        int(on_host), shared, _p(out), _p(probs_out), _p(scratch), _stream()), "sample")

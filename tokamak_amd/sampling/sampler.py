@@ -49,23 +49,19 @@ def sample_tokens(logits: torch.Tensor, params: list[SamplingParams], seeds: lis
     if all(p.is_greedy for p in params) and not return_probs:
         return greedy_tokens(logits, out)
     dev = logits.device
-    # one host buffer, one copy: [seeds | draws] int64, then [temperature | top_p] float32 and top_k int32
-    host = np.empty(7 * m, dtype=np.int32)
-    wide = host[:4 * m].view(np.int64)
-    wide[:m] = [s & 0x7FFFFFFFFFFFFFFF for s in seeds]
-    wide[m:] = draws
-    floats = host[4 * m:6 * m].view(np.float32)
-    floats[:m] = [p.temperature for p in params]
-    floats[m:] = [p.top_p for p in params]
-    host[6 * m:] = [p.top_k for p in params]
-    # through pinned memory and without waiting: a copy from pageable memory would hold the
-    # host until the GPU has run everything queued before it
-    packed = torch.from_numpy(host).pin_memory().to(dev, non_blocking=True)
-    seed_t, draw_t = packed[:2 * m].view(torch.int64), packed[2 * m:4 * m].view(torch.int64)
-    temperature, top_p = packed[4 * m:5 * m].view(torch.float32), packed[5 * m:6 * m].view(torch.float32)
-    top_k = packed[6 * m:]
+    temperatures, thresholds_p, thresholds_k = [p.temperature for p in params], [p.top_p for p in params], [p.top_k for p in params]
+    vocab = logits.shape[1]
+    shared = [i for i in range(m) if temperatures[i] > 0.0 and (thresholds_p[i] < 1.0 or 0 < thresholds_k[i] < vocab)]
+    # one host buffer: [seeds | draws] int64, then [temperature | top_p] float32, top_k and the rows with thresholds int32
+    host = np.empty(7 * m + len(shared), dtype=np.int32)
+    host[:4 * m].view(np.int64)[:] = [s & 0x7FFFFFFFFFFFFFFF for s in seeds] + list(draws)
+    host[4 * m:6 * m].view(np.float32)[:] = temperatures + thresholds_p
+    host[6 * m:] = thresholds_k + shared
+    if m > ops.SAMPLE_INLINE_ROWS:
+        # through pinned memory and without waiting: a copy from pageable memory would hold the
+        # host until the GPU has run everything queued before it
+        host = torch.from_numpy(host).pin_memory().to(dev, non_blocking=True)
     out = _output(out, m, dev)
     probs = torch.zeros_like(logits) if return_probs else None
-    thresholds = any(p.top_p < 1.0 or 0 < p.top_k < logits.shape[1] for p in params if not p.is_greedy)
-    ops.sample(logits, temperature, top_k, top_p, seed_t, draw_t, out, probs, thresholds)
+    ops.sample(logits, host, out, probs, len(shared))
     return (out, probs) if return_probs else out
