@@ -340,7 +340,7 @@ __device__ __forceinline__ float delta_token(const DeltaToken<PIECES>& x, f32x4 
 template <int PIECES, int TB, bool WIDE>
 __global__ __launch_bounds__(kScanThreads, 1) void delta_scan_kernel(
     const float* __restrict__ in, float* __restrict__ state, const int* __restrict__ q_start,
-    const int* __restrict__ state_slots, float* __restrict__ y, DeltaShape sh) {
+    const int* __restrict__ state_slots, float* __restrict__ y, DeltaShape sh, int least) {
   constexpr int DP = kLanes * 4 * PIECES;      // rows with the padding (zeros behind dim)
   constexpr int SET = TB * DP;
   constexpr int ALL = (3 * SET + TB * kColumns) / 4;      // pieces of four numbers that a round stages
@@ -350,6 +350,7 @@ __global__ __launch_bounds__(kScanThreads, 1) void delta_scan_kernel(
   float* bb = vv + TB * kColumns;
   const int req = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
   const int first = q_start[req], end = q_start[req + 1];
+  if (end - first >= least) return;            // (the whole block, before any barrier: delta_chunks.hip's work)
   const int ks = tid & (kLanes - 1), jl = tid / kLanes;
   const int col0 = blockIdx.z * kColumns, j = col0 + jl;
   const int dim = sh.dim, vdim = sh.vdim, row = sh.row();
@@ -501,8 +502,9 @@ TK_API int tk_delta_inputs(int dtype, const void* proj, int in_f32, int parts, l
 }
 
 // in: what tk_delta_inputs left; state float32 [slots, heads, vdim, dim rounded up to 4]; y float32 [N, heads * vdim].
+// Requests of `least` tokens and more are left alone.
 TK_API int tk_delta_scan(const float* in, float* state, const int* q_start, const int* state_slots, float* y, int R,
-                         int heads, int kv, int dim, int vdim, hipStream_t stream) {
+                         int heads, int kv, int dim, int vdim, int least, hipStream_t stream) {
   if (R <= 0) return 0;
   if (heads < 1 || heads > 65535 || kv < 1 || heads % kv != 0 || dim < 1 || dim > 512 || vdim < 1) return -1;
   const DeltaShape sh{heads, kv, dim, vdim, 1};
@@ -511,8 +513,8 @@ TK_API int tk_delta_scan(const float* in, float* state, const int* q_start, cons
   const bool wide = dim % 4 == 0 && vdim % 4 == 0 && (uintptr_t)in % 16 == 0;
 #define TK_DS(PIECES, TB)                                                                                              \
   {                                                                                                                    \
-    if (wide) delta_scan_kernel<PIECES, TB, true><<<grid, kScanThreads, 0, stream>>>(in, state, q_start, state_slots, y, sh); \
-    else delta_scan_kernel<PIECES, TB, false><<<grid, kScanThreads, 0, stream>>>(in, state, q_start, state_slots, y, sh);     \
+    if (wide) delta_scan_kernel<PIECES, TB, true><<<grid, kScanThreads, 0, stream>>>(in, state, q_start, state_slots, y, sh, least); \
+    else delta_scan_kernel<PIECES, TB, false><<<grid, kScanThreads, 0, stream>>>(in, state, q_start, state_slots, y, sh, least);     \
   }
   if (dim <= 64) TK_DS(1, 16)
   else if (dim <= 128) TK_DS(2, 16)

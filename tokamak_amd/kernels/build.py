@@ -29,7 +29,7 @@ HIPCC_FLAGS = [
     "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option",
 ]
 LIBRARIES = ("elementwise", "gemm_tiled", "gemm_float32", "attention_generic", "sampling", "gemm_mfma",
-             "gemm_wholek", "gemm_direct", "gemm_many", "gemm_flow", "attention_mfma", "blas_lt", "peaks", "replay", "attention_pooled", "attention_pooled_portions", "recurrent", "moe", "latent", "attention_tiles", "ssm", "delta", "linear_chunks", "scan_chunks", "ssm_chunks", "moe_operands")
+             "gemm_wholek", "gemm_direct", "gemm_many", "gemm_flow", "attention_mfma", "blas_lt", "peaks", "replay", "attention_pooled", "attention_pooled_portions", "recurrent", "moe", "latent", "attention_tiles", "ssm", "delta", "delta_chunks", "linear_chunks", "scan_chunks", "ssm_chunks", "moe_operands")
 # libraries a source links against (blas_lt is host code around hipBLASLt)
 LINK_FLAGS = {"blas_lt": ["-lhipblaslt"]}
 

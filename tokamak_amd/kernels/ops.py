@@ -369,7 +369,11 @@ _SIGS = {
         "tk_delta_inputs": [c_int, c_void_p, c_int, c_int, c_long, c_long, c_void_p, c_int, c_int, c_long, c_long,
                             c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                             c_int, c_int, c_int, c_float, c_int, c_void_p],
-        "tk_delta_scan": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
+        "tk_delta_scan": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+    },
+    "delta_chunks": {
+        "tk_delta_chunks": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
+                            c_int, c_void_p],
     },
     "attention_fused": {
         "tk_attention_decode_fused": [c_void_p, c_int, c_int, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
@@ -1410,6 +1414,7 @@ def _scan_chunks(batch, n: int, heads: int, state_size: int, vdim: int, device):
 
 
 DELTA_MAX_DIM = 512          # key channels of a head of the delta-rule scan (csrc/delta.hip)
+DELTA_CHUNKS_FROM_TOKENS = 160   # a request's tokens in a step from which it is scanned in chunks
 
 
 def delta_row(heads: int, kv_heads: int, dim: int, vdim: int) -> int:
@@ -1460,11 +1465,21 @@ def delta_inputs(proj: torch.Tensor, up: torch.Tensor, conv: torch.Tensor, conv_
         float(q_scale), batch.max_q_len, _stream()), "delta_inputs")
 
 
+def _delta_in_chunks(dim: int, vdim: int, longest: int) -> bool:
+    """Whether the delta rule's scan has requests that run in chunks of 16 tokens on the matrix cores: 160 tokens and more of
+    heads that are whole tiles.  The line looks at a request's own tokens alone, so that its bits do not depend on its
+    neighbours.  Walked and in chunks, us, heads of 128 x 128: 32 heads, one request of 64 tokens 15 and 21, of 128 25 and 26, of
+    256 48 and 40, of 2,048 357 and 200, sixteen of 128 223 and 227; 8 heads, one of 128 24 and 23, of 256 44 and 32, sixteen of 128
+    60 and 62."""
+    return longest >= DELTA_CHUNKS_FROM_TOKENS and dim % 16 == 0 and vdim % 16 == 0 and max(dim, vdim) <= SCAN_CHUNKS_MAX_DIM
+
+
 def delta_scan(operands: torch.Tensor, state: torch.Tensor, y: torch.Tensor, batch, *, heads: int, kv_heads: int, dim: int,
-               vdim: int) -> None:
+               vdim: int, chunks: bool = False) -> None:
     """Per request and head over the step's tokens in order: S <- diag(decay) S, u = beta (v - S^T k), S <- S + k u^T,
     y = S^T q, from the rows that ``delta_inputs`` leaves.  S float32 [slots, heads, vdim, dim rounded up to 4] (kept;
-    a value column's rows next to each other), y float32 [N, heads * vdim]."""
+    a value column's rows next to each other), y float32 [N, heads * vdim].  ``chunks``: long portions may be scanned in
+    chunks, whose bits depend on how a prompt is cut."""
     _gpu(operands, state, y)
     n = y.shape[0]
     _need(kv_heads >= 1 and heads % kv_heads == 0 and 1 <= dim <= DELTA_MAX_DIM and vdim >= 1, "the delta rule's sizes do not fit its kernels")
@@ -1476,8 +1491,18 @@ def delta_scan(operands: torch.Tensor, state: torch.Tensor, y: torch.Tensor, bat
     # (what a call has to move: the rows, the outputs, and every request's state in and out)
     _note(f"{n}x{heads}x{dim}x{vdim}", (operands.numel() + y.numel() + 2 * batch.num_requests * heads * dim * vdim) * 4,
           7.0 * n * heads * dim * vdim)
+    leave = EVERY_REQUEST
+    if chunks and _delta_in_chunks(dim, vdim, batch.max_q_len) and operands.data_ptr() % 16 == 0 and state.data_ptr() % 16 == 0:
+        leave = DELTA_CHUNKS_FROM_TOKENS
+        count, room = _tiles_of_long(batch.q_lens, n, SCAN_CHUNK, leave)
+        scaled = torch.empty((room, heads, 49 * dim + 16 * vdim + 256), dtype=torch.float32, device=y.device)
+        _check(_fn("delta_chunks", "tk_delta_chunks")(
+            _p(operands), _p(state), _p(batch.q_start), _p(batch.state_slots), _p(y), _p(scaled), batch.num_requests, leave, count,
+            heads, kv_heads, dim, vdim, _stream()), "delta_chunks")
+        if min(batch.q_lens) >= leave:
+            return
     _check(_fn("delta", "tk_delta_scan")(_p(operands), _p(state), _p(batch.q_start), _p(batch.state_slots), _p(y),
-                                         batch.num_requests, heads, kv_heads, dim, vdim, _stream()), "delta_scan")
+                                         batch.num_requests, heads, kv_heads, dim, vdim, leave, _stream()), "delta_scan")
 
 
 def gated_group_norm(y: torch.Tensor, proj: torch.Tensor, z_col: int, weight: torch.Tensor, out: torch.Tensor, *,

@@ -118,7 +118,8 @@ class ChannelDeltaRule(Mixer):
         ops.delta_inputs(proj, up, self.conv, store.state.get("conv"), self.a_log, self.dt_bias, operands, batch,
                          q_scale=self.head_dim ** -0.5, **sizes)
         y = torch.empty((n, self.num_heads * self.value_dim), dtype=torch.float32, device=h.device)
-        ops.delta_scan(operands, store.state["S"], y, batch, **sizes)
+        # (float32 keeps the walk a token at a time, whose bits do not depend on how a prompt is cut)
+        ops.delta_scan(operands, store.state["S"], y, batch, chunks=self.dtype == torch.bfloat16, **sizes)
         gated = torch.empty(y.shape, dtype=self.dtype, device=h.device)
         ops.gated_group_norm(y, up, self.num_heads * self.head_dim, self.gain, gated, groups=self.num_heads,
                              eps=self.norm_eps, gate_after=True)
