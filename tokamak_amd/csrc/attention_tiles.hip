@@ -4,9 +4,9 @@
 // bf16 in, float32 softmax and accumulation.  Tokens that run alone have a form of their own (third
 // kernel below) where a kv head has many query heads.
 //
-// A wave owns one tile (up to 16 consecutive tokens of one request) at one query head.  With fewer than
-// four query heads a kv head, the four waves of a block take four heads of the same tile and every wave
-// fetches its operands itself; with four and more, the waves of a block are heads of one kv head and
+// A wave owns one tile (up to 16 consecutive tokens of one request) at one query head.  With one query head a
+// kv head, and with two or three of more than 128 channels, the four waves of a block take four heads of the same tile and every
+// wave fetches its operands itself; else the waves of a block are heads of one kv head and
 // share the operands through LDS (second kernel below).  Keys are walked 16 at a time, operands straight from the pages (no LDS):
 //   S^T[key][token] = K[key][:] . Q[token][:]      v_mfma_f32_16x16x32_bf16, K rows as A (a lane
 //       (key, kb) reads the 16-byte piece of dims 32 c + 8 kb of its key), Q rows as B, kept in registers
@@ -23,6 +23,7 @@
 // Cache pages: K [nkv][hd/8][ps][8], V [nkv][vd/16][ps/4][16][4]; ps a multiple of 16, so that 16
 // consecutive keys from a multiple of 16 lie in one page.
 #include "common.h"
+#include "lds_copy.h"
 #include "slots.h"
 #include "soft_cap.h"
 
@@ -164,15 +165,24 @@ __global__ __launch_bounds__(kHeadsPerBlock * 64) void attention_tiles_kernel(
   }
 }
 
-// The same products for kv heads with four query heads and more: a block of HB waves takes HB heads of
+// The same products for kv heads with several query heads: a block of HB waves takes HB heads of
 // ONE kv head at one tile and shares every 16 keys' operands through LDS (each wave of the kernel above
 // fetches them from L2 for itself: with 32 heads on one kv head that is L2's rate, not the matrix
 // cores').  A stage is the 16 keys' slice of the K page (hd/8 runs of 256 bytes) and of the V page
 // (vd/16 runs of 512 bytes), copied as they lie, so the operand reads are those of the pages: a lane's
-// 16-byte key piece at ((4 c + kb) 16 + key) 8, its 8-byte value piece at ((4 d + kb) 16 + dim) 4.  Two
-// stages: the next one is fetched into registers before this one's products and written after them,
-// one barrier a stage.  Operands are read from LDS per instruction, which leaves a wave under 256
-// registers: two waves a SIMD.
+// 16-byte key piece at ((4 c + kb) 16 + key) 8, its 8-byte value piece at ((4 d + kb) 16 + dim) 4.
+// A ring of four stages, copied from the pages to LDS without registers (lds_copy.h) three stages ahead of their
+// products, the pages' numbers a stage before that; one barrier a stage.  A stage's products are shorter than a trip to memory:
+// fetched through registers one stage ahead, with the page's number asked for on the way, a stage of 512 + 448 channels took 5 us.
+// 2,048 tokens, 32 heads on one kv head of 512 / 448 channels, window 1,024: 690 -> 280 us (0.35 PFLOP/s); 32 / 8 heads of 128,
+// window 1,024 + 4: 192 -> 118.  What bounds it now: a stage's chain (barrier, scores, softmax, output) at two waves a SIMD, some
+// 4,500 clocks a stage of 960 channels of which LDS is busy 1,900 and the matrix cores 1,000.
+// Also for two and three heads a kv head where a ring is 32 KB (16 / 8 heads of 128, 1,024 tokens 88 -> 71 us, 300 behind
+// 2,000 96 -> 65); of larger heads a block of two waves would have the CU's LDS to itself.
+// Operands are read from LDS per instruction, which leaves a wave under 256 registers: two waves a SIMD.
+constexpr int kStages = 4;
+__host__ __device__ constexpr int stage_kb(int channels) { return (2 * channels + 63) / 64; }      // of 16 keys: whole runs of 64 pieces
+
 template <int KCH, int DBL, int HB, bool CAP>
 __global__ __launch_bounds__(HB * 64) void attention_tiles_shared_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
@@ -180,17 +190,17 @@ __global__ __launch_bounds__(HB * 64) void attention_tiles_shared_kernel(
     const int* __restrict__ req_of_token, const int* __restrict__ tile_first, const int* __restrict__ tile_count,
     bf16_t* __restrict__ out, int nh, int nkv, int hd, int vd, int ps, float scale_log2, int span, int keep,
     const float* __restrict__ sinks, SoftCap cap) {
-  extern __shared__ __attribute__((aligned(16))) bf16_t stage_s[];   // two stages of (hd + vd) * 16 elements
-  constexpr int THREADS = HB * 64;
-  constexpr int KPT = (KCH * 64 + THREADS - 1) / THREADS;    // 16-byte pieces of K (hd / 8 * 16 = 2 hd) a thread copies
-  constexpr int VPT = (DBL * 32 + THREADS - 1) / THREADS;    // and of V (vd / 16 * 32 = 2 vd)
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, kb = lane >> 4;
+  extern __shared__ __attribute__((aligned(16))) bf16_t stage_s[];   // kStages stages of stage_bytes(hd, vd)
+  constexpr int PER = (KCH + DBL / 2 + HB - 1) / HB;                  // KB of a stage that a wave copies
+  // chunks and blocks of a group (two groups' reads are held in registers), and those that are walked or passed over together
+  constexpr int KG = KCH > 4 ? 2 : 4, KPART = KCH > 4 ? KCH / 2 : KCH, VG = DBL > 8 ? 4 : 8, VPART = DBL > 8 ? DBL / 2 : DBL;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, kb = lane >> 4;
   const int group = nh / nkv, blocks_per_kv = (group + HB - 1) / HB;
   const int kvh = blockIdx.y / blocks_per_kv;
   const int in_group = (blockIdx.y % blocks_per_kv) * HB + wave;
   const bool computes = in_group < group;                   // (a wave without a head still copies and waits)
   const int head = kvh * group + (computes ? in_group : 0);
-  const int tile = blockIdx.x;
+  const int tile = gridDim.x - 1 - blockIdx.x;              // (a portion's last tiles walk furthest: they start first)
   const int n0 = tile_first[tile], cnt = tile_count[tile];
   const int pos0 = positions[n0];
   const int my = min(col, cnt - 1);
@@ -202,8 +212,7 @@ __global__ __launch_bounds__(HB * 64) void attention_tiles_shared_kernel(
   const size_t k_page = (size_t)nkv * hd * ps, v_page = (size_t)nkv * vd * ps;
   const size_t k_head = (size_t)kvh * hd * ps, v_head = (size_t)kvh * vd * ps;
   const int kch = (hd + 31) >> 5, dbl = vd >> 4;
-  const int k_pieces = 2 * hd, v_pieces = 2 * vd;           // 16-byte pieces of a stage
-  const int stage_elems = (hd + vd) * 16;
+  const int k_kb = stage_kb(hd), all_kb = k_kb + stage_kb(vd);
 
   bf16x8 qreg[KCH];
   const bf16_t* qp = q + ((size_t)(n0 + my) * nh + head) * hd + kb * 8;
@@ -213,67 +222,106 @@ __global__ __launch_bounds__(HB * 64) void attention_tiles_shared_kernel(
     f.u = (c * 32 + kb * 8 < hd) ? *reinterpret_cast<const uint4*>(qp + c * 32) : make_uint4(0, 0, 0, 0);
     qreg[c] = f.v;
   }
+  // (the queries are here before the first copy is asked for: a wait for them in the walk would be one for every copy)
+#pragma unroll
+  for (int c = 0; c < KCH; ++c) asm volatile("" : "+v"(qreg[c]));
   float m_run = -INFINITY, l_run = 0.f;
   float4v acc[DBL];
 #pragma unroll
   for (int d = 0; d < DBL; ++d) acc[d] = float4v{0.f, 0.f, 0.f, 0.f};
 
-  uint4 kt[KPT], vt[VPT];
-  // piece p of K: run j = p / 16 (8 dims), key p % 16; piece p of V: block d = p / 32, 16 bytes r = p % 32 of its 512
-#define TK_SFETCH(C0_)                                                                                         \
-  {                                                                                                            \
-    const int page_ = table[(C0_) / ps], off_ = (C0_) % ps;                                                    \
-    const bf16_t* kp_ = k_cache + (size_t)page_ * k_page + k_head + (size_t)off_ * 8;                          \
-    const bf16_t* vp_ = v_cache + (size_t)page_ * v_page + v_head + (size_t)(off_ >> 2) * 64;                  \
-    _Pragma("unroll") for (int i = 0; i < KPT; ++i) {                                                          \
-      const int p_ = i * THREADS + threadIdx.x;                                                                \
-      if (p_ < k_pieces) kt[i] = *reinterpret_cast<const uint4*>(kp_ + ((size_t)(p_ >> 4) * ps + (p_ & 15)) * 8); \
-    }                                                                                                          \
-    _Pragma("unroll") for (int i = 0; i < VPT; ++i) {                                                          \
-      const int p_ = i * THREADS + threadIdx.x;                                                                \
-      if (p_ < v_pieces) vt[i] = *reinterpret_cast<const uint4*>(vp_ + (size_t)(p_ >> 5) * (ps >> 2) * 64 + (p_ & 31) * 8); \
-    }                                                                                                          \
+  // What this wave copies of a stage: PER runs of 64 pieces of 16 bytes, of K (piece p: 8 dims p / 16, key p % 16) or of V (block
+  // p / 32, 16 bytes p % 32 of its 512).  Runs behind the last are the last once more (every wave copies as much, so that its
+  // count of copies says which stage has come), pieces behind the last of K or V its last.
+  uint32_t from[PER], to[PER];
+  bool of_k[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int run = min(wave + i * HB, all_kb - 1);
+    of_k[i] = run < k_kb;
+    const int piece = min((of_k[i] ? run : run - k_kb) * 64 + lane, 2 * (of_k[i] ? hd : vd) - 1);
+    from[i] = of_k[i] ? (uint32_t)(((piece >> 4) * ps + (piece & 15)) * 16)
+                      : (uint32_t)((piece >> 5) * (ps >> 2) * 128 + (piece & 31) * 16);
+    to[i] = run * 1024;
   }
-#define TK_SSTORE(BUF_)                                                                                        \
-  {                                                                                                            \
-    bf16_t* ks_ = stage_s + (size_t)(BUF_) * stage_elems;                                                      \
-    bf16_t* vs_ = ks_ + hd * 16;                                                                               \
-    _Pragma("unroll") for (int i = 0; i < KPT; ++i) {                                                          \
-      const int p_ = i * THREADS + threadIdx.x;                                                                \
-      if (p_ < k_pieces) *reinterpret_cast<uint4*>(ks_ + (size_t)p_ * 8) = kt[i];                              \
-    }                                                                                                          \
-    _Pragma("unroll") for (int i = 0; i < VPT; ++i) {                                                          \
-      const int p_ = i * THREADS + threadIdx.x;                                                                \
-      if (p_ < v_pieces) *reinterpret_cast<uint4*>(vs_ + (size_t)p_ * 8) = vt[i];                              \
-    }                                                                                                          \
-  }
+  const uint32_t lds = (uint32_t)(uintptr_t)(TK_LDS char*)stage_s, stage_size = all_kb * 1024;
   const int c_first = lo & ~15;
   const int c_start = keep > 0 ? 0 : c_first;
-  TK_SFETCH(c_start)
-  TK_SSTORE(0)
-  __syncthreads();
-  int buf = 0;
-  for (int c0 = c_start, c_next; c0 <= hi; c0 = c_next, buf ^= 1) {
-    c_next = (c0 + 16 >= keep && c0 + 16 < c_first) ? c_first : c0 + 16;    // (past the kept first positions: on to the window)
-    const bool more = c_next <= hi;
-    if (more) TK_SFETCH(c_next)
-    if (computes) {
-      const bf16_t* ks = stage_s + (size_t)buf * stage_elems;
-      const bf16_t* vs = ks + hd * 16;
-      float4v sc = {0.f, 0.f, 0.f, 0.f}, sc2 = {0.f, 0.f, 0.f, 0.f};
+  const auto behind = [&](int c) { return (c + 16 >= keep && c + 16 < c_first) ? c_first : c + 16; };   // (past the kept first positions: on to the window)
+  const auto copy = [&](int c, int page, int slot) {
+    const int off = c % ps;
+    const char* const kp = reinterpret_cast<const char*>(k_cache + (size_t)page * k_page + k_head + (size_t)off * 8);
+    const char* const vp = reinterpret_cast<const char*>(v_cache + (size_t)page * v_page + v_head + (size_t)(off >> 2) * 64);
 #pragma unroll
-      for (int c = 0; c < KCH; c += 2) {
-        if (c < kch) {     // (the same for every lane; a piece behind the key's end is absent from the stage: zeros)
-          Frag8 kf;
-          kf.u = (c * 32 + kb * 8 < hd) ? *reinterpret_cast<const uint4*>(ks + ((size_t)(c * 4 + kb) * 16 + col) * 8)
-                                        : make_uint4(0, 0, 0, 0);
-          sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf.v, qreg[c], sc, 0, 0, 0);
-        }
-        if (c + 1 < kch) {
-          Frag8 kf;
-          kf.u = ((c + 1) * 32 + kb * 8 < hd) ? *reinterpret_cast<const uint4*>(ks + ((size_t)((c + 1) * 4 + kb) * 16 + col) * 8)
-                                              : make_uint4(0, 0, 0, 0);
-          sc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf.v, qreg[c + 1], sc2, 0, 0, 0);
+    for (int i = 0; i < PER; ++i) copy_to_lds<false>(lds + slot * stage_size + to[i], from[i], of_k[i] ? kp : vp);
+  };
+  int c_copy = c_start, slot_copy = 0, ahead = 0;      // the next stage to copy, its place, stages copied and not yet used
+#pragma unroll
+  for (int i = 0; i < kStages - 1; ++i) {
+    if (c_copy <= hi) {
+      copy(c_copy, table[c_copy / ps], slot_copy++);
+      c_copy = behind(c_copy);
+      ++ahead;
+    }
+  }
+  int page_copy = c_copy <= hi ? table[c_copy / ps] : 0;
+  int buf = 0;
+  for (int c0 = c_start; c0 <= hi; c0 = behind(c0)) {
+    // this wave's part of the stage has come when only those of the stages behind it are on their way; everyone's, behind the
+    // barrier, where nobody reads the stage before any more either: its place is the next copy's
+    static_assert(kStages == 4, "the counts below");
+    if (ahead >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER) : "memory");
+    else if (ahead == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    --ahead;
+    if (c_copy <= hi) {
+      copy(c_copy, page_copy, slot_copy);
+      slot_copy = (slot_copy + 1) % kStages;
+      c_copy = behind(c_copy);
+      ++ahead;
+      if (c_copy <= hi) page_copy = table[c_copy / ps];
+    }
+    if (c0 + 15 > hi) {      // the last stage: values of positions that hold nothing yet are zeros, whatever their weight of zero meets
+      bf16_t* const vz = stage_s + (size_t)buf * (stage_size / 2) + k_kb * 512;
+      for (int p = threadIdx.x; p < vd * 4; p += HB * 64) {      // 8 bytes: keys 4 (p / 16 % 4) .. + 3 of a channel
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c0 + (p >> 4 & 3) * 4 + e > hi) vz[(size_t)p * 4 + e] = 0;
+      }
+      __syncthreads();
+    }
+    if (computes) {
+      const bf16_t* ks = stage_s + (size_t)buf * (stage_size / 2);
+      const bf16_t* vs = ks + k_kb * 512;
+      // Operands are asked for a group ahead of the group whose products run, with nothing that branches around a read: a read
+      // behind a branch of its own is waited for there.
+      float4v sc = {0.f, 0.f, 0.f, 0.f}, sc2 = {0.f, 0.f, 0.f, 0.f};
+      const auto keys = [&](int c) { return *reinterpret_cast<const uint4*>(ks + (size_t)((c * 4 + kb) * 16 + col) * 8); };
+#pragma unroll
+      for (int part = 0; part < KCH; part += KPART) {
+        if (part >= kch) continue;      // (the same for every lane)
+        Frag8 kf[2][KG];
+#pragma unroll
+        for (int i = 0; i < KG; ++i) kf[0][i].u = keys(part + i);
+#pragma unroll
+        for (int c = part; c < part + KPART; c += KG) {
+          Frag8(&now)[KG] = kf[c / KG & 1];
+          if (c + KG < part + KPART) {
+#pragma unroll
+            for (int i = 0; i < KG; ++i) kf[(c / KG & 1) ^ 1][i].u = keys(c + KG + i);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          if ((c + KG) * 32 > hd) {      // (pieces behind the key's end: zeros, whatever lies there)
+#pragma unroll
+            for (int i = 0; i < KG; ++i)
+              if ((c + i) * 32 + kb * 8 >= hd) now[i].u = make_uint4(0, 0, 0, 0);
+          }
+#pragma unroll
+          for (int i = 0; i < KG; i += 2) {
+            sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(now[i].v, qreg[c + i], sc, 0, 0, 0);
+            sc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(now[i + 1].v, qreg[c + i + 1], sc2, 0, 0, 0);
+          }
         }
       }
       sc += sc2;
@@ -301,29 +349,31 @@ __global__ __launch_bounds__(HB * 64) void attention_tiles_shared_kernel(
       l_run = l_run * alpha + psum;
       Frag4 pb;
       pb.u = make_uint2(pack_bf16x2(pr[0], pr[1]), pack_bf16x2(pr[2], pr[3]));
-      const bool edge = c0 + 15 > hi;
-      const bool rescale = __builtin_amdgcn_ballot_w64(alpha != 1.f) != 0;
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
-      for (int d = 0; d < DBL; ++d) {
-        if (d >= dbl) continue;
-        Frag4 vf;
-        vf.u = *reinterpret_cast<const uint2*>(vs + ((size_t)(d * 4 + kb) * 16 + col) * 4);
-        short4v tv = vf.v;
-        if (edge) {
+        for (int d = 0; d < DBL; ++d) acc[d] *= alpha;
+      }
+      const auto values = [&](int d) { return *reinterpret_cast<const uint2*>(vs + (size_t)((d * 4 + kb) * 16 + col) * 4); };
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (c0 + kb * 4 + e > hi) tv[e] = 0;
+      for (int part = 0; part < DBL; part += VPART) {
+        if (part >= dbl) continue;
+        Frag4 vf[2][VG];              // (of blocks behind the last whatever lies there, in sums that are never stored)
+#pragma unroll
+        for (int i = 0; i < VG; ++i) vf[0][i].u = values(part + i);
+#pragma unroll
+        for (int d = part; d < part + VPART; d += VG) {
+          if (d + VG < part + VPART) {
+#pragma unroll
+            for (int i = 0; i < VG; ++i) vf[(d / VG & 1) ^ 1][i].u = values(d + VG + i);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < VG; ++i) acc[d + i] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf[d / VG & 1][i].v, pb.v, acc[d + i], 0, 0, 0);
         }
-        float4v a = acc[d];
-        if (rescale) a *= alpha;
-        acc[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(tv, pb.v, a, 0, 0, 0);
       }
     }
-    if (more) TK_SSTORE(buf ^ 1)
-    __syncthreads();
+    buf = (buf + 1) % kStages;
   }
-#undef TK_SFETCH
-#undef TK_SSTORE
 
   if (!computes) return;
   float l = l_run;
@@ -349,12 +399,14 @@ static int launch_shared(const void* q, const void* k_cache, const void* v_cache
                          int num_tiles, void* out, int nh, int nkv, int hd, int vd, int ps, float scale, int span, int keep,
                          const float* sinks, float softcap, hipStream_t stream) {
   const int group = nh / nkv;
-  const size_t lds = (size_t)2 * (hd + vd) * 16 * sizeof(bf16_t);
+  // (up to 128 KB; reads of chunks and blocks behind the true sizes stay inside, also in the last stage)
+  const int all_kb = stage_kb(hd) + stage_kb(vd);
+  const size_t lds = (size_t)(kStages * all_kb + KCH + DBL / 2 - all_kb) * 1024;
   if (lds > 48 * 1024) {
     static bool raised = false;   // per template instance
     if (!raised) {
       if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_tiles_shared_kernel<KCH, DBL, HB, CAP>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024) != hipSuccess) {
+                              hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) != hipSuccess) {
         (void)hipGetLastError();
         return -2;
       }
@@ -549,15 +601,15 @@ TK_API int tk_attention_tiles(const void* q, const void* k_cache, const void* v_
       (uintptr_t)out % 8 != 0)
     return -2;
   const int group = nh / nkv;
-  if (group >= 4) {
-    // the heads of a kv head share its keys and values through LDS
+  if (group >= 4 || (group >= 2 && hd <= 128 && vd <= 128)) {
+    // the heads of a kv head share its keys and values through LDS (see the kernel: where the lines lie)
 #define TK_SHARED_AS(KCH_, DBL_, HB_, CAP_)                                                                     \
   launch_shared<KCH_, DBL_, HB_, CAP_>(q, k_cache, v_cache, block_tables, max_pages, positions, req_of_token,   \
                                        tile_first, tile_count, num_tiles, out, nh, nkv, hd, vd, ps, scale, span, \
                                        keep, sinks, softcap, stream)
 #define TK_SHARED(KCH_, DBL_, HB_) \
   (softcap > 0.f ? TK_SHARED_AS(KCH_, DBL_, HB_, true) : TK_SHARED_AS(KCH_, DBL_, HB_, false))
-    if (hd <= 128 && vd <= 128) return group > 4 ? TK_SHARED(4, 8, 8) : TK_SHARED(4, 8, 4);
+    if (hd <= 128 && vd <= 128) return group > 4 ? TK_SHARED(4, 8, 8) : group > 2 ? TK_SHARED(4, 8, 4) : TK_SHARED(4, 8, 2);
     if (hd <= 256 && vd <= 256) return group > 4 ? TK_SHARED(8, 16, 8) : TK_SHARED(8, 16, 4);
     return group > 4 ? TK_SHARED(16, 32, 8) : TK_SHARED(16, 32, 4);
 #undef TK_SHARED
