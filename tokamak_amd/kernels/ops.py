@@ -1492,7 +1492,8 @@ def delta_scan(operands: torch.Tensor, state: torch.Tensor, y: torch.Tensor, bat
     _note(f"{n}x{heads}x{dim}x{vdim}", (operands.numel() + y.numel() + 2 * batch.num_requests * heads * dim * vdim) * 4,
           7.0 * n * heads * dim * vdim)
     leave = EVERY_REQUEST
-    if chunks and _delta_in_chunks(dim, vdim, batch.max_q_len) and operands.data_ptr() % 16 == 0 and state.data_ptr() % 16 == 0:
+    if (chunks and _delta_in_chunks(dim, vdim, batch.max_q_len) and batch.num_requests <= 65535 and operands.data_ptr() % 16 == 0
+            and state.data_ptr() % 16 == 0):
         leave = DELTA_CHUNKS_FROM_TOKENS
         count, room = _tiles_of_long(batch.q_lens, n, SCAN_CHUNK, leave)
         scaled = torch.empty((room, heads, 49 * dim + 16 * vdim + 256), dtype=torch.float32, device=y.device)
