@@ -19,6 +19,7 @@
 // With more than one split the block writes an unnormalised partial (o, m, l) and
 // a second kernel merges the splits of each (token, head).
 #include "common.h"
+#include "lds_limit.h"
 #include "slots.h"
 #include "soft_cap.h"
 
@@ -1383,15 +1384,8 @@ static int launch_prefill_group(const void* q, const void* k_cache, const void* 
   constexpr size_t lds = stage_bytes > merge_bytes ? stage_bytes : merge_bytes;
   static_assert(lds <= 160 * 1024, "a stage must fit the CU's LDS");
   if (lds > 48 * 1024) {
-    static bool raised[2] = {false, false};  // per template instance
-    if (!raised[capped]) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
-          hipSuccess) {
-        (void)hipGetLastError();
-        return -2;
-      }
-      raised[capped] = true;
-    }
+    static LdsLimits limits[2];      // per template instance
+    if (!raise_lds_limit(reinterpret_cast<const void*>(kernel), lds, limits[capped])) return -2;
   }
   dim3 grid(nkv * ((G + GB - 1) / GB), num_items);
   kernel<<<grid, GB * S * 64, lds, stream>>>(
@@ -1452,15 +1446,8 @@ static int launch(const void* q, const void* k_cache, const void* v_cache, const
   const size_t lds = (size_t)(kDecodeWaves * G * HD + 2 * kDecodeWaves * 16) * 4 + (FUSED ? (size_t)(G + 2) * HD * 2 : 0);
   if (lds > 160 * 1024) return -2;
   if (lds > 48 * 1024) {  // beyond the default limit of dynamic LDS (at a head size of 128, groups of 12 heads and more, FUSED 11)
-    static bool raised[2] = {false, false};  // per template instance
-    if (!raised[capped]) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) !=
-          hipSuccess) {
-        (void)hipGetLastError();
-        return -2;
-      }
-      raised[capped] = true;
-    }
+    static LdsLimits limits[2];      // per template instance
+    if (!raise_lds_limit(reinterpret_cast<const void*>(kernel), 160 * 1024, limits[capped])) return -2;
   }
   kernel<<<grid, kDecodeWaves * 64, lds, stream>>>(
       (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, max_pages, positions,

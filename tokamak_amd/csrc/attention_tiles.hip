@@ -24,6 +24,7 @@
 // consecutive keys from a multiple of 16 lie in one page.
 #include "common.h"
 #include "lds_copy.h"
+#include "lds_limit.h"
 #include "slots.h"
 #include "soft_cap.h"
 
@@ -403,15 +404,8 @@ static int launch_shared(const void* q, const void* k_cache, const void* v_cache
   const int all_kb = stage_kb(hd) + stage_kb(vd);
   const size_t lds = (size_t)(kStages * all_kb + KCH + DBL / 2 - all_kb) * 1024;
   if (lds > 48 * 1024) {
-    static bool raised = false;   // per template instance
-    if (!raised) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_tiles_shared_kernel<KCH, DBL, HB, CAP>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) != hipSuccess) {
-        (void)hipGetLastError();
-        return -2;
-      }
-      raised = true;
-    }
+    static LdsLimits limits;      // per template instance
+    if (!raise_lds_limit(reinterpret_cast<const void*>(&attention_tiles_shared_kernel<KCH, DBL, HB, CAP>), 128 * 1024, limits)) return -2;
   }
   const dim3 grid(num_tiles, nkv * ((group + HB - 1) / HB));
   if (grid.y > 65535) return -1;

@@ -9,6 +9,7 @@
 // (chunk_outputs).  Powers of a never exceed one.  All of it is float32: the products are the float32
 // matrix instruction's (16 x 16 x 4), the operands are rounded nowhere behind the projection.
 #include "common.h"
+#include "lds_limit.h"
 #include "short_conv.h"
 #include "slots.h"
 
@@ -218,13 +219,10 @@ int launch(RowsIn in, const float* decay, float* state, const int* q_start, cons
   const int kp = sh.dk() + 4, vp = sh.dv() + 4;
   const size_t sums_lds = ((size_t)kChunk * (kp + vp) + kChunk) * 4;
   const size_t out_lds = ((size_t)kChunk * (kp + max(kp, kChunk + 4) + vp) + kChunk + 1) * 4;
-  static bool raised = false;
-  if (!raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&chunk_sums_kernel<T, WIDE>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&chunk_outputs_kernel<T, WIDE>), hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) != hipSuccess)
-      return -1;
-    raised = true;
-  }
+  static LdsLimits sums_limits, outputs_limits;
+  if (!raise_lds_limit(reinterpret_cast<const void*>(&chunk_sums_kernel<T, WIDE>), 128 * 1024, sums_limits) ||
+      !raise_lds_limit(reinterpret_cast<const void*>(&chunk_outputs_kernel<T, WIDE>), 128 * 1024, outputs_limits))
+    return -1;
   const dim3 grid(R * max_chunks, sh.heads);
   chunk_sums_kernel<T, WIDE><<<grid, kThreads, sums_lds, stream>>>(in, decay, q_start, chunk_state, sh, max_chunks);
   chunk_starts_kernel<<<dim3(R, sh.heads, (sh.elems() + 255) / 256), 256, 0, stream>>>(state, decay, q_start, slots, chunk_state,

@@ -20,6 +20,7 @@
 // Step sizes, decays with their exponentials, the recurrence, its state, the gate's product and the
 // norm are float32 whatever the storage type; x, B and C enter as the convolution stored them.
 #include "common.h"
+#include "lds_limit.h"
 #include "short_conv.h"
 #include "slots.h"
 
@@ -480,13 +481,9 @@ int launch_scan(const void* u, int C, SsmIn dt, long ld, int dt_col, const float
 #define TK_SSD_AS(RS, KS, MODE)                                                                               \
   {                                                                                                           \
     if (lds > 48 * 1024) {                                                                                    \
-      static bool raised = false;                                                                             \
-      if (!raised) {                                                                                          \
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&ssd_scan_kernel<T, RS, KS, MODE, SILU>),             \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 72 * 1024) != hipSuccess)         \
-          return -1;                                                                                          \
-        raised = true;                                                                                        \
-      }                                                                                                       \
+      static LdsLimits limits;                                                                                \
+      if (!raise_lds_limit(reinterpret_cast<const void*>(&ssd_scan_kernel<T, RS, KS, MODE, SILU>), 72 * 1024, limits)) \
+        return -1;                                                                                            \
     }                                                                                                         \
     ssd_scan_kernel<T, RS, KS, MODE, SILU><<<grid, threads, lds, stream>>>((const T*)u, C, dt, ld, dt_col, dt_bias, \
                                                                     a_log, skip, state, q_start, state_slots, \
