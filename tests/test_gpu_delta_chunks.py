@@ -24,7 +24,7 @@ def recurrence(q, k, v, a, beta, state):
 @pytest.mark.parametrize("heads,kv,dim,vdim,spans", [
     (2, 2, 128, 128, [129]), (4, 2, 64, 64, [16, 1, 47]), (8, 8, 16, 16, [32]), (3, 1, 48, 32, [100, 15, 17]),
     (4, 4, 80, 112, [64, 2]), (2, 1, 128, 16, [33, 400]),
-    (2, 2, 16, 128, [31, 5])])
+    (2, 2, 16, 128, [31, 5]), (3, 1, 96, 128, [100, 15, 17]), (2, 2, 112, 112, [47, 400]), (8, 4, 80, 128, [64, 2, 33])])
 @pytest.mark.parametrize("decays", ["slow", "fast", "none"])
 def test_chunks(heads, kv, dim, vdim, spans, decays, monkeypatch):
     from tokamak_amd.kernels import ops

@@ -36,6 +36,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTokens = 16;       // tokens of a chunk
 constexpr int kMaxDim = 128;
+constexpr int kTiles = 2;         // of 16 key channels that a wave of the walk holds (the last of them may not exist)
 
 struct Shape {
   int R, heads, kv, dim, vdim, least;
@@ -50,7 +51,7 @@ struct Shape {
   __host__ __device__ size_t floats() const { return (size_t)49 * dim + 256 + (size_t)16 * vdim; }
 };
 
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void delta_operands_kernel(const float* __restrict__ in, const int* __restrict__ q_start,
+__global__ __launch_bounds__(2 * kWave) __attribute__((amdgpu_waves_per_eu(2))) void delta_operands_kernel(const float* __restrict__ in, const int* __restrict__ q_start,
                                                              float* __restrict__ operands, Shape sh) {
   constexpr int kPitch = 64 + 4, kTriPitch = 16 + 4;
   static_assert(kPitch * kTokens >= 512 && kPitch >= kTriPitch, "what follows the rounds lies where they had their rows");
@@ -74,10 +75,9 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void d
   const int x = lane & 15, g = lane >> 4;
   const float beta_of_lane = x < n ? x0[(size_t)x * row + sh.b_at() + head] : 0.f;
   f32x4 v[kMaxDim / 32];           // this wave's tiles of 16 value columns (asked for here: a wait for a load waits for the stores before it, too)
-  const int waves = blockDim.x / kWave;
 #pragma unroll
   for (int s = 0; s < kMaxDim / 32; ++s) {
-    const int v0 = min(16 * (wave + s * waves), sh.vdim - 16);
+    const int v0 = min(16 * (wave + 2 * s), sh.vdim - 16);
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[s][r] = x0[(size_t)min(4 * g + r, n - 1) * row + sh.v_at() + head * sh.vdim + v0 + x];
   }
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void d
   }
   // M and A: lane (i = lane & 15 as a row, j = lane & 15 as a column); D holds column j = lane & 15, rows 4 (lane >> 4) + r
   f32x4 m = {0.f, 0.f, 0.f, 0.f}, av = {0.f, 0.f, 0.f, 0.f};
-  const int steps = max(0, min(4, (sh.dim - wave * kWave + 15) / 16));
+  const int steps = min(4, sh.dim / 16 - 4 * wave);
 #pragma unroll
   for (int round = 0; round < 5; ++round) {
     const int half = round < 4 ? 8 >> round : 0;
@@ -161,10 +161,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void d
   *reinterpret_cast<f32x4*>(ql + 4 * lane) = m;
   *reinterpret_cast<f32x4*>(ql + 256 + 4 * lane) = av;
   __syncthreads();
-  if (blockDim.x > kWave) {
-    m = *reinterpret_cast<const f32x4*>(rows[0][0] + 4 * lane) + *reinterpret_cast<const f32x4*>(rows[1][0] + 4 * lane);
-    av = *reinterpret_cast<const f32x4*>(rows[0][0] + 256 + 4 * lane) + *reinterpret_cast<const f32x4*>(rows[1][0] + 256 + 4 * lane);
-  }
+  m = *reinterpret_cast<const f32x4*>(rows[0][0] + 4 * lane) + *reinterpret_cast<const f32x4*>(rows[1][0] + 4 * lane);
+  av = *reinterpret_cast<const f32x4*>(rows[0][0] + 256 + 4 * lane) + *reinterpret_cast<const f32x4*>(rows[1][0] + 256 + 4 * lane);
   if (wave == 0) *reinterpret_cast<f32x4*>(mine + 49 * sh.dim + x * 16 + 4 * g) = av;
   // either wave finds T, column x a lane (its four groups of lanes the same), from above
   float* const tr = kl;
@@ -202,7 +200,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void d
   }
 #pragma unroll
   for (int s = 0; s < kMaxDim / 32; ++s) {
-    const int v0 = 16 * (wave + s * waves);
+    const int v0 = 16 * (wave + 2 * s);
     if (v0 >= sh.vdim) continue;
     f32x4 u = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -211,17 +209,15 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void d
   }
 }
 
-template <int TILES>
 struct WalkIn {        // a chunk's operands as a lane of the walk holds them
-  f32x4 q[TILES], w[TILES], k[TILES], d[TILES], u;
+  f32x4 q[kTiles], w[kTiles], k[kTiles], d[kTiles], u;
   float a;
 };
 
-// Four waves; wave w holds the tiles w and (TILES 2) w + 4 of 16 key channels of the block's 16 value columns: S[i][r] is
+// Four waves; wave w holds the tiles w and w + 4 of 16 key channels of the block's 16 value columns: S[i][r] is
 // channel 16 tile + 4 (lane >> 4) + r of column lane & 15.  One barrier a chunk: the waves' shares of W S meet behind it, their
 // shares of the outputs behind the next chunk's.  Operands are asked for kAhead chunks ahead, without a branch around any load.
 constexpr int kAhead = 4;
-template <int TILES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void delta_walk_kernel(const float* __restrict__ operands,
                                                          float* __restrict__ state, const int* __restrict__ q_start,
                                                          const int* __restrict__ state_slots, float* __restrict__ y, Shape sh) {
@@ -235,20 +231,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const float* op = operands + ((size_t)before * sh.heads + head) * sh.floats();
   const size_t pitch = sh.heads * sh.floats();
   float* const S = state + (((size_t)state_slots[req] * sh.heads + head) * sh.vdim + v0 + x) * sh.dim;
-  bool have[TILES];
-  int channel[TILES];       // the first of a tile's channels (of a tile that exists: loads need no branch)
-  f32x4 s[TILES];
+  bool have[kTiles];
+  int channel[kTiles];       // the first of a tile's channels (of a tile that exists: loads need no branch)
+  f32x4 s[kTiles];
 #pragma unroll
-  for (int i = 0; i < TILES; ++i) {
+  for (int i = 0; i < kTiles; ++i) {
     have[i] = 16 * (wave + 4 * i) < sh.dim;
     channel[i] = have[i] ? 16 * (wave + 4 * i) : 0;
     s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (have[i]) s[i] = *reinterpret_cast<const f32x4*>(S + channel[i] + 4 * g);
   }
   // (a chunk's numbers from a scalar address on, at 32-bit offsets a lane keeps: no address arithmetic in the walk)
-  uint32_t row_at[TILES], key_at[TILES], decay_at[TILES];
+  uint32_t row_at[kTiles], key_at[kTiles], decay_at[kTiles];
 #pragma unroll
-  for (int i = 0; i < TILES; ++i) {
+  for (int i = 0; i < kTiles; ++i) {
     row_at[i] = (x * sh.dim + channel[i] + 4 * g) * 4;
     key_at[i] = ((channel[i] + x) * kTokens + 4 * g) * 4;
     decay_at[i] = (channel[i] + 4 * g) * 4;
@@ -258,18 +254,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     asm volatile("" : "+v"(offset));      // (widened here, where the load can take a scalar base and a 32-bit offset)
     return base + offset;
   };
-  const auto fetch = [&](int ci, WalkIn<TILES>& in) {
+  const auto fetch = [&](int ci, WalkIn& in) {
     const char* const o = reinterpret_cast<const char*>(op + (size_t)min(ci, chunks - 1) * pitch);
     const uint32_t rows = 64 * sh.dim;      // bytes of 16 rows of channels
 #pragma unroll
-    for (int i = 0; i < TILES; ++i) in.w[i] = *reinterpret_cast<const f32x4*>(at(o + rows, row_at[i]));
+    for (int i = 0; i < kTiles; ++i) in.w[i] = *reinterpret_cast<const f32x4*>(at(o + rows, row_at[i]));
 #pragma unroll
-    for (int i = 0; i < TILES; ++i) in.q[i] = *reinterpret_cast<const f32x4*>(at(o, row_at[i]));
+    for (int i = 0; i < kTiles; ++i) in.q[i] = *reinterpret_cast<const f32x4*>(at(o, row_at[i]));
     in.u = *reinterpret_cast<const f32x4*>(at(o + 3 * rows + 4 * sh.dim + 1024, u_at));
 #pragma unroll
-    for (int i = 0; i < TILES; ++i) in.k[i] = *reinterpret_cast<const f32x4*>(at(o + 2 * rows, key_at[i]));
+    for (int i = 0; i < kTiles; ++i) in.k[i] = *reinterpret_cast<const f32x4*>(at(o + 2 * rows, key_at[i]));
 #pragma unroll
-    for (int i = 0; i < TILES; ++i) in.d[i] = *reinterpret_cast<const f32x4*>(at(o + 3 * rows, decay_at[i]));
+    for (int i = 0; i < kTiles; ++i) in.d[i] = *reinterpret_cast<const f32x4*>(at(o + 3 * rows, decay_at[i]));
     in.a = *reinterpret_cast<const float*>(at(o + 3 * rows + 4 * sh.dim, a_at));
   };
   const auto sum_of = [&](int half) {      // token 4 wave + g of a chunk: register g of lanes 16 wave ..
@@ -285,9 +281,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       *reinterpret_cast<float*>(reinterpret_cast<char*>(y_first + (size_t)ci * kTokens * VW) + y_at) = sum;
     }
   };
-  constexpr int kSums = 4 / TILES;
+  constexpr int kSums = 4 / kTiles;
   const bool odd = threadIdx.x & kWave, upper = threadIdx.x & (2 * kWave);      // (of the wave's number, as lane masks: no branches)
-  WalkIn<TILES> ahead[kAhead];
+  WalkIn ahead[kAhead];
 #pragma unroll
   for (int u = 0; u < kAhead; ++u) {
     fetch(u, ahead[u]);
@@ -299,14 +295,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int u = 0; u < kAhead; ++u) {
       // (no branch around a chunk: the loads in flight would be waited for there.  One past the last leaves nothing behind)
       const int ci = c0 + u;
-      const WalkIn<TILES>& now = ahead[u];
+      const WalkIn& now = ahead[u];
       f32x4 ks[4], o[4];      // (sums of eight channels each, then a tree: no more roundings than the walk's)
 #pragma unroll
       for (int i = 0; i < 4; ++i) ks[i] = o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int i = 0; i < TILES; ++i) {
+        for (int i = 0; i < kTiles; ++i) {
           f32x4& sum = ks[i * kSums + r % kSums];
           sum = __builtin_amdgcn_mfma_f32_16x16x4f32(now.w[i][r], s[i][r], sum, 0, 0, 0);
         }
@@ -321,22 +317,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int i = 0; i < TILES; ++i) {
+        for (int i = 0; i < kTiles; ++i) {
           f32x4& sum = o[i * kSums + r % kSums];
           sum = __builtin_amdgcn_mfma_f32_16x16x4f32(now.q[i][r], s[i][r], sum, 0, 0, 0);
         }
       const f32x4 un = now.u - ((rest[0] + rest[1]) + (rest[2] + rest[3]));      // u of token 4 r + g in register r
       put(ci < chunks + 1 ? ci - 1 : -1, sum);
-      f32x4 own[TILES];
+      f32x4 own[kTiles];
 #pragma unroll
-      for (int i = 0; i < TILES; ++i) own[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < kTiles; ++i) own[i] = f32x4{0.f, 0.f, 0.f, 0.f};
       // the chunk's tokens by themselves, oldest first, then the decayed state: one rounding of the state a chunk
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int i = 0; i < TILES; ++i) own[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[i][r], un[r], own[i], 0, 0, 0);
+        for (int i = 0; i < kTiles; ++i) own[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[i][r], un[r], own[i], 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < TILES; ++i) {
+      for (int i = 0; i < kTiles; ++i) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) own[i][r] = fmaf(now.d[i][r], s[i][r], own[i][r]);
       }
@@ -347,7 +343,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       fetch(ci + kAhead, ahead[u]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < TILES; ++i) {
+      for (int i = 0; i < kTiles; ++i) {
         const uint32_t moves = have[i] && ci < chunks ? ~0u : 0u;      // (bits, not a condition: no branch)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -359,29 +355,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   __syncthreads();
   if (chunks % kAhead == 0) put(chunks - 1, sum_of((chunks - 1) & 1));      // (else a turn past the last chunk has put them)
 #pragma unroll
-  for (int i = 0; i < TILES; ++i)
+  for (int i = 0; i < kTiles; ++i)
     if (have[i]) *reinterpret_cast<f32x4*>(S + channel[i] + 4 * g) = s[i];
 }
 
 }  // namespace
 
-// in, state, y as in tk_delta_scan (delta.hip); dim and vdim multiples of 16 up to 128, in and state on 16-byte borders.  least:
+// in, state, y as in tk_delta_scan (delta.hip); dim (80 to 128) and vdim (up to 128) multiples of 16, in and state on 16-byte borders.  least:
 // requests of fewer tokens are left alone; chunks: at least the chunks of 16 tokens that the others have together; operands
 // (float32 [chunks, heads, 49 dim + 16 vdim + 256], on a 16-byte border) is scratch.
 TK_API int tk_delta_chunks(const float* in, float* state, const int* q_start, const int* state_slots, float* y, float* operands,
                            int R, int least, int chunks, int heads, int kv, int dim, int vdim, hipStream_t stream) {
   if (R <= 0) return 0;
-  if (heads < 1 || heads > 65535 || kv < 1 || heads % kv || dim < 16 || dim > kMaxDim || dim % 16 || vdim < 16 || vdim > kMaxDim ||
+  if (heads < 1 || heads > 65535 || kv < 1 || heads % kv || dim <= kWave || dim > kMaxDim || dim % 16 || vdim < 16 || vdim > kMaxDim ||
       vdim % 16 || least < 1 || chunks < 1 || R > 65535 || operands == nullptr || (uintptr_t)in % 16 || (uintptr_t)state % 16 ||
       (uintptr_t)operands % 16)
     return -1;
   const Shape sh{R, heads, kv, dim, vdim, least};
-  delta_operands_kernel<<<dim3(chunks, heads), (max(dim, vdim) + kWave - 1) / kWave * kWave, 0, stream>>>(in, q_start, operands, sh);
+  delta_operands_kernel<<<dim3(chunks, heads), 2 * kWave, 0, stream>>>(in, q_start, operands, sh);
   // (heads the fastest index: the value columns' blocks of a head, which read the same operands, then share an XCD's L2
   // where the heads are a multiple of eight)
   const dim3 walks(heads, vdim / 16, R);
-  if (dim <= 64) delta_walk_kernel<1><<<walks, 256, 0, stream>>>(operands, state, q_start, state_slots, y, sh);
-  else delta_walk_kernel<2><<<walks, 256, 0, stream>>>(operands, state, q_start, state_slots, y, sh);
+  delta_walk_kernel<<<walks, 256, 0, stream>>>(operands, state, q_start, state_slots, y, sh);
   return launch_status();
 }
 

@@ -1414,7 +1414,7 @@ def _scan_chunks(batch, n: int, heads: int, state_size: int, vdim: int, device):
 
 
 DELTA_MAX_DIM = 512          # key channels of a head of the delta-rule scan (csrc/delta.hip)
-DELTA_CHUNKS_FROM_TOKENS = 160   # a request's tokens in a step from which it is scanned in chunks
+DELTA_CHUNKS_FROM_TOKENS = 320   # a request's tokens in a step from which it is scanned in chunks
 
 
 def delta_row(heads: int, kv_heads: int, dim: int, vdim: int) -> int:
@@ -1466,12 +1466,18 @@ def delta_inputs(proj: torch.Tensor, up: torch.Tensor, conv: torch.Tensor, conv_
 
 
 def _delta_in_chunks(dim: int, vdim: int, longest: int) -> bool:
-    """Whether the delta rule's scan has requests that run in chunks of 16 tokens on the matrix cores: 160 tokens and more of
-    heads that are whole tiles.  The line looks at a request's own tokens alone, so that its bits do not depend on its
-    neighbours.  Walked and in chunks, us, heads of 128 x 128: 32 heads, one request of 64 tokens 15 and 21, of 128 25 and 26, of
-    256 48 and 40, of 2,048 357 and 200, sixteen of 128 223 and 227; 8 heads, one of 128 24 and 23, of 256 44 and 32, sixteen of 128
-    60 and 62."""
-    return longest >= DELTA_CHUNKS_FROM_TOKENS and dim % 16 == 0 and vdim % 16 == 0 and max(dim, vdim) <= SCAN_CHUNKS_MAX_DIM
+    """Whether the delta rule's scan has requests that run in chunks of 16 tokens on the matrix cores: 320 tokens and more of heads
+    of 80 to 128 key channels and 112 or 128 values, whole tiles.  The line looks at a request's own tokens alone, so that its bits
+    do not depend on its neighbours: it lies where chunks are ahead beside any of them.  2 to 64 heads, 1 to 64 requests, 5,000 scans
+    (walk over chunks):
+
+    - 320 tokens 1.02 to 1.54 times as fast, 2,048 1.25 to 2.43 (128 x 128, 32 heads: one request of 320 tokens 63 -> 49 us, of 2,048
+      357 -> 207); 256 0.98 to 1.43, 160 0.82 to 1.31, many requests behind;
+    - fewer values share a chunk's operands among fewer blocks, and many requests fill the GPU by the walk alone: at 320 tokens and more
+      96 x 96 0.98, 128 x 64 0.85, 64 x 64 and 32 x 32 0.69, 128 x 16 0.36, though one request alone is ahead there, too;
+    - up to 64 key channels the walk holds a state in half the registers: 64 x 112 0.88, 48 x 112 0.96, 32 x 112 0.98."""
+    return (longest >= DELTA_CHUNKS_FROM_TOKENS and dim % 16 == vdim % 16 == 0 and 64 < dim <= SCAN_CHUNKS_MAX_DIM
+            and 112 <= vdim <= SCAN_CHUNKS_MAX_DIM)
 
 
 def delta_scan(operands: torch.Tensor, state: torch.Tensor, y: torch.Tensor, batch, *, heads: int, kv_heads: int, dim: int,
