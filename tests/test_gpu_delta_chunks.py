@@ -73,3 +73,43 @@ def test_chunks(heads, kv, dim, vdim, spans, decays, monkeypatch):
     near((got, walked), want)
     for slot, s in want_state.items():
         near((got_state[slot], walked_state[slot]), s)
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v", "a", "beta", "state"])
+@pytest.mark.parametrize("number", [float("inf"), float("-inf"), float("nan")])
+def test_numbers_that_are_not_finite_look_ahead_alone(where, number, monkeypatch):
+    """A token's number that is not finite shows from that token on, and, as the walk has it, only in what depends on it."""
+    from tokamak_amd.kernels import ops
+
+    monkeypatch.setattr(ops, "DELTA_CHUNKS_FROM_TOKENS", 16)
+    heads, kv, dim, vdim, spans, bad = 4, 2, 96, 128, [100, 45], 100 + 23
+    g = torch.Generator().manual_seed(5)
+    n = sum(spans)
+    rand = lambda *shape: torch.randn(*shape, generator=g)
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)
+    parts = {"q": unit(rand(n, kv, dim)) * dim ** -0.5, "k": unit(rand(n, kv, dim)), "v": rand(n, heads, vdim),
+             "a": torch.exp(-torch.exp(rand(n, heads, dim) - 2.0)), "beta": torch.sigmoid(rand(n, heads))}
+    state = rand(len(spans) + 1, heads, vdim, dim)
+    if where == "state":
+        state[1, 1, 9, 17] = number
+    elif where == "beta":
+        parts[where][bad, 1] = number
+    else:
+        parts[where][bad, 1, 17] = number
+    row = torch.zeros((n, ops.delta_row(heads, kv, dim, vdim)))
+    flat = torch.cat([parts[x].flatten(1) for x in ("q", "k", "v", "a", "beta")], 1)
+    row[:, :flat.shape[1]] = flat
+    batch = make_batch([(t, 50, [0] * 64) for t in spans])
+    batch.state_slots.copy_(torch.tensor([0, 1], dtype=torch.int32))
+
+    def run(chunks):
+        s, y = state.to(DEV), torch.empty((n, heads * vdim), device=DEV)
+        ops.delta_scan(row.to(DEV), s, y, batch, heads=heads, kv_heads=kv, dim=dim, vdim=vdim, chunks=chunks)
+        return y.cpu(), s.cpu()
+
+    for got, walked in zip(run(True), run(False)):
+        assert torch.equal(got.isfinite(), walked.isfinite()) and not bool(got.isfinite().all()) or where == "q"
+        if where == "q":      # (its own token's outputs of the two heads that share it, and nothing else)
+            assert got.dim() > 2 or got.isfinite().logical_not().nonzero()[:, 0].unique().tolist() == [bad]
+        there = walked.isfinite() & got.isfinite()
+        assert bool(((got - walked)[there].abs() <= 2.0 ** -18 * walked[there].abs().max()).all())

@@ -14,6 +14,9 @@
 //   delta_walk: a block a (head, 16 value columns, request), the chunks in order, the state in the waves' accumulators (a
 //     wave a quarter of the key channels).
 //
+// Where the state ends up with numbers that are not finite, the walk repeats the request a token at a time: products of whole tiles
+// carry a token's infinity to tokens before it, which no decay may undo.
+//
 // Requests of `least` tokens and more; shorter ones are the walk's (delta.hip), whoever stands beside them.  Everything is float32.
 //
 // Walked, a token is a chain of some 430 clocks whatever else the GPU does.  2,048 tokens of 128 x 128: 32 heads 357 us ->
@@ -218,7 +221,7 @@ struct WalkIn {        // a chunk's operands as a lane of the walk holds them
 // channel 16 tile + 4 (lane >> 4) + r of column lane & 15.  One barrier a chunk: the waves' shares of W S meet behind it, their
 // shares of the outputs behind the next chunk's.  Operands are asked for kAhead chunks ahead, without a branch around any load.
 constexpr int kAhead = 4;
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void delta_walk_kernel(const float* __restrict__ operands,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void delta_walk_kernel(const float* __restrict__ in, const float* __restrict__ operands,
                                                          float* __restrict__ state, const int* __restrict__ q_start,
                                                          const int* __restrict__ state_slots, float* __restrict__ y, Shape sh) {
   __shared__ __align__(16) float seen[2][4][256];     // shares of W S
@@ -354,6 +357,55 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   } while (c0 < chunks);
   __syncthreads();
   if (chunks % kAhead == 0) put(chunks - 1, sum_of((chunks - 1) & 1));      // (else a turn past the last chunk has put them)
+  // A number that is not finite has met the zeros of T, A and the rows past the end above, and made tokens before its own NaN.  It
+  // stays in the state: the request again, then, a token at a time, from the state as it was.
+  bool lost = false;
+#pragma unroll
+  for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) lost |= !(fabsf(s[i][r]) < INFINITY);
+  if (__syncthreads_or(lost)) {
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i)
+      if (have[i]) s[i] = *reinterpret_cast<const f32x4*>(S + channel[i] + 4 * g);
+    const int kvh = head / (sh.heads / sh.kv);
+    const float* row = in + (size_t)first * sh.row();
+    for (int t = 0; t < tokens; ++t, row += sh.row()) {
+      const float v = row[sh.v_at() + head * sh.vdim + v0 + x], beta = row[sh.b_at() + head];
+      f32x4 k[kTiles], q[kTiles];
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < kTiles; ++i) {
+        if (!have[i]) continue;
+        q[i] = *reinterpret_cast<const f32x4*>(row + kvh * sh.dim + channel[i] + 4 * g);
+        k[i] = *reinterpret_cast<const f32x4*>(row + (sh.kv + kvh) * sh.dim + channel[i] + 4 * g);
+        s[i] *= *reinterpret_cast<const f32x4*>(row + sh.g_at() + head * sh.dim + channel[i] + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum = fmaf(k[i][r], s[i][r], sum);
+      }
+      sum = sum32(sum16(sum));
+      if (g == 0) seen[t & 1][wave][x] = sum;
+      __syncthreads();      // (either copy is written again behind the next token's barriers)
+      const float* const before_u = &seen[t & 1][0][x];
+      const float u = beta * (v - (((before_u[0] + before_u[256]) + before_u[512]) + before_u[768]));
+      sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < kTiles; ++i) {
+        if (!have[i]) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[i][r] = fmaf(k[i][r], u, s[i][r]);
+          sum = fmaf(q[i][r], s[i][r], sum);
+        }
+      }
+      sum = sum32(sum16(sum));
+      if (g == 0) outs[t & 1][wave][x] = sum;
+      __syncthreads();
+      // (by the thread that has put this token's output above)
+      const float* const all = &outs[t & 1][0][x];
+      if ((t & (kTokens - 1)) == mine_at) y_first[(size_t)t * VW + v0 + x] = ((all[0] + all[256]) + all[512]) + all[768];
+    }
+  }
 #pragma unroll
   for (int i = 0; i < kTiles; ++i)
     if (have[i]) *reinterpret_cast<f32x4*>(S + channel[i] + 4 * g) = s[i];
@@ -376,7 +428,7 @@ TK_API int tk_delta_chunks(const float* in, float* state, const int* q_start, co
   // (heads the fastest index: the value columns' blocks of a head, which read the same operands, then share an XCD's L2
   // where the heads are a multiple of eight)
   const dim3 walks(heads, vdim / 16, R);
-  delta_walk_kernel<<<walks, 256, 0, stream>>>(operands, state, q_start, state_slots, y, sh);
+  delta_walk_kernel<<<walks, 256, 0, stream>>>(in, operands, state, q_start, state_slots, y, sh);
   return launch_status();
 }
 
