@@ -113,3 +113,29 @@ def test_more_tokens_alone_than_cus(dtype, hd, kw):
         part = dict(s, q=s["q"][at:at + 6], positions=s["positions"][at:at + 6], requests=s["requests"][at:at + 6])
         few[at:at + 6] = attend(part, nh, nkv, hd, hd, ps, False, False, **kw)
     assert torch.equal(many, few) and torch.equal(many, attend(s, nh, nkv, hd, hd, ps, False, True, **kw)) and not bool(many.isnan().any())
+
+
+# (the tiles' product takes all keys of a tile's tokens: a value of a later token must not meet an earlier one's weight of zero)
+@pytest.mark.parametrize("number", [float("inf"), float("nan")])
+@pytest.mark.parametrize("where", ["v", "k"])
+@pytest.mark.parametrize("form", [f for f in FORMS if f[2] == f[3] and f[2] in (64, 128) and f[4] % 16 == 0])
+def test_numbers_that_are_not_finite_show_where_they_are_seen(form, where, number):
+    nh, nkv, hd, vd, ps, kw = form
+    kw = dict(kw, sinks=torch.linspace(-1.0, 1.0, nh, device=DEV)) if "sinks" in kw else kw
+    requests = [(63, 33), (0, 17), (130, 20), (64, 16)]
+    s = step(requests, nh, nkv, hd, vd, ps, torch.float32)
+    # the last token's key of a tile, one amid a tile, one that a window leaves behind within a tile, the first one's
+    for r, key in enumerate([78, 9, 100, 64]):
+        page = int(s["tables"][r, key // ps])
+        if where == "v":
+            s["v"][page, :, 1, key % ps // 4, 5, key % 4] = number
+        else:
+            s["k"][page, :, 1, key % ps, 3] = number
+    tiled, alone = (attend(s, nh, nkv, hd, vd, ps, tiles, False, **kw) for tiles in (True, False))
+    assert torch.equal(tiled.isnan(), alone.isnan()) and torch.equal(tiled.nan_to_num(nan=7.0), alone.nan_to_num(nan=7.0))
+    row = 0
+    for (cached, new), key in zip(requests, [78, 9, 100, 64]):
+        for t in range(new):
+            there = seen(cached + t, cached + new, **{n: v for n, v in kw.items() if n not in ("sinks", "softcap")})
+            assert bool(there[key]) or bool(tiled[row + t].isfinite().all())
+        row += new

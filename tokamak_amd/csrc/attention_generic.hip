@@ -535,7 +535,10 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_float32_tiles_kernel
 #pragma unroll
         for (int e = 0; e < 4; ++e) mine[(h * kWave + 16 * t + 4 * g + e) * kTileTokens + a] = sc[h][t][e];
     wave_lds_sync();
-    const bool whole = (c0 >= lo || c0 + kWave <= keep) && c0 + kWave - 1 <= hi;      // no key of the round is another's or none
+    // Where not every token sees every key of the round: a key that is another's or none counts as zeros, and so do numbers of the
+    // others that are not finite, which would make NaN of a weight of zero; those are added for the tokens that see them.
+    const bool every = c0 + kWave - 1 <= pos0 && (c0 >= first_of(hi) || c0 + kWave <= keep);
+    bool apart = false;
 #pragma unroll
     for (int h = 0; h < H; ++h)
 #pragma unroll
@@ -549,13 +552,17 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_float32_tiles_kernel
         for (int s = 0; s < 4; ++s) pr[h][s] = mine[(h * kWave + 16 * t + 4 * s) * kTileTokens + lane];
       if (t + 1 < KEYS) ask_values(t + 1);
       __builtin_amdgcn_sched_barrier(0);
-      if (!whole) {
+      if (!every) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           const int c = c0 + 16 * t + 4 * s + g;
           const bool in = (c >= lo || c < keep) && c <= hi;
 #pragma unroll
-          for (int i = 0; i < DIMS; ++i) held[t & 1][i][s] = in ? held[t & 1][i][s] : 0.f;
+          for (int i = 0; i < DIMS; ++i) {
+            const bool number = fabsf(held[t & 1][i][s]) < INFINITY;
+            apart |= in && !number;
+            held[t & 1][i][s] = in && number ? held[t & 1][i][s] : 0.f;
+          }
         }
       }
 #pragma unroll
@@ -565,6 +572,23 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_float32_tiles_kernel
 #pragma unroll
           for (int h = 0; h < H; ++h) acc[h][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(held[t & 1][i][s], pr[h][s], acc[h][i], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if (__ballot(apart) != 0) {
+#pragma unroll 1
+      for (int key = 0; key < kWave; ++key) {
+        const int c = c0 + key;
+        if (c > hi || !(c >= lo || c < keep)) continue;
+        const float* const base = v_head + (size_t)scalar(table[c / ps]) * page_elems + (size_t)(c % ps >> 2) * 64 + (c & 3);
+#pragma unroll
+        for (int i = 0; i < DIMS; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float v = base[(size_t)i * (ps >> 2) * 64 + (4 * g + e) * 4];
+            if (!sees(c) || fabsf(v) < INFINITY) continue;
+#pragma unroll
+            for (int h = 0; h < H; ++h) acc[h][i][e] = fmaf(mine[(h * kWave + key) * kTileTokens + a], v, acc[h][i][e]);
+          }
+      }
     }
   }
   // merge in wave order, a head after the other
