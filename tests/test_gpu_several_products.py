@@ -4,7 +4,7 @@ K's steps."""
 import pytest
 import torch
 
-from tokamak_amd.kernels import linear, ops
+from tokamak_amd.kernels import gemm_bf16, linear, ops
 
 DEV = "cuda:0"
 
@@ -13,6 +13,28 @@ def test_the_rule():
     assert ops.several_pay(4, 129, 4096, 4096) and ops.several_pay(4, 2048, 4096, 4096) and ops.several_pay(2, 300, 1024, 1024)
     assert not ops.several_pay(1, 2048, 4096, 4096) and not ops.several_pay(2, 129, 512, 8192)
     assert {ops.several_plan(4, m, n, k) for m, n, k in [(129, 4096, 4096), (512, 4096, 4096), (2048, 4096, 4096)]} >= {(128, 128), (256, 256)}
+
+
+@pytest.mark.parametrize("m, n, k, several", [(129, 4096, 9216, False), (512, 12288, 12288, False), (1000, 4096, 16384, False), (129, 4096, 4096, True),
+                                              (1101, 4096, 9216, True), (512, 2048, 8192, True)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_products_in_shares_of_k_keep_their_sums(m, n, k, several, shared, monkeypatch):
+    """What a product leaves for its reader to add in float32, several do, too."""
+    went = []
+    monkeypatch.setattr(ops, "gemm_several", lambda *a: went.append("several"))
+    monkeypatch.setattr(gemm_bf16, "split_many", lambda x, w: went.append("shares"))
+    x, w = (torch.empty(s, dtype=torch.bfloat16, device="meta") for s in ((m, k) if shared else (4, m, k), (4, n, k)))
+    linear.several_linears(x, w)
+    assert ops.several_pay(4, m, n, k) and went == (["several"] if several else ["shares"] * 4)
+
+
+def test_more_than_a_launch_takes_or_off_its_borders_are_single_products(monkeypatch):
+    went = []
+    monkeypatch.setattr(linear, "linear", lambda x, w, allow_partials: went.append(tuple(x.shape)))
+    made = lambda *s: torch.empty(s, dtype=torch.bfloat16, device="meta")      # noqa: E731
+    linear.several_linears(made(200, 256), made(65, 256, 256))
+    linear.several_linears(made(200, 256), made(3, 256 * 256 + 4)[:, :256 * 256].unflatten(1, (256, 256)))
+    assert went == [(200, 256)] * 68
 
 
 # integers, whose products and sums are exact in bfloat16's and float32's terms: every bit is known

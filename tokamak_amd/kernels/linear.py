@@ -141,11 +141,15 @@ def linear(x: torch.Tensor | DeferredNorm, weight: torch.Tensor, out_dtype: torc
 
 def several_linears(x: torch.Tensor, weights: torch.Tensor) -> list[torch.Tensor]:
     """``linear(x_i, weights[i], allow_partials=True)`` for every i: ``weights`` [C, N, K], ``x`` [C, M, K], or [M, K] for all of them.  More than
-    128 rows: one launch where that pays (``ops.several_pay``)."""
+    128 rows into bfloat16: one launch where that pays (``ops.several_pay``).  Long products whose reader adds float32 sums of shares of K
+    (``gemm_bf16.splits_many``) stay such products: one launch would round each to bfloat16."""
+    from tokamak_amd.kernels import gemm_bf16
+
     count, n, k = weights.shape
     m = x.shape[-2]
-    if (m > ops.STREAM_MAX_ROWS and x.dtype == torch.bfloat16 and ops.gemm_many_fits(x if x.dim() == 2 else x[0], weights[0], n)
-            and ops.several_pay(count, m, n, k)):
+    first = x if x.dim() == 2 else x[0]
+    if (m > ops.STREAM_MAX_ROWS and x.dtype == torch.bfloat16 and ops.gemm_several_fits(x, weights)
+            and ops.several_pay(count, m, n, k) and not gemm_bf16.splits_many(first, weights[0])):
         out = torch.empty((count, m, n), dtype=x.dtype, device=x.device)
         ops.gemm_several(x, weights, out)
         return list(out)

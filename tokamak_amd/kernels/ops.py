@@ -2338,6 +2338,16 @@ def several_pay(count: int, m: int, n: int, k: int) -> bool:
     return count > 1 and (k <= 2048 or -(-m // rows) * -(-n // columns) * count >= 0.4 * MANY_PRICES[rows, columns][0])
 
 
+GEMM_SEVERAL_MOST = 64      # products of one launch (csrc/gemm_many.hip)
+
+
+def gemm_several_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gemm_several`` takes these operands, a [C, M, K] or [M, K], w [C, N, K]: up to 64 products of ``gemm_many``'s operands,
+    one behind the other on 16-byte borders."""
+    return (w.shape[0] <= GEMM_SEVERAL_MOST and all(t.dim() == 2 or t.stride(0) % 8 == 0 for t in (a, w))
+            and gemm_many_fits(a if a.dim() == 2 else a[0], w[0], w.shape[1]))
+
+
 def gemm_several(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
     """out[i] = a[i] @ w[i]^T in bfloat16, i below the number of matrices: w [C, N, K], out [C, M, N], a [C, M, K], or [M, K] for all."""
     for t in (a, w, out):
@@ -2346,8 +2356,8 @@ def gemm_several(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
     m = a.shape[-2]
     _need(a.shape[-1] == k and out.shape == (count, m, n) and (a.dim() == 2 or a.shape[0] == count), "gemm shapes disagree")
     first = a if a.dim() == 2 else a[0]
-    _need(gemm_many_fits(first, w[0], n) and out.data_ptr() % 16 == 0 and out.stride(1) % 8 == 0 and count <= 64
-          and all(t.dim() == 2 or t.stride(0) % 8 == 0 for t in (a, w, out)), "products of many rows take whole steps of 64 k and rows on 16-byte borders")
+    _need(gemm_several_fits(a, w) and out.data_ptr() % 16 == 0 and out.stride(0) % 8 == 0 and out.stride(1) % 8 == 0,
+          "products of many rows take whole steps of 64 k and rows on 16-byte borders, up to 64 of them")
     _note(f"{count}x{m}x{n}x{k}", count * (n * k + m * k + m * n) * 2, 2.0 * count * m * n * k)
     _check(_fn("gemm_many", "tk_gemm_several")(
         _p(a), _p(w), _p(out), m, n, k, first.stride(0), w.stride(1), out.stride(1), count, 0 if a.dim() == 2 else a.stride(0), w.stride(0),
