@@ -12,6 +12,9 @@ DEV = "cuda:0"
 def test_the_rule():
     assert ops.several_pay(4, 129, 4096, 4096) and ops.several_pay(4, 2048, 4096, 4096) and ops.several_pay(2, 300, 1024, 1024)
     assert not ops.several_pay(1, 2048, 4096, 4096) and not ops.several_pay(2, 129, 512, 8192)
+    # a round and a bit of tiles of 256 x 256: four products, or two whose K is short, but not two or three that fill most of one each
+    assert ops.several_pay(4, 2048, 2304, 6144) and ops.several_pay(2, 700, 12288, 1024) and ops.several_pay(2, 2048, 8192, 6144)
+    assert not ops.several_pay(2, 700, 12288, 6144) and not ops.several_pay(3, 1500, 4096, 5120) and not ops.several_pay(4, 4096, 12288, 256)
     assert {ops.several_plan(4, m, n, k) for m, n, k in [(129, 4096, 4096), (512, 4096, 4096), (2048, 4096, 4096)]} >= {(128, 128), (256, 256)}
 
 

@@ -2330,12 +2330,20 @@ def several_plan(count: int, m: int, n: int, k: int) -> tuple[int, int]:
 
 
 def several_pay(count: int, m: int, n: int, k: int) -> bool:
-    """Whether ``count`` products of more than 128 rows go out as one launch of ``gemm_several`` rather than each to the library: by the
-    share of the blocks that run at once which their tiles fill, or K short enough.  Beside as many launches of the library, weights from memory:
-    four of 4,096 x 4,096 at 129 / 512 / 1,000 / 2,048 rows 91 / 123 / 164 / 241 us, here 44 / 59 / 96 / 184; three of 2,048 x 2,048 at 2,048
-    rows 69 and 49; one alone 0.6 to 1.06 times as fast.  (A product's 64 to 256 tiles are a fraction of a round; several fill whole ones.)"""
+    """Whether ``count`` products of more than 128 rows go out as one launch of ``gemm_several`` rather than each to the library.  A
+    product's 64 to 256 tiles are a fraction of a round; several fill whole ones.  Beside as many launches of the library, weights from
+    memory, two to four products of 129 to 4,096 rows, 256 to 12,288 weight rows of 256 to 10,240, by the tiles of 256 x 256 that all have:
+
+    - up to 256, a round, if K is short or the tiles fill two fifths of the blocks that run at once: 1.65 times as fast on average, 3 of
+      1,028 more than 5 % behind (four of 4,096 x 4,096 at 129 / 512 / 1,000 rows 91 / 123 / 164 us, here 44 / 59 / 96);
+    - more, four products: 1.25, 0.94 to 2.1 (that one at 2,048 rows 241 and 184); from 2,048 tiles on 0.98, with K of 256 0.87;
+    - more, two or three: 1.10, 0.88 to 2.0, with a last round four fifths full; with less of it and K above 1,024 0.99, 70 of 136 behind,
+      since a product's tiles fill most of a round by themselves (two of 12,288 x 6,144 at 700 rows 205 us, here 245), else 1.41."""
     rows, columns = several_plan(count, m, n, k)
-    return count > 1 and (k <= 2048 or -(-m // rows) * -(-n // columns) * count >= 0.4 * MANY_PRICES[rows, columns][0])
+    if count < 2 or (k > 2048 and -(-m // rows) * -(-n // columns) * count < 0.4 * MANY_PRICES[rows, columns][0]):
+        return False
+    tiles = -(-m // 256) * -(-n // 256) * count
+    return tiles <= 256 or (tiles < 2048 and (count > 3 or k <= 1024 or tiles >= 0.8 * 256 * -(-tiles // 256)))
 
 
 GEMM_SEVERAL_MOST = 64      # products of one launch (csrc/gemm_many.hip)
