@@ -1,6 +1,7 @@
 """Loader errors and the random-weights folder writer."""
 
 import json
+import weakref
 
 import pytest
 import torch
@@ -9,6 +10,7 @@ from safetensors.torch import load_file, save_file
 
 from tiny import TINIES, make_folder
 from tokamak_amd.config import load_model_description
+from tokamak_amd.config.registry import get_part
 from tokamak_amd.engine.model import LayeredModel
 from tokamak_amd.weights import SafetensorsSource, WeightError, load_weights, write_random_model
 
@@ -134,3 +136,28 @@ def test_a_tensor_is_held_as_its_spec_says_whatever_its_role():
         TensorSpec((4,), held="float64")
     with pytest.raises(ValueError, match="role"):
         TensorSpec((4,), role="scalar")
+
+
+@pytest.mark.parametrize("name, sizes, together", [
+    ("decayed_state_time_mix", {"head_dim": 16, "decay_rank": 4}, "rkvg"),
+    ("gated_linear_attention", {"head_dim": 16, "value_dim": 16, "tau": 16.0, "decay_rank": 4}, "qkvg"),
+    ("gated_linear_attention", {"head_dim": 16, "value_dim": 32, "tau": 16.0, "decay_rank": 4}, "qkvg")])
+def test_matrices_that_lie_together_are_in_memory_twice_one_at_a_time(name, sizes, together):
+    part = get_part("mixer", name)(hidden_size=32, num_heads=2, norm_eps=1e-5, dtype=torch.float32, device="cpu", **sizes)
+    specs = part.expected_tensors("p.")
+    held, given = [], {}
+
+    def fetch(tensor):
+        assert not [n for n, ref in held if ref() is not None]
+        shape = tuple(4 if s is None else s for s in specs[tensor].shape)
+        made = torch.randn(shape, generator=torch.Generator().manual_seed(len(tensor) + sum(map(ord, tensor))))
+        given[tensor] = made.clone()
+        if tensor[2:] in together:
+            held.append((tensor, weakref.ref(made)))
+        return made
+
+    part.bind("p.", fetch)
+    groups = [n for n in ("rkvg", "qkvg", "qk", "vg") if getattr(part, n, None) is not None]
+    assert "".join(groups) == together
+    for names in groups:
+        assert torch.equal(getattr(part, names), torch.stack([given["p." + n] for n in names]))

@@ -41,6 +41,18 @@ from tokamak_amd.weights.spec import TensorSpec
 Fetch = Callable[[str], "torch.Tensor | None"]
 
 
+def fetch_together(fetch: Fetch, names: list[str]) -> torch.Tensor:
+    """Tensors of one shape in one, [names, ...].  Each is copied as it comes and let go, so that only one at a time lies in memory twice."""
+    out = None
+    for i, name in enumerate(names):
+        tensor = fetch(name)
+        if out is None:
+            out = torch.empty((len(names), *tensor.shape), dtype=tensor.dtype, device=tensor.device)
+        out[i] = tensor
+        del tensor
+    return out
+
+
 class Part:
     """Common base: parameters, expected tensors, binding.
 

@@ -7,7 +7,7 @@ import torch
 from tokamak_amd.config.registry import register_part
 from tokamak_amd.kernels import ops
 from tokamak_amd.kernels.linear import linear, several_linears
-from tokamak_amd.parts.base import Fetch, Mixer, PositionData, StateArray
+from tokamak_amd.parts.base import Fetch, Mixer, PositionData, StateArray, fetch_together
 from tokamak_amd.weights.spec import TensorSpec
 
 
@@ -62,7 +62,7 @@ class GatedLinearAttention(Mixer):
     def bind(self, prefix: str, fetch: Fetch) -> None:
         groups = ("qkvg",) if self.head_dim == self.value_dim else ("qk", "vg")
         for names in groups:
-            setattr(self, names, torch.stack([fetch(prefix + n) for n in names]))
+            setattr(self, names, fetch_together(fetch, [prefix + n for n in names]))
         for n in ("o", "a1", "a2"):
             setattr(self, n, fetch(prefix + n))
         if self.a2.shape[1] != self.a1.shape[0]:

@@ -7,7 +7,7 @@ import torch
 from tokamak_amd.config.registry import register_part
 from tokamak_amd.kernels import ops
 from tokamak_amd.kernels.linear import linear, several_linears
-from tokamak_amd.parts.base import Fetch, Mixer, PositionData, StateArray
+from tokamak_amd.parts.base import Fetch, Mixer, PositionData, StateArray, fetch_together
 from tokamak_amd.weights.spec import TensorSpec
 
 MIXES = ("r", "k", "v", "g", "w")
@@ -63,7 +63,7 @@ class DecayedStateTimeMix(Mixer):
 
     def bind(self, prefix: str, fetch: Fetch) -> None:
         self.mu = torch.stack([fetch(prefix + "mu." + s) for s in MIXES]).contiguous()
-        self.rkvg = torch.stack([fetch(prefix + n) for n in MIXES[:4]])
+        self.rkvg = fetch_together(fetch, [prefix + n for n in MIXES[:4]])
         for n in ("w1", "w2", "o", "w0"):
             setattr(self, n, fetch(prefix + n))
         if self.w2.shape[1] != self.w1.shape[0]:
