@@ -45,3 +45,46 @@ def test_what_is_refused():
         ops.sample(logits, params[:14], out, None, 1)                        # no room for the row's number
     with pytest.raises(ops.KernelError):
         ops.sample(logits.repeat(33, 1), np.zeros(66 * 7, dtype=np.int32), torch.zeros(66, dtype=torch.int32, device=DEV))
+
+
+@pytest.mark.parametrize("rows", [65, 77])
+def test_more_rows_than_travel_with_the_launch_are_shared(rows):
+    """At 151,936 logits up to 77 rows with thresholds are shared between blocks: with their parameters in device memory as with the launch,
+    and as a block a row chooses."""
+    vocab = 151936
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    logits = torch.randn(rows, vocab, generator=gen, device=DEV) * 3.0
+    logits[3] = logits[3].round()                                            # (many values in the threshold's bin)
+    params, seeds, draws = [KINDS[i % len(KINDS)] for i in range(rows)], [977 * i for i in range(rows)], list(range(rows))
+    whole = sample_tokens(logits, params, seeds, draws)
+    for at in (0, rows - 64):
+        part = slice(at, at + 64)
+        assert torch.equal(sample_tokens(logits[part], params[part], seeds[part], draws[part]), whole[part])
+    more = 78 - rows
+    alone = sample_tokens(torch.cat([logits, logits[:more]]), params + params[:more], seeds + seeds[:more], draws + draws[:more])
+    assert torch.equal(alone[:rows], whole)
+
+
+@pytest.mark.parametrize("rows", [7, 66])
+def test_rows_left_out_of_the_list_are_sampled_alone(rows):
+    """The list of rows with thresholds is the caller's: what it leaves out, has out of order or out of range is not read unmade."""
+    vocab = 151936
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    logits = torch.randn(rows, vocab, generator=gen, device=DEV) * 3.0
+    host = np.zeros(8 * rows, dtype=np.int32)
+    host[:4 * rows].view(np.int64)[:] = np.arange(2 * rows) * 31
+    host[4 * rows:6 * rows].view(np.float32)[:] = [0.8] * rows + [0.9, 1.0] * (rows // 2) + [0.95] * (rows % 2)
+    host[6 * rows:7 * rows] = [0, 40] * (rows // 2) + [300] * (rows % 2)
+
+    def chosen(listed):
+        given = host[:7 * rows + len(listed)].copy()
+        given[7 * rows:] = listed
+        out = torch.full((rows,), -1, dtype=torch.int32, device=DEV)
+        ops.sample(logits, given if rows <= 64 else torch.from_numpy(given).to(DEV), out, None, len(listed))
+        return out
+
+    whole = chosen(list(range(rows)))
+    for listed in ([], [0], [rows - 1], list(range(1, rows, 2)), list(range(rows - 1, -1, -1))):
+        assert torch.equal(chosen(listed), whole)
+    if rows > 64:      # (with the launch these are refused)
+        assert torch.equal(chosen([2, 2, 5, 5, rows, 1 << 30]), whole) and torch.equal(chosen([-1, -7, 3]), whole)

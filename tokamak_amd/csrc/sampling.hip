@@ -41,8 +41,16 @@ constexpr int kShareThreads = 256;
 constexpr int kFew = 256;          // values among which a threshold is found by ranks
 constexpr int kLevelBins = 1024;   // of the second and the third level (ten bits each)
 
+struct FirstLevel {
+  int bin;                          // the first histogram's bin that holds the threshold
+  uint32_t k_remaining;             // of top-k: how many of that bin's values still count
+  unsigned long long p_remaining;   // of top-p alone: how much of that bin's mass
+  uint32_t total;                   // values in that bin and above it (of a row whose first pass is still to be made: 0)
+  uint32_t inside;                  // values in that bin
+};
+
 // Scratch of the rows with thresholds, null: every row is sampled by one block alone.  The argmax pass zeroes what the
-// kernels add into (hist32, hist64, count).
+// kernels add into (hist32, hist64, count), and says of every row that has a threshold that its first pass is still to be made (level).
 struct SharedRows {
   uint32_t* hist32;              // [M][kBins + kCoarse]: the bins, then the sums of every 64 of them
   unsigned long long* hist64;    // [M][kBins + kCoarse]
@@ -50,7 +58,7 @@ struct SharedRows {
   uint32_t* cand;                // [M][kCandidates] ordered images
   uint8_t* segment;              // [M][kCandidates]
   unsigned long long* above;     // [M][segments] mass of what is kept for certain and not listed
-  struct FirstLevel* level;      // [M] where the first threshold lies
+  FirstLevel* level;             // [M] where the first threshold lies
 };
 
 // A step's sampling parameters in device memory.
@@ -58,7 +66,7 @@ struct RowParams {
   const unsigned long long *seeds, *draws;     // [M] the request's seed and how many draws it has made
   const float *temperature, *top_p;            // [M]
   const int* top_k;                            // [M]
-  const int* rows;                             // [shared] the rows that have a threshold
+  const int* rows;                             // [shared] the rows that have a threshold, ascending (those left out are a block's alone)
 };
 
 // The same of up to kInlineRows rows as an argument of the first launch, which leaves them in device memory for the others: a copy
@@ -146,7 +154,10 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_segments_kernel(
       clear.hist32[(size_t)blockIdx.y * kHistWords + i] = 0u;
       clear.hist64[(size_t)blockIdx.y * kHistWords + i] = 0ull;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) clear.count[blockIdx.y] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      clear.count[blockIdx.y] = 0u;
+      clear.level[blockIdx.y].total = 0u;
+    }
   }
   if (vec) {
     use_quads<kArgmaxThreads>(row4, quads, held, [&](int at, const float4& v) {
@@ -464,14 +475,6 @@ struct Segment {
   }
 };
 
-struct FirstLevel {
-  int bin;                          // the first histogram's bin that holds the threshold
-  uint32_t k_remaining;             // of top-k: how many of that bin's values still count
-  unsigned long long p_remaining;   // of top-p alone: how much of that bin's mass
-  uint32_t total;                   // values in that bin and above it
-  uint32_t inside;                  // values in that bin
-};
-
 // Where the first threshold of a row lies, from its first histograms (in LDS, or in memory on a 16-byte border: a thread's bins
 // lie side by side and are asked for together).  THREADS threads call; `scan` an entry a wave, `found` one.
 template <int THREADS>
@@ -574,12 +577,20 @@ __device__ __forceinline__ FirstLevel first_level_by_wave(const uint32_t* __rest
   return {group * kWave + bin, (uint32_t)left, left, seen, __shfl(c, kWave - 1 - bin, kWave)};
 }
 
+// The row of a block of the two kernels below, -1 if there is none: the list is the caller's, and a row named twice in a run would be added
+// up twice.
+__device__ __forceinline__ int shared_row(const int* __restrict__ rows, int M) {
+  const int r = rows[blockIdx.y], before = blockIdx.y > 0 ? rows[blockIdx.y - 1] : -1;
+  return r > before && r < M ? r : -1;
+}
+
 __global__ __launch_bounds__(kShareThreads) void sample_hist_kernel(
-    const float* __restrict__ logits, long ld, int V, RowParams params, const float* __restrict__ seg_max, float* __restrict__ row_max,
+    const float* __restrict__ logits, long ld, int M, int V, RowParams params, const float* __restrict__ seg_max, float* __restrict__ row_max,
     SharedRows sh) {
   __shared__ uint32_t h32[kBins];
   __shared__ unsigned long long h64[kBins];
-  const int seg = blockIdx.x, r = params.rows[blockIdx.y], lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int seg = blockIdx.x, r = shared_row(params.rows, M), lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  if (r < 0) return;
   bool k_on, p_on;
   const float temperature = params.temperature[r];
   if (!has_threshold(temperature, params.top_k[r], params.top_p[r], V, k_on, p_on)) return;
@@ -620,11 +631,12 @@ __global__ __launch_bounds__(kShareThreads) void sample_hist_kernel(
 }
 
 __global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
-    const float* __restrict__ logits, long ld, int V, RowParams params, const float* __restrict__ row_max, SharedRows sh) {
+    const float* __restrict__ logits, long ld, int M, int V, RowParams params, const float* __restrict__ row_max, SharedRows sh) {
   __shared__ uint32_t kept[kBins];
   __shared__ unsigned long long scan[kShareThreads / kWave];
   __shared__ uint32_t count, first;
-  const int seg = blockIdx.x, r = params.rows[blockIdx.y];
+  const int seg = blockIdx.x, r = shared_row(params.rows, M);
+  if (r < 0) return;
   bool k_on, p_on;
   const float temperature = params.temperature[r], p_keep = params.top_p[r];
   const int k = params.top_k[r];
@@ -654,8 +666,10 @@ __global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
       if (at < (uint32_t)kBins) kept[at] = o;
       else {                                      // (a segment with more: one by one)
         const uint32_t to = atomicAdd(&sh.count[r], 1u);
-        sh.cand[(size_t)r * kCandidates + to] = o;
-        sh.segment[(size_t)r * kCandidates + to] = (uint8_t)seg;
+        if (to < (uint32_t)kCandidates) {
+          sh.cand[(size_t)r * kCandidates + to] = o;
+          sh.segment[(size_t)r * kCandidates + to] = (uint8_t)seg;
+        }
       }
     } else if (bin > low) {
       above += draw_mass(x, mx, scale);
@@ -668,7 +682,7 @@ __global__ __launch_bounds__(kShareThreads) void sample_collect_kernel(
   const uint32_t n = min(count, (uint32_t)kBins);
   if (threadIdx.x == 0) first = n ? atomicAdd(&sh.count[r], n) : 0u;
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < n; i += kShareThreads) {
+  for (uint32_t i = threadIdx.x; i < n && first + i < (uint32_t)kCandidates; i += kShareThreads) {
     sh.cand[(size_t)r * kCandidates + first + i] = kept[i];
     sh.segment[(size_t)r * kCandidates + first + i] = (uint8_t)seg;
   }
@@ -723,6 +737,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   const float drawn = uniform01(params.seeds[r], params.draws[r]);
   const uint32_t first_cand = shared.hist32 != nullptr ? shared.cand[(size_t)r * kCandidates + tid] : 0u;
   const uint8_t first_segment = shared.hist32 != nullptr ? shared.segment[(size_t)r * kCandidates + tid] : (uint8_t)0;
+  FirstLevel made{};
+  if (shared.hist32 != nullptr) made = shared.level[r];
   const float* row = logits + (size_t)r * ld;
   const float inv_t = 1.f / temperature;
   const int k = params.top_k[r];
@@ -743,7 +759,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
   const int chunk = ((V + kArgmaxSegments - 1) / kArgmaxSegments + 3) & ~3;      // a segment of the argmax pass
   int ncand = -1;                      // >= 0: cand[0 .. ncand) hold every value that can be a threshold
   if (k_on || p_on) {
-    const bool ready = shared.hist32 != nullptr;     // (the row's first pass is done)
+    const bool ready = made.total != 0;     // (the row's first pass is done)
     if (tid == 0) cand_count = 0;
     if (!ready) {
       for (int i = tid; i < kBins; i += nt) {
@@ -759,7 +775,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
       });
       __syncthreads();
     }
-    const FirstLevel level = ready ? shared.level[r] : first_level<kSampleThreads>(hist32, hist64, k_on, k, p_keep, scan64, &first);
+    const FirstLevel level = ready ? made : first_level<kSampleThreads>(hist32, hist64, k_on, k, p_keep, scan64, &first);
     const int low_bin = level.bin;
     if (k_on) {
       k_prefix = (uint32_t)low_bin;
@@ -1094,10 +1110,9 @@ TK_API int tk_sample_scratch_bytes(int M, int V) {
 // Every row's next token: greedy rows (temperature 0) their argmax, the others a draw; a row whose search falls through
 // (rounding at an edge) keeps its argmax.  scratch: tk_sample_scratch_bytes(M, V), on a 16-byte border.  params: seeds and draw counts
 // (M 64-bit numbers each), temperatures and top-p (M floats each), top-k (M integers) and the numbers of the `shared` rows that
-// have a threshold (integers; those kernels are left out where there are none), one behind the other, on an 8-byte border; in device memory, or (on_host,
-// up to tk_sample_inline_rows() rows) in host memory that is free again when the call returns.
-TK_API int tk_sample_inline_rows() { return kInlineRows; }
-
+// have a threshold (integers, each once, ascending; the kernels that share such rows are left out where there are none, and a row that is not
+// named is sampled by a block alone), one behind the other, on an 8-byte border; in device memory, or (on_host, up to kInlineRows rows)
+// in host memory that is free again when the call returns.
 TK_API int tk_sample(const float* logits, long ld, int M, int V, const void* params, int on_host, int shared, int* out, float* probs_out,
                      void* scratch, hipStream_t stream) {
   if (M <= 0) return 0;
@@ -1145,8 +1160,11 @@ TK_API int tk_sample(const float* logits, long ld, int M, int V, const void* par
     std::memcpy(in.top_p, from.top_p, sizeof(float) * M);
     std::memcpy(in.top_k, from.top_k, sizeof(int) * M);
     std::memcpy(in.rows, from.rows, sizeof(int) * shared);
-    for (int i = 0; i < shared; ++i)
-      if (in.rows[i] < 0 || in.rows[i] >= M) return -1;
+    unsigned long long named = 0;
+    for (int i = 0; i < shared; ++i) {
+      if (in.rows[i] < 0 || in.rows[i] >= M || (share && (named >> in.rows[i] & 1))) return -1;
+      named |= 1ull << in.rows[i];
+    }
     in.to = rows;
     in.shared = shared;
     argmax_segments_kernel<<<all, kArgmaxThreads, 0, stream>>>(logits, seg_max, seg_index, V, ld, in, seg_mass, sh);
@@ -1156,8 +1174,8 @@ TK_API int tk_sample(const float* logits, long ld, int M, int V, const void* par
   }
   if (share) {
     const dim3 shares(kArgmaxSegments, shared);
-    sample_hist_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, V, rows, seg_max, row_max, sh);
-    sample_collect_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, V, rows, row_max, sh);
+    sample_hist_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, M, V, rows, seg_max, row_max, sh);
+    sample_collect_kernel<<<shares, kShareThreads, 0, stream>>>(logits, ld, M, V, rows, row_max, sh);
   }
   sample_kernel<<<M, kSampleThreads, 0, stream>>>(logits, ld, V, rows, seg_max, seg_index, seg_mass, out, probs_out, sh);
   return launch_status();

@@ -2885,9 +2885,9 @@ SAMPLE_INLINE_ROWS = 64     # rows up to which the parameters travel as an argum
 def sample(logits: torch.Tensor, params: torch.Tensor | np.ndarray, out: torch.Tensor, probs_out: torch.Tensor | None = None,
            shared: int = 0) -> None:
     """Temperature / top-k / top-p sampling, one row per request.  ``params`` int32: the rows' seeds and draw counts (64 bits each), temperatures
-    and top-p (float32), top-k, and the numbers of the ``shared`` rows that have a threshold, one behind the other; on the GPU, or,
-    of up to ``SAMPLE_INLINE_ROWS`` rows, a numpy array, which the launch takes along.  Two launches share the rows with a threshold between
-    blocks; without such rows they are left out."""
+    and top-p (float32), top-k, and the numbers of the ``shared`` rows that have a threshold (each once, ascending), one behind the other; on the GPU, or,
+    of up to ``SAMPLE_INLINE_ROWS`` rows, a numpy array, which the launch takes along.  Two launches share the rows so named between
+    blocks; without such rows they are left out, and a row with a threshold that is not named is sampled by a block alone."""
     _need(logits.is_cuda and logits.dim() == 2 and logits.stride(1) == 1 and logits.dtype == torch.float32,
           "logits are float32 [M, V] on the GPU")
     _gpu(out, probs_out)
