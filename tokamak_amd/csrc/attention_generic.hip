@@ -108,7 +108,7 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
     int hd, int vd, int ps, int max_pages, float scale, int span, int keep, const float* __restrict__ sinks, float cap) {
   __shared__ __attribute__((aligned(16))) float q_s[QT][kMaxHd];
   __shared__ __attribute__((aligned(16))) float p_s[kWaves][kWave][QT];
-  __shared__ long base_s[kWaves][kWave];  // where a key's values lie (a quad's, for tokens that run alone), or -1
+  __shared__ long base_s[kWaves][kWave];  // where a key's values lie (a quad's, for heads that share a block), or -1
   __shared__ float m_s[kWaves], l_s[kWaves];
   __shared__ float acc_s[kWaves][kMaxHd];
 
@@ -209,8 +209,8 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
       if (MANY) ask_values(0, 0);
       else if (SLOTS > 1 && kWave < vd) ask_values(1, 1);
     }
-    // Tokens that run alone (decode) are bound by round trips to memory, not by arithmetic: they
-    // ask for eight pieces of a key at once and for the values of four keys in one piece (four
+    // Heads that share a block at a token (decode of many) are bound by round trips to memory, too: they
+    // ask for several pieces of a key at once and for the values of four keys in one piece (four
     // such pieces at once).  Tiles of a prompt portion, eight queries to a key, are bound by
     // their multiply-adds and keep the plain loops.  The order of every sum is the same.
     constexpr bool BATCHED = HEADS;

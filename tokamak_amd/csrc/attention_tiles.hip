@@ -180,7 +180,8 @@ __global__ __launch_bounds__(kHeadsPerBlock * 64) void attention_tiles_kernel(
 // 4,500 clocks a stage of 960 channels of which LDS is busy 1,900 and the matrix cores 1,000.
 // Also for two and three heads a kv head where a ring is 32 KB (16 / 8 heads of 128, 1,024 tokens 88 -> 71 us, 300 behind
 // 2,000 96 -> 65); of larger heads a block of two waves would have the CU's LDS to itself.
-// Operands are read from LDS per instruction, which leaves a wave under 256 registers: two waves a SIMD.
+// Of operands two groups are held in registers, the one that is multiplied and the next (whole stages would be more than the 256
+// registers that two waves a SIMD leave each).
 constexpr int kStages = 4;
 __host__ __device__ constexpr int stage_kb(int channels) { return (2 * channels + 63) / 64; }      // of 16 keys: whole runs of 64 pieces
 

@@ -7,7 +7,8 @@
 // reads and loads stands in the walk: both operands go from memory to LDS without passing through registers (global_load_lds,
 // rows of 128 bytes, three stages of 32 k), and a lane reads each step's number by itself (piece p of a row holds four k, a lane of
 // group g takes word g: 64 banks), into the register that the step's last product has just read.  One barrier a stage, in its
-// middle, ahead of which the second half's operands have been read.  Two or three blocks share a CU and fill each other's gaps.
+// middle, ahead of which the second half's operands have been read.  Two blocks share a CU and fill each other's gaps (of 32 x 32 six; 160
+// x 64, whose rings are 84 KB, has the CU to itself).
 //
 // Tiles come in five sizes, so that the CUs' shares of a product are even (1,053 rows, 2,048 columns: 144 blocks of 128 x 128 or 544 of
 // 64 x 64 for the 512 that ran at once, here 242 of 96 x 96); which, ops.float32_tile prices.  Beside tiles of 64 x 64 and 128 x
@@ -37,7 +38,7 @@ struct Job {
 
 // RT, CT: 16-row tiles of a wave along M and N; the block's four waves are two by two.
 template <int RT, int CT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT * CT > 16 ? 1 : 2))) void gemm_float32_kernel(Job job) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_float32_kernel(Job job) {
   constexpr int BM = 32 * RT, BN = 32 * CT, LOADS = RT + CT;
   constexpr uint32_t W_AT = kRing * BM * 128;      // in LDS: the stages of A's rows, then those of W's
   extern __shared__ __attribute__((aligned(1024))) unsigned char float32_lds[];

@@ -108,9 +108,8 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const TI* __restrict__ 
 // lane and as many for the total).  A lane's operand of a step is one float, A[row lane % 32][k + lane / 32]: a row of
 // a stage lies in LDS as its even k, then its odd k, so that one 16-byte read is four steps' operand.
 // A wave's step is 64 cycles a pair of tiles, so a stage of 16 k of 64 x 64 outputs was over long before the next one's loads
-// had come (47 TFLOP/s): stages hold 64 k there and 32 k of 128 x 128, two of them in LDS (one barrier a stage),
-// loaded without a branch (1,000 rows: weights of 2,048 x 6,144 413 -> 267 us, 2,048 x 2,048 141 -> 92, 12,288 x 2,048 497 -> 439;
-// 130 rows: 321 -> 153, 98 -> 55, 178 -> 143).
+// had come (47 TFLOP/s): stages hold 64 k there and 32 k of 128 x 128, two of them in LDS, one barrier a stage.  (1.1 to 2.1 times as
+// fast so, measured on operands on their borders; what those off them take stands at the loads below.)
 typedef float float16v __attribute__((ext_vector_type(16)));
 
 template <typename TO, int H>

@@ -475,12 +475,11 @@ struct Segment {
   }
 };
 
-// Where the first threshold of a row lies, from its first histograms (in LDS, or in memory on a 16-byte border: a thread's bins
-// lie side by side and are asked for together).  THREADS threads call; `scan` an entry a wave, `found` one.
-template <int THREADS>
+// Where the first threshold of a row lies, from its first histograms in LDS (a thread's bins lie side by side).  A block of
+// kSampleThreads calls; `scan` an entry a wave, `found` one.
 __device__ __forceinline__ FirstLevel first_level(const uint32_t* h32, const unsigned long long* h64, bool k_on, int k, float p_keep,
                                                   unsigned long long* scan, FirstLevel* found) {
-  constexpr int PER = kBins / THREADS;
+  constexpr int PER = kBins / kSampleThreads;
   const int tid = threadIdx.x, low = kBins - PER * (tid + 1);     // this thread's bins [low, low + PER), walked from the top
   uint32_t c[PER], count = 0, upto_c, all_c;
   unsigned long long m[PER], mass = 0;
@@ -506,7 +505,7 @@ __device__ __forceinline__ FirstLevel first_level(const uint32_t* h32, const uns
     const double share = (double)p_keep * (double)whole;
     target = share < 1.0 ? 1ull : (unsigned long long)share;
   }
-  if (tid == THREADS - 1 && upto < target) {     // beyond everything (rounding): the lowest bin
+  if (tid == kSampleThreads - 1 && upto < target) {     // beyond everything (rounding): the lowest bin
     const unsigned long long left = target - (upto - (k_on ? (unsigned long long)c[0] : m[0]));
     *found = {0, (uint32_t)left, left, all_c, c[0]};
   }
@@ -775,7 +774,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
       });
       __syncthreads();
     }
-    const FirstLevel level = ready ? made : first_level<kSampleThreads>(hist32, hist64, k_on, k, p_keep, scan64, &first);
+    const FirstLevel level = ready ? made : first_level(hist32, hist64, k_on, k, p_keep, scan64, &first);
     const int low_bin = level.bin;
     if (k_on) {
       k_prefix = (uint32_t)low_bin;
@@ -1093,7 +1092,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(
 }
 
 // Whether a step's rows with thresholds are shared between blocks: two more kernels (some 8 us, and 0.3 us a row beside its
-// bytes) against passes of one block over its row alone, which all rows make side by side.  us with top-k / with top-p
+// bytes) against passes of one block over its row alone, which all rows make side by side.  The line looks at all rows of the step (the
+// scratch is theirs), the figures are of steps whose rows all have a threshold: of more rows, few of them with one, sharing would still be
+// ahead (one row with top-p 91 us alone, 37 shared, whatever stands beside it).  us with top-k / with top-p
 // alone, shared against a block a row: 151,936 logits, 1 row 25 / 37 against 42 / 91, 16 rows 33 / 43 and 44 / 99, 64 rows 59 / 77
 // and 60 / 128, 77 rows 66 / 90 and 62 / 131, 140 rows 91 / 123 and 68 / 136; 65,536 logits, 1 row 23 / 28 and 27 / 43, 16
 // rows 29 / 37 and 28 / 50, 64 rows 47 / 62 and 31 / 54; 32,003 logits, 1 row 23 / 28 and 21 / 31, 64 rows 47 / 53 and 24 / 36.

@@ -254,8 +254,10 @@ def gemm(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype, allow_pa
             used = ops.gemm_stream(x, weight, out, splits=splits)
             return out[:used]
     if m > ops.STREAM_MAX_ROWS and out_dtype == torch.float32 and ops.gemm_many_fits(x, weight, n):
-        # The many-rows kernel in one share of K.  Beside the streaming one 128 rows at a time: 2,048 rows, 4,096 x 64 (a decay's low rank, whose
-        # sums stay in float32) 194 -> 14 us, 4,096 x 4,096 1,000 -> 61; 129 rows 28 -> 12 and 84 -> 33, 151,936 x 1,024 164 -> 102
+        # The many-rows kernel in one share of K, whatever the size: beside the streaming one, 64 or 128 rows at a time, 652 products of 129 to
+        # 2,048 rows, 8 to 151,936 weight rows of 64 to 16,384, weights from memory, were all faster, also narrow ones of a long K in one
+        # or two blocks, whose passes are as long a chain each: 1.15 to 35 times, 6 on average (129 rows: 4,096 x 64 12 -> 7 us, 64 x 4,096
+        # 60 -> 26, 4,096 x 4,096 88 -> 38; 2,048 rows: 4,096 x 64, a decay's low rank, whose sums stay in float32, 133 -> 14)
         out = torch.empty((m, n), dtype=torch.float32, device=dev)
         rows, columns = ops.several_plan(1, m, n, k)
         ops.gemm_many(x, weight, out[None], rows=rows, columns=columns)
