@@ -1,0 +1,18 @@
+"""The lines between forms of the generic attention kernel, which give the same bits, lie where both were measured."""
+
+import pytest
+
+from tokamak_amd.kernels.build import load_library
+
+
+# us with a block a head and with heads that share one, over 600 keys
+@pytest.mark.parametrize("float32, tokens, heads, kv_heads, shares", [
+    (1, 8, 64, 8, False),       # 23 and 56: 64 blocks would leave most CUs idle
+    (1, 16, 64, 8, False), (1, 24, 64, 8, True), (1, 96, 64, 8, True),      # 48 and 58, 103 and 57
+    (1, 24, 16, 8, False), (1, 32, 16, 8, True),                            # 32 and 39, 45 and 41
+    (1, 16, 32, 4, False), (1, 32, 16, 2, False), (1, 64, 8, 1, False),     # 23 and 56 each
+    (0, 12, 64, 8, False), (0, 16, 64, 8, False), (0, 24, 64, 8, True),     # 35 and 56, 41 and 57, 66 and 58
+    (0, 32, 16, 8, False), (0, 52, 16, 8, True), (0, 16, 32, 8, False), (0, 32, 32, 8, True),
+    (0, 96, 16, 16, False), (1, 96, 32, 32, False), (0, 1, 64, 4, False)])
+def test_heads_share_a_block_where_that_fills_the_gpu(float32, tokens, heads, kv_heads, shares):
+    assert bool(load_library("attention_generic").tk_attention_heads_share(float32, tokens, heads, kv_heads)) is shares

@@ -653,6 +653,20 @@ bool launch_float32_tiles<float>(const float* q, const float* k_cache, const flo
   return true;
 }
 
+// Heads of a group that share a block at most.
+static int heads_a_block(int group) { return group <= 4 ? 4 : kQueries; }
+
+// Whether the heads of a group share a block for tokens that run alone (the result is the same either way): where each in a block of its
+// own would be more blocks than two a CU and some (float32, whose keys are twice the bytes: than two), and the shared ones, which take two to
+// four times as long, are enough of them.  us alone and shared over 600 keys, heads of 128: bfloat16, 16 heads over 8 kv heads, 32 tokens 26 |
+// 38, 44 43 | 44, 52 50 | 44, 32 over 8, 16 tokens 22 | 38, 24 39 | 38, 32 52 | 39, 64 over 8, 12 tokens (96 shared blocks) 35 | 56, 18 54 | 57, 24 66 | 58;
+// float32, 16 over 8, 24 32 | 39, 32 45 | 41, 48 72 | 51, 64 over 8, 8 23 | 56, 16 48 | 58, 18 65 | 57, 24 103 | 57.  2,432 launches of each type (groups
+// of 2 to 16, heads of 64 to 256, 1 to 96 tokens over 100 to 6,000 keys): 1 % and 2 % behind the faster form on average, 0.56 and 0.49 at worst.
+static bool heads_share(bool float32, long tokens, int nh, int nkv) {
+  const int group = nh / nkv, qt = heads_a_block(group);
+  return group > 1 && tokens * nh > (float32 ? 511 : 576) && tokens * nkv * ((group + qt - 1) / qt) >= (float32 ? 160 : 192);
+}
+
 template <typename T, int SLOTS>
 static void launch_generic(const T* q, const T* k_cache, const T* v_cache, const int* block_tables,
                            const int* positions, const int* req_of_token, GenericItems items,
@@ -666,12 +680,8 @@ static void launch_generic(const T* q, const T* k_cache, const T* v_cache, const
           q, k_cache, v_cache, block_tables, positions, req_of_token, items, out, nh, nkv, hd, vd,  \
           ps, max_pages, scale, span, keep, sinks, cap)
   if (num_single > 0) {
-    // The heads of a group share a block (the result is the same either way) where each in a block of its own would be more blocks
-    // than two a CU and some, us alone and shared: bfloat16, 300 and 1,100 keys, 32 requests of 16 heads over 8 kv heads 15.5 | 20.4 and
-    // 40.9 | 52.3, 40 requests 23.4 | 24.2 and 61.2 | 60.6, 48 28.1 | 24.6 and 69 | 62, 64 of 16 over 4 27.7 | 21.8 and 83 | 54;
-    // float32, whose keys are twice the bytes, 24 15.4 | 21.3 and 54 | 55, 32 18.4 | 22.6 and 80 | 67, 48 36 | 28 and 133 | 97.
-    const int qt = group <= 4 ? 4 : kQueries;
-    const bool shared = group > 1 && (share_heads < 0 ? (long)num_single * nh > (sizeof(T) == 4 ? 511 : 640) : share_heads > 0);
+    const int qt = heads_a_block(group);
+    const bool shared = share_heads < 0 ? heads_share(sizeof(T) == 4, num_single, nh, nkv) : group > 1 && share_heads > 0;
     if (!shared && (long)num_single * nh > 256) TK_ALONE(1, true);
     else if (!shared) TK_ALONE(1, false);
     else if (qt == 4) TK_ALONE(4, false);
@@ -726,6 +736,9 @@ TK_API int tk_paged_attention_generic(int dtype, const void* q, const void* k_ca
 #undef TK_GENERIC
   return launch_status();
 }
+
+// Whether the heads of a group share a block (1 or 0) for so many tokens that run alone.
+TK_API int tk_attention_heads_share(int float32, int tokens, int nh, int nkv) { return heads_share(float32 != 0, tokens, nh, nkv); }
 
 // the same entry points in slot form (slots.h), for launch lists
 TK_SLOTS(tk_paged_attention_generic)
