@@ -16,3 +16,12 @@ from tokamak_amd.kernels.build import load_library
     (0, 96, 16, 16, False), (1, 96, 32, 32, False), (0, 1, 64, 4, False)])
 def test_heads_share_a_block_where_that_fills_the_gpu(float32, tokens, heads, kv_heads, shares):
     assert bool(load_library("attention_generic").tk_attention_heads_share(float32, tokens, heads, kv_heads)) is shares
+
+
+# us with one head a block and with two
+@pytest.mark.parametrize("tiles, heads, kv_heads, dim, a_block", [
+    (2, 16, 8, 128, 1), (16, 16, 8, 128, 1), (17, 16, 8, 128, 2), (64, 32, 8, 128, 2),      # 17 tokens 16 and 24, 1,024 150 and 114
+    (64, 12, 4, 128, 1), (64, 16, 16, 128, 1),                                              # (groups without pairs)
+    (2, 16, 8, 64, 1), (64, 16, 8, 64, 1), (128, 32, 8, 64, 1)])                            # 12 and 17, 78 and 73
+def test_two_heads_share_a_float32_tile_where_blocks_are_many(tiles, heads, kv_heads, dim, a_block):
+    assert load_library("attention_generic").tk_attention_tile_heads(tiles, heads, kv_heads, dim) == a_block

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from tokamak_amd.kernels import ops
+from tokamak_amd.kernels.build import load_library
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -139,3 +140,19 @@ def test_numbers_that_are_not_finite_show_where_they_are_seen(form, where, numbe
             there = seen(cached + t, cached + new, **{n: v for n, v in kw.items() if n not in ("sinks", "softcap")})
             assert bool(there[key]) or bool(tiled[row + t].isfinite().all())
         row += new
+
+
+@pytest.mark.parametrize("hd, kw", [(128, {}), (128, {"window": 70, "keep_first": 3}), (64, {}), (64, {"chunk": 90})])
+def test_many_tiles_of_many_heads(hd, kw):
+    """Enough tiles for blocks of two heads where the head size has them; infinities among the values, too."""
+    nh, nkv, ps = 16, 4, 16
+    s = step([(0, 170), (33, 140), (90, 16)], nh, nkv, hd, hd, ps, torch.float32)
+    if "window" in kw:
+        give_back(s, ps, kw["window"], kw.get("keep_first", 0))
+    assert load_library("attention_generic").tk_attention_tile_heads(s["tiles"][2], nh, nkv, hd) == (2 if hd == 128 else 1)
+    tiled, alone = (attend(s, nh, nkv, hd, hd, ps, tiles, False, **kw) for tiles in (True, False))
+    assert torch.equal(tiled, alone) and bool(tiled.isfinite().all())
+    page = int(s["tables"][0, 100 // ps])
+    s["v"][page, :, 1, 100 % ps // 4, 5, 100 % 4] = float("inf")
+    tiled, alone = (attend(s, nh, nkv, hd, hd, ps, tiles, False, **kw) for tiles in (True, False))
+    assert torch.equal(tiled, alone) and bool(tiled[:100].isfinite().all()) and bool(tiled[100].isinf().any())

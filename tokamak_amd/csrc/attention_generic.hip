@@ -630,6 +630,12 @@ __global__ __launch_bounds__(kWaves * kWave) void attention_float32_tiles_kernel
   }
 }
 
+// Heads of a block of that kernel.  Two read a key's operands once for both, but their blocks are half as many and take twice the products:
+// heads of 128 where one a block would be more blocks than CUs.  us with one and two, 16 heads over 8 kv heads: 17 tokens 16 | 24, 300 39 |
+// 33, 64 behind 2,000 87 | 114, 1,024 150 | 114.  Heads of 64, whose blocks of one head have two to a CU, one: 17 tokens 12 | 17, 300 18 | 22, 1,024
+// 78 | 73.  Beside the form on the vector unit, 972 portions of 2 to 2,048 tokens, 2 to 64 heads: 1.05 to 3.5 times as fast (0.82 with two a block throughout).
+static int tile_heads(int num_tiles, int nh, int nkv, int hd) { return hd == 128 && nh / nkv % 2 == 0 && (long)num_tiles * nh > 256 ? 2 : 1; }
+
 // Whether a portion's tiles took that kernel.
 template <typename T>
 static bool launch_float32_tiles(const T*, const T*, const T*, const int*, const int*, const int*, GenericItems, int, T*, int, int, int, int, int,
@@ -641,13 +647,11 @@ bool launch_float32_tiles<float>(const float* q, const float* k_cache, const flo
                                  const int* req_of_token, GenericItems items, int num_tiles, float* out, int nh, int nkv, int hd, int vd,
                                  int ps, int max_pages, float scale, int span, int keep, const float* sinks, float cap, hipStream_t stream) {
   if (hd != vd || (hd != 64 && hd != 128) || ps % 16 != 0) return false;
-  const bool pairs = nh / nkv % 2 == 0;
 #define TK_TILES(HD_, H_)                                                                                                   \
   attention_float32_tiles_kernel<HD_, H_><<<dim3(num_tiles, nh / H_), kWaves * kWave, 0, stream>>>(                          \
       q, k_cache, v_cache, block_tables, positions, req_of_token, items, out, nh, nkv, ps, max_pages, scale, span, keep, sinks, cap)
-  if (hd == 64 && pairs) TK_TILES(64, 2);
-  else if (hd == 64) TK_TILES(64, 1);
-  else if (pairs) TK_TILES(128, 2);
+  if (hd == 64) TK_TILES(64, 1);
+  else if (tile_heads(num_tiles, nh, nkv, hd) == 2) TK_TILES(128, 2);
   else TK_TILES(128, 1);
 #undef TK_TILES
   return true;
@@ -739,6 +743,9 @@ TK_API int tk_paged_attention_generic(int dtype, const void* q, const void* k_ca
 
 // Whether the heads of a group share a block (1 or 0) for so many tokens that run alone.
 TK_API int tk_attention_heads_share(int float32, int tokens, int nh, int nkv) { return heads_share(float32 != 0, tokens, nh, nkv); }
+
+// Heads of a block for so many tiles of a float32 portion.
+TK_API int tk_attention_tile_heads(int num_tiles, int nh, int nkv, int hd) { return tile_heads(num_tiles, nh, nkv, hd); }
 
 // the same entry points in slot form (slots.h), for launch lists
 TK_SLOTS(tk_paged_attention_generic)
