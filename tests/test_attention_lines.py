@@ -25,3 +25,11 @@ def test_heads_share_a_block_where_that_fills_the_gpu(float32, tokens, heads, kv
     (2, 16, 8, 64, 1), (64, 16, 8, 64, 1), (128, 32, 8, 64, 1)])                            # 12 and 17, 78 and 73
 def test_two_heads_share_a_float32_tile_where_blocks_are_many(tiles, heads, kv_heads, dim, a_block):
     assert load_library("attention_generic").tk_attention_tile_heads(tiles, heads, kv_heads, dim) == a_block
+
+
+# us apart and together, 16 heads over 8 kv heads, 1,024 tokens: 88 and 71 at 128 / 128, 67 and 75 at 64 / 64
+@pytest.mark.parametrize("group, dim, value_dim, shares", [
+    (1, 128, 128, False), (2, 128, 128, True), (3, 128, 64, True), (2, 96, 96, True), (2, 64, 64, False), (3, 64, 48, False),
+    (2, 192, 128, False), (4, 64, 64, True), (4, 512, 448, True)])
+def test_heads_share_a_bfloat16_tile(group, dim, value_dim, shares):
+    assert bool(load_library("attention_tiles").tk_attention_tiles_share(group, dim, value_dim)) is shares

@@ -56,6 +56,8 @@ def near(out, want, bound):
 @pytest.mark.parametrize("heads,kv,hd,vd,ps,portions,window,keep", [
     (4, 2, 64, 64, 16, [(1, 0), (16, 0), (17, 31)], None, 0),          # two waves a block; one to three stages
     (6, 2, 40, 48, 32, [(33, 15), (5, 200)], None, 0),                 # pieces and blocks behind the true sizes
+    (4, 2, 80, 64, 16, [(1, 0), (16, 0), (17, 31)], None, 0),          # two heads a kv head share from 144 channels on
+    (6, 2, 72, 80, 32, [(33, 15), (5, 200)], None, 0),
     (8, 2, 128, 128, 16, [(64, 0), (3, 333)], 50, 0),
     (5, 1, 8, 16, 48, [(20, 90)], 33, 20),                             # the smallest sizes; kept positions, then the window
     (9, 1, 136, 272, 16, [(40, 100)], 64, 4),                          # a second block of heads with one of its own

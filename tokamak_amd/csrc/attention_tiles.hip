@@ -5,7 +5,7 @@
 // kernel below) where a kv head has many query heads.
 //
 // A wave owns one tile (up to 16 consecutive tokens of one request) at one query head.  With one query head a
-// kv head, and with two or three of more than 128 channels, the four waves of a block take four heads of the same tile and every
+// kv head, and with two or three of more than 128 or up to 64 channels, the four waves of a block take four heads of the same tile and every
 // wave fetches its operands itself; else the waves of a block are heads of one kv head and
 // share the operands through LDS (second kernel below).  Keys are walked 16 at a time, operands straight from the pages (no LDS):
 //   S^T[key][token] = K[key][:] . Q[token][:]      v_mfma_f32_16x16x32_bf16, K rows as A (a lane
@@ -178,8 +178,9 @@ __global__ __launch_bounds__(kHeadsPerBlock * 64) void attention_tiles_kernel(
 // 2,048 tokens, 32 heads on one kv head of 512 / 448 channels, window 1,024: 690 -> 280 us (0.35 PFLOP/s); 32 / 8 heads of 128,
 // window 1,024 + 4: 192 -> 118.  What bounds it now: a stage's chain (barrier, scores, softmax, output) at two waves a SIMD, some
 // 4,500 clocks a stage of 960 channels of which LDS is busy 1,900 and the matrix cores 1,000.
-// Also for two and three heads a kv head where a ring is 32 KB (16 / 8 heads of 128, 1,024 tokens 88 -> 71 us, 300 behind
-// 2,000 96 -> 65); of larger heads a block of two waves would have the CU's LDS to itself.
+// Also for two and three heads a kv head where a ring is 24 to 32 KB (16 / 8 heads of 128, 1,024 tokens 88 -> 71 us, 300 behind
+// 2,000 96 -> 65; 1.26 times as fast over 26 portions of 2 to 1,024 tokens, of 96 and of 128 / 64 1.11 and 1.07, 0.95 at worst); of larger heads a
+// block of two waves would have the CU's LDS to itself, of 64 / 64, whose stages are short, it is level (0.89 to 1.20, 16 / 8 heads, 1,024 tokens 67 | 75).
 // Of operands two groups are held in registers, the one that is multiplied and the next (whole stages would be more than the 256
 // registers that two waves a SIMD leave each).
 constexpr int kStages = 4;
@@ -574,6 +575,9 @@ __global__ __launch_bounds__(256) void attention_heads_merge_kernel(
     out[((size_t)single[item] * nh + head) * vd + d] = float_to_bf16(((sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane])) / denom);
 }
 
+// Whether the heads of a kv head share its keys and values through LDS (see the shared kernel).
+bool tiles_share(int group, int hd, int vd) { return group >= 4 || (group >= 2 && hd <= 128 && vd <= 128 && hd + vd > 128); }
+
 }  // namespace
 
 // Tiles of up to 16 consecutive tokens of one request (tile_first, tile_count), bfloat16.  Returns -2
@@ -589,8 +593,7 @@ TK_API int tk_attention_tiles(const void* q, const void* k_cache, const void* v_
       (uintptr_t)out % 8 != 0)
     return -2;
   const int group = nh / nkv;
-  if (group >= 4 || (group >= 2 && hd <= 128 && vd <= 128)) {
-    // the heads of a kv head share its keys and values through LDS (see the kernel: where the lines lie)
+  if (tiles_share(group, hd, vd)) {
 #define TK_SHARED_AS(KCH_, DBL_, HB_, CAP_)                                                                     \
   launch_shared<KCH_, DBL_, HB_, CAP_>(q, k_cache, v_cache, block_tables, max_pages, positions, req_of_token,   \
                                        tile_first, tile_count, num_tiles, out, nh, nkv, hd, vd, ps, scale, span, \
@@ -658,6 +661,9 @@ TK_API int tk_attention_heads(const void* q, const void* k_cache, const void* v_
       part_o, part_ml, single, (bf16_t*)out, nsplit * 4, nh, vd, sinks);
   return launch_status();
 }
+
+// Whether tk_attention_tiles has the heads of a kv head share a block (1 or 0).
+TK_API int tk_attention_tiles_share(int group, int hd, int vd) { return tiles_share(group, hd, vd); }
 
 TK_SLOTS(tk_attention_tiles)
 TK_SLOTS(tk_attention_heads)
