@@ -78,6 +78,7 @@ def test_shared_tiles(heads, kv, hd, vd, ps, portions, window, keep):
     (8, 1, 64, 48, [63, 5], 20, 0, 5),                # most parts have no keys
     (17, 1, 136, 272, [300, 1], None, 0, 5),
     (16, 2, 128, 128, [700], 100, 4, 3),
+    (32, 1, 512, 448, [1040, 90], 1024, 0, 2), (8, 1, 64, 272, [0, 400, 33], None, 0, 4), (24, 2, 40, 80, [130, 7], 50, 20, 1),      # 8, 16 and 4
     (32, 1, 512, 448, [1040], 1024, 0, 16)])          # 64 parts and one step more
 def test_single_tokens_merged(heads, kv, hd, vd, contexts, window, keep, splits):
     """A token's keys dealt to parts, from one to as many as the merge takes, some of them without keys."""

@@ -541,23 +541,26 @@ __global__ __launch_bounds__(256) void attention_heads_kernel(
 }
 
 // out[token][head] = sum_p w_p o_p / (sum_p w_p l_p + exp(sink)), w_p = exp2(m_p - max m); a part without
-// keys has m = -inf and weighs nothing (whatever lies in its output).  A block a (token, head, 64 value channels): its waves
-// take every fourth part, a lane a channel, and add up in wave order; lane p of every wave finds part p's weight (up to 64 parts)
-// while the outputs are on their way, all asked for together.  Asked for eight at a time, each behind a look at its weight,
-// 36 parts of 448 channels of 32 heads took 9.8 us, so 3.
-constexpr int kMergeLoads = 16;      // of a lane: 64 parts by four waves
+// keys has m = -inf and weighs nothing (whatever lies in its output).  A block is 256 channels of a (token, head), a lane one of them, or
+// (SHARED, of more than 16 parts) 64, of which its waves take every fourth part and add up in wave order.  Lane p of every wave finds
+// part p's weight (up to 64 parts) while the outputs are on their way, a lane's LOADS asked for together: fetched eight at a time, each behind a
+// look at its weight, 36 parts of 448 channels of 32 heads took 9.8 us, so 3.  Few parts are a step of many tokens, bound by its blocks and
+// loads: with four waves a channel and 16 loads whatever the parts, 100 tokens of 32 heads of 512 / 448, 300 keys, took 69 us with their attention, so 48.
+template <bool SHARED, int LOADS>
 __global__ __launch_bounds__(256) void attention_heads_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ single,
     bf16_t* __restrict__ out, int parts, int nh, int vd, const float* __restrict__ sinks) {
+  constexpr int kEvery = SHARED ? 4 : 1;
   __shared__ float sums[4][64];
   const int item = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int d = blockIdx.z * 64 + lane;
+  const int d = SHARED ? blockIdx.z * 64 + lane : blockIdx.z * 256 + threadIdx.x, first = SHARED ? wave : 0;
+  if (!SHARED && d - lane >= vd) return;      // (the whole wave)
   const size_t row = ((size_t)item * nh + head) * parts;
   const float2 ml = reinterpret_cast<const float2*>(part_ml)[row + min(lane, parts - 1)];
   const float* po = part_o + row * vd + min(d, vd - 1);
-  float v[kMergeLoads];
+  float v[LOADS];
 #pragma unroll
-  for (int u = 0; u < kMergeLoads; ++u) v[u] = po[(size_t)min(wave + 4 * u, parts - 1) * vd];
+  for (int u = 0; u < LOADS; ++u) v[u] = po[(size_t)min(first + kEvery * u, parts - 1) * vd];
   const float m = lane < parts ? ml.x : -INFINITY;
   const float mx = wave_max(m);                       // finite: the part that holds the token's own key
   const float w = m == -INFINITY ? 0.f : fast_exp2(m - mx);
@@ -565,14 +568,18 @@ __global__ __launch_bounds__(256) void attention_heads_merge_kernel(
   if (sinks) denom += fast_exp2(sinks[head] * 1.4426950408889634f - mx);
   float o = 0.f;
 #pragma unroll
-  for (int u = 0; u < kMergeLoads; ++u) {
-    const float of = __shfl(w, min(wave + 4 * u, 63), kWave);      // (zero from `parts` on)
+  for (int u = 0; u < LOADS; ++u) {
+    const float of = __shfl(w, min(first + kEvery * u, 63), kWave);      // (zero from `parts` on)
     o = of != 0.f ? fmaf(of, v[u], o) : o;
   }
-  sums[wave][lane] = o;
-  __syncthreads();
-  if (wave == 0 && d < vd)
-    out[((size_t)single[item] * nh + head) * vd + d] = float_to_bf16(((sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane])) / denom);
+  bf16_t* const op = out + ((size_t)single[item] * nh + head) * vd + d;
+  if constexpr (SHARED) {
+    sums[wave][lane] = o;
+    __syncthreads();
+    if (wave == 0 && d < vd) *op = float_to_bf16(((sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane])) / denom);
+  } else if (d < vd) {
+    *op = float_to_bf16(o / denom);
+  }
 }
 
 // Whether the heads of a kv head share its keys and values through LDS (see the shared kernel).
@@ -657,8 +664,16 @@ TK_API int tk_attention_heads(const void* q, const void* k_cache, const void* v_
   else TK_HEADS(16, 32);
 #undef TK_HEADS
 #undef TK_HEADS_AS
-  attention_heads_merge_kernel<<<dim3(num_single, nh, (vd + 63) / 64), 256, 0, stream>>>(
-      part_o, part_ml, single, (bf16_t*)out, nsplit * 4, nh, vd, sinks);
+  const int parts = nsplit * 4;
+#define TK_MERGE(SHARED_, LOADS_, CHANNELS_)                                                                              \
+  attention_heads_merge_kernel<SHARED_, LOADS_>                                                                           \
+      <<<dim3(num_single, nh, (vd + CHANNELS_ - 1) / CHANNELS_), CHANNELS_ > vd && !SHARED_ ? (vd + 63) / 64 * 64 : 256, 0, stream>>>( \
+          part_o, part_ml, single, (bf16_t*)out, parts, nh, vd, sinks)
+  if (parts <= 4) TK_MERGE(false, 4, 256);
+  else if (parts <= 8) TK_MERGE(false, 8, 256);
+  else if (parts <= 16) TK_MERGE(false, 16, 256);
+  else TK_MERGE(true, 16, 64);
+#undef TK_MERGE
   return launch_status();
 }
 
