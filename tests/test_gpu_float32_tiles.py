@@ -20,6 +20,26 @@ def test_the_rule_meets_every_tile():
     assert not ops.float32_tiles_pay(40, 4096, 2048) and not ops.float32_tiles_pay(64, 2048, 6144)
 
 
+# us in tiles through LDS and through registers
+@pytest.mark.parametrize("m, n, k, registers", [
+    (2048, 4096, 64, True), (200, 4096, 64, True), (4096, 32768, 32, True), (4096, 8192, 96, True),      # 22.2 and 18.7, 5.9 and 5.2, 346 and 155, 82 and 77
+    (100, 4096, 64, False), (1053, 2048, 32, False), (2048, 4096, 96, False), (4096, 16384, 128, False), (2048, 4096, 1024, False)])
+def test_a_short_k_of_many_results_goes_through_registers(m, n, k, registers):
+    assert ops.float32_through_registers(m, n, k) is registers
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m, n, k", [(130, 4100, 64), (2049, 2057, 32), (129, 4099, 36)])
+def test_both_give_the_same_bits_there(m, n, k):
+    gen = torch.Generator(device=DEV).manual_seed(m)
+    x, w = (torch.randn(s, generator=gen, device=DEV) for s in ((m, k), (n, k)))
+    out, tiles = torch.empty(m, n, device=DEV), torch.empty(m, n, device=DEV)
+    assert ops.float32_through_registers(m, n, k)
+    ops.gemm_tiled(x, w, out)
+    ops._check(ops._fn("gemm_float32", "tk_gemm_float32")(ops._p(x), ops._p(w), ops._p(tiles), m, n, k, k, k, n, 96, 96, ops._stream()), "gemm_float32")
+    assert torch.equal(out, tiles)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("more_m, more_n, k", SHAPES)
 @pytest.mark.parametrize("tile", sorted(ops.FLOAT32_PRICES))

@@ -14,7 +14,8 @@
 // 64 x 64 for the 512 that ran at once, here 242 of 96 x 96); which, ops.float32_tile prices.  Beside tiles of 64 x 64 and 128 x
 // 128 in 32x32x2 products through registers, us: 1,053 rows, weights of 4,096 x 2,048 309 -> 154, 2,048 x 2,048 139 -> 87, 12,288 x
 // 2,048 597 -> 438, 2,048 x 6,144 403 -> 251; 2,048 rows, 12,288 x 2,048 871 -> 780 (132 TFLOP/s); 80 rows, 12,288 x 2,048 91 ->
-// 57, 1,024 x 2,048 54 -> 30; 247 sizes of 65 to 2,048 rows 1.10 to 2.08 times as fast.
+// 57, 1,024 x 2,048 54 -> 30; 247 sizes of 65 to 2,048 rows 1.10 to 2.08 times as fast, others of K of 512 to 1,024 0.95 to 2.1.  A short K of
+// many results is left to that kernel (ops.float32_through_registers).
 #include "common.h"
 #include "lds_copy.h"
 #include "slots.h"

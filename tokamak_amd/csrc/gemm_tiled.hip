@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const TI* __restrict__ 
 }
 
 // The same product on the matrix cores, for operands that gemm_float32.hip does not take (rows off 16-byte borders, K not a
-// multiple of four): v_mfma_f32_32x32x2_f32 multiplies and adds in full
+// multiple of four) and a short K of many results (ops.float32_through_registers): v_mfma_f32_32x32x2_f32 multiplies and adds in full
 // float32 and, for every output element, gives exactly the bits of fmaf over its two k in
 // ascending order (measured against the chain on random operands: every output of every
 // step equal), so a walk over k in steps of two is the chain of the kernels above and below,

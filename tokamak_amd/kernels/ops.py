@@ -1779,6 +1779,15 @@ def float32_tile(m: int, n: int, k: int) -> tuple[int, int]:
     return min(FLOAT32_PRICES, key=lambda tile: _float32_price(*tile, m, n, k))
 
 
+def float32_through_registers(m: int, n: int, k: int) -> bool:
+    """Whether a float32 product takes ``gemm_tiled``'s kernel for operands off their borders, whose operands go through registers, also on them:
+    K of up to three stages and so many results that writing them is most of it, which that kernel does in longer runs.  Beside the tiles of
+    ``gemm_float32``, 1,800 products of 65 to 4,096 rows, 16 to 151,936 weight rows: K of up to 32 from 4 M results on 1.18 times as fast on average
+    (4,096 x 32,768 x 32 346 -> 155 us), of 64 from half a million 1.07 (2,048 x 4,096 22.2 -> 18.7), of 96 from 16 M 1.04; fewer results 0.57 to 1.11.
+    With this line 18 of them are more than 5 % behind that kernel, 0.75 at worst (32,768 weight rows, K of 128), without it 232, 0.47."""
+    return k <= 96 and m * n >= (4 << 20 if k <= 32 else 1 << 19 if k <= 64 else 16 << 20)
+
+
 @functools.lru_cache(maxsize=4096)
 def float32_tiles_pay(m: int, n: int, k: int) -> bool:
     """Whether a float32 product of up to ``FEWROWS_MAX_ROWS`` rows takes tiles where ``fewrows_pays`` would stream the weights, once
@@ -1835,7 +1844,7 @@ def gemm_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, fewrows_spli
     """out[M, N] = a[M, K] @ w[N, K]^T, float32 multiply-add (rows may be strided).  float32
     operands of up to 64 rows go to the weight-streaming kernel where that pays
     (``fewrows_pays``, ``float32_tiles_pay``), others whose rows lie on 16-byte borders to tiles of a size that the product asks
-    for (csrc/gemm_float32.hip); all give the same bits (``fewrows_split``: that kernel with operands split between as many pieces
+    for (csrc/gemm_float32.hip; ``float32_through_registers`` says which do not); all give the same bits (``fewrows_split``: that kernel with operands split between as many pieces
     of K as the rows allow, or not split; None chooses the kernel and the split by the shape)."""
     for t in (a, w, out):
         _need(t.is_cuda and t.dim() == 2 and t.stride(1) == 1, "gemm operands are 2-D GPU tensors with unit inner stride")
@@ -1857,7 +1866,7 @@ def gemm_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, fewrows_spli
                                                         int(fewrows_split is None and fewrows_dealt(rows, n)), _stream()),
                    "gemm_fewrows")
         return
-    if on_borders and m > 0 and n > 0 and max(a.stride(0), w.stride(0)) <= FLOAT32_MAX_STRIDE:
+    if on_borders and m > 0 and n > 0 and max(a.stride(0), w.stride(0)) <= FLOAT32_MAX_STRIDE and not float32_through_registers(m, n, k):
         _check(_fn("gemm_float32", "tk_gemm_float32")(_p(a), _p(w), _p(out), m, n, k, a.stride(0), w.stride(0), out.stride(0),
                                                       *float32_tile(m, n, k), _stream()), "gemm_float32")
         return
