@@ -18,6 +18,7 @@ def test_the_rule_meets_every_tile():
     assert met == set(ops.FLOAT32_PRICES)
     assert ops.float32_tiles_pay(24, 151936, 1024) and ops.float32_tiles_pay(64, 1024, 1024)
     assert not ops.float32_tiles_pay(40, 4096, 2048) and not ops.float32_tiles_pay(64, 2048, 6144)
+    assert not any(ops.float32_tiles_pay(m, 12288, k) for m in (17, 20, 24, 28, 32) for k in (1024, 2048))      # 43 us and 49
 
 
 # us in tiles through LDS and through registers

@@ -1793,10 +1793,11 @@ def float32_tiles_pay(m: int, n: int, k: int) -> bool:
     """Whether a float32 product of up to ``FEWROWS_MAX_ROWS`` rows takes tiles where ``fewrows_pays`` would stream the weights, once
     for every 16 rows: where the passes (each the trips of K, or the weights at 5 TB/s) are priced well above the tiles, whose
     price knows nothing of rows that meet in the same memory channels.  In recorded chains, weights from memory, us: 24 rows, 151,936 x
-    1,024 360 -> 157; 40, 1,024 x 6,144 27.6 -> 18.2 (12,288 x 2,048 66 -> 50; 4,096 x 2,048 stays, 28.2 against 44); 64, 1,024 x
-    1,024 23.2 -> 16.5, 512 x 1,024 22.3 -> 12.2 (2,048 x 6,144 stays, 87 against 126)."""
+    1,024 237 -> 146; 40, 12,288 x 2,048 66 -> 52 (at 17 to 32 rows it stays, 42 to 46 against 49; 4,096 x 2,048 stays, 29 against 44); 64, 1,024
+    x 1,024 24 -> 17, 512 x 1,024 24 -> 13 (2,048 x 6,144 stays, 87 against 127).  Of 1,660 products of 17 to 64 rows none is more than 5 % behind
+    ``fewrows_pays`` alone; 125 that stay would be more than 10 % faster in tiles (6,144 x 1,024 at 40 rows 28 against 19)."""
     passes = -(-m // FEWROWS_GROUP) * max(4.0 + k / 350, 2.0 + n * k / 1.25e6)
-    return passes > 1.4 * _float32_price(*float32_tile(m, n, k), m, n, k)
+    return passes > 1.45 * _float32_price(*float32_tile(m, n, k), m, n, k)
 
 
 def fewrows_dealt(m: int, n: int) -> bool:
