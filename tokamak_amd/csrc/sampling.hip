@@ -1102,6 +1102,9 @@ constexpr int kSharedVocabulary = 65536;
 inline bool shares_rows(int M, int V) { return V >= kSharedVocabulary && M <= (V - kSharedVocabulary / 2) / 1536; }
 constexpr size_t kSharedWords = 3 * kHistWords + 2;     // of a row: counts, masses, the list's length
 
+// The same for callers, who need not say which rows have a threshold where none is shared (1 or 0).
+TK_API int tk_sample_shares_rows(int M, int V) { return shares_rows(M, V); }
+
 TK_API int tk_sample_scratch_bytes(int M, int V) {
   const long rows = M < 1 ? 0 : M;
   const long parts = rows * kArgmaxSegments * 12 + rows * 4 + 16 + rows * 32;

@@ -386,6 +386,7 @@ _SIGS = {
         "tk_argmax_segments": [],
         "tk_sample": [c_void_p, c_long, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p],
         "tk_sample_scratch_bytes": [c_int, c_int],
+        "tk_sample_shares_rows": [c_int, c_int],
     },
 }
 _LIBRARY_FILE = {"attention_fused": "attention_mfma", "attention_pooled_split": "attention_pooled"}   # signature group -> library that holds it
@@ -461,7 +462,7 @@ def _fn(library: str, name: str):
         except AttributeError:
             fn.slots_address = None
         _fns[name] = fn
-    if _profile is not None and name not in ("tk_argmax_segments", "tk_sample_scratch_bytes"):
+    if _profile is not None and name not in ("tk_argmax_segments", "tk_sample_scratch_bytes", "tk_sample_shares_rows"):
         profile = _profile
         return lambda *args: profile.timed(name, fn, args)
     if _recorder is not None:
@@ -2887,6 +2888,12 @@ def argmax(logits: torch.Tensor, out: torch.Tensor, values: torch.Tensor | None 
     part_i = torch.empty(m * segments, dtype=torch.int32, device=logits.device)
     _check(_fn("sampling", "tk_argmax")(_p(logits), _p(out), _p(values), _p(part_v), _p(part_i), m, v,
                                         logits.stride(0), _stream()), "argmax")
+
+
+@functools.lru_cache(maxsize=4096)
+def sample_shares_rows(m: int, v: int) -> bool:
+    """Whether ``sample`` shares the rows that have a threshold between blocks, and so wants to be told which they are."""
+    return bool(_fn("sampling", "tk_sample_shares_rows")(m, v))
 
 
 SAMPLE_INLINE_ROWS = 64     # rows up to which the parameters travel as an argument of the launch (csrc/sampling.hip: kInlineRows)
