@@ -1,7 +1,8 @@
-"""The lines between forms of the generic attention kernel, which give the same bits, lie where both were measured."""
+"""The lines between forms of attention kernels lie where both were measured; operands off the borders of a kernel's loads are refused."""
 
 import pytest
 
+from tokamak_amd.kernels import ops
 from tokamak_amd.kernels.build import load_library
 
 
@@ -33,3 +34,11 @@ def test_two_heads_share_a_float32_tile_where_blocks_are_many(tiles, heads, kv_h
     (2, 192, 128, False), (4, 64, 64, True), (4, 512, 448, True)])
 def test_heads_share_a_bfloat16_tile(group, dim, value_dim, shares):
     assert bool(load_library("attention_tiles").tk_attention_tiles_share(group, dim, value_dim)) is shares
+
+
+def test_parts_off_their_borders_are_refused():
+    heads = load_library("attention_tiles").tk_attention_heads
+    heads.argtypes = ops._SIGS["attention_tiles"]["tk_attention_heads"]
+    for off in (4, 12, 2):      # (of the parts' maxima and sums, read in pairs; the call ends before a launch)
+        at = [4096] * 4 + [16] + [4096] * 3 + [1, 4096, 4096, 4096 + off, 2, 8, 1, 64, 64, 16, 0.125, 0, 0, None, 0.0, None]
+        assert heads(*at) == -2

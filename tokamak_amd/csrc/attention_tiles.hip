@@ -644,7 +644,7 @@ TK_API int tk_attention_heads(const void* q, const void* k_cache, const void* v_
   if (keep < 0 || (keep > 0 && span <= 0) || !(softcap >= 0.f)) return -1;
   if (nkv <= 0 || nh % nkv != 0 || hd < 8 || hd % 8 != 0 || vd < 16 || vd % 16 != 0 || ps < 16 || ps % 16 != 0) return -2;
   if (hd > 512 || vd > 512 || (uintptr_t)q % 16 != 0 || (uintptr_t)k_cache % 16 != 0 || (uintptr_t)v_cache % 16 != 0 ||
-      (uintptr_t)part_o % 16 != 0 || nsplit < 1 || nsplit > 16 || nh > 65535)    // (the merge: up to 64 parts)
+      (uintptr_t)part_o % 16 != 0 || (uintptr_t)part_ml % 8 != 0 || nsplit < 1 || nsplit > 16 || nh > 65535)    // (the merge: up to 64 parts)
     return -2;
   const int group = nh / nkv;
   const dim3 grid(num_single, nkv * ((group + 15) / 16), nsplit);
